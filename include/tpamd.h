@@ -292,6 +292,14 @@ int tpamd_attention_decode_rope_devpos(const void *q_dev, const void *k_dev, con
                                        int64_t Hq, int64_t Hkv, int64_t D, const int64_t *pos_dev, int64_t cache_len,
                                        const int64_t *strides, float scale, int dtype, void *stream);
 
+/* y[r][d] = w[d] * round(x[r][d] * rsqrt(mean over d of x[r][d]^2 + eps)) for `rows` rows of D elements: the RMS norm of the
+ * wrapped Llama-pattern modules (run by src/tensor_parallel/wrapper.py:69-72), which every rank computes on whole rows. Sum
+ * and scaling in fp32, the scaled value rounded to `dtype`, the product with the weight rounded again, as the module's own
+ * sequence of torch ops does. x, w, y in `dtype` (BF16, F16 or F32); y may be x. 16-bit rows of up to 16384 elements on
+ * 16-byte boundaries are read once; anything else takes a kernel with element loads. */
+int tpamd_rms_norm(const void *x_dev, const void *w_dev, void *y_dev, int64_t rows, int64_t D, int64_t ldx, int64_t ldy, float eps,
+                   int dtype, void *stream);
+
 /* Weight-only int8 shard Linear with fp16/bf16 outlier columns:
  *   y[m,n] = act( scale[n] * sum_k x[m,k]*wq[n,k]  +  sum_j x[m,outlier_idx[j]] * w_out[n,j]  + bias[n] )
  * wq is int8 [N,K] (zero in the outlier columns), scale fp32 [N], outlier_idx int32 [n_out] (sorted,

@@ -36,6 +36,7 @@ EXPORTS = (
     "tpamd_swiglu_up",
     "tpamd_linear_w8",
     "tpamd_attention",
+    "tpamd_rms_norm",
     "tpamd_rope_append",
     "tpamd_attention_decode_rope",
     "tpamd_attention_decode_rope_devpos",
@@ -127,6 +128,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_attention_decode_rope_devpos.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, vp, i64, c.POINTER(i64), c.c_float, ci, vp]
     lib.tpamd_rope_append.restype = ci
     lib.tpamd_rope_append.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, c.POINTER(i64), ci, vp]
+    lib.tpamd_rms_norm.restype = ci
+    lib.tpamd_rms_norm.argtypes = [vp, vp, vp, i64, i64, i64, i64, c.c_float, ci, vp]
     lib.tpamd_linear_w8.restype = ci
     lib.tpamd_linear_w8.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, i64, i64, i64, i64, i64, i64, i64, ci, ci, vp]
 
@@ -456,6 +459,24 @@ def swiglu_up(x: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor) -> torch.Tens
             "tpamd_swiglu_up",
         )
     return h.view(*x.shape[:-1], N)
+
+
+def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    """w * (x * rsqrt(mean(x^2) + eps)) over the last axis, sums in fp32, rounded as the two products of tensors of x's dtype."""
+    require_device(x, "rms_norm")
+    if w.dtype != x.dtype or w.device != x.device or w.dim() != 1 or x.dim() == 0 or x.shape[-1] != w.shape[0]:
+        raise ValueError(f"rms_norm: x {tuple(x.shape)} {x.dtype} on {x.device} and w {tuple(w.shape)} {w.dtype} on {w.device} do not fit")
+    x2 = _as_2d(x)
+    w = w.contiguous()
+    rows, D = x2.shape
+    y = torch.empty((rows, D), dtype=x.dtype, device=x.device)
+    with _on_device(x.device):
+        _check(
+            lib().tpamd_rms_norm(x2.data_ptr(), w.data_ptr(), y.data_ptr(), rows, D, _ld(x2), D, float(eps), dtype_code(x.dtype),
+                                 ctypes.c_void_p(current_stream_ptr(x.device))),
+            "tpamd_rms_norm",
+        )
+    return y.view(x.shape)
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None, causal: bool = True,

@@ -8,6 +8,7 @@ blocks with `gate_proj` / `up_proj` / `down_proj` children get a fused gate/up f
 src/tensor_parallel/slicing_configs.py:192-201) is re-classed to a subclass whose forward is the same `tpamd_linear`:
 its weight keeps the [in, out] shape every rule and state dict expects but is stored with the `in` axis fastest, which
 is the kernel's [out, in] layout; the transposing mover writes it that way while slicing, or once at the first forward.
+transformers' `LlamaRMSNorm`, which every rank computes on whole rows, becomes one launch (`tpamd_rms_norm`) in the same way.
 
 Inference only: the kernels have no backward; asking for one raises. Autocast is not applied by these modules: the
 input must already have the weight's dtype (a mismatch raises TypeError where `nn.Linear` under autocast would cast).
@@ -104,6 +105,30 @@ def _shard_conv1d_class(base: type) -> type:
     return cls
 
 
+def is_rms_norm(module: nn.Module) -> bool:
+    """transformers' LlamaRMSNorm: a weight over the last axis and `variance_epsilon`, statistics in fp32."""
+    return type(module).__name__ == "LlamaRMSNorm" and type(module).__module__.split(".")[0] == "transformers" and \
+        isinstance(getattr(module, "weight", None), torch.Tensor) and module.weight.dim() == 1 and hasattr(module, "variance_epsilon")
+
+
+def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
+    w = self.weight
+    if hidden_states.dtype != w.dtype or hidden_states.device.type != "cuda":  # a promoting norm: the module's own forward
+        return type(self).__mro__[1].forward(self, hidden_states)
+    return _guard(_native.rms_norm(hidden_states.detach(), w.detach(), self.variance_epsilon), hidden_states, w)
+
+
+_rms_norm_classes: dict = {}
+
+
+def _shard_rms_norm_class(base: type) -> type:
+    cls = _rms_norm_classes.get(base)
+    if cls is None:
+        cls = _rms_norm_classes[base] = type("Shard" + base.__name__, (base,), {"forward": _rms_norm_forward, "__doc__": "The base class with "
+                                                                             "its forward as one launch (`tpamd_rms_norm`)."})
+    return cls
+
+
 def _is_silu(fn) -> bool:
     if isinstance(fn, nn.SiLU):
         return True
@@ -165,6 +190,8 @@ def install_shard_kernels(shard: nn.Module) -> None:
             module.__class__ = ShardLinear
         elif is_conv1d(module) and type(module).__name__ == "Conv1D" and module.weight.dim() == 2 and module.weight.dtype in (torch.bfloat16, torch.float16, torch.float32):
             module.__class__ = _shard_conv1d_class(type(module))
+        elif is_rms_norm(module) and module.weight.dtype in (torch.bfloat16, torch.float16, torch.float32):
+            module.__class__ = _shard_rms_norm_class(type(module))
     for module in shard.modules():
         if is_gated_silu_mlp(module):
             module.forward = types.MethodType(_gated_mlp_first_forward, module)

@@ -1,0 +1,62 @@
+"""`tpamd_rms_norm` against the definition in fp64 on the host, rounded as the module's own sequence of torch ops rounds: row
+lengths at the edges of the kernel's block shapes and outside its vector path."""
+import pytest
+import torch
+
+from tensor_parallel_amd import _native
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def rms_ref(x, w, eps):
+    x64 = x.double()
+    n = (x64 * torch.rsqrt(x64.square().mean(-1, keepdim=True) + eps)).to(x.dtype)
+    return w * n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,D", [(1, 8), (3, 512), (2, 520), (5, 2048), (2, 2056), (1, 4096), (37, 4096), (3, 4104), (2, 8192), (2, 16384), (2, 16392),
+                                    (4, 100), (3, 7)])
+def test_rms_norm(dtype, rows, D):
+    g = torch.Generator().manual_seed(D)
+    x = (torch.randn(rows, D, generator=g) * 3).to(dtype)
+    w = (1 + 0.3 * torch.randn(D, generator=g)).to(dtype)
+    got = _native.rms_norm(x.to(DEV), w.to(DEV), 1e-5).cpu()
+    # the fp32 statistics may put a scaled value on the other side of a rounding boundary: one unit of the dtype in the scaled
+    # value, which the product with the weight and its own rounding can carry to two
+    unit = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -22}[dtype]
+    torch.testing.assert_close(got.double(), rms_ref(x, w, 1e-5).double(), rtol=4 * unit, atol=1e-6)
+    if dtype != torch.float32:  # ... and that is rare
+        assert (got != rms_ref(x, w, 1e-5)).double().mean().item() < 0.02
+
+
+def test_rms_norm_takes_strided_rows_and_refuses_what_does_not_fit():
+    g = torch.Generator().manual_seed(0)
+    big = torch.randn(6, 4096, generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.ones(2048, dtype=torch.bfloat16, device=DEV)
+    for part in (big[:, 2048:], big[:, 1:2049]):  # 16-byte aligned rows, and rows that are not
+        assert torch.equal(_native.rms_norm(part, w, 1e-6), _native.rms_norm(part.contiguous(), w, 1e-6))
+    with pytest.raises(ValueError):
+        _native.rms_norm(big, w, 1e-6)
+    with pytest.raises(ValueError):
+        _native.rms_norm(big[:, :2048], w.float(), 1e-6)
+    assert _native.rms_norm(big[:0, :2048], w, 1e-6).shape == (0, 2048)
+
+
+def test_shards_of_a_llama_use_it():
+    import transformers as tf
+
+    import tensor_parallel_amd as tp
+
+    torch.manual_seed(0)
+    cfg = tf.LlamaConfig(vocab_size=96, hidden_size=64, intermediate_size=128, num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2)
+    model = tf.LlamaForCausalLM(cfg).to(torch.bfloat16).eval()
+    split = tp.tensor_parallel(model, [DEV, DEV])
+    norms = [m for m in split.modules() if type(m).__name__ == "ShardLlamaRMSNorm"]
+    assert len(norms) == 2 * 5
+    x = torch.randn(3, 64).to(torch.bfloat16)
+    with torch.no_grad():
+        torch.testing.assert_close(norms[0](x.to(DEV)).float().cpu(), model.model.norm(x.to(model.device)).float().cpu(), rtol=2e-2, atol=1e-2)
+        promoted = norms[0](x.float().to(DEV))  # another dtype than the weight's: the module's own forward
+    assert promoted.dtype == torch.float32
