@@ -16,7 +16,7 @@
  *     message the library keeps one piece of state: tpamd_linear / tpamd_linear_add / tpamd_swiglu_up split K for
  *     shapes with few output tiles (M from 17 to a few thousand, decided by a cost model), tpamd_linear_w8 does so
  *     from 2 rows on large matrices, tpamd_attention splits long key ranges, and they keep fp32 scratch buffers for
- *     the partial results: one per (device, stream), 64 MiB on a 256-CU part, allocated with hipMalloc at the
+ *     the partial results: one per (device, stream), 68 MiB on a 256-CU part, allocated with hipMalloc at the
  *     stream's first such call and kept until the process ends (at most 32 streams per device get one; calls on
  *     further streams run unsplit). Streams never share a buffer, so such calls on different streams of a device
  *     need no ordering among themselves. Nothing can be allocated while a stream is being captured: the first
@@ -305,8 +305,9 @@ int tpamd_rms_norm(const void *x_dev, const void *w_dev, void *y_dev, int64_t ro
  * wq is int8 [N,K] (zero in the outlier columns), scale fp32 [N], outlier_idx int32 [n_out] (sorted,
  * distinct, < K), w_out [N,n_out] in `dtype` with leading dimension ld_wout. Not part of the reference
  * (its README points to LLM.int8 notebooks); defined here in closed form.
- * Up to 64 rows the weights are streamed once (HBM-bound kernels); up to 128-256 rows once per slab of 64 rows; above
- * that they go through the matrix pipe once, converted to `dtype` (exactly) on their way into LDS.
+ * Up to 64 rows (up to 128 on small matrices, once per 64 rows) the weights are streamed by HBM-bound kernels; above that
+ * they go through the matrix pipe once, converted to `dtype` (exactly) in front of it; K % 64 == 0 takes the faster of two
+ * such kernels.
  * Requirements: dtype is F16 or BF16; K % 16 == 0; ldw (int8 elements) % 16 == 0. */
 int tpamd_linear_w8(const void *x_dev, const void *wq_dev, const void *scale_dev, const void *outlier_idx_dev,
                     const void *w_out_dev, int64_t n_out, const void *bias_dev, void *y_dev, int64_t M, int64_t N,

@@ -47,6 +47,8 @@ struct Tuning {
     int skinny_pair;         // TPAMD_SKINNY_PAIR: 8-column form of the gated pair
     int skinny_resident;     // TPAMD_SKINNY_RESIDENT: x-resident kernel on/off
     int w8_split;            // TPAMD_W8_SPLIT: int8 K-split kernel on/off
+    int w8_tile;             // TPAMD_W8_TILE: 256 or 128 rows per tile of the tiled int8 kernel
+    int w8_tile_splits;      // TPAMD_W8_TILE_SPLITS: its K splits
     int w8_cols;             // TPAMD_W8_COLS: int8 K-split kernel whose wavefronts own columns (x of the split in LDS): 0 = off, 1 = whenever the shape allows
     int skinny_max_m;        // TPAMD_SKINNY_MAX_M: most rows of a single 16-bit matrix that go to the weight-streaming kernels (16 to 64; unset: by shape)
     int skinny_xlds;         // TPAMD_SKINNY_XLDS: 0 = gated pair at 4-16 rows through the older kernels
@@ -66,7 +68,9 @@ int device_cus(int dev, int *cus_out);
 // fp32 scratch memory of the K-split kernels (split-K partial tiles, split-key attention partials): defined in
 // runtime.hip. Callers hold splitk_mutex(dev), the lock of their device, from the lookup until their launches that use
 // the buffer are enqueued (two host threads that share a stream must not interleave a K-split launch and its finishing
-// pass), and pass reserve = 4 * CUs * 64 KiB, so that a stream's buffer is allocated with the size every shape can live with.
+// pass), and pass reserve = scratch_reserve(CUs), so that a stream's buffer is allocated with the size every shape can live
+// with: four 128 x 128 partial tiles per CU, and 4 MiB for the packed outlier columns of an int8 Linear beside them.
+static inline size_t scratch_reserve(int cus) { return static_cast<size_t>(4) * cus * 128 * 128 * sizeof(float) + (static_cast<size_t>(4) << 20); }
 std::mutex &splitk_mutex(int dev);
 int splitk_scratch(int dev, hipStream_t stream, size_t need, size_t reserve, void **out);
 // While one of these lives on a host thread, splitk_scratch() on that thread hands out the library's fixed array and

@@ -1289,6 +1289,8 @@ struct W8Extra {
     const char *w_out;
     int n_out;
     int64_t ld_wout;
+    const char *xo, *wo;  // outlier columns of x and w packed to rows of 32 * o_steps elements (gemm_w8_direct_kernel)
+    int o_steps;
 };
 
 template <int DT, int BM, int BN, int WAVES_M, int WAVES_N>
@@ -1481,6 +1483,385 @@ int launch_gemm_w8(GemmParams p, const W8Extra &q, hipStream_t s) {
     const int64_t blocks = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
     TPAMD_REQUIRE(blocks < (1ll << 31), "gemm: too many tiles");
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(NT), LDS, s, p, q);
+    TPAMD_HIP(hipGetLastError());
+    return TPAMD_OK;
+}
+
+// gemm_w8_direct_kernel: the tiled int8 kernel for K % 64 == 0. 16 * TMX x-rows by 256 w-rows per block, 4 wavefronts side by
+// side along the columns (each all x rows by 64 w rows), K tiles of 64 in NS LDS stages.
+//
+// Bound: the matrix pipe (M >= 512), with one vector instruction per weight (bf16: 1.5) for the conversion running beside it:
+// 16384 x 8192 at 1024 rows 316 -> 228 us (1.21 PFLOP/s; the same product on f16 weights takes 215), 8192 x 16384 479 -> 232,
+// 4608 x 8192 150 -> 98, 8192 x 4096 133 -> 69; at 200 rows 192 -> 80, 191 -> 79, 92 -> 40 and 95 -> 38 us (before: a tiled kernel
+// that staged the weights through registers, slabs of 64 rows below 257 rows). What the
+// split between the wavefronts is for: every weight of the block is converted by exactly one wavefront (two wavefronts per
+// w row would double the conversions), right before it is multiplied, so that the weights cross LDS as bytes and reach
+// it without passing through registers (global->LDS loads, like x). A weight fragment read of 16 bytes holds both k steps of
+// a lane: lane group lq owns bytes 16 lq ... 16 lq + 15 of the 64 of a K tile, eight per step, and x is read in the
+// same order (its 16-byte chunk 2 lq + kk), which permutes k inside a tile alike for both operands.
+//   step A (kk 0)  MFMAs on weight buffer 0; converts the upper halves of the weight bytes into buffer 1
+//   step B (kk 1)  MFMAs on weight buffer 1; a few MFMAs in, the barrier: tile g+1 has landed ((NS-2) younger tiles in flight),
+//                  the stage of tile g is read out; then the weight bytes of tile g+1 are read and their lower halves
+//                  converted into buffer 0, and tile g+NS is requested into the stage of tile g
+// x fragments need no second buffer: the four MFMAs that use one done, it is read again for the next step, a whole step ahead
+// of its use (with two buffers the 256-row tile ran out of registers and moved 32 of them to AGPRs and back per K tile).
+// LDS: x as in gemm_direct_kernel; w in blocks of 16 rows x 64 bytes (1 KiB, one wavefront-wide load), chunk c of row r in slot
+// c ^ ((r / 2) % 4) ^ (r / 8): 8 rows that follow one another, and rows 4 apart, hit different banks.
+// After the K loop the sums are multiplied by the rows' scales; the outlier columns (packed by
+// w8_pack_outliers_kernel, zeros up to a multiple of 32) follow in steps of 32 into the same accumulators.
+// SPLIT: unit u is tile u % tiles, K range u / tiles; the scaled sums (range 0: with the outlier columns) go to p.ws as
+// 128 x 128 tiles for splitk_finish_kernel.
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void unrolled(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        unrolled<N, I + 1>(f);
+    }
+}
+
+// All but the YOUNGER last LDS reads of this wavefront have arrived, the named registers among them (the reads are asm
+// statements: the waits are ours).
+template <int YOUNGER>
+__device__ __forceinline__ void reads_landed(u32x4 &r) {
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "n"(YOUNGER) : "memory");
+}
+__device__ __forceinline__ void already_landed(u32x4 &r) { asm volatile("" : "+v"(r)); }  // uses stay behind the wait in front of this
+template <int YOUNGER>
+__device__ __forceinline__ void reads_landed(u32x4 (&r)[4]) {
+    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "n"(YOUNGER) : "memory");
+}
+
+// cvt_i8x4 one instruction at a time: step<0>, step<1>, ... step<OPS - 1> leave the four converted weights in lo, hi. The
+// conversions take their byte through the sub-dword selects (f16: 4 instructions where bias, permute and subtract took 5; bf16: 6
+// where they took 11).
+template <int DT>
+struct W8Convert;
+template <>
+struct W8Convert<TPAMD_F16> {
+    static constexpr int OPS = 4;
+    template <int OP>
+    __device__ __forceinline__ void step(uint32_t q, uint32_t &lo, uint32_t &hi) {
+        // the upper halves are written two instructions or more behind the lower ones that they keep
+        if constexpr (OP == 0) asm("v_cvt_f16_i16_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(lo) : "v"(q));
+        if constexpr (OP == 1) asm("v_cvt_f16_i16_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(hi) : "v"(q));
+        if constexpr (OP == 2) asm("v_cvt_f16_i16_sdwa %0, sext(%1) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_1" : "+v"(lo) : "v"(q));
+        if constexpr (OP == 3) asm("v_cvt_f16_i16_sdwa %0, sext(%1) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_3" : "+v"(hi) : "v"(q));
+    }
+};
+template <>
+struct W8Convert<TPAMD_BF16> {
+    static constexpr int OPS = 6;
+    float f0, f1;
+    template <int OP>
+    __device__ __forceinline__ void step(uint32_t q, uint32_t &lo, uint32_t &hi) {
+        // an integer of 8 bits is exact in the upper half of its fp32 value
+        if constexpr (OP == 0) f0 = static_cast<float>(static_cast<signed char>(q));
+        if constexpr (OP == 1) f1 = static_cast<float>(static_cast<signed char>(q >> 8));
+        if constexpr (OP == 2) lo = __builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
+        if constexpr (OP == 3) f0 = static_cast<float>(static_cast<signed char>(q >> 16));
+        if constexpr (OP == 4) f1 = static_cast<float>(static_cast<signed char>(q >> 24));
+        if constexpr (OP == 5) hi = __builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
+    }
+};
+
+template <int DT, int TMX, int NS, bool SPLIT>
+__global__ __launch_bounds__(256) void gemm_w8_direct_kernel(GemmParams p, W8Extra q) {
+    constexpr int BM = 16 * TMX, BN = 256;
+    constexpr int BLK = 1152;                       // 8 staged x rows
+    constexpr int XREG = (BM / 8) * BLK, STAGE = XREG + BN * 64;
+    constexpr int XB = BM / 32, WB = 4;             // global->LDS loads per wavefront and K tile
+    constexpr int LPT = XB + WB;
+    static_assert(NS * STAGE <= 160 * 1024, "LDS");
+    extern __shared__ __align__(16) char smem[];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, lq = lane >> 4;
+    const int total_tiles = p.tiles_m * p.tiles_n;
+    const int tile = SPLIT ? blockIdx.x % total_tiles : blockIdx.x;
+    const int split = SPLIT ? blockIdx.x / total_tiles : 0;
+    const int KT_ALL = p.K / BK;
+    const int kbase = SPLIT ? split * p.kt_per_split : 0;
+    const int KT = SPLIT ? min(p.kt_per_split, KT_ALL - kbase) : KT_ALL;
+    int tile_m, tile_n;
+    tile_of_block(tile, total_tiles, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    const int m0 = tile_m * BM, n0 = tile_n * BN;
+
+    // ---- load addresses: four consecutive blocks share one LDS base and differ in the immediate offset, which the hardware also
+    // adds to the global address (taken off here; rows past the end are clamped, a negative difference wraps and reads zeros)
+    uint32_t x_off[XB], w_off[WB];
+    const int rb = lane >> 3;
+#pragma unroll
+    for (int i = 0; i < XB; ++i) {
+        int r = (wave * XB + i) * 8 + rb;
+        r = m0 + r < p.M ? r : p.M - 1 - m0;
+        x_off[i] = static_cast<uint32_t>(r) * static_cast<uint32_t>(p.ldx * 2) + ((lane & 7) ^ rb) * 16 - (i & 3) * BLK;
+    }
+    auto w_slot = [](int row) { return ((row >> 1) & 3) ^ ((row >> 3) & 1); };
+    const int wr16 = lane >> 2;  // row inside a block of 16
+#pragma unroll
+    for (int i = 0; i < WB; ++i) {
+        int r = (wave * WB + i) * 16 + wr16;
+        r = n0 + r < p.N ? r : p.N - 1 - n0;
+        w_off[i] = static_cast<uint32_t>(r) * static_cast<uint32_t>(p.ldw) + ((lane & 3) ^ w_slot(wr16)) * 16 - i * 1024;
+    }
+    const int x_rows = p.M - m0 < BM ? p.M - m0 : BM, w_rows = p.N - n0 < BN ? p.N - n0 : BN;
+    const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(p.x + static_cast<int64_t>(m0) * p.ldx * 2,
+                                                    static_cast<uint32_t>(x_rows - 1) * static_cast<uint32_t>(p.ldx * 2) + static_cast<uint32_t>(p.K) * 2);
+    const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(p.w + static_cast<int64_t>(n0) * p.ldw,
+                                                    static_cast<uint32_t>(w_rows - 1) * static_cast<uint32_t>(p.ldw) + static_cast<uint32_t>(p.K));
+    auto load = [&](auto ic, int kt, int stage_off) {  // load number ic of K tile kt
+        constexpr int i = decltype(ic)::value;
+        if constexpr (i < XB)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, (lds_void *)(smem + stage_off + (wave * XB + (i & ~3)) * BLK), 16,
+                                                     static_cast<int>(x_off[i]), (kbase + kt) * (BK * 2), (i & 3) * BLK, 0);
+        else
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(smem + stage_off + XREG + wave * (WB * 1024)), 16,
+                                                     static_cast<int>(w_off[i - XB]), (kbase + kt) * BK, (i - XB) * 1024, 0);
+    };
+
+    // ---- fragment addresses
+    const uint32_t smem_base = lds_addr_of(smem);
+    const uint32_t x_rd = smem_base + (l16 >> 3) * BLK + (l16 & 7) * 128;
+    const uint32_t kk_off[2] = {static_cast<uint32_t>(((2 * lq) ^ (l16 & 7)) * 16), static_cast<uint32_t>(((2 * lq + 1) ^ (l16 & 7)) * 16)};
+    const uint32_t w_rd = smem_base + XREG + wave * (WB * 1024) + l16 * 64 + (lq ^ w_slot(l16)) * 16;
+
+    f32x4 acc[TMX][4];
+    u32x4 xq[TMX], wq[2][4], raw[4];
+#pragma unroll
+    for (int a = 0; a < TMX; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // The conversion of one dword (4 weights; dword j % 2 of k step h of row tile j / 2) as single instructions, so that they can
+    // be placed one or two behind every MFMA: the vector port takes them while the matrix pipe works on that MFMA, but a run
+    // of five behind a run of four MFMAs waits for the pipe first and then keeps it idle.
+    constexpr int UOPS = W8Convert<DT>::OPS;
+    W8Convert<DT> cv;
+    auto convert_op = [&](auto hc, auto oc) {
+        constexpr int h = decltype(hc)::value, j = decltype(oc)::value / UOPS, op = decltype(oc)::value % UOPS, b = j / 2, d = j % 2;
+        uint32_t lo = wq[h][b][2 * d], hi = wq[h][b][2 * d + 1];
+        cv.template step<op>(raw[b][2 * h + d], lo, hi);
+        wq[h][b][2 * d] = lo;
+        wq[h][b][2 * d + 1] = hi;
+    };
+    auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
+    constexpr int MF = TMX * 4;                // MFMAs of a step, fragment a = m / 4 against row tile m % 4
+    constexpr int BAR = TMX == 16 ? 4 : 2;     // pair of MFMAs of step B in front of which the barrier sits
+    constexpr int CV0 = TMX == 16 ? 20 : 14;   // first MFMA of step B with a conversion behind it
+    const std::integral_constant<int, 0> half0{};
+    const std::integral_constant<int, 1> half1{};
+
+    // ---- first tiles
+    unrolled<NS>([&](auto sc) {
+        constexpr int s = decltype(sc)::value;
+        const int kt = s < KT ? s : KT - 1;
+        unrolled<LPT>([&](auto ic) { load(ic, kt, s * STAGE); });
+    });
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * LPT) : "memory");
+    unrolled<4>([&](auto bc) { raw[decltype(bc)::value] = lds_read16<decltype(bc)::value * 1024>(w_rd); });
+    unrolled<TMX>([&](auto ac) { xq[decltype(ac)::value] = lds_read16<decltype(ac)::value * 2 * BLK>(x_rd + kk_off[0]); });
+    reads_landed<TMX - 1>(raw);
+    unrolled<8 * UOPS>([&](auto oc) { convert_op(half0, oc); });
+    fence();
+
+    int cur = 0, nxt = STAGE;  // stage offsets of tiles g and g + 1
+    for (int g = 0; g < KT; ++g) {
+        {   // step A
+            const uint32_t xa = x_rd + cur + kk_off[1];
+            unrolled<MF>([&](auto mc) {
+                constexpr int m = decltype(mc)::value, a = m / 4, b = m % 4;
+                // in step B and here a fragment's next read follows its last use: TMX - 1 reads are younger than fragment a's
+                if constexpr (b == 0) { reads_landed<TMX - 1>(xq[a]); fence(); }
+                acc[a][b] = mfma16<DT>(wq[0][b], xq[a], acc[a][b]);
+                fence();
+                if constexpr (b == 3) xq[a] = lds_read16<a * 2 * BLK>(xa);
+                constexpr int o0 = m * 8 * UOPS / MF, o1 = (m + 1) * 8 * UOPS / MF;
+                unrolled<o1 - o0>([&](auto oc) { convert_op(half1, std::integral_constant<int, o0 + decltype(oc)::value>{}); });
+                fence();
+            });
+        }
+        {   // step B
+            const uint32_t xa = x_rd + nxt + kk_off[0], wa = w_rd + nxt;
+            const int kload = g + NS < KT ? g + NS : KT - 1;  // past the end the last tile again, into a stage nobody reads any more
+            unrolled<MF>([&](auto mc) {
+                constexpr int m = decltype(mc)::value, a = m / 4, b = m % 4, s = m / 2;
+                if constexpr (m == 2 * BAR) {
+                    // this wavefront has read tile g out, its part of tile g + 1 has landed; then everybody's
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * LPT) : "memory");
+                    fence();
+                }
+                // TMX - 1 - a reads of step A are younger than fragment a's; the barrier has waited for all of them
+                if constexpr (b == 0 && s < BAR) { reads_landed<TMX - 1 - a>(xq[a]); fence(); }
+                if constexpr (b == 0 && s >= BAR) already_landed(xq[a]);
+                acc[a][b] = mfma16<DT>(wq[1][b], xq[a], acc[a][b]);
+                fence();
+                if constexpr (m % 2 == 1) {
+                    // reads in order: the weight bytes, then the x fragments, each behind its last use and the barrier
+                    if constexpr (s == BAR || s == BAR + 1) {
+                        raw[2 * (s - BAR)] = lds_read16<2 * (s - BAR) * 1024>(wa);
+                        raw[2 * (s - BAR) + 1] = lds_read16<(2 * (s - BAR) + 1) * 1024>(wa);
+                    }
+                    constexpr int xs = s - BAR - 2;  // x fragments 0, 1, ... from pair BAR + 2 on, one per pair while behind
+                    constexpr int xr = xs < 0 ? -1 : (2 * xs + 1 <= s ? xs : (s % 2 == 1 ? (s - 1) / 2 : -1));
+                    if constexpr (xr >= 0 && xr < TMX) xq[xr] = lds_read16<xr * 2 * BLK>(xa);
+                } else {
+                    constexpr int ls = MF / 2 - BAR - 1;  // loads evenly over the pairs behind the barrier
+                    constexpr int l0 = s > BAR ? (s - BAR - 1) * LPT / ls : 0, l1 = s > BAR ? (s - BAR) * LPT / ls : 0;
+                    if constexpr (l1 > l0) load(std::integral_constant<int, l0>{}, kload, cur);
+                }
+                if constexpr (m >= CV0) {
+                    if constexpr (m == CV0) reads_landed<TMX == 16 ? 4 : 3>(raw);  // that many x fragments were asked for since
+                    constexpr int n = MF - CV0, o0 = (m - CV0) * 8 * UOPS / n, o1 = (m + 1 - CV0) * 8 * UOPS / n;
+                    unrolled<o1 - o0>([&](auto oc) { convert_op(half0, std::integral_constant<int, o0 + decltype(oc)::value>{}); });
+                }
+                fence();
+            });
+        }
+        cur = nxt;
+        nxt = nxt + STAGE == NS * STAGE ? 0 : nxt + STAGE;
+    }
+    // every load and fragment read of this wavefront is done before another use of the stages and registers
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    unrolled<TMX>([&](auto ac) { reads_landed<0>(xq[decltype(ac)::value]); });
+    fence();
+    drain_and_barrier();
+
+    // ---- the int8 sums become real ones: lane (l16, lq) holds columns 16 b + 4 lq ... + 3 of row 16 a + l16
+    const int n_wave = n0 + wave * 64;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            int n = n_wave + b * 16 + lq * 4 + j;
+            n = n < p.N ? n : p.N - 1;
+            const float sc = q.scale[n];
+#pragma unroll
+            for (int a = 0; a < TMX; ++a) acc[a][b][j] *= sc;
+        }
+    if (q.o_steps > 0 && split == 0) {
+        const uint32_t pitch = static_cast<uint32_t>(q.o_steps) * 64;
+        const __amdgpu_buffer_rsrc_t xo = make_rsrc(q.xo + static_cast<int64_t>(m0) * pitch, static_cast<uint32_t>(x_rows) * pitch);
+        const __amdgpu_buffer_rsrc_t wo = make_rsrc(q.wo + static_cast<int64_t>(n0) * pitch, static_cast<uint32_t>(w_rows) * pitch);
+        const uint32_t chunk = ((lane & 3) ^ w_slot(wr16)) * 16;
+        const uint32_t o_rd = smem_base + l16 * 64 + (lq ^ w_slot(l16)) * 16;
+        for (int o = 0; o < q.o_steps; ++o) {
+            // rows past the end read zeros
+            unrolled<TMX / 4>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int blk = wave * (TMX / 4) + i;
+                buffer_load16_to_lds(xo, static_cast<uint32_t>(blk * 16 + wr16) * pitch + chunk, o * 64, smem + blk * 1024);
+            });
+            unrolled<4>([&](auto ic) {
+                const int blk = wave * 4 + decltype(ic)::value;
+                buffer_load16_to_lds(wo, static_cast<uint32_t>(blk * 16 + wr16) * pitch + chunk, o * 64, smem + TMX * 1024 + blk * 1024);
+            });
+            drain_and_barrier();
+            unrolled<TMX>([&](auto ac) { xq[decltype(ac)::value] = lds_read16<decltype(ac)::value * 1024>(o_rd); });
+            unrolled<4>([&](auto bc) { raw[decltype(bc)::value] = lds_read16<decltype(bc)::value * 1024>(o_rd + TMX * 1024 + wave * 4096); });
+            reads_landed<0>(raw);
+            unrolled<TMX>([&](auto ac) { reads_landed<0>(xq[decltype(ac)::value]); });
+            drain_and_barrier();  // the next step overwrites what was read
+            fence();
+#pragma unroll
+            for (int a = 0; a < TMX; ++a)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) acc[a][b] = mfma16<DT>(raw[b], xq[a], acc[a][b]);
+        }
+    }
+    if constexpr (SPLIT) {
+        const int tm128 = (p.M + 127) / 128, tn128 = (p.N + 127) / 128;
+        const int n128 = n_wave >> 7;
+        if (n128 < tn128) {
+#pragma unroll
+            for (int a = 0; a < TMX; ++a) {
+                const int m = m0 + a * 16 + l16, m128 = m >> 7;
+                if (m >= p.M) continue;  // the finishing pass reads valid rows only
+                float *ws = p.ws + (static_cast<int64_t>(split) * tm128 * tn128 + static_cast<int64_t>(m128) * tn128 + n128) * (128 * 128) +
+                            (m & 127) * 128 + (n_wave & 64) + lq * 4;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) *reinterpret_cast<f32x4 *>(ws + b * 16) = acc[a][b];
+            }
+        }
+    } else {
+        const bool wide = (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && p.ldy % 8 == 0;
+        char *slab = smem + wave * (16 * EP_PITCH);  // the stages (and the outlier tiles) are read out
+        if (p.act == TPAMD_ACT_GELU) staged_epilogue<DT, MODE_LINEAR, true, TMX, 4, 1, 4, 0>(p, acc, slab, m0, n_wave, lane, wide);
+        else staged_epilogue<DT, MODE_LINEAR, false, TMX, 4, 1, 4, 0>(p, acc, slab, m0, n_wave, lane, wide);
+    }
+}
+
+// The outlier columns of x and w as rows of 32 * steps elements (zeros behind the last): xo [M][...], then wo [N][...]. One
+// thread per 8 elements.
+__global__ __launch_bounds__(256) void w8_pack_outliers_kernel(GemmParams p, W8Extra q, char *xo, char *wo) {
+    const int chunks = q.o_steps * 4;
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t row = e / chunks;
+    const int c = static_cast<int>(e - row * chunks);
+    if (row >= static_cast<int64_t>(p.M) + p.N) return;
+    const bool is_x = row < p.M;
+    const int64_t r = is_x ? row : row - p.M;
+    const uint16_t *src = is_x ? reinterpret_cast<const uint16_t *>(p.x) + r * p.ldx : reinterpret_cast<const uint16_t *>(q.w_out) + r * q.ld_wout;
+    uint32_t v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int o = c * 8 + i, oc = o < q.n_out ? o : q.n_out - 1;
+        v[i] = o < q.n_out ? src[is_x ? q.outlier_idx[oc] : oc] : 0u;
+    }
+    *reinterpret_cast<uint4 *>((is_x ? xo : wo) + (r * chunks + c) * 16) =
+        make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
+}
+
+template <int DT, int TMX, int NS>
+int launch_w8_direct(GemmParams p, W8Extra q, int cus, int splits, hipStream_t s) {
+    constexpr int BM = 16 * TMX, LDS = NS * ((BM / 8) * 1152 + 256 * 64);
+    static thread_local int configured_dev = -1;
+    int dev = 0;
+    TPAMD_HIP(hipGetDevice(&dev));
+    if (configured_dev != dev) {
+        TPAMD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_w8_direct_kernel<DT, TMX, NS, false>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        TPAMD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_w8_direct_kernel<DT, TMX, NS, true>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        configured_dev = dev;
+    }
+    p.tiles_m = (p.M + BM - 1) / BM;
+    p.tiles_n = (p.N + 255) / 256;
+    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
+    const int KT = p.K / BK;
+    p.kt_per_split = (KT + splits - 1) / splits;
+    p.splits = (KT + p.kt_per_split - 1) / p.kt_per_split;
+    TPAMD_REQUIRE(tiles * p.splits < (1ll << 31), "gemm: too many tiles");
+    GemmParams f = p;  // the finishing pass sees the 128 x 128 tiling
+    f.tiles_m = (p.M + 127) / 128;
+    f.tiles_n = (p.N + 127) / 128;
+    const int64_t tiles128 = static_cast<int64_t>(f.tiles_m) * f.tiles_n;
+    q.o_steps = (q.n_out + 31) / 32;
+    const size_t xo_bytes = static_cast<size_t>(p.M) * q.o_steps * 64, wo_bytes = static_cast<size_t>(p.N) * q.o_steps * 64;
+    const size_t part_bytes = p.splits > 1 ? static_cast<size_t>(p.splits) * tiles128 * 128 * 128 * sizeof(float) : 0;
+    if (xo_bytes + wo_bytes + part_bytes == 0) {
+        hipLaunchKernelGGL((gemm_w8_direct_kernel<DT, TMX, NS, false>), dim3(static_cast<unsigned>(tiles)), dim3(256), LDS, s, p, q);
+        TPAMD_HIP(hipGetLastError());
+        return TPAMD_OK;
+    }
+    std::lock_guard<std::mutex> hold(splitk_mutex(dev));  // the scratch buffer is ours until every launch below is enqueued
+    void *ws = nullptr;
+    if (int rc = splitk_scratch(dev, s, xo_bytes + wo_bytes + part_bytes, scratch_reserve(cus), &ws); rc != TPAMD_OK) return rc;
+    if (ws == nullptr) return TPAMD_ERR_UNSUPPORTED;
+    if (q.o_steps > 0) {
+        char *xo = static_cast<char *>(ws) + part_bytes, *wo = xo + xo_bytes;
+        q.xo = xo;
+        q.wo = wo;
+        const int64_t threads = (static_cast<int64_t>(p.M) + p.N) * q.o_steps * 4;
+        hipLaunchKernelGGL(w8_pack_outliers_kernel, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, s, p, q, xo, wo);
+        TPAMD_HIP(hipGetLastError());
+    }
+    if (p.splits == 1) {
+        hipLaunchKernelGGL((gemm_w8_direct_kernel<DT, TMX, NS, false>), dim3(static_cast<unsigned>(tiles)), dim3(256), LDS, s, p, q);
+        TPAMD_HIP(hipGetLastError());
+        return TPAMD_OK;
+    }
+    p.ws = f.ws = static_cast<float *>(ws);
+    hipLaunchKernelGGL((gemm_w8_direct_kernel<DT, TMX, NS, true>), dim3(static_cast<unsigned>(tiles * p.splits)), dim3(256), LDS, s, p, q);
+    TPAMD_HIP(hipGetLastError());
+    hipLaunchKernelGGL((splitk_finish_kernel<DT, MODE_LINEAR>), dim3(16, static_cast<unsigned>(tiles128)), dim3(256), 0, s, f, p.splits);
     TPAMD_HIP(hipGetLastError());
     return TPAMD_OK;
 }
@@ -1810,7 +2191,7 @@ int launch_direct(GemmParams p, int cus, int splits, hipStream_t s) {
             const size_t ws_bytes = static_cast<size_t>(p.splits) * tiles128 * 128 * 128 * sizeof(float);
             std::lock_guard<std::mutex> hold(splitk_mutex(dev));
             void *ws = nullptr;
-            const int rc = splitk_scratch(dev, s, ws_bytes, static_cast<size_t>(4) * cus * 128 * 128 * sizeof(float), &ws);
+            const int rc = splitk_scratch(dev, s, ws_bytes, scratch_reserve(cus), &ws);
             if (rc != TPAMD_OK) return rc;
             if (ws != nullptr) {
                 p.ws = f.ws = static_cast<float *>(ws);
@@ -1921,7 +2302,7 @@ int launch_direct128(GemmParams p, int cus, hipStream_t s) {
         // the scratch buffer is ours until both launches are enqueued
         std::lock_guard<std::mutex> hold(splitk_mutex(dev));
         void *ws = nullptr;
-        if (int rc = splitk_scratch(dev, s, ws_bytes, static_cast<size_t>(4) * cus * 128 * 128 * sizeof(float), &ws); rc != TPAMD_OK) return rc;
+        if (int rc = splitk_scratch(dev, s, ws_bytes, scratch_reserve(cus), &ws); rc != TPAMD_OK) return rc;
         if (ws != nullptr) {
             p.ws = static_cast<float *>(ws);
             const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(splits));
@@ -2046,8 +2427,40 @@ int gemm_dispatch(const void *x, const void *w, const void *w2, const void *bias
     return dtype == TPAMD_BF16 ? gemm_large<TPAMD_BF16>(p, swiglu, s) : gemm_large<TPAMD_F16>(p, swiglu, s);
 }
 
+// gemm_w8_direct_kernel steps K in tiles of 64 and addresses a tile with 32-bit byte offsets from its origin.
+bool w8_direct_ok(int64_t K, int64_t ldx, int64_t ldw) { return K % 64 == 0 && K >= 128 && ldx < (1ll << 22) && ldw < (1ll << 22); }
+
+// Rows per tile and K splits of gemm_w8_direct_kernel with the smallest predicted time (microseconds). The model is linear in
+// what the launches do, fitted (non-negative least squares on relative errors) to 1560 timings of 10 matrices at 65-2048 rows
+// with both tile heights and 1-16 splits inside a HIP graph: a fixed cost (launches, first tiles, epilogue, outlier columns), a
+// time per K tile and round of one block per CU (shorter where the round leaves CUs idle: the part clocks higher), and for a
+// split the second launch and the megabytes of partial tiles that are written and read back. Over that sweep the choices are
+// 0.7 % off the best one per shape in f16 and 0.8 % in bf16; examples at 1024 rows (256 rows / 128 rows per tile): 16384 x 8192
+// 228 / 251 us, 8192 x 16384 in two / one splits 249 / 237 us, 4096 x 4096 64 (four splits) / 52 us (two).
+void w8_tiling(int64_t M, int64_t N, int KT, int cus, int *rows, int *splits) {
+    double best = 1e30;
+    for (int r = 256; r >= 128; r -= 128) {
+        const double fixed = r == 256 ? 13.7 : 14.6, full = r == 256 ? 1.576 : 0.855;
+        const double idle[3] = {r == 256 ? 1.23 : 0.619, r == 256 ? 1.35 : 0.685, r == 256 ? 1.381 : 0.73};  // last round at most 1/2, 3/4, all full
+        const int64_t tiles = ((M + r - 1) / r) * ((N + 255) / 256);
+        const double part_mb = static_cast<double>((N + 127) / 128 * 128) * M * 4.0e-6;
+        for (int sp = 1; sp <= 16; ++sp) {
+            const int kt = (KT + sp - 1) / sp;
+            if (sp > 1 && (kt < 4 || tiles * sp > 2ll * cus || (KT + kt - 1) / kt != sp)) continue;
+            // the partial tiles have to fit the stream's buffer
+            if (sp > 1 && sp * ((M + 127) / 128) * ((N + 127) / 128) > 4ll * cus) break;
+            const int64_t units = tiles * sp, last = units % cus;
+            double t = fixed + static_cast<double>(units / cus) * kt * full;
+            if (last > 0) t += kt * (last * 2 <= cus ? idle[0] : last * 4 <= 3ll * cus ? idle[1] : idle[2]);
+            if (sp > 1) t += (r == 256 ? 12.0 + 0.245 * sp * part_mb : 3.1 + 0.345 * sp * part_mb);
+            if (t < best) { best = t; *rows = r; *splits = sp; }
+        }
+    }
+}
+
 // int8 weights above the weight-streaming kernels' row count. x, wq 16-byte aligned, K and ldw multiples of 16, ldx of 8
-// (checked by the caller); N and ldy multiples of 4 and y 8-byte aligned for the packed stores.
+// (checked by the caller); N and ldy multiples of 4 and y 8-byte aligned for the packed stores. gemm_w8_kernel is left with K
+// that is no multiple of 64, and with streams that have no scratch memory for the outlier columns.
 int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out,
                      const void *bias, void *y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout,
                      int64_t ldy, int dtype, int act, hipStream_t s) {
@@ -2060,14 +2473,24 @@ int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const voi
     p.ldx = ldx; p.ldw = ldw; p.ldy = ldy;
     p.act = act;
     W8Extra q{static_cast<const float *>(scale), static_cast<const int *>(outlier_idx), static_cast<const char *>(w_out),
-              static_cast<int>(n_out), ld_wout};
+              static_cast<int>(n_out), ld_wout, nullptr, nullptr, 0};
     int dev = 0, cus = 256;
     TPAMD_HIP(hipGetDevice(&dev));
     if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
-    const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
-    const bool big = tiles256 * 2 >= cus;
-    if (dtype == TPAMD_BF16) return big ? launch_gemm_w8<TPAMD_BF16, 256, 256, 2, 4>(p, q, s) : launch_gemm_w8<TPAMD_BF16, 128, 128, 2, 2>(p, q, s);
-    return big ? launch_gemm_w8<TPAMD_F16, 256, 256, 2, 4>(p, q, s) : launch_gemm_w8<TPAMD_F16, 128, 128, 2, 2>(p, q, s);
+    if (w8_direct_ok(K, ldx, ldw)) {
+        int rows = 128, splits = 1;
+        w8_tiling(M, N, static_cast<int>(K / 64), cus, &rows, &splits);
+        if (tuning().w8_tile != TUNE_UNSET && tuning().w8_tile > 0) rows = tuning().w8_tile;
+        if (tuning().w8_tile_splits != TUNE_UNSET) splits = tuning().w8_tile_splits;
+        auto run = [&](int sp) {
+            if (dtype == TPAMD_BF16) return rows == 256 ? launch_w8_direct<TPAMD_BF16, 16, 3>(p, q, cus, sp, s) : launch_w8_direct<TPAMD_BF16, 8, 4>(p, q, cus, sp, s);
+            return rows == 256 ? launch_w8_direct<TPAMD_F16, 16, 3>(p, q, cus, sp, s) : launch_w8_direct<TPAMD_F16, 8, 4>(p, q, cus, sp, s);
+        };
+        int rc = run(splits);
+        if (rc == TPAMD_ERR_UNSUPPORTED && splits > 1) rc = run(1);
+        if (rc != TPAMD_ERR_UNSUPPORTED) return rc;  // else no scratch memory for the outlier columns: the kernel that needs none
+    }
+    return dtype == TPAMD_BF16 ? launch_gemm_w8<TPAMD_BF16, 128, 128, 2, 2>(p, q, s) : launch_gemm_w8<TPAMD_F16, 128, 128, 2, 2>(p, q, s);
 }
 
 }  // namespace tpamd

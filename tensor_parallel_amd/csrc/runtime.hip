@@ -30,6 +30,8 @@ Tuning read_tuning() {
     t.skinny_pair = env_int("TPAMD_SKINNY_PAIR");
     t.skinny_resident = env_int("TPAMD_SKINNY_RESIDENT");
     t.w8_split = env_int("TPAMD_W8_SPLIT");
+    t.w8_tile = env_int("TPAMD_W8_TILE");
+    t.w8_tile_splits = env_int("TPAMD_W8_TILE_SPLITS");
     t.w8_cols = env_int("TPAMD_W8_COLS");
     t.skinny_xlds = env_int("TPAMD_SKINNY_XLDS");
     t.skinny_max_m = env_int("TPAMD_SKINNY_MAX_M");

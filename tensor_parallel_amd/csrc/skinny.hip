@@ -1534,7 +1534,7 @@ int launch_w8_split(const SkinnyParams &p, hipStream_t s, bool *done) {
     const size_t need = static_cast<size_t>(splits) * p.M * p.N * sizeof(float);
     std::lock_guard<std::mutex> hold(splitk_mutex(dev));
     void *ws = nullptr;
-    const int rc = splitk_scratch(dev, s, need, static_cast<size_t>(4) * cus * 128 * 128 * sizeof(float), &ws);
+    const int rc = splitk_scratch(dev, s, need, scratch_reserve(cus), &ws);
     if (rc != TPAMD_OK) return rc;
     if (ws == nullptr) return TPAMD_OK;
     float *part = static_cast<float *>(ws);
@@ -1585,7 +1585,7 @@ int launch_w8_cols_mt(const SkinnyParams &p, int dev, int cus, hipStream_t s, bo
     const size_t need = static_cast<size_t>(planes) * p.M * p.N * sizeof(float);
     std::lock_guard<std::mutex> hold(splitk_mutex(dev));
     void *ws = nullptr;
-    const int rc = splitk_scratch(dev, s, need, static_cast<size_t>(4) * cus * 128 * 128 * sizeof(float), &ws);
+    const int rc = splitk_scratch(dev, s, need, scratch_reserve(cus), &ws);
     if (rc != TPAMD_OK) return rc;
     if (ws == nullptr) return TPAMD_OK;
     float *part = static_cast<float *>(ws);

@@ -286,3 +286,37 @@ def test_falcon_mlp_shard_full_shape_at_prefill():
     down = _native.linear_w8(up, dev(wq2), dev(s2), dev(c2.astype(np.int32)), dev(o2, torch.float16))
     want_down = oq.linear_w8_f64(up[rows].cpu().float().numpy(), wq2, s2, c2, o2)
     torch.testing.assert_close(down[rows].double().cpu(), torch.from_numpy(want_down), rtol=2e-2, atol=2e-2 * float(np.abs(want_down).std()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("M,N,K,n_out,splits", [
+    (65, 64, 128, 0, 1),       # two K tiles (fewer than LDS stages), part of one column tile, no outliers
+    (127, 260, 192, 32, 1),    # one row short of a tile, 4 columns in the second tile, a full step of outlier columns
+    (129, 252, 320, 33, 1),    # one row over, outliers one over a step
+    (256, 256, 512, 1, 2),     # whole tiles, two K ranges
+    (257, 516, 832, 41, 3),    # ragged everywhere, 13 K tiles over 3 ranges (5 + 5 + 3)
+    (300, 128, 1024, 256, 4),  # the most outlier columns
+])
+def test_tiled_kernel_edges(tune, dtype, rows, M, N, K, n_out, splits):
+    """The tiled int8 kernel with both tile heights forced, unsplit and with K ranges, at the edges of its tiles."""
+    tune("TPAMD_W8_TILE", rows)
+    tune("TPAMD_W8_TILE_SPLITS", splits)
+    x, wq, scale, cols, w_out = make_case(M, N, K, n_out, dtype, seed=M + N)
+    wide = torch.zeros(M, K + 8, dtype=dtype)
+    wide[:, :K] = x
+    args = (wide.to(DEV)[:, :K], torch.from_numpy(wq).to(DEV), torch.from_numpy(scale).to(DEV),
+            torch.from_numpy(cols.astype(np.int32)).to(DEV) if n_out else None,
+            torch.from_numpy(w_out).to(dtype).to(DEV) if n_out else None)
+    bias = (torch.randn(N, generator=torch.Generator().manual_seed(5)) * 0.1).to(dtype)
+    want = oq.linear_w8_f64(x.float().numpy(), wq, scale, cols, w_out)
+    atol = RTOL_TILED * 0.02 * math.sqrt(K + 400 * n_out)
+    torch.testing.assert_close(_native.linear_w8(*args).double().cpu(), torch.from_numpy(want), rtol=RTOL_TILED, atol=atol)
+    want = torch.nn.functional.gelu(torch.from_numpy(want) + bias.double())
+    got = _native.linear_w8(*args, bias=bias.to(DEV), act=_native.ACT_GELU)
+    torch.testing.assert_close(got.double().cpu(), want, rtol=RTOL_TILED, atol=atol)
+
+
+# exact products of 16-bit and 8-bit values summed in fp32 and rounded once to 8 (bf16) bits or more: half a unit is 2^-9, and four
+# times that leaves room for the order of the sums
+RTOL_TILED = 8e-3
