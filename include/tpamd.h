@@ -300,6 +300,13 @@ int tpamd_attention_decode_rope_devpos(const void *q_dev, const void *k_dev, con
 int tpamd_rms_norm(const void *x_dev, const void *w_dev, void *y_dev, int64_t rows, int64_t D, int64_t ldx, int64_t ldy, float eps,
                    int dtype, void *stream);
 
+/* The cos / sin tables of a rotary embedding (the module's forward on position_ids, run by src/tensor_parallel/wrapper.py:69-72):
+ * cos[b][s][i] = cos[b][s][i + half] = round(cosf(position * inv_freq[i]) * scaling), sin likewise, for positions
+ * pos_dev[b * pos_b + s * pos_s] (int64; pos_b = 0: one row for every sequence). Angles and scaling in fp32; inv_freq [half] in
+ * `freq_dtype`, the tables [B, S, 2 * half], contiguous, in `dtype`. */
+int tpamd_rope_tables(const void *inv_freq_dev, int freq_dtype, const int64_t *pos_dev, int64_t pos_b, int64_t pos_s, int64_t B,
+                      int64_t S, int64_t half, float scaling, void *cos_dev, void *sin_dev, int dtype, void *stream);
+
 /* Weight-only int8 shard Linear with fp16/bf16 outlier columns:
  *   y[m,n] = act( scale[n] * sum_k x[m,k]*wq[n,k]  +  sum_j x[m,outlier_idx[j]] * w_out[n,j]  + bias[n] )
  * wq is int8 [N,K] (zero in the outlier columns), scale fp32 [N], outlier_idx int32 [n_out] (sorted,

@@ -37,6 +37,7 @@ EXPORTS = (
     "tpamd_linear_w8",
     "tpamd_attention",
     "tpamd_rms_norm",
+    "tpamd_rope_tables",
     "tpamd_rope_append",
     "tpamd_attention_decode_rope",
     "tpamd_attention_decode_rope_devpos",
@@ -130,6 +131,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_rope_append.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, c.POINTER(i64), ci, vp]
     lib.tpamd_rms_norm.restype = ci
     lib.tpamd_rms_norm.argtypes = [vp, vp, vp, i64, i64, i64, i64, c.c_float, ci, vp]
+    lib.tpamd_rope_tables.restype = ci
+    lib.tpamd_rope_tables.argtypes = [vp, ci, vp, i64, i64, i64, i64, i64, c.c_float, vp, vp, ci, vp]
     lib.tpamd_linear_w8.restype = ci
     lib.tpamd_linear_w8.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, i64, i64, i64, i64, i64, i64, i64, ci, ci, vp]
 
@@ -509,6 +512,27 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional
             "tpamd_attention",
         )
     return out
+
+
+def rope_tables(inv_freq: torch.Tensor, position_ids: torch.Tensor, scaling: float, dtype: torch.dtype) -> tuple:
+    """(cos, sin) [B, S, 2 * len(inv_freq)] of the angles position * inv_freq, scaled, in `dtype` (arithmetic in fp32)."""
+    require_device(position_ids, "rope_tables")
+    if inv_freq.dim() != 1 or position_ids.dim() != 2 or position_ids.dtype != torch.int64 or inv_freq.device != position_ids.device:
+        raise ValueError(f"rope_tables: inv_freq {tuple(inv_freq.shape)} and int64 position_ids [B, S] on one device are needed, got "
+                         f"{tuple(position_ids.shape)} {position_ids.dtype}")
+    B, S = position_ids.shape
+    half = inv_freq.shape[0]
+    inv_freq = inv_freq.contiguous()
+    cos = torch.empty((B, S, 2 * half), dtype=dtype, device=position_ids.device)
+    sin = torch.empty_like(cos)
+    with _on_device(position_ids.device):
+        _check(
+            lib().tpamd_rope_tables(inv_freq.data_ptr(), dtype_code(inv_freq.dtype), position_ids.data_ptr(), position_ids.stride(0),
+                                    position_ids.stride(1), B, S, half, float(scaling), cos.data_ptr(), sin.data_ptr(), dtype_code(dtype),
+                                    ctypes.c_void_p(current_stream_ptr(position_ids.device))),
+            "tpamd_rope_tables",
+        )
+    return cos, sin
 
 
 def rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,

@@ -62,6 +62,35 @@ __global__ __launch_bounds__(256) void rope_append_kernel(RopeParams p) {
     *reinterpret_cast<uint4 *>(dst + at + half_bytes) = rot8<DT>(x2, c2, x1, s2, 1.0f);
 }
 
+// cos / sin tables of a forward: out[row][i] = out[row][i + half] = round(f(position[row] * inv_freq[i]) * scaling). One thread per
+// (row, frequency), latency-bound: the module's own forward is ten launches (two casts, a K = 1 matrix product, a
+// concatenation, and three passes for each table), 2 us each in a recorded decode step.
+template <int DT>
+__global__ __launch_bounds__(256) void rope_tables_kernel(const char *inv_freq, int freq_dtype, const int64_t *pos, int64_t pos_b, int64_t pos_s, int S,
+                                                          int half, float scaling, char *cos_out, char *sin_out, int64_t n) {
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (e >= n) return;
+    const int64_t row = e / half;
+    const int i = static_cast<int>(e - row * half);
+    const int64_t b = row / S;
+    float f;
+    if (freq_dtype == TPAMD_F32) f = reinterpret_cast<const float *>(inv_freq)[i];
+    else if (freq_dtype == TPAMD_BF16) f = bf16_to_f32(reinterpret_cast<const uint16_t *>(inv_freq)[i]);
+    else f = f16_to_f32(reinterpret_cast<const uint16_t *>(inv_freq)[i]);
+    const float angle = f * static_cast<float>(pos[b * pos_b + (row - b * S) * pos_s]);
+    const float c = cosf(angle) * scaling, s = sinf(angle) * scaling;
+    const int64_t at = row * 2 * half + i;
+    if constexpr (DT == TPAMD_F32) {
+        float *co = reinterpret_cast<float *>(cos_out), *so = reinterpret_cast<float *>(sin_out);
+        co[at] = co[at + half] = c;
+        so[at] = so[at + half] = s;
+    } else {
+        uint16_t *co = reinterpret_cast<uint16_t *>(cos_out), *so = reinterpret_cast<uint16_t *>(sin_out);
+        co[at] = co[at + half] = f32_to_half<DT>(c);
+        so[at] = so[at + half] = f32_to_half<DT>(s);
+    }
+}
+
 }  // namespace
 }  // namespace tpamd
 
@@ -109,6 +138,28 @@ extern "C" int tpamd_rope_append(const void *q_dev, const void *k_dev, const voi
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == TPAMD_BF16) hipLaunchKernelGGL(rope_append_kernel<TPAMD_BF16>, grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL(rope_append_kernel<TPAMD_F16>, grid, dim3(256), 0, s, p);
+    TPAMD_HIP(hipGetLastError());
+    return TPAMD_OK;
+}
+
+extern "C" int tpamd_rope_tables(const void *inv_freq_dev, int freq_dtype, const int64_t *pos_dev, int64_t pos_b, int64_t pos_s, int64_t B, int64_t S,
+                                 int64_t half, float scaling, void *cos_dev, void *sin_dev, int dtype, void *stream) {
+    const char *who = "tpamd_rope_tables";
+    TPAMD_REQUIRE((dtype == TPAMD_BF16 || dtype == TPAMD_F16 || dtype == TPAMD_F32) &&
+                      (freq_dtype == TPAMD_BF16 || freq_dtype == TPAMD_F16 || freq_dtype == TPAMD_F32), "%s: unknown dtype", who);
+    TPAMD_REQUIRE(B >= 0 && S >= 0 && half >= 0 && B < (1ll << 31) && S < (1ll << 31) && half < (1ll << 31), "%s: bad dimension", who);
+    if (B == 0 || S == 0 || half == 0) return TPAMD_OK;
+    TPAMD_REQUIRE(inv_freq_dev && pos_dev && cos_dev && sin_dev, "%s: null pointer", who);
+    TPAMD_REQUIRE(B * S < (1ll << 31) && B * S * half < (1ll << 38), "%s: too many positions for one launch", who);
+    const int64_t n = B * S * half;
+    const dim3 grid(static_cast<unsigned>((n + 255) / 256));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const char *f = static_cast<const char *>(inv_freq_dev);
+    char *c = static_cast<char *>(cos_dev), *si = static_cast<char *>(sin_dev);
+    const int Si = static_cast<int>(S), h = static_cast<int>(half);
+    if (dtype == TPAMD_BF16) hipLaunchKernelGGL(rope_tables_kernel<TPAMD_BF16>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, n);
+    else if (dtype == TPAMD_F16) hipLaunchKernelGGL(rope_tables_kernel<TPAMD_F16>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, n);
+    else hipLaunchKernelGGL(rope_tables_kernel<TPAMD_F32>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, n);
     TPAMD_HIP(hipGetLastError());
     return TPAMD_OK;
 }

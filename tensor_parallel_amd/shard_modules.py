@@ -8,7 +8,8 @@ blocks with `gate_proj` / `up_proj` / `down_proj` children get a fused gate/up f
 src/tensor_parallel/slicing_configs.py:192-201) is re-classed to a subclass whose forward is the same `tpamd_linear`:
 its weight keeps the [in, out] shape every rule and state dict expects but is stored with the `in` axis fastest, which
 is the kernel's [out, in] layout; the transposing mover writes it that way while slicing, or once at the first forward.
-transformers' `LlamaRMSNorm`, which every rank computes on whole rows, becomes one launch (`tpamd_rms_norm`) in the same way.
+transformers' `LlamaRMSNorm` and the rotary tables of Llama and Falcon, which every rank computes whole, become one launch
+each (`tpamd_rms_norm`, `tpamd_rope_tables`) in the same way.
 
 Inference only: the kernels have no backward; asking for one raises. Autocast is not applied by these modules: the
 input must already have the weight's dtype (a mismatch raises TypeError where `nn.Linear` under autocast would cast).
@@ -118,14 +119,30 @@ def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
     return _guard(_native.rms_norm(hidden_states.detach(), w.detach(), self.variance_epsilon), hidden_states, w)
 
 
-_rms_norm_classes: dict = {}
+def is_rotary_tables(module: nn.Module) -> bool:
+    """The rotary embedding modules of transformers' Llama and Falcon: cos / sin of position * inv_freq, the halves repeated."""
+    return type(module).__name__ in ("LlamaRotaryEmbedding", "FalconRotaryEmbedding") and type(module).__module__.split(".")[0] == "transformers" and \
+        isinstance(getattr(module, "inv_freq", None), torch.Tensor) and hasattr(module, "attention_scaling") and hasattr(module, "rope_type")
 
 
-def _shard_rms_norm_class(base: type) -> type:
-    cls = _rms_norm_classes.get(base)
+def _rotary_tables_forward(self, x: torch.Tensor, position_ids: torch.Tensor):
+    f, kind = self.inv_freq, self.rope_type
+    # rope types that change their frequencies with the length of the sequence keep the module's own forward
+    if (position_ids.dtype != torch.int64 or position_ids.dim() != 2 or position_ids.device.type != "cuda" or f.device != position_ids.device or f.dim() != 1
+            or not isinstance(kind, str) or "dynamic" in kind or kind == "longrope"
+            or x.dtype not in (torch.bfloat16, torch.float16, torch.float32) or f.dtype not in (torch.bfloat16, torch.float16, torch.float32)):
+        return type(self).__mro__[1].forward(self, x, position_ids)
+    return _native.rope_tables(f, position_ids, self.attention_scaling, x.dtype)
+
+
+_fused_classes: dict = {}
+
+
+def _fused_class(base: type, forward, doc: str) -> type:
+    """Subclass of a module's own class with another forward (isinstance checks keep working)."""
+    cls = _fused_classes.get((base, forward))
     if cls is None:
-        cls = _rms_norm_classes[base] = type("Shard" + base.__name__, (base,), {"forward": _rms_norm_forward, "__doc__": "The base class with "
-                                                                             "its forward as one launch (`tpamd_rms_norm`)."})
+        cls = _fused_classes[base, forward] = type("Shard" + base.__name__, (base,), {"forward": forward, "__doc__": doc})
     return cls
 
 
@@ -191,7 +208,9 @@ def install_shard_kernels(shard: nn.Module) -> None:
         elif is_conv1d(module) and type(module).__name__ == "Conv1D" and module.weight.dim() == 2 and module.weight.dtype in (torch.bfloat16, torch.float16, torch.float32):
             module.__class__ = _shard_conv1d_class(type(module))
         elif is_rms_norm(module) and module.weight.dtype in (torch.bfloat16, torch.float16, torch.float32):
-            module.__class__ = _shard_rms_norm_class(type(module))
+            module.__class__ = _fused_class(type(module), _rms_norm_forward, "The base class with its forward as one launch (`tpamd_rms_norm`).")
+        elif is_rotary_tables(module):
+            module.__class__ = _fused_class(type(module), _rotary_tables_forward, "The base class with its forward as one launch (`tpamd_rope_tables`).")
     for module in shard.modules():
         if is_gated_silu_mlp(module):
             module.forward = types.MethodType(_gated_mlp_first_forward, module)

@@ -113,3 +113,49 @@ def test_argument_errors():
     cache32 = torch.zeros(B, Hkv, 4, 32, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(RuntimeError):
         _native.rope_append(q32, q32, q32, c32, c32, cache32, cache32.clone(), 0)  # head_dim 32: no kernel
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("freq_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,S,half,one_row", [(1, 1, 32, False), (3, 5, 64, False), (2, 257, 64, True), (1, 3, 5, False)])
+def test_rope_tables(dtype, freq_dtype, B, S, half, one_row):
+    """`tpamd_rope_tables` against the angles in fp32 and their cosines in fp64. fp32 cosines are good to 2 units of 2^-24 (of values up
+    to 1); rounding to a dtype with p significant bits (bf16 8, f16 11, fp32 24) adds at most 2^-p of the result, the scaling 2^-24."""
+    g = torch.Generator().manual_seed(S)
+    pos = torch.randint(0, 8192, (1 if one_row else B, S), generator=g)
+    pos = pos.expand(B, S)
+    inv = (1.0 / 10000.0 ** (torch.arange(half) / half)).to(freq_dtype)
+    cos, sin = _native.rope_tables(inv.to(DEV), pos.to(DEV) if not one_row else pos[:1].to(DEV).expand(B, S), 1.25, dtype)
+    angle = (pos[..., None].float() * inv.float()).double()
+    angle = torch.cat([angle, angle], -1)
+    unit = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dtype]
+    for got, want in ((cos, angle.cos() * 1.25), (sin, angle.sin() * 1.25)):
+        assert got.shape == (B, S, 2 * half) and got.dtype == dtype
+        torch.testing.assert_close(got.double().cpu(), want, rtol=unit + 2.0 ** -24, atol=1.25 * 2.0 ** -22)
+    with pytest.raises(ValueError):
+        _native.rope_tables(inv.to(DEV), pos.to(DEV).int(), 1.0, dtype)
+
+
+@pytest.mark.parametrize("family", ["llama", "falcon"])
+def test_rotary_modules_of_the_shards_use_the_tables(family):
+    import transformers as tf
+
+    import tensor_parallel_amd as tp
+
+    torch.manual_seed(0)
+    if family == "llama":
+        model = tf.LlamaModel(tf.LlamaConfig(vocab_size=96, hidden_size=64, intermediate_size=128, num_hidden_layers=1, num_attention_heads=4,
+                                             num_key_value_heads=2)).to(torch.bfloat16).eval()
+    else:
+        model = tf.FalconModel(tf.FalconConfig(vocab_size=96, hidden_size=256, num_hidden_layers=1, num_attention_heads=4, num_kv_heads=2,
+                                               new_decoder_architecture=True, alibi=False, bias=False)).to(torch.bfloat16).eval()
+    pos = torch.randint(0, 2048, (2, 7))
+    x = torch.zeros(2, 7, 8, dtype=torch.bfloat16)
+    want = model.rotary_emb(x, pos)
+    split = tp.tensor_parallel(model, [DEV, DEV])
+    mine = [m for m in split.modules() if type(m).__name__ in ("ShardLlamaRotaryEmbedding", "ShardFalconRotaryEmbedding")]
+    assert len(mine) == 2
+    for g, w in zip(mine[1](x.to(DEV), pos.to(DEV)), want):  # the host's fp32 cosines may round the other way on a boundary
+        torch.testing.assert_close(g.cpu().float(), w.float(), rtol=2.0 ** -7, atol=1e-6)
+    mine[0].rope_type = "dynamic"  # frequencies that change with the length: the module's own forward
+    assert mine[0](x.to(DEV), pos.to(DEV))[0].shape == want[0].shape
