@@ -14,7 +14,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 OUT_DIR = PKG / "_lib"
 LIB = OUT_DIR / "libtpamd.so"
-SOURCES = ["api.hip", "runtime.hip", "noalloc.hip", "slice.hip", "reduce.hip", "gemm.hip", "skinny.hip", "attention.hip", "rope.hip", "norm.hip"]
+SOURCES = ["api.hip", "runtime.hip", "noalloc.hip", "slice.hip", "reduce.hip", "gemm.hip", "gemm_mid.hip", "skinny.hip", "attention.hip", "rope.hip", "norm.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -45,7 +45,7 @@ def _compile(src: str, verbose: bool) -> Path:
     return obj
 
 
-def build(verbose: bool = True, jobs: int = 4) -> Path:
+def build(verbose: bool = True, jobs: int = 8) -> Path:
     """Compile every HIP source and link the shared library. Always recompiles."""
     OUT_DIR.mkdir(exist_ok=True)
     with ThreadPoolExecutor(max_workers=jobs) as pool:

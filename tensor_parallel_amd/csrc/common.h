@@ -40,7 +40,7 @@ struct Tuning {
     int gemm_w4;             // TPAMD_GEMM_W4: 0 = the 8-wavefront 256 x 256 kernel instead of the 4-wavefront one
     int gemm_splitk;         // TPAMD_GEMM_SPLITK: K splits of the 128 x 128 tiling
     int gemm_splitk256;      // TPAMD_GEMM_SPLITK256: K splits of the 256 x 256 tiling
-    int gemm_tile;           // TPAMD_GEMM_TILE: 256 or 128
+    int gemm_tile;           // TPAMD_GEMM_TILE: 256, 128, or 1000 * rows + columns of a gemm_mid_kernel tile (128192, ...)
     int gemm_stages;         // TPAMD_GEMM_STAGES: 4 / 2 = the K-split 128 x 128 kernel with four / two LDS stages (unset: four when there is at most one block per CU)
     int gemm_part_x;         // TPAMD_GEMM_PART_X: 0 = the K-split 128 x 128 kernel loads whole x tiles also for M <= 64
     int skinny_cg;           // TPAMD_SKINNY_CG: column groups per block (1, 2, 4)

@@ -14,7 +14,7 @@
 //                       kernel elsewhere (TPAMD_GEMM_W4=0 selects it).
 //   gemm_kernel         any K (multiple of 8) and the 128x128 tiling for small problems, v_mfma_f32_32x32x16; next
 //                       K tile prefetched into registers while the current one is multiplied.
-#include "common.h"
+#include "gemm_tile.h"
 
 #include <stdlib.h>
 #include <mutex>
@@ -24,31 +24,7 @@
 namespace tpamd {
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
-
-enum { MODE_LINEAR = 0, MODE_SWIGLU = 1 };
-
-struct GemmParams {
-    const char *x;
-    const char *w;   // linear: weight; swiglu: gate weight
-    const char *w2;  // swiglu: up weight
-    const char *bias;
-    const char *addend;  // linear: added to the rounded result (another rank's partial sum), or NULL
-    char *y;
-    int M, N, K;
-    int64_t ldx, ldw, ldy, ldadd;  // elements
-    int act;
-    int tiles_m, tiles_n;
-    float *ws;          // split-K: partial tiles, [split][tile][128 x rows][128 w rows] fp32
-    int kt_per_split;   // split-K: K tiles (of 64) per split
-    int splits;         // split-K of the 256 x 256 kernel: work units = tiles x splits
-};
-
-constexpr int BK = 64;            // K elements per stage (128 bytes of a row)
-constexpr int LDS_ROW = 144;      // bytes per staged row: 128 + 16 pad, conflict-free for b128 reads
-constexpr int GROUP_M = 4;        // tile rows per L2 reuse group
 
 template <int DT>
 __device__ __forceinline__ f32x16 mfma32(uint4 a, uint4 b, f32x16 c) {
@@ -56,22 +32,6 @@ __device__ __forceinline__ f32x16 mfma32(uint4 a, uint4 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     else
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
-// Hardware spreads consecutive workgroup ids round-robin over the 8 XCDs (each with its own L2).
-// Give every XCD one contiguous range of logical tile ids, then walk tiles in groups of GROUP_M tile
-// rows so that the blocks resident on an XCD at one time share x and w tiles.
-__device__ __forceinline__ void tile_of_block(int bid, int nblocks, int tiles_m, int tiles_n, int &tm, int &tn) {
-    const int per = nblocks >> 3, rem = nblocks & 7;
-    const int xcd = bid & 7, in_xcd = bid >> 3;
-    const int logical = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + in_xcd;
-    const int group_size = GROUP_M * tiles_n;
-    const int g = logical / group_size;
-    const int first_m = g * GROUP_M;
-    const int gm = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
-    const int in_group = logical - g * group_size;
-    tm = first_m + in_group % gm;
-    tn = in_group / gm;
 }
 
 // Epilogue shared by both kernels. D[n_local][m_local]: lane -> m_local = l32, register i -> n_local = 8*(i/4) + 4*lhi + i%4,
@@ -261,223 +221,6 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_kernel(GemmParams 
     }
 
     epilogue<DT, MODE, BM, BN, WAVES_M, WAVES_N>(p, acc, m0, n0, wm, wn, l32, lhi);
-}
-
-typedef __attribute__((address_space(3))) void lds_void;
-// Global->LDS load through a buffer descriptor: each lane's 16 bytes land at lds_base + lane * 16 (lds_base must be
-// the same for the whole wavefront); address = descriptor base + per-lane 32-bit offset + wavefront-uniform
-// offset, range-checked by the hardware against the descriptor's extent (a load beyond it returns zeros).
-// No per-lane 64-bit address arithmetic is needed to step through K.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, uint32_t extent_bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, static_cast<int>(extent_bytes), 0x00020000);
-}
-__device__ __forceinline__ void buffer_load16_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_t lane_off, uint32_t uniform_off, void *lds_base) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void *)lds_base, 16, static_cast<int>(lane_off), static_cast<int>(uniform_off), 0, 0);
-}
-// Fragment read that the compiler does not see as an LDS access. With ordinary loads it waits for every
-// in-flight global->LDS load before each LDS read (it cannot tell that they go to the other stage), which
-// serialises the pipeline; this way the waits are the counted ones written out in the main loop.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-template <int OFFSET>
-__device__ __forceinline__ u32x4 lds_read16(uint32_t lds_addr) {
-    static_assert(OFFSET >= 0 && OFFSET < 65536, "ds offset field is 16 bits");
-    u32x4 v;
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(lds_addr), "n"(OFFSET));
-    return v;
-}
-__device__ __forceinline__ uint32_t lds_addr_of(const void *p) {
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char *)p));
-}
-// All of this wavefront's loads and LDS accesses done, then the workgroup barrier. The memory clobber keeps
-// the compiler from moving LDS accesses across it.
-__device__ __forceinline__ void drain_and_barrier() {
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-template <int DT>
-__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-    if constexpr (DT == TPAMD_BF16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
-// Four consecutive output columns n..n+3 of one row, from fp32 sums to the packed 16-bit store value.
-// linear: v = bias/activation of g; swiglu: g = gate sums, u = up sums.
-template <int DT, int MODE>
-__device__ __forceinline__ uint2 finish4(const GemmParams &p, const float (&g)[4], const float (&u)[4], int n, const char *add_row = nullptr) {
-    uint2 o;
-    if constexpr (MODE == MODE_SWIGLU) {
-        // gate and up products rounded to the tensor dtype, then silu and the product each rounded again
-        uint32_t out[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t g2 = pack2_half<DT>(g[2 * j], g[2 * j + 1]);
-            const uint32_t u2 = pack2_half<DT>(u[2 * j], u[2 * j + 1]);
-            const uint32_t s2 = pack2_half<DT>(silu_f32(lo_half_to_f32<DT>(g2)), silu_f32(hi_half_to_f32<DT>(g2)));
-            out[j] = pack2_half<DT>(lo_half_to_f32<DT>(s2) * lo_half_to_f32<DT>(u2), hi_half_to_f32<DT>(s2) * hi_half_to_f32<DT>(u2));
-        }
-        o.x = out[0];
-        o.y = out[1];
-    } else {
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = g[j];
-        if (p.bias) {
-            const uint2 braw = *reinterpret_cast<const uint2 *>(p.bias + static_cast<int64_t>(n) * 2);
-            v[0] += lo_half_to_f32<DT>(braw.x); v[1] += hi_half_to_f32<DT>(braw.x);
-            v[2] += lo_half_to_f32<DT>(braw.y); v[3] += hi_half_to_f32<DT>(braw.y);
-        }
-        if (p.act == TPAMD_ACT_GELU) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = gelu_erf(v[j]);
-        }
-        o.x = pack2_half<DT>(v[0], v[1]);
-        o.y = pack2_half<DT>(v[2], v[3]);
-        if (add_row != nullptr) {  // the row of p.addend this output row belongs to
-            const uint2 araw = *reinterpret_cast<const uint2 *>(add_row + static_cast<int64_t>(n) * 2);
-            o.x = add_packed2<DT>(o.x, araw.x);
-            o.y = add_packed2<DT>(o.y, araw.y);
-        }
-    }
-    return o;
-}
-
-// Epilogue of the direct kernels. With w as the first MFMA operand a lane holds D[n = 4*(lane/16) + i][m = lane%16],
-// i = 0..3: four consecutive output columns of one output row, one 8-byte store.
-// acc[a][b]: a = 16-row tile of x (TMX per wavefront), b = 16-row tile of w (4 per wavefront; swiglu: 2 gate + 2 up).
-template <int DT, int MODE, int TMX>
-__device__ __forceinline__ void epilogue16(const GemmParams &p, f32x4 (&acc)[TMX][4], int m_wave, int n_wave, int l16, int lq) {
-#pragma unroll
-    for (int a = 0; a < TMX; ++a) {
-        const int m = m_wave + a * 16 + l16;
-        if (m >= p.M) continue;
-        char *yrow = p.y + static_cast<int64_t>(m) * p.ldy * 2;
-#pragma unroll
-        for (int b = 0; b < (MODE == MODE_SWIGLU ? 2 : 4); ++b) {
-            const int n = n_wave + b * 16 + lq * 4;
-            if (n >= p.N) continue;  // N is a multiple of 4: the group of 4 is all in or all out
-            float g[4], u[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                g[j] = acc[a][b][j];
-                u[j] = MODE == MODE_SWIGLU ? acc[a][(b + 2) & 3][j] : 0.f;
-            }
-            const char *add_row = MODE == MODE_LINEAR && p.addend != nullptr ? p.addend + static_cast<int64_t>(m) * p.ldadd * 2 : nullptr;
-            *reinterpret_cast<uint2 *>(yrow + static_cast<int64_t>(n) * 2) = finish4<DT, MODE>(p, g, u, n, add_row);
-        }
-    }
-}
-
-// Epilogue of the 4-wavefront kernels. A lane holds 4 consecutive columns of one row per accumulator tile; stored like
-// that, an instruction would write 32-byte pieces of 16 rows. Instead the packed results of 16 rows x (16 * GB)
-// columns go through a wavefront-private LDS slab (16 rows, EP_PITCH bytes apart) and leave as 16 bytes per lane:
-// whole 128-byte lines, 8 rows per store instruction, when GB = 4.
-// acc[a][b]: a = 16-row tile of x, b = 16-row tile of w. The wavefront's columns are GROUPS runs of 16 * GB; gated pair:
-// tile b holds gate sums and tile b + UP the up sums of the same columns. wide: 16-byte stores are aligned.
-constexpr int EP_PITCH = 144;
-// ADD: the addend (p.addend, not NULL) of the 16 rows after next is requested while the current 16 rows are converted and
-// stored, one set of registers ahead: asked for at the point of use, every piece is a full memory round trip with
-// nothing else to do on this SIMD (10 us on the 4096 x 4096 x 5504 down projection).
-template <int DT, int MODE, bool GELU, int TMX, int NBT, int GROUPS, int GB, int UP, bool ADD = false>
-__device__ __forceinline__ void staged_epilogue(const GemmParams &p, f32x4 (&acc)[TMX][NBT], char *slab, int m_wave, int n_wave,
-                                                int lane, bool wide) {
-    static_assert(GB == 4 || GB == 2, "64 or 32 columns per slab");
-    const int l16 = lane & 15, lq = lane >> 4;
-    uint2 braw[GROUPS * GB];
-    if constexpr (MODE == MODE_LINEAR) {
-#pragma unroll
-        for (int b = 0; b < GROUPS * GB; ++b) {
-            const int n = n_wave + b * 16 + lq * 4;
-            braw[b] = p.bias != nullptr && n < p.N ? *reinterpret_cast<const uint2 *>(p.bias + static_cast<int64_t>(n) * 2) : make_uint2(0, 0);
-        }
-    }
-    constexpr int LANES_PER_ROW = GB * 2;            // 16 bytes per lane
-    constexpr int ROWS_PER_READ = 64 / LANES_PER_ROW;
-    constexpr int READS = 16 / ROWS_PER_READ;
-    const int rd_row = lane / LANES_PER_ROW, rd_col = lane % LANES_PER_ROW;
-    uint2 addv[2][ADD ? GROUPS * READS : 1][2];
-    auto request_addend = [&](int a) {
-#pragma unroll
-        for (int gq = 0; gq < GROUPS; ++gq)
-#pragma unroll
-            for (int h = 0; h < READS; ++h) {
-                const int m = m_wave + a * 16 + h * ROWS_PER_READ + rd_row;
-                const int n = n_wave + gq * (16 * GB) + rd_col * 8;
-                const bool in = m < p.M && n < p.N;
-                const char *ap = p.addend + (in ? (static_cast<int64_t>(m) * p.ldadd + n) * 2 : 0);
-                addv[a & 1][gq * READS + h][0] = *reinterpret_cast<const uint2 *>(ap);
-                addv[a & 1][gq * READS + h][1] = in && n + 8 <= p.N ? *reinterpret_cast<const uint2 *>(ap + 8) : make_uint2(0, 0);
-            }
-    };
-    if constexpr (ADD) request_addend(0);
-#pragma unroll
-    for (int a = 0; a < TMX; ++a) {
-        if constexpr (ADD) {
-            if (a + 1 < TMX) request_addend(a + 1);
-        }
-#pragma unroll
-        for (int gq = 0; gq < GROUPS; ++gq) {
-#pragma unroll
-            for (int bb = 0; bb < GB; ++bb) {
-                const int b = gq * GB + bb;
-                uint2 o;
-                if constexpr (MODE == MODE_SWIGLU) {
-                    float gsum[4], usum[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        gsum[j] = acc[a][b][j];
-                        usum[j] = acc[a][b + UP][j];
-                    }
-                    o = finish4<DT, MODE>(p, gsum, usum, 0);
-                } else {
-                    float v[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = acc[a][b][j];
-                    v[0] += lo_half_to_f32<DT>(braw[b].x); v[1] += hi_half_to_f32<DT>(braw[b].x);
-                    v[2] += lo_half_to_f32<DT>(braw[b].y); v[3] += hi_half_to_f32<DT>(braw[b].y);
-                    if constexpr (GELU) {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) v[j] = gelu_erf(v[j]);
-                    }
-                    o.x = pack2_half<DT>(v[0], v[1]);
-                    o.y = pack2_half<DT>(v[2], v[3]);
-                }
-                *reinterpret_cast<uint2 *>(slab + l16 * EP_PITCH + bb * 32 + lq * 8) = o;
-            }
-            __builtin_amdgcn_wave_barrier();
-            asm volatile("" ::: "memory");
-#pragma unroll
-            for (int h = 0; h < READS; ++h) {
-                const int row = h * ROWS_PER_READ + rd_row;
-                const uint4 vs = *reinterpret_cast<const uint4 *>(slab + row * EP_PITCH + rd_col * 16);
-                const int m = m_wave + a * 16 + row;
-                const int n = n_wave + gq * (16 * GB) + rd_col * 8;
-                if (m >= p.M || n >= p.N) continue;
-                char *dst = p.y + (static_cast<int64_t>(m) * p.ldy + n) * 2;
-                uint4 v = vs;
-                if constexpr (ADD) {
-                    {  // the lane that stores 8 outputs adds the same 8 elements of the addend
-                        const uint2 a0 = addv[a & 1][gq * READS + h][0], a1 = addv[a & 1][gq * READS + h][1];
-                        v.x = add_packed2<DT>(v.x, a0.x); v.y = add_packed2<DT>(v.y, a0.y);
-                        v.z = add_packed2<DT>(v.z, a1.x); v.w = add_packed2<DT>(v.w, a1.y);
-                    }
-                }
-                if (n + 8 <= p.N) {
-                    if (wide) *reinterpret_cast<uint4 *>(dst) = v;
-                    else {
-                        *reinterpret_cast<uint2 *>(dst) = make_uint2(v.x, v.y);
-                        *reinterpret_cast<uint2 *>(dst + 8) = make_uint2(v.z, v.w);
-                    }
-                } else {
-                    *reinterpret_cast<uint2 *>(dst) = make_uint2(v.x, v.y);  // N is a multiple of 4
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-            asm volatile("" ::: "memory");
-        }
-    }
 }
 
 // gemm_direct_kernel: 256 x 256 x 64 tiles, 8 wavefronts (2 x 4, 128 x-rows by 64 w-rows each), 2 LDS stages.
@@ -1511,26 +1254,6 @@ int launch_gemm_w8(GemmParams p, const W8Extra &q, hipStream_t s) {
 // w8_pack_outliers_kernel, zeros up to a multiple of 32) follow in steps of 32 into the same accumulators.
 // SPLIT: unit u is tile u % tiles, K range u / tiles; the scaled sums (range 0: with the outlier columns) go to p.ws as
 // 128 x 128 tiles for splitk_finish_kernel.
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void unrolled(F &&f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        unrolled<N, I + 1>(f);
-    }
-}
-
-// All but the YOUNGER last LDS reads of this wavefront have arrived, the named registers among them (the reads are asm
-// statements: the waits are ours).
-template <int YOUNGER>
-__device__ __forceinline__ void reads_landed(u32x4 &r) {
-    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "n"(YOUNGER) : "memory");
-}
-__device__ __forceinline__ void already_landed(u32x4 &r) { asm volatile("" : "+v"(r)); }  // uses stay behind the wait in front of this
-template <int YOUNGER>
-__device__ __forceinline__ void reads_landed(u32x4 (&r)[4]) {
-    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "n"(YOUNGER) : "memory");
-}
-
 // cvt_i8x4 one instruction at a time: step<0>, step<1>, ... step<OPS - 1> leave the four converted weights in lo, hi. The
 // conversions take their byte through the sub-dword selects (f16: 4 instructions where bias, permute and subtract took 5; bf16: 6
 // where they took 11).
@@ -2332,6 +2055,32 @@ int launch_direct128(GemmParams p, int cus, hipStream_t s) {
     return TPAMD_OK;
 }
 
+// Predicted time (microseconds) of gemm_mid_kernel on the best of its tiles, and that tile: a launch, rounds of one block per CU, each with
+// a fixed cost (first tiles, epilogue) and a time per K tile, shorter where the last round leaves CUs idle (the part clocks higher).
+// Non-negative least squares on relative errors over 237 shapes (9 matrices at 128-8192 rows, 90 random ones), each tile forced and timed
+// inside a HIP graph. There the choice among these tiles, the 256 x 256 and the 128 x 128 tiling is 1.7 % off the best one (geometric
+// mean; 6.4 % without these tiles) and nowhere slower than without them. Examples: the pair 5504 x 4096 at 512 rows 64 -> 51 us (128 x 192; two
+// K splits of 256 x 256 before) and at 645 rows 84 -> 60 us, 4096 x 5504 at 2103 rows 105 -> 78 us (192 x 192; 144 tiles of 256 x 256 before).
+struct MidTile { int tmx, tnx; double launch, round, full, idle[3]; };  // idle: last round at most 1/2, at most 3/4, more of the CUs
+constexpr MidTile MID_TILES[2][4] = {
+    {{4, 6, 0.5, 5.0, 0.643, {0.537, 0.588, 0.693}}, {4, 8, 0.4, 5.8, 0.827, {0.663, 0.740, 0.820}},
+     {6, 6, 2.6, 6.7, 0.858, {0.635, 0.714, 0.789}}, {6, 8, 0.1, 5.4, 1.226, {0.922, 0.977, 1.211}}},
+    {{4, 6, 0.7, 3.2, 0.642, {0.661, 0.715, 0.688}}, {4, 8, 1.4, 3.6, 0.837, {0.756, 0.808, 0.832}},
+     {6, 6, 0.0, 7.2, 0.827, {0.727, 0.755, 0.820}}, {6, 8, 1.3, 2.0, 1.223, {1.099, 1.088, 1.233}}},
+};
+
+inline double estimate_mid(int64_t M, int64_t N, int KT, int cus, bool swiglu, int *tmx, int *tnx) {
+    double best = 1e30;
+    for (const MidTile &t : MID_TILES[swiglu ? 1 : 0]) {
+        const int64_t bm = 32 * t.tmx, bn = (swiglu ? 16 : 32) * t.tnx;
+        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn), full = tiles / cus, last = tiles % cus;
+        double us = t.launch + full * (t.round + KT * t.full);
+        if (last > 0) us += t.round + KT * t.idle[last * 2 <= cus ? 0 : last * 4 <= 3ll * cus ? 1 : 2];
+        if (us < best) { best = us; *tmx = t.tmx; *tnx = t.tnx; }
+    }
+    return best;
+}
+
 // Prefill-sized dispatch; called by linear.hip once M is above the skinny range.
 template <int DT>
 int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
@@ -2372,6 +2121,15 @@ int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
     const int64_t small_tiles_m = (p.M + 127) / 128;
     const double t128 = estimate128(small_tiles, small_tiles_m, small_tiles / small_tiles_m, KT, cus,
                                     static_cast<double>(p.M) / (small_tiles_m * 128.0), swiglu, &unused_splits, &unused_deep);
+    if (direct_ok) {
+        int tmx = 0, tnx = 0;
+        if (tuning().gemm_tile != TUNE_UNSET) {
+            if (tuning().gemm_tile > 1000) { tmx = tuning().gemm_tile / 32000; tnx = tuning().gemm_tile % 1000 / 32; }
+        } else if (estimate_mid(p.M, p.N, KT, cus, swiglu, &tmx, &tnx) >= (t256 < t128 ? t256 : t128)) {
+            tmx = 0;
+        }
+        if (tmx > 0) return gemm_mid(p, DT, swiglu, tmx, tnx, s);
+    }
     const bool big = tuning().gemm_tile != TUNE_UNSET ? tuning().gemm_tile == 256 : t256 < t128;
     if (direct_ok) {
         if (big) return swiglu ? launch_direct<DT, MODE_SWIGLU>(p, cus, splits256, s) : launch_direct<DT, MODE_LINEAR>(p, cus, splits256, s);

@@ -274,6 +274,28 @@ def test_256_tiles_on_ragged_shapes(dtype, M, N, K, waves, tune):
     check_half(got, F.linear(strided.float().cpu(), w.float()), K)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(17, 8, 64), (129, 196, 128), (193, 260, 192), (384, 512, 256), (700, 1028, 320)])
+@pytest.mark.parametrize("tile", [128192, 128256, 192192, 192256])
+def test_mid_tiles_on_ragged_shapes(dtype, M, N, K, tile, tune):
+    """The tiles of gemm_mid_kernel (forced; by default the cost model decides): fewer K tiles than LDS stages, rows and columns past the end,
+    whole tiles, output rows on 8-byte boundaries, bias and GELU, an addend, the gated pair, and a strided x."""
+    tune("TPAMD_GEMM_TILE", tile)
+    x, w, b, a = rnd((M, K), 1, 1.0, dtype), rnd((N, K), 0, 0.02, dtype), rnd((N,), 2, 0.1, dtype), rnd((M, N), 7, 1.0, dtype)
+    xd, wd, bd = x.to(DEV), w.to(DEV), b.to(DEV)
+    check_half(_native.linear(xd, wd, bd, act=_native.ACT_GELU), F.gelu(F.linear(x.float(), w.float(), b.float())), K)
+    plain = _native.linear(xd, wd, bd)
+    check_half(plain, F.linear(x.float(), w.float(), b.float()), K)
+    assert torch.equal(_native.linear(xd, wd, bd, addend=a.to(DEV)).cpu(), plain.cpu() + a)
+    w2 = rnd((N, K), 5, 0.02, dtype)
+    h = _native.swiglu_up(xd, wd, w2.to(DEV))
+    sigma = (0.02 * math.sqrt(K)) ** 2
+    torch.testing.assert_close(h.float().cpu(), ofw.gated_mlp_hidden(x.float(), w.float(), w2.float()), rtol=RTOL_HALF, atol=RTOL_HALF * sigma)
+    wide = torch.empty((M, 2 * K), dtype=dtype, device=DEV)
+    wide[:, K:] = xd
+    assert torch.equal(_native.linear(wide[:, K:], wd, bd), plain)
+
+
 def test_both_256_tile_kernels_agree_bit_for_bit(tune):
     """Same products added in the same order: the 4- and the 8-wavefront kernel must give identical results, also
     when a block walks through several tiles (3 x 96 = 288 tiles on at most 256 blocks)."""
