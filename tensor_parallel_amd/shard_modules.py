@@ -114,9 +114,12 @@ def is_rms_norm(module: nn.Module) -> bool:
 
 def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
     w = self.weight
-    if hidden_states.dtype != w.dtype or hidden_states.device.type != "cuda":  # a promoting norm: the module's own forward
+    # a promoting norm, and one that a backward pass may go through (its gradients were there before any Linear's), keep the module's
+    # own forward
+    if (hidden_states.dtype != w.dtype or hidden_states.device.type != "cuda" or hidden_states.device != w.device
+            or torch.is_grad_enabled() and (hidden_states.requires_grad or w.requires_grad)):
         return type(self).__mro__[1].forward(self, hidden_states)
-    return _guard(_native.rms_norm(hidden_states.detach(), w.detach(), self.variance_epsilon), hidden_states, w)
+    return _native.rms_norm(hidden_states.detach(), w.detach(), self.variance_epsilon)
 
 
 def is_rotary_tables(module: nn.Module) -> bool:
@@ -139,11 +142,20 @@ _fused_classes: dict = {}
 
 
 def _fused_class(base: type, forward, doc: str) -> type:
-    """Subclass of a module's own class with another forward (isinstance checks keep working)."""
+    """Subclass of a module's own class with another forward (isinstance checks keep working, and so does pickling)."""
     cls = _fused_classes.get((base, forward))
     if cls is None:
-        cls = _fused_classes[base, forward] = type("Shard" + base.__name__, (base,), {"forward": forward, "__doc__": doc})
+        def reduce_ex(self, protocol):  # the class is made here and has no name to be found by: pickle what makes it
+            return (_new_fused, (base, forward, doc), *super(cls, self).__reduce_ex__(protocol)[2:])
+
+        cls = type("Shard" + base.__name__, (base,), {"forward": forward, "__doc__": doc, "__reduce_ex__": reduce_ex})
+        cls = _fused_classes.setdefault((base, forward), cls)
     return cls
+
+
+def _new_fused(base: type, forward, doc: str) -> nn.Module:
+    cls = _fused_class(base, forward, doc)
+    return cls.__new__(cls)
 
 
 def _is_silu(fn) -> bool:

@@ -60,3 +60,22 @@ def test_shards_of_a_llama_use_it():
         torch.testing.assert_close(norms[0](x.to(DEV)).float().cpu(), model.model.norm(x.to(model.device)).float().cpu(), rtol=2e-2, atol=1e-2)
         promoted = norms[0](x.float().to(DEV))  # another dtype than the weight's: the module's own forward
     assert promoted.dtype == torch.float32
+
+
+def test_a_norm_that_a_backward_pass_goes_through_keeps_its_gradients():
+    import transformers as tf
+
+    import tensor_parallel_amd as tp
+
+    torch.manual_seed(0)
+    cfg = tf.LlamaConfig(vocab_size=96, hidden_size=64, intermediate_size=128, num_hidden_layers=1, num_attention_heads=4, num_key_value_heads=2)
+    norm = next(m for m in tp.tensor_parallel(tf.LlamaModel(cfg).eval(), [DEV, DEV]).modules() if type(m).__name__ == "ShardLlamaRMSNorm")
+    x = torch.randn(5, 64, device=DEV, requires_grad=True)
+    w = norm.weight.requires_grad_(True)
+    c = torch.randn(5, 64, device=DEV)  # not the norm itself: the length of a normalised row does not depend on x, its gradient is rounding noise
+    gx, gw = torch.autograd.grad((norm(x) * c).sum(), (x, w))
+    x64, w64 = x.detach().double().requires_grad_(True), w.detach().double().requires_grad_(True)
+    want = torch.autograd.grad((w64 * x64 * torch.rsqrt(x64.square().mean(-1, keepdim=True) + norm.variance_epsilon) * c).sum(), (x64, w64))
+    # fp32 sums of 64 terms: 64 * 2^-24 of the largest of them
+    for g, r in zip((gx, gw), want):
+        torch.testing.assert_close(g.double(), r, rtol=1e-5, atol=64 * 2.0 ** -24 * r.abs().max().item())

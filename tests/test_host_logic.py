@@ -796,3 +796,23 @@ def test_graph_capture_needs_a_hip_device():
     module = torch.nn.Linear(8, 8)
     with pytest.raises(ValueError, match="one HIP device"):
         tp.graphs.capture(module, torch.zeros(2, 8))
+
+
+def test_shards_with_fused_modules_can_be_pickled_and_copied():
+    """The classes made for a shard's norms and rotary tables have no importable name; saving a whole model goes on working."""
+    import copy
+    import pickle
+
+    import torch
+    import transformers as tf
+
+    from tensor_parallel_amd import shard_modules as sm
+
+    torch.manual_seed(0)
+    model = tf.LlamaModel(tf.LlamaConfig(vocab_size=32, hidden_size=32, intermediate_size=48, num_hidden_layers=1, num_attention_heads=2)).eval()
+    sm.install_shard_kernels(model)
+    for other in (pickle.loads(pickle.dumps(model)), copy.deepcopy(model)):
+        assert type(other.norm) is type(model.norm) and type(other.rotary_emb) is type(model.rotary_emb)
+        x = torch.randn(2, 32)
+        with torch.no_grad():
+            assert torch.equal(other.norm(x), model.norm(x))
