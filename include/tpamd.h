@@ -307,6 +307,10 @@ int tpamd_rms_norm(const void *x_dev, const void *w_dev, void *y_dev, int64_t ro
 int tpamd_rope_tables(const void *inv_freq_dev, int freq_dtype, const int64_t *pos_dev, int64_t pos_b, int64_t pos_s, int64_t B,
                       int64_t S, int64_t half, float scaling, void *cos_dev, void *sin_dev, int dtype, void *stream);
 
+/* Causal mask of `rows` queries on `cols` keys, a byte each (1: seen): mask[i][j] = (kv_offset + j <= *q_offset_dev + i), the
+ * queries' first position (int64) read from the device, mask [rows, cols] contiguous. */
+int tpamd_causal_mask(const int64_t *q_offset_dev, int64_t kv_offset, int64_t rows, int64_t cols, void *mask_dev, void *stream);
+
 /* Weight-only int8 shard Linear with fp16/bf16 outlier columns:
  *   y[m,n] = act( scale[n] * sum_k x[m,k]*wq[n,k]  +  sum_j x[m,outlier_idx[j]] * w_out[n,j]  + bias[n] )
  * wq is int8 [N,K] (zero in the outlier columns), scale fp32 [N], outlier_idx int32 [n_out] (sorted,

@@ -38,6 +38,7 @@ EXPORTS = (
     "tpamd_attention",
     "tpamd_rms_norm",
     "tpamd_rope_tables",
+    "tpamd_causal_mask",
     "tpamd_rope_append",
     "tpamd_attention_decode_rope",
     "tpamd_attention_decode_rope_devpos",
@@ -133,6 +134,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_rms_norm.argtypes = [vp, vp, vp, i64, i64, i64, i64, c.c_float, ci, vp]
     lib.tpamd_rope_tables.restype = ci
     lib.tpamd_rope_tables.argtypes = [vp, ci, vp, i64, i64, i64, i64, i64, c.c_float, vp, vp, ci, vp]
+    lib.tpamd_causal_mask.restype = ci
+    lib.tpamd_causal_mask.argtypes = [vp, i64, i64, i64, vp, vp]
     lib.tpamd_linear_w8.restype = ci
     lib.tpamd_linear_w8.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, i64, i64, i64, i64, i64, i64, i64, ci, ci, vp]
 
@@ -533,6 +536,21 @@ def rope_tables(inv_freq: torch.Tensor, position_ids: torch.Tensor, scaling: flo
             "tpamd_rope_tables",
         )
     return cos, sin
+
+
+def causal_mask(q_offset: torch.Tensor, kv_offset: int, q_length: int, kv_length: int) -> torch.Tensor:
+    """Boolean [1, 1, q_length, kv_length]: kv_offset + j <= q_offset + i, the offset of the queries (one int64) read on the device."""
+    require_device(q_offset, "causal_mask")
+    if q_offset.dtype != torch.int64 or q_offset.numel() != 1:
+        raise ValueError(f"causal_mask: q_offset must be one int64, got {tuple(q_offset.shape)} {q_offset.dtype}")
+    out = torch.empty((1, 1, q_length, kv_length), dtype=torch.bool, device=q_offset.device)
+    with _on_device(q_offset.device):
+        _check(
+            lib().tpamd_causal_mask(q_offset.data_ptr(), kv_offset, q_length, kv_length, out.data_ptr(),
+                                    ctypes.c_void_p(current_stream_ptr(q_offset.device))),
+            "tpamd_causal_mask",
+        )
+    return out
 
 
 def rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,

@@ -49,14 +49,29 @@ def attention_forward(module: torch.nn.Module, query: torch.Tensor, key: torch.T
     return out, None
 
 
+def attention_mask_of(*args, **kwargs) -> Optional[torch.Tensor]:
+    """transformers' `sdpa_mask`, the same result with one launch where a decode step on a static cache asks for it: the plain causal
+    mask, no padding, no right to skip it, the position of the first query a number on the device. All else goes to `sdpa_mask`."""
+    from transformers.masking_utils import causal_mask_function, sdpa_mask
+
+    q_offset, q_length, kv_length, kv_offset = (kwargs.get(n) for n in ("q_offset", "q_length", "kv_length", "kv_offset"))
+    if (args or kwargs.get("mask_function") is not causal_mask_function or kwargs.get("allow_is_causal_skip", True)
+            or kwargs.get("allow_is_bidirectional_skip", False) or kwargs.get("attention_mask") is not None or kwargs.get("use_vmap", False)
+            or type(q_offset) is not torch.Tensor or q_offset.device.type != "cuda" or q_offset.dtype != torch.int64 or q_offset.dim() > 1
+            or q_offset.numel() != 1 or torch.device(kwargs.get("device", "cpu")) != q_offset.device
+            or not all(type(n) is int for n in (q_length, kv_length, kv_offset, kwargs.get("batch_size")))
+            or torch.compiler.is_compiling() or torch.jit.is_tracing()):
+        return sdpa_mask(*args, **kwargs)
+    return _native.causal_mask(q_offset, kv_offset, q_length, kv_length).expand(kwargs["batch_size"], -1, q_length, kv_length)
+
+
 def register() -> str:
     """Adds "tpamd" to transformers' attention (and mask) registries; returns the name."""
     from transformers import AttentionInterface, AttentionMaskInterface
-    from transformers.masking_utils import sdpa_mask
 
     AttentionInterface.register(IMPLEMENTATION_NAME, attention_forward)
     # mask construction as for sdpa: a purely causal mask is skipped (None reaches attention_forward)
-    AttentionMaskInterface.register(IMPLEMENTATION_NAME, sdpa_mask)
+    AttentionMaskInterface.register(IMPLEMENTATION_NAME, attention_mask_of)
     return IMPLEMENTATION_NAME
 
 

@@ -226,3 +226,20 @@ def test_llama_with_the_registered_attention_implementation():
     with torch.no_grad():
         tp_logits = model_tp(input_ids=ids, use_cache=False).logits
     torch.testing.assert_close(tp_logits.float(), ref.logits.float(), rtol=RTOL, atol=3 * RTOL * scale)
+
+
+@pytest.mark.parametrize("batch,q_length,kv_length,offset", [(1, 1, 1, 0), (2, 1, 256, 255), (3, 1, 257, 100), (1, 1, 4160, 4159), (2, 7, 33, 20), (1, 300, 513, 5)])
+def test_mask_of_a_static_cache(batch, q_length, kv_length, offset):
+    """The one-launch mask is the mask transformers builds, for the forms it takes and (through transformers) those it does not."""
+    from transformers.masking_utils import causal_mask_function, sdpa_mask
+
+    from tensor_parallel_amd.attention import attention_mask_of
+
+    dev = torch.device("cuda", 0)
+    for kv_offset in (0, 3):
+        for q_offset in (torch.tensor(offset, device=dev), torch.tensor([offset], device=dev), torch.tensor(offset, device=dev, dtype=torch.int32), offset):
+            for padding in (None, torch.rand(batch, kv_length + kv_offset, device=dev) > 0.3):
+                form = dict(batch_size=batch, q_length=q_length, kv_length=kv_length, q_offset=q_offset, kv_offset=kv_offset, attention_mask=padding,
+                            mask_function=causal_mask_function, allow_is_causal_skip=False, use_vmap=False, device=dev, dtype=torch.bfloat16, config=None)
+                want, got = sdpa_mask(**form), attention_mask_of(**form)
+                assert got.dtype == want.dtype and got.stride() == want.stride() and torch.equal(got, want), (kv_offset, q_offset, padding is None)
