@@ -307,6 +307,11 @@ int tpamd_rms_norm(const void *x_dev, const void *w_dev, void *y_dev, int64_t ro
 int tpamd_rope_tables(const void *inv_freq_dev, int freq_dtype, const int64_t *pos_dev, int64_t pos_b, int64_t pos_s, int64_t B,
                       int64_t S, int64_t half, float scaling, void *cos_dev, void *sin_dev, int dtype, void *stream);
 
+/* The norm of a sum: sum = r + x (rounded to the dtype), y = the RMS norm of sum as tpamd_rms_norm computes it. x [rows, D] with leading
+ * dimension ldx, r with ldr, sum and y with ldy; sum and y overlap neither each other nor an input. */
+int tpamd_add_rms_norm(const void *x_dev, const void *r_dev, const void *w_dev, void *sum_dev, void *y_dev, int64_t rows, int64_t D,
+                       int64_t ldx, int64_t ldr, int64_t ldy, float eps, int dtype, void *stream);
+
 /* Causal mask of `rows` queries on `cols` keys, a byte each (1: seen): mask[i][j] = (kv_offset + j <= *q_offset_dev + i), the
  * queries' first position (int64) read from the device, mask [rows, cols] contiguous. */
 int tpamd_causal_mask(const int64_t *q_offset_dev, int64_t kv_offset, int64_t rows, int64_t cols, void *mask_dev, void *stream);

@@ -37,6 +37,7 @@ EXPORTS = (
     "tpamd_linear_w8",
     "tpamd_attention",
     "tpamd_rms_norm",
+    "tpamd_add_rms_norm",
     "tpamd_rope_tables",
     "tpamd_causal_mask",
     "tpamd_rope_append",
@@ -132,6 +133,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_rope_append.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, c.POINTER(i64), ci, vp]
     lib.tpamd_rms_norm.restype = ci
     lib.tpamd_rms_norm.argtypes = [vp, vp, vp, i64, i64, i64, i64, c.c_float, ci, vp]
+    lib.tpamd_add_rms_norm.restype = ci
+    lib.tpamd_add_rms_norm.argtypes = [vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, c.c_float, ci, vp]
     lib.tpamd_rope_tables.restype = ci
     lib.tpamd_rope_tables.argtypes = [vp, ci, vp, i64, i64, i64, i64, i64, c.c_float, vp, vp, ci, vp]
     lib.tpamd_causal_mask.restype = ci
@@ -483,6 +486,27 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
             "tpamd_rms_norm",
         )
     return y.view(x.shape)
+
+
+def add_rms_norm(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float) -> tuple:
+    """(r + x, the RMS norm of that sum) of two tensors of one shape, dtype and device; arithmetic as in `rms_norm`."""
+    require_device(x, "add_rms_norm")
+    if (r.shape != x.shape or r.dtype != x.dtype or r.device != x.device or w.dtype != x.dtype or w.device != x.device or w.dim() != 1 or x.dim() == 0
+            or x.shape[-1] != w.shape[0]):
+        raise ValueError(f"add_rms_norm: r {tuple(r.shape)} {r.dtype} on {r.device}, x {tuple(x.shape)} {x.dtype} on {x.device} and w {tuple(w.shape)} "
+                         f"{w.dtype} on {w.device} do not fit")
+    x2, r2 = _as_2d(x), _as_2d(r)
+    w = w.contiguous()
+    rows, D = x2.shape
+    total = torch.empty((rows, D), dtype=x.dtype, device=x.device)
+    y = torch.empty_like(total)
+    with _on_device(x.device):
+        _check(
+            lib().tpamd_add_rms_norm(x2.data_ptr(), r2.data_ptr(), w.data_ptr(), total.data_ptr(), y.data_ptr(), rows, D, _ld(x2), _ld(r2), D,
+                                     float(eps), dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device))),
+            "tpamd_add_rms_norm",
+        )
+    return total.view(x.shape), y.view(x.shape)
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None, causal: bool = True,

@@ -9,7 +9,8 @@ src/tensor_parallel/slicing_configs.py:192-201) is re-classed to a subclass whos
 its weight keeps the [in, out] shape every rule and state dict expects but is stored with the `in` axis fastest, which
 is the kernel's [out, in] layout; the transposing mover writes it that way while slicing, or once at the first forward.
 transformers' `LlamaRMSNorm` and the rotary tables of Llama and Falcon, which every rank computes whole, become one launch
-each (`tpamd_rms_norm`, `tpamd_rope_tables`) in the same way.
+each (`tpamd_rms_norm`, `tpamd_rope_tables`) in the same way; a Llama decoder layer has the addition behind its attention in the
+launch of its second norm (`tpamd_add_rms_norm`).
 
 Inference only: the kernels have no backward; asking for one raises. Autocast is not applied by these modules: the
 input must already have the weight's dtype (a mismatch raises TypeError where `nn.Linear` under autocast would cast).
@@ -122,6 +123,36 @@ def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
     return _native.rms_norm(hidden_states.detach(), w.detach(), self.variance_epsilon)
 
 
+def is_llama_layer(module: nn.Module) -> bool:
+    """transformers' LlamaDecoderLayer as the fused forward below knows it: its forward touches its two norms, the attention and the
+    MLP in this order and nothing else, and takes these arguments."""
+    code = getattr(type(module).forward, "__code__", None)
+    return type(module).__name__ == "LlamaDecoderLayer" and type(module).__module__.split(".")[0] == "transformers" and code is not None and \
+        "forward" not in module.__dict__ and code.co_names == ("input_layernorm", "self_attn", "post_attention_layernorm", "mlp") and \
+        code.co_varnames == ("self", "hidden_states", *_LAYER_DEFAULTS, "kwargs", "residual", "_")
+
+
+_LAYER_DEFAULTS = {"attention_mask": None, "position_ids": None, "past_key_values": None, "use_cache": False, "position_embeddings": None}
+
+
+def _llama_layer_forward(self, hidden_states: torch.Tensor, *args, **kwargs) -> torch.Tensor:
+    """The layer's own forward with the addition behind the attention inside the second norm's launch."""
+    norm = self.post_attention_layernorm
+    hooks = torch.nn.modules.module
+    if (args or getattr(type(norm), "forward", None) is not _rms_norm_forward or "forward" in norm.__dict__ or _has_hooks(norm)
+            or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or torch.is_grad_enabled()):
+        return type(self).__mro__[1].forward(self, hidden_states, *args, **kwargs)
+    attended, _ = self.self_attn(hidden_states=self.input_layernorm(hidden_states), **{**_LAYER_DEFAULTS, **kwargs})
+    w = norm.weight
+    if (hidden_states.device.type == "cuda" and hidden_states.device == attended.device == w.device and hidden_states.dtype == attended.dtype == w.dtype
+            and hidden_states.shape == attended.shape):
+        total, normed = _native.add_rms_norm(hidden_states, attended, w, norm.variance_epsilon)
+    else:
+        total = hidden_states + attended
+        normed = norm(total)
+    return total + self.mlp(normed)
+
+
 def is_rotary_tables(module: nn.Module) -> bool:
     """The rotary embedding modules of transformers' Llama and Falcon: cos / sin of position * inv_freq, the halves repeated."""
     return type(module).__name__ in ("LlamaRotaryEmbedding", "FalconRotaryEmbedding") and type(module).__module__.split(".")[0] == "transformers" and \
@@ -221,6 +252,9 @@ def install_shard_kernels(shard: nn.Module) -> None:
             module.__class__ = _shard_conv1d_class(type(module))
         elif is_rms_norm(module) and module.weight.dtype in (torch.bfloat16, torch.float16, torch.float32):
             module.__class__ = _fused_class(type(module), _rms_norm_forward, "The base class with its forward as one launch (`tpamd_rms_norm`).")
+        elif is_llama_layer(module):
+            module.__class__ = _fused_class(type(module), _llama_layer_forward, "The base class with an addition and a norm as one launch (`tpamd_add_rms_norm`).")
+            module.__class__.__name__ = type(module).__mro__[1].__name__  # programs look decoder layers up by the name of their class
         elif is_rotary_tables(module):
             module.__class__ = _fused_class(type(module), _rotary_tables_forward, "The base class with its forward as one launch (`tpamd_rope_tables`).")
     for module in shard.modules():

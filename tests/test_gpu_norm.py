@@ -79,3 +79,45 @@ def test_a_norm_that_a_backward_pass_goes_through_keeps_its_gradients():
     # fp32 sums of 64 terms: 64 * 2^-24 of the largest of them
     for g, r in zip((gx, gw), want):
         torch.testing.assert_close(g.double(), r, rtol=1e-5, atol=64 * 2.0 ** -24 * r.abs().max().item())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,D", [(1, 8), (3, 512), (2, 520), (5, 2048), (2, 2056), (37, 4096), (2, 8192), (2, 16384), (2, 16392), (4, 100), (3, 7), (0, 64)])
+def test_add_rms_norm_is_the_sum_and_its_norm(dtype, rows, D):
+    """Bit for bit what torch's addition and `tpamd_rms_norm` give, also on strided and unaligned rows. The vector and the element-wise
+    kernel add their squares in different orders, so the norm of unaligned rows is compared with that of a sum that is unaligned too."""
+    g = torch.Generator().manual_seed(D)
+    x, r = ((torch.randn(rows, 2 * D + 16, generator=g) * 3).to(dtype).to(DEV) for _ in range(2))
+    w = (1 + 0.3 * torch.randn(D, generator=g)).to(dtype).to(DEV)
+    odd = torch.empty_like(x)[:, 1:D + 1]
+    for a, b in ((x[:, :D].contiguous(), r[:, :D].contiguous()), (x[:, 1:D + 1], r[:, :D]), (x[:, :D], r[:, 16:D + 16])):
+        total, y = _native.add_rms_norm(b, a, w, 1e-5)
+        want = b + a if a.data_ptr() % 16 == 0 else odd.copy_(b + a)
+        assert torch.equal(total, b + a) and torch.equal(y, _native.rms_norm(want, w, 1e-5))
+    with pytest.raises(ValueError):
+        _native.add_rms_norm(r[:, :D], x[:, :D].double(), w, 1e-5)
+
+
+def test_decoder_layer_with_the_addition_in_its_norm():
+    """The fused layer gives its own forward's bits, and leaves the work to it where a hook watches the norm."""
+    import transformers as tf
+
+    import tensor_parallel_amd as tp
+    from tensor_parallel_amd import shard_modules
+
+    torch.manual_seed(0)
+    cfg = tf.LlamaConfig(vocab_size=96, hidden_size=64, intermediate_size=128, num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2)
+    split = tp.tensor_parallel(tf.LlamaForCausalLM(cfg).to(torch.bfloat16).eval(), [DEV, DEV])
+    layers = [m for m in split.modules() if type(m).forward is shard_modules._llama_layer_forward]
+    assert len(layers) == 4 and all(type(m).__name__ == "LlamaDecoderLayer" for m in layers)
+    ids = torch.randint(0, 96, (3, 9), device=DEV)
+    seen = []
+    with torch.no_grad():
+        split(input_ids=ids)  # the first call settles which kernels the modules use
+        fused = split(input_ids=ids, output_hidden_states=True)
+        handles = [m.post_attention_layernorm.register_forward_hook(lambda mod, inp, out: seen.append(inp[0])) for m in layers]
+        own = split(input_ids=ids, output_hidden_states=True)
+        for h in handles:
+            h.remove()
+    assert len(seen) == 4 and torch.equal(fused.logits, own.logits)
+    assert all(torch.equal(a, b) for a, b in zip(fused.hidden_states, own.hidden_states))
