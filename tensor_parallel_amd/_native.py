@@ -201,6 +201,16 @@ def require_device(t: torch.Tensor, what: str) -> None:
         )
 
 
+def on_hip(t: torch.Tensor) -> bool:
+    return t.device.type == "cuda"
+
+
+def calls_are_followed() -> bool:
+    """Whether something follows the torch calls that are being made, and would miss a kernel launched in their place: a
+    forward-mode derivative level."""
+    return torch.autograd.forward_ad._current_level >= 0
+
+
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
