@@ -205,10 +205,15 @@ def on_hip(t: torch.Tensor) -> bool:
     return t.device.type == "cuda"
 
 
-def calls_are_followed() -> bool:
-    """Whether something follows the torch calls that are being made, and would miss a kernel launched in their place: a
-    forward-mode derivative level."""
-    return torch.autograd.forward_ad._current_level >= 0
+def plain_call(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel launched on these tensors' memory may stand in for torch calls on them: the tensors are torch's own, and nothing
+    follows the calls that would miss the kernel (forward-mode derivatives; vmap and the other functorch transforms, whose wrappers
+    have no memory; compilation and tracing; dispatch modes)."""
+    for t in tensors:
+        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
+            return False
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0)
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)

@@ -57,10 +57,9 @@ def attention_mask_of(*args, **kwargs) -> Optional[torch.Tensor]:
     q_offset, q_length, kv_length, kv_offset = (kwargs.get(n) for n in ("q_offset", "q_length", "kv_length", "kv_offset"))
     if (args or kwargs.get("mask_function") is not causal_mask_function or kwargs.get("allow_is_causal_skip", True)
             or kwargs.get("allow_is_bidirectional_skip", False) or kwargs.get("attention_mask") is not None or kwargs.get("use_vmap", False)
-            or type(q_offset) is not torch.Tensor or q_offset.device.type != "cuda" or q_offset.dtype != torch.int64 or q_offset.dim() > 1
+            or not _native.plain_call(q_offset) or not _native.on_hip(q_offset) or q_offset.dtype != torch.int64 or q_offset.dim() > 1
             or q_offset.numel() != 1 or torch.device(kwargs.get("device", "cpu")) != q_offset.device
-            or not all(type(n) is int for n in (q_length, kv_length, kv_offset, kwargs.get("batch_size")))
-            or torch.compiler.is_compiling() or torch.jit.is_tracing()):
+            or not all(type(n) is int for n in (q_length, kv_length, kv_offset, kwargs.get("batch_size")))):
         return sdpa_mask(*args, **kwargs)
     return _native.causal_mask(q_offset, kv_offset, q_length, kv_length).expand(kwargs["batch_size"], -1, q_length, kv_length)
 

@@ -117,7 +117,7 @@ def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
     w = self.weight
     # a promoting norm, and one that derivatives may go through in either mode (they were there before any Linear's), keep the module's
     # own forward
-    if (hidden_states.dtype != w.dtype or not _native.on_hip(hidden_states) or hidden_states.device != w.device or _native.calls_are_followed()
+    if (not _native.plain_call(hidden_states, w) or hidden_states.dtype != w.dtype or not _native.on_hip(hidden_states) or hidden_states.device != w.device
             or torch.is_grad_enabled() and (hidden_states.requires_grad or w.requires_grad)):
         return type(self).__mro__[1].forward(self, hidden_states)
     return _native.rms_norm(hidden_states.detach(), w.detach(), self.variance_epsilon)
@@ -140,11 +140,12 @@ def _llama_layer_forward(self, hidden_states: torch.Tensor, *args, **kwargs) -> 
     norm = self.post_attention_layernorm
     hooks = torch.nn.modules.module
     if (args or getattr(type(norm), "forward", None) is not _rms_norm_forward or "forward" in norm.__dict__ or _has_hooks(norm)
-            or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or torch.is_grad_enabled() or _native.calls_are_followed()):
+            or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or torch.is_grad_enabled()
+            or not _native.plain_call(hidden_states, norm.weight)):
         return type(self).__mro__[1].forward(self, hidden_states, *args, **kwargs)
     attended, _ = self.self_attn(hidden_states=self.input_layernorm(hidden_states), **{**_LAYER_DEFAULTS, **kwargs})
     w = norm.weight
-    if (_native.on_hip(hidden_states) and hidden_states.device == attended.device == w.device and hidden_states.dtype == attended.dtype == w.dtype
+    if (_native.plain_call(attended) and _native.on_hip(hidden_states) and hidden_states.device == attended.device == w.device and hidden_states.dtype == attended.dtype == w.dtype
             and hidden_states.shape == attended.shape):
         total, normed = _native.add_rms_norm(hidden_states, attended, w, norm.variance_epsilon)
     else:
@@ -162,8 +163,8 @@ def is_rotary_tables(module: nn.Module) -> bool:
 def _rotary_tables_forward(self, x: torch.Tensor, position_ids: torch.Tensor):
     f, kind = self.inv_freq, self.rope_type
     # rope types that change their frequencies with the length of the sequence keep the module's own forward
-    if (position_ids.dtype != torch.int64 or position_ids.dim() != 2 or not _native.on_hip(position_ids) or f.device != position_ids.device or f.dim() != 1
-            or not isinstance(kind, str) or "dynamic" in kind or kind == "longrope" or _native.calls_are_followed()
+    if (not _native.plain_call(x, position_ids, f) or position_ids.dtype != torch.int64 or position_ids.dim() != 2 or not _native.on_hip(position_ids) or f.device != position_ids.device or f.dim() != 1
+            or not isinstance(kind, str) or "dynamic" in kind or kind == "longrope"
             or x.dtype not in (torch.bfloat16, torch.float16, torch.float32) or f.dtype not in (torch.bfloat16, torch.float16, torch.float32)):
         return type(self).__mro__[1].forward(self, x, position_ids)
     return _native.rope_tables(f, position_ids, self.attention_scaling, x.dtype)

@@ -79,3 +79,61 @@ def test_forward_mode_derivatives_go_through(kernels):
         model.norm.weight = forward_ad.make_dual(weight, torch.ones(32))
         assert forward_ad.unpack_dual(model.norm(x)).tangent is not None
     assert not kernels
+
+
+class _Seen(torch.utils._python_dispatch.TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.calls = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.calls.append(func)
+        return func(*args, **(kwargs or {}))
+
+
+def test_what_follows_the_torch_calls_sees_the_modules_own(kernels):
+    """vmap, vmap over stacked weights, jvp, tracing, compilation, a dispatch mode and a tensor subclass: kernels on raw memory would raise or go unseen."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    own, model, x = llama(), sharded(), torch.randn(3, 5, 32)
+    position_ids = torch.arange(5)[None]
+    with torch.no_grad():
+        run_layer(model, x)
+        kernels.clear()
+        want = own.norm(x)
+        assert torch.equal(torch.func.vmap(model.norm)(x), want)
+        stacked = torch.stack([own.norm.weight, 2 * own.norm.weight])
+        many = torch.func.vmap(lambda w: torch.func.functional_call(model.norm, {"weight": w}, (x,)))(stacked)
+        assert torch.equal(many, torch.stack([want, 2 * want]))
+        assert torch.equal(torch.func.vmap(lambda r: run_layer(model, r[None])[0])(x), torch.func.vmap(lambda r: run_layer(own, r[None])[0])(x))
+        shifted = torch.func.vmap(lambda p: model.rotary_emb(x, p))(torch.stack([position_ids, position_ids + 7]))
+        assert torch.equal(shifted[0][1], own.rotary_emb(x, position_ids + 7)[0])
+        assert torch.equal(torch.func.jvp(model.norm, (x,), (x,))[1], torch.func.jvp(own.norm, (x,), (x,))[1])
+        for traced in (torch.jit.trace(model.norm, x, check_trace=False), make_fx(model.norm)(x), torch.fx.symbolic_trace(model.norm), torch.compile(model.norm, backend="eager", fullgraph=True)):
+            assert torch.equal(traced(x + 1), own.norm(x + 1))
+        assert torch.equal(make_fx(model.rotary_emb)(x, position_ids)(x, position_ids + 3)[0], own.rotary_emb(x, position_ids + 3)[0])
+        with _Seen() as seen:
+            assert torch.equal(model.norm(x), want)
+        assert len(seen.calls) > 3
+        assert torch.equal(model.norm(x.as_subclass(type("Sub", (torch.Tensor,), {}))), want)
+    assert not kernels
+
+
+def test_a_mask_inside_a_transform_is_transformers_own(monkeypatch):
+    from transformers.masking_utils import causal_mask_function, sdpa_mask
+
+    from tensor_parallel_amd.attention import attention_mask_of
+
+    asked = []
+    monkeypatch.setattr(_native, "on_hip", lambda t: True)
+    monkeypatch.setattr(_native, "causal_mask", lambda q_offset, kv_offset, rows, cols: asked.append(rows) or (
+        torch.arange(cols) + kv_offset <= torch.arange(rows)[:, None] + q_offset)[None, None])
+
+    def mask(build, q_offset):
+        return build(batch_size=2, q_length=3, kv_length=9, q_offset=q_offset, kv_offset=0, attention_mask=None, mask_function=causal_mask_function,
+                     allow_is_causal_skip=False, use_vmap=False, device=torch.device("cpu"), dtype=torch.float32, config=None)
+
+    offsets = torch.tensor([2, 5])
+    assert torch.equal(mask(attention_mask_of, offsets[0]), mask(sdpa_mask, offsets[0])) and asked == [3]
+    assert torch.equal(torch.func.vmap(lambda o: mask(attention_mask_of, o))(offsets), torch.stack([mask(sdpa_mask, o) for o in offsets]))
+    assert asked == [3]
