@@ -107,29 +107,41 @@ def _shard_conv1d_class(base: type) -> type:
     return cls
 
 
+def _stock_forward(cls: type, names: tuple, variables: tuple) -> bool:
+    """Whether the class's forward is the one its own module in transformers defines, decorated by nobody but torch and transformers, and
+    known here by the names that it looks up and its arguments and locals: a forward that a program has put in its place is not stood in for."""
+    f = getattr(cls, "forward", None)
+    while True:
+        if getattr(f, "__code__", None) is None or f.__globals__.get("__name__", "").split(".")[0] not in ("torch", "transformers"):
+            return False
+        if not hasattr(f, "__wrapped__"):
+            break
+        f = f.__wrapped__
+    return f.__globals__["__name__"] == cls.__module__ and f.__qualname__ == f"{cls.__qualname__}.forward" and \
+        f.__code__.co_names == names and f.__code__.co_varnames == variables
+
+
 def is_rms_norm(module: nn.Module) -> bool:
     """transformers' LlamaRMSNorm: a weight over the last axis and `variance_epsilon`, statistics in fp32."""
-    return type(module).__name__ == "LlamaRMSNorm" and type(module).__module__.split(".")[0] == "transformers" and \
+    return type(module).__name__ == "LlamaRMSNorm" and _takes_stand_in(type(module), _rms_norm_forward) and \
         isinstance(getattr(module, "weight", None), torch.Tensor) and module.weight.dim() == 1 and hasattr(module, "variance_epsilon")
 
 
 def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
-    w = self.weight
-    # a promoting norm, and one that derivatives may go through in either mode (they were there before any Linear's), keep the module's
-    # own forward
-    if (not _native.plain_call(hidden_states, w) or hidden_states.dtype != w.dtype or not _native.on_hip(hidden_states) or hidden_states.device != w.device
+    w, own = self.weight, self._tp_base.forward
+    # a norm whose class has been given another forward since, a promoting norm, and one that derivatives may go through in either mode
+    # (they were there before any Linear's), keep the module's own forward
+    if (own is not self._tp_replaced or not _native.plain_call(hidden_states, w) or hidden_states.dtype != w.dtype
+            or not _native.on_hip(hidden_states) or hidden_states.device != w.device
             or torch.is_grad_enabled() and (hidden_states.requires_grad or w.requires_grad)):
-        return type(self).__mro__[1].forward(self, hidden_states)
+        return own(self, hidden_states)
     return _native.rms_norm(hidden_states.detach(), w.detach(), self.variance_epsilon)
 
 
 def is_llama_layer(module: nn.Module) -> bool:
     """transformers' LlamaDecoderLayer as the fused forward below knows it: its forward touches its two norms, the attention and the
     MLP in this order and nothing else, and takes these arguments."""
-    code = getattr(type(module).forward, "__code__", None)
-    return type(module).__name__ == "LlamaDecoderLayer" and type(module).__module__.split(".")[0] == "transformers" and code is not None and \
-        "forward" not in module.__dict__ and code.co_names == ("input_layernorm", "self_attn", "post_attention_layernorm", "mlp") and \
-        code.co_varnames == ("self", "hidden_states", *_LAYER_DEFAULTS, "kwargs", "residual", "_")
+    return type(module).__name__ == "LlamaDecoderLayer" and "forward" not in module.__dict__ and _takes_stand_in(type(module), _llama_layer_forward)
 
 
 _LAYER_DEFAULTS = {"attention_mask": None, "position_ids": None, "past_key_values": None, "use_cache": False, "position_embeddings": None}
@@ -137,16 +149,17 @@ _LAYER_DEFAULTS = {"attention_mask": None, "position_ids": None, "past_key_value
 
 def _llama_layer_forward(self, hidden_states: torch.Tensor, *args, **kwargs) -> torch.Tensor:
     """The layer's own forward with the addition behind the attention inside the second norm's launch."""
-    norm = self.post_attention_layernorm
+    norm, own = self.post_attention_layernorm, self._tp_base.forward
     hooks = torch.nn.modules.module
-    if (args or getattr(type(norm), "forward", None) is not _rms_norm_forward or "forward" in norm.__dict__ or _has_hooks(norm)
+    if (args or own is not self._tp_replaced or getattr(type(norm), "forward", None) is not _rms_norm_forward
+            or norm._tp_base.forward is not norm._tp_replaced or "forward" in norm.__dict__ or _has_hooks(norm)
             or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or torch.is_grad_enabled()
             or not _native.plain_call(hidden_states, norm.weight)):
-        return type(self).__mro__[1].forward(self, hidden_states, *args, **kwargs)
+        return own(self, hidden_states, *args, **kwargs)
     attended, _ = self.self_attn(hidden_states=self.input_layernorm(hidden_states), **{**_LAYER_DEFAULTS, **kwargs})
     w = norm.weight
-    if (_native.plain_call(attended) and _native.on_hip(hidden_states) and hidden_states.device == attended.device == w.device and hidden_states.dtype == attended.dtype == w.dtype
-            and hidden_states.shape == attended.shape):
+    if (_native.plain_call(attended) and _native.on_hip(hidden_states) and hidden_states.device == attended.device == w.device
+            and hidden_states.dtype == attended.dtype == w.dtype and hidden_states.shape == attended.shape):
         total, normed = _native.add_rms_norm(hidden_states, attended, w, norm.variance_epsilon)
     else:
         total = hidden_states + attended
@@ -156,31 +169,50 @@ def _llama_layer_forward(self, hidden_states: torch.Tensor, *args, **kwargs) -> 
 
 def is_rotary_tables(module: nn.Module) -> bool:
     """The rotary embedding modules of transformers' Llama and Falcon: cos / sin of position * inv_freq, the halves repeated."""
-    return type(module).__name__ in ("LlamaRotaryEmbedding", "FalconRotaryEmbedding") and type(module).__module__.split(".")[0] == "transformers" and \
+    return type(module).__name__ in ("LlamaRotaryEmbedding", "FalconRotaryEmbedding") and _takes_stand_in(type(module), _rotary_tables_forward) and \
         isinstance(getattr(module, "inv_freq", None), torch.Tensor) and hasattr(module, "attention_scaling") and hasattr(module, "rope_type")
 
 
 def _rotary_tables_forward(self, x: torch.Tensor, position_ids: torch.Tensor):
-    f, kind = self.inv_freq, self.rope_type
+    f, kind, own = self.inv_freq, self.rope_type, self._tp_base.forward
     # rope types that change their frequencies with the length of the sequence keep the module's own forward
-    if (not _native.plain_call(x, position_ids, f) or position_ids.dtype != torch.int64 or position_ids.dim() != 2 or not _native.on_hip(position_ids) or f.device != position_ids.device or f.dim() != 1
+    if (own is not self._tp_replaced or not _native.plain_call(x, position_ids, f) or position_ids.dtype != torch.int64 or position_ids.dim() != 2
+            or not _native.on_hip(position_ids) or f.device != position_ids.device or f.dim() != 1
             or not isinstance(kind, str) or "dynamic" in kind or kind == "longrope"
             or x.dtype not in (torch.bfloat16, torch.float16, torch.float32) or f.dtype not in (torch.bfloat16, torch.float16, torch.float32)):
-        return type(self).__mro__[1].forward(self, x, position_ids)
+        return own(self, x, position_ids)
     return _native.rope_tables(f, position_ids, self.attention_scaling, x.dtype)
+
+
+# What each fused forward stands in for: the names its own forward looks up, and that one's arguments and locals.
+_STOOD_IN_FOR = {
+    _rms_norm_forward: (("dtype", "to", "torch", "float32", "pow", "mean", "rsqrt", "variance_epsilon", "weight"),
+                        ("self", "hidden_states", "input_dtype", "variance")),
+    _llama_layer_forward: (("input_layernorm", "self_attn", "post_attention_layernorm", "mlp"),
+                           ("self", "hidden_states", *_LAYER_DEFAULTS, "kwargs", "residual", "_")),
+    _rotary_tables_forward: (("inv_freq", "expand", "shape", "to", "torch", "float", "device", "isinstance", "type", "str", "maybe_autocast", "transpose",
+                              "cat", "cos", "attention_scaling", "sin", "dtype"),
+                             ("self", "x", "position_ids", "inv_freq_expanded", "position_ids_expanded", "device_type", "freqs", "emb", "cos", "sin")),
+}
+
+
+def _takes_stand_in(cls: type, forward) -> bool:
+    return cls.__module__.split(".")[0] == "transformers" and _stock_forward(cls, *_STOOD_IN_FOR[forward])
 
 
 _fused_classes: dict = {}
 
 
 def _fused_class(base: type, forward, doc: str) -> type:
-    """Subclass of a module's own class with another forward (isinstance checks keep working, and so does pickling)."""
+    """Subclass of a module's own class with another forward (isinstance checks keep working, and so does pickling). `_tp_replaced` is the
+    forward it stands in for; once the class has another (None: it had when the subclass was made), that one runs."""
     cls = _fused_classes.get((base, forward))
     if cls is None:
         def reduce_ex(self, protocol):  # the class is made here and has no name to be found by: pickle what makes it
             return (_new_fused, (base, forward, doc), *super(cls, self).__reduce_ex__(protocol)[2:])
 
-        cls = type("Shard" + base.__name__, (base,), {"forward": forward, "__doc__": doc, "__reduce_ex__": reduce_ex})
+        cls = type("Shard" + base.__name__, (base,), {"forward": forward, "__doc__": doc, "__reduce_ex__": reduce_ex, "_tp_base": base,
+                                                      "_tp_replaced": staticmethod(base.forward if _takes_stand_in(base, forward) else None)})
         cls = _fused_classes.setdefault((base, forward), cls)
     return cls
 

@@ -137,3 +137,56 @@ def test_a_mask_inside_a_transform_is_transformers_own(monkeypatch):
     assert torch.equal(mask(attention_mask_of, offsets[0]), mask(sdpa_mask, offsets[0])) and asked == [3]
     assert torch.equal(torch.func.vmap(lambda o: mask(attention_mask_of, o))(offsets), torch.stack([mask(sdpa_mask, o) for o in offsets]))
     assert asked == [3]
+
+
+def _replacements():
+    import functools
+
+    from transformers.models.llama import modeling_llama as ml
+
+    def norm(self, hidden_states):  # another formula
+        return hidden_states * self.weight + self.variance_epsilon
+
+    def rotary(self, x, position_ids):  # another position scaling
+        angle = position_ids[..., None].float() * self.inv_freq / 4
+        angle = torch.cat([angle, angle], -1)
+        return angle.cos().to(x.dtype), angle.sin().to(x.dtype)
+
+    def layer(self, hidden_states, **kwargs):
+        return 2 * hidden_states
+
+    own = ml.LlamaRMSNorm.forward
+
+    @functools.wraps(own)
+    def around(self, hidden_states):  # a wrapper that looks like what it wraps
+        return 3 * own(self, hidden_states)
+
+    own_tables = ml.LlamaRotaryEmbedding.forward
+    scaled = functools.wraps(own_tables)(lambda self, x, position_ids: own_tables(self, x, position_ids * 2))
+    return [(ml.LlamaRMSNorm, norm), (ml.LlamaRMSNorm, around), (ml.LlamaRotaryEmbedding, rotary), (ml.LlamaRotaryEmbedding, scaled), (ml.LlamaDecoderLayer, layer)]
+
+
+@pytest.mark.parametrize("which", range(5))
+@pytest.mark.parametrize("when", ["before", "after", "between"])
+def test_a_forward_that_a_program_has_put_in_place_is_honoured(kernels, monkeypatch, which, when):
+    """... also where it was put there behind the shards' making, and where the shards' classes were made before it."""
+    cls, forward = _replacements()[which]
+    x = torch.randn(2, 5, 32)
+
+    def everything(model):
+        return model.norm(x), *model.rotary_emb(x, torch.arange(5)[None]), run_layer(model, x)
+
+    if when != "before":
+        with torch.no_grad():
+            stock = sharded()
+            run_layer(stock, x)
+    if when != "after":
+        monkeypatch.setattr(cls, "forward", forward)
+    model = stock if when == "after" else sharded()
+    monkeypatch.setattr(cls, "forward", forward)
+    own = llama()
+    with torch.no_grad():
+        run_layer(model, x)
+        for got, want in zip(everything(model), everything(own)):
+            assert torch.allclose(got, want, atol=1e-5)
+    monkeypatch.undo()
