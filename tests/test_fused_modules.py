@@ -190,3 +190,23 @@ def test_a_forward_that_a_program_has_put_in_place_is_honoured(kernels, monkeypa
         for got, want in zip(everything(model), everything(own)):
             assert torch.allclose(got, want, atol=1e-5)
     monkeypatch.undo()
+
+
+def test_a_parametrised_norm_or_layer_runs_its_own_forward_once(kernels):
+    """A parametrisation makes a subclass of the fused class: falling back to the next class of the method resolution order came back here for ever."""
+    from torch.nn.utils import parametrize
+
+    class Doubled(torch.nn.Module):
+        def forward(self, w):
+            return 2 * w
+
+    own, model, x = llama(), sharded(), torch.randn(2, 5, 32)
+    for m in (own, model):
+        parametrize.register_parametrization(m.norm, "weight", Doubled())
+        m.layers[0].extra = torch.nn.Parameter(torch.zeros(1), requires_grad=False)
+        parametrize.register_parametrization(m.layers[0], "extra", Doubled())
+    for mode in (torch.no_grad, torch.enable_grad):
+        with mode():
+            assert torch.equal(model.norm(x.double()), own.norm(x.double()))  # a promoting norm: its own forward
+            assert torch.allclose(model.norm(x), own.norm(x), atol=1e-6)
+            assert torch.allclose(run_layer(model, x), run_layer(own, x), atol=1e-5)
