@@ -205,14 +205,16 @@ _fused_classes: dict = {}
 
 def _fused_class(base: type, forward, doc: str) -> type:
     """Subclass of a module's own class with another forward (isinstance checks keep working, and so does pickling). `_tp_replaced` is the
-    forward it stands in for; once the class has another (None: it had when the subclass was made), that one runs."""
+    forward it stands in for; once the class has another (None: it had when the subclass was made), that one runs. A decoder layer's
+    class keeps its name, which programs look such layers up by; the others are named as `ShardLinear` is."""
     cls = _fused_classes.get((base, forward))
     if cls is None:
         def reduce_ex(self, protocol):  # the class is made here and has no name to be found by: pickle what makes it
             return (_new_fused, (base, forward, doc), *super(cls, self).__reduce_ex__(protocol)[2:])
 
-        cls = type("Shard" + base.__name__, (base,), {"forward": forward, "__doc__": doc, "__reduce_ex__": reduce_ex, "_tp_base": base,
-                                                      "_tp_replaced": staticmethod(base.forward if _takes_stand_in(base, forward) else None)})
+        name = base.__name__ if forward is _llama_layer_forward else "Shard" + base.__name__
+        cls = type(name, (base,), {"forward": forward, "__doc__": doc, "__reduce_ex__": reduce_ex, "_tp_base": base,
+                                "_tp_replaced": staticmethod(base.forward if _takes_stand_in(base, forward) else None)})
         cls = _fused_classes.setdefault((base, forward), cls)
     return cls
 
@@ -287,7 +289,6 @@ def install_shard_kernels(shard: nn.Module) -> None:
             module.__class__ = _fused_class(type(module), _rms_norm_forward, "The base class with its forward as one launch (`tpamd_rms_norm`).")
         elif is_llama_layer(module):
             module.__class__ = _fused_class(type(module), _llama_layer_forward, "The base class with an addition and a norm as one launch (`tpamd_add_rms_norm`).")
-            module.__class__.__name__ = type(module).__mro__[1].__name__  # programs look decoder layers up by the name of their class
         elif is_rotary_tables(module):
             module.__class__ = _fused_class(type(module), _rotary_tables_forward, "The base class with its forward as one launch (`tpamd_rope_tables`).")
     for module in shard.modules():

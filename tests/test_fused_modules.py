@@ -210,3 +210,22 @@ def test_a_parametrised_norm_or_layer_runs_its_own_forward_once(kernels):
             assert torch.equal(model.norm(x.double()), own.norm(x.double()))  # a promoting norm: its own forward
             assert torch.allclose(model.norm(x), own.norm(x), atol=1e-6)
             assert torch.allclose(run_layer(model, x), run_layer(own, x), atol=1e-5)
+
+
+def test_an_unpickled_layer_has_the_name_of_its_class(tmp_path):
+    """In a process that has made no shard before: programs look decoder layers up by the name of their class."""
+    import os
+    import pickle
+    import subprocess
+    import sys
+
+    import tensor_parallel_amd
+
+    model = sharded()
+    (tmp_path / "model.pkl").write_bytes(pickle.dumps(model))
+    code = "import pickle, sys; m = pickle.load(open(sys.argv[1], 'rb')); print(*(type(x).__name__ for x in (m.layers[0], m.norm, m.rotary_emb)))"
+    root = os.path.dirname(os.path.dirname(tensor_parallel_amd.__file__))
+    child = subprocess.run([sys.executable, "-c", code, str(tmp_path / "model.pkl")], capture_output=True, text=True, timeout=300, cwd=root)
+    assert child.returncode == 0, child.stderr
+    assert child.stdout.split() == [type(m).__name__ for m in (model.layers[0], model.norm, model.rotary_emb)]
+    assert child.stdout.split()[0] == "LlamaDecoderLayer"
