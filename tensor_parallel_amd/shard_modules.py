@@ -127,13 +127,20 @@ def is_rms_norm(module: nn.Module) -> bool:
         isinstance(getattr(module, "weight", None), torch.Tensor) and module.weight.dim() == 1 and hasattr(module, "variance_epsilon")
 
 
+_KERNEL_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
+
+
+def _norm_kernel_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """What `tpamd_rms_norm` is made for; a promoting norm, one moved to another dtype (`.double()`) or with a weight that broadcasts is not."""
+    return _native.plain_call(x, w) and x.dtype == w.dtype and w.dtype in _KERNEL_DTYPES and w.dim() == 1 and x.dim() > 0 and x.shape[-1] == w.shape[0] \
+        and _native.on_hip(x) and x.device == w.device
+
+
 def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
     w, own = self.weight, self._tp_base.forward
-    # a norm whose class has been given another forward since, a promoting norm, and one that derivatives may go through in either mode
-    # (they were there before any Linear's), keep the module's own forward
-    if (own is not self._tp_replaced or not _native.plain_call(hidden_states, w) or hidden_states.dtype != w.dtype
-            or not _native.on_hip(hidden_states) or hidden_states.device != w.device
-            or torch.is_grad_enabled() and (hidden_states.requires_grad or w.requires_grad)):
+    # a norm whose class has been given another forward since, and one that derivatives may go through (they were there before any
+    # Linear's), keep the module's own forward
+    if own is not self._tp_replaced or not _norm_kernel_takes(hidden_states, w) or torch.is_grad_enabled() and (hidden_states.requires_grad or w.requires_grad):
         return own(self, hidden_states)
     return _native.rms_norm(hidden_states.detach(), w.detach(), self.variance_epsilon)
 
@@ -153,14 +160,11 @@ def _llama_layer_forward(self, hidden_states: torch.Tensor, *args, **kwargs) -> 
     hooks = torch.nn.modules.module
     if (args or own is not self._tp_replaced or getattr(type(norm), "forward", None) is not _rms_norm_forward
             or norm._tp_base.forward is not norm._tp_replaced or "forward" in norm.__dict__ or _has_hooks(norm)
-            or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or torch.is_grad_enabled()
-            or not _native.plain_call(hidden_states, norm.weight)):
+            or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or torch.is_grad_enabled() or not _norm_kernel_takes(hidden_states, norm.weight)):
         return own(self, hidden_states, *args, **kwargs)
     attended, _ = self.self_attn(hidden_states=self.input_layernorm(hidden_states), **{**_LAYER_DEFAULTS, **kwargs})
-    w = norm.weight
-    if (_native.plain_call(attended) and _native.on_hip(hidden_states) and hidden_states.device == attended.device == w.device
-            and hidden_states.dtype == attended.dtype == w.dtype and hidden_states.shape == attended.shape):
-        total, normed = _native.add_rms_norm(hidden_states, attended, w, norm.variance_epsilon)
+    if _norm_kernel_takes(attended, norm.weight) and hidden_states.shape == attended.shape:
+        total, normed = _native.add_rms_norm(hidden_states, attended, norm.weight, norm.variance_epsilon)
     else:
         total = hidden_states + attended
         normed = norm(total)
@@ -179,7 +183,7 @@ def _rotary_tables_forward(self, x: torch.Tensor, position_ids: torch.Tensor):
     if (own is not self._tp_replaced or not _native.plain_call(x, position_ids, f) or position_ids.dtype != torch.int64 or position_ids.dim() != 2
             or not _native.on_hip(position_ids) or f.device != position_ids.device or f.dim() != 1
             or not isinstance(kind, str) or "dynamic" in kind or kind == "longrope"
-            or x.dtype not in (torch.bfloat16, torch.float16, torch.float32) or f.dtype not in (torch.bfloat16, torch.float16, torch.float32)):
+            or x.dtype not in _KERNEL_DTYPES or f.dtype not in _KERNEL_DTYPES):
         return own(self, x, position_ids)
     return _native.rope_tables(f, position_ids, self.attention_scaling, x.dtype)
 
@@ -283,9 +287,9 @@ def install_shard_kernels(shard: nn.Module) -> None:
     for module in shard.modules():
         if type(module) is nn.Linear:
             module.__class__ = ShardLinear
-        elif is_conv1d(module) and type(module).__name__ == "Conv1D" and module.weight.dim() == 2 and module.weight.dtype in (torch.bfloat16, torch.float16, torch.float32):
+        elif is_conv1d(module) and type(module).__name__ == "Conv1D" and module.weight.dim() == 2 and module.weight.dtype in _KERNEL_DTYPES:
             module.__class__ = _shard_conv1d_class(type(module))
-        elif is_rms_norm(module) and module.weight.dtype in (torch.bfloat16, torch.float16, torch.float32):
+        elif is_rms_norm(module) and module.weight.dtype in _KERNEL_DTYPES:
             module.__class__ = _fused_class(type(module), _rms_norm_forward, "The base class with its forward as one launch (`tpamd_rms_norm`).")
         elif is_llama_layer(module):
             module.__class__ = _fused_class(type(module), _llama_layer_forward, "The base class with an addition and a norm as one launch (`tpamd_add_rms_norm`).")

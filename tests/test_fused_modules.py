@@ -229,3 +229,28 @@ def test_an_unpickled_layer_has_the_name_of_its_class(tmp_path):
     assert child.returncode == 0, child.stderr
     assert child.stdout.split() == [type(m).__name__ for m in (model.layers[0], model.norm, model.rotary_emb)]
     assert child.stdout.split()[0] == "LlamaDecoderLayer"
+
+
+@pytest.mark.parametrize("change", [lambda m: m.double(), lambda m: setattr(m, "weight", torch.nn.Parameter(torch.full((1,), 2.0))),
+                                    lambda m: setattr(m, "weight", torch.nn.Parameter(torch.arange(160.0).view(5, 32)))])
+def test_a_norm_that_the_kernel_does_not_take_keeps_its_own_forward(kernels, change):
+    """Another dtype than the kernel's three, and weights that broadcast."""
+    own, model = llama(), sharded()
+    with torch.no_grad():
+        for m in (own, model):
+            change(m.norm)
+        for dtype in (torch.float32, torch.float64):
+            x = torch.randn(2, 5, 32, dtype=dtype)
+            got, want = model.norm(x), own.norm(x)
+            assert got.dtype == want.dtype and torch.equal(got, want)
+        x = torch.randn(2, 5, 32, dtype=torch.float64)
+        layers = llama().double().layers[0], sharded().double().layers[0]
+        for layer in layers:
+            layer.self_attn, layer.mlp = _Attention(), torch.nn.Identity()
+        assert torch.equal(layers[0](x), layers[1](x))
+    assert not kernels
+
+
+class _Attention(torch.nn.Module):
+    def forward(self, hidden_states, **kwargs):
+        return hidden_states * 0.5, None
