@@ -177,14 +177,15 @@ def is_rotary_tables(module: nn.Module) -> bool:
         isinstance(getattr(module, "inv_freq", None), torch.Tensor) and hasattr(module, "attention_scaling") and hasattr(module, "rope_type")
 
 
-def _rotary_tables_forward(self, x: torch.Tensor, position_ids: torch.Tensor):
+def _rotary_tables_forward(self, x: torch.Tensor, position_ids: torch.Tensor, **kwargs):
     f, kind, own = self.inv_freq, self.rope_type, self._tp_base.forward
-    # rope types that change their frequencies with the length of the sequence keep the module's own forward
-    if (own is not self._tp_replaced or not _native.plain_call(x, position_ids, f) or position_ids.dtype != torch.int64 or position_ids.dim() != 2
+    # rope types that change their frequencies with the length of the sequence keep the module's own forward; so do the further arguments
+    # of its decorator
+    if (kwargs or own is not self._tp_replaced or not _native.plain_call(x, position_ids, f) or position_ids.dtype != torch.int64 or position_ids.dim() != 2
             or not _native.on_hip(position_ids) or f.device != position_ids.device or f.dim() != 1
             or not isinstance(kind, str) or "dynamic" in kind or kind == "longrope"
             or x.dtype not in _KERNEL_DTYPES or f.dtype not in _KERNEL_DTYPES):
-        return own(self, x, position_ids)
+        return own(self, x, position_ids, **kwargs)
     return _native.rope_tables(f, position_ids, self.attention_scaling, x.dtype)
 
 

@@ -254,3 +254,11 @@ def test_a_norm_that_the_kernel_does_not_take_keeps_its_own_forward(kernels, cha
 class _Attention(torch.nn.Module):
     def forward(self, hidden_states, **kwargs):
         return hidden_states * 0.5, None
+
+
+def test_rotary_tables_take_the_arguments_of_the_modules_own_forward(kernels):
+    own, model, x, position_ids = llama(), sharded(), torch.randn(2, 5, 32), torch.arange(5)[None]
+    for kwargs in ({}, {"layer_type": None}):
+        for got, want in zip(model.rotary_emb(x=x, position_ids=position_ids, **kwargs), own.rotary_emb(x=x, position_ids=position_ids, **kwargs)):
+            assert torch.equal(got, want)
+    assert kernels == ["rope_tables"]
