@@ -14,6 +14,7 @@
 //                       kernel elsewhere (TPAMD_GEMM_W4=0 selects it).
 //   gemm_kernel         any K (multiple of 8) and the 128x128 tiling for small problems, v_mfma_f32_32x32x16; next
 //                       K tile prefetched into registers while the current one is multiplied.
+#include "gemm_model.h"
 #include "gemm_tile.h"
 
 #include <stdlib.h>
@@ -2055,32 +2056,6 @@ int launch_direct128(GemmParams p, int cus, hipStream_t s) {
     return TPAMD_OK;
 }
 
-// Predicted time (microseconds) of gemm_mid_kernel on the best of its tiles, and that tile: a launch, rounds of one block per CU, each with
-// a fixed cost (first tiles, epilogue) and a time per K tile, shorter where the last round leaves CUs idle (the part clocks higher).
-// Non-negative least squares on relative errors over 237 shapes (9 matrices at 128-8192 rows, 90 random ones), each tile forced and timed
-// inside a HIP graph. There the choice among these tiles, the 256 x 256 and the 128 x 128 tiling is 1.7 % off the best one (geometric
-// mean; 6.4 % without these tiles) and nowhere slower than without them. Examples: the pair 5504 x 4096 at 512 rows 64 -> 51 us (128 x 192; two
-// K splits of 256 x 256 before) and at 645 rows 84 -> 60 us, 4096 x 5504 at 2103 rows 105 -> 78 us (192 x 192; 144 tiles of 256 x 256 before).
-struct MidTile { int tmx, tnx; double launch, round, full, idle[3]; };  // idle: last round at most 1/2, at most 3/4, more of the CUs
-constexpr MidTile MID_TILES[2][4] = {
-    {{4, 6, 0.5, 5.0, 0.643, {0.537, 0.588, 0.693}}, {4, 8, 0.4, 5.8, 0.827, {0.663, 0.740, 0.820}},
-     {6, 6, 2.6, 6.7, 0.858, {0.635, 0.714, 0.789}}, {6, 8, 0.1, 5.4, 1.226, {0.922, 0.977, 1.211}}},
-    {{4, 6, 0.7, 3.2, 0.642, {0.661, 0.715, 0.688}}, {4, 8, 1.4, 3.6, 0.837, {0.756, 0.808, 0.832}},
-     {6, 6, 0.0, 7.2, 0.827, {0.727, 0.755, 0.820}}, {6, 8, 1.3, 2.0, 1.223, {1.099, 1.088, 1.233}}},
-};
-
-inline double estimate_mid(int64_t M, int64_t N, int KT, int cus, bool swiglu, int *tmx, int *tnx) {
-    double best = 1e30;
-    for (const MidTile &t : MID_TILES[swiglu ? 1 : 0]) {
-        const int64_t bm = 32 * t.tmx, bn = (swiglu ? 16 : 32) * t.tnx;
-        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn), full = tiles / cus, last = tiles % cus;
-        double us = t.launch + full * (t.round + KT * t.full);
-        if (last > 0) us += t.round + KT * t.idle[last * 2 <= cus ? 0 : last * 4 <= 3ll * cus ? 1 : 2];
-        if (us < best) { best = us; *tmx = t.tmx; *tnx = t.tnx; }
-    }
-    return best;
-}
-
 // Prefill-sized dispatch; called by linear.hip once M is above the skinny range.
 template <int DT>
 int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
@@ -2099,9 +2074,8 @@ int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
         const int64_t full = units / cus, last = units % cus;
         return kt * (full * 1.47 + (last == 0 ? 0.0 : last * 4 <= 3ll * cus ? 1.2 : 1.3));
     };
-    // no launch streams the weights faster than 5 TB/s (what bounds a few rows of a wide matrix: the pair 8192 x 8192 at
-    // 17 rows took 79.8 us on this tiling in four splits, predicted 57 without this term, and 63.8 us on the other)
-    const double stream = static_cast<double>(p.N) * p.K * (swiglu ? 4.0 : 2.0) / 5.0e6;
+    const double stream = stream_floor(p.N, p.K, swiglu);  // the pair 8192 x 8192 at 17 rows took 79.8 us on this tiling in four splits, predicted
+                                                           // 57 without this term, and 63.8 us on the other
     auto floor256 = [&](double loop) { return loop > stream ? loop : stream; };
     double t256 = floor256(rounds256(big_tiles, KT));
     // ... or split over K while all units still fit one round; the partial tiles cost 9 us + 0.33 us per MB (more than

@@ -1,0 +1,41 @@
+// Cost models that choose between the GEMM kernels: host code, microseconds on this part.
+#pragma once
+#include <stdint.h>
+
+namespace tpamd {
+
+// No launch streams the weights of a 16-bit matrix (or gated pair) faster than 5 TB/s, which is what bounds a few rows of a wide one.
+inline double stream_floor(int64_t N, int64_t K, bool swiglu) { return static_cast<double>(N) * K * (swiglu ? 4.0 : 2.0) / 5.0e6; }
+
+// Predicted time (microseconds) of gemm_mid_kernel on the best of its tiles, and that tile: a launch, rounds of one block per CU, each with
+// a fixed cost (first tiles, epilogue) and a time per K tile, shorter where the last round leaves CUs idle (the part clocks higher).
+// Non-negative least squares on relative errors over 237 shapes (9 matrices at 128-8192 rows, 90 random ones), each tile forced and timed
+// inside a HIP graph. Over those, all at 128 rows or more, the choice among these tiles, the 256 x 256 and the 128 x 128 tiling is 1.7 % off the
+// best one (geometric mean; 6.4 % without these tiles) and nowhere slower than without them. Examples: the pair 5504 x 4096 at 512 rows 64 -> 51 us (128 x 192; two
+// K splits of 256 x 256 before) and at 645 rows 84 -> 60 us, 4096 x 5504 at 2103 rows 105 -> 78 us (192 x 192; 144 tiles of 256 x 256 before).
+struct MidTile { int tmx, tnx; double launch, round, full, idle[3]; };  // idle: last round at most 1/2, at most 3/4, more of the CUs
+constexpr MidTile MID_TILES[2][4] = {
+    {{4, 6, 0.5, 5.0, 0.643, {0.537, 0.588, 0.693}}, {4, 8, 0.4, 5.8, 0.827, {0.663, 0.740, 0.820}},
+     {6, 6, 2.6, 6.7, 0.858, {0.635, 0.714, 0.789}}, {6, 8, 0.1, 5.4, 1.226, {0.922, 0.977, 1.211}}},
+    {{4, 6, 0.7, 3.2, 0.642, {0.661, 0.715, 0.688}}, {4, 8, 1.4, 3.6, 0.837, {0.756, 0.808, 0.832}},
+     {6, 6, 0.0, 7.2, 0.827, {0.727, 0.755, 0.820}}, {6, 8, 1.3, 2.0, 1.223, {1.099, 1.088, 1.233}}},
+};
+
+// Up to 128 rows, where nothing was fitted, at least what streaming the weights takes. Without that floor few rows of a wide matrix were
+// predicted faster than HBM and taken off the 128 x 128 tiling, where a tie leaves them (us there / on these tiles): 28672 x 4096 at
+// 17 / 40 / 64 / 128 rows 52 52 53 58 / 56 58 61 68, 32000 x 4096 62 62 63 62 / 65 65 67 67, the pair 14336 x 4096 52 52 53 57 / 56 56 57 60.
+// Above, the floor would be wrong: 64128 x 4096 at 160 / 192 rows takes 133 / 136 us on these tiles and 142 / 144 on 256 x 256.
+inline double estimate_mid(int64_t M, int64_t N, int KT, int cus, bool swiglu, int *tmx, int *tnx) {
+    double best = 1e30;
+    for (const MidTile &t : MID_TILES[swiglu ? 1 : 0]) {
+        const int64_t bm = 32 * t.tmx, bn = (swiglu ? 16 : 32) * t.tnx;
+        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn), full = tiles / cus, last = tiles % cus;
+        double us = t.launch + full * (t.round + KT * t.full);
+        if (last > 0) us += t.round + KT * t.idle[last * 2 <= cus ? 0 : last * 4 <= 3ll * cus ? 1 : 2];
+        if (us < best) { best = us; *tmx = t.tmx; *tnx = t.tnx; }
+    }
+    const double stream = stream_floor(N, 64ll * KT, swiglu);
+    return M <= 128 && best < stream ? stream : best;
+}
+
+}  // namespace tpamd

@@ -1,0 +1,31 @@
+"""The cost models that choose between the GEMM kernels (csrc/gemm_model.h) are host code: compiled into a small program and asked here."""
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+CSRC = Path(__file__).resolve().parent.parent / "tensor_parallel_amd" / "csrc"
+
+
+def ask(tmp_path, body):
+    """The program's output for a body that prints rows of numbers, as lists of floats."""
+    if shutil.which("g++") is None:
+        pytest.skip("no host compiler")
+    (tmp_path / "ask.cpp").write_text('#include <stdio.h>\n#include <initializer_list>\n#include "gemm_model.h"\nusing namespace tpamd;\nint main() {\n' + body + "\n}\n")
+    subprocess.run(["g++", "-std=c++17", "-I", str(CSRC), str(tmp_path / "ask.cpp"), "-o", str(tmp_path / "ask")], check=True)
+    out = subprocess.run([str(tmp_path / "ask")], check=True, capture_output=True, text=True, timeout=60).stdout
+    return [[float(v) for v in line.split()] for line in out.splitlines()]
+
+
+def test_no_mid_tile_is_predicted_faster_than_its_weights_stream(tmp_path):
+    """Up to 128 rows of wide matrices: every tiling is floored at the same 5 TB/s, so a tie decides there, and not which model lacks the floor."""
+    rows = ask(tmp_path, """
+    const long long shapes[][2] = {{64128, 4096}, {32000, 4096}, {28672, 8192}, {28672, 4096}, {4096, 5504}, {260, 64}};
+    for (auto &s : shapes) for (int swiglu = 0; swiglu < 2; ++swiglu) for (int m : {17, 40, 64, 100, 128}) {
+        int tmx = 0, tnx = 0;
+        printf("%d %lld %lld %d %.9g\\n", m, s[0], s[1], swiglu, estimate_mid(m, s[0], (int)(s[1] / 64), 256, swiglu != 0, &tmx, &tnx));
+    }""")
+    assert len(rows) == 6 * 2 * 5
+    for m, n, k, swiglu, us in rows:
+        assert us * 5e6 >= n * k * (4 if swiglu else 2) * (1 - 1e-6), (m, n, k, swiglu, us)
