@@ -216,6 +216,18 @@ def plain_call(*tensors: torch.Tensor) -> bool:
                 or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0)
 
 
+def stock_function(f, module: str, qualname: str, names: tuple, variables: tuple) -> bool:
+    """Whether f is the function of this name that this module of transformers defines, decorated by nobody but torch and transformers, and known
+    here by the names that it looks up and its arguments and locals: a kernel does not stand in for what a program has put in its place."""
+    while True:
+        if getattr(f, "__code__", None) is None or f.__globals__.get("__name__", "").split(".")[0] not in ("torch", "transformers"):
+            return False
+        if not hasattr(f, "__wrapped__"):
+            break
+        f = f.__wrapped__
+    return f.__globals__["__name__"] == module and f.__qualname__ == qualname and f.__code__.co_names == names and f.__code__.co_varnames == variables
+
+
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 

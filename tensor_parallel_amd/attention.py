@@ -49,9 +49,18 @@ def attention_forward(module: torch.nn.Module, query: torch.Tensor, key: torch.T
     return out, None
 
 
+# What the mask kernel stands in for: the names that `sdpa_mask` and the causal rule look up, their arguments and locals.
+_SDPA_MASK = (("prepare_padding_mask", "_ignore_causal_mask_sdpa", "_ignore_bidirectional_mask_sdpa", "and_masks", "padding_mask_function", "torch", "arange",
+               "_non_vmap_expansion_sdpa", "expand", "_is_torch_greater_or_equal_than_2_6", "TransformGetItemToIndex", "_vmap_expansion_sdpa", "ValueError"),
+              ("batch_size", "q_length", "kv_length", "q_offset", "kv_offset", "mask_function", "attention_mask", "local_size", "allow_is_causal_skip",
+               "allow_is_bidirectional_skip", "allow_torch_fix", "use_vmap", "device", "kwargs", "padding_mask", "batch_arange", "head_arange", "q_arange", "kv_arange"))
+_CAUSAL = ((), ("batch_idx", "head_idx", "q_idx", "kv_idx"))
+
+
 def attention_mask_of(*args, **kwargs) -> Optional[torch.Tensor]:
     """transformers' `sdpa_mask`, the same result with one launch where a decode step on a static cache asks for it: the plain causal
-    mask, no padding, no right to skip it, the position of the first query a number on the device. All else goes to `sdpa_mask`."""
+    mask, no padding, no right to skip it, the position of the first query a number on the device. All else goes to `sdpa_mask`, and so does everything
+    once a program has put another function in the place of that one or of the causal rule."""
     from transformers.masking_utils import causal_mask_function, sdpa_mask
 
     q_offset, q_length, kv_length, kv_offset = (kwargs.get(n) for n in ("q_offset", "q_length", "kv_length", "kv_offset"))
@@ -59,7 +68,9 @@ def attention_mask_of(*args, **kwargs) -> Optional[torch.Tensor]:
             or kwargs.get("allow_is_bidirectional_skip", False) or kwargs.get("attention_mask") is not None or kwargs.get("use_vmap", False)
             or not _native.plain_call(q_offset) or not _native.on_hip(q_offset) or q_offset.dtype != torch.int64 or q_offset.dim() > 1
             or q_offset.numel() != 1 or torch.device(kwargs.get("device", "cpu")) != q_offset.device
-            or not all(type(n) is int for n in (q_length, kv_length, kv_offset, kwargs.get("batch_size")))):
+            or not all(type(n) is int for n in (q_length, kv_length, kv_offset, kwargs.get("batch_size")))
+            or not _native.stock_function(sdpa_mask, "transformers.masking_utils", "sdpa_mask", *_SDPA_MASK)
+            or not _native.stock_function(causal_mask_function, "transformers.masking_utils", "causal_mask_function", *_CAUSAL)):
         return sdpa_mask(*args, **kwargs)
     return _native.causal_mask(q_offset, kv_offset, q_length, kv_length).expand(kwargs["batch_size"], -1, q_length, kv_length)
 

@@ -107,20 +107,6 @@ def _shard_conv1d_class(base: type) -> type:
     return cls
 
 
-def _stock_forward(cls: type, names: tuple, variables: tuple) -> bool:
-    """Whether the class's forward is the one its own module in transformers defines, decorated by nobody but torch and transformers, and
-    known here by the names that it looks up and its arguments and locals: a forward that a program has put in its place is not stood in for."""
-    f = getattr(cls, "forward", None)
-    while True:
-        if getattr(f, "__code__", None) is None or f.__globals__.get("__name__", "").split(".")[0] not in ("torch", "transformers"):
-            return False
-        if not hasattr(f, "__wrapped__"):
-            break
-        f = f.__wrapped__
-    return f.__globals__["__name__"] == cls.__module__ and f.__qualname__ == f"{cls.__qualname__}.forward" and \
-        f.__code__.co_names == names and f.__code__.co_varnames == variables
-
-
 def is_rms_norm(module: nn.Module) -> bool:
     """transformers' LlamaRMSNorm: a weight over the last axis and `variance_epsilon`, statistics in fp32."""
     return type(module).__name__ == "LlamaRMSNorm" and _takes_stand_in(type(module), _rms_norm_forward) and \
@@ -202,7 +188,8 @@ _STOOD_IN_FOR = {
 
 
 def _takes_stand_in(cls: type, forward) -> bool:
-    return cls.__module__.split(".")[0] == "transformers" and _stock_forward(cls, *_STOOD_IN_FOR[forward])
+    return cls.__module__.split(".")[0] == "transformers" and \
+        _native.stock_function(getattr(cls, "forward", None), cls.__module__, f"{cls.__qualname__}.forward", *_STOOD_IN_FOR[forward])
 
 
 _fused_classes: dict = {}

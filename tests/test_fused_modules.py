@@ -139,6 +139,30 @@ def test_a_mask_inside_a_transform_is_transformers_own(monkeypatch):
     assert asked == [3]
 
 
+@pytest.mark.parametrize("name", ["sdpa_mask", "causal_mask_function"])
+def test_a_mask_function_that_a_program_has_put_in_place_is_honoured(monkeypatch, name):
+    from transformers import masking_utils
+
+    from tensor_parallel_amd.attention import attention_mask_of
+
+    asked = []
+    monkeypatch.setattr(_native, "on_hip", lambda t: True)
+    monkeypatch.setattr(_native, "causal_mask", lambda q_offset, kv_offset, rows, cols: asked.append(rows))
+    offset = torch.tensor(4)
+
+    def form():
+        return dict(batch_size=2, q_length=3, kv_length=9, q_offset=offset, kv_offset=0, attention_mask=None, mask_function=masking_utils.causal_mask_function,
+                    allow_is_causal_skip=False, use_vmap=False, device=torch.device("cpu"), dtype=torch.float32, config=None)
+
+    stock = masking_utils.sdpa_mask(**form())
+    if name == "sdpa_mask":
+        monkeypatch.setattr(masking_utils, name, lambda **kwargs: ~stock)
+    else:  # a window of two keys
+        monkeypatch.setattr(masking_utils, name, lambda batch_idx, head_idx, q_idx, kv_idx: (kv_idx <= q_idx) & (kv_idx > q_idx - 2))
+    want = masking_utils.sdpa_mask(**form())
+    assert not torch.equal(want, stock) and torch.equal(attention_mask_of(**form()), want) and not asked
+
+
 def _replacements():
     import functools
 
