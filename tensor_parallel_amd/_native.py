@@ -12,6 +12,7 @@ from pathlib import Path
 from typing import Optional, Sequence
 
 import torch  # imported first on purpose: the library binds to the HIP runtime torch has loaded
+from torch.utils._device import DeviceContext
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libtpamd.so"
 
@@ -208,9 +209,12 @@ def on_hip(t: torch.Tensor) -> bool:
 def plain_call(*tensors: torch.Tensor) -> bool:
     """Whether a kernel launched on these tensors' memory may stand in for torch calls on them: the tensors are torch's own, and nothing
     follows the calls that would miss the kernel (forward-mode derivatives; vmap and the other functorch transforms, whose wrappers
-    have no memory; compilation and tracing; dispatch modes)."""
+    have no memory; compilation and tracing; dispatch modes, and function modes other than a default device)."""
     for t in tensors:
         if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
+            return False
+    for i in range(torch._C._len_torch_function_stack()):
+        if type(torch._C._get_function_stack_at(i)) is not DeviceContext:
             return False
     return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0
                 or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0)

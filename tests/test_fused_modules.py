@@ -119,6 +119,23 @@ def test_what_follows_the_torch_calls_sees_the_modules_own(kernels):
     assert not kernels
 
 
+class _Doubled(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        out = func(*args, **(kwargs or {}))
+        return 2 * out if func in (torch.rsqrt, torch.Tensor.cos) else out
+
+
+def test_a_function_mode_sees_the_modules_own_calls(kernels):
+    own, model, x, position_ids = llama(), sharded(), torch.randn(2, 5, 32), torch.arange(5)[None]
+    with torch.no_grad():
+        with _Doubled():
+            assert torch.equal(model.norm(x), own.norm(x)) and torch.equal(model.rotary_emb(x, position_ids)[0], own.rotary_emb(x, position_ids)[0])
+            assert not kernels
+        with torch.device("cpu"):  # a default device is a function mode too, of no account here
+            model.norm(x)
+    assert kernels == ["rms_norm"]
+
+
 def test_a_mask_inside_a_transform_is_transformers_own(monkeypatch):
     from transformers.masking_utils import causal_mask_function, sdpa_mask
 
