@@ -143,7 +143,7 @@ __global__ __launch_bounds__(256) void rms_norm_any_kernel(NormParams p) {
 }
 
 template <int DT, bool ADD>
-void launch(const NormParams &p, int64_t rows, bool vec, hipStream_t s) {
+void launch_rows(const NormParams &p, int64_t rows, bool vec, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>(rows));
     const int n = p.D / 8;  // 16-byte chunks per row
     // one chunk per lane as far as a block of 16 wavefronts goes: a lone row is then one load away from its sum
@@ -158,6 +158,24 @@ void launch(const NormParams &p, int64_t rows, bool vec, hipStream_t s) {
     }
 }
 
+// A launch has at most 2^32 - 1 threads, and one that asks for more runs, without an error, what is left of the count modulo 2^32: further
+// rows go into further launches.
+constexpr int64_t ROWS_PER_LAUNCH = 1ll << 21;
+
+template <int DT, bool ADD>
+void launch(NormParams p, int64_t rows, bool vec, hipStream_t s) {
+    constexpr int64_t ESZ = DT == TPAMD_F32 ? 4 : 2;
+    for (; rows > 0; rows -= ROWS_PER_LAUNCH) {
+        launch_rows<DT, ADD>(p, rows < ROWS_PER_LAUNCH ? rows : ROWS_PER_LAUNCH, vec, s);
+        p.x += ROWS_PER_LAUNCH * p.ldx * ESZ;
+        p.y += ROWS_PER_LAUNCH * p.ldy * ESZ;
+        if constexpr (ADD) {
+            p.r += ROWS_PER_LAUNCH * p.ldr * ESZ;
+            p.s += ROWS_PER_LAUNCH * p.ldy * ESZ;
+        }
+    }
+}
+
 }  // namespace
 }  // namespace tpamd
 
@@ -166,7 +184,7 @@ using namespace tpamd;
 static int run_norm(const char *who, const void *x_dev, const void *r_dev, const void *w_dev, void *s_dev, void *y_dev, int64_t rows, int64_t D,
                     int64_t ldx, int64_t ldr, int64_t ldy, float eps, int dtype, void *stream, bool add) {
     TPAMD_REQUIRE(dtype == TPAMD_BF16 || dtype == TPAMD_F16 || dtype == TPAMD_F32, "%s: unknown dtype %d", who, dtype);
-    TPAMD_REQUIRE(rows >= 0 && D >= 0 && rows < (1ll << 31) && D < (1ll << 31), "%s: bad dimension", who);
+    TPAMD_REQUIRE(rows >= 0 && D >= 0 && D < (1ll << 31), "%s: bad dimension", who);
     if (rows == 0 || D == 0) return TPAMD_OK;
     TPAMD_REQUIRE(x_dev && w_dev && y_dev && (!add || (r_dev && s_dev)), "%s: null pointer", who);
     TPAMD_REQUIRE(ldx >= D && ldy >= D && (!add || ldr >= D), "%s: leading dimension smaller than the row", who);

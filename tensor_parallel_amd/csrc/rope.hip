@@ -67,8 +67,8 @@ __global__ __launch_bounds__(256) void rope_append_kernel(RopeParams p) {
 // concatenation, and three passes for each table), 2 us each in a recorded decode step.
 template <int DT>
 __global__ __launch_bounds__(256) void rope_tables_kernel(const char *inv_freq, int freq_dtype, const int64_t *pos, int64_t pos_b, int64_t pos_s, int S,
-                                                          int half, float scaling, char *cos_out, char *sin_out, int64_t n) {
-    const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+                                                          int half, float scaling, char *cos_out, char *sin_out, int64_t first, int64_t n) {
+    const int64_t e = first + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (e >= n) return;
     const int64_t row = e / half;
     const int i = static_cast<int>(e - row * half);
@@ -150,16 +150,21 @@ extern "C" int tpamd_rope_tables(const void *inv_freq_dev, int freq_dtype, const
     TPAMD_REQUIRE(B >= 0 && S >= 0 && half >= 0 && B < (1ll << 31) && S < (1ll << 31) && half < (1ll << 31), "%s: bad dimension", who);
     if (B == 0 || S == 0 || half == 0) return TPAMD_OK;
     TPAMD_REQUIRE(inv_freq_dev && pos_dev && cos_dev && sin_dev, "%s: null pointer", who);
-    TPAMD_REQUIRE(B * S < (1ll << 31) && B * S * half < (1ll << 38), "%s: too many positions for one launch", who);
+    TPAMD_REQUIRE(B * S < (1ll << 31) && B * S * half < (1ll << 38), "%s: too many positions", who);
     const int64_t n = B * S * half;
-    const dim3 grid(static_cast<unsigned>((n + 255) / 256));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const char *f = static_cast<const char *>(inv_freq_dev);
     char *c = static_cast<char *>(cos_dev), *si = static_cast<char *>(sin_dev);
     const int Si = static_cast<int>(S), h = static_cast<int>(half);
-    if (dtype == TPAMD_BF16) hipLaunchKernelGGL(rope_tables_kernel<TPAMD_BF16>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, n);
-    else if (dtype == TPAMD_F16) hipLaunchKernelGGL(rope_tables_kernel<TPAMD_F16>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, n);
-    else hipLaunchKernelGGL(rope_tables_kernel<TPAMD_F32>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, n);
+    // a launch has at most 2^32 - 1 threads, and one that asks for more runs, without an error, what is left of the count modulo 2^32
+    constexpr int64_t PER_LAUNCH = 1ll << 31;
+    for (int64_t e = 0; e < n; e += PER_LAUNCH) {
+        const int64_t part = n - e < PER_LAUNCH ? n - e : PER_LAUNCH;
+        const dim3 grid(static_cast<unsigned>((part + 255) / 256));
+        if (dtype == TPAMD_BF16) hipLaunchKernelGGL(rope_tables_kernel<TPAMD_BF16>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, e, n);
+        else if (dtype == TPAMD_F16) hipLaunchKernelGGL(rope_tables_kernel<TPAMD_F16>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, e, n);
+        else hipLaunchKernelGGL(rope_tables_kernel<TPAMD_F32>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, e, n);
+    }
     TPAMD_HIP(hipGetLastError());
     return TPAMD_OK;
 }

@@ -121,3 +121,13 @@ def test_decoder_layer_with_the_addition_in_its_norm():
             h.remove()
     assert len(seen) == 4 and torch.equal(fused.logits, own.logits)
     assert all(torch.equal(a, b) for a, b in zip(fused.hidden_states, own.hidden_states))
+
+
+def test_more_rows_than_one_launch_takes():
+    """A launch has fewer than 2^32 threads: 2^24 rows of the element-wise kernel (256 threads each) and 2^22 of the widest rows have them all."""
+    rows, w = (1 << 24) + 3, torch.tensor([1.0, 2.0, 0.5], device=DEV)
+    x = torch.randn(rows, 3, device=DEV)
+    total, y = _native.add_rms_norm(x, x, w, 1e-6)
+    for at in (slice(0, 5), slice((1 << 23) - 2, (1 << 23) + 2), slice(rows - 5, rows)):
+        assert torch.equal(_native.rms_norm(x, w, 1e-6)[at], _native.rms_norm(x[at].contiguous(), w, 1e-6))
+        assert torch.equal(total[at], 2 * x[at]) and torch.equal(y[at], _native.rms_norm(2 * x[at], w, 1e-6))

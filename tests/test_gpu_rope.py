@@ -159,3 +159,16 @@ def test_rotary_modules_of_the_shards_use_the_tables(family):
         torch.testing.assert_close(g.cpu().float(), w.float(), rtol=2.0 ** -7, atol=1e-6)
     mine[0].rope_type = "dynamic"  # frequencies that change with the length: the module's own forward
     assert mine[0](x.to(DEV), pos.to(DEV))[0].shape == want[0].shape
+
+
+def test_tables_of_more_elements_than_one_launch_takes():
+    """A launch has fewer than 2^32 threads, one per position and frequency here: a batch whose rows go over several launches has them all."""
+    S, half, B = 1 << 14, 256, (1 << 10) + 1
+    if torch.cuda.mem_get_info(DEV)[0] < 48 << 30:
+        pytest.skip("the tables take 35 GB")
+    freq = 10000.0 ** (-torch.arange(half, device=DEV) / half)
+    positions = torch.arange(S, device=DEV)[None].expand(B, -1) + torch.arange(B, device=DEV)[:, None]
+    cos, sin = _native.rope_tables(freq, positions, 1.0, torch.bfloat16)
+    for b in (0, B // 2, B - 2, B - 1):
+        c, s = _native.rope_tables(freq, positions[b:b + 1], 1.0, torch.bfloat16)
+        assert torch.equal(cos[b], c[0]) and torch.equal(sin[b], s[0])
