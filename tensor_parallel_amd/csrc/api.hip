@@ -275,9 +275,11 @@ extern "C" int tpamd_linear_w8(const void *x_dev, const void *wq_dev, const void
     bool tiled = w8_direct_ok(K, ldx, ldw) ? M > 128 || (M > SKINNY_W8_SLAB && N * K >= (M <= 80 ? 22ll : 6ll) * 1000 * 1000)
                                            : M > 256 || (M > 128 && tiles128 >= 256);
     if (tuning().w8_tile != TUNE_UNSET) tiled = tuning().w8_tile > 0 && M > 16;
-    if (tiled && N % 4 == 0 && ldy % 4 == 0 && aligned(y_dev, 8) && (!bias_dev || aligned(bias_dev, 8)) && n_out <= 256)
-        return gemm_w8_dispatch(x_dev, wq_dev, scale_dev, outlier_idx_dev, w_out_dev, n_out, bias_dev, y_dev, M, N, K, ldx, ldw,
-                                ld_wout, ldy, dtype, act, s);
+    if (tiled && N % 4 == 0 && ldy % 4 == 0 && aligned(y_dev, 8) && (!bias_dev || aligned(bias_dev, 8)) && n_out <= 256) {
+        const int rc = gemm_w8_dispatch(x_dev, wq_dev, scale_dev, outlier_idx_dev, w_out_dev, n_out, bias_dev, y_dev, M, N, K, ldx, ldw,
+                                        ld_wout, ldy, dtype, act, s);
+        if (rc != TPAMD_ERR_UNSUPPORTED) return rc;  // else no scratch memory, and the slabs need none
+    }
     for (int64_t m0 = 0; m0 < M; m0 += SKINNY_W8_SLAB) {  // weights are re-streamed once per slab of 64 rows
         const int64_t mm = M - m0 < SKINNY_W8_SLAB ? M - m0 : SKINNY_W8_SLAB;
         int rc = skinny_dispatch(static_cast<const char *>(x_dev) + m0 * ldx * esz, wq_dev, nullptr, bias_dev, nullptr, 0, scale_dev,

@@ -2192,7 +2192,8 @@ void w8_tiling(int64_t M, int64_t N, int KT, int cus, int *rows, int *splits) {
 
 // int8 weights above the weight-streaming kernels' row count. x, wq 16-byte aligned, K and ldw multiples of 16, ldx of 8
 // (checked by the caller); N and ldy multiples of 4 and y 8-byte aligned for the packed stores. gemm_w8_kernel is left with K
-// that is no multiple of 64, and with streams that have no scratch memory for the outlier columns.
+// that is no multiple of 64, and with streams that have no scratch memory for the outlier columns. TPAMD_ERR_UNSUPPORTED, with nothing
+// launched: the stream has no scratch memory and the slabs are faster than what needs none.
 int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out,
                      const void *bias, void *y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout,
                      int64_t ldy, int dtype, int act, hipStream_t s) {
@@ -2219,8 +2220,11 @@ int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const voi
             return rows == 256 ? launch_w8_direct<TPAMD_F16, 16, 3>(p, q, cus, sp, s) : launch_w8_direct<TPAMD_F16, 8, 4>(p, q, cus, sp, s);
         };
         int rc = run(splits);
-        if (rc == TPAMD_ERR_UNSUPPORTED && splits > 1) rc = run(1);
-        if (rc != TPAMD_ERR_UNSUPPORTED) return rc;  // else no scratch memory for the outlier columns: the kernel that needs none
+        if (rc == TPAMD_ERR_UNSUPPORTED && splits > 1 && n_out > 0) rc = run(1);  // the partial tiles and the outlier columns may not fit a buffer together
+        if (rc != TPAMD_ERR_UNSUPPORTED) return rc;
+        // no scratch memory on this stream
+        if (tuning().w8_tile == TUNE_UNSET && w8_slabs_without_scratch(M, N, K, n_out > 0)) return rc;
+        if (n_out == 0) return run(1);
     }
     return dtype == TPAMD_BF16 ? launch_gemm_w8<TPAMD_BF16, 128, 128, 2, 2>(p, q, s) : launch_gemm_w8<TPAMD_F16, 128, 128, 2, 2>(p, q, s);
 }

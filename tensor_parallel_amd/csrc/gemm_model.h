@@ -38,4 +38,15 @@ inline double estimate_mid(int64_t M, int64_t N, int KT, int cus, bool swiglu, i
     return M <= 128 && best < stream ? stream : best;
 }
 
+// Rows, columns and K of an int8 Linear whose stream has no scratch memory (captured before its first use, or beyond the 32 buffers of a
+// device): whether slabs of 64 rows through the weight-streaming kernels take it, or a tiled kernel in one K range (without outlier columns
+// gemm_w8_direct_kernel, with them gemm_w8_kernel, which needs no packed ones). Predicted times, fitted to 288 timings of 18 matrices (512-65536
+// columns, K 1024-16384) at 65-400 rows with 0 and 41 outlier columns on such a stream; the choice is 0.4 % off the better one (geometric mean; at
+// worst 36 %, 32 us for 24). Tiles alone are 20 % off on the larger eight of them: 4096 x 5504 at 65 rows 60 us (79 with outliers) for 25 (26),
+// 1024 x 16384 at 128 rows 157 (217) for 69 (70).
+inline bool w8_slabs_without_scratch(int64_t M, int64_t N, int64_t K, bool outliers) {
+    const double k = static_cast<double>(K) / 4096.0;
+    return M / 64.0 * (5.0 + k * (5.5 + N / 512.0)) <= 6.0 + k * (outliers ? 53.0 : 36.0);
+}
+
 }  // namespace tpamd

@@ -29,3 +29,11 @@ def test_no_mid_tile_is_predicted_faster_than_its_weights_stream(tmp_path):
     assert len(rows) == 6 * 2 * 5
     for m, n, k, swiglu, us in rows:
         assert us * 5e6 >= n * k * (4 if swiglu else 2) * (1 - 1e-6), (m, n, k, swiglu, us)
+
+
+def test_slabs_are_taken_without_scratch_memory_where_they_measured_faster(tmp_path):
+    """Rows, columns, K, outliers, and which of the two was faster by 15 % or more on a stream without scratch memory."""
+    cases = [(65, 4096, 5504, 0, 1), (65, 4096, 5504, 1, 1), (129, 4096, 5504, 0, 1), (257, 4096, 5504, 0, 0), (400, 4096, 5504, 1, 0), (65, 8192, 4096, 0, 1),
+             (200, 8192, 4096, 1, 0), (65, 28672, 4096, 0, 0), (65, 28672, 4096, 1, 0), (256, 1024, 16384, 1, 1), (400, 1024, 16384, 0, 0), (100, 16384, 8192, 0, 0)]
+    rows = ask(tmp_path, "".join(f'printf("%d\\n", w8_slabs_without_scratch({m}, {n}, {k}, {o}) ? 1 : 0);\n' for m, n, k, o, _ in cases))
+    assert [r[0] for r in rows] == [c[4] for c in cases]

@@ -320,3 +320,45 @@ def test_tiled_kernel_edges(tune, dtype, rows, M, N, K, n_out, splits):
 # exact products of 16-bit and 8-bit values summed in fp32 and rounded once to 8 (bf16) bits or more: half a unit is 2^-9, and four
 # times that leaves room for the order of the sums
 RTOL_TILED = 8e-3
+
+
+@pytest.fixture
+def bare_stream(tune):
+    """A stream on which a capture finds no scratch memory: it has none of its own, and the device's spare is gone."""
+    tune("TPAMD_GEMM_TILE", "128")
+    tune("TPAMD_GEMM_SPLITK", "4")
+    x, w = torch.randn(256, 4096).bfloat16().to(DEV), torch.randn(512, 4096).bfloat16().to(DEV)
+    _native.linear(x, w)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for s in streams:
+        _native.release_scratch(DEV, s.cuda_stream)
+    with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=streams[0]):
+        _native.linear(x, w)  # takes the spare if there is one
+    tune("TPAMD_GEMM_TILE", "")
+    tune("TPAMD_GEMM_SPLITK", "")
+    return streams[1]
+
+
+@pytest.mark.parametrize("M,N,K,n_out", [(65, 4096, 5504, 41), (128, 8192, 4096, 1), (200, 1024, 2048, 9), (100, 520, 16384, 33), (100, 4096, 4096, 0), (65, 4096, 5504, 0)])
+def test_slabs_where_tiles_find_no_scratch_memory(bare_stream, tune, M, N, K, n_out):
+    """K ranges and packed outlier columns need scratch memory. Without it a few rows run in slabs of 64, not on tiles in one K range or on the slower
+    of the tiled kernels: the same bits as with the slabs asked for."""
+    x, wq, scale, cols, w_out = make_case(M, N, K, n_out, torch.float16, seed=3)
+    args = (x.to(DEV), torch.from_numpy(wq).to(DEV), torch.from_numpy(scale).to(DEV),
+            torch.from_numpy(cols.astype(np.int32)).to(DEV) if n_out else None, torch.from_numpy(w_out).half().to(DEV) if n_out else None)
+    outs, graphs = [], []
+    for tile in ("", "0"):
+        tune("TPAMD_W8_TILE", tile)
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1], stream=bare_stream):
+            outs.append(_native.linear_w8(*args))
+    assert _native.scratch_of_stream(DEV, bare_stream.cuda_stream) == (None, 0)
+    for _ in range(2):
+        for g, out in zip(graphs, outs):
+            out.zero_()
+            g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(*outs)
+    want = oq.linear_w8_f64(x.float().numpy(), wq, scale, cols, w_out)
+    torch.testing.assert_close(outs[0].double().cpu(), torch.from_numpy(want), rtol=2e-2, atol=2e-2 * 0.02 * math.sqrt(K + 400 * n_out))
