@@ -2214,7 +2214,7 @@ int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const voi
         int rows = 128, splits = 1;
         w8_tiling(M, N, static_cast<int>(K / 64), cus, &rows, &splits);
         if (tuning().w8_tile != TUNE_UNSET && tuning().w8_tile > 0) rows = tuning().w8_tile;
-        if (tuning().w8_tile_splits != TUNE_UNSET) splits = tuning().w8_tile_splits;
+        if (tuning().w8_tile_splits != TUNE_UNSET) splits = forced_splits(tuning().w8_tile_splits, static_cast<int>(K / 64), 16);
         auto run = [&](int sp) {
             if (dtype == TPAMD_BF16) return rows == 256 ? launch_w8_direct<TPAMD_BF16, 16, 3>(p, q, cus, sp, s) : launch_w8_direct<TPAMD_BF16, 8, 4>(p, q, cus, sp, s);
             return rows == 256 ? launch_w8_direct<TPAMD_F16, 16, 3>(p, q, cus, sp, s) : launch_w8_direct<TPAMD_F16, 8, 4>(p, q, cus, sp, s);

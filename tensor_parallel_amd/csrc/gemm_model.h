@@ -49,4 +49,10 @@ inline bool w8_slabs_without_scratch(int64_t M, int64_t N, int64_t K, bool outli
     return M / 64.0 * (5.0 + k * (5.5 + N / 512.0)) <= 6.0 + k * (outliers ? 53.0 : 36.0);
 }
 
+// A K split count that the environment asks for, as a launch takes it: 1 to `most`, none without a K tile.
+inline int forced_splits(int wanted, int KT, int most) {
+    const int top = KT < most ? KT : most;
+    return wanted > top ? top : wanted < 1 ? 1 : wanted;
+}
+
 }  // namespace tpamd

@@ -31,6 +31,13 @@ def test_no_mid_tile_is_predicted_faster_than_its_weights_stream(tmp_path):
         assert us * 5e6 >= n * k * (4 if swiglu else 2) * (1 - 1e-6), (m, n, k, swiglu, us)
 
 
+def test_a_forced_split_count_is_one_that_a_launch_takes(tmp_path):
+    """TPAMD_W8_TILE_SPLITS is taken as it stands in the environment: 0 was a division by zero in the launch."""
+    rows = ask(tmp_path, """
+    for (int wanted : {-7, 0, 1, 3, 16, 17, 1 << 30}) for (int kt : {2, 5, 64}) printf("%d %d %d\\n", wanted, kt, forced_splits(wanted, kt, 16));""")
+    assert [r[2] for r in rows] == [1, 1, 1, 1, 1, 1, 1, 1, 1, 2, 3, 3, 2, 5, 16, 2, 5, 16, 2, 5, 16]
+
+
 def test_slabs_are_taken_without_scratch_memory_where_they_measured_faster(tmp_path):
     """Rows, columns, K, outliers, and which of the two was faster by 15 % or more on a stream without scratch memory."""
     cases = [(65, 4096, 5504, 0, 1), (65, 4096, 5504, 1, 1), (129, 4096, 5504, 0, 1), (257, 4096, 5504, 0, 0), (400, 4096, 5504, 1, 0), (65, 8192, 4096, 0, 1),
