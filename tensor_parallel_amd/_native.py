@@ -12,6 +12,7 @@ from pathlib import Path
 from typing import Optional, Sequence
 
 import torch  # imported first on purpose: the library binds to the HIP runtime torch has loaded
+from torch.autograd import forward_ad
 from torch.utils._device import DeviceContext
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libtpamd.so"
@@ -203,7 +204,14 @@ def require_device(t: torch.Tensor, what: str) -> None:
 
 
 def on_hip(t: torch.Tensor) -> bool:
-    return t.device.type == "cuda"
+    return t.is_cuda
+
+
+_is_compiling = torch.compiler.is_compiling
+_is_tracing = torch._C._is_tracing
+_function_modes = torch._C._len_torch_function_stack
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_transform = torch._C._functorch.peek_interpreter_stack
 
 
 def plain_call(*tensors: torch.Tensor) -> bool:
@@ -213,11 +221,9 @@ def plain_call(*tensors: torch.Tensor) -> bool:
     for t in tensors:
         if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
             return False
-    for i in range(torch._C._len_torch_function_stack()):
-        if type(torch._C._get_function_stack_at(i)) is not DeviceContext:
-            return False
-    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0
-                or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0)
+    if _is_compiling() or _is_tracing() or forward_ad._current_level >= 0 or _transform() is not None or _dispatch_modes():
+        return False
+    return not _function_modes() or all(type(torch._C._get_function_stack_at(i)) is DeviceContext for i in range(_function_modes()))
 
 
 def stock_function(f, module: str, qualname: str, names: tuple, variables: tuple) -> bool:
@@ -504,7 +510,7 @@ def swiglu_up(x: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor) -> torch.Tens
 def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     """w * (x * rsqrt(mean(x^2) + eps)) over the last axis, sums in fp32, rounded as the two products of tensors of x's dtype."""
     require_device(x, "rms_norm")
-    if w.dtype != x.dtype or w.device != x.device or w.dim() != 1 or x.dim() == 0 or x.shape[-1] != w.shape[0]:
+    if w.dtype != x.dtype or w.get_device() != x.get_device() or w.dim() != 1 or x.dim() == 0 or x.shape[-1] != w.shape[0]:
         raise ValueError(f"rms_norm: x {tuple(x.shape)} {x.dtype} on {x.device} and w {tuple(w.shape)} {w.dtype} on {w.device} do not fit")
     x2 = _as_2d(x)
     w = w.contiguous()
@@ -522,8 +528,8 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 def add_rms_norm(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float) -> tuple:
     """(r + x, the RMS norm of that sum) of two tensors of one shape, dtype and device; arithmetic as in `rms_norm`."""
     require_device(x, "add_rms_norm")
-    if (r.shape != x.shape or r.dtype != x.dtype or r.device != x.device or w.dtype != x.dtype or w.device != x.device or w.dim() != 1 or x.dim() == 0
-            or x.shape[-1] != w.shape[0]):
+    if (r.shape != x.shape or r.dtype != x.dtype or r.get_device() != x.get_device() or w.dtype != x.dtype or w.get_device() != x.get_device() or w.dim() != 1
+            or x.dim() == 0 or x.shape[-1] != w.shape[0]):
         raise ValueError(f"add_rms_norm: r {tuple(r.shape)} {r.dtype} on {r.device}, x {tuple(x.shape)} {x.dtype} on {x.device} and w {tuple(w.shape)} "
                          f"{w.dtype} on {w.device} do not fit")
     x2, r2 = _as_2d(x), _as_2d(r)

@@ -119,7 +119,7 @@ _KERNEL_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 def _norm_kernel_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
     """What `tpamd_rms_norm` is made for; a promoting norm, one moved to another dtype (`.double()`) or with a weight that broadcasts is not."""
     return _native.plain_call(x, w) and x.dtype == w.dtype and w.dtype in _KERNEL_DTYPES and w.dim() == 1 and x.dim() > 0 and x.shape[-1] == w.shape[0] \
-        and _native.on_hip(x) and x.device == w.device
+        and _native.on_hip(x) and x.get_device() == w.get_device()
 
 
 def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
@@ -128,7 +128,7 @@ def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
     # Linear's), keep the module's own forward
     if own is not self._tp_replaced or not _norm_kernel_takes(hidden_states, w) or torch.is_grad_enabled() and (hidden_states.requires_grad or w.requires_grad):
         return own(self, hidden_states)
-    return _native.rms_norm(hidden_states.detach(), w.detach(), self.variance_epsilon)
+    return _native.rms_norm(hidden_states, w, self.variance_epsilon)
 
 
 def is_llama_layer(module: nn.Module) -> bool:
@@ -149,7 +149,7 @@ def _llama_layer_forward(self, hidden_states: torch.Tensor, *args, **kwargs) -> 
             or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or torch.is_grad_enabled() or not _norm_kernel_takes(hidden_states, norm.weight)):
         return own(self, hidden_states, *args, **kwargs)
     attended, _ = self.self_attn(hidden_states=self.input_layernorm(hidden_states), **{**_LAYER_DEFAULTS, **kwargs})
-    if _norm_kernel_takes(attended, norm.weight) and hidden_states.shape == attended.shape:
+    if type(attended) is torch.Tensor and attended.dtype == hidden_states.dtype and attended.shape == hidden_states.shape and attended.get_device() == hidden_states.get_device():
         total, normed = _native.add_rms_norm(hidden_states, attended, norm.weight, norm.variance_epsilon)
     else:
         total = hidden_states + attended
