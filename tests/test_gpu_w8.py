@@ -322,22 +322,29 @@ def test_tiled_kernel_edges(tune, dtype, rows, M, N, K, n_out, splits):
 RTOL_TILED = 8e-3
 
 
-@pytest.fixture
-def bare_stream(tune):
-    """A stream on which a capture finds no scratch memory: it has none of its own, and the device's spare is gone."""
-    tune("TPAMD_GEMM_TILE", "128")
-    tune("TPAMD_GEMM_SPLITK", "4")
+@pytest.fixture(scope="module")
+def bare_stream():
+    """A stream on which a capture finds no scratch memory: it has none of its own, and the device's spare is gone. Afterwards its neighbour has
+    given the spare back and torch's pool of 32 streams is where it was, so that other tests meet the streams they would have met."""
     x, w = torch.randn(256, 4096).bfloat16().to(DEV), torch.randn(512, 4096).bfloat16().to(DEV)
-    _native.linear(x, w)
+    with pytest.MonkeyPatch.context() as m:
+        m.setenv("TPAMD_GEMM_TILE", "128")
+        m.setenv("TPAMD_GEMM_SPLITK", "4")
+        _native.reload_tuning()
+        _native.linear(x, w)
+        torch.cuda.synchronize()
+        streams = [torch.cuda.Stream() for _ in range(32)][:2]
+        had = [_native.scratch_of_stream(DEV, s.cuda_stream)[0] is not None for s in streams]
+        for s in streams:
+            _native.release_scratch(DEV, s.cuda_stream)
+        with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=streams[0]):
+            _native.linear(x, w)  # takes the spare if there is one
+    _native.reload_tuning()
+    yield streams[1]
     torch.cuda.synchronize()
-    streams = [torch.cuda.Stream() for _ in range(2)]
-    for s in streams:
-        _native.release_scratch(DEV, s.cuda_stream)
-    with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=streams[0]):
-        _native.linear(x, w)  # takes the spare if there is one
-    tune("TPAMD_GEMM_TILE", "")
-    tune("TPAMD_GEMM_SPLITK", "")
-    return streams[1]
+    for s, before in zip(streams, had):
+        if not before:
+            _native.release_scratch(DEV, s.cuda_stream)
 
 
 @pytest.mark.parametrize("M,N,K,n_out", [(65, 4096, 5504, 41), (128, 8192, 4096, 1), (200, 1024, 2048, 9), (100, 520, 16384, 33), (100, 4096, 4096, 0), (65, 4096, 5504, 0)])
