@@ -310,16 +310,17 @@ def test_tiled_kernel_edges(tune, dtype, rows, M, N, K, n_out, splits):
             torch.from_numpy(w_out).to(dtype).to(DEV) if n_out else None)
     bias = (torch.randn(N, generator=torch.Generator().manual_seed(5)) * 0.1).to(dtype)
     want = oq.linear_w8_f64(x.float().numpy(), wq, scale, cols, w_out)
-    atol = RTOL_TILED * 0.02 * math.sqrt(K + 400 * n_out)
-    torch.testing.assert_close(_native.linear_w8(*args).double().cpu(), torch.from_numpy(want), rtol=RTOL_TILED, atol=atol)
+    rtol = RTOL_TILED[dtype]
+    atol = rtol * 0.02 * math.sqrt(K + 400 * n_out)
+    torch.testing.assert_close(_native.linear_w8(*args).double().cpu(), torch.from_numpy(want), rtol=rtol, atol=atol)
     want = torch.nn.functional.gelu(torch.from_numpy(want) + bias.double())
     got = _native.linear_w8(*args, bias=bias.to(DEV), act=_native.ACT_GELU)
-    torch.testing.assert_close(got.double().cpu(), want, rtol=RTOL_TILED, atol=atol)
+    torch.testing.assert_close(got.double().cpu(), want, rtol=rtol, atol=atol)
 
 
-# exact products of 16-bit and 8-bit values summed in fp32 and rounded once to 8 (bf16) bits or more: half a unit is 2^-9, and four
-# times that leaves room for the order of the sums
-RTOL_TILED = 8e-3
+# exact products of 16-bit and 8-bit values summed in fp32 and rounded once to the dtype: half a unit is 2^-9 of the value in bf16 (8 bits) and 2^-12 in
+# fp16 (11 bits), and four times that leaves room for the order of the sums (at most 1280 + 256 terms: 1.3 K^0.5 2^-24 of their size, 3e-6)
+RTOL_TILED = {torch.bfloat16: 4 * 2.0 ** -9, torch.float16: 4 * 2.0 ** -12}
 
 
 @pytest.fixture(scope="module")
