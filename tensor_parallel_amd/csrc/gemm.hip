@@ -1020,11 +1020,12 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(GemmParams p) {
     }
 }
 
-// ---- int8 weights at prefill sizes: dequantised on the way into LDS ---------------------------------------------------
+// ---- int8 weights at prefill sizes -------------------------------------------------------------------------------------
 // y = act(scale[n] * (x . wq^T) + x[:, outliers] . w_out^T + bias) for more rows than the weight-streaming kernels
-// take. Same tiling, staging and MFMA as gemm_kernel; a K tile of the weight is 64 bytes of every row (four 16-byte
-// chunks of 16 int8), converted to the activation dtype in registers (exact) and stored as the 128 bytes the MFMA
-// fragments read. After the last K tile the sums are multiplied by the rows' scales, and the outlier columns follow
+// take: gemm_w8_direct_kernel (below) where K % 64 == 0 and the outlier columns find scratch memory, gemm_w8_kernel
+// elsewhere. It has the tiling, staging and MFMA of gemm_kernel; a K tile of the weight is 64 bytes of every row (four
+// 16-byte chunks of 16 int8), converted to the activation dtype in registers (exact) and stored as the 128 bytes the
+// MFMA fragments read. After the last K tile the sums are multiplied by the rows' scales, and the outlier columns follow
 // as up to 4 further K tiles of 64 (x gathered through outlier_idx, w_out read as it lies, both element by element:
 // a percent of the work) into the same accumulators.
 struct W8Extra {
@@ -1231,30 +1232,6 @@ int launch_gemm_w8(GemmParams p, const W8Extra &q, hipStream_t s) {
     return TPAMD_OK;
 }
 
-// gemm_w8_direct_kernel: the tiled int8 kernel for K % 64 == 0. 16 * TMX x-rows by 256 w-rows per block, 4 wavefronts side by
-// side along the columns (each all x rows by 64 w rows), K tiles of 64 in NS LDS stages.
-//
-// Bound: the matrix pipe (M >= 512), with one vector instruction per weight (bf16: 1.5) for the conversion running beside it:
-// 16384 x 8192 at 1024 rows 316 -> 228 us (1.21 PFLOP/s; the same product on f16 weights takes 215), 8192 x 16384 479 -> 232,
-// 4608 x 8192 150 -> 98, 8192 x 4096 133 -> 69; at 200 rows 192 -> 80, 191 -> 79, 92 -> 40 and 95 -> 38 us (before: a tiled kernel
-// that staged the weights through registers, slabs of 64 rows below 257 rows). What the
-// split between the wavefronts is for: every weight of the block is converted by exactly one wavefront (two wavefronts per
-// w row would double the conversions), right before it is multiplied, so that the weights cross LDS as bytes and reach
-// it without passing through registers (global->LDS loads, like x). A weight fragment read of 16 bytes holds both k steps of
-// a lane: lane group lq owns bytes 16 lq ... 16 lq + 15 of the 64 of a K tile, eight per step, and x is read in the
-// same order (its 16-byte chunk 2 lq + kk), which permutes k inside a tile alike for both operands.
-//   step A (kk 0)  MFMAs on weight buffer 0; converts the upper halves of the weight bytes into buffer 1
-//   step B (kk 1)  MFMAs on weight buffer 1; a few MFMAs in, the barrier: tile g+1 has landed ((NS-2) younger tiles in flight),
-//                  the stage of tile g is read out; then the weight bytes of tile g+1 are read and their lower halves
-//                  converted into buffer 0, and tile g+NS is requested into the stage of tile g
-// x fragments need no second buffer: the four MFMAs that use one done, it is read again for the next step, a whole step ahead
-// of its use (with two buffers the 256-row tile ran out of registers and moved 32 of them to AGPRs and back per K tile).
-// LDS: x as in gemm_direct_kernel; w in blocks of 16 rows x 64 bytes (1 KiB, one wavefront-wide load), chunk c of row r in slot
-// c ^ ((r / 2) % 4) ^ (r / 8): 8 rows that follow one another, and rows 4 apart, hit different banks.
-// After the K loop the sums are multiplied by the rows' scales; the outlier columns (packed by
-// w8_pack_outliers_kernel, zeros up to a multiple of 32) follow in steps of 32 into the same accumulators.
-// SPLIT: unit u is tile u % tiles, K range u / tiles; the scaled sums (range 0: with the outlier columns) go to p.ws as
-// 128 x 128 tiles for splitk_finish_kernel.
 // cvt_i8x4 one instruction at a time: step<0>, step<1>, ... step<OPS - 1> leave the four converted weights in lo, hi. The
 // conversions take their byte through the sub-dword selects (f16: 4 instructions where bias, permute and subtract took 5; bf16: 6
 // where they took 11).
@@ -1288,6 +1265,31 @@ struct W8Convert<TPAMD_BF16> {
     }
 };
 
+// gemm_w8_direct_kernel: the tiled int8 kernel for K % 64 == 0. 16 * TMX x-rows by 256 w-rows per block, 4 wavefronts side by
+// side along the columns (each all x rows by 64 w rows), K tiles of 64 in NS LDS stages.
+//
+// Bound: the matrix pipe (M >= 512; by the SQ counters busy 65-70 % of a launch without K ranges, 57 % with a GELU in its epilogue; waits for LDS 4 %),
+// with one vector instruction per weight (bf16: 1.5) for the conversion running beside it:
+// 16384 x 8192 at 1024 rows 316 -> 228 us (1.21 PFLOP/s; the same product on f16 weights takes 215), 8192 x 16384 479 -> 232,
+// 4608 x 8192 150 -> 98, 8192 x 4096 133 -> 69; at 200 rows 192 -> 80, 191 -> 79, 92 -> 40 and 95 -> 38 us (before: a tiled kernel
+// that staged the weights through registers, slabs of 64 rows below 257 rows). What the
+// split between the wavefronts is for: every weight of the block is converted by exactly one wavefront (two wavefronts per
+// w row would double the conversions), right before it is multiplied, so that the weights cross LDS as bytes and reach
+// it without passing through registers (global->LDS loads, like x). A weight fragment read of 16 bytes holds both k steps of
+// a lane: lane group lq owns bytes 16 lq ... 16 lq + 15 of the 64 of a K tile, eight per step, and x is read in the
+// same order (its 16-byte chunk 2 lq + kk), which permutes k inside a tile alike for both operands.
+//   step A (kk 0)  MFMAs on weight buffer 0; converts the upper halves of the weight bytes into buffer 1
+//   step B (kk 1)  MFMAs on weight buffer 1; a few MFMAs in, the barrier: tile g+1 has landed ((NS-2) younger tiles in flight),
+//                  the stage of tile g is read out; then the weight bytes of tile g+1 are read and their lower halves
+//                  converted into buffer 0, and tile g+NS is requested into the stage of tile g
+// x fragments need no second buffer: the four MFMAs that use one done, it is read again for the next step, a whole step ahead
+// of its use (with two buffers the 256-row tile ran out of registers and moved 32 of them to AGPRs and back per K tile).
+// LDS: x as in gemm_direct_kernel; w in blocks of 16 rows x 64 bytes (1 KiB, one wavefront-wide load), chunk c of row r in slot
+// c ^ ((r / 2) % 4) ^ (r / 8): 8 rows that follow one another, and rows 4 apart, hit different banks.
+// After the K loop the sums are multiplied by the rows' scales; the outlier columns (packed by
+// w8_pack_outliers_kernel, zeros up to a multiple of 32) follow in steps of 32 into the same accumulators.
+// SPLIT: unit u is tile u % tiles, K range u / tiles; the scaled sums (range 0: with the outlier columns) go to p.ws as
+// 128 x 128 tiles for splitk_finish_kernel.
 template <int DT, int TMX, int NS, bool SPLIT>
 __global__ __launch_bounds__(256) void gemm_w8_direct_kernel(GemmParams p, W8Extra q) {
     constexpr int BM = 16 * TMX, BN = 256;

@@ -14,8 +14,10 @@ namespace {
 //   step A  MFMAs of k 0-31; behind the first TNX of them the reads of the w fragments of k 32-63, behind each row of MFMAs its x fragment
 //   step B  MFMAs of k 32-63; after one row of them the barrier: tile g + 1 has landed (NS - 2 younger tiles in flight) and the stage of
 //           tile g is read out; then the fragments of tile g + 1, and tile g + NS into the stage of tile g, spread over the MFMAs
-// Bound: the matrix pipe and LDS together. A K tile of 192 x 192 takes 0.64 us on an idle chip and 0.83 in a full round, where its MFMAs
-// need 0.48 at 2.4 GHz and its 144 KB through LDS as much (128 bytes per clock); 192 x 256, on two stages, 0.92-1.23 (0.64 of MFMAs).
+// Bound: the matrix pipe at the clock its power leaves (1.8-2.0 GHz), the start and the epilogue of a launch, and CUs without a tile. By the SQ counters
+// of 2103 rows in fp16 the pipes are busy 54 % of a launch of 242 tiles of 192 x 192 and 58 % of one of 473 gated tiles of 192 x 256 (two rounds); the
+// fragment reads keep LDS busy 15-20 % of it and wavefronts wait for LDS 4-5 % of their time. A K tile of 192 x 192 takes 0.64 us on an idle
+// chip and 0.83 in a full round, where its MFMAs need 0.48 at 2.4 GHz; 192 x 256, on two stages, 0.92-1.23 (0.64).
 template <int DT, int MODE, int TMX, int TNX, int NS>
 __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
     constexpr int BM = 32 * TMX, BN = 32 * TNX, BN_OUT = MODE == MODE_SWIGLU ? BN / 2 : BN;
