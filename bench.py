@@ -772,7 +772,7 @@ def w8_decode(torch, _native, dev, m=1, graph=True) -> dict:
     if not graph:  # prefill-sized: bound by the matrix pipe, not by the weight bytes
         flops = 4.0 * m * d * f
         return {"us_per_step": us, "tokens_per_s": m * 1e6 / us, "TFLOPs": flops / us / 1e6, "mfma_frac": flops / us / 1e6 / PEAK_BF16_TFLOPS,
-                "algorithmic_flops": flops, "step": "int8 up + GELU + down of the Falcon-40B MLP shard, weights dequantised on their way into LDS"}
+                "algorithmic_flops": flops, "step": "int8 up + GELU + down of the Falcon-40B MLP shard, weights converted to the activation dtype between the MFMAs"}
     try:
         gus = _graph_us(torch, fn, per=12)
         entry["graph"] = {"us_per_step": gus, "tokens_per_s": m * 1e6 / gus, "GBps": by / gus / 1e3, "hbm_frac": by / gus / 1e3 / PEAK_HBM_GBS}

@@ -80,7 +80,7 @@ int tpamd_scratch_query(void *stream, void **ptr_out, uint64_t *bytes_out);
 /* Gives back the scratch buffer of `stream` on the current device (no-op when it has none): call it before destroying a
  * stream that ran K-split work, with none of that work captured in a graph that will still be replayed. The stream is
  * synchronised, the buffer freed, and its slot can serve another stream. Without it a buffer lives until the process
- * ends: at most 33 per device (32 streams and the spare), 64 MiB each on a 256-CU part, i.e. up to 2.1 GiB per device for
+ * ends: at most 33 per device (32 streams and the spare), 68 MiB each on a 256-CU part, i.e. up to 2.2 GiB per device for
  * a process that keeps creating streams. No counterpart in the reference. */
 int tpamd_scratch_release(void *stream);
 
@@ -197,7 +197,7 @@ int tpamd_linear_add(const void *x_dev, const void *w_dev, const void *bias_dev,
  * result, bit for bit, as tpamd_linear; the call allocates nothing (no hipMalloc, no hipFree), also at its first use
  * and under stream capture. Where tpamd_linear would put the fp32 partial tiles of a K split into its stream's
  * scratch buffer, this entry point puts them into a fixed array of tpamd_noalloc_scratch_bytes() = 64 MiB that every
- * GPU the library is loaded on holds until the process ends: the size of a stream's buffer on a 256-CU part, so every
+ * GPU the library is loaded on holds until the process ends: the room for partial tiles in a stream's buffer on a 256-CU part, so every
  * K split the library picks by itself there fits. A K split that needs more (a part with more CUs, a split forced
  * through the TPAMD_* variables; the message names the size) is refused with TPAMD_ERR_UNSUPPORTED and nothing is
  * launched; tpamd_linear takes such shapes.
@@ -323,7 +323,8 @@ int tpamd_causal_mask(const int64_t *q_offset_dev, int64_t kv_offset, int64_t ro
  * (its README points to LLM.int8 notebooks); defined here in closed form.
  * Up to 64 rows (up to 128 on small matrices, once per 64 rows) the weights are streamed by HBM-bound kernels; above that
  * they go through the matrix pipe once, converted to `dtype` (exactly) in front of it; K % 64 == 0 takes the faster of two
- * such kernels.
+ * such kernels, whose K ranges and outlier columns need the stream's scratch buffer: a stream without one runs slabs of 64 rows
+ * or the other kernel, whichever is faster.
  * Requirements: dtype is F16 or BF16; K % 16 == 0; ldw (int8 elements) % 16 == 0. */
 int tpamd_linear_w8(const void *x_dev, const void *wq_dev, const void *scale_dev, const void *outlier_idx_dev,
                     const void *w_out_dev, int64_t n_out, const void *bias_dev, void *y_dev, int64_t M, int64_t N,

@@ -75,7 +75,7 @@ std::mutex &splitk_mutex(int dev);
 int splitk_scratch(int dev, hipStream_t stream, size_t need, size_t reserve, void **out);
 // While one of these lives on a host thread, splitk_scratch() on that thread hands out the library's fixed array and
 // allocates nothing.
-// 64 MiB: what a stream's buffer holds on a 256-CU part (4 * CUs * 64 KiB), so every K split the cost models pick there fits.
+// 64 MiB: the partial tiles a stream's buffer has room for on a 256-CU part (4 * CUs * 64 KiB), so every K split the cost models pick there fits.
 constexpr size_t TPAMD_NOALLOC_SCRATCH_BYTES = static_cast<size_t>(64) << 20;
 bool static_scratch_active();
 int static_scratch(int dev, size_t need, void **out);
