@@ -204,8 +204,13 @@ def _fused_class(base: type, forward, doc: str) -> type:
         def reduce_ex(self, protocol):  # the class is made here and has no name to be found by: pickle what makes it
             return (_new_fused, (base, forward, doc), *super(cls, self).__reduce_ex__(protocol)[2:])
 
+        def prepare_scriptable(self):  # TorchScript compiles the module's own forward
+            own = base.__new__(base)
+            own.__dict__.update(self.__dict__)
+            return own
+
         name = base.__name__ if forward is _llama_layer_forward else "Shard" + base.__name__
-        cls = type(name, (base,), {"forward": forward, "__doc__": doc, "__reduce_ex__": reduce_ex, "_tp_base": base,
+        cls = type(name, (base,), {"forward": forward, "__doc__": doc, "__reduce_ex__": reduce_ex, "__prepare_scriptable__": prepare_scriptable, "_tp_base": base,
                                 "_tp_replaced": staticmethod(base.forward if _takes_stand_in(base, forward) else None)})
         cls = _fused_classes.setdefault((base, forward), cls)
     return cls

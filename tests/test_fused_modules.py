@@ -119,6 +119,14 @@ def test_what_follows_the_torch_calls_sees_the_modules_own(kernels):
     assert not kernels
 
 
+def test_a_norm_can_be_scripted(kernels):
+    own, model, x = llama(), sharded(), torch.randn(2, 5, 32)
+    with torch.no_grad():
+        assert torch.equal(torch.jit.script(model.norm)(x), own.norm(x)) and not kernels
+        model.norm(x)
+    assert kernels == ["rms_norm"]
+
+
 class _Doubled(torch.overrides.TorchFunctionMode):
     def __torch_function__(self, func, types, args=(), kwargs=None):
         out = func(*args, **(kwargs or {}))
