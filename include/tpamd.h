@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define TPAMD_ABI_VERSION 5
+#define TPAMD_ABI_VERSION 6
 
 typedef enum tpamd_status {
     TPAMD_OK = 0,
@@ -311,6 +311,40 @@ int tpamd_rope_tables(const void *inv_freq_dev, int freq_dtype, const int64_t *p
  * dimension ldx, r with ldr, sum and y with ldy; sum and y overlap neither each other nor an input. */
 int tpamd_add_rms_norm(const void *x_dev, const void *r_dev, const void *w_dev, void *sum_dev, void *y_dev, int64_t rows, int64_t D,
                        int64_t ldx, int64_t ldr, int64_t ldy, float eps, int dtype, void *stream);
+
+/* ---- one call for the shards of several ranks that live on this device -----------------------------------------------------------
+ * The reference runs W ranks side by side, one thread each (src/tensor_parallel/tensor_parallel.py:237-287); where they share a device
+ * their equal calls can be handed in together. Each entry point below makes the calls of the entry point it is named after for n ranks:
+ * operand i of every array is rank i's, all dimensions, leading dimensions and flags are shared, results are those of n single calls
+ * (the choice of a kernel sees the work of both ranks of a launch, so sums may be added up in another order). Two ranks go into one
+ * launch wherever the kernels that take the shape can: a rank's share of a decode step is too little work to fill the device and its
+ * launches follow one another. Outputs of different ranks overlap neither each other nor an input. */
+int tpamd_linear_ranks(int n, const void *const *x_dev, const void *const *w_dev, const void *const *bias_dev /* NULL: none */,
+                       void *const *y_dev, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, int act,
+                       void *stream);
+int tpamd_swiglu_up_ranks(int n, const void *const *x_dev, const void *const *wg_dev, const void *const *wu_dev, void *const *h_dev,
+                          int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldh, int dtype, void *stream);
+int tpamd_rms_norm_ranks(int n, const void *const *x_dev, const void *const *w_dev, void *const *y_dev, int64_t rows, int64_t D,
+                         int64_t ldx, int64_t ldy, float eps, int dtype, void *stream);
+int tpamd_add_rms_norm_ranks(int n, const void *const *x_dev, const void *const *r_dev, const void *const *w_dev, void *const *sum_dev,
+                             void *const *y_dev, int64_t rows, int64_t D, int64_t ldx, int64_t ldr, int64_t ldy, float eps, int dtype,
+                             void *stream);
+
+typedef struct {
+    const void *q, *k, *v, *cos, *sin;
+    void *k_cache, *v_cache, *out;
+    const int64_t *pos; /* the count on the device, or NULL in every rank: `pos0` positions are cached */
+} tpamd_decode_rank;
+/* tpamd_attention_decode_rope, or tpamd_attention_decode_rope_devpos where `pos` is set. */
+int tpamd_attention_decode_rope_ranks(int n, const tpamd_decode_rank *ranks, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t pos0,
+                                      int64_t cache_len, const int64_t *strides, float scale, int dtype, void *stream);
+
+typedef struct {
+    const void *x, *wq, *scale, *outlier_idx, *w_out, *bias;
+    void *y;
+} tpamd_w8_rank;
+int tpamd_linear_w8_ranks(int n, const tpamd_w8_rank *ranks, int64_t n_out, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                          int64_t ld_wout, int64_t ldy, int dtype, int act, void *stream);
 
 /* Causal mask of `rows` queries on `cols` keys, a byte each (1: seen): mask[i][j] = (kv_offset + j <= *q_offset_dev + i), the
  * queries' first position (int64) read from the device, mask [rows, cols] contiguous. */

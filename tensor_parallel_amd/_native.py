@@ -45,9 +45,15 @@ EXPORTS = (
     "tpamd_rope_append",
     "tpamd_attention_decode_rope",
     "tpamd_attention_decode_rope_devpos",
+    "tpamd_linear_ranks",
+    "tpamd_swiglu_up_ranks",
+    "tpamd_rms_norm_ranks",
+    "tpamd_add_rms_norm_ranks",
+    "tpamd_attention_decode_rope_ranks",
+    "tpamd_linear_w8_ranks",
 )
 
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 BF16, F16, F32 = 0, 1, 2
 ACCUM_STEPWISE, ACCUM_F32 = 0, 1
@@ -80,6 +86,14 @@ class TransposeJob(ctypes.Structure):
         ("src_pitch", ctypes.c_uint64),
         ("dst_pitch", ctypes.c_uint64),
     ]
+
+
+class DecodeRank(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in ("q", "k", "v", "cos", "sin", "k_cache", "v_cache", "out", "pos")]
+
+
+class W8Rank(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in ("x", "wq", "scale", "outlier_idx", "w_out", "bias", "y")]
 
 
 _lib: Optional[ctypes.CDLL] = None
@@ -141,6 +155,19 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_rope_tables.argtypes = [vp, ci, vp, i64, i64, i64, i64, i64, c.c_float, vp, vp, ci, vp]
     lib.tpamd_causal_mask.restype = ci
     lib.tpamd_causal_mask.argtypes = [vp, i64, i64, i64, vp, vp]
+    pp = c.POINTER(vp)
+    lib.tpamd_linear_ranks.restype = ci
+    lib.tpamd_linear_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, i64, i64, ci, ci, vp]
+    lib.tpamd_swiglu_up_ranks.restype = ci
+    lib.tpamd_swiglu_up_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, i64, i64, ci, vp]
+    lib.tpamd_rms_norm_ranks.restype = ci
+    lib.tpamd_rms_norm_ranks.argtypes = [ci, pp, pp, pp, i64, i64, i64, i64, c.c_float, ci, vp]
+    lib.tpamd_add_rms_norm_ranks.restype = ci
+    lib.tpamd_add_rms_norm_ranks.argtypes = [ci, pp, pp, pp, pp, pp, i64, i64, i64, i64, i64, c.c_float, ci, vp]
+    lib.tpamd_attention_decode_rope_ranks.restype = ci
+    lib.tpamd_attention_decode_rope_ranks.argtypes = [ci, c.POINTER(DecodeRank), i64, i64, i64, i64, i64, i64, c.POINTER(i64), c.c_float, ci, vp]
+    lib.tpamd_linear_w8_ranks.restype = ci
+    lib.tpamd_linear_w8_ranks.argtypes = [ci, c.POINTER(W8Rank), i64, i64, i64, i64, i64, i64, i64, i64, ci, ci, vp]
     lib.tpamd_linear_w8.restype = ci
     lib.tpamd_linear_w8.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, i64, i64, i64, i64, i64, i64, i64, ci, ci, vp]
 
@@ -438,11 +465,7 @@ def release_scratch(device: torch.device, stream_ptr: Optional[int] = None) -> N
         _check(lib().tpamd_scratch_release(ctypes.c_void_p(stream_ptr)), "tpamd_scratch_release")
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act: int = ACT_NONE,
-           addend: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """y = act(x @ w.T + bias) with w of shape [N, K]; leading dimensions of x are kept. With `addend` (same shape
-    and dtype as y): y = (that result, rounded to the dtype) + addend, one step of the sum over rank partials, in the
-    same launch. `out` (contiguous, may be `addend`) receives the result."""
+def _check_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> None:
     require_device(x, "linear")
     require_device(w, "linear")
     if x.dtype != w.dtype:
@@ -451,10 +474,45 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
         raise ValueError(f"linear: x has {x.shape[-1]} input features, w is {tuple(w.shape)}")
     if w.device != x.device:
         raise ValueError(f"linear: x is on {x.device}, w on {w.device}")
+    if bias is not None and (bias.shape != (w.shape[0],) or bias.dtype != x.dtype or bias.device != x.device):
+        raise ValueError("linear: bias must have shape [N], the dtype of x and live on its device")
+
+
+# The *_ranks functions take the operands of several ranks whose tensors agree in shape, strides, dtype and device (together.GreenTurn.meet compares
+# them): what holds for the first rank's holds for all.
+_pointer_arrays = [ctypes.c_void_p * n for n in range(9)]
+
+
+def _pointers(tensors: Sequence[torch.Tensor]):
+    n = len(tensors)
+    return (_pointer_arrays[n] if n < len(_pointer_arrays) else ctypes.c_void_p * n)(*[t.data_ptr() for t in tensors])
+
+
+def linear_ranks(calls: Sequence[tuple]) -> list:
+    """`linear(x, w, bias)` for the (x, w, bias) of several ranks."""
+    x, w, bias = calls[0]
+    _check_linear(x, w, bias)
+    xs, ws = [_as_2d(c[0]) for c in calls], [_as_2d(c[1]) for c in calls]
+    (M, K), N = xs[0].shape, w.shape[0]
+    ys = [torch.empty((M, N), dtype=x.dtype, device=x.device) for _ in calls]
+    bs = None if bias is None else [c[2].contiguous() for c in calls]
+    with _on_device(x.device):
+        _check(
+            lib().tpamd_linear_ranks(len(calls), _pointers(xs), _pointers(ws), None if bs is None else _pointers(bs), _pointers(ys), M, N, K,
+                                     _ld(xs[0]), _ld(ws[0]), N, dtype_code(x.dtype), ACT_NONE, ctypes.c_void_p(current_stream_ptr(x.device))),
+            "tpamd_linear_ranks",
+        )
+    return [y.view(*x.shape[:-1], N) for y in ys]
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act: int = ACT_NONE,
+           addend: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """y = act(x @ w.T + bias) with w of shape [N, K]; leading dimensions of x are kept. With `addend` (same shape
+    and dtype as y): y = (that result, rounded to the dtype) + addend, one step of the sum over rank partials, in the
+    same launch. `out` (contiguous, may be `addend`) receives the result."""
+    _check_linear(x, w, bias)
     N, K = w.shape
     M = x.numel() // K if K else 0
-    if bias is not None and (bias.shape != (N,) or bias.dtype != x.dtype or bias.device != x.device):
-        raise ValueError("linear: bias must have shape [N], the dtype of x and live on its device")
     if addend is not None and (addend.dtype != x.dtype or addend.device != x.device or addend.numel() != M * N
                                or addend.shape[-1] != N):
         raise ValueError("linear: addend must have the shape, dtype and device of the result")
@@ -484,13 +542,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
 
 def swiglu_up(x: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor) -> torch.Tensor:
     """h = silu(x @ wg.T) * (x @ wu.T)."""
-    require_device(x, "swiglu_up")
-    if not (x.dtype == wg.dtype == wu.dtype):
-        raise TypeError("swiglu_up: x, wg, wu must share one dtype")
-    if wg.dim() != 2 or wg.shape != wu.shape or x.shape[-1] != wg.shape[1]:
-        raise ValueError("swiglu_up: shape mismatch")
-    if wg.device != x.device or wu.device != x.device:
-        raise ValueError(f"swiglu_up: x is on {x.device}, wg on {wg.device}, wu on {wu.device}")
+    _check_swiglu_up(x, wg, wu)
     x2, g2, u2 = _as_2d(x), _as_2d(wg), _as_2d(wu)
     if _ld(g2) != _ld(u2):
         u2 = u2.contiguous()
@@ -507,43 +559,81 @@ def swiglu_up(x: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor) -> torch.Tens
     return h.view(*x.shape[:-1], N)
 
 
+def _check_swiglu_up(x: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor) -> None:
+    require_device(x, "swiglu_up")
+    if not (x.dtype == wg.dtype == wu.dtype):
+        raise TypeError("swiglu_up: x, wg, wu must share one dtype")
+    if wg.dim() != 2 or wg.shape != wu.shape or x.shape[-1] != wg.shape[1]:
+        raise ValueError("swiglu_up: shape mismatch")
+    if wg.device != x.device or wu.device != x.device:
+        raise ValueError(f"swiglu_up: x is on {x.device}, wg on {wg.device}, wu on {wu.device}")
+
+
+def swiglu_up_ranks(calls: Sequence[tuple]) -> list:
+    """`swiglu_up(x, wg, wu)` for the operands of several ranks."""
+    x, wg, wu = calls[0]
+    _check_swiglu_up(x, wg, wu)
+    xs, gs, us = ([_as_2d(c[i]) for c in calls] for i in range(3))
+    if _ld(gs[0]) != _ld(us[0]):
+        gs, us = [g.contiguous() for g in gs], [u.contiguous() for u in us]
+    (M, K), N = xs[0].shape, wg.shape[0]
+    hs = [torch.empty((M, N), dtype=x.dtype, device=x.device) for _ in calls]
+    with _on_device(x.device):
+        _check(
+            lib().tpamd_swiglu_up_ranks(len(calls), _pointers(xs), _pointers(gs), _pointers(us), _pointers(hs), M, N, K, _ld(xs[0]), _ld(gs[0]), N,
+                                        dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device))),
+            "tpamd_swiglu_up_ranks",
+        )
+    return [h.view(*x.shape[:-1], N) for h in hs]
+
+
 def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     """w * (x * rsqrt(mean(x^2) + eps)) over the last axis, sums in fp32, rounded as the two products of tensors of x's dtype."""
+    return rms_norm_ranks([(x, w, eps)])[0]
+
+
+def rms_norm_ranks(calls: Sequence[tuple]) -> list:
+    """`rms_norm(x, w, eps)` for the operands of several ranks (with one eps)."""
+    x, w, eps = calls[0]
     require_device(x, "rms_norm")
     if w.dtype != x.dtype or w.get_device() != x.get_device() or w.dim() != 1 or x.dim() == 0 or x.shape[-1] != w.shape[0]:
         raise ValueError(f"rms_norm: x {tuple(x.shape)} {x.dtype} on {x.device} and w {tuple(w.shape)} {w.dtype} on {w.device} do not fit")
-    x2 = _as_2d(x)
-    w = w.contiguous()
-    rows, D = x2.shape
-    y = torch.empty((rows, D), dtype=x.dtype, device=x.device)
+    xs, ws = [_as_2d(c[0]) for c in calls], [c[1].contiguous() for c in calls]
+    rows, D = xs[0].shape
+    ys = [torch.empty((rows, D), dtype=x.dtype, device=x.device) for _ in calls]
     with _on_device(x.device):
         _check(
-            lib().tpamd_rms_norm(x2.data_ptr(), w.data_ptr(), y.data_ptr(), rows, D, _ld(x2), D, float(eps), dtype_code(x.dtype),
-                                 ctypes.c_void_p(current_stream_ptr(x.device))),
+            lib().tpamd_rms_norm_ranks(len(calls), _pointers(xs), _pointers(ws), _pointers(ys), rows, D, _ld(xs[0]), D, float(eps),
+                                       dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device))),
             "tpamd_rms_norm",
         )
-    return y.view(x.shape)
+    return [y.view(x.shape) for y in ys]
 
 
 def add_rms_norm(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float) -> tuple:
     """(r + x, the RMS norm of that sum) of two tensors of one shape, dtype and device; arithmetic as in `rms_norm`."""
+    return add_rms_norm_ranks([(r, x, w, eps)])[0]
+
+
+def add_rms_norm_ranks(calls: Sequence[tuple]) -> list:
+    """`add_rms_norm(r, x, w, eps)` for the operands of several ranks (with one eps)."""
+    r, x, w, eps = calls[0]
     require_device(x, "add_rms_norm")
     if (r.shape != x.shape or r.dtype != x.dtype or r.get_device() != x.get_device() or w.dtype != x.dtype or w.get_device() != x.get_device() or w.dim() != 1
             or x.dim() == 0 or x.shape[-1] != w.shape[0]):
         raise ValueError(f"add_rms_norm: r {tuple(r.shape)} {r.dtype} on {r.device}, x {tuple(x.shape)} {x.dtype} on {x.device} and w {tuple(w.shape)} "
                          f"{w.dtype} on {w.device} do not fit")
-    x2, r2 = _as_2d(x), _as_2d(r)
-    w = w.contiguous()
-    rows, D = x2.shape
-    total = torch.empty((rows, D), dtype=x.dtype, device=x.device)
-    y = torch.empty_like(total)
+    rs, xs, ws = [_as_2d(c[0]) for c in calls], [_as_2d(c[1]) for c in calls], [c[2].contiguous() for c in calls]
+    rows, D = xs[0].shape
+    totals = [torch.empty((rows, D), dtype=x.dtype, device=x.device) for _ in calls]
+    ys = [torch.empty_like(t) for t in totals]
     with _on_device(x.device):
         _check(
-            lib().tpamd_add_rms_norm(x2.data_ptr(), r2.data_ptr(), w.data_ptr(), total.data_ptr(), y.data_ptr(), rows, D, _ld(x2), _ld(r2), D,
-                                     float(eps), dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device))),
+            lib().tpamd_add_rms_norm_ranks(len(calls), _pointers(xs), _pointers(rs), _pointers(ws), _pointers(totals), _pointers(ys), rows, D,
+                                           _ld(xs[0]), _ld(rs[0]), D, float(eps), dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device))),
             "tpamd_add_rms_norm",
         )
-    return total.view(x.shape), y.view(x.shape)
+    return [(total.view(x.shape), y.view(x.shape)) for total, y in zip(totals, ys)]
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None, causal: bool = True,
@@ -668,17 +758,9 @@ def rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Te
     return q_out
 
 
-def attention_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
-                          k_cache: torch.Tensor, v_cache: torch.Tensor, pos0, scale: Optional[float] = None,
-                          out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """`rope_append` and `attention` for one new position per sequence, in two launches instead of three.
-    q [B, 1, Hq, D] or [B, 1, Hkv, Hq / Hkv, D], k / v [B, 1, Hkv, D] (views of the projection output), cos / sin [B or 1, 1, D]
-    (or [1, D] / [D]); the caches [B, Hkv, L, D] hold pos0 positions and receive the new one at pos0. Returns [B, 1, Hq, D].
-    Where the library has no scratch buffer for the stream (first use under graph capture) the two calls are made instead.
-
-    `pos0` may also be an int64 tensor of one element on the device: the kernels then read the count when they run
-    (`tpamd_attention_decode_rope_devpos`), the launches are laid out for the L positions the caches can hold, and the call
-    can sit in a HIP graph that is replayed for every decode step. The caller advances the count."""
+def _decode_operands(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor,
+                     v_cache: torch.Tensor) -> tuple:
+    """Checks the operands of a decode step; (elements between query heads, between groups of them, cos, sin as rows of D)."""
     require_device(q, "attention_decode_rope")
     if not (q.dtype == k.dtype == v.dtype == cos.dtype == sin.dtype == k_cache.dtype == v_cache.dtype) or q.dtype not in (
             torch.bfloat16, torch.float16):
@@ -703,17 +785,72 @@ def attention_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos
             raise ValueError(f"attention_decode_rope: {name} must have contiguous rows")
     if sin.stride() != cos.stride():
         sin, cos = sin.contiguous(), cos.contiguous()
+    return q_head, q_group, cos, sin
+
+
+def _decode_strides(q, q_head: int, q_group: int, k, v, cos, k_cache, v_cache, out):
+    return (ctypes.c_int64 * 16)(q.stride(0), q_head, q_group, k.stride(0), k.stride(2), v.stride(0), v.stride(2),
+                                 cos.stride(0) if cos.shape[0] > 1 else 0, k_cache.stride(0), k_cache.stride(1), k_cache.stride(2),
+                                 v_cache.stride(0), v_cache.stride(1), v_cache.stride(2), out.stride(0), out.stride(2))
+
+
+def _check_device_position(q: torch.Tensor, pos0: torch.Tensor) -> None:
+    if pos0.dtype != torch.int64 or pos0.numel() != 1 or pos0.device != q.device:
+        raise ValueError(f"attention_decode_rope: a position on the device must be one int64 element on {q.device}, "
+                         f"got {tuple(pos0.shape)} {pos0.dtype} on {pos0.device}")
+
+
+def attention_decode_rope_ranks(calls: Sequence[tuple]) -> list:
+    """`attention_decode_rope(q, k, v, cos, sin, k_cache, v_cache, pos0, scale)` for the operands of several ranks (with one scale, and one pos0
+    where that is a number)."""
+    q, k, v, cos, sin, k_cache, v_cache, pos0, scale = calls[0]
+    q_head, q_group, cos, sin = _decode_operands(q, k, v, cos, sin, k_cache, v_cache)
+    on_device = isinstance(pos0, torch.Tensor)
+    if on_device:
+        _check_device_position(q, pos0)
+    B, _, Hkv, D = k.shape
+    Hq = q.shape[2] if q.dim() == 4 else q.shape[2] * q.shape[3]
+    ranks, keep = (DecodeRank * len(calls))(), []
+    for rank, (rq, rk, rv, rcos, rsin, rk_cache, rv_cache, rpos, _) in zip(ranks, calls):
+        rcos, rsin = rcos.reshape(-1, D), rsin.reshape(-1, D)
+        if rsin.stride() != rcos.stride():
+            rsin, rcos = rsin.contiguous(), rcos.contiguous()
+        out = torch.empty((B, 1, Hq, D), dtype=q.dtype, device=q.device)
+        keep.append((rcos, rsin, out))
+        rank.q, rank.k, rank.v, rank.cos, rank.sin = rq.data_ptr(), rk.data_ptr(), rv.data_ptr(), rcos.data_ptr(), rsin.data_ptr()
+        rank.k_cache, rank.v_cache, rank.out, rank.pos = rk_cache.data_ptr(), rv_cache.data_ptr(), out.data_ptr(), rpos.data_ptr() if on_device else None
+    strides = _decode_strides(q, q_head, q_group, k, v, cos, k_cache, v_cache, out)
+    with _on_device(q.device):
+        rc = lib().tpamd_attention_decode_rope_ranks(len(calls), ranks, B, Hq, Hkv, D, 0 if on_device else int(pos0), k_cache.shape[2], strides,
+                                                     float(scale if scale is not None else D ** -0.5), dtype_code(q.dtype),
+                                                     ctypes.c_void_p(current_stream_ptr(q.device)))
+    if rc == -2 and not on_device:  # no scratch buffer for this stream: rank by rank, with the two calls that need none
+        return [attention_decode_rope(*call) for call in calls]
+    _check(rc, "tpamd_attention_decode_rope_ranks")
+    return [out for _, _, out in keep]
+
+
+def attention_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                          k_cache: torch.Tensor, v_cache: torch.Tensor, pos0, scale: Optional[float] = None,
+                          out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """`rope_append` and `attention` for one new position per sequence, in two launches instead of three.
+    q [B, 1, Hq, D] or [B, 1, Hkv, Hq / Hkv, D], k / v [B, 1, Hkv, D] (views of the projection output), cos / sin [B or 1, 1, D]
+    (or [1, D] / [D]); the caches [B, Hkv, L, D] hold pos0 positions and receive the new one at pos0. Returns [B, 1, Hq, D].
+    Where the library has no scratch buffer for the stream (first use under graph capture) the two calls are made instead.
+
+    `pos0` may also be an int64 tensor of one element on the device: the kernels then read the count when they run
+    (`tpamd_attention_decode_rope_devpos`), the launches are laid out for the L positions the caches can hold, and the call
+    can sit in a HIP graph that is replayed for every decode step. The caller advances the count."""
+    q_head, q_group, cos, sin = _decode_operands(q, k, v, cos, sin, k_cache, v_cache)
+    B, _, Hkv, D = k.shape
+    Hq = q.shape[2] if q.dim() == 4 else q.shape[2] * q.shape[3]
     if out is None:
         out = torch.empty((B, 1, Hq, D), dtype=q.dtype, device=q.device)
     elif out.shape != (B, 1, Hq, D) or out.dtype != q.dtype or out.device != q.device or out.stride(3) != 1:
         raise ValueError(f"attention_decode_rope: out must be a [{B}, 1, {Hq}, {D}] {q.dtype} tensor on {q.device} with contiguous rows")
-    strides = (ctypes.c_int64 * 16)(q.stride(0), q_head, q_group, k.stride(0), k.stride(2), v.stride(0), v.stride(2),
-                                    cos.stride(0) if cos.shape[0] > 1 else 0, k_cache.stride(0), k_cache.stride(1), k_cache.stride(2),
-                                    v_cache.stride(0), v_cache.stride(1), v_cache.stride(2), out.stride(0), out.stride(2))
+    strides = _decode_strides(q, q_head, q_group, k, v, cos, k_cache, v_cache, out)
     if isinstance(pos0, torch.Tensor):
-        if pos0.dtype != torch.int64 or pos0.numel() != 1 or pos0.device != q.device:
-            raise ValueError(f"attention_decode_rope: a position on the device must be one int64 element on {q.device}, "
-                             f"got {tuple(pos0.shape)} {pos0.dtype} on {pos0.device}")
+        _check_device_position(q, pos0)
         with _on_device(q.device):
             rc = lib().tpamd_attention_decode_rope_devpos(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(),
                                                           k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), B, Hq, Hkv, D,
@@ -737,6 +874,23 @@ def attention_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos
 def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale_: torch.Tensor, outlier_idx: Optional[torch.Tensor],
               w_out: Optional[torch.Tensor], bias: Optional[torch.Tensor] = None, act: int = ACT_NONE) -> torch.Tensor:
     """Weight-only int8 Linear with outlier columns kept in the activation dtype."""
+    x2, wq, scale_, outlier_idx, w_out, b = _w8_operands(x, wq, scale_, outlier_idx, w_out, bias)
+    (M, K), N = x2.shape, wq.shape[0]
+    n_out = 0 if outlier_idx is None else int(outlier_idx.numel())
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    with _on_device(x.device):
+        _check(
+            lib().tpamd_linear_w8(x2.data_ptr(), wq.data_ptr(), scale_.data_ptr(),
+                                  outlier_idx.data_ptr() if n_out else None, w_out.data_ptr() if n_out else None, n_out,
+                                  b.data_ptr() if b is not None else None, y.data_ptr(), M, N, K, _ld(x2), K, max(n_out, 1), N,
+                                  dtype_code(x.dtype), act, ctypes.c_void_p(current_stream_ptr(x.device))),
+            "tpamd_linear_w8",
+        )
+    return y.view(*x.shape[:-1], N)
+
+
+def _w8_operands(x, wq, scale_, outlier_idx, w_out, bias) -> tuple:
+    """The checked operands of an int8 Linear as the library takes them (no outlier columns: None)."""
     require_device(x, "linear_w8")
     if wq.dtype != torch.int8 or scale_.dtype != torch.float32:
         raise TypeError("linear_w8: wq must be int8 and scale float32")
@@ -763,14 +917,25 @@ def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale_: torch.Tensor, outlier_i
             raise ValueError(f"linear_w8: {n_out} outlier columns for K = {K}")
         w_out = w_out.contiguous()
         outlier_idx = outlier_idx.contiguous()
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    b = bias.contiguous() if bias is not None else None
+    return x2, wq, scale_.contiguous(), outlier_idx if n_out else None, w_out if n_out else None, None if bias is None else bias.contiguous()
+
+
+def linear_w8_ranks(calls: Sequence[tuple]) -> list:
+    """`linear_w8(x, wq, scale, outlier_idx, w_out, bias)` for the operands of several ranks."""
+    ranks, keep = (W8Rank * len(calls))(), []
+    for rank, call in zip(ranks, calls):
+        ops = _w8_operands(*call)
+        x2, wq = ops[:2]
+        (M, K), N = x2.shape, wq.shape[0]
+        y = torch.empty((M, N), dtype=x2.dtype, device=x2.device)
+        keep.append((ops, y))
+        rank.x, rank.wq, rank.scale, rank.outlier_idx, rank.w_out, rank.bias = (None if t is None else t.data_ptr() for t in ops)
+        rank.y = y.data_ptr()
+    x, n_out = calls[0][0], 0 if ops[3] is None else int(ops[3].numel())
     with _on_device(x.device):
         _check(
-            lib().tpamd_linear_w8(x2.data_ptr(), wq.data_ptr(), scale_.contiguous().data_ptr(),
-                                  outlier_idx.data_ptr() if n_out else None, w_out.data_ptr() if n_out else None, n_out,
-                                  b.data_ptr() if b is not None else None, y.data_ptr(), M, N, K, _ld(x2), K, max(n_out, 1), N,
-                                  dtype_code(x.dtype), act, ctypes.c_void_p(current_stream_ptr(x.device))),
-            "tpamd_linear_w8",
+            lib().tpamd_linear_w8_ranks(len(calls), ranks, n_out, M, N, K, _ld(x2), K, max(n_out, 1), N, dtype_code(x.dtype), ACT_NONE,
+                                        ctypes.c_void_p(current_stream_ptr(x.device))),
+            "tpamd_linear_w8_ranks",
         )
-    return y.view(*x.shape[:-1], N)
+    return [y.view(*x.shape[:-1], N) for _, y in keep]

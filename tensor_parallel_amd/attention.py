@@ -24,7 +24,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from . import _native
+from . import _native, together
 
 IMPLEMENTATION_NAME = "tpamd"
 
@@ -190,7 +190,7 @@ def _project_qkv(self, hidden_states: torch.Tensor, D: int):
                       and k_proj.weight.data_ptr() == w.data_ptr() + nq * row_bytes
                       and v_proj.weight.data_ptr() == w.data_ptr() + (nq + nk) * row_bytes)
         if intact and hidden_states.dtype == w.dtype:
-            qkv = _guard(_native.linear(hidden_states.detach(), w, b), hidden_states, q_proj.weight)
+            qkv = _guard(together.linear(hidden_states.detach(), w, b), hidden_states, q_proj.weight)
             return (qkv[..., :nq].view(B, S, -1, D), qkv[..., nq:nq + nk].view(B, S, -1, D), qkv[..., nq + nk:].view(B, S, -1, D))
         if not intact:  # a projection was replaced (quantised, re-assigned): three calls from now on
             del self.__dict__["_tp_qkv"]
@@ -222,7 +222,7 @@ def _attend_on_cache(q, k, v, cos, sin, layer, static, scale, layer_idx: int) ->
                              f"[{B}, {Hkv}, positions, {D}] {k.dtype}")
         count = static.cumulative_length
         if S == 1:
-            out = _native.attention_decode_rope(q, k, v, cos, sin, kb, vb, count.reshape(1), scale=scale)
+            out = together.attention_decode_rope(q, k, v, cos, sin, kb, vb, count.reshape(1), scale=scale)
         else:
             pos0 = int(count)
             if pos0 + S > kb.shape[2]:
@@ -234,7 +234,7 @@ def _attend_on_cache(q, k, v, cos, sin, layer, static, scale, layer_idx: int) ->
     pos0 = layer.get_seq_length()
     kb, vb = _buffers_with_room(layer, B, Hkv, D, pos0 + S, k)
     if S == 1:
-        out = _native.attention_decode_rope(q, k, v, cos, sin, kb, vb, pos0, scale=scale)
+        out = together.attention_decode_rope(q, k, v, cos, sin, kb, vb, pos0, scale=scale)
     else:
         q_rot = _native.rope_append(q, k, v, cos, sin, kb, vb, pos0)
         out = _native.attention(q_rot, kb[:, :, :pos0 + S], vb[:, :, :pos0 + S], scale=scale, causal=True)

@@ -21,16 +21,16 @@ import torch
 from . import _native
 from .shard_modules import _guard
 from .slicing import concat_dim
+from .together import GreenTurn, current_turn, set_turn_lock  # noqa: F401 - the names under which forwards look them up
 
 RENDEZVOUS_TIMEOUT_S = 600.0
 
 # Ranks that share ONE device take turns on the host: a rank holds the turn while it runs module code and gives it up
-# only while it waits in a collective. All ranks enqueue onto the same device anyway, so nothing is lost, and host-side
-# lazy initialisation inside torch (attention backends, BLAS handles) is never entered by two ranks at once. The ranks
-# are greenlets of the calling thread where the greenlet package is there (a switch costs about a microsecond), else
+# only while it waits, in a collective or for a peer that makes the same library call (together.GreenTurn). All ranks enqueue onto the same
+# device anyway, so nothing is lost, and host-side lazy initialisation inside torch (attention backends, BLAS handles) is never entered by two ranks at
+# once. The ranks are greenlets of the calling thread where the greenlet package is there (a switch costs about a microsecond), else
 # threads (a hand-over through a condition variable costs tens of microseconds, twice per collective). The turn of the
-# running forward is published per rank here: context variables are per thread and per greenlet.
-_turn: contextvars.ContextVar = contextvars.ContextVar("tpamd_turn", default=None)
+# running forward is published per rank (together.current_turn).
 
 
 class Turn:
@@ -56,37 +56,6 @@ class Turn:
         """Called by a failing rank while it holds the lock: wakes every waiting peer."""
         self.failed = True
         self.cond.notify_all()
-
-
-class GreenTurn:
-    """The same for ranks that are greenlets of one thread: the turn is whichever greenlet runs. A rank that waits
-    switches to `hub`, the greenlet that started the ranks and hands the turn round (tensor_parallel.parallel_apply_simple);
-    `events` counts completed rounds and finished ranks, which is how the hub sees that the ranks still get anywhere."""
-
-    __slots__ = ("hub", "events", "failed")
-
-    def __init__(self, hub):
-        self.hub = hub
-        self.events = 0
-        self.failed = False
-
-    def wait(self, timeout: float) -> bool:
-        self.hub.switch()
-        return True
-
-    def wake(self) -> None:
-        self.events += 1
-
-    def fail(self) -> None:
-        self.failed = True
-
-
-def set_turn_lock(turn) -> None:
-    _turn.set(turn)
-
-
-def current_turn():
-    return _turn.get()
 
 
 # ---- the sum folded into the last Linear of a row-parallel module -------------------------------------------------
@@ -122,6 +91,7 @@ class SumContext:
         elif self.last_linear is not None:
             feeds = value is self.last_out and self.calls.get(id(self.last_linear)) == 1
             self.last_linear.__dict__["_tp_feeds_sum"] = self.owner if feeds else None
+            self.owner.__dict__["_tp_sum_known"] = True
 
 
 def push_sum_context(ctx: Optional[SumContext]) -> None:

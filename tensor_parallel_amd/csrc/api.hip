@@ -16,11 +16,11 @@ void set_error(const char *fmt, ...) {
 
 int gemm_dispatch(const void *x, const void *w, const void *w2, const void *bias, const void *addend, int64_t ldadd, void *y,
                   int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, int act, bool swiglu,
-                  bool generic, hipStream_t s);
+                  bool generic, hipStream_t s, const RankStep *second = nullptr);
 int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bias, const void *addend, int64_t ldadd,
                     const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out, void *y, int64_t M, int64_t N,
                     int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int64_t ld_wout, int dtype, int act, bool swiglu, bool w8,
-                    hipStream_t s);
+                    hipStream_t s, const RankStep *second = nullptr);
 
 bool w8_direct_ok(int64_t K, int64_t ldx, int64_t ldw);
 int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out,
@@ -31,7 +31,7 @@ int attention_dispatch(const void *q, const void *k, const void *v, void *o, int
                        int64_t Skv, int64_t D, const int64_t *strides, float scale, int causal, int dtype, hipStream_t s);
 int attention_decode_rope_dispatch(const void *q, const void *k, const void *v, const void *cos, const void *sin, void *k_cache,
                                    void *v_cache, void *o, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t pos0, const int64_t *pos_dev,
-                                   const int64_t *strides, float scale, int dtype, hipStream_t s);
+                                   const int64_t *strides, float scale, int dtype, hipStream_t s, const tpamd_decode_rank *second = nullptr);
 
 namespace {
 
@@ -170,6 +170,62 @@ extern "C" int tpamd_swiglu_up(const void *x_dev, const void *wg_dev, const void
                          !fast, s);
 }
 
+// n ranks' Linears (w2: gated pairs) of one shape, two to a launch where both have what the fast kernels need. A rank's half of a decode-sized
+// matrix streams at 3-5.7 TB/s because a launch starts and drains in about 2 us; both halves in one reach 5.5-6.7. Two launches / one, in a
+// recorded decode step (us, kernel trace, bf16, one row): QKV 6144 x 4096 21.0 / 16.4, the pair 5504 x 4096 31.6 / 28.4, head 16000 x 4096
+// 41.2 / 39.1; 40 rows in fp16: the pair 58.4 (two K splits and their finishing launches) / 40.2 (unsplit, its tiles now fill the device),
+// QKV 3072 x 4096 27.8 / 17.9 a rank; 512 rows: the pair 106 / 104 (464 tiles of 128 x 192: 1.8 rounds for twice 0.9).
+static int matmul_ranks(const char *who, int n, const void *const *x, const void *const *w, const void *const *w2, const void *const *bias,
+                        void *const *y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, int act, void *stream) {
+    TPAMD_REQUIRE(n >= 0 && x && w && y, "%s: null pointer", who);
+    const bool pair = w2 != nullptr;
+    auto single = [&](int i) {
+        return pair ? tpamd_swiglu_up(x[i], w[i], w2[i], y[i], M, N, K, ldx, ldw, ldy, dtype, stream)
+                    : linear_entry(who, x[i], w[i], bias ? bias[i] : nullptr, nullptr, 0, y[i], M, N, K, ldx, ldw, ldy, dtype, act, stream);
+    };
+    for (int i = 0; i < n; ++i) {
+        const void *b0 = bias ? bias[i] : nullptr, *b1 = bias && i + 1 < n ? bias[i + 1] : nullptr;
+        bool both = i + 1 < n && M > 0 && N > 0 && dtype != TPAMD_F32 && (b0 == nullptr) == (b1 == nullptr) && (act == TPAMD_ACT_NONE || act == TPAMD_ACT_GELU);
+        for (int j = i; both && j < i + 2; ++j) {
+            if (int rc = check_common(who, x[j], w[j], y[j], M, N, K, ldx, ldw, ldy, dtype); rc != TPAMD_OK) return rc;
+            TPAMD_REQUIRE(!pair || w2[j] != nullptr, "%s: null pointer", who);
+            both = mfma_ok(x[j], w[j], pair ? w2[j] : nullptr, j == i ? b0 : b1, y[j], N, K, ldx, ldw, ldy);
+        }
+        if (!both) {
+            if (int rc = single(i); rc != TPAMD_OK) return rc;
+            continue;
+        }
+        RankStep to{};
+        to.x = bytes_from(x[i], x[i + 1]);
+        to.w = bytes_from(w[i], w[i + 1]);
+        to.w2 = pair ? bytes_from(w2[i], w2[i + 1]) : 0;
+        to.bias = bytes_from(b0, b1);
+        to.y = bytes_from(y[i], y[i + 1]);
+        int64_t rows = SKINNY_MAX_M;
+        if (M > SKINNY_MAX_M && M <= 64) {
+            if (int rc = pair ? (M <= 32 ? pair_row_limit(2 * N, K, &rows) : TPAMD_OK) : skinny_row_limit(2 * N, K, &rows); rc != TPAMD_OK) return rc;
+        }
+        const int rc = M <= rows ? skinny_dispatch(x[i], w[i], pair ? w2[i] : nullptr, b0, nullptr, 0, nullptr, nullptr, nullptr, 0, y[i], M, N, K, ldx, ldw,
+                                                   ldy, 0, dtype, act, pair, false, static_cast<hipStream_t>(stream), &to)
+                                 : gemm_dispatch(x[i], w[i], pair ? w2[i] : nullptr, b0, nullptr, 0, y[i], M, N, K, ldx, ldw, ldy, dtype, act, pair, false,
+                                                 static_cast<hipStream_t>(stream), &to);
+        if (rc != TPAMD_OK) return rc;
+        ++i;
+    }
+    return TPAMD_OK;
+}
+
+extern "C" int tpamd_linear_ranks(int n, const void *const *x_dev, const void *const *w_dev, const void *const *bias_dev, void *const *y_dev, int64_t M,
+                                  int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, int act, void *stream) {
+    return matmul_ranks("tpamd_linear_ranks", n, x_dev, w_dev, nullptr, bias_dev, y_dev, M, N, K, ldx, ldw, ldy, dtype, act, stream);
+}
+
+extern "C" int tpamd_swiglu_up_ranks(int n, const void *const *x_dev, const void *const *wg_dev, const void *const *wu_dev, void *const *h_dev, int64_t M,
+                                     int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldh, int dtype, void *stream) {
+    TPAMD_REQUIRE(wu_dev != nullptr, "tpamd_swiglu_up_ranks: wu is NULL");
+    return matmul_ranks("tpamd_swiglu_up_ranks", n, x_dev, wg_dev, wu_dev, nullptr, h_dev, M, N, K, ldx, ldw, ldh, dtype, TPAMD_ACT_NONE, stream);
+}
+
 extern "C" int tpamd_attention(const void *q_dev, const void *k_dev, const void *v_dev, void *out_dev, int64_t B, int64_t Hq,
                                int64_t Hkv, int64_t Sq, int64_t Skv, int64_t D, const int64_t *strides, float scale, int causal,
                                int dtype, void *stream) {
@@ -194,28 +250,46 @@ extern "C" int tpamd_attention(const void *q_dev, const void *k_dev, const void 
                               static_cast<hipStream_t>(stream));
 }
 
-extern "C" int tpamd_attention_decode_rope(const void *q_dev, const void *k_dev, const void *v_dev, const void *cos_dev,
-                                           const void *sin_dev, void *k_cache_dev, void *v_cache_dev, void *out_dev, int64_t B,
-                                           int64_t Hq, int64_t Hkv, int64_t D, int64_t pos0, int64_t cache_len,
-                                           const int64_t *strides, float scale, int dtype, void *stream) {
-    const char *who = "tpamd_attention_decode_rope";
+// What a decode step needs of its arguments; *empty: nothing to do.
+static int check_decode(const char *who, const tpamd_decode_rank &r, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t pos0, int64_t cache_len,
+                        const int64_t *strides, int dtype, bool devpos, bool *empty) {
+    *empty = false;
     TPAMD_REQUIRE(dtype == TPAMD_BF16 || dtype == TPAMD_F16, "%s: dtype must be BF16 or F16", who);
     TPAMD_REQUIRE(B >= 0 && Hq > 0 && Hkv > 0, "%s: bad dimension", who);
     TPAMD_REQUIRE(Hq % Hkv == 0, "%s: %lld query heads are not a multiple of %lld key/value heads", who, (long long)Hq, (long long)Hkv);
-    TPAMD_REQUIRE(pos0 >= 0 && pos0 < cache_len, "%s: position %lld does not fit a cache of %lld positions", who, (long long)pos0,
-                  (long long)cache_len);
+    if (devpos) {
+        TPAMD_REQUIRE(cache_len > 0 && cache_len < (1ll << 30), "%s: the caches must hold between 1 and 2^30 positions", who);
+    } else {
+        TPAMD_REQUIRE(pos0 >= 0 && pos0 < cache_len, "%s: position %lld does not fit a cache of %lld positions", who, (long long)pos0,
+                      (long long)cache_len);
+    }
     TPAMD_REQUIRE(strides != nullptr, "%s: strides is NULL", who);
-    if (B == 0) return TPAMD_OK;
-    TPAMD_REQUIRE(q_dev && k_dev && v_dev && cos_dev && sin_dev && k_cache_dev && v_cache_dev && out_dev, "%s: null pointer", who);
-    TPAMD_REQUIRE(Hq / Hkv < (1ll << 20) && pos0 < (1ll << 30), "%s: sequence too long", who);
-    bool ok = (D == 64 || D == 128) && aligned(q_dev, 16) && aligned(k_dev, 16) && aligned(v_dev, 16) && aligned(cos_dev, 16) &&
-              aligned(sin_dev, 16) && aligned(k_cache_dev, 16) && aligned(v_cache_dev, 16) && aligned(out_dev, 8);
+    if (B == 0) {
+        *empty = true;
+        return TPAMD_OK;
+    }
+    TPAMD_REQUIRE(r.q && r.k && r.v && r.cos && r.sin && r.k_cache && r.v_cache && r.out && (!devpos || r.pos), "%s: null pointer", who);
+    TPAMD_REQUIRE(Hq / Hkv < (1ll << 20), "%s: too many query heads per key/value head", who);
+    TPAMD_REQUIRE(devpos || pos0 < (1ll << 30), "%s: sequence too long", who);
+    bool ok = (D == 64 || D == 128) && aligned(r.q, 16) && aligned(r.k, 16) && aligned(r.v, 16) && aligned(r.cos, 16) && aligned(r.sin, 16) &&
+              aligned(r.k_cache, 16) && aligned(r.v_cache, 16) && aligned(r.out, 8) && aligned(r.pos, 8);
     for (int i = 0; i < 14; ++i) ok = ok && strides[i] % 8 == 0;   // 16-byte loads of every row
     for (int i = 14; i < 16; ++i) ok = ok && strides[i] % 4 == 0;  // 8-byte stores
     if (!ok) {
         set_error("%s: head_dim must be 64 or 128 and rows 16-byte aligned", who);
         return TPAMD_ERR_UNSUPPORTED;
     }
+    return TPAMD_OK;
+}
+
+extern "C" int tpamd_attention_decode_rope(const void *q_dev, const void *k_dev, const void *v_dev, const void *cos_dev,
+                                           const void *sin_dev, void *k_cache_dev, void *v_cache_dev, void *out_dev, int64_t B,
+                                           int64_t Hq, int64_t Hkv, int64_t D, int64_t pos0, int64_t cache_len,
+                                           const int64_t *strides, float scale, int dtype, void *stream) {
+    const tpamd_decode_rank r = {q_dev, k_dev, v_dev, cos_dev, sin_dev, k_cache_dev, v_cache_dev, out_dev, nullptr};
+    bool empty = false;
+    const int rc = check_decode("tpamd_attention_decode_rope", r, B, Hq, Hkv, D, pos0, cache_len, strides, dtype, false, &empty);
+    if (rc != TPAMD_OK || empty) return rc;
     return attention_decode_rope_dispatch(q_dev, k_dev, v_dev, cos_dev, sin_dev, k_cache_dev, v_cache_dev, out_dev, B, Hq, Hkv, D,
                                           pos0, nullptr, strides, scale, dtype, static_cast<hipStream_t>(stream));
 }
@@ -225,25 +299,39 @@ extern "C" int tpamd_attention_decode_rope_devpos(const void *q_dev, const void 
                                                   int64_t B, int64_t Hq, int64_t Hkv, int64_t D, const int64_t *pos_dev,
                                                   int64_t cache_len, const int64_t *strides, float scale, int dtype,
                                                   void *stream) {
-    const char *who = "tpamd_attention_decode_rope_devpos";
-    TPAMD_REQUIRE(dtype == TPAMD_BF16 || dtype == TPAMD_F16, "%s: dtype must be BF16 or F16", who);
-    TPAMD_REQUIRE(B >= 0 && Hq > 0 && Hkv > 0, "%s: bad dimension", who);
-    TPAMD_REQUIRE(Hq % Hkv == 0, "%s: %lld query heads are not a multiple of %lld key/value heads", who, (long long)Hq, (long long)Hkv);
-    TPAMD_REQUIRE(cache_len > 0 && cache_len < (1ll << 30), "%s: the caches must hold between 1 and 2^30 positions", who);
-    TPAMD_REQUIRE(strides != nullptr, "%s: strides is NULL", who);
-    if (B == 0) return TPAMD_OK;
-    TPAMD_REQUIRE(q_dev && k_dev && v_dev && cos_dev && sin_dev && k_cache_dev && v_cache_dev && out_dev && pos_dev, "%s: null pointer", who);
-    TPAMD_REQUIRE(Hq / Hkv < (1ll << 20), "%s: too many query heads per key/value head", who);
-    bool ok = (D == 64 || D == 128) && aligned(q_dev, 16) && aligned(k_dev, 16) && aligned(v_dev, 16) && aligned(cos_dev, 16) &&
-              aligned(sin_dev, 16) && aligned(k_cache_dev, 16) && aligned(v_cache_dev, 16) && aligned(out_dev, 8) && aligned(pos_dev, 8);
-    for (int i = 0; i < 14; ++i) ok = ok && strides[i] % 8 == 0;   // 16-byte loads of every row
-    for (int i = 14; i < 16; ++i) ok = ok && strides[i] % 4 == 0;  // 8-byte stores
-    if (!ok) {
-        set_error("%s: head_dim must be 64 or 128 and rows 16-byte aligned", who);
-        return TPAMD_ERR_UNSUPPORTED;
-    }
+    const tpamd_decode_rank r = {q_dev, k_dev, v_dev, cos_dev, sin_dev, k_cache_dev, v_cache_dev, out_dev, pos_dev};
+    bool empty = false;
+    const int rc = check_decode("tpamd_attention_decode_rope_devpos", r, B, Hq, Hkv, D, 0, cache_len, strides, dtype, true, &empty);
+    if (rc != TPAMD_OK || empty) return rc;
     return attention_decode_rope_dispatch(q_dev, k_dev, v_dev, cos_dev, sin_dev, k_cache_dev, v_cache_dev, out_dev, B, Hq, Hkv, D,
                                           cache_len, pos_dev, strides, scale, dtype, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tpamd_attention_decode_rope_ranks(int n, const tpamd_decode_rank *ranks, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t pos0,
+                                                 int64_t cache_len, const int64_t *strides, float scale, int dtype, void *stream) {
+    const char *who = "tpamd_attention_decode_rope_ranks";
+    TPAMD_REQUIRE(n >= 0 && (n == 0 || ranks != nullptr), "%s: null pointer", who);
+    for (int i = 0; i < n; ++i) {
+        TPAMD_REQUIRE((ranks[i].pos != nullptr) == (ranks[0].pos != nullptr), "%s: the count is on the device for every rank or for none", who);
+        bool empty = false;
+        const int rc = check_decode(who, ranks[i], B, Hq, Hkv, D, pos0, cache_len, strides, dtype, ranks[0].pos != nullptr, &empty);
+        if (rc != TPAMD_OK || empty) return rc;
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    auto step = [&](const tpamd_decode_rank &r, const tpamd_decode_rank *second) {
+        return attention_decode_rope_dispatch(r.q, r.k, r.v, r.cos, r.sin, r.k_cache, r.v_cache, r.out, B, Hq, Hkv, D, r.pos ? cache_len : pos0, r.pos,
+                                              strides, scale, dtype, s, second);
+    };
+    for (int i = 0; i < n; ++i) {
+        if (i + 1 < n && B * Hkv * 2 < 65536) {
+            const int rc = step(ranks[i], &ranks[i + 1]);
+            if (rc == TPAMD_OK) ++i;
+            if (rc == TPAMD_OK) continue;
+            if (rc != TPAMD_ERR_UNSUPPORTED) return rc;  // else nothing was launched: no scratch memory, or too little for two
+        }
+        if (int rc = step(ranks[i], nullptr); rc != TPAMD_OK) return rc;
+    }
+    return TPAMD_OK;
 }
 
 extern "C" int tpamd_linear_w8(const void *x_dev, const void *wq_dev, const void *scale_dev, const void *outlier_idx_dev,
@@ -285,6 +373,38 @@ extern "C" int tpamd_linear_w8(const void *x_dev, const void *wq_dev, const void
         int rc = skinny_dispatch(static_cast<const char *>(x_dev) + m0 * ldx * esz, wq_dev, nullptr, bias_dev, nullptr, 0, scale_dev,
                                  outlier_idx_dev, w_out_dev, n_out, static_cast<char *>(y_dev) + m0 * ldy * esz, mm, N, K, ldx,
                                  ldw, ldy, ld_wout, dtype, act, false, true, s);
+        if (rc != TPAMD_OK) return rc;
+    }
+    return TPAMD_OK;
+}
+
+extern "C" int tpamd_linear_w8_ranks(int n, const tpamd_w8_rank *ranks, int64_t n_out, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                                     int64_t ld_wout, int64_t ldy, int dtype, int act, void *stream) {
+    const char *who = "tpamd_linear_w8_ranks";
+    TPAMD_REQUIRE(n >= 0 && (n == 0 || ranks != nullptr), "%s: null pointer", who);
+    for (int i = 0; i < n; ++i) {
+        const tpamd_w8_rank &a = ranks[i];
+        // one slab of the weight-streaming kernels; what single calls refuse or take elsewhere stays with them
+        bool both = i + 1 < n && M > 0 && M <= SKINNY_W8_SLAB && N > 0 && n_out >= 0 && n_out <= K && K < (1ll << 31) && N < (1ll << 31) &&
+                    (dtype == TPAMD_BF16 || dtype == TPAMD_F16) && (act == TPAMD_ACT_NONE || act == TPAMD_ACT_GELU) && K % 16 == 0 && ldw % 16 == 0 &&
+                    ldx % 8 == 0 && ldx >= K && ldw >= K && ldy >= N && (n_out == 0 || ld_wout >= n_out) && tuning().w8_tile == TUNE_UNSET;
+        for (int j = i; both && j < i + 2; ++j) {
+            const tpamd_w8_rank &r = ranks[j];
+            both = r.x && r.wq && r.scale && r.y && aligned(r.x, 16) && aligned(r.wq, 16) && (n_out == 0 || (r.outlier_idx && r.w_out)) &&
+                   (r.bias == nullptr) == (a.bias == nullptr);
+        }
+        if (both) {
+            const tpamd_w8_rank &b = ranks[i + 1];
+            const bool o = n_out > 0;
+            const RankStep to = {bytes_from(a.x, b.x), bytes_from(a.wq, b.wq), 0, bytes_from(a.bias, b.bias), bytes_from(a.y, b.y),
+                                 bytes_from(a.scale, b.scale), o ? bytes_from(a.outlier_idx, b.outlier_idx) : 0, o ? bytes_from(a.w_out, b.w_out) : 0};
+            const int rc = skinny_dispatch(a.x, a.wq, nullptr, a.bias, nullptr, 0, a.scale, a.outlier_idx, a.w_out, n_out, a.y, M, N, K, ldx, ldw, ldy,
+                                           ld_wout, dtype, act, false, true, static_cast<hipStream_t>(stream), &to);
+            if (rc != TPAMD_OK) return rc;
+            ++i;
+            continue;
+        }
+        const int rc = tpamd_linear_w8(a.x, a.wq, a.scale, a.outlier_idx, a.w_out, n_out, a.bias, a.y, M, N, K, ldx, ldw, ld_wout, ldy, dtype, act, stream);
         if (rc != TPAMD_OK) return rc;
     }
     return TPAMD_OK;

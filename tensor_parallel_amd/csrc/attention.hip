@@ -80,7 +80,22 @@ struct AttnParams {
     // The number of cached positions read on the device (tpamd_attention_decode_rope_devpos): Skv above is then the
     // capacity of the caches, which the launch geometry is made for, and the kernels take the key count from here.
     const int64_t *skv_dev;
+    // Decode with the rotary embedding folded in: 1, or 2 ranks of one shape in a launch (one sequence on 500 positions, 16 heads a rank: 22.6 us
+    // in four launches, 11.2 in two), whose batch * kv head indices follow one another
+    // in blockIdx.y; byte distances from the first rank's operands to the second's (k, v: the caches).
+    int ranks;
+    struct { int64_t q, k, v, o, cos, sin, new_k, new_v, pos; } to;
 };
+
+// This block's rank; returns the batch * kv head index inside it.
+__device__ __forceinline__ int take_rank(AttnParams &p, int bh) {
+    if (p.ranks == 1 || bh < p.B * p.Hkv) return bh;
+    p.q += p.to.q; p.k += p.to.k; p.v += p.to.v; p.o += p.to.o;
+    p.cos += p.to.cos; p.sin += p.to.sin; p.new_k += p.to.new_k; p.new_v += p.to.new_v;
+    p.k_cache_w += p.to.k; p.v_cache_w += p.to.v;
+    p.skv_dev = reinterpret_cast<const int64_t *>(reinterpret_cast<const char *>(p.skv_dev) + p.to.pos);
+    return bh - p.B * p.Hkv;
+}
 
 constexpr int AT_KEYS = 64;   // keys per tile
 
@@ -102,6 +117,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) voi
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, lq = lane >> 4;
     const int nrows = p.G * p.Sq;
+    int bh = blockIdx.y, row_tile = blockIdx.x;
+    const int bh_all = bh;  // among those of both ranks
+    bh = take_rank(p, bh);  // (one rank where the causal order below applies)
     // keys in the cache and keys per block of a split: launch arguments, or derived from a count that lives on the device
     int Skv = p.Skv, keys_per_split = p.keys_per_split;
     if (p.skv_dev != nullptr) {
@@ -115,7 +133,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) voi
     // index runs fastest, so equally long blocks are neighbours and spread over the XCDs; the row tiles follow with the
     // longest first: all heads' last position tile, then the one before, ... when heads are whole numbers of
     // tiles, else simply the row tiles from the last to the first.
-    int bh = blockIdx.y, row_tile = blockIdx.x;
     if (p.causal) {
         const int lin = blockIdx.x + gridDim.x * blockIdx.y;
         bh = lin % gridDim.y;
@@ -449,7 +466,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) voi
                 *reinterpret_cast<uint2 *>(orow + (16 * dt + 4 * lq) * 2) = o2;
             }
         } else {
-            float *pr = p.part + ((static_cast<int64_t>(blockIdx.z) * gridDim.y + bh) * p.rows_pad + row[r]) * (D + 4);
+            float *pr = p.part + ((static_cast<int64_t>(blockIdx.z) * gridDim.y + (p.ranks > 1 ? bh_all : bh)) * p.rows_pad + row[r]) * (D + 4);
 #pragma unroll
             for (int dt = 0; dt < DT16; ++dt) *reinterpret_cast<f32x4 *>(pr + 16 * dt + 4 * lq) = acc[r][dt];
             if (lq == 0) {
@@ -519,7 +536,7 @@ __global__ __launch_bounds__(256) void attention_combine_newkey_kernel(AttnParam
     constexpr int per_row = D / 4;
     const int nrows = p.G;  // Sq = 1: a row is a query head of the group
     const int e = blockIdx.x * 256 + threadIdx.x;
-    const int bh = blockIdx.y;
+    const int bh = take_rank(p, blockIdx.y);
     const int b = bh / p.Hkv, hkv = bh % p.Hkv;
     // threads past the last row work on row 0 (they take part in the shuffles) and store nothing
     const bool live = e < nrows * per_row;
@@ -558,7 +575,7 @@ __global__ __launch_bounds__(256) void attention_combine_newkey_kernel(AttnParam
     if (!live) return;
 
     const int64_t split_pitch = static_cast<int64_t>(gridDim.y) * p.rows_pad * (D + 4);
-    const float *pr0 = p.part + (static_cast<int64_t>(bh) * p.rows_pad + row) * (D + 4);
+    const float *pr0 = p.part + (static_cast<int64_t>(blockIdx.y) * p.rows_pad + row) * (D + 4);
     float M = x_new;
     for (int s0 = 0; s0 < p.nsplit; s0 += 8) {
         float ms[8];
@@ -603,10 +620,11 @@ int launch(AttnParams p, int cus, hipStream_t s) {
     constexpr int RING = D == 64 ? 4 : 2;  // tiles requested ahead by the ring kernel: 64 registers either way
     constexpr int RING_MIN_TILES = 8;      // shorter key ranges: the ring's extra loads and idle rounds cost more than it hides
     // 128 rows per block (two 16-row tiles per wavefront) once that still leaves every CU a few blocks
-    const bool wide = nrows >= 128 && static_cast<int64_t>((nrows + 127) / 128) * p.B * p.Hkv >= 2 * cus;
+    const bool wide = nrows >= 128 && static_cast<int64_t>((nrows + 127) / 128) * p.B * p.Hkv * p.ranks >= 2 * cus;
     const int block_rows = wide ? 128 : 64;
     const int row_tiles = (nrows + block_rows - 1) / block_rows;
-    const int64_t blocks = static_cast<int64_t>(row_tiles) * p.B * p.Hkv;
+    const int bhs = p.B * p.Hkv * p.ranks;
+    const int64_t blocks = static_cast<int64_t>(row_tiles) * bhs;
     // Split the keys when the rows alone leave CUs idle. Fitted on a sweep of 144 decode shapes (D = 64 / 128, 1-1024
     // blocks, 512-32768 keys) and 32 shapes with several positions per sequence (short causal prefills, 8-256 new
     // positions on 2048-8192 cached keys), each with 1-64 splits, with and without the ring kernel, inside a HIP graph
@@ -679,8 +697,8 @@ int launch(AttnParams p, int cus, hipStream_t s) {
     p.nsplit = nsplit;
     p.rows_pad = row_tiles * block_rows;
     p.force_partials = newkey ? 1 : 0;
-    TPAMD_REQUIRE(p.B * p.Hkv < 65536 && nsplit < 65536, "attention: batch * kv heads too large for one launch");
-    const dim3 grid(row_tiles, p.B * p.Hkv, nsplit > 0 ? nsplit : 1);
+    TPAMD_REQUIRE(bhs < 65536 && nsplit < 65536, "attention: batch * kv heads too large for one launch");
+    const dim3 grid(row_tiles, bhs, nsplit > 0 ? nsplit : 1);
     auto run = [&](const AttnParams &prm, dim3 g, bool with_ring) {
         if (wide) hipLaunchKernelGGL((attention_kernel<DT, D, 2, 1>), g, dim3(256), 0, s, prm);
         else if (with_ring) hipLaunchKernelGGL((attention_kernel<DT, D, 1, RING>), g, dim3(256), 0, s, prm);
@@ -692,7 +710,7 @@ int launch(AttnParams p, int cus, hipStream_t s) {
         return TPAMD_OK;
     }
     if (nsplit > 0) {
-        const size_t need = static_cast<size_t>(nsplit) * p.B * p.Hkv * p.rows_pad * (D + 4) * sizeof(float);
+        const size_t need = static_cast<size_t>(nsplit) * bhs * p.rows_pad * (D + 4) * sizeof(float);
         std::lock_guard<std::mutex> hold(splitk_mutex(dev));
         void *ws = nullptr;
         int rc = splitk_scratch(dev, s, need, scratch_reserve(cus), &ws);
@@ -706,21 +724,21 @@ int launch(AttnParams p, int cus, hipStream_t s) {
             }
             p.nsplit = 1;  // one split, no partials
             p.keys_per_split = (p.Skv + AT_KEYS - 1) / AT_KEYS * AT_KEYS;
-            TPAMD_HIP(run(p, dim3(row_tiles, p.B * p.Hkv, 1), p.Skv >= RING_MIN_TILES * AT_KEYS));
+            TPAMD_HIP(run(p, dim3(row_tiles, bhs, 1), p.Skv >= RING_MIN_TILES * AT_KEYS));
             return TPAMD_OK;
         }
         p.part = static_cast<float *>(ws);
         TPAMD_HIP(run(p, grid, ring));
         // (the merge below is enqueued under the same lock: the buffer is this call's until then)
         const unsigned cblocks = static_cast<unsigned>((static_cast<int64_t>(nrows) * (D / 4) + 255) / 256);
-        if (newkey) hipLaunchKernelGGL((attention_combine_newkey_kernel<DT, D>), dim3(cblocks, p.B * p.Hkv), dim3(256), 0, s, p);
-        else hipLaunchKernelGGL((attention_combine_kernel<DT, D>), dim3(cblocks, p.B * p.Hkv), dim3(256), 0, s, p);
+        if (newkey) hipLaunchKernelGGL((attention_combine_newkey_kernel<DT, D>), dim3(cblocks, bhs), dim3(256), 0, s, p);
+        else hipLaunchKernelGGL((attention_combine_kernel<DT, D>), dim3(cblocks, bhs), dim3(256), 0, s, p);
         TPAMD_HIP(hipGetLastError());
         return TPAMD_OK;
     }
     // newkey on an empty cache
     const unsigned cblocks = static_cast<unsigned>((static_cast<int64_t>(nrows) * (D / 4) + 255) / 256);
-    hipLaunchKernelGGL((attention_combine_newkey_kernel<DT, D>), dim3(cblocks, p.B * p.Hkv), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((attention_combine_newkey_kernel<DT, D>), dim3(cblocks, bhs), dim3(256), 0, s, p);
     TPAMD_HIP(hipGetLastError());
     return TPAMD_OK;
 }
@@ -746,6 +764,7 @@ int attention_dispatch(const void *q, const void *k, const void *v, void *o, int
     p.q_sg = p.G * p.q_sh;
     p.scale_log2 = scale * 1.4426950408889634f;
     p.causal = causal;
+    p.ranks = 1;
     const bool bf = dtype == TPAMD_BF16;
     if (D == 64) return bf ? launch<TPAMD_BF16, 64>(p, cus, s) : launch<TPAMD_F16, 64>(p, cus, s);
     return bf ? launch<TPAMD_BF16, 128>(p, cus, s) : launch<TPAMD_F16, 128>(p, cus, s);
@@ -756,9 +775,10 @@ int attention_dispatch(const void *q, const void *k, const void *v, void *o, int
 // v_cache position, out batch, out head}.
 // pos_dev == NULL: `pos0` positions are cached. Otherwise the count is read from *pos_dev by the kernels and `pos0` is the
 // capacity of the caches: the grid and the key splits are made for the capacity, the blocks share out the keys there are.
+// `second`: another rank's step of the same shape, in the same launches.
 int attention_decode_rope_dispatch(const void *q, const void *k, const void *v, const void *cos, const void *sin, void *k_cache,
                                    void *v_cache, void *o, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t pos0,
-                                   const int64_t *pos_dev, const int64_t *strides, float scale, int dtype, hipStream_t s) {
+                                   const int64_t *pos_dev, const int64_t *strides, float scale, int dtype, hipStream_t s, const tpamd_decode_rank *second) {
     int dev = 0, cus = 256;
     TPAMD_HIP(hipGetDevice(&dev));
     if (int rc_cus = device_cus(dev, &cus); rc_cus != TPAMD_OK) return rc_cus;
@@ -785,6 +805,11 @@ int attention_decode_rope_dispatch(const void *q, const void *k, const void *v, 
     p.o_sb = strides[14]; p.o_sh = strides[15]; p.o_ss = 0;
     p.scale_log2 = scale * 1.4426950408889634f;
     p.causal = 0;  // the one new position sees every cached key
+    p.ranks = second != nullptr ? 2 : 1;
+    if (second != nullptr) {
+        p.to = {bytes_from(q, second->q), bytes_from(k_cache, second->k_cache), bytes_from(v_cache, second->v_cache), bytes_from(o, second->out),
+                bytes_from(cos, second->cos), bytes_from(sin, second->sin), bytes_from(k, second->k), bytes_from(v, second->v), bytes_from(pos_dev, second->pos)};
+    }
     const bool bf = dtype == TPAMD_BF16;
     if (D == 64) return bf ? launch<TPAMD_BF16, 64>(p, cus, s) : launch<TPAMD_F16, 64>(p, cus, s);
     return bf ? launch<TPAMD_BF16, 128>(p, cus, s) : launch<TPAMD_F16, 128>(p, cus, s);

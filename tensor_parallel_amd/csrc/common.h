@@ -86,6 +86,16 @@ struct StaticScratchScope {
     StaticScratchScope &operator=(const StaticScratchScope &) = delete;
 };
 
+// Two rank shards that live on one device do the same work on operands of their own: a launch that takes both is told how many bytes the
+// second rank's operands lie from the first one's (zero for operands that are not there).
+struct RankStep {
+    int64_t x, w, w2, bias, y;
+    int64_t scale, outlier_idx, w_out;  // int8 weights
+};
+static inline int64_t bytes_from(const void *a, const void *b) {
+    return a != nullptr && b != nullptr ? reinterpret_cast<intptr_t>(b) - reinterpret_cast<intptr_t>(a) : 0;
+}
+
 // Body of tpamd_linear / tpamd_linear_add / tpamd_linear_noalloc (api.hip).
 int linear_entry(const char *who, const void *x_dev, const void *w_dev, const void *bias_dev, const void *addend_dev,
                  int64_t ldadd, void *y_dev, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype,

@@ -699,7 +699,9 @@ __global__ __launch_bounds__(256) void gemm_direct128_kernel(GemmParams p) {
     extern __shared__ __align__(16) char smem[];
 
     int tile_m, tile_n;
-    tile_of_block(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    tile_of_block(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n * p.ranks, tile_m, tile_n);
+    const int part_n = tile_n;  // among the column tiles of both ranks
+    take_rank(p, tile_n);
     const int m0 = tile_m * BM;
     const int n0 = tile_n * (MODE == MODE_SWIGLU ? BN / 2 : BN);
 
@@ -874,8 +876,8 @@ __global__ __launch_bounds__(256) void gemm_direct128_kernel(GemmParams p) {
 
     if constexpr (SPLIT) {
         // partial tile [x row][w row]: a lane's 4 values are 4 consecutive w rows of one x row, one 16-byte store
-        const int tile = tile_m * p.tiles_n + tile_n;
-        float *ws = p.ws + (static_cast<int64_t>(blockIdx.y) * p.tiles_m * p.tiles_n + tile) * (BM * BN);
+        const int tile = tile_m * p.tiles_n * p.ranks + part_n;
+        float *ws = p.ws + (static_cast<int64_t>(blockIdx.y) * p.tiles_m * p.tiles_n * p.ranks + tile) * (BM * BN);
 #pragma unroll
         for (int a = 0; a < 4; ++a)
 #pragma unroll
@@ -910,8 +912,10 @@ template <int DT, int MODE>
 __global__ __launch_bounds__(256) void splitk_finish_kernel(GemmParams p, int splits) {
     constexpr int PER_ROW = MODE == MODE_SWIGLU ? 16 : 32;
     const int tile = blockIdx.y;
-    const int tile_m = tile / p.tiles_n, tile_n = tile % p.tiles_n;
-    const int64_t split_stride = static_cast<int64_t>(p.tiles_m) * p.tiles_n * (128 * 128);
+    const int tile_m = tile / (p.tiles_n * p.ranks);
+    int tile_n = tile % (p.tiles_n * p.ranks);
+    take_rank(p, tile_n);
+    const int64_t split_stride = static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.ranks * (128 * 128);
     const float *tile0 = p.ws + static_cast<int64_t>(tile) * (128 * 128);
     {
         const int idx = blockIdx.x * 256 + threadIdx.x;
@@ -2005,12 +2009,12 @@ int launch_direct128(GemmParams p, int cus, hipStream_t s) {
     p.tiles_m = (p.M + 127) / 128;
     constexpr int BN_OUT = MODE == MODE_SWIGLU ? 64 : 128;
     p.tiles_n = (p.N + BN_OUT - 1) / BN_OUT;
-    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
+    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.ranks;
     TPAMD_REQUIRE(tiles < (1ll << 31), "gemm: too many tiles");
     const int KT = p.K / 64;
     int splits = 1;
     bool deep = false;
-    estimate128(tiles, p.tiles_m, p.tiles_n, KT, cus, static_cast<double>(p.M) / (p.tiles_m * 128.0), MODE == MODE_SWIGLU, &splits, &deep);
+    estimate128(tiles, p.tiles_m, p.tiles_n * p.ranks, KT, cus, static_cast<double>(p.M) / (p.tiles_m * 128.0), MODE == MODE_SWIGLU, &splits, &deep);
     if (tuning().gemm_splitk != TUNE_UNSET) {
         splits = tuning().gemm_splitk;
         deep = tiles * splits <= cus;
@@ -2070,7 +2074,7 @@ int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
     // run in rounds of one per CU; fitted on the same timings, a K tile takes 1.47 us in a full round (the part is
     // power-limited then), 1.2 us in a round that fills at most three quarters of the CUs and 1.3 us in between.
     const int64_t big_tiles = static_cast<int64_t>((p.M + 255) / 256) * ((p.N + (swiglu ? 127 : 255)) / (swiglu ? 128 : 256));
-    const int64_t small_tiles = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + (swiglu ? 63 : 127)) / (swiglu ? 64 : 128));
+    const int64_t small_tiles = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + (swiglu ? 63 : 127)) / (swiglu ? 64 : 128)) * p.ranks;
     const int KT = static_cast<int>(p.K / 64);
     auto rounds256 = [&](int64_t units, int kt) {
         const int64_t full = units / cus, last = units % cus;
@@ -2092,6 +2096,7 @@ int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
         if (t < t256) { t256 = t; splits256 = sp; }
     }
     if (tuning().gemm_splitk256 != TUNE_UNSET) splits256 = tuning().gemm_splitk256;
+    t256 *= p.ranks;  // this tiling takes two ranks in two launches: whole rounds of large tiles gain nothing from one
     int unused_splits = 1;
     bool unused_deep = false;
     const int64_t small_tiles_m = (p.M + 127) / 128;
@@ -2101,12 +2106,18 @@ int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
         int tmx = 0, tnx = 0;
         if (tuning().gemm_tile != TUNE_UNSET) {
             if (tuning().gemm_tile > 1000) { tmx = tuning().gemm_tile / 32000; tnx = tuning().gemm_tile % 1000 / 32; }
-        } else if (estimate_mid(p.M, p.N, KT, cus, swiglu, &tmx, &tnx) >= (t256 < t128 ? t256 : t128)) {
+        } else if (estimate_mid(p.M, p.N, KT, cus, swiglu, &tmx, &tnx, p.ranks) >= (t256 < t128 ? t256 : t128)) {
             tmx = 0;
         }
         if (tmx > 0) return gemm_mid(p, DT, swiglu, tmx, tnx, s);
     }
     const bool big = tuning().gemm_tile != TUNE_UNSET ? tuning().gemm_tile == 256 : t256 < t128;
+    if (p.ranks == 2 && (big || !direct_ok)) {
+        p.ranks = 1;
+        if (int rc = gemm_large<DT>(p, swiglu, s); rc != TPAMD_OK) return rc;
+        p.x += p.to.x; p.w += p.to.w; p.w2 += p.to.w2; p.bias += p.to.bias; p.y += p.to.y;
+        return gemm_large<DT>(p, swiglu, s);
+    }
     if (direct_ok) {
         if (big) return swiglu ? launch_direct<DT, MODE_SWIGLU>(p, cus, splits256, s) : launch_direct<DT, MODE_LINEAR>(p, cus, splits256, s);
         return swiglu ? launch_direct128<DT, MODE_SWIGLU>(p, cus, s) : launch_direct128<DT, MODE_LINEAR>(p, cus, s);
@@ -2130,10 +2141,13 @@ int generic_dispatch(const GemmParams &p, int dtype, bool swiglu, hipStream_t s)
     return dtype == TPAMD_BF16 ? launch_generic<TPAMD_BF16>(p, swiglu, s) : launch_generic<TPAMD_F16>(p, swiglu, s);
 }
 
+// `second` (16-bit operands of the fast kernels, no addend): the same work for a second rank, its operands that far from the first one's.
 int gemm_dispatch(const void *x, const void *w, const void *w2, const void *bias, const void *addend, int64_t ldadd, void *y,
                   int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, int act, bool swiglu,
-                  bool generic, hipStream_t s) {
+                  bool generic, hipStream_t s, const RankStep *second) {
     GemmParams p{};
+    p.ranks = second != nullptr ? 2 : 1;
+    if (second != nullptr) p.to = *second;
     p.x = static_cast<const char *>(x);
     p.w = static_cast<const char *>(w);
     p.w2 = static_cast<const char *>(w2);
@@ -2200,6 +2214,7 @@ int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const voi
                      const void *bias, void *y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout,
                      int64_t ldy, int dtype, int act, hipStream_t s) {
     GemmParams p{};
+    p.ranks = 1;
     p.x = static_cast<const char *>(x);
     p.w = static_cast<const char *>(wq);
     p.bias = static_cast<const char *>(bias);

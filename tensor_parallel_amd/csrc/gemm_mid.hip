@@ -32,7 +32,8 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, lq = lane >> 4, wm = wave & 1, wn = wave >> 1;
     int tile_m, tile_n;
-    tile_of_block(blockIdx.x, p.tiles_m * p.tiles_n, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    tile_of_block(blockIdx.x, p.tiles_m * p.tiles_n * p.ranks, p.tiles_m, p.tiles_n * p.ranks, tile_m, tile_n);
+    take_rank(p, tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN_OUT, KT = p.K / BK;
 
     // ---- load addresses: rows past the end of an operand are clamped to its last one
@@ -188,7 +189,7 @@ int launch_mid(GemmParams p, hipStream_t s) {
     }
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN_OUT - 1) / BN_OUT;
-    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
+    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.ranks;
     TPAMD_REQUIRE(tiles < (1ll << 31), "gemm: too many tiles");
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles)), dim3(256), LDS, s, p);
     TPAMD_HIP(hipGetLastError());

@@ -25,16 +25,17 @@ constexpr MidTile MID_TILES[2][4] = {
 // predicted faster than HBM and taken off the 128 x 128 tiling, where a tie leaves them (us there / on these tiles): 28672 x 4096 at
 // 17 / 40 / 64 / 128 rows 52 52 53 58 / 56 58 61 68, 32000 x 4096 62 62 63 62 / 65 65 67 67, the pair 14336 x 4096 52 52 53 57 / 56 56 57 60.
 // Above, the floor would be wrong: 64128 x 4096 at 160 / 192 rows takes 133 / 136 us on these tiles and 142 / 144 on 256 x 256.
-inline double estimate_mid(int64_t M, int64_t N, int KT, int cus, bool swiglu, int *tmx, int *tnx) {
+// `ranks`: matrices of N columns in one launch.
+inline double estimate_mid(int64_t M, int64_t N, int KT, int cus, bool swiglu, int *tmx, int *tnx, int ranks = 1) {
     double best = 1e30;
     for (const MidTile &t : MID_TILES[swiglu ? 1 : 0]) {
         const int64_t bm = 32 * t.tmx, bn = (swiglu ? 16 : 32) * t.tnx;
-        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn), full = tiles / cus, last = tiles % cus;
+        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * ranks, full = tiles / cus, last = tiles % cus;
         double us = t.launch + full * (t.round + KT * t.full);
         if (last > 0) us += t.round + KT * t.idle[last * 2 <= cus ? 0 : last * 4 <= 3ll * cus ? 1 : 2];
         if (us < best) { best = us; *tmx = t.tmx; *tnx = t.tnx; }
     }
-    const double stream = stream_floor(N, 64ll * KT, swiglu);
+    const double stream = stream_floor(N * ranks, 64ll * KT, swiglu);
     return M <= 128 && best < stream ? stream : best;
 }
 

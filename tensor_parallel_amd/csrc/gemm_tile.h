@@ -25,7 +25,16 @@ struct GemmParams {
     float *ws;          // split-K: partial tiles, [split][tile][128 x rows][128 w rows] fp32
     int kt_per_split;   // split-K: K tiles (of 64) per split
     int splits;         // split-K of the 256 x 256 kernel: work units = tiles x splits
+    int ranks;          // 1, or 2: a second rank's columns follow the first one's, `to` leads to its operands
+    RankStep to;
 };
+
+// Which rank's column tile this is.
+__device__ __forceinline__ void take_rank(GemmParams &p, int &tile_n) {
+    if (tile_n < p.tiles_n) return;
+    tile_n -= p.tiles_n;
+    p.x += p.to.x; p.w += p.to.w; p.w2 += p.to.w2; p.bias += p.to.bias; p.y += p.to.y;
+}
 
 constexpr int BK = 64;            // K elements per stage (128 bytes of a row)
 constexpr int LDS_ROW = 144;      // bytes per staged row: 128 + 16 pad, conflict-free for b128 reads

@@ -22,7 +22,14 @@ struct NormParams {
     int64_t ldx, ldr, ldy;  // elements between rows (ldy: of y and s)
     int D;
     float eps;
+    // blockIdx.y = 1: the rows of a second rank, byte distances to its operands (one row of 4096: two launches of 3.1 us, one of 3.7)
+    struct { int64_t x, w, r, y, s; } to;
 };
+
+__device__ __forceinline__ void take_rank(NormParams &p) {
+    if (blockIdx.y == 0) return;
+    p.x += p.to.x; p.w += p.to.w; p.r += p.to.r; p.y += p.to.y; p.s += p.to.s;
+}
 
 // Sum over the block, the same value in every thread. `part` has one float per wavefront.
 template <int WAVES>
@@ -53,6 +60,7 @@ __device__ __forceinline__ uint32_t add2(uint32_t a, uint32_t b) {
 // 16-bit rows of D elements, D a multiple of 8 and at most 64 * WAVES * CH * 8, every row on a 16-byte boundary.
 template <int DT, int WAVES, int CH, bool ADD>
 __global__ __launch_bounds__(64 * WAVES) void rms_norm_kernel(NormParams p) {
+    take_rank(p);
     constexpr int T = 64 * WAVES;
     __shared__ float part[WAVES];
     const int64_t row = blockIdx.x;
@@ -111,6 +119,7 @@ __global__ __launch_bounds__(64 * WAVES) void rms_norm_kernel(NormParams p) {
 // that has read or stored it before).
 template <int DT, bool ADD>
 __global__ __launch_bounds__(256) void rms_norm_any_kernel(NormParams p) {
+    take_rank(p);
     __shared__ float part[4];
     const int64_t row = blockIdx.x;
     float sum = 0.f;
@@ -143,8 +152,8 @@ __global__ __launch_bounds__(256) void rms_norm_any_kernel(NormParams p) {
 }
 
 template <int DT, bool ADD>
-void launch_rows(const NormParams &p, int64_t rows, bool vec, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>(rows));
+void launch_rows(const NormParams &p, int64_t rows, int ranks, bool vec, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(rows), ranks);
     const int n = p.D / 8;  // 16-byte chunks per row
     // one chunk per lane as far as a block of 16 wavefronts goes: a lone row is then one load away from its sum
     // (4096 elements on 8 wavefronts)
@@ -160,13 +169,13 @@ void launch_rows(const NormParams &p, int64_t rows, bool vec, hipStream_t s) {
 
 // A launch has at most 2^32 - 1 threads, and one that asks for more runs, without an error, what is left of the count modulo 2^32: further
 // rows go into further launches.
-constexpr int64_t ROWS_PER_LAUNCH = 1ll << 21;
+constexpr int64_t ROWS_PER_LAUNCH = 1ll << 20;  // of two ranks, in blocks of up to 1024 threads
 
 template <int DT, bool ADD>
-void launch(NormParams p, int64_t rows, bool vec, hipStream_t s) {
+void launch(NormParams p, int64_t rows, int ranks, bool vec, hipStream_t s) {
     constexpr int64_t ESZ = DT == TPAMD_F32 ? 4 : 2;
     for (; rows > 0; rows -= ROWS_PER_LAUNCH) {
-        launch_rows<DT, ADD>(p, rows < ROWS_PER_LAUNCH ? rows : ROWS_PER_LAUNCH, vec, s);
+        launch_rows<DT, ADD>(p, rows < ROWS_PER_LAUNCH ? rows : ROWS_PER_LAUNCH, ranks, vec, s);
         p.x += ROWS_PER_LAUNCH * p.ldx * ESZ;
         p.y += ROWS_PER_LAUNCH * p.ldy * ESZ;
         if constexpr (ADD) {
@@ -181,31 +190,55 @@ void launch(NormParams p, int64_t rows, bool vec, hipStream_t s) {
 
 using namespace tpamd;
 
-static int run_norm(const char *who, const void *x_dev, const void *r_dev, const void *w_dev, void *s_dev, void *y_dev, int64_t rows, int64_t D,
-                    int64_t ldx, int64_t ldr, int64_t ldy, float eps, int dtype, void *stream, bool add) {
+// n ranks' rows of one shape, two ranks to a launch.
+static int run_norm(const char *who, int n, const void *const *x, const void *const *r, const void *const *w, void *const *sum, void *const *y,
+                    int64_t rows, int64_t D, int64_t ldx, int64_t ldr, int64_t ldy, float eps, int dtype, void *stream) {
+    const bool add = r != nullptr;
+    TPAMD_REQUIRE(n >= 0 && x && w && y && (!add || sum), "%s: null pointer", who);
     TPAMD_REQUIRE(dtype == TPAMD_BF16 || dtype == TPAMD_F16 || dtype == TPAMD_F32, "%s: unknown dtype %d", who, dtype);
     TPAMD_REQUIRE(rows >= 0 && D >= 0 && D < (1ll << 31), "%s: bad dimension", who);
     if (rows == 0 || D == 0) return TPAMD_OK;
-    TPAMD_REQUIRE(x_dev && w_dev && y_dev && (!add || (r_dev && s_dev)), "%s: null pointer", who);
     TPAMD_REQUIRE(ldx >= D && ldy >= D && (!add || ldr >= D), "%s: leading dimension smaller than the row", who);
-    NormParams p{static_cast<const char *>(x_dev), static_cast<const char *>(w_dev), static_cast<const char *>(r_dev), static_cast<char *>(y_dev),
-                 static_cast<char *>(s_dev), ldx, ldr, ldy, static_cast<int>(D), eps};
-    const bool vec = dtype != TPAMD_F32 && D % 8 == 0 && D <= 16 * 64 * 2 * 8 && ldx % 8 == 0 && ldr % 8 == 0 && ldy % 8 == 0 && aligned(x_dev, 16) &&
-                     aligned(w_dev, 16) && aligned(y_dev, 16) && aligned(r_dev, 16) && aligned(s_dev, 16);  // null pointers are aligned
+    bool vec = dtype != TPAMD_F32 && D % 8 == 0 && D <= 16 * 64 * 2 * 8 && ldx % 8 == 0 && ldr % 8 == 0 && ldy % 8 == 0;
+    for (int i = 0; i < n; ++i) {
+        TPAMD_REQUIRE(x[i] && w[i] && y[i] && (!add || (r[i] && sum[i])), "%s: null pointer", who);
+        vec = vec && aligned(x[i], 16) && aligned(w[i], 16) && aligned(y[i], 16) && (!add || (aligned(r[i], 16) && aligned(sum[i], 16)));
+    }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == TPAMD_BF16) add ? launch<TPAMD_BF16, true>(p, rows, vec, s) : launch<TPAMD_BF16, false>(p, rows, vec, s);
-    else if (dtype == TPAMD_F16) add ? launch<TPAMD_F16, true>(p, rows, vec, s) : launch<TPAMD_F16, false>(p, rows, vec, s);
-    else add ? launch<TPAMD_F32, true>(p, rows, vec, s) : launch<TPAMD_F32, false>(p, rows, vec, s);
-    TPAMD_HIP(hipGetLastError());
+    for (int i = 0; i < n; i += 2) {
+        const int ranks = i + 1 < n ? 2 : 1;
+        NormParams p{static_cast<const char *>(x[i]), static_cast<const char *>(w[i]), static_cast<const char *>(add ? r[i] : nullptr), static_cast<char *>(y[i]),
+                     static_cast<char *>(add ? sum[i] : nullptr), ldx, ldr, ldy, static_cast<int>(D), eps, {}};
+        if (ranks == 2) {
+            p.to = {bytes_from(x[i], x[i + 1]), bytes_from(w[i], w[i + 1]), add ? bytes_from(r[i], r[i + 1]) : 0, bytes_from(y[i], y[i + 1]),
+                    add ? bytes_from(sum[i], sum[i + 1]) : 0};
+        }
+        if (dtype == TPAMD_BF16) add ? launch<TPAMD_BF16, true>(p, rows, ranks, vec, s) : launch<TPAMD_BF16, false>(p, rows, ranks, vec, s);
+        else if (dtype == TPAMD_F16) add ? launch<TPAMD_F16, true>(p, rows, ranks, vec, s) : launch<TPAMD_F16, false>(p, rows, ranks, vec, s);
+        else add ? launch<TPAMD_F32, true>(p, rows, ranks, vec, s) : launch<TPAMD_F32, false>(p, rows, ranks, vec, s);
+        TPAMD_HIP(hipGetLastError());
+    }
     return TPAMD_OK;
 }
 
 extern "C" int tpamd_rms_norm(const void *x_dev, const void *w_dev, void *y_dev, int64_t rows, int64_t D, int64_t ldx, int64_t ldy,
                               float eps, int dtype, void *stream) {
-    return run_norm("tpamd_rms_norm", x_dev, nullptr, w_dev, nullptr, y_dev, rows, D, ldx, 0, ldy, eps, dtype, stream, false);
+    return run_norm("tpamd_rms_norm", 1, &x_dev, nullptr, &w_dev, nullptr, &y_dev, rows, D, ldx, 0, ldy, eps, dtype, stream);
+}
+
+extern "C" int tpamd_rms_norm_ranks(int n, const void *const *x_dev, const void *const *w_dev, void *const *y_dev, int64_t rows, int64_t D,
+                                    int64_t ldx, int64_t ldy, float eps, int dtype, void *stream) {
+    return run_norm("tpamd_rms_norm_ranks", n, x_dev, nullptr, w_dev, nullptr, y_dev, rows, D, ldx, 0, ldy, eps, dtype, stream);
 }
 
 extern "C" int tpamd_add_rms_norm(const void *x_dev, const void *r_dev, const void *w_dev, void *sum_dev, void *y_dev, int64_t rows, int64_t D,
                                   int64_t ldx, int64_t ldr, int64_t ldy, float eps, int dtype, void *stream) {
-    return run_norm("tpamd_add_rms_norm", x_dev, r_dev, w_dev, sum_dev, y_dev, rows, D, ldx, ldr, ldy, eps, dtype, stream, true);
+    return run_norm("tpamd_add_rms_norm", 1, &x_dev, &r_dev, &w_dev, &sum_dev, &y_dev, rows, D, ldx, ldr, ldy, eps, dtype, stream);
+}
+
+extern "C" int tpamd_add_rms_norm_ranks(int n, const void *const *x_dev, const void *const *r_dev, const void *const *w_dev, void *const *sum_dev,
+                                        void *const *y_dev, int64_t rows, int64_t D, int64_t ldx, int64_t ldr, int64_t ldy, float eps, int dtype,
+                                        void *stream) {
+    TPAMD_REQUIRE(r_dev != nullptr, "tpamd_add_rms_norm_ranks: null pointer");
+    return run_norm("tpamd_add_rms_norm_ranks", n, x_dev, r_dev, w_dev, sum_dev, y_dev, rows, D, ldx, ldr, ldy, eps, dtype, stream);
 }

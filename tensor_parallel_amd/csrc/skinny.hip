@@ -43,7 +43,18 @@ struct SkinnyParams {
     int n_out;
     int64_t ldx, ldw, ldy, ld_wout, ldadd;
     int act;
+    int ranks;     // 1, or 2: blockIdx.z is the rank, `to` the way to the second one's operands
+    RankStep to;
 };
+
+// This block's rank.
+__device__ __forceinline__ void take_rank(SkinnyParams &p) {
+    if (blockIdx.z == 0) return;
+    p.x += p.to.x; p.w += p.to.w; p.w2 += p.to.w2; p.bias += p.to.bias; p.y += p.to.y;
+    p.scale = reinterpret_cast<const float *>(reinterpret_cast<const char *>(p.scale) + p.to.scale);
+    p.outlier_idx = reinterpret_cast<const int *>(reinterpret_cast<const char *>(p.outlier_idx) + p.to.outlier_idx);
+    p.w_out += p.to.w_out;
+}
 
 template <int DT>
 __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
@@ -94,6 +105,7 @@ __device__ __forceinline__ void skinny_store_output(const SkinnyParams &p, float
 // NW = wavefronts per block.
 template <int DT, bool W8, int MT, int MODE, int CG, int NW = SK_WAVES, bool PAIR = false>
 __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
+    take_rank(p);
     static_assert(!PAIR || (MODE == SK_SWIGLU && CG == 1 && !W8), "PAIR is the gated pair with 16-bit weights");
     constexpr int NMAT = (MODE == SK_SWIGLU && !PAIR) ? 2 : 1;
     constexpr int NA = NMAT * CG;             // weight tiles per chunk: index a = cg * NMAT + matrix
@@ -410,6 +422,7 @@ __device__ __forceinline__ void static_for(F &&f) {
 // MODE SK_SWIGLU: the tile is 8 gate rows + the 8 up rows of the same 8 columns (16-bit weights only).
 template <int DT, int MODE, int NW, int NCH, int DEPTH>
 __global__ __launch_bounds__(NW * 64) void skinny_resident_kernel(SkinnyParams p) {
+    take_rank(p);
     static_assert(NCH % DEPTH == 0, "a chunk's slot must not depend on the tile");
     constexpr bool PAIR = MODE == SK_SWIGLU;
     constexpr int COLS = PAIR ? 8 : 16;
@@ -547,6 +560,8 @@ __global__ __launch_bounds__(NW * 64) void skinny_resident_kernel(SkinnyParams p
 // splits, bias and activation. DIRECT (a single split): bias, activation and the store to y happen here.
 template <int DT, int MT, int NCH, bool DIRECT>
 __global__ __launch_bounds__(SK_THREADS) void skinny_w8_split_kernel(SkinnyParams p, float *part, int cols_per_block) {
+    take_rank(p);
+    part += static_cast<int64_t>(blockIdx.z) * gridDim.y * p.M * p.N;
     constexpr int NW = SK_WAVES;
     constexpr int CHUNK_K = 256;                // K elements per chunk: 256 bytes of a weight row, 512 of an x row
     constexpr int TROW = 272;
@@ -721,7 +736,9 @@ __global__ __launch_bounds__(SK_THREADS) void skinny_w8_split_kernel(SkinnyParam
 // the planes requested eight at a time and added in plane order
 template <int DT, bool VEC>
 __global__ __launch_bounds__(256) void skinny_w8_finish_kernel(SkinnyParams p, const float *part, int splits) {
+    take_rank(p);
     const int64_t plane = static_cast<int64_t>(p.M) * p.N;
+    part += static_cast<int64_t>(blockIdx.z) * splits * plane;
     if constexpr (VEC) {
         const int64_t e = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
         if (e >= plane) return;
@@ -752,8 +769,8 @@ __global__ __launch_bounds__(256) void skinny_w8_finish_kernel(SkinnyParams p, c
 template <int DT>
 int launch_w8_finish(const SkinnyParams &p, const float *part, int splits, hipStream_t s) {
     const int64_t outputs = static_cast<int64_t>(p.M) * p.N;
-    if (p.N % 4 == 0) hipLaunchKernelGGL((skinny_w8_finish_kernel<DT, true>), dim3(static_cast<unsigned>((outputs / 4 + 255) / 256)), dim3(256), 0, s, p, part, splits);
-    else hipLaunchKernelGGL((skinny_w8_finish_kernel<DT, false>), dim3(static_cast<unsigned>((outputs + 255) / 256)), dim3(256), 0, s, p, part, splits);
+    if (p.N % 4 == 0) hipLaunchKernelGGL((skinny_w8_finish_kernel<DT, true>), dim3(static_cast<unsigned>((outputs / 4 + 255) / 256), 1, p.ranks), dim3(256), 0, s, p, part, splits);
+    else hipLaunchKernelGGL((skinny_w8_finish_kernel<DT, false>), dim3(static_cast<unsigned>((outputs + 255) / 256), 1, p.ranks), dim3(256), 0, s, p, part, splits);
     TPAMD_HIP(hipGetLastError());
     return TPAMD_OK;
 }
@@ -778,6 +795,8 @@ constexpr int WC_NW = 8, WC_UNIT_K = 128, WC_STAGE = 32 * 128;  // per wavefront
 
 template <int DT, int MT, int KU, bool DIRECT>
 __global__ __launch_bounds__(WC_NW * 64, MT == 1 ? 4 : 1) void skinny_w8_cols_kernel(SkinnyParams p, float *part, int cols_per_block, int k_planes) {
+    take_rank(p);
+    part += static_cast<int64_t>(blockIdx.z) * (k_planes + (p.n_out > 0 ? 1 : 0)) * p.M * p.N;
     constexpr int NW = WC_NW;
     extern __shared__ __align__(16) char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1035,6 +1054,7 @@ __device__ __forceinline__ float wave_sum(float v) {
 // GV_WAVES wavefronts per block; K_BATCH = loads per row in flight before anything is multiplied.
 template <int DT, bool W8, int MODE, int MR, int GV_WAVES, int K_BATCH>
 __global__ __launch_bounds__(GV_WAVES * 64) void gemv_kernel(SkinnyParams p) {
+    take_rank(p);
     constexpr int GV_THREADS = GV_WAVES * 64;
     constexpr int NMAT = MODE == SK_SWIGLU ? 2 : 1;
     constexpr int STEP_K = W8 ? 1024 : 512;          // K elements per wavefront-wide 16-byte load of w
@@ -1150,12 +1170,12 @@ int launch_gemv(const SkinnyParams &p, hipStream_t s) {
     constexpr int GV_WAVES = MODE == SK_SWIGLU ? 4 : 8;
     constexpr int GV_THREADS = GV_WAVES * 64;
     constexpr int KB = MODE == SK_SWIGLU ? 4 : 12;
-    const unsigned grid = static_cast<unsigned>((p.N + GV_WAVES - 1) / GV_WAVES);
+    const dim3 grid(static_cast<unsigned>((p.N + GV_WAVES - 1) / GV_WAVES), 1, p.ranks);
     const size_t lds = static_cast<size_t>(p.M) * p.K * 2;
     switch (p.M) {
-        case 1: hipLaunchKernelGGL((gemv_kernel<DT, W8, MODE, 1, GV_WAVES, KB>), dim3(grid), dim3(GV_THREADS), lds, s, p); break;
-        case 2: hipLaunchKernelGGL((gemv_kernel<DT, W8, MODE, 2, GV_WAVES, KB>), dim3(grid), dim3(GV_THREADS), lds, s, p); break;
-        default: hipLaunchKernelGGL((gemv_kernel<DT, W8, MODE, 3, GV_WAVES, KB>), dim3(grid), dim3(GV_THREADS), lds, s, p); break;
+        case 1: hipLaunchKernelGGL((gemv_kernel<DT, W8, MODE, 1, GV_WAVES, KB>), grid, dim3(GV_THREADS), lds, s, p); break;
+        case 2: hipLaunchKernelGGL((gemv_kernel<DT, W8, MODE, 2, GV_WAVES, KB>), grid, dim3(GV_THREADS), lds, s, p); break;
+        default: hipLaunchKernelGGL((gemv_kernel<DT, W8, MODE, 3, GV_WAVES, KB>), grid, dim3(GV_THREADS), lds, s, p); break;
     }
     TPAMD_HIP(hipGetLastError());
     return TPAMD_OK;
@@ -1188,6 +1208,7 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
 // columns) and the row's scale are requested ahead of everything else, so that no wavefront ends on a memory round trip.
 template <int DT, bool W8, int MODE, int MR, int WAVES, int NP, bool WHOLE>
 __global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(SkinnyParams p) {
+    take_rank(p);
     static_assert(!W8 || MODE == SK_LINEAR, "int8 weights: plain linear only");
     constexpr int THREADS = WAVES * 64;
     constexpr int NMAT = MODE == SK_SWIGLU ? 2 : 1;
@@ -1303,7 +1324,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(SkinnyParams p) {
 
 template <int DT, bool W8, int MODE, int WAVES, int NP>
 void launch_gemv_rows_m(const SkinnyParams &p, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>((p.N + WAVES - 1) / WAVES)), block(WAVES * 64);
+    const dim3 grid(static_cast<unsigned>((p.N + WAVES - 1) / WAVES), 1, p.ranks), block(WAVES * 64);
     const size_t lds = W8 ? static_cast<size_t>(p.M) * ((p.K * 2 + 2047) / 2048 * 2048) : static_cast<size_t>(p.M) * p.K * 2;
     const bool whole = p.K == NP * (W8 ? 1024 : 512);
 #define TPAMD_ROWS_M(MRV) \
@@ -1394,8 +1415,8 @@ int launch_gemv_rows(const SkinnyParams &p, hipStream_t s, RowsPath path, bool *
 inline int pick_cg(const SkinnyParams &p, bool w8, bool swiglu) {
     if (const int v = tuning().skinny_cg; v != TUNE_UNSET) return v == 4 ? 4 : v == 2 ? 2 : 1;
     if (p.M < (w8 ? 4 : 12)) return 1;  // measured: below this the prefetching single-group kernel is faster
-    if (!swiglu && p.N % 64 == 0 && p.N / 64 >= 256) return 4;
-    if (p.N % 32 == 0 && p.N / 32 >= 256) return 2;
+    if (!swiglu && p.N % 64 == 0 && p.N / 64 * p.ranks >= 256) return 4;
+    if (p.N % 32 == 0 && p.N / 32 * p.ranks >= 256) return 2;
     return 1;
 }
 
@@ -1420,7 +1441,7 @@ template <int MODE>
 inline bool pick_resident(const SkinnyParams &p, int cus) {
     if (p.M > 16 || p.K > 8192) return false;
     if (tuning().skinny_resident != TUNE_UNSET) return tuning().skinny_resident != 0;
-    const int64_t tiles = (p.N + (MODE == SK_SWIGLU ? 7 : 15)) / (MODE == SK_SWIGLU ? 8 : 16);
+    const int64_t tiles = (p.N + (MODE == SK_SWIGLU ? 7 : 15)) / (MODE == SK_SWIGLU ? 8 : 16) * p.ranks;
     if (p.M < (MODE == SK_SWIGLU ? 3 : 2) || p.K < 3072) return false;  // 2 rows of a gated pair: up to 26 % slower here (11008 x 6144)
     if (MODE == SK_SWIGLU) {
         // Refitted on a sweep of 220 pair shapes (N from 1376 to 14336, K from 2048 to 8192, 4 to 16 rows, in a HIP graph,
@@ -1458,14 +1479,15 @@ inline bool pick_resident(const SkinnyParams &p, int cus) {
 template <int DT, int MODE>
 int launch_resident(const SkinnyParams &p, int cus, hipStream_t s) {
     const int64_t tiles = (p.N + (MODE == SK_SWIGLU ? 7 : 15)) / (MODE == SK_SWIGLU ? 8 : 16);
-    const unsigned grid = static_cast<unsigned>(tiles < cus ? tiles : cus);
+    const int64_t share = cus / p.ranks;  // blocks of a rank: a block per CU
+    const dim3 grid(static_cast<unsigned>(tiles < share ? tiles : share), 1, p.ranks);
     // K <= 4096: 4 chunks per wavefront, a slot each; up to 6144: 6 chunks and 3 slots (6 slots do not fit the
     // registers); up to 8192: 8 chunks and 2 slots.
     // (Two blocks of 4 wavefronts per CU, 8 chunks each and 4 slots, were measured too: the registers do not fit and
     // the kernel takes twice as long.)
-    if (p.K <= 4096) hipLaunchKernelGGL((skinny_resident_kernel<DT, MODE, 8, 4, 4>), dim3(grid), dim3(512), 0, s, p);
-    else if (p.K <= 6144) hipLaunchKernelGGL((skinny_resident_kernel<DT, MODE, 8, 6, 3>), dim3(grid), dim3(512), 0, s, p);
-    else hipLaunchKernelGGL((skinny_resident_kernel<DT, MODE, 8, 8, 2>), dim3(grid), dim3(512), 0, s, p);
+    if (p.K <= 4096) hipLaunchKernelGGL((skinny_resident_kernel<DT, MODE, 8, 4, 4>), grid, dim3(512), 0, s, p);
+    else if (p.K <= 6144) hipLaunchKernelGGL((skinny_resident_kernel<DT, MODE, 8, 6, 3>), grid, dim3(512), 0, s, p);
+    else hipLaunchKernelGGL((skinny_resident_kernel<DT, MODE, 8, 8, 2>), grid, dim3(512), 0, s, p);
     TPAMD_HIP(hipGetLastError());
     return TPAMD_OK;
 }
@@ -1484,18 +1506,18 @@ int launch_resident(const SkinnyParams &p, int cus, hipStream_t s) {
 //  - K < 4096: cols on 18000 columns or more, and from 11008 columns on for 2 rows and from 24 rows on.
 enum W8Path { W8_PLAIN, W8_SPLIT, W8_COLS };
 inline W8Path pick_w8_path(const SkinnyParams &p, int cus) {
-    const int64_t tiles = (p.N + 15) / 16;
+    const int64_t N = static_cast<int64_t>(p.N) * p.ranks, tiles = (N + 15) / 16;
     const bool whole = tiles == cus || (tiles % (2ll * cus) == 0 && tiles <= 4ll * cus);
     if (p.M < 2) return W8_PLAIN;
     if (p.K >= 4096) {
-        if (p.N > 4096) {
+        if (N > 4096) {
             if (!whole || p.M == 2 || p.K > 11008) return p.K < 5120 && p.M >= 24 && p.M <= 32 && !whole ? W8_SPLIT : W8_COLS;
-            if (p.M >= 48) return p.K >= 5120 || p.N >= 16384 ? W8_COLS : W8_SPLIT;
+            if (p.M >= 48) return p.K >= 5120 || N >= 16384 ? W8_COLS : W8_SPLIT;
             return W8_PLAIN;
         }
-        return p.K >= 16384 || (p.K >= 11008 && p.M >= 48 && p.N >= 3072) ? W8_COLS : W8_PLAIN;
+        return p.K >= 16384 || (p.K >= 11008 && p.M >= 48 && N >= 3072) ? W8_COLS : W8_PLAIN;
     }
-    const bool wide = p.N >= 18000 || (p.N >= 11008 && (p.M == 2 || (p.M >= 24 && (!whole || (p.K >= 3072 && p.M >= 48)))));
+    const bool wide = N >= 18000 || (N >= 11008 && (p.M == 2 || (p.M >= 24 && (!whole || (p.K >= 3072 && p.M >= 48)))));
     return wide ? W8_COLS : W8_PLAIN;
 }
 
@@ -1518,11 +1540,11 @@ int launch_w8_split(const SkinnyParams &p, hipStream_t s, bool *done) {
     const int nch = p.M <= 16 ? 4 : p.M <= 32 ? 2 : 1;
     const int splits = (p.K + nch * 2048 - 1) / (nch * 2048);
     if (splits > cus) return TPAMD_OK;  // K in the millions: not what this kernel is laid out for
-    int col_blocks = cus / splits > 0 ? cus / splits : 1;
+    int col_blocks = cus / (splits * p.ranks) > 0 ? cus / (splits * p.ranks) : 1;
     int cols_per_block = (p.N + col_blocks - 1) / col_blocks;
     cols_per_block = (cols_per_block + 15) / 16 * 16;
     col_blocks = (p.N + cols_per_block - 1) / cols_per_block;
-    const dim3 grid(static_cast<unsigned>(col_blocks), static_cast<unsigned>(splits));
+    const dim3 grid(static_cast<unsigned>(col_blocks), static_cast<unsigned>(splits), p.ranks);
     if (splits == 1) {  // nothing to add up: no scratch buffer, no second launch
         if (p.M <= 16) hipLaunchKernelGGL((skinny_w8_split_kernel<DT, 1, 4, true>), grid, dim3(SK_THREADS), 0, s, p, nullptr, cols_per_block);
         else if (p.M <= 32) hipLaunchKernelGGL((skinny_w8_split_kernel<DT, 2, 2, true>), grid, dim3(SK_THREADS), 0, s, p, nullptr, cols_per_block);
@@ -1531,7 +1553,7 @@ int launch_w8_split(const SkinnyParams &p, hipStream_t s, bool *done) {
         *done = true;
         return TPAMD_OK;
     }
-    const size_t need = static_cast<size_t>(splits) * p.M * p.N * sizeof(float);
+    const size_t need = static_cast<size_t>(splits) * p.ranks * p.M * p.N * sizeof(float);
     std::lock_guard<std::mutex> hold(splitk_mutex(dev));
     void *ws = nullptr;
     const int rc = splitk_scratch(dev, s, need, scratch_reserve(cus), &ws);
@@ -1566,14 +1588,15 @@ int launch_w8_cols_mt(const SkinnyParams &p, int dev, int cus, hipStream_t s, bo
     const int k_planes = (p.K + KU * WC_UNIT_K - 1) / (KU * WC_UNIT_K);
     const int planes = k_planes + (p.n_out > 0 ? 1 : 0);
     if (k_planes > cus) return TPAMD_OK;
-    int col_blocks = cus / k_planes;
+    // (MT = 1: two blocks share a CU, so two ranks' blocks run side by side)
+    int col_blocks = MT > 1 && cus >= k_planes * p.ranks ? cus / (k_planes * p.ranks) : cus / k_planes;
     int cols_per_block = (p.N + col_blocks - 1) / col_blocks;
     cols_per_block = (cols_per_block + 16 * WC_NW - 1) / (16 * WC_NW) * (16 * WC_NW);
     col_blocks = (p.N + cols_per_block - 1) / cols_per_block;
     const size_t lds = static_cast<size_t>(KU) * 4 * MT * 1024 + WC_NW * WC_STAGE;
     // the outlier plane is worked on by one block per 8 tiles of a column range (a tile per wavefront)
     const int outlier_blocks = p.n_out > 0 ? (cols_per_block / 16 + WC_NW - 1) / WC_NW : 0;
-    const dim3 grid(static_cast<unsigned>(col_blocks), static_cast<unsigned>(k_planes + outlier_blocks));
+    const dim3 grid(static_cast<unsigned>(col_blocks), static_cast<unsigned>(k_planes + outlier_blocks), p.ranks);
     if (planes == 1) {
         if (int rc = configure_w8_cols<DT, MT, true>(dev, lds); rc != TPAMD_OK) return rc;
         hipLaunchKernelGGL((skinny_w8_cols_kernel<DT, MT, KU, true>), grid, dim3(WC_NW * 64), lds, s, p, nullptr, cols_per_block, k_planes);
@@ -1582,7 +1605,7 @@ int launch_w8_cols_mt(const SkinnyParams &p, int dev, int cus, hipStream_t s, bo
         return TPAMD_OK;
     }
     if (int rc = configure_w8_cols<DT, MT, false>(dev, lds); rc != TPAMD_OK) return rc;
-    const size_t need = static_cast<size_t>(planes) * p.M * p.N * sizeof(float);
+    const size_t need = static_cast<size_t>(planes) * p.ranks * p.M * p.N * sizeof(float);
     std::lock_guard<std::mutex> hold(splitk_mutex(dev));
     void *ws = nullptr;
     const int rc = splitk_scratch(dev, s, need, scratch_reserve(cus), &ws);
@@ -1635,6 +1658,7 @@ constexpr size_t XL_LDS = 2 * XL_CH * 2048 + 2048 + XL_NW * 16 * XL_SROW;
 
 template <int DT, int NW, int D, int CH>
 __global__ __launch_bounds__(NW * 64) void skinny_pair_xlds_kernel(SkinnyParams p) {
+    take_rank(p);
     constexpr int COLS = 8;
     constexpr int XS = CH * 2 / NW;      // 1 KiB slots of a chunk of x per wavefront
     constexpr int PER_TILE = CH / NW;    // list entries per tile and chunk
@@ -1769,8 +1793,8 @@ template <int DT>
 int launch_pair_xlds(const SkinnyParams &p, int cus, hipStream_t s, bool *done) {
     *done = false;
     if (tuning().skinny_xlds == 0) return TPAMD_OK;
-    const int64_t tiles = (p.N + 7) / 8;
-    if (p.M < 4 || p.M > 16 || p.K % 8 != 0 || tiles > static_cast<int64_t>(XL_T_MAX) * cus) return TPAMD_OK;
+    const int64_t tiles = (p.N + 7) / 8 * p.ranks, share = cus / p.ranks;
+    if (p.M < 4 || p.M > 16 || p.K % 8 != 0 || tiles / p.ranks > static_cast<int64_t>(XL_T_MAX) * share) return TPAMD_OK;
     if (tuning().skinny_xlds == TUNE_UNSET) {
         // Measured against the older kernels (inside a HIP graph, rows 4 / 8 / 16): 5504 columns at K = 4096 19.6 / 21.1 /
         // 21.9 -> 18.5 / 18.9 / 20.3 us, 2752 columns 13.8 / 15.1 / 16.6 -> 13.6 / 13.7 / 15.1 us, 14336 columns 43.3 / 44.9 /
@@ -1793,8 +1817,8 @@ int launch_pair_xlds(const SkinnyParams &p, int cus, hipStream_t s, bool *done) 
                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(XL_LDS)));
         configured_dev = dev;
     }
-    const unsigned grid = static_cast<unsigned>(tiles < cus ? tiles : cus);
-    hipLaunchKernelGGL((skinny_pair_xlds_kernel<DT, XL_NW, XL_D, XL_CH>), dim3(grid), dim3(XL_NW * 64), XL_LDS, s, p);
+    const dim3 grid(static_cast<unsigned>(tiles / p.ranks < share ? tiles / p.ranks : share), 1, p.ranks);
+    hipLaunchKernelGGL((skinny_pair_xlds_kernel<DT, XL_NW, XL_D, XL_CH>), grid, dim3(XL_NW * 64), XL_LDS, s, p);
     TPAMD_HIP(hipGetLastError());
     *done = true;
     return TPAMD_OK;
@@ -1829,16 +1853,16 @@ int launch_skinny(const SkinnyParams &p, hipStream_t s) {
     }
     if constexpr (MODE == SK_SWIGLU && !W8) {
         if (p.M <= 32 && pick_pair(p)) {
-            const unsigned grid8 = static_cast<unsigned>((p.N + 7) / 8);
-            if (p.M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, false, 1, MODE, 1, SK_WAVES, true>), dim3(grid8), dim3(SK_THREADS), 0, s, p);
-            else hipLaunchKernelGGL((skinny_kernel<DT, false, 2, MODE, 1, SK_WAVES, true>), dim3(grid8), dim3(SK_THREADS), 0, s, p);
+            const dim3 grid8(static_cast<unsigned>((p.N + 7) / 8), 1, p.ranks);
+            if (p.M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, false, 1, MODE, 1, SK_WAVES, true>), grid8, dim3(SK_THREADS), 0, s, p);
+            else hipLaunchKernelGGL((skinny_kernel<DT, false, 2, MODE, 1, SK_WAVES, true>), grid8, dim3(SK_THREADS), 0, s, p);
             TPAMD_HIP(hipGetLastError());
             return TPAMD_OK;
         }
     }
     int cg = pick_cg(p, W8, MODE == SK_SWIGLU);
     if (MODE == SK_SWIGLU && cg > 2) cg = 2;  // two matrices per group: registers for 2 groups
-    const unsigned grid = static_cast<unsigned>((p.N + 16 * cg - 1) / (16 * cg));
+    const dim3 grid(static_cast<unsigned>((p.N + 16 * cg - 1) / (16 * cg)), 1, p.ranks);
     if (cg > 1 && p.M > 32) {
         // the column-group kernels take 32 rows of x at a time; the weights of the later slabs come from L2 / the
         // Infinity Cache rather than HBM when they fit
@@ -1856,20 +1880,20 @@ int launch_skinny(const SkinnyParams &p, hipStream_t s) {
     if (cg > 1) {
         TPAMD_REQUIRE(p.N % (16 * cg) == 0, "skinny: N %% %d != 0", 16 * cg);
         if constexpr (MODE == SK_SWIGLU) {
-            if (p.M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, W8, 1, MODE, 2>), dim3(grid), dim3(SK_THREADS), 0, s, p);
-            else hipLaunchKernelGGL((skinny_kernel<DT, W8, 2, MODE, 2>), dim3(grid), dim3(SK_THREADS), 0, s, p);
+            if (p.M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, W8, 1, MODE, 2>), grid, dim3(SK_THREADS), 0, s, p);
+            else hipLaunchKernelGGL((skinny_kernel<DT, W8, 2, MODE, 2>), grid, dim3(SK_THREADS), 0, s, p);
         } else if (cg == 2) {
-            if (p.M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, W8, 1, MODE, 2>), dim3(grid), dim3(SK_THREADS), 0, s, p);
-            else hipLaunchKernelGGL((skinny_kernel<DT, W8, 2, MODE, 2>), dim3(grid), dim3(SK_THREADS), 0, s, p);
+            if (p.M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, W8, 1, MODE, 2>), grid, dim3(SK_THREADS), 0, s, p);
+            else hipLaunchKernelGGL((skinny_kernel<DT, W8, 2, MODE, 2>), grid, dim3(SK_THREADS), 0, s, p);
         } else {
-            if (p.M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, W8, 1, MODE, 4>), dim3(grid), dim3(SK_THREADS), 0, s, p);
-            else hipLaunchKernelGGL((skinny_kernel<DT, W8, 2, MODE, 4>), dim3(grid), dim3(SK_THREADS), 0, s, p);
+            if (p.M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, W8, 1, MODE, 4>), grid, dim3(SK_THREADS), 0, s, p);
+            else hipLaunchKernelGGL((skinny_kernel<DT, W8, 2, MODE, 4>), grid, dim3(SK_THREADS), 0, s, p);
         }
     } else {
-        const unsigned grid1 = static_cast<unsigned>((p.N + 15) / 16);
-        if (p.M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, W8, 1, MODE, 1>), dim3(grid1), dim3(SK_THREADS), 0, s, p);
-        else if (p.M <= 32) hipLaunchKernelGGL((skinny_kernel<DT, W8, 2, MODE, 1>), dim3(grid1), dim3(SK_THREADS), 0, s, p);
-        else hipLaunchKernelGGL((skinny_kernel<DT, W8, 4, MODE, 1>), dim3(grid1), dim3(SK_THREADS), 0, s, p);
+        const dim3 grid1(static_cast<unsigned>((p.N + 15) / 16), 1, p.ranks);
+        if (p.M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, W8, 1, MODE, 1>), grid1, dim3(SK_THREADS), 0, s, p);
+        else if (p.M <= 32) hipLaunchKernelGGL((skinny_kernel<DT, W8, 2, MODE, 1>), grid1, dim3(SK_THREADS), 0, s, p);
+        else hipLaunchKernelGGL((skinny_kernel<DT, W8, 4, MODE, 1>), grid1, dim3(SK_THREADS), 0, s, p);
     }
     TPAMD_HIP(hipGetLastError());
     return TPAMD_OK;
@@ -1877,12 +1901,15 @@ int launch_skinny(const SkinnyParams &p, hipStream_t s) {
 
 }  // namespace
 
-// M <= 64. dtype is BF16 or F16. `w8` selects the int8 weight path (linear only).
+// M <= 64. dtype is BF16 or F16. `w8` selects the int8 weight path (linear only). `second`: the same work for a second rank in the same
+// launches, its operands that far from the first one's (no addend); the rules then see the columns of both.
 int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bias, const void *addend, int64_t ldadd,
                     const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out, void *y, int64_t M, int64_t N,
                     int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int64_t ld_wout, int dtype, int act, bool swiglu, bool w8,
-                    hipStream_t s) {
+                    hipStream_t s, const RankStep *second) {
     SkinnyParams p{};
+    p.ranks = second != nullptr ? 2 : 1;
+    if (second != nullptr) p.to = *second;
     p.x = static_cast<const char *>(x);
     p.w = static_cast<const char *>(w);
     p.w2 = static_cast<const char *>(w2);
@@ -1911,7 +1938,7 @@ int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bi
             TPAMD_HIP(hipGetDevice(&dev));
             if (int rc_cus = device_cus(dev, &cus); rc_cus != TPAMD_OK) return rc_cus;
             const int knob = tuning().gemv_rows;  // -1: the MFMA kernels; other values: launch_gemv_rows
-            path = knob == -1 ? ROWS_MFMA : knob != TUNE_UNSET ? ROWS_W8 : pick_rows_path(swiglu, M, N, K, cus);
+            path = knob == -1 ? ROWS_MFMA : knob != TUNE_UNSET ? ROWS_W8 : pick_rows_path(swiglu, M, N * p.ranks, K, cus);
         }
         if (path != ROWS_MFMA) {
             bool done = false;

@@ -21,7 +21,7 @@ from typing import Callable, Mapping, Optional, Sequence, Tuple, Union
 import torch
 from torch import nn
 
-from . import _native
+from . import _native, together
 from . import shard_modules
 from .shard_modules import _guard, is_conv1d
 
@@ -92,7 +92,7 @@ class ShardLinearW8(nn.Module):
         if input.dtype != self.dtype:
             raise TypeError(f"ShardLinearW8: the input is {input.dtype}, the Linear was quantised for {self.dtype}")
         n_out = self.outlier_idx.numel()
-        out = _native.linear_w8(input.detach(), self.wq, self.scale, self.outlier_idx if n_out else None,
+        out = together.linear_w8(input.detach(), self.wq, self.scale, self.outlier_idx if n_out else None,
                                 self.w_out if n_out else None, self.bias)
         return _guard(out, input)
 

@@ -22,7 +22,7 @@ import types
 import torch
 from torch import nn
 
-from . import _native
+from . import _native, together
 from .slicing import is_k_major
 
 
@@ -54,7 +54,7 @@ def linear_in_context(module: nn.Module, x: torch.Tensor, w: torch.Tensor, bias)
     ctx = current_sum_context()
     b = None if bias is None else bias.detach()
     if ctx is None:
-        return _guard(_native.linear(x.detach(), w.detach(), b), x, w, bias)
+        return _guard(together.linear(x.detach(), w.detach(), b), x, w, bias)
     key = id(module)
     ctx.calls[key] = ctx.calls.get(key, 0) + 1
     addend = None
@@ -67,7 +67,12 @@ def linear_in_context(module: nn.Module, x: torch.Tensor, w: torch.Tensor, bias)
             t, mask = waiting
             if t.dtype == x.dtype and t.device == x.device and t.shape == (*x.shape[:-1], w.shape[0]):
                 addend, ctx.fused_mask = t.detach(), mask
-    out = _guard(_native.linear(x.detach(), w.detach(), b, addend=addend), x, w, bias)
+    # Ranks do not meet in the Linear that feeds the sum (the one that comes last adds the others' partials), nor before a first call has shown which one that is.
+    if "_tp_sum_known" in ctx.owner.__dict__ and module.__dict__.get("_tp_feeds_sum") is not ctx.owner:
+        out = together.linear(x.detach(), w.detach(), b)
+    else:
+        out = _native.linear(x.detach(), w.detach(), b, addend=addend)
+    out = _guard(out, x, w, bias)
     if addend is not None:
         ctx.fused_out = out
     ctx.last_linear, ctx.last_out = module, out
@@ -128,7 +133,7 @@ def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
     # Linear's), keep the module's own forward
     if own is not self._tp_replaced or not _norm_kernel_takes(hidden_states, w) or torch.is_grad_enabled() and (hidden_states.requires_grad or w.requires_grad):
         return own(self, hidden_states)
-    return _native.rms_norm(hidden_states, w, self.variance_epsilon)
+    return together.rms_norm(hidden_states, w, self.variance_epsilon)
 
 
 def is_llama_layer(module: nn.Module) -> bool:
@@ -150,7 +155,7 @@ def _llama_layer_forward(self, hidden_states: torch.Tensor, *args, **kwargs) -> 
         return own(self, hidden_states, *args, **kwargs)
     attended, _ = self.self_attn(hidden_states=self.input_layernorm(hidden_states), **{**_LAYER_DEFAULTS, **kwargs})
     if type(attended) is torch.Tensor and attended.dtype == hidden_states.dtype and attended.shape == hidden_states.shape and attended.get_device() == hidden_states.get_device():
-        total, normed = _native.add_rms_norm(hidden_states, attended, norm.weight, norm.variance_epsilon)
+        total, normed = together.add_rms_norm(hidden_states, attended, norm.weight, norm.variance_epsilon)
     else:
         total = hidden_states + attended
         normed = norm(total)
@@ -230,7 +235,7 @@ def _is_silu(fn) -> bool:
 
 def _gated_mlp_forward(self, x: torch.Tensor) -> torch.Tensor:
     gate, up, down = self.gate_proj, self.up_proj, self.down_proj
-    h = _native.swiglu_up(x.detach(), gate.weight.detach(), up.weight.detach())
+    h = together.swiglu_up(x.detach(), gate.weight.detach(), up.weight.detach())
     h = _guard(h, x, gate.weight, up.weight)
     return down(h)
 

@@ -255,12 +255,10 @@ RANK_GREENLETS = _greenlet is not None and os.environ.get("TPAMD_RANK_GREENLETS"
 
 def _apply_in_greenlets(modules: Sequence[nn.Module], inputs, kwargs_tup, device: torch.device):
     """The ranks of one device as greenlets of the calling thread. They run on the caller's stream, device and grad mode
-    because they are the caller's thread. A rank runs until it has to wait in a collective, which switches back here;
-    the ranks get the turn in rotation until all have returned. When a whole rotation passes in which no collective
-    completed and no rank finished, the live ranks wait for one that will not come (it has returned or failed): they
-    are told to give up."""
+    because they are the caller's thread. A rank runs until it has to wait, in a collective or for its peers' part of a library call,
+    and then gives the turn to the next (together.GreenTurn). When all live ranks wait for something that will not come (a rank has returned or
+    failed, or makes other calls), library calls they wanted to make together are made one by one, and where there are none they give up."""
     hub = _greenlet.getcurrent()
-    turn = GreenTurn(hub)
     results: dict = {}
 
     def body(i, module, args, kwargs):
@@ -275,21 +273,12 @@ def _apply_in_greenlets(modules: Sequence[nn.Module], inputs, kwargs_tup, device
 
     ranks = [_greenlet.greenlet(functools.partial(body, i, m, a, k), parent=hub)
              for i, (m, a, k) in enumerate(zip(modules, inputs, kwargs_tup))]
-    alive = list(range(len(ranks)))
     with torch.cuda.device(device) if device.type == "cuda" else contextlib.nullcontext():
-        position = idle = 0
-        while alive:
-            r = alive[position % len(alive)]
-            before = turn.events
-            ranks[r].switch()
-            if ranks[r].dead:
-                alive.remove(r)
-                turn.events += 1
-            else:
-                position += 1
-            idle = 0 if turn.events != before else idle + 1
-            if idle > len(alive):
-                turn.fail()
+        turn = GreenTurn(len(ranks), device.index if device.type == "cuda" else None)
+        turn.ring = list(ranks)
+        while turn.ring:
+            turn.ring[turn.at].switch()  # comes back when a rank has returned
+            turn.returned()
     failures = [results[i] for i in range(len(ranks)) if not results[i][0]]
     if failures:
         real = [e for ok, e in failures if not isinstance(e, threading.BrokenBarrierError)]

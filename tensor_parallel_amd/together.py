@@ -1,0 +1,197 @@
+"""Ranks of one device that make equal library calls hand them in together.
+
+The reference runs its W ranks side by side, a thread each (src/tensor_parallel/tensor_parallel.py:237-287). Here the ranks of
+a device are greenlets of one thread: one runs until it has to wait. If they waited only for each other's partial sums, their kernels
+would follow one another on the device, each with 1/W of the work: a decode step is then twice as many launches as it needs, every one
+too small to fill the device. So a rank that reaches a call which its peers will make too gives the turn away (`GreenTurn.meet`), and whoever comes
+last makes the call for all of them (`tpamd_*_ranks`). Two Llama-2-7B-shaped rank shards of two layers, recorded decode step: one row on 500
+positions 321 -> 278 us, 8 on 2048 479 -> 423, 40 on 1000 (grouped queries) 534 -> 454; the Falcon-40B-shaped int8 layer, 16 on 2048, 372 -> 339.
+On the host a meeting costs 4 to 5 us for both ranks, about what the call that it saves costs (eager decode steps and scoring stay where they were, within 2 %).
+
+A rank meets its peers only in the state it was started in (`_thread_state`): inside a stream, a grad or autocast mode or a function
+mode of its own, giving the turn away would take its peers there.
+"""
+from __future__ import annotations
+
+import contextvars
+import threading
+from typing import Any, Callable, List, Optional, Sequence
+
+import torch
+
+from . import _native
+
+# The turn of the running forward, per rank: context variables are per thread and per greenlet.
+_turn: contextvars.ContextVar = contextvars.ContextVar("tpamd_turn", default=None)
+
+
+def set_turn_lock(turn) -> None:
+    _turn.set(turn)
+
+
+def current_turn():
+    return _turn.get()
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+_grad, _inference, _autocast = torch.is_grad_enabled, torch.is_inference_mode_enabled, torch.is_autocast_enabled
+_function_modes, _dispatch_modes = torch._C._len_torch_function_stack, torch._C._len_torch_dispatch_stack
+
+
+def _thread_state(index: Optional[int]) -> tuple:
+    """What of the calling thread's state a rank would find changed if a peer gave it the turn from somewhere else. `index`: of the HIP device, or None."""
+    return (_grad(), _inference(), _autocast(), _function_modes(), _dispatch_modes(),
+            None if index is None else (_current_device(), _raw_stream(index)))
+
+
+class _Meeting:
+    __slots__ = ("one", "many", "more", "calls", "results", "error")
+
+    def __init__(self, one, many, more):
+        self.one, self.many, self.more = one, many, more
+        self.calls: List[tuple] = []
+        self.results: Optional[Sequence[Any]] = None
+        self.error: Optional[BaseException] = None
+
+
+def _alike(a: tuple, b: tuple) -> bool:
+    """Whether two ranks' tensors (or None) have the same forms."""
+    for s, t in zip(a, b):
+        if s is not t and (s is None or t is None or s.shape != t.shape or s.dtype is not t.dtype or s.stride() != t.stride() or s.get_device() != t.get_device()):
+            return False
+    return True
+
+
+class GreenTurn:
+    """The turn of ranks that are greenlets of one thread: whichever greenlet runs has it. `ring` holds the ranks that have not returned, `at` the
+    place of the one that runs; a rank that waits switches to the next, and one that returns ends up in its parent, the greenlet that started
+    them (tensor_parallel._apply_in_greenlets). `idle` counts the waits since a collective or a meeting was last complete or a rank returned: when every
+    rank has waited twice, all wait for something that will not come."""
+
+    __slots__ = ("ring", "at", "idle", "failed", "world", "index", "state", "open")
+
+    def __init__(self, world: int = 1, index: Optional[int] = None):
+        self.ring: List[Any] = []
+        self.at = self.idle = 0
+        self.failed = False
+        self.world = world
+        self.index = index
+        self.state = _thread_state(index)
+        self.open: List[_Meeting] = []  # meetings that not every rank has come to, oldest first
+
+    def wait(self, timeout: float = 0.0) -> bool:
+        ring = self.ring
+        self.idle += 1
+        if self.idle > 2 * len(ring):
+            self.idle = 0
+            if not self.part():
+                self.failed = True
+        at = self.at + 1
+        self.at = at = at if at < len(ring) else 0
+        if len(ring) > 1:
+            ring[at].switch()
+        return True
+
+    def wake(self) -> None:
+        self.idle = 0
+
+    def fail(self) -> None:
+        self.failed = True
+        self.idle = 0
+
+    def returned(self) -> None:
+        """The rank that has the turn is through."""
+        del self.ring[self.at]
+        if self.at == len(self.ring):
+            self.at = 0
+        self.idle = 0
+
+    def meet(self, one: Callable[..., Any], many: Callable[[List[tuple]], Sequence[Any]], tensors: tuple, more: tuple) -> Any:
+        """one(*tensors, *more), made as many([...]) for all ranks that come with tensors of the same forms and the same `more`. A rank whose
+        peers do not come (they wait elsewhere or have returned) makes the call alone (`part`)."""
+        for meeting in self.open:
+            if meeting.one is one and meeting.more == more and _alike(meeting.calls[0], tensors):
+                break
+        else:
+            meeting = _Meeting(one, many, more)
+            self.open.append(meeting)
+        place = len(meeting.calls)
+        meeting.calls.append(tensors)
+        if place + 1 == self.world:
+            self.open.remove(meeting)
+            try:
+                meeting.results = many([tensors + more for tensors in meeting.calls])
+            except BaseException as e:  # every rank that handed something in sees it
+                meeting.error = e
+            self.idle = 0
+        else:
+            while meeting.results is None and meeting.error is None:
+                if self.failed:
+                    raise threading.BrokenBarrierError
+                self.wait()
+        if meeting.error is not None:
+            raise meeting.error
+        return meeting.results[place]
+
+    def part(self) -> bool:
+        """Nobody gets any further: the calls handed in so far are made one by one. False: there were none."""
+        if not self.open:
+            return False
+        meetings, self.open = self.open, []
+        for m in meetings:
+            try:
+                m.results = [m.one(*tensors, *m.more) for tensors in m.calls]
+            except BaseException as e:
+                m.error = e
+        return True
+
+
+def _call(one: Callable[..., Any], many: Callable[[List[tuple]], Sequence[Any]], tensors: tuple, more: tuple = ()) -> Any:
+    turn = _turn.get()
+    if type(turn) is not GreenTurn or turn.world < 2 or turn.failed or _thread_state(turn.index) != turn.state:
+        return one(*tensors, *more)
+    return turn.meet(one, many, tensors, more)
+
+
+# From this many rows on a product fills the device by itself, in 256 x 256 tiles that take two ranks in two launches anyway, and each rank's
+# follow-up work finds its operands still cached: prefill of 4096 rows 3312 us rank by rank, 3325 together; of 2103 rows 1758 and 1730.
+ALONE_ROWS = 4096
+
+
+def _few_rows(x: torch.Tensor) -> bool:
+    return x.dtype is not torch.float32 and x.dim() > 0 and x.numel() < ALONE_ROWS * x.shape[-1]
+
+
+# The library calls that ranks make together; arguments and results are those of the functions of the same name in _native.
+# fp32 products have no launch of several ranks.
+def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    if not _few_rows(x):
+        return _native.linear(x, w, bias)
+    return _call(_native.linear, _native.linear_ranks, (x, w, bias))
+
+
+def swiglu_up(x: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor) -> torch.Tensor:
+    if not _few_rows(x):
+        return _native.swiglu_up(x, wg, wu)
+    return _call(_native.swiglu_up, _native.swiglu_up_ranks, (x, wg, wu))
+
+
+def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    return _call(_native.rms_norm, _native.rms_norm_ranks, (x, w), (eps,))
+
+
+def add_rms_norm(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float) -> tuple:
+    return _call(_native.add_rms_norm, _native.add_rms_norm_ranks, (r, x, w), (eps,))
+
+
+def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, outlier_idx: Optional[torch.Tensor], w_out: Optional[torch.Tensor],
+              bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    return _call(_native.linear_w8, _native.linear_w8_ranks, (x, wq, scale, outlier_idx, w_out, bias))
+
+
+def attention_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor,
+                          v_cache: torch.Tensor, pos0, scale: Optional[float] = None) -> torch.Tensor:
+    if isinstance(pos0, torch.Tensor):
+        return _call(_native.attention_decode_rope, _native.attention_decode_rope_ranks, (q, k, v, cos, sin, k_cache, v_cache, pos0), (scale,))
+    return _call(_native.attention_decode_rope, _native.attention_decode_rope_ranks, (q, k, v, cos, sin, k_cache, v_cache), (pos0, scale))

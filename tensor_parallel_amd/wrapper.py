@@ -113,7 +113,9 @@ class TensorParallelWrapper(nn.Module):
         self._sum_op = action if isinstance(action, DeviceAllReduce) else None
 
     def forward(self, *args, **kwargs):
-        call_args, call_kwargs = process_input(self.input_actions, self.rank, self.world_size, *args, **kwargs)
+        call_args, call_kwargs = args, kwargs
+        if self.input_actions:
+            call_args, call_kwargs = process_input(self.input_actions, self.rank, self.world_size, *args, **kwargs)
         # Every wrapper publishes its own context, or none: Linears and rules inside a wrapper without a foldable sum must
         # not be taken for those of an enclosing module whose output is summed.
         foldable = self._sum_op is not None and self._sum_op.fusable

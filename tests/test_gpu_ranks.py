@@ -1,0 +1,139 @@
+"""The calls of several ranks in one launch (tpamd_*_ranks, together.py): every rank's result against its own reference in fp32, at sizes on both
+sides of every line where the choice of a kernel changes; and ranks that come with different calls, or not at all."""
+import pytest
+import torch
+
+from tensor_parallel_amd import _native
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def close(got, want, dtype):
+    # products rounded once to the dtype: 2^-8 (bf16), 2^-11 (fp16) of the value; sums of K products in fp32 stay far below the floor of 1 % of a deviation
+    torch.testing.assert_close(got.float(), want, rtol=2.0 ** (-8 if dtype is torch.bfloat16 else -10), atol=1e-2 * want.std().item())
+
+
+def draws(n, *shape, dtype, scale=1.0, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return [(torch.randn(*shape, device=DEV, generator=g) * scale).to(dtype) for _ in range(n)]
+
+
+# rows: the row kernels up to 3, weight streaming up to 16 or 64, tiles of 128 with K splits, mid-sized tiles, 256 x 256
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 12, 16, 17, 40, 64, 65, 300, 700])
+@pytest.mark.parametrize("cols,K", [(4, 8), (516, 264), (1376, 2048), (2048, 4096), (3072, 4096), (4100, 1088), (1024, 8192)])
+def test_linear_of_two_ranks(rows, cols, K):
+    dtype = torch.float16 if rows % 2 else torch.bfloat16
+    xs, ws = draws(2, rows, K, dtype=dtype), draws(2, cols, K, dtype=dtype, scale=0.05, seed=1)
+    bs = draws(2, cols, dtype=dtype, seed=2) if cols % 8 else [None, None]
+    for (x, w, b), y in zip(zip(xs, ws, bs), _native.linear_ranks(list(zip(xs, ws, bs)))):
+        close(y, x.float() @ w.float().t() + (0 if b is None else b.float()), dtype)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 12, 16, 17, 32, 33, 64, 130, 520])
+@pytest.mark.parametrize("cols,K", [(4, 8), (1376, 2048), (2752, 4096), (5504, 4096), (5504, 2048), (1028, 1096)])
+def test_gated_pair_of_two_ranks(rows, cols, K):
+    dtype = torch.bfloat16 if rows % 2 else torch.float16
+    xs, gs, us = draws(2, rows, K, dtype=dtype), draws(2, cols, K, dtype=dtype, scale=0.02, seed=1), draws(2, cols, K, dtype=dtype, scale=0.02, seed=2)
+    for x, g, u, h in zip(xs, gs, us, _native.swiglu_up_ranks(list(zip(xs, gs, us)))):
+        want = torch.nn.functional.silu(x.float() @ g.float().t()) * (x.float() @ u.float().t())
+        # gate, SiLU and product are each rounded: 4 roundings of 2^-9 (2^-12) and what SiLU makes of them
+        torch.testing.assert_close(h.float(), want, rtol=2e-2, atol=2e-2 * want.std().item())
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 16, 17, 33, 64, 65])
+@pytest.mark.parametrize("cols,K,n_out", [(2048, 4096, 20), (9216, 8192, 40), (8192, 16384, 0), (4100, 1040, 3)])
+def test_int8_of_two_ranks(rows, cols, K, n_out):
+    dtype = torch.float16
+    calls, wants = [], []
+    for r in range(2):
+        x, w = draws(1, rows, K, dtype=dtype, seed=r)[0], draws(1, cols, K, dtype=dtype, scale=0.05, seed=5 + r)[0]
+        g = torch.Generator().manual_seed(r)
+        keep = torch.randperm(K, generator=g)[:n_out].sort().values
+        wz = w.float().clone()
+        wz[:, keep.to(DEV)] = 0
+        scale = wz.abs().amax(1) / 127
+        q = torch.round(wz / scale[:, None]).to(torch.int8)
+        idx, w_out = (keep.to(DEV, torch.int32), w[:, keep.to(DEV)].contiguous()) if n_out else (None, None)
+        calls.append((x, q, scale, idx, w_out, None))
+        want = (x.float() @ q.float().t()) * scale
+        wants.append(want + x.float()[:, keep.to(DEV)] @ w_out.float().t() if n_out else want)
+    for y, want in zip(_native.linear_w8_ranks(calls), wants):
+        close(y, want, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,D,n", [(1, 4096, 2), (5, 8, 3), (129, 4096, 2), (7, 16392, 2), (3, 100, 4)])
+def test_norms_of_several_ranks_are_those_of_single_calls(rows, D, n, dtype):
+    xs, rs, ws = draws(n, rows, D, dtype=dtype), draws(n, rows, D, dtype=dtype, seed=1), draws(n, D, dtype=dtype, seed=2)
+    for x, w, y in zip(xs, ws, _native.rms_norm_ranks([(x, w, 1e-5) for x, w in zip(xs, ws)])):
+        assert torch.equal(y, _native.rms_norm(x, w, 1e-5))
+    for r, x, w, (total, y) in zip(rs, xs, ws, _native.add_rms_norm_ranks([(r, x, w, 1e-5) for r, x, w in zip(rs, xs, ws)])):
+        assert torch.equal(total, r + x) and torch.equal(y, _native.rms_norm(r + x, w, 1e-5))
+
+
+@pytest.mark.parametrize("on_device", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,D,cached,n", [(1, 16, 16, 128, 500, 2), (3, 16, 2, 128, 65, 2), (2, 8, 8, 64, 0, 2), (5, 32, 4, 64, 1000, 3), (40, 16, 4, 128, 1000, 2)])
+def test_decode_of_several_ranks(B, Hq, Hkv, D, cached, n, on_device):
+    dtype, room = torch.bfloat16, cached + 3
+    calls, alone = [], []
+    for r in range(n):
+        q, k, v = (draws(1, B, 1, h, D, dtype=dtype, seed=10 * r + i)[0] for i, h in enumerate((Hq, Hkv, Hkv)))
+        cos, sin = (draws(1, B, 1, D, dtype=dtype, seed=10 * r + 3 + i)[0] for i in range(2))
+        caches = [draws(1, B, Hkv, room, D, dtype=dtype, seed=10 * r + 5 + i)[0] for i in range(2)]
+        count = torch.tensor([cached - (r if cached and on_device else 0)], device=DEV)  # counts on the device may differ
+        calls.append((q, k, v, cos, sin, *caches, count if on_device else cached, None))
+        alone.append((q, k, v, cos, sin, *[c.clone() for c in caches], count if on_device else cached, None))
+    outs = _native.attention_decode_rope_ranks(calls)
+    for call, mine, out in zip(calls, alone, outs):
+        want = _native.attention_decode_rope(*mine)
+        assert torch.equal(call[5], mine[5]) and torch.equal(call[6], mine[6])
+        # The key range is cut in other places, so probabilities are rounded to the dtype (2^-9 of each) against other maxima: over the keys that adds
+        # up to 2^-9 * sqrt(2 / 3) = 1.6e-3 deviations of the result, 4.5 times that for the largest of 80000; and one rounding of the result on each side.
+        torch.testing.assert_close(out.float(), want.float(), rtol=2.0 ** -7, atol=2e-2 * want.float().std().item())
+
+
+def test_ranks_that_do_not_fit_each_other_make_their_calls_alone():
+    from tensor_parallel_amd.tensor_parallel import RANK_GREENLETS, _apply_in_greenlets
+
+    if not RANK_GREENLETS:
+        pytest.skip("the ranks of a device are threads")
+    from tensor_parallel_amd import together
+
+    x, w = draws(2, 5, 256, dtype=torch.bfloat16), draws(2, 512, 256, dtype=torch.bfloat16, seed=1)
+    side = torch.cuda.Stream()
+
+    def rank(r):
+        def body(turns):
+            outs = []
+            for turn in turns:
+                if turn == "both":
+                    outs.append(together.linear(x[r], w[r]))
+                elif turn == "different":
+                    outs.append(together.linear(x[r], w[r][: 128 * (r + 1)]))
+                elif turn == "one" and r == 1:
+                    outs.append(together.linear(x[r], w[r]))
+                elif turn == "stream":  # a stream of the rank's own: the turn stays
+                    with torch.cuda.stream(side):
+                        side.wait_stream(torch.cuda.default_stream())
+                        outs.append(together.linear(x[r], w[r]))
+                    torch.cuda.current_stream().wait_stream(side)
+            return outs
+        return body
+
+    calls = []
+    many = _native.linear_ranks
+    try:
+        _native.linear_ranks = lambda items: calls.append(len(items)) or many(items)
+        with torch.no_grad():
+            got = _apply_in_greenlets([rank(0), rank(1)], [(["both", "different", "stream", "one", "both"],)] * 2, [{}] * 2, DEV)
+    finally:
+        _native.linear_ranks = many
+    torch.cuda.synchronize()
+    assert calls == [2, 2]
+    for r in range(2):
+        full = x[r].float() @ w[r].float().t()
+        wants = [full, full[:, : 128 * (r + 1)], full] + ([full] if r else []) + [full]
+        assert len(got[r]) == len(wants)
+        for a, b in zip(got[r], wants):
+            close(a, b, torch.bfloat16)

@@ -1,0 +1,148 @@
+"""Ranks that hand equal calls in together (together.py), on the CPU with the library calls stubbed: which ranks meet, what each gets back, and
+that nobody waits for a peer that does not come."""
+import contextlib
+
+import pytest
+import torch
+
+from tensor_parallel_amd import _native, together
+from tensor_parallel_amd.tensor_parallel import RANK_GREENLETS, _apply_in_greenlets
+
+pytestmark = pytest.mark.skipif(not RANK_GREENLETS, reason="the greenlet package is not there: the ranks of a device are threads")
+CPU = torch.device("cpu")
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    made = []
+
+    def one(x, w, bias=None):
+        made.append(1)
+        return torch.nn.functional.linear(x, w, bias)
+
+    def many(items):
+        made.append(len(items))
+        return [torch.nn.functional.linear(*item) for item in items]
+
+    monkeypatch.setattr(_native, "linear", one)
+    monkeypatch.setattr(_native, "linear_ranks", many)
+    return made
+
+
+def run(*bodies):
+    return _apply_in_greenlets(list(bodies), [(r,) for r in range(len(bodies))], [{}] * len(bodies), CPU)
+
+
+@contextlib.contextmanager
+def _device_autocast():  # what torch.autocast("cuda") sets, also where there is no device
+    torch.set_autocast_enabled("cuda", True)
+    try:
+        yield
+    finally:
+        torch.set_autocast_enabled("cuda", False)
+
+
+def operands(r, rows=3, cols=4, K=8):
+    g = torch.Generator().manual_seed(r)
+    return torch.randn(rows, K, generator=g).bfloat16(), torch.randn(cols, K, generator=g).bfloat16()
+
+
+@pytest.mark.parametrize("world", [1, 2, 3])
+def test_equal_calls_are_made_at_once_and_each_rank_gets_its_own(calls, world):
+    def body(r):
+        return [together.linear(*operands(r)) for _ in range(3)]
+
+    for r, got in enumerate(run(*[body] * world)):
+        assert all(torch.equal(y, torch.nn.functional.linear(*operands(r))) for y in got)
+    assert calls == [world] * 3
+
+
+@pytest.mark.parametrize("form", ["cols", "rows", "strides", "dtype", "bias", "fp32", "many rows"])
+def test_calls_of_other_forms_are_made_alone(calls, form):
+    def body(r):
+        x, w = operands(r)
+        b = None
+        if r == 1 or form in ("fp32", "many rows"):
+            if form == "cols":
+                w = torch.cat([w, w])
+            elif form == "rows":
+                x = x[:2]
+            elif form == "strides":
+                x = torch.cat([x, x], 1)[:, :8]
+            elif form == "dtype":
+                x, w = x.half(), w.half()
+            elif form == "bias":
+                b = w[:, 0].contiguous()
+            elif form == "fp32":
+                x, w = x.float(), w.float()
+            else:
+                x = x[:1].expand(together.ALONE_ROWS, -1)
+        return together.linear(x, w, b), torch.nn.functional.linear(x, w, b)
+
+    for got, want in run(body, body):
+        assert torch.equal(got, want)
+    assert calls == [1, 1]
+
+
+@pytest.mark.parametrize("mode", ["grad", "inference", "autocast", "function mode"])
+def test_a_rank_in_a_state_of_its_own_keeps_the_turn(calls, mode):
+    def own():
+        if mode == "grad":
+            return torch.no_grad()
+        if mode == "inference":
+            return torch.inference_mode()
+        if mode == "autocast":
+            return _device_autocast()
+        return torch.device("cpu")
+
+    seen = []
+
+    def body(r):
+        with own():
+            y = together.linear(*operands(r))
+            seen.append(r)
+        assert torch.is_grad_enabled() and not torch.is_inference_mode_enabled()
+        return y + together.linear(*operands(r))
+
+    run(body, body)
+    assert calls == [1, 1, 2] and seen == [0, 1]
+
+
+def test_a_peer_that_returned_or_waits_elsewhere_is_not_waited_for(calls):
+    from tensor_parallel_amd.collectives import CollectiveOperation
+
+    op = CollectiveOperation(2, lambda *xs: [sum(xs)] * 2, timeout=5.0)
+
+    def body(r):
+        got = []
+        if r == 0:
+            got.append(together.linear(*operands(0)))  # the peer is in the collective
+        total = op(r + 1, r)
+        if r == 0:
+            got.append(together.linear(*operands(0)))  # the peer has returned
+        return total, got
+
+    (t0, got), (t1, _) = run(body, body)
+    assert t0 == t1 == 3 and calls == [1, 1]
+    assert all(torch.equal(y, torch.nn.functional.linear(*operands(0))) for y in got)
+
+
+@pytest.mark.parametrize("where", ["before", "in the call"])
+def test_a_failure_reaches_every_rank_and_the_next_forward_works(calls, monkeypatch, where):
+    good = _native.linear_ranks
+
+    def bad(items):
+        raise KeyError("bad operands")
+
+    def body(r):
+        if where == "before" and r == 1:
+            raise KeyError("bad operands")
+        return together.linear(*operands(r))
+
+    if where == "in the call":
+        monkeypatch.setattr(_native, "linear_ranks", bad)
+    with pytest.raises(KeyError, match="bad operands"):
+        run(body, body)
+    monkeypatch.setattr(_native, "linear_ranks", good)
+    run(lambda r: together.linear(*operands(r)), lambda r: together.linear(*operands(r)))
+    assert calls[-1] == 2
