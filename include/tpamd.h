@@ -192,6 +192,13 @@ int tpamd_linear_add(const void *x_dev, const void *w_dev, const void *bias_dev,
                      int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldadd, int64_t ldy, int dtype,
                      int act, void *stream);
 
+/* tpamd_linear_add that stores every result twice, to y and to copy (leading dimension ldy): the sum over two ranks, each of which goes
+ * on with a tensor of its own (ScatterReduce and AllGather, src/tensor_parallel/communications.py:119-171). copy_dev may be addend_dev
+ * (then ldadd must equal ldy) and overlaps neither y nor another input. */
+int tpamd_linear_add_copy(const void *x_dev, const void *w_dev, const void *bias_dev, const void *addend_dev, void *y_dev, void *copy_dev,
+                          int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldadd, int64_t ldy, int dtype, int act,
+                          void *stream);
+
 /* tpamd_linear for callers that cannot allocate device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc. It has no counterpart in the reference. Same arguments, same kernels and the same
  * result, bit for bit, as tpamd_linear; the call allocates nothing (no hipMalloc, no hipFree), also at its first use
@@ -322,6 +329,12 @@ int tpamd_add_rms_norm(const void *x_dev, const void *r_dev, const void *w_dev, 
 int tpamd_linear_ranks(int n, const void *const *x_dev, const void *const *w_dev, const void *const *bias_dev /* NULL: none */,
                        void *const *y_dev, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, int act,
                        void *stream);
+/* Column-parallel Linears whose outputs every rank needs whole: y[r][:, i N : (i + 1) N] = act(x[i] . w[i]^T + bias[i]) for every r and i
+ * (the `"gather -1"` output rule behind a column-parallel Linear, src/tensor_parallel/communications.py:142-171, each
+ * rank with a copy of its own). ldy >= n N. */
+int tpamd_linear_gather_ranks(int n, const void *const *x_dev, const void *const *w_dev, const void *const *bias_dev /* NULL: none */,
+                              void *const *y_dev, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, int act,
+                              void *stream);
 int tpamd_swiglu_up_ranks(int n, const void *const *x_dev, const void *const *wg_dev, const void *const *wu_dev, void *const *h_dev,
                           int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldh, int dtype, void *stream);
 int tpamd_rms_norm_ranks(int n, const void *const *x_dev, const void *const *w_dev, void *const *y_dev, int64_t rows, int64_t D,

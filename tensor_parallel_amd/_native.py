@@ -51,6 +51,8 @@ EXPORTS = (
     "tpamd_add_rms_norm_ranks",
     "tpamd_attention_decode_rope_ranks",
     "tpamd_linear_w8_ranks",
+    "tpamd_linear_add_copy",
+    "tpamd_linear_gather_ranks",
 )
 
 ABI_VERSION = 6
@@ -158,6 +160,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     pp = c.POINTER(vp)
     lib.tpamd_linear_ranks.restype = ci
     lib.tpamd_linear_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, i64, i64, ci, ci, vp]
+    lib.tpamd_linear_gather_ranks.restype = ci
+    lib.tpamd_linear_gather_ranks.argtypes = lib.tpamd_linear_ranks.argtypes
+    lib.tpamd_linear_add_copy.restype = ci
+    lib.tpamd_linear_add_copy.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, ci, ci, vp]
     lib.tpamd_swiglu_up_ranks.restype = ci
     lib.tpamd_swiglu_up_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, i64, i64, ci, vp]
     lib.tpamd_rms_norm_ranks.restype = ci
@@ -505,11 +511,29 @@ def linear_ranks(calls: Sequence[tuple]) -> list:
     return [y.view(*x.shape[:-1], N) for y in ys]
 
 
+def linear_gather_ranks(calls: Sequence[tuple]) -> list:
+    """The `linear(x, w, bias)` of all ranks side by side along the last axis, for each rank a tensor of its own."""
+    x, w, bias = calls[0]
+    _check_linear(x, w, bias)
+    xs, ws = [_as_2d(c[0]) for c in calls], [_as_2d(c[1]) for c in calls]
+    (M, K), N = xs[0].shape, w.shape[0]
+    whole = N * len(calls)
+    ys = [torch.empty((M, whole), dtype=x.dtype, device=x.device) for _ in calls]
+    bs = None if bias is None else [c[2].contiguous() for c in calls]
+    with _on_device(x.device):
+        _check(
+            lib().tpamd_linear_gather_ranks(len(calls), _pointers(xs), _pointers(ws), None if bs is None else _pointers(bs), _pointers(ys), M, N, K,
+                                            _ld(xs[0]), _ld(ws[0]), whole, dtype_code(x.dtype), ACT_NONE, ctypes.c_void_p(current_stream_ptr(x.device))),
+            "tpamd_linear_gather_ranks",
+        )
+    return [y.view(*x.shape[:-1], whole) for y in ys]
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act: int = ACT_NONE,
-           addend: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+           addend: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, copy: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = act(x @ w.T + bias) with w of shape [N, K]; leading dimensions of x are kept. With `addend` (same shape
     and dtype as y): y = (that result, rounded to the dtype) + addend, one step of the sum over rank partials, in the
-    same launch. `out` (contiguous, may be `addend`) receives the result."""
+    same launch. `out` (contiguous, may be `addend`) receives the result; with an addend, `copy` (contiguous) receives it too."""
     _check_linear(x, w, bias)
     N, K = w.shape
     M = x.numel() // K if K else 0
@@ -518,6 +542,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
         raise ValueError("linear: addend must have the shape, dtype and device of the result")
     if out is not None and (out.dtype != x.dtype or out.device != x.device or out.numel() != M * N or not out.is_contiguous()):
         raise ValueError("linear: out must be a contiguous tensor of the result's size, dtype and device")
+    if copy is not None and (addend is None or copy.dtype != x.dtype or copy.device != x.device or copy.numel() != M * N or not copy.is_contiguous()):
+        raise ValueError("linear: copy goes with an addend and must be a contiguous tensor of the result's size, dtype and device")
     x2, w2 = _as_2d(x), _as_2d(w)
     M = x2.shape[0]
     y = torch.empty((M, N), dtype=x.dtype, device=x.device) if out is None else out.view(M, N)
@@ -530,6 +556,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
                 lib().tpamd_linear(x2.data_ptr(), w2.data_ptr(), b.data_ptr() if b is not None else None, y.data_ptr(),
                                    M, N, K, _ld(x2), _ld(w2), N, dtype_code(x.dtype), act, stream),
                 "tpamd_linear",
+            )
+        elif copy is not None:
+            _check(
+                lib().tpamd_linear_add_copy(x2.data_ptr(), w2.data_ptr(), b.data_ptr() if b is not None else None, a2.data_ptr(), y.data_ptr(),
+                                            copy.data_ptr(), M, N, K, _ld(x2), _ld(w2), _ld(a2), N, dtype_code(x.dtype), act, stream),
+                "tpamd_linear_add_copy",
             )
         else:
             _check(

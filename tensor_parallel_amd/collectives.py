@@ -71,11 +71,11 @@ _contexts: contextvars.ContextVar = contextvars.ContextVar("tpamd_sum_contexts",
 class SumContext:
     """One call of a wrapped module whose output 0 goes to `op`, on one rank."""
 
-    __slots__ = ("op", "rank", "owner", "last_linear", "last_out", "calls", "fused_out", "fused_mask")
+    __slots__ = ("op", "rank", "owner", "last_linear", "last_out", "calls", "fused_out", "fused_mask", "fused_copy")
 
     def __init__(self, op: "DeviceAllReduce", rank: int, owner: Any):
         self.op, self.rank, self.owner = op, rank, owner
-        self.last_linear = self.last_out = self.fused_out = None
+        self.last_linear = self.last_out = self.fused_out = self.fused_copy = None
         self.calls: dict = {}
         self.fused_mask = 0
 
@@ -212,6 +212,7 @@ class DeviceAllReduce(CollectiveOperation):
         super().__init__(world_size, self._reduce, timeout)
         self.accum = accum
         self._masks: List[int] = [0] * world_size
+        self._copy: Optional[torch.Tensor] = None  # of a value that covers every rank
 
     @property
     def fusable(self) -> bool:
@@ -240,11 +241,14 @@ class DeviceAllReduce(CollectiveOperation):
         ctx = current_sum_context()
         if ctx is not None and ctx.op is self and ctx.fused_out is not None and x is ctx.fused_out:
             mask |= ctx.fused_mask  # this value already holds what the rank's Linear was given by addend_for()
+            if ctx.fused_copy is not None and ctx.fused_copy[1] == x._version:  # nobody has written to the value since
+                self._copy = ctx.fused_copy[0]
         self._masks[rank] = mask
         try:
             return super().__call__(x, rank)
         finally:
             self._masks[rank] = 0
+            self._copy = None
 
     def _reduce(self, *parts: torch.Tensor):
         masks = list(self._masks)
@@ -253,6 +257,8 @@ class DeviceAllReduce(CollectiveOperation):
         # the widest value is a running sum from rank 0 on (or covers both of two ranks); what it lacks are higher ranks
         out = todo[0].detach() if len(todo) == 1 else _native.reduce_partials([p.detach() for p in todo], accum=self.accum)
         # each rank continues with a tensor of its own: later in-place ops on one rank must not leak
+        if len(todo) == 1 and self._copy is not None and self.world_size == 2:
+            return [_guard(o, *parts) for o in (out, self._copy)]
         return [_guard(o, *parts) for o in [out] + [out.clone() for _ in range(self.world_size - 1)]]
 
 

@@ -16,11 +16,11 @@ void set_error(const char *fmt, ...) {
 
 int gemm_dispatch(const void *x, const void *w, const void *w2, const void *bias, const void *addend, int64_t ldadd, void *y,
                   int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, int act, bool swiglu,
-                  bool generic, hipStream_t s, const RankStep *second = nullptr);
+                  bool generic, hipStream_t s, const RankStep *second = nullptr, int64_t copy = 0);
 int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bias, const void *addend, int64_t ldadd,
                     const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out, void *y, int64_t M, int64_t N,
                     int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int64_t ld_wout, int dtype, int act, bool swiglu, bool w8,
-                    hipStream_t s, const RankStep *second = nullptr);
+                    hipStream_t s, const RankStep *second = nullptr, int64_t copy = 0);
 
 bool w8_direct_ok(int64_t K, int64_t ldx, int64_t ldw);
 int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out,
@@ -116,7 +116,7 @@ extern "C" const char *tpamd_last_error(void) { return g_err; }
 // y = act(x . w^T + bias), then, with an addend, y = round(y + addend) in the tensor dtype.
 int tpamd::linear_entry(const char *who, const void *x_dev, const void *w_dev, const void *bias_dev, const void *addend_dev,
                         int64_t ldadd, void *y_dev, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy,
-                        int dtype, int act, void *stream) {
+                        int dtype, int act, void *stream, void *copy_dev) {
     int rc = check_common(who, x_dev, w_dev, y_dev, M, N, K, ldx, ldw, ldy, dtype);
     if (rc != TPAMD_OK) return rc;
     TPAMD_REQUIRE(act == TPAMD_ACT_NONE || act == TPAMD_ACT_GELU, "%s: unknown activation %d", who, act);
@@ -124,7 +124,8 @@ int tpamd::linear_entry(const char *who, const void *x_dev, const void *w_dev, c
     TPAMD_REQUIRE(addend_dev == nullptr || ldadd >= N, "%s: ldadd=%lld is smaller than N=%lld", who, (long long)ldadd, (long long)N);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool fast = dtype != TPAMD_F32 && mfma_ok(x_dev, w_dev, nullptr, bias_dev, y_dev, N, K, ldx, ldw, ldy) &&
-                      (addend_dev == nullptr || (aligned(addend_dev, 8) && ldadd % 4 == 0));
+                      (addend_dev == nullptr || (aligned(addend_dev, 8) && ldadd % 4 == 0)) && aligned(copy_dev, 8);
+    const int64_t copy = bytes_from(y_dev, copy_dev);
     int64_t skinny_rows = SKINNY_MAX_M;
     if (fast && M > SKINNY_MAX_M && M <= 64) {
         rc = skinny_row_limit(N, K, &skinny_rows);
@@ -132,9 +133,9 @@ int tpamd::linear_entry(const char *who, const void *x_dev, const void *w_dev, c
     }
     if (fast && M <= skinny_rows)
         return skinny_dispatch(x_dev, w_dev, nullptr, bias_dev, addend_dev, ldadd, nullptr, nullptr, nullptr, 0, y_dev, M, N, K,
-                               ldx, ldw, ldy, 0, dtype, act, false, false, s);
+                               ldx, ldw, ldy, 0, dtype, act, false, false, s, nullptr, copy);
     return gemm_dispatch(x_dev, w_dev, nullptr, bias_dev, addend_dev, ldadd, y_dev, M, N, K, ldx, ldw, ldy, dtype, act, false,
-                         !fast, s);
+                         !fast, s, nullptr, copy);
 }
 
 extern "C" int tpamd_linear(const void *x_dev, const void *w_dev, const void *bias_dev, void *y_dev, int64_t M, int64_t N,
@@ -148,6 +149,17 @@ extern "C" int tpamd_linear_add(const void *x_dev, const void *w_dev, const void
     TPAMD_REQUIRE(addend_dev != nullptr || M == 0 || N == 0, "tpamd_linear_add: addend is NULL");
     return linear_entry("tpamd_linear_add", x_dev, w_dev, bias_dev, addend_dev, ldadd, y_dev, M, N, K, ldx, ldw, ldy, dtype, act,
                         stream);
+}
+
+// The second store instead of a copying launch behind the sum (2.9 us for one row of 4096, 4.7 for 8, 6.2 for 2103, four in a recorded step of two
+// layers): 8 rows on 2048 positions 423 -> 409 us, with the head's gather.
+extern "C" int tpamd_linear_add_copy(const void *x_dev, const void *w_dev, const void *bias_dev, const void *addend_dev, void *y_dev, void *copy_dev,
+                                     int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldadd, int64_t ldy, int dtype, int act,
+                                     void *stream) {
+    TPAMD_REQUIRE((addend_dev != nullptr && copy_dev != nullptr && copy_dev != y_dev) || M == 0 || N == 0,
+                  "tpamd_linear_add_copy: the addend or the copy is NULL, or the copy is y");
+    return linear_entry("tpamd_linear_add_copy", x_dev, w_dev, bias_dev, addend_dev, ldadd, y_dev, M, N, K, ldx, ldw, ldy, dtype, act,
+                        stream, copy_dev);
 }
 
 extern "C" int tpamd_swiglu_up(const void *x_dev, const void *wg_dev, const void *wu_dev, void *h_dev, int64_t M, int64_t N,
@@ -224,6 +236,57 @@ extern "C" int tpamd_swiglu_up_ranks(int n, const void *const *x_dev, const void
                                      int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldh, int dtype, void *stream) {
     TPAMD_REQUIRE(wu_dev != nullptr, "tpamd_swiglu_up_ranks: wu is NULL");
     return matmul_ranks("tpamd_swiglu_up_ranks", n, x_dev, wg_dev, wu_dev, nullptr, h_dev, M, N, K, ldx, ldw, ldh, dtype, TPAMD_ACT_NONE, stream);
+}
+
+// Column-parallel Linears of n ranks, each rank's columns written into every rank's whole output: two launches and a concatenation in one. What bounded
+// the small ones was launches: fp32 [128 x 768] by two halves of 384 columns 13.0 + 13.0 + 7.7 us, now 13.9; OPT-125m on 2 x 64 tokens, 72 of them,
+// 445 -> 300 launches and 7.66 -> 5.37 ms eager (kernels 3.4 -> 2.0 ms). A recorded decode step's output head on one row 20.6 + 20.6 + 4.8 -> 37.9 us.
+extern "C" int tpamd_linear_gather_ranks(int n, const void *const *x_dev, const void *const *w_dev, const void *const *bias_dev, void *const *y_dev,
+                                         int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, int act, void *stream) {
+    const char *who = "tpamd_linear_gather_ranks";
+    TPAMD_REQUIRE(n >= 0 && (n == 0 || (x_dev && w_dev && y_dev)), "%s: null pointer", who);
+    TPAMD_REQUIRE(dtype == TPAMD_BF16 || dtype == TPAMD_F16 || dtype == TPAMD_F32, "%s: unknown dtype %d", who, dtype);
+    TPAMD_REQUIRE(act == TPAMD_ACT_NONE || act == TPAMD_ACT_GELU, "%s: unknown activation %d", who, act);
+    const int64_t esz = dtype == TPAMD_F32 ? 4 : 2;
+    bool fast = n == 2 && M > 0 && N > 0 && (bias_dev == nullptr || (bias_dev[0] == nullptr) == (bias_dev[1] == nullptr));
+    for (int i = 0; i < n; ++i) {
+        const void *b = bias_dev ? bias_dev[i] : nullptr;
+        if (int rc = check_common(who, x_dev[i], w_dev[i], y_dev[i], M, N, K, ldx, ldw, ldy, dtype); rc != TPAMD_OK) return rc;
+        TPAMD_REQUIRE(M == 0 || N == 0 || ldy >= n * N, "%s: ldy=%lld does not hold %d ranks' columns", who, (long long)ldy, n);
+        fast = fast && (dtype == TPAMD_F32 ? aligned(x_dev[i], 16) && aligned(w_dev[i], 16) && aligned(y_dev[i], 16) && aligned(b, 16) && K >= 4 && K % 4 == 0 &&
+                                                 N % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && ldy % 4 == 0
+                                           : mfma_ok(x_dev[i], w_dev[i], nullptr, b, y_dev[i], N, K, ldx, ldw, ldy));
+    }
+    if (M == 0 || N == 0) return TPAMD_OK;
+    if (!fast) {  // rank by rank into the first output, which is then copied
+        for (int i = 0; i < n; ++i) {
+            const int rc = linear_entry(who, x_dev[i], w_dev[i], bias_dev ? bias_dev[i] : nullptr, nullptr, 0, static_cast<char *>(y_dev[0]) + i * N * esz, M, N, K,
+                                        ldx, ldw, ldy, dtype, act, stream);
+            if (rc != TPAMD_OK) return rc;
+        }
+        for (int i = 1; i < n; ++i) {
+            const uint64_t pitch = static_cast<uint64_t>(ldy * esz);
+            const tpamd_copy_job job = {y_dev[0], y_dev[i], static_cast<uint64_t>(M), static_cast<uint64_t>(n * N * esz), pitch, pitch};
+            if (int rc = tpamd_copy_jobs_run(&job, 1, stream); rc != TPAMD_OK) return rc;
+        }
+        return TPAMD_OK;
+    }
+    const void *b0 = bias_dev ? bias_dev[0] : nullptr, *b1 = bias_dev ? bias_dev[1] : nullptr;
+    RankStep to{};
+    to.x = bytes_from(x_dev[0], x_dev[1]);
+    to.w = bytes_from(w_dev[0], w_dev[1]);
+    to.bias = bytes_from(b0, b1);
+    to.y = N * esz;
+    const int64_t copy = bytes_from(y_dev[0], y_dev[1]);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    int64_t rows = dtype == TPAMD_F32 ? 0 : SKINNY_MAX_M;
+    if (dtype != TPAMD_F32 && M > SKINNY_MAX_M && M <= 64) {
+        if (int rc = skinny_row_limit(2 * N, K, &rows); rc != TPAMD_OK) return rc;
+    }
+    if (M <= rows)
+        return skinny_dispatch(x_dev[0], w_dev[0], nullptr, b0, nullptr, 0, nullptr, nullptr, nullptr, 0, y_dev[0], M, N, K, ldx, ldw, ldy, 0, dtype, act, false,
+                               false, s, &to, copy);
+    return gemm_dispatch(x_dev[0], w_dev[0], nullptr, b0, nullptr, 0, y_dev[0], M, N, K, ldx, ldw, ldy, dtype, act, false, false, s, &to, copy);
 }
 
 extern "C" int tpamd_attention(const void *q_dev, const void *k_dev, const void *v_dev, void *out_dev, int64_t B, int64_t Hq,

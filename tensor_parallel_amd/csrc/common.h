@@ -99,7 +99,7 @@ static inline int64_t bytes_from(const void *a, const void *b) {
 // Body of tpamd_linear / tpamd_linear_add / tpamd_linear_noalloc (api.hip).
 int linear_entry(const char *who, const void *x_dev, const void *w_dev, const void *bias_dev, const void *addend_dev,
                  int64_t ldadd, void *y_dev, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype,
-                 int act, void *stream);
+                 int act, void *stream, void *copy_dev = nullptr);
 
 static inline bool aligned(const void *p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 

@@ -94,6 +94,7 @@ __device__ __forceinline__ void epilogue(const GemmParams &p, f32x16 (&acc)[TM][
                         o.y = add_packed2<DT>(o.y, araw.y);
                     }
                     *reinterpret_cast<uint2 *>(yrow + static_cast<int64_t>(n) * 2) = o;
+                    if (p.copy) *reinterpret_cast<uint2 *>(yrow + static_cast<int64_t>(n) * 2 + p.copy) = o;
                 }
             }
         }
@@ -527,7 +528,7 @@ __global__ __launch_bounds__(256) void gemm_direct4_kernel(GemmParams p) {
     const uint32_t smem_base = lds_addr_of(smem);
     // epilogue staging behind the two stages: 16 rows x 64 packed outputs per wavefront
     char *ep_slab = smem + 2 * STAGE + wave * (16 * EP_PITCH);
-    const bool wide_stores = (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && p.ldy % 8 == 0;
+    const bool wide = wide_stores(p);
 
 #define T4_SB __builtin_amdgcn_sched_barrier(0)
 #define T4_MFMA(buf, a, b) acc[a][b] = mfma16<DT>(wq[buf][b], xq[buf][a], acc[a][b])
@@ -650,13 +651,13 @@ __global__ __launch_bounds__(256) void gemm_direct4_kernel(GemmParams p) {
         const int m_wave = tile_m * BM + wm * 128;
         const int n_wave = tile_n * BN_OUT + (MODE == MODE_SWIGLU ? wn * 64 : wn * 128);
         if constexpr (MODE == MODE_SWIGLU) {
-            staged_epilogue<DT, MODE, false, 8, 8, 1, 4, 4>(p, acc, ep_slab, m_wave, n_wave, lane, wide_stores);
+            staged_epilogue<DT, MODE, false, 8, 8, 1, 4, 4>(p, acc, ep_slab, m_wave, n_wave, lane, wide);
         } else {
             if (p.act == TPAMD_ACT_GELU) {
-                if (p.addend != nullptr) staged_epilogue<DT, MODE, true, 8, 8, 2, 4, 0, true>(p, acc, ep_slab, m_wave, n_wave, lane, wide_stores);
-                else staged_epilogue<DT, MODE, true, 8, 8, 2, 4, 0>(p, acc, ep_slab, m_wave, n_wave, lane, wide_stores);
-            } else if (p.addend != nullptr) staged_epilogue<DT, MODE, false, 8, 8, 2, 4, 0, true>(p, acc, ep_slab, m_wave, n_wave, lane, wide_stores);
-            else staged_epilogue<DT, MODE, false, 8, 8, 2, 4, 0>(p, acc, ep_slab, m_wave, n_wave, lane, wide_stores);
+                if (p.addend != nullptr) staged_epilogue<DT, MODE, true, 8, 8, 2, 4, 0, true>(p, acc, ep_slab, m_wave, n_wave, lane, wide);
+                else staged_epilogue<DT, MODE, true, 8, 8, 2, 4, 0>(p, acc, ep_slab, m_wave, n_wave, lane, wide);
+            } else if (p.addend != nullptr) staged_epilogue<DT, MODE, false, 8, 8, 2, 4, 0, true>(p, acc, ep_slab, m_wave, n_wave, lane, wide);
+            else staged_epilogue<DT, MODE, false, 8, 8, 2, 4, 0>(p, acc, ep_slab, m_wave, n_wave, lane, wide);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no global->LDS load in flight when the wavefront leaves
@@ -890,7 +891,7 @@ __global__ __launch_bounds__(256) void gemm_direct128_kernel(GemmParams p) {
         // the stages are free once every wavefront has read its last fragments: a slab per wavefront at their start
         __syncthreads();
         char *slab = smem + wave * (16 * EP_PITCH);
-        const bool wide = (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && p.ldy % 8 == 0;
+        const bool wide = wide_stores(p);
         const int m_wave = m0 + wm * 64, n_wave = n0 + (MODE == MODE_SWIGLU ? wn * 32 : wn * 64);
         if constexpr (MODE == MODE_SWIGLU) {
             staged_epilogue<DT, MODE, false, 4, 4, 1, 2, 2>(p, acc, slab, m_wave, n_wave, lane, wide);
@@ -936,7 +937,10 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(GemmParams p, int sp
             }
         }
         const char *add_row = MODE == MODE_LINEAR && p.addend != nullptr ? p.addend + static_cast<int64_t>(m) * p.ldadd * 2 : nullptr;
-        *reinterpret_cast<uint2 *>(p.y + (static_cast<int64_t>(m) * p.ldy + n) * 2) = finish4<DT, MODE>(p, g, u, n, add_row);
+        const uint2 o = finish4<DT, MODE>(p, g, u, n, add_row);
+        char *dst = p.y + (static_cast<int64_t>(m) * p.ldy + n) * 2;
+        *reinterpret_cast<uint2 *>(dst) = o;
+        if (p.copy) *reinterpret_cast<uint2 *>(dst + p.copy) = o;
     }
 }
 
@@ -1020,6 +1024,7 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(GemmParams p) {
                 }
             }
             store_elem<DT>(p.y, static_cast<int64_t>(m) * p.ldy + n, v);
+            if (p.copy) store_elem<DT>(p.y + p.copy, static_cast<int64_t>(m) * p.ldy + n, v);
         }
     }
 }
@@ -1513,7 +1518,7 @@ __global__ __launch_bounds__(256) void gemm_w8_direct_kernel(GemmParams p, W8Ext
             }
         }
     } else {
-        const bool wide = (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && p.ldy % 8 == 0;
+        const bool wide = wide_stores(p);
         char *slab = smem + wave * (16 * EP_PITCH);  // the stages (and the outlier tiles) are read out
         if (p.act == TPAMD_ACT_GELU) staged_epilogue<DT, MODE_LINEAR, true, TMX, 4, 1, 4, 0>(p, acc, slab, m0, n_wave, lane, wide);
         else staged_epilogue<DT, MODE_LINEAR, false, TMX, 4, 1, 4, 0>(p, acc, slab, m0, n_wave, lane, wide);
@@ -1618,7 +1623,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_f32_kernel(GemmPar
     extern __shared__ __align__(16) char smem[];
 
     int tile_m, tile_n;
-    tile_of_block(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    tile_of_block(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n * p.ranks, tile_m, tile_n);
+    take_rank(p, tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
@@ -1721,6 +1727,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_f32_kernel(GemmPar
                 }
                 if (p.addend != nullptr) v += *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(p.addend) + static_cast<int64_t>(m) * p.ldadd + n);
                 *reinterpret_cast<f32x4 *>(yrow + n) = v;
+                if (p.copy) *reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(yrow + n) + p.copy) = v;
             }
     }
 }
@@ -1734,7 +1741,9 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(GemmParams p) {
     constexpr int XC = T * CPR / NT;  // 16-byte chunks per thread and operand
     constexpr int STAGE = 2 * T * ROW;
     extern __shared__ __align__(16) char smem[];
-    const int tile_n = blockIdx.x % p.tiles_n, tile_m = blockIdx.x / p.tiles_n;
+    int tile_n = blockIdx.x % (p.tiles_n * p.ranks);
+    const int tile_m = blockIdx.x / (p.tiles_n * p.ranks);
+    take_rank(p, tile_n);
     const int m0 = tile_m * T, n0 = tile_n * T;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, lhi = lane >> 5;
@@ -1815,7 +1824,9 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(GemmParams p) {
         for (int j = 0; j < 4; ++j) v[j] = gelu_erf(v[j]);
     }
     if (p.addend != nullptr) v += *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(p.addend) + static_cast<int64_t>(m) * p.ldadd + n);
-    *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(p.y) + static_cast<int64_t>(m) * p.ldy + n) = v;
+    float *dst = reinterpret_cast<float *>(p.y) + static_cast<int64_t>(m) * p.ldy + n;
+    *reinterpret_cast<f32x4 *>(dst) = v;
+    if (p.copy) *reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(dst) + p.copy) = v;
 }
 
 int launch_gemm_f32_small(GemmParams p, hipStream_t s) {
@@ -1829,7 +1840,7 @@ int launch_gemm_f32_small(GemmParams p, hipStream_t s) {
     }
     p.tiles_m = (p.M + 31) / 32;
     p.tiles_n = (p.N + 31) / 32;
-    const int64_t blocks = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
+    const int64_t blocks = static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.ranks;
     TPAMD_REQUIRE(blocks < (1ll << 31), "gemm: too many tiles");
     hipLaunchKernelGGL(gemm_f32_small_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), LDS, s, p);
     TPAMD_HIP(hipGetLastError());
@@ -1850,7 +1861,7 @@ int launch_gemm_f32(GemmParams p, hipStream_t s) {
     }
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
-    const int64_t blocks = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
+    const int64_t blocks = static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.ranks;
     TPAMD_REQUIRE(blocks < (1ll << 31), "gemm: too many tiles");
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(NT), LDS, s, p);
     TPAMD_HIP(hipGetLastError());
@@ -2141,11 +2152,13 @@ int generic_dispatch(const GemmParams &p, int dtype, bool swiglu, hipStream_t s)
     return dtype == TPAMD_BF16 ? launch_generic<TPAMD_BF16>(p, swiglu, s) : launch_generic<TPAMD_F16>(p, swiglu, s);
 }
 
-// `second` (16-bit operands of the fast kernels, no addend): the same work for a second rank, its operands that far from the first one's.
+// `second` (operands of the kernels with 16-byte accesses, no addend): the same work for a second rank, its operands that far from the first one's.
+// `copy`: bytes to a second place for every output, 0 for none.
 int gemm_dispatch(const void *x, const void *w, const void *w2, const void *bias, const void *addend, int64_t ldadd, void *y,
                   int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, int act, bool swiglu,
-                  bool generic, hipStream_t s, const RankStep *second) {
+                  bool generic, hipStream_t s, const RankStep *second, int64_t copy) {
     GemmParams p{};
+    p.copy = copy;
     p.ranks = second != nullptr ? 2 : 1;
     if (second != nullptr) p.to = *second;
     p.x = static_cast<const char *>(x);
@@ -2159,19 +2172,22 @@ int gemm_dispatch(const void *x, const void *w, const void *w2, const void *bias
     p.act = act;
     if (dtype == TPAMD_F32 && !swiglu && K >= 4 && K % 4 == 0 && N % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && ldy % 4 == 0 &&
         aligned(x, 16) && aligned(w, 16) && aligned(y, 16) && (!bias || aligned(bias, 16)) &&
-        (!addend || (aligned(addend, 16) && ldadd % 4 == 0))) {
+        (!addend || (aligned(addend, 16) && ldadd % 4 == 0)) && copy % 16 == 0) {
         // fp32 rows that 16-byte accesses can take: the matrix pipe. 128 x 128 tiles once they fill the CUs, else 64 x 64.
         int dev = 0, cus = 256;
         TPAMD_HIP(hipGetDevice(&dev));
         if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
-        const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
+        const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128) * p.ranks;
         if (tiles128 >= cus) return launch_gemm_f32<128, 128, 2, 2, 32>(p, s);
-        const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
+        const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64) * p.ranks;
         if (tiles64 >= 2 * cus) return launch_gemm_f32<64, 64, 2, 2, 32>(p, s);
         if (tiles64 * 2 >= cus) return launch_gemm_f32<64, 64, 2, 2, 128>(p, s);  // few tiles: long stages, a block per CU
         return launch_gemm_f32_small(p, s);  // fewer still: 32 x 32 tiles whose K is shared by the block's wavefronts
     }
-    if (dtype == TPAMD_F32 || generic) return generic_dispatch(p, dtype, swiglu, s);
+    if (dtype == TPAMD_F32 || generic) {
+        TPAMD_REQUIRE(p.ranks == 1, "linear (generic kernel): one rank per launch");
+        return generic_dispatch(p, dtype, swiglu, s);
+    }
     return dtype == TPAMD_BF16 ? gemm_large<TPAMD_BF16>(p, swiglu, s) : gemm_large<TPAMD_F16>(p, swiglu, s);
 }
 

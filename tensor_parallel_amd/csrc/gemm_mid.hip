@@ -160,7 +160,7 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
     fence();
     drain_and_barrier();
 
-    const bool wide = (reinterpret_cast<uintptr_t>(p.y) & 15) == 0 && p.ldy % 8 == 0;
+    const bool wide = wide_stores(p);
     char *slab = smem + wave * (16 * EP_PITCH);  // the stages are read out
     const int m_wave = m0 + wm * TMX * 16;
     if constexpr (MODE == MODE_SWIGLU) {

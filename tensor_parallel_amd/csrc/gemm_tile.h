@@ -27,7 +27,12 @@ struct GemmParams {
     int splits;         // split-K of the 256 x 256 kernel: work units = tiles x splits
     int ranks;          // 1, or 2: a second rank's columns follow the first one's, `to` leads to its operands
     RankStep to;
+    int64_t copy;       // every output is stored a second time that many bytes on (0: once)
 };
+
+__device__ __forceinline__ bool wide_stores(const GemmParams &p) {  // 16 bytes each
+    return ((reinterpret_cast<uintptr_t>(p.y) | static_cast<uintptr_t>(p.copy)) & 15) == 0 && p.ldy % 8 == 0;
+}
 
 // Which rank's column tile this is.
 __device__ __forceinline__ void take_rank(GemmParams &p, int &tile_n) {
@@ -158,7 +163,9 @@ __device__ __forceinline__ void epilogue16(const GemmParams &p, f32x4 (&acc)[TMX
                 u[j] = MODE == MODE_SWIGLU ? acc[a][(b + 2) & 3][j] : 0.f;
             }
             const char *add_row = MODE == MODE_LINEAR && p.addend != nullptr ? p.addend + static_cast<int64_t>(m) * p.ldadd * 2 : nullptr;
-            *reinterpret_cast<uint2 *>(yrow + static_cast<int64_t>(n) * 2) = finish4<DT, MODE>(p, g, u, n, add_row);
+            const uint2 o = finish4<DT, MODE>(p, g, u, n, add_row);
+            *reinterpret_cast<uint2 *>(yrow + static_cast<int64_t>(n) * 2) = o;
+            if (p.copy) *reinterpret_cast<uint2 *>(yrow + static_cast<int64_t>(n) * 2 + p.copy) = o;
         }
     }
 }
@@ -261,14 +268,20 @@ __device__ __forceinline__ void staged_epilogue(const GemmParams &p, f32x4 (&acc
                         v.z = add_packed2<DT>(v.z, a1.x); v.w = add_packed2<DT>(v.w, a1.y);
                     }
                 }
-                if (n + 8 <= p.N) {
-                    if (wide) *reinterpret_cast<uint4 *>(dst) = v;
-                    else {
-                        *reinterpret_cast<uint2 *>(dst) = make_uint2(v.x, v.y);
-                        *reinterpret_cast<uint2 *>(dst + 8) = make_uint2(v.z, v.w);
+                auto put = [&](char *to) {
+                    if (n + 8 <= p.N) {
+                        if (wide) *reinterpret_cast<uint4 *>(to) = v;
+                        else {
+                            *reinterpret_cast<uint2 *>(to) = make_uint2(v.x, v.y);
+                            *reinterpret_cast<uint2 *>(to + 8) = make_uint2(v.z, v.w);
+                        }
+                    } else {
+                        *reinterpret_cast<uint2 *>(to) = make_uint2(v.x, v.y);  // N is a multiple of 4
                     }
-                } else {
-                    *reinterpret_cast<uint2 *>(dst) = make_uint2(v.x, v.y);  // N is a multiple of 4
+                };
+                put(dst);
+                if constexpr (MODE == MODE_LINEAR) {
+                    if (p.copy) put(dst + p.copy);
                 }
             }
             __builtin_amdgcn_wave_barrier();

@@ -45,6 +45,7 @@ struct SkinnyParams {
     int act;
     int ranks;     // 1, or 2: blockIdx.z is the rank, `to` the way to the second one's operands
     RankStep to;
+    int64_t copy;  // every output is stored a second time that many bytes on (0: once)
 };
 
 // This block's rank.
@@ -83,6 +84,9 @@ __device__ __forceinline__ void skinny_store_output(const SkinnyParams &p, float
             out = f32_to_half<DT>(half_to_f32<DT>(out) + half_to_f32<DT>(reinterpret_cast<const uint16_t *>(p.addend)[static_cast<int64_t>(m) * p.ldadd + n]));
     }
     reinterpret_cast<uint16_t *>(p.y)[static_cast<int64_t>(m) * p.ldy + n] = out;
+    if constexpr (MODE == SK_LINEAR) {
+        if (p.copy) reinterpret_cast<uint16_t *>(p.y + p.copy)[static_cast<int64_t>(m) * p.ldy + n] = out;
+    }
 }
 
 // W8 = weight is int8. MT = number of 16-row tiles of x (M <= 16*MT). MODE = SK_LINEAR / SK_SWIGLU.
@@ -1903,11 +1907,13 @@ int launch_skinny(const SkinnyParams &p, hipStream_t s) {
 
 // M <= 64. dtype is BF16 or F16. `w8` selects the int8 weight path (linear only). `second`: the same work for a second rank in the same
 // launches, its operands that far from the first one's (no addend); the rules then see the columns of both.
+// `copy`: bytes to a second place for every output, 0 for none.
 int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bias, const void *addend, int64_t ldadd,
                     const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out, void *y, int64_t M, int64_t N,
                     int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int64_t ld_wout, int dtype, int act, bool swiglu, bool w8,
-                    hipStream_t s, const RankStep *second) {
+                    hipStream_t s, const RankStep *second, int64_t copy) {
     SkinnyParams p{};
+    p.copy = copy;
     p.ranks = second != nullptr ? 2 : 1;
     if (second != nullptr) p.to = *second;
     p.x = static_cast<const char *>(x);

@@ -57,7 +57,7 @@ def linear_in_context(module: nn.Module, x: torch.Tensor, w: torch.Tensor, bias)
         return _guard(together.linear(x.detach(), w.detach(), b), x, w, bias)
     key = id(module)
     ctx.calls[key] = ctx.calls.get(key, 0) + 1
-    addend = None
+    addend = copy = None
     if module.__dict__.get("_tp_feeds_sum") is ctx.owner and ctx.owner is not None:
         if ctx.fused_out is not None:
             raise RuntimeError("tensor_parallel_amd: the Linear that feeds a \"sum\" rule ran twice in one call of its module "
@@ -67,16 +67,35 @@ def linear_in_context(module: nn.Module, x: torch.Tensor, w: torch.Tensor, bias)
             t, mask = waiting
             if t.dtype == x.dtype and t.device == x.device and t.shape == (*x.shape[:-1], w.shape[0]):
                 addend, ctx.fused_mask = t.detach(), mask
+                if ctx.op.world_size == 2:  # the sum is complete then: a second tensor for the other rank comes out of the same launch
+                    copy = torch.empty_like(addend, memory_format=torch.contiguous_format)
     # Ranks do not meet in the Linear that feeds the sum (the one that comes last adds the others' partials), nor before a first call has shown which one that is.
     if "_tp_sum_known" in ctx.owner.__dict__ and module.__dict__.get("_tp_feeds_sum") is not ctx.owner:
         out = together.linear(x.detach(), w.detach(), b)
     else:
-        out = _native.linear(x.detach(), w.detach(), b, addend=addend)
+        out = _native.linear(x.detach(), w.detach(), b, addend=addend, **({} if copy is None else {"copy": copy}))
     out = _guard(out, x, w, bias)
     if addend is not None:
         ctx.fused_out = out
+        if copy is not None and not out.is_inference():  # (whose changes are not counted)
+            ctx.fused_copy = copy, out._version
     ctx.last_linear, ctx.last_out = module, out
     return out
+
+
+def gathered_linear(module: nn.Module, op, rank: int, args, kwargs):
+    """The gathered output of a column-parallel Linear, written by one launch for two ranks (`tpamd_linear_gather_ranks`) instead of a Linear
+    for each and a concatenation behind them; None where that is not to be had: another module than a plain shard Linear, somebody who watches its
+    own output, another axis, a rank whose peer does not come with a Linear of the same form."""
+    hooks = torch.nn.modules.module
+    if (type(module) is not ShardLinear or "forward" in module.__dict__ or kwargs or len(args) != 1 or _has_hooks(module)
+            or hooks._global_forward_hooks or hooks._global_forward_pre_hooks):
+        return None
+    x, w, bias = args[0], module.weight, module.bias
+    if not _native.plain_call(x, w) or not x.is_cuda or op.dim not in (-1, x.dim() - 1) or x.dtype != w.dtype:
+        return None
+    whole = together.linear_gathered(x.detach(), w.detach(), None if bias is None else bias.detach(), rank, op.world_size)
+    return None if whole is None else _guard(whole, x, w, bias)
 
 
 class ShardLinear(nn.Linear):

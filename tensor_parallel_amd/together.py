@@ -107,21 +107,21 @@ class GreenTurn:
             self.at = 0
         self.idle = 0
 
-    def meet(self, one: Callable[..., Any], many: Callable[[List[tuple]], Sequence[Any]], tensors: tuple, more: tuple) -> Any:
-        """one(*tensors, *more), made as many([...]) for all ranks that come with tensors of the same forms and the same `more`. A rank whose
-        peers do not come (they wait elsewhere or have returned) makes the call alone (`part`)."""
+    def meet(self, one: Callable[..., Any], many: Callable[[List[tuple]], Sequence[Any]], tensors: tuple, more: tuple, own: tuple = ()) -> Any:
+        """one(*tensors, *more, *own), made as many([...]) for all ranks that come with tensors of the same forms and the same `more`, in the order in
+        which they came. A rank whose peers do not come (they wait elsewhere or have returned) makes the call alone (`part`)."""
         for meeting in self.open:
-            if meeting.one is one and meeting.more == more and _alike(meeting.calls[0], tensors):
+            if meeting.one is one and meeting.more == more and _alike(meeting.calls[0][0], tensors):
                 break
         else:
             meeting = _Meeting(one, many, more)
             self.open.append(meeting)
         place = len(meeting.calls)
-        meeting.calls.append(tensors)
+        meeting.calls.append((tensors, own))
         if place + 1 == self.world:
             self.open.remove(meeting)
             try:
-                meeting.results = many([tensors + more for tensors in meeting.calls])
+                meeting.results = many([tensors + more + own for tensors, own in meeting.calls])
             except BaseException as e:  # every rank that handed something in sees it
                 meeting.error = e
             self.idle = 0
@@ -141,17 +141,17 @@ class GreenTurn:
         meetings, self.open = self.open, []
         for m in meetings:
             try:
-                m.results = [m.one(*tensors, *m.more) for tensors in m.calls]
+                m.results = [m.one(*tensors, *m.more, *own) for tensors, own in m.calls]
             except BaseException as e:
                 m.error = e
         return True
 
 
-def _call(one: Callable[..., Any], many: Callable[[List[tuple]], Sequence[Any]], tensors: tuple, more: tuple = ()) -> Any:
+def _call(one: Callable[..., Any], many: Callable[[List[tuple]], Sequence[Any]], tensors: tuple, more: tuple = (), own: tuple = ()) -> Any:
     turn = _turn.get()
     if type(turn) is not GreenTurn or turn.world < 2 or turn.failed or _thread_state(turn.index) != turn.state:
-        return one(*tensors, *more)
-    return turn.meet(one, many, tensors, more)
+        return one(*tensors, *more, *own)
+    return turn.meet(one, many, tensors, more, own)
 
 
 # From this many rows on a product fills the device by itself, in 256 x 256 tiles that take two ranks in two launches anyway, and each rank's
@@ -171,6 +171,21 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     return _call(_native.linear, _native.linear_ranks, (x, w, bias))
 
 
+def _not_together(*_: Any) -> None:
+    return None
+
+
+def _gather(calls: List[tuple]) -> Sequence[torch.Tensor]:
+    return _native.linear_gather_ranks([call[:3] for call in sorted(calls, key=lambda call: call[3])])  # (every rank's result is the same)
+
+
+def linear_gathered(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], rank: int, world: int) -> Optional[torch.Tensor]:
+    """The Linears of two ranks with their results side by side, a whole one for each, in one launch; None where this rank is on its own."""
+    if world != 2:
+        return None
+    return _call(_not_together, _gather, (x, w, bias), (), (rank,))
+
+
 def swiglu_up(x: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor) -> torch.Tensor:
     if not _few_rows(x):
         return _native.swiglu_up(x, wg, wu)
@@ -178,10 +193,14 @@ def swiglu_up(x: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor) -> torch.Tens
 
 
 def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    if x.numel() >= ALONE_ROWS * w.numel():
+        return _native.rms_norm(x, w, eps)
     return _call(_native.rms_norm, _native.rms_norm_ranks, (x, w), (eps,))
 
 
 def add_rms_norm(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float) -> tuple:
+    if x.numel() >= ALONE_ROWS * w.numel():
+        return _native.add_rms_norm(r, x, w, eps)
     return _call(_native.add_rms_norm, _native.add_rms_norm_ranks, (r, x, w), (eps,))
 
 

@@ -15,8 +15,9 @@ import torch
 from torch import nn
 
 from . import _native
-from .collectives import DeviceAllReduce, SumContext, pop_sum_context, push_sum_context
+from .collectives import DeviceAllGather, DeviceAllReduce, SumContext, pop_sum_context, push_sum_context
 from .config import MappedActions
+from .shard_modules import gathered_linear
 from .slicing import SliceSpec, apply_spec, normalize_dim, tensor_split_range
 
 
@@ -111,11 +112,17 @@ class TensorParallelWrapper(nn.Module):
         # output 0 summed over the ranks on one device: the module's last Linear may take the sum into its epilogue
         action = output_actions.get(0) if output_actions else None
         self._sum_op = action if isinstance(action, DeviceAllReduce) else None
+        # ... and a Linear whose output is nothing but gathered may write every rank's whole output itself
+        self._gather_op = action if type(action) is DeviceAllGather and len(output_actions) == 1 else None
 
     def forward(self, *args, **kwargs):
         call_args, call_kwargs = args, kwargs
         if self.input_actions:
             call_args, call_kwargs = process_input(self.input_actions, self.rank, self.world_size, *args, **kwargs)
+        if self._gather_op is not None:
+            whole = gathered_linear(self.tp_wrapped_module, self._gather_op, self.rank, call_args, call_kwargs)
+            if whole is not None:
+                return whole
         # Every wrapper publishes its own context, or none: Linears and rules inside a wrapper without a foldable sum must
         # not be taken for those of an enclosing module whose output is summed.
         foldable = self._sum_op is not None and self._sum_op.fusable

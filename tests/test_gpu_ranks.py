@@ -137,3 +137,71 @@ def test_ranks_that_do_not_fit_each_other_make_their_calls_alone():
         assert len(got[r]) == len(wants)
         for a, b in zip(got[r], wants):
             close(a, b, torch.bfloat16)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows", [1, 3, 4, 16, 33, 64, 129, 700])
+@pytest.mark.parametrize("cols,K,n", [(4, 8, 2), (384, 768, 2), (3072, 768, 2), (1000, 1088, 2), (516, 264, 3), (7, 30, 2)])
+def test_gathered_linears_are_the_linears_side_by_side(rows, cols, K, n, dtype):
+    xs, ws = draws(n, rows, K, dtype=dtype), draws(n, cols, K, dtype=dtype, scale=0.05, seed=1)
+    bs = draws(n, cols, dtype=dtype, seed=2) if rows % 2 else [None] * n
+    ys = _native.linear_gather_ranks(list(zip(xs, ws, bs)))
+    want = torch.cat([x.double() @ w.double().t() + (0 if b is None else b.double()) for x, w, b in zip(xs, ws, bs)], -1)
+    assert len({y.data_ptr() for y in ys}) == n and all(torch.equal(y, ys[0]) for y in ys)
+    if dtype is torch.float32:  # sums of K products in fp32: at most K * 2^-24 of the sum of their magnitudes
+        bound = K * 2.0 ** -24 * max(float((x.abs().double() @ w.abs().double().t()).max()) for x, w in zip(xs, ws)) + 1e-6
+        assert float((ys[0].double() - want).abs().max()) <= bound
+    else:
+        close(ys[0], want.float(), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows", [1, 3, 4, 16, 17, 64, 129, 700, 2100])
+@pytest.mark.parametrize("cols,K", [(4, 8), (516, 264), (4096, 2048), (1030, 1096), (7, 30)])
+def test_the_copy_of_a_sum_is_the_sum(rows, cols, K, dtype):
+    x, w, addend = draws(1, rows, K, dtype=dtype)[0], draws(1, cols, K, dtype=dtype, scale=0.05, seed=1)[0], draws(1, rows, cols, dtype=dtype, seed=2)[0]
+    copy = torch.full_like(addend, float("nan"))
+    y = _native.linear(x, w, addend=addend, copy=copy)
+    assert torch.equal(y, copy) and torch.equal(y, _native.linear(x, w, addend=addend))
+
+
+@pytest.mark.parametrize("rank", [0, 1])
+def test_a_sum_that_somebody_writes_to_is_copied_as_it_is(rank):
+    from types import SimpleNamespace
+
+    import tensor_parallel_amd as tp
+    from tensor_parallel_amd.slicing_configs import get_llama_config
+    from torch import nn
+
+    class Mlp(nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.gate_proj, self.up_proj, self.down_proj = nn.Linear(64, 128, bias=False), nn.Linear(64, 128, bias=False), nn.Linear(128, 64, bias=False)
+            self.act_fn = nn.SiLU()
+
+        def forward(self, x):
+            return self.down_proj(self.act_fn(self.gate_proj(x)) * self.up_proj(x))
+
+    class Block(nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.mlp = Mlp()
+
+        def forward(self, x):
+            return self.mlp(x)
+
+    torch.manual_seed(0)
+    cfg = get_llama_config(SimpleNamespace(model_type="llama", hidden_size=64, num_attention_heads=4, num_key_value_heads=4), [DEV] * 2)
+    model = tp.TensorParallel(Block().bfloat16().to(DEV), [DEV] * 2, tensor_parallel_config=cfg, sharded=False)
+    x = torch.randn(5, 64, device=DEV).bfloat16()
+    with torch.no_grad():
+        want = [model(x) for _ in range(3)][-1]
+        # one of the ranks comes last and its down projection holds the sum: what a hook adds to that in place is in the sum of both ranks
+        handle = model.module_shards[rank].mlp.tp_wrapped_module.down_proj.register_forward_hook(lambda m, i, out: out.add_(1.0))
+        ranks = []
+        for shard in model.module_shards:
+            shard.register_forward_hook(lambda m, i, out: ranks.append(out))
+        model(x)
+        handle.remove()
+    assert len(ranks) == 2 and torch.equal(ranks[0], ranks[1])
+    torch.testing.assert_close(ranks[0], want + 1.0, rtol=2.0 ** -7, atol=0)  # added before or after the sum: two roundings of 2^-9 around 1

@@ -146,3 +146,15 @@ def test_a_failure_reaches_every_rank_and_the_next_forward_works(calls, monkeypa
     monkeypatch.setattr(_native, "linear_ranks", good)
     run(lambda r: together.linear(*operands(r)), lambda r: together.linear(*operands(r)))
     assert calls[-1] == 2
+
+
+def test_gathered_columns_are_in_rank_order_whoever_came_first(monkeypatch):
+    monkeypatch.setattr(_native, "linear_gather_ranks", lambda items: [torch.cat([torch.nn.functional.linear(*item) for item in items], -1)] * len(items))
+    want = torch.cat([torch.nn.functional.linear(*operands(r)) for r in range(2)], -1)
+
+    def body(r):
+        return [together.linear_gathered(*operands(r), None, r, 2) for _ in range(3)]
+
+    for got in run(body, body):  # whoever came last goes on first
+        assert all(torch.equal(y, want) for y in got)
+    assert run(lambda r: together.linear_gathered(*operands(r), None, r, 2), lambda r: r) == [None, 1]  # the peer does not come: nothing is gathered
