@@ -343,6 +343,12 @@ int tpamd_add_rms_norm_ranks(int n, const void *const *x_dev, const void *const 
                              void *const *y_dev, int64_t rows, int64_t D, int64_t ldx, int64_t ldr, int64_t ldy, float eps, int dtype,
                              void *stream);
 
+/* y[r] = (x - mean) * rsqrt(var + eps) * w + b over rows of D elements (torch.nn.LayerNorm of the wrapped modules, which every rank computes on
+ * whole rows; src/tensor_parallel/wrapper.py:69-72): mean and variance in fp32, one rounding to `dtype` (BF16, F16 or F32). b_dev NULL: no
+ * bias. y may be x. Rows of up to 16384 (F32: 8192) elements on 16-byte boundaries are read once; anything else takes a kernel with element loads. */
+int tpamd_layer_norm_ranks(int n, const void *const *x_dev, const void *const *w_dev, const void *const *b_dev, void *const *y_dev, int64_t rows,
+                           int64_t D, int64_t ldx, int64_t ldy, float eps, int dtype, void *stream);
+
 typedef struct {
     const void *q, *k, *v, *cos, *sin;
     void *k_cache, *v_cache, *out;

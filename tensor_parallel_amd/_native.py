@@ -53,6 +53,7 @@ EXPORTS = (
     "tpamd_linear_w8_ranks",
     "tpamd_linear_add_copy",
     "tpamd_linear_gather_ranks",
+    "tpamd_layer_norm_ranks",
 )
 
 ABI_VERSION = 6
@@ -168,6 +169,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_swiglu_up_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, i64, i64, ci, vp]
     lib.tpamd_rms_norm_ranks.restype = ci
     lib.tpamd_rms_norm_ranks.argtypes = [ci, pp, pp, pp, i64, i64, i64, i64, c.c_float, ci, vp]
+    lib.tpamd_layer_norm_ranks.restype = ci
+    lib.tpamd_layer_norm_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, c.c_float, ci, vp]
     lib.tpamd_add_rms_norm_ranks.restype = ci
     lib.tpamd_add_rms_norm_ranks.argtypes = [ci, pp, pp, pp, pp, pp, i64, i64, i64, i64, i64, c.c_float, ci, vp]
     lib.tpamd_attention_decode_rope_ranks.restype = ci
@@ -666,6 +669,31 @@ def add_rms_norm_ranks(calls: Sequence[tuple]) -> list:
             "tpamd_add_rms_norm",
         )
     return [(total.view(x.shape), y.view(x.shape)) for total, y in zip(totals, ys)]
+
+
+def layer_norm(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], eps: float) -> torch.Tensor:
+    """(x - mean) * rsqrt(var + eps) * w + b over the last axis, in fp32, rounded once."""
+    return layer_norm_ranks([(x, w, b, eps)])[0]
+
+
+def layer_norm_ranks(calls: Sequence[tuple]) -> list:
+    """`layer_norm(x, w, b, eps)` for the operands of several ranks (with one eps)."""
+    x, w, b, eps = calls[0]
+    require_device(x, "layer_norm")
+    for t in (w, b):
+        if t is not None and (t.dtype != x.dtype or t.get_device() != x.get_device() or t.dim() != 1 or x.dim() == 0 or x.shape[-1] != t.shape[0]):
+            raise ValueError(f"layer_norm: x {tuple(x.shape)} {x.dtype} on {x.device} and {tuple(t.shape)} {t.dtype} on {t.device} do not fit")
+    xs, ws = [_as_2d(c[0]) for c in calls], [c[1].contiguous() for c in calls]
+    bs = None if b is None else [c[2].contiguous() for c in calls]
+    rows, D = xs[0].shape
+    ys = [torch.empty((rows, D), dtype=x.dtype, device=x.device) for _ in calls]
+    with _on_device(x.device):
+        _check(
+            lib().tpamd_layer_norm_ranks(len(calls), _pointers(xs), _pointers(ws), None if bs is None else _pointers(bs), _pointers(ys), rows, D,
+                                         _ld(xs[0]), D, float(eps), dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device))),
+            "tpamd_layer_norm",
+        )
+    return [y.view(x.shape) for y in ys]
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None, causal: bool = True,

@@ -204,6 +204,12 @@ def add_rms_norm(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float) 
     return _call(_native.add_rms_norm, _native.add_rms_norm_ranks, (r, x, w), (eps,))
 
 
+def layer_norm(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], eps: float) -> torch.Tensor:
+    if x.numel() >= ALONE_ROWS * w.numel():
+        return _native.layer_norm(x, w, b, eps)
+    return _call(_native.layer_norm, _native.layer_norm_ranks, (x, w, b), (eps,))
+
+
 def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, outlier_idx: Optional[torch.Tensor], w_out: Optional[torch.Tensor],
               bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     return _call(_native.linear_w8, _native.linear_w8_ranks, (x, wq, scale, outlier_idx, w_out, bias))

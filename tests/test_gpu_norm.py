@@ -131,3 +131,56 @@ def test_more_rows_than_one_launch_takes():
     for at in (slice(0, 5), slice((1 << 23) - 2, (1 << 23) + 2), slice(rows - 5, rows)):
         assert torch.equal(_native.rms_norm(x, w, 1e-6)[at], _native.rms_norm(x[at].contiguous(), w, 1e-6))
         assert torch.equal(total[at], 2 * x[at]) and torch.equal(y[at], _native.rms_norm(2 * x[at], w, 1e-6))
+
+
+# one row, odd rows; a lone element, a row of less than a chunk, ragged rows (element loads), whole chunks on both sides of every block size, the longest
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,D", [(1, 1), (3, 7), (5, 8), (2, 512), (2, 520), (129, 768), (7, 2048), (3, 2056), (2, 4104), (16, 8192), (2, 8200), (1, 16384), (1, 16392)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_layer_norm_against_64_bits(rows, D, dtype, bias):
+    g = torch.Generator(device="cuda").manual_seed(rows * D)
+    x = (torch.randn(rows, D, device="cuda", generator=g) * 2 + 3).to(dtype)
+    w, b = (torch.randn(D, device="cuda", generator=g).to(dtype) for _ in range(2))
+    b = b if bias else None
+    y = _native.layer_norm(x, w, b, 1e-5)
+    want = torch.nn.functional.layer_norm(x.double(), (D,), w.double(), None if b is None else b.double(), 1e-5)
+    torchs = torch.nn.functional.layer_norm(x, (D,), w, b, 1e-5)
+    # one rounding of the result; in fp32 what the sums of D elements leave (pairwise over lanes: log2 of their number), and no further off than torch's own
+    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -20}[dtype]
+    err, theirs = ((t.double() - want).abs().max().item() for t in (y, torchs))
+    assert err <= max(eps * want.abs().max().item(), 1.5 * theirs)
+    if D > 8:  # rows that are pieces of longer ones, a pitch that 16-byte loads cannot take
+        wide = torch.cat([x, x], -1)[:, 1:D + 1] if D % 2 else torch.cat([x, x[:, :1]], -1)[:, :D]
+        got = _native.layer_norm(wide, w, b, 1e-5)
+        ref = torch.nn.functional.layer_norm(wide.double(), (D,), w.double(), None if b is None else b.double(), 1e-5)
+        assert (got.double() - ref).abs().max().item() <= max(eps * ref.abs().max().item(), 1.5 * theirs)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 60000.0])
+def test_layer_norm_of_extreme_rows_is_torchs(value):
+    x = torch.randn(3, 264, device="cuda", dtype=torch.float16)
+    x[1, 5] = value
+    w, b = torch.ones(264, device="cuda", dtype=torch.float16), torch.zeros(264, device="cuda", dtype=torch.float16)
+    want = torch.nn.functional.layer_norm(x, (264,), w, b, 1e-5)
+    torch.testing.assert_close(_native.layer_norm(x, w, b, 1e-5), want, rtol=2.0 ** -9, atol=2.0 ** -10, equal_nan=True)  # a rounding on each side
+
+
+def test_layer_norms_of_a_shard():
+    from tensor_parallel_amd.shard_modules import ShardLayerNorm, install_shard_kernels
+
+    D = 2048
+    plain = torch.nn.LayerNorm(D).cuda()
+    m = torch.nn.Sequential(torch.nn.LayerNorm(D), torch.nn.LayerNorm((2, D)), torch.nn.LayerNorm(D, elementwise_affine=False)).cuda()
+    m[0].load_state_dict(plain.state_dict())
+    install_shard_kernels(m)
+    assert type(m[0]) is ShardLayerNorm and type(m[2]) is torch.nn.LayerNorm
+    x = torch.randn(5, 2, D, device="cuda")
+    with torch.no_grad():
+        torch.testing.assert_close(m(x), torch.nn.functional.layer_norm(torch.nn.functional.layer_norm(plain(x), (2, D)), (D,)), rtol=1e-5, atol=1e-6)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert m[0](x.bfloat16()).dtype == torch.float32 == plain(x.bfloat16()).dtype
+        scripted = torch.jit.script(m[0])
+        torch.testing.assert_close(scripted(x), plain(x), rtol=1e-5, atol=1e-6)
+    y = x.requires_grad_()
+    m[0](y).sum().backward()
+    assert y.grad is not None
