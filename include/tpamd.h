@@ -384,6 +384,12 @@ int tpamd_linear_w8(const void *x_dev, const void *wq_dev, const void *scale_dev
                     int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout, int64_t ldy, int dtype, int act,
                     void *stream);
 
+/* tpamd_linear_w8 followed by one step of the partial-sum reduction, y = round_dtype(round_dtype(...) + addend), as tpamd_linear_add; with
+ * copy_dev (may be NULL) every result is stored there too (leading dimension ldy), as tpamd_linear_add_copy. */
+int tpamd_linear_w8_add(const void *x_dev, const void *wq_dev, const void *scale_dev, const void *outlier_idx_dev, const void *w_out_dev,
+                        int64_t n_out, const void *bias_dev, const void *addend_dev, void *y_dev, void *copy_dev, int64_t M, int64_t N,
+                        int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout, int64_t ldadd, int64_t ldy, int dtype, int act, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

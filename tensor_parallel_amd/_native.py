@@ -54,6 +54,7 @@ EXPORTS = (
     "tpamd_linear_add_copy",
     "tpamd_linear_gather_ranks",
     "tpamd_layer_norm_ranks",
+    "tpamd_linear_w8_add",
 )
 
 ABI_VERSION = 6
@@ -169,6 +170,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_swiglu_up_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, i64, i64, ci, vp]
     lib.tpamd_rms_norm_ranks.restype = ci
     lib.tpamd_rms_norm_ranks.argtypes = [ci, pp, pp, pp, i64, i64, i64, i64, c.c_float, ci, vp]
+    lib.tpamd_linear_w8_add.restype = ci
+    lib.tpamd_linear_w8_add.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, i64, ci, ci, vp]
     lib.tpamd_layer_norm_ranks.restype = ci
     lib.tpamd_layer_norm_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, c.c_float, ci, vp]
     lib.tpamd_add_rms_norm_ranks.restype = ci
@@ -932,20 +935,33 @@ def attention_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos
 
 
 def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale_: torch.Tensor, outlier_idx: Optional[torch.Tensor],
-              w_out: Optional[torch.Tensor], bias: Optional[torch.Tensor] = None, act: int = ACT_NONE) -> torch.Tensor:
-    """Weight-only int8 Linear with outlier columns kept in the activation dtype."""
+              w_out: Optional[torch.Tensor], bias: Optional[torch.Tensor] = None, act: int = ACT_NONE,
+              addend: Optional[torch.Tensor] = None, copy: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Weight-only int8 Linear with outlier columns kept in the activation dtype. `addend` and `copy` as in `linear`."""
     x2, wq, scale_, outlier_idx, w_out, b = _w8_operands(x, wq, scale_, outlier_idx, w_out, bias)
     (M, K), N = x2.shape, wq.shape[0]
     n_out = 0 if outlier_idx is None else int(outlier_idx.numel())
+    if addend is not None and (addend.dtype != x.dtype or addend.device != x.device or addend.numel() != M * N or addend.shape[-1] != N):
+        raise ValueError("linear_w8: addend must have the shape, dtype and device of the result")
+    if copy is not None and (addend is None or copy.dtype != x.dtype or copy.device != x.device or copy.numel() != M * N or not copy.is_contiguous()):
+        raise ValueError("linear_w8: copy goes with an addend and must be a contiguous tensor of the result's size, dtype and device")
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    head = (x2.data_ptr(), wq.data_ptr(), scale_.data_ptr(), outlier_idx.data_ptr() if n_out else None, w_out.data_ptr() if n_out else None, n_out,
+            b.data_ptr() if b is not None else None)
     with _on_device(x.device):
-        _check(
-            lib().tpamd_linear_w8(x2.data_ptr(), wq.data_ptr(), scale_.data_ptr(),
-                                  outlier_idx.data_ptr() if n_out else None, w_out.data_ptr() if n_out else None, n_out,
-                                  b.data_ptr() if b is not None else None, y.data_ptr(), M, N, K, _ld(x2), K, max(n_out, 1), N,
-                                  dtype_code(x.dtype), act, ctypes.c_void_p(current_stream_ptr(x.device))),
-            "tpamd_linear_w8",
-        )
+        stream = ctypes.c_void_p(current_stream_ptr(x.device))
+        if addend is None:
+            _check(
+                lib().tpamd_linear_w8(*head, y.data_ptr(), M, N, K, _ld(x2), K, max(n_out, 1), N, dtype_code(x.dtype), act, stream),
+                "tpamd_linear_w8",
+            )
+        else:
+            a2 = _as_2d(addend)
+            _check(
+                lib().tpamd_linear_w8_add(*head, a2.data_ptr(), y.data_ptr(), None if copy is None else copy.data_ptr(), M, N, K, _ld(x2), K, max(n_out, 1),
+                                          _ld(a2), N, dtype_code(x.dtype), act, stream),
+                "tpamd_linear_w8_add",
+            )
     return y.view(*x.shape[:-1], N)
 
 

@@ -24,8 +24,8 @@ int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bi
 
 bool w8_direct_ok(int64_t K, int64_t ldx, int64_t ldw);
 int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out,
-                     const void *bias, void *y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout,
-                     int64_t ldy, int dtype, int act, hipStream_t s);
+                     const void *bias, const void *addend, int64_t ldadd, int64_t copy, void *y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                     int64_t ld_wout, int64_t ldy, int dtype, int act, hipStream_t s);
 
 int attention_dispatch(const void *q, const void *k, const void *v, void *o, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
                        int64_t Skv, int64_t D, const int64_t *strides, float scale, int causal, int dtype, hipStream_t s);
@@ -397,11 +397,10 @@ extern "C" int tpamd_attention_decode_rope_ranks(int n, const tpamd_decode_rank 
     return TPAMD_OK;
 }
 
-extern "C" int tpamd_linear_w8(const void *x_dev, const void *wq_dev, const void *scale_dev, const void *outlier_idx_dev,
-                               const void *w_out_dev, int64_t n_out, const void *bias_dev, void *y_dev, int64_t M, int64_t N,
-                               int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout, int64_t ldy, int dtype, int act,
-                               void *stream) {
-    const char *who = "tpamd_linear_w8";
+// The int8 Linear, with an addend (another rank's partial sum) added to the rounded result, and that stored to `copy_dev` too (NULL: not).
+static int w8_entry(const char *who, const void *x_dev, const void *wq_dev, const void *scale_dev, const void *outlier_idx_dev, const void *w_out_dev,
+                    int64_t n_out, const void *bias_dev, const void *addend_dev, int64_t ldadd, void *y_dev, void *copy_dev, int64_t M, int64_t N, int64_t K,
+                    int64_t ldx, int64_t ldw, int64_t ld_wout, int64_t ldy, int dtype, int act, void *stream) {
     TPAMD_REQUIRE(dtype == TPAMD_BF16 || dtype == TPAMD_F16, "%s: dtype must be BF16 or F16", who);
     TPAMD_REQUIRE(M >= 0 && N >= 0 && K >= 0 && n_out >= 0, "%s: negative dimension", who);
     TPAMD_REQUIRE(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "%s: dimension over 2^31", who);
@@ -413,6 +412,8 @@ extern "C" int tpamd_linear_w8(const void *x_dev, const void *wq_dev, const void
     TPAMD_REQUIRE(aligned(x_dev, 16) && aligned(wq_dev, 16), "%s: x and wq must be 16-byte aligned", who);
     TPAMD_REQUIRE(K % 16 == 0 && ldw % 16 == 0 && ldx % 8 == 0, "%s: K, ldw multiples of 16 and ldx of 8 required", who);
     TPAMD_REQUIRE(ldx >= K && ldw >= K && ldy >= N, "%s: leading dimension smaller than the row", who);
+    TPAMD_REQUIRE(addend_dev == nullptr || ldadd >= N, "%s: ldadd=%lld is smaller than N=%lld", who, (long long)ldadd, (long long)N);
+    const int64_t copy = bytes_from(y_dev, copy_dev);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int esz = 2;
     // The weight-streaming kernels take slabs of 64 rows; above one slab the weights go through the matrix pipe once, converted
@@ -426,19 +427,41 @@ extern "C" int tpamd_linear_w8(const void *x_dev, const void *wq_dev, const void
     bool tiled = w8_direct_ok(K, ldx, ldw) ? M > 128 || (M > SKINNY_W8_SLAB && N * K >= (M <= 80 ? 22ll : 6ll) * 1000 * 1000)
                                            : M > 256 || (M > 128 && tiles128 >= 256);
     if (tuning().w8_tile != TUNE_UNSET) tiled = tuning().w8_tile > 0 && M > 16;
-    if (tiled && N % 4 == 0 && ldy % 4 == 0 && aligned(y_dev, 8) && (!bias_dev || aligned(bias_dev, 8)) && n_out <= 256) {
-        const int rc = gemm_w8_dispatch(x_dev, wq_dev, scale_dev, outlier_idx_dev, w_out_dev, n_out, bias_dev, y_dev, M, N, K, ldx, ldw,
-                                        ld_wout, ldy, dtype, act, s);
+    if (tiled && N % 4 == 0 && ldy % 4 == 0 && aligned(y_dev, 8) && (!bias_dev || aligned(bias_dev, 8)) && n_out <= 256 &&
+        aligned(addend_dev, 8) && ldadd % 4 == 0 && aligned(copy_dev, 8)) {
+        const int rc = gemm_w8_dispatch(x_dev, wq_dev, scale_dev, outlier_idx_dev, w_out_dev, n_out, bias_dev, addend_dev, ldadd, copy, y_dev, M, N, K, ldx,
+                                        ldw, ld_wout, ldy, dtype, act, s);
         if (rc != TPAMD_ERR_UNSUPPORTED) return rc;  // else no scratch memory, and the slabs need none
     }
     for (int64_t m0 = 0; m0 < M; m0 += SKINNY_W8_SLAB) {  // weights are re-streamed once per slab of 64 rows
         const int64_t mm = M - m0 < SKINNY_W8_SLAB ? M - m0 : SKINNY_W8_SLAB;
-        int rc = skinny_dispatch(static_cast<const char *>(x_dev) + m0 * ldx * esz, wq_dev, nullptr, bias_dev, nullptr, 0, scale_dev,
+        int rc = skinny_dispatch(static_cast<const char *>(x_dev) + m0 * ldx * esz, wq_dev, nullptr, bias_dev,
+                                 addend_dev ? static_cast<const char *>(addend_dev) + m0 * ldadd * esz : nullptr, ldadd, scale_dev,
                                  outlier_idx_dev, w_out_dev, n_out, static_cast<char *>(y_dev) + m0 * ldy * esz, mm, N, K, ldx,
-                                 ldw, ldy, ld_wout, dtype, act, false, true, s);
+                                 ldw, ldy, ld_wout, dtype, act, false, true, s, nullptr, copy);
         if (rc != TPAMD_OK) return rc;
     }
     return TPAMD_OK;
+}
+
+extern "C" int tpamd_linear_w8(const void *x_dev, const void *wq_dev, const void *scale_dev, const void *outlier_idx_dev,
+                               const void *w_out_dev, int64_t n_out, const void *bias_dev, void *y_dev, int64_t M, int64_t N,
+                               int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout, int64_t ldy, int dtype, int act,
+                               void *stream) {
+    return w8_entry("tpamd_linear_w8", x_dev, wq_dev, scale_dev, outlier_idx_dev, w_out_dev, n_out, bias_dev, nullptr, 0, y_dev, nullptr, M, N, K, ldx, ldw,
+                    ld_wout, ldy, dtype, act, stream);
+}
+
+// As tpamd_linear_add and tpamd_linear_add_copy: the sum of two ranks' int8 Linears without a launch for the sum and one for its copy (5.0 and 4.6 us at
+// 16 rows of 8192, 9.7 and 7.8 at 1024).
+extern "C" int tpamd_linear_w8_add(const void *x_dev, const void *wq_dev, const void *scale_dev, const void *outlier_idx_dev, const void *w_out_dev,
+                                   int64_t n_out, const void *bias_dev, const void *addend_dev, void *y_dev, void *copy_dev, int64_t M, int64_t N, int64_t K,
+                                   int64_t ldx, int64_t ldw, int64_t ld_wout, int64_t ldadd, int64_t ldy, int dtype, int act, void *stream) {
+    const char *who = "tpamd_linear_w8_add";
+    TPAMD_REQUIRE(addend_dev != nullptr || M == 0 || N == 0, "%s: addend is NULL", who);
+    TPAMD_REQUIRE(copy_dev == nullptr || copy_dev != y_dev, "%s: the copy is y", who);
+    return w8_entry(who, x_dev, wq_dev, scale_dev, outlier_idx_dev, w_out_dev, n_out, bias_dev, addend_dev, ldadd, y_dev, copy_dev, M, N, K, ldx, ldw,
+                    ld_wout, ldy, dtype, act, stream);
 }
 
 extern "C" int tpamd_linear_w8_ranks(int n, const tpamd_w8_rank *ranks, int64_t n_out, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,

@@ -1520,7 +1520,10 @@ __global__ __launch_bounds__(256) void gemm_w8_direct_kernel(GemmParams p, W8Ext
     } else {
         const bool wide = wide_stores(p);
         char *slab = smem + wave * (16 * EP_PITCH);  // the stages (and the outlier tiles) are read out
-        if (p.act == TPAMD_ACT_GELU) staged_epilogue<DT, MODE_LINEAR, true, TMX, 4, 1, 4, 0>(p, acc, slab, m0, n_wave, lane, wide);
+        if (p.act == TPAMD_ACT_GELU) {
+            if (p.addend != nullptr) staged_epilogue<DT, MODE_LINEAR, true, TMX, 4, 1, 4, 0, true>(p, acc, slab, m0, n_wave, lane, wide);
+            else staged_epilogue<DT, MODE_LINEAR, true, TMX, 4, 1, 4, 0>(p, acc, slab, m0, n_wave, lane, wide);
+        } else if (p.addend != nullptr) staged_epilogue<DT, MODE_LINEAR, false, TMX, 4, 1, 4, 0, true>(p, acc, slab, m0, n_wave, lane, wide);
         else staged_epilogue<DT, MODE_LINEAR, false, TMX, 4, 1, 4, 0>(p, acc, slab, m0, n_wave, lane, wide);
     }
 }
@@ -2223,14 +2226,17 @@ void w8_tiling(int64_t M, int64_t N, int KT, int cus, int *rows, int *splits) {
 }
 
 // int8 weights above the weight-streaming kernels' row count. x, wq 16-byte aligned, K and ldw multiples of 16, ldx of 8
-// (checked by the caller); N and ldy multiples of 4 and y 8-byte aligned for the packed stores. gemm_w8_kernel is left with K
+// (checked by the caller); N, ldy and ldadd multiples of 4 and y, the addend and the copy (bytes from y to it, 0: none) 8-byte aligned for the packed stores. gemm_w8_kernel is left with K
 // that is no multiple of 64, and with streams that have no scratch memory for the outlier columns. TPAMD_ERR_UNSUPPORTED, with nothing
 // launched: the stream has no scratch memory and the slabs are faster than what needs none.
 int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out,
-                     const void *bias, void *y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout,
-                     int64_t ldy, int dtype, int act, hipStream_t s) {
+                     const void *bias, const void *addend, int64_t ldadd, int64_t copy, void *y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                     int64_t ld_wout, int64_t ldy, int dtype, int act, hipStream_t s) {
     GemmParams p{};
     p.ranks = 1;
+    p.addend = static_cast<const char *>(addend);
+    p.ldadd = ldadd;
+    p.copy = copy;
     p.x = static_cast<const char *>(x);
     p.w = static_cast<const char *>(wq);
     p.bias = static_cast<const char *>(bias);

@@ -45,19 +45,24 @@ def _guard(out: torch.Tensor, *inputs: torch.Tensor) -> torch.Tensor:
 
 
 def linear_in_context(module: nn.Module, x: torch.Tensor, w: torch.Tensor, bias) -> torch.Tensor:
-    """`tpamd_linear` for a shard's Linear. Inside a wrapped module whose output goes to a "sum" rule
-    (collectives.SumContext) the Linear that was seen to produce that output adds the partial sums already waiting in
+    """`tpamd_linear` for a shard's Linear; see `product_in_context`."""
+    xd, wd, b = x.detach(), w.detach(), None if bias is None else bias.detach()
+    return product_in_context(module, x, w.shape[0], (x, w, bias), lambda: together.linear(xd, wd, b), lambda **more: _native.linear(xd, wd, b, **more))
+
+
+def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs: tuple, with_peers, alone) -> torch.Tensor:
+    """A shard's Linear with `columns` outputs, made by with_peers() or, with an addend, alone(addend=, copy=). Inside a wrapped module whose output goes to a
+    "sum" rule (collectives.SumContext) the Linear that was seen to produce that output adds the partial sums already waiting in
     the reduction, in its epilogue (`tpamd_linear_add`): the product rounded to the dtype, then one rounded add, which
     is the same arithmetic as the reduction kernel's step."""
     from .collectives import current_sum_context
 
     ctx = current_sum_context()
-    b = None if bias is None else bias.detach()
     if ctx is None:
-        return _guard(together.linear(x.detach(), w.detach(), b), x, w, bias)
+        return _guard(with_peers(), *inputs)
     key = id(module)
     ctx.calls[key] = ctx.calls.get(key, 0) + 1
-    addend = copy = None
+    more = {}
     if module.__dict__.get("_tp_feeds_sum") is ctx.owner and ctx.owner is not None:
         if ctx.fused_out is not None:
             raise RuntimeError("tensor_parallel_amd: the Linear that feeds a \"sum\" rule ran twice in one call of its module "
@@ -65,20 +70,19 @@ def linear_in_context(module: nn.Module, x: torch.Tensor, w: torch.Tensor, bias)
         waiting = ctx.op.addend_for(ctx.rank)
         if waiting is not None:
             t, mask = waiting
-            if t.dtype == x.dtype and t.device == x.device and t.shape == (*x.shape[:-1], w.shape[0]):
-                addend, ctx.fused_mask = t.detach(), mask
+            if t.dtype == x.dtype and t.device == x.device and t.shape == (*x.shape[:-1], columns):
+                more["addend"], ctx.fused_mask = t.detach(), mask
                 if ctx.op.world_size == 2:  # the sum is complete then: a second tensor for the other rank comes out of the same launch
-                    copy = torch.empty_like(addend, memory_format=torch.contiguous_format)
+                    more["copy"] = torch.empty_like(more["addend"], memory_format=torch.contiguous_format)
+        out = alone(**more)
     # Ranks do not meet in the Linear that feeds the sum (the one that comes last adds the others' partials), nor before a first call has shown which one that is.
-    if "_tp_sum_known" in ctx.owner.__dict__ and module.__dict__.get("_tp_feeds_sum") is not ctx.owner:
-        out = together.linear(x.detach(), w.detach(), b)
     else:
-        out = _native.linear(x.detach(), w.detach(), b, addend=addend, **({} if copy is None else {"copy": copy}))
-    out = _guard(out, x, w, bias)
-    if addend is not None:
+        out = with_peers() if "_tp_sum_known" in ctx.owner.__dict__ else alone()
+    out = _guard(out, *inputs)
+    if more:
         ctx.fused_out = out
-        if copy is not None and not out.is_inference():  # (whose changes are not counted)
-            ctx.fused_copy = copy, out._version
+        if "copy" in more and not out.is_inference():  # (whose changes are not counted)
+            ctx.fused_copy = more["copy"], out._version
     ctx.last_linear, ctx.last_out = module, out
     return out
 

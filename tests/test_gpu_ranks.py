@@ -205,3 +205,21 @@ def test_a_sum_that_somebody_writes_to_is_copied_as_it_is(rank):
         handle.remove()
     assert len(ranks) == 2 and torch.equal(ranks[0], ranks[1])
     torch.testing.assert_close(ranks[0], want + 1.0, rtol=2.0 ** -7, atol=0)  # added before or after the sum: two roundings of 2^-9 around 1
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 2, 4, 17, 64, 65, 130, 300, 1024])
+@pytest.mark.parametrize("cols,K,n_out,gelu", [(2048, 4096, 20, False), (8192, 16384, 41, False), (1028, 1088, 0, True), (4100, 1040, 3, False)])
+def test_int8_linear_adds_a_partial_sum_and_copies_it(rows, cols, K, n_out, gelu, dtype):
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x, addend = draws(1, rows, K, dtype=dtype)[0], draws(1, rows, cols, dtype=dtype, seed=2)[0]
+    q = torch.randint(-127, 128, (cols, K), device=DEV, generator=g, dtype=torch.int8)
+    scale = torch.rand(cols, device=DEV, generator=g) * 1e-3
+    idx = torch.arange(0, 2 * n_out, 2, device=DEV, dtype=torch.int32) if n_out else None
+    w_out = draws(1, cols, n_out, dtype=dtype, seed=3)[0] if n_out else None
+    act = _native.ACT_GELU if gelu else _native.ACT_NONE
+    plain = _native.linear_w8(x, q, scale, idx, w_out, act=act)
+    copy = torch.full_like(addend, float("nan"))
+    y = _native.linear_w8(x, q, scale, idx, w_out, act=act, addend=addend, copy=copy)
+    assert torch.equal(y, plain + addend) and torch.equal(copy, y)
+    assert torch.equal(_native.linear_w8(x, q, scale, idx, w_out, act=act, addend=addend), y)
