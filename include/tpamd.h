@@ -164,6 +164,10 @@ int tpamd_scale(const void *in_dev, void *out_dev, uint64_t n_elems, int dtype, 
  * ---------------------------------------------------------------------------------------------- */
 int tpamd_reduce_partials(const void *const *parts_dev, int world_size, void *out_dev, uint64_t n_elems,
                           int dtype, int accum, void *stream);
+/* The same, stored to copy_dev as well (NULL: not): the sum for two ranks, each of which goes on with a tensor of its own. copy overlaps neither out nor a
+ * partial other than element for element. */
+int tpamd_reduce_partials_copy(const void *const *parts_dev, int world_size, void *out_dev, void *copy_dev, uint64_t n_elems, int dtype,
+                               int accum, void *stream);
 
 /* ------------------------------------------------------------------------------------------------
  * Rank-shard Linears. y[M,N] = act(x[M,K] . w[N,K]^T + bias[N]); fp32 accumulation, one rounding to
@@ -337,6 +341,13 @@ int tpamd_linear_gather_ranks(int n, const void *const *x_dev, const void *const
                               void *stream);
 int tpamd_swiglu_up_ranks(int n, const void *const *x_dev, const void *const *wg_dev, const void *const *wu_dev, void *const *h_dev,
                           int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldh, int dtype, void *stream);
+/* Row-parallel Linears of two ranks and their sum in one call: y[0] = y[1] = round(x[0] . w[0]^T + bias[0]) + round(x[1] . w[1]^T + bias[1]), rounded, the
+ * arithmetic of tpamd_linear followed by tpamd_linear_add_copy. TPAMD_ERR_UNSUPPORTED with nothing launched where those two calls are the better
+ * way (many rows, short rows, fp32) or a stream has no scratch memory. */
+int tpamd_linear_sum_ranks(const void *const *x_dev, const void *const *w_dev, const void *const *bias_dev /* NULL: none */, void *const *y_dev,
+                           int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, void *stream);
+/* 1 where tpamd_linear_sum_ranks takes aligned operands of these sizes, else 0 (host arithmetic on the sizes and the tuning knobs). */
+int tpamd_linear_sum_pays(int64_t M, int64_t N, int64_t K, int dtype);
 int tpamd_rms_norm_ranks(int n, const void *const *x_dev, const void *const *w_dev, void *const *y_dev, int64_t rows, int64_t D,
                          int64_t ldx, int64_t ldy, float eps, int dtype, void *stream);
 int tpamd_add_rms_norm_ranks(int n, const void *const *x_dev, const void *const *r_dev, const void *const *w_dev, void *const *sum_dev,
@@ -364,6 +375,9 @@ typedef struct {
 } tpamd_w8_rank;
 int tpamd_linear_w8_ranks(int n, const tpamd_w8_rank *ranks, int64_t n_out, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                           int64_t ld_wout, int64_t ldy, int dtype, int act, void *stream);
+/* As tpamd_linear_sum_ranks, for int8 weights (two ranks, 2 to 64 rows). */
+int tpamd_linear_w8_sum_ranks(const tpamd_w8_rank *ranks, int64_t n_out, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout,
+                              int64_t ldy, int dtype, void *stream);
 
 /* Causal mask of `rows` queries on `cols` keys, a byte each (1: seen): mask[i][j] = (kv_offset + j <= *q_offset_dev + i), the
  * queries' first position (int64) read from the device, mask [rows, cols] contiguous. */

@@ -7,6 +7,7 @@ entry point raises `NativeLibraryError`: there is no other implementation to fal
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from pathlib import Path
 from typing import Optional, Sequence
@@ -55,6 +56,10 @@ EXPORTS = (
     "tpamd_linear_gather_ranks",
     "tpamd_layer_norm_ranks",
     "tpamd_linear_w8_add",
+    "tpamd_linear_sum_ranks",
+    "tpamd_linear_sum_pays",
+    "tpamd_linear_w8_sum_ranks",
+    "tpamd_reduce_partials_copy",
 )
 
 ABI_VERSION = 6
@@ -170,6 +175,14 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_swiglu_up_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, i64, i64, ci, vp]
     lib.tpamd_rms_norm_ranks.restype = ci
     lib.tpamd_rms_norm_ranks.argtypes = [ci, pp, pp, pp, i64, i64, i64, i64, c.c_float, ci, vp]
+    lib.tpamd_linear_sum_ranks.restype = ci
+    lib.tpamd_linear_sum_ranks.argtypes = [pp, pp, pp, pp, i64, i64, i64, i64, i64, i64, ci, vp]
+    lib.tpamd_linear_sum_pays.restype = ci
+    lib.tpamd_linear_sum_pays.argtypes = [i64, i64, i64, ci]
+    lib.tpamd_linear_w8_sum_ranks.restype = ci
+    lib.tpamd_linear_w8_sum_ranks.argtypes = [c.POINTER(W8Rank), i64, i64, i64, i64, i64, i64, i64, i64, ci, vp]
+    lib.tpamd_reduce_partials_copy.restype = ci
+    lib.tpamd_reduce_partials_copy.argtypes = [pp, ci, vp, vp, u64, ci, ci, vp]
     lib.tpamd_linear_w8_add.restype = ci
     lib.tpamd_linear_w8_add.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, i64, ci, ci, vp]
     lib.tpamd_layer_norm_ranks.restype = ci
@@ -419,7 +432,9 @@ def scale(inp: torch.Tensor, world_size: int, multiply: bool = False) -> torch.T
     return out
 
 
-def reduce_partials(parts: Sequence[torch.Tensor], accum: int = ACCUM_STEPWISE, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+def reduce_partials(parts: Sequence[torch.Tensor], accum: int = ACCUM_STEPWISE, out: Optional[torch.Tensor] = None,
+                    copy: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The sum of the partials in their order; `copy` (contiguous, as the result) receives it too."""
     if len(parts) == 0:
         raise ValueError("reduce_partials: no partials")
     first = parts[0]
@@ -431,11 +446,13 @@ def reduce_partials(parts: Sequence[torch.Tensor], accum: int = ACCUM_STEPWISE, 
         keep.append(p.contiguous())
     if out is None:
         out = torch.empty_like(keep[0])
+    if copy is not None and (copy.numel() != first.numel() or copy.dtype != first.dtype or copy.device != first.device or not copy.is_contiguous()):
+        raise ValueError("reduce_partials: copy must be a contiguous tensor of the result's size, dtype and device")
     ptrs = (ctypes.c_void_p * len(keep))(*[p.data_ptr() for p in keep])
     with _on_device(first.device):
         _check(
-            lib().tpamd_reduce_partials(ptrs, len(keep), out.data_ptr(), first.numel(), dtype_code(first.dtype), accum,
-                                        ctypes.c_void_p(current_stream_ptr(first.device))),
+            lib().tpamd_reduce_partials_copy(ptrs, len(keep), out.data_ptr(), None if copy is None else copy.data_ptr(), first.numel(),
+                                             dtype_code(first.dtype), accum, ctypes.c_void_p(current_stream_ptr(first.device))),
             "tpamd_reduce_partials",
         )
     return out
@@ -457,6 +474,7 @@ def _ld(t: torch.Tensor) -> int:
 def reload_tuning() -> None:
     """Make the library read its TPAMD_* environment variables again (it reads them once, at load time)."""
     lib().tpamd_tuning_reload()
+    linear_sum_pays.cache_clear()
 
 
 def scratch_of_stream(device: torch.device, stream_ptr: Optional[int] = None) -> tuple:
@@ -514,6 +532,29 @@ def linear_ranks(calls: Sequence[tuple]) -> list:
                                      _ld(xs[0]), _ld(ws[0]), N, dtype_code(x.dtype), ACT_NONE, ctypes.c_void_p(current_stream_ptr(x.device))),
             "tpamd_linear_ranks",
         )
+    return [y.view(*x.shape[:-1], N) for y in ys]
+
+
+@functools.lru_cache(maxsize=4096)
+def linear_sum_pays(M: int, N: int, K: int, dtype: torch.dtype) -> bool:
+    """Whether `linear_sum_ranks` has a launch for these sizes that is faster than two (a rule on sizes and tuning knobs)."""
+    return lib().tpamd_linear_sum_pays(M, N, K, dtype_code(dtype)) == 1
+
+
+def linear_sum_ranks(calls: Sequence[tuple]) -> Optional[list]:
+    """The sum of two ranks' `linear(x, w, bias)`, for each a tensor of its own, in one launch; None where there is none for the shape."""
+    x, w, bias = calls[0]
+    _check_linear(x, w, bias)
+    xs, ws = [_as_2d(c[0]) for c in calls], [_as_2d(c[1]) for c in calls]
+    (M, K), N = xs[0].shape, w.shape[0]
+    ys = [torch.empty((M, N), dtype=x.dtype, device=x.device) for _ in calls]
+    bs = None if bias is None else [c[2].contiguous() for c in calls]
+    with _on_device(x.device):
+        rc = lib().tpamd_linear_sum_ranks(_pointers(xs), _pointers(ws), None if bs is None else _pointers(bs), _pointers(ys), M, N, K, _ld(xs[0]), _ld(ws[0]), N,
+                                          dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device)))
+    if rc == -2:
+        return None
+    _check(rc, "tpamd_linear_sum_ranks")
     return [y.view(*x.shape[:-1], N) for y in ys]
 
 
@@ -996,8 +1037,7 @@ def _w8_operands(x, wq, scale_, outlier_idx, w_out, bias) -> tuple:
     return x2, wq, scale_.contiguous(), outlier_idx if n_out else None, w_out if n_out else None, None if bias is None else bias.contiguous()
 
 
-def linear_w8_ranks(calls: Sequence[tuple]) -> list:
-    """`linear_w8(x, wq, scale, outlier_idx, w_out, bias)` for the operands of several ranks."""
+def _w8_ranks(calls: Sequence[tuple]) -> tuple:
     ranks, keep = (W8Rank * len(calls))(), []
     for rank, call in zip(ranks, calls):
         ops = _w8_operands(*call)
@@ -1007,11 +1047,26 @@ def linear_w8_ranks(calls: Sequence[tuple]) -> list:
         keep.append((ops, y))
         rank.x, rank.wq, rank.scale, rank.outlier_idx, rank.w_out, rank.bias = (None if t is None else t.data_ptr() for t in ops)
         rank.y = y.data_ptr()
-    x, n_out = calls[0][0], 0 if ops[3] is None else int(ops[3].numel())
+    n_out = 0 if ops[3] is None else int(ops[3].numel())
+    return ranks, keep, (n_out, M, N, K, _ld(x2), K, max(n_out, 1), N, dtype_code(x2.dtype))
+
+
+def linear_w8_ranks(calls: Sequence[tuple]) -> list:
+    """`linear_w8(x, wq, scale, outlier_idx, w_out, bias)` for the operands of several ranks."""
+    x = calls[0][0]
     with _on_device(x.device):
-        _check(
-            lib().tpamd_linear_w8_ranks(len(calls), ranks, n_out, M, N, K, _ld(x2), K, max(n_out, 1), N, dtype_code(x.dtype), ACT_NONE,
-                                        ctypes.c_void_p(current_stream_ptr(x.device))),
-            "tpamd_linear_w8_ranks",
-        )
-    return [y.view(*x.shape[:-1], N) for _, y in keep]
+        ranks, keep, dims = _w8_ranks(calls)
+        _check(lib().tpamd_linear_w8_ranks(len(calls), ranks, *dims, ACT_NONE, ctypes.c_void_p(current_stream_ptr(x.device))), "tpamd_linear_w8_ranks")
+    return [y.view(*x.shape[:-1], y.shape[1]) for _, y in keep]
+
+
+def linear_w8_sum_ranks(calls: Sequence[tuple]) -> Optional[list]:
+    """The sum of two ranks' `linear_w8`, for each a tensor of its own; None where no launch of both adds it up."""
+    x = calls[0][0]
+    with _on_device(x.device):
+        ranks, keep, dims = _w8_ranks(calls)
+        rc = lib().tpamd_linear_w8_sum_ranks(ranks, *dims, ctypes.c_void_p(current_stream_ptr(x.device)))
+    if rc == -2:
+        return None
+    _check(rc, "tpamd_linear_w8_sum_ranks")
+    return [y.view(*x.shape[:-1], y.shape[1]) for _, y in keep]

@@ -71,11 +71,11 @@ _contexts: contextvars.ContextVar = contextvars.ContextVar("tpamd_sum_contexts",
 class SumContext:
     """One call of a wrapped module whose output 0 goes to `op`, on one rank."""
 
-    __slots__ = ("op", "rank", "owner", "last_linear", "last_out", "calls", "fused_out", "fused_mask", "fused_copy")
+    __slots__ = ("op", "rank", "owner", "last_linear", "last_out", "calls", "fused_out", "fused_mask", "fused_copy", "fused_whole", "last_version")
 
     def __init__(self, op: "DeviceAllReduce", rank: int, owner: Any):
         self.op, self.rank, self.owner = op, rank, owner
-        self.last_linear = self.last_out = self.fused_out = self.fused_copy = None
+        self.last_linear = self.last_out = self.last_version = self.fused_out = self.fused_copy = self.fused_whole = None
         self.calls: dict = {}
         self.fused_mask = 0
 
@@ -89,7 +89,7 @@ class SumContext:
                     "tensor_parallel_amd: a row-parallel Linear added the other ranks' partial sums in its epilogue, but its "
                     "module then returned a different tensor; set TPAMD_FUSE_SUM=0 to keep the sum in its own kernel")
         elif self.last_linear is not None:
-            feeds = value is self.last_out and self.calls.get(id(self.last_linear)) == 1
+            feeds = value is self.last_out and self.calls.get(id(self.last_linear)) == 1 and (self.last_version is None or value._version == self.last_version)
             self.last_linear.__dict__["_tp_feeds_sum"] = self.owner if feeds else None
             self.owner.__dict__["_tp_sum_known"] = True
 
@@ -213,6 +213,7 @@ class DeviceAllReduce(CollectiveOperation):
         self.accum = accum
         self._masks: List[int] = [0] * world_size
         self._copy: Optional[torch.Tensor] = None  # of a value that covers every rank
+        self._whole: List[bool] = [False] * world_size  # ranks whose value is a sum over all ranks made for that rank
 
     @property
     def fusable(self) -> bool:
@@ -241,6 +242,12 @@ class DeviceAllReduce(CollectiveOperation):
         ctx = current_sum_context()
         if ctx is not None and ctx.op is self and ctx.fused_out is not None and x is ctx.fused_out:
             mask |= ctx.fused_mask  # this value already holds what the rank's Linear was given by addend_for()
+            if ctx.fused_whole is not None:
+                if ctx.fused_whole != x._version:
+                    raise RuntimeError(
+                        "tensor_parallel_amd: the output of a row-parallel Linear was changed in place on its way to a \"sum\" rule; it held the sum over the "
+                        "ranks already. Set TPAMD_FUSE_SUM=0 to keep the sum in its own kernel")
+                self._whole[rank] = True
             if ctx.fused_copy is not None and ctx.fused_copy[1] == x._version:  # nobody has written to the value since
                 self._copy = ctx.fused_copy[0]
         self._masks[rank] = mask
@@ -249,17 +256,26 @@ class DeviceAllReduce(CollectiveOperation):
         finally:
             self._masks[rank] = 0
             self._copy = None
+            self._whole[rank] = False
 
     def _reduce(self, *parts: torch.Tensor):
+        if all(self._whole):
+            return [_guard(p.detach(), *parts) for p in parts]
         masks = list(self._masks)
         widest = max(range(self.world_size), key=lambda r: bin(masks[r]).count("1"))
         todo = [parts[widest]] + [parts[r] for r in range(self.world_size) if not masks[widest] >> r & 1]
         # the widest value is a running sum from rank 0 on (or covers both of two ranks); what it lacks are higher ranks
-        out = todo[0].detach() if len(todo) == 1 else _native.reduce_partials([p.detach() for p in todo], accum=self.accum)
+        copy = self._copy if len(todo) == 1 else None
+        if len(todo) == 1:
+            out = todo[0].detach()
+        elif self.world_size == 2:
+            copy = torch.empty_like(todo[0], memory_format=torch.contiguous_format)
+            out = _native.reduce_partials([p.detach() for p in todo], accum=self.accum, copy=copy)
+        else:
+            out = _native.reduce_partials([p.detach() for p in todo], accum=self.accum)
         # each rank continues with a tensor of its own: later in-place ops on one rank must not leak
-        if len(todo) == 1 and self._copy is not None and self.world_size == 2:
-            return [_guard(o, *parts) for o in (out, self._copy)]
-        return [_guard(o, *parts) for o in [out] + [out.clone() for _ in range(self.world_size - 1)]]
+        rest = [copy] if copy is not None and self.world_size == 2 else [out.clone() for _ in range(self.world_size - 1)]
+        return [_guard(o, *parts) for o in [out] + rest]
 
 
 class DeviceAllGather(CollectiveOperation):

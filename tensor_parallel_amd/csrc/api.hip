@@ -33,6 +33,15 @@ int attention_decode_rope_dispatch(const void *q, const void *k, const void *v, 
                                    void *v_cache, void *o, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t pos0, const int64_t *pos_dev,
                                    const int64_t *strides, float scale, int dtype, hipStream_t s, const tpamd_decode_rank *second = nullptr);
 
+int skinny_sum_dispatch(const void *x, const void *w, const void *bias, const RankStep &to, void *y, int64_t copy, int64_t M, int64_t N, int64_t K, int64_t ldx,
+                        int64_t ldw, int64_t ldy, int dtype, int row_waves, hipStream_t s);
+bool sum128_pays(int64_t M, int64_t N, int64_t K, int cus);
+int gemm_sum_dispatch(const void *x, const void *w, const void *bias, const RankStep &to, void *y, int64_t copy, int64_t M, int64_t N, int64_t K, int64_t ldx,
+                      int64_t ldw, int64_t ldy, int dtype, hipStream_t s, bool *done);
+int skinny_w8_sum_dispatch(const void *x, const void *wq, const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out, const void *bias,
+                           const RankStep &to, void *y, int64_t copy, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout, int64_t ldy,
+                           int dtype, hipStream_t s, bool *done);
+
 namespace {
 
 // Largest M served by the weight-streaming kernels; above it the tiled MFMA kernels take over.
@@ -287,6 +296,109 @@ extern "C" int tpamd_linear_gather_ranks(int n, const void *const *x_dev, const 
         return skinny_dispatch(x_dev[0], w_dev[0], nullptr, b0, nullptr, 0, nullptr, nullptr, nullptr, 0, y_dev[0], M, N, K, ldx, ldw, ldy, 0, dtype, act, false,
                                false, s, &to, copy);
     return gemm_dispatch(x_dev[0], w_dev[0], nullptr, b0, nullptr, 0, y_dev[0], M, N, K, ldx, ldw, ldy, dtype, act, false, false, s, &to, copy);
+}
+
+// What takes the sum of two ranks' row-parallel Linears. Measured inside a HIP graph on rotated weights against tpamd_linear + tpamd_linear_add_copy (us, two
+// launches / row kernel with 8 wavefronts / with 16 / MFMA weight streaming / K ranges of 128 x 128 tiles):
+//   1 row    4096 x 2048   9.4 /  7.1  7.2            4096 x 5504 19.2 / 18.6 17.6     8192 x 4096 24.1 / 23.5 22.7     1024 x 1408 5.8 / 3.4  4.4
+//   2 rows   4096 x 2048  10.2 /  8.3  8.7            4096 x 5504 20.3 / 22.2 43.1     8192 x 4096 26.5 / 30.4 41.9     2048 x 2816 10.0 / 7.6 11.5
+//   4 rows   4096 x 2048  12.0 /           9.3        4096 x 5504 23.0 /      19.7     8192 x 4096 28.4 /      23.8     2048 x 2816 11.7 /      8.3
+//   16 rows  4096 x 2048  13.4 /          10.1        4096 x 5504 25.2 /      21.5     8192 x 4096 30.6 /      27.1     5120 x 6912 34.5 / 39.3, 31.1 in tiles
+//   40 rows  4096 x 2048  19.9 /               14.0   4096 x 5504 35.3 /      26.8     8192 x 4096 38.3 /      35.4     5120 x 6912 40.8 /      32.2
+// So the row kernel takes one row, and two where they are short or few; weight streaming the others up to the row count it has for one matrix of both ranks' K,
+// unless its tiles are a ragged number of rounds; K ranges of tiles the rest while they are predicted to be faster than two launches. Two launches keep
+// matrices that the kernels for one of them stream as fast: one of long rows at 1 row (4096 x 8192: 24.9, 26.2 in one; ragged 5120 x 5504: 24.1, 26.8), ragged ones
+// between K = 2048 and 3072 at 2 (4544 x 2752: 15.1, 15.8) and of 1.5 rounds or more from K = 3072 on up to 16 (7168 x 4096 at 8 rows: 25.1, 29.1). On 372 random
+// shapes (1024-8192 columns, K 1024-8192, 1-600 rows) one launch took 0.77 of the time of two in the geometric mean, and was slower on the 18 that these exceptions
+// and the margin of sum128_pays take out and on 5120 x 2048 at 3 rows (13.2, 13.7).
+enum SumPath { SUM_NONE, SUM_ROWS8, SUM_ROWS16, SUM_STREAM, SUM_TILES };
+static int sum_path(int64_t M, int64_t N, int64_t K, SumPath *path) {
+    *path = SUM_NONE;
+    if (K < 1024 || M < 1) return TPAMD_OK;  // no shorter row was measured
+    int dev = 0, cus = 256;
+    TPAMD_HIP(hipGetDevice(&dev));
+    if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
+    const int64_t tiles = (N + 15) / 16;
+    const bool ragged = tiles > cus && tiles % cus != 0;
+    if (M == 1 && K > (ragged ? 4096 : 11 * 512)) return TPAMD_OK;
+    if (ragged && ((M <= 2 && K > 2048 && K < 3072) || (M > 1 && M <= SKINNY_MAX_M && K >= 3072 && tiles * 2 >= 3ll * cus))) return TPAMD_OK;
+    if (K <= 11 * 512 && (M == 1 || (M == 2 && (K <= 2048 || N <= 2048)) || (M == 3 && K <= 2048 && N <= 1024))) {
+        *path = M == 1 && K > 2048 && N >= 4096 ? SUM_ROWS16 : SUM_ROWS8;
+        return TPAMD_OK;
+    }
+    int64_t rows = SKINNY_MAX_M;
+    if (M > SKINNY_MAX_M && M <= 64) {
+        if (int rc = skinny_row_limit(N, 2 * K, &rows); rc != TPAMD_OK) return rc;
+    }
+    if (M <= rows && !ragged) *path = SUM_STREAM;
+    else if (M <= 64 ? K % 64 == 0 && (M > 1 || !ragged) : sum128_pays(M, N, K, cus)) *path = SUM_TILES;
+    return TPAMD_OK;
+}
+
+extern "C" int tpamd_linear_sum_pays(int64_t M, int64_t N, int64_t K, int dtype) {
+    SumPath path = SUM_NONE;
+    return dtype != TPAMD_F32 && sum_path(M, N, K, &path) == TPAMD_OK && path != SUM_NONE ? 1 : 0;
+}
+
+// Row-parallel Linears of two ranks and their sum, delivered to both. TPAMD_ERR_UNSUPPORTED, with nothing launched, where two launches
+// (tpamd_linear, then tpamd_linear_add_copy) are the better way or the kernels do not take the operands.
+extern "C" int tpamd_linear_sum_ranks(const void *const *x_dev, const void *const *w_dev, const void *const *bias_dev, void *const *y_dev, int64_t M, int64_t N,
+                                      int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, void *stream) {
+    const char *who = "tpamd_linear_sum_ranks";
+    TPAMD_REQUIRE(x_dev && w_dev && y_dev, "%s: null pointer", who);
+    bool fast = dtype != TPAMD_F32 && M > 0 && N > 0 && (bias_dev == nullptr || (bias_dev[0] == nullptr) == (bias_dev[1] == nullptr));
+    for (int i = 0; i < 2; ++i) {
+        if (int rc = check_common(who, x_dev[i], w_dev[i], y_dev[i], M, N, K, ldx, ldw, ldy, dtype); rc != TPAMD_OK) return rc;
+        fast = fast && mfma_ok(x_dev[i], w_dev[i], nullptr, bias_dev ? bias_dev[i] : nullptr, y_dev[i], N, K, ldx, ldw, ldy);
+    }
+    if (M == 0 || N == 0) return TPAMD_OK;
+    SumPath path = SUM_NONE;
+    if (fast) {
+        if (int rc = sum_path(M, N, K, &path); rc != TPAMD_OK) return rc;
+    }
+    if (path != SUM_NONE) {
+        const void *b0 = bias_dev ? bias_dev[0] : nullptr, *b1 = bias_dev ? bias_dev[1] : nullptr;
+        RankStep to{};
+        to.x = bytes_from(x_dev[0], x_dev[1]);
+        to.w = bytes_from(w_dev[0], w_dev[1]);
+        to.bias = bytes_from(b0, b1);
+        const int64_t copy = bytes_from(y_dev[0], y_dev[1]);
+        hipStream_t s = static_cast<hipStream_t>(stream);
+        if (path != SUM_TILES)
+            return skinny_sum_dispatch(x_dev[0], w_dev[0], b0, to, y_dev[0], copy, M, N, K, ldx, ldw, ldy, dtype,
+                                       path == SUM_ROWS8 ? 8 : path == SUM_ROWS16 ? 16 : 0, s);
+        bool done = false;
+        const int rc = gemm_sum_dispatch(x_dev[0], w_dev[0], b0, to, y_dev[0], copy, M, N, K, ldx, ldw, ldy, dtype, s, &done);
+        if (rc != TPAMD_OK || done) return rc;
+    }
+    set_error("%s: no launch of both ranks for this shape", who);
+    return TPAMD_ERR_UNSUPPORTED;
+}
+
+// The same for int8 weights on 2 to 64 rows whose kernels split K over blocks.
+extern "C" int tpamd_linear_w8_sum_ranks(const tpamd_w8_rank *ranks, int64_t n_out, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout,
+                                         int64_t ldy, int dtype, void *stream) {
+    const char *who = "tpamd_linear_w8_sum_ranks";
+    TPAMD_REQUIRE(ranks != nullptr, "%s: null pointer", who);
+    bool ok = M > 0 && M <= SKINNY_W8_SLAB && N > 0 && n_out >= 0 && n_out <= K && K < (1ll << 31) && N < (1ll << 31) && (dtype == TPAMD_BF16 || dtype == TPAMD_F16) &&
+              K % 16 == 0 && ldw % 16 == 0 && ldx % 8 == 0 && ldx >= K && ldw >= K && ldy >= N && (n_out == 0 || ld_wout >= n_out) && tuning().w8_tile == TUNE_UNSET;
+    for (int j = 0; ok && j < 2; ++j) {
+        const tpamd_w8_rank &r = ranks[j];
+        ok = r.x && r.wq && r.scale && r.y && aligned(r.x, 16) && aligned(r.wq, 16) && (n_out == 0 || (r.outlier_idx && r.w_out)) &&
+             (r.bias == nullptr) == (ranks[0].bias == nullptr);
+    }
+    if (ok) {
+        const tpamd_w8_rank &a = ranks[0], &b = ranks[1];
+        const bool o = n_out > 0;
+        const RankStep to = {bytes_from(a.x, b.x), bytes_from(a.wq, b.wq), 0, bytes_from(a.bias, b.bias), 0,
+                             bytes_from(a.scale, b.scale), o ? bytes_from(a.outlier_idx, b.outlier_idx) : 0, o ? bytes_from(a.w_out, b.w_out) : 0};
+        bool done = false;
+        const int rc = skinny_w8_sum_dispatch(a.x, a.wq, a.scale, a.outlier_idx, a.w_out, n_out, a.bias, to, a.y, bytes_from(a.y, b.y), M, N, K, ldx, ldw, ld_wout,
+                                              ldy, dtype, static_cast<hipStream_t>(stream), &done);
+        if (rc != TPAMD_OK || done) return rc;
+    }
+    set_error("%s: no launch of both ranks for this shape", who);
+    return TPAMD_ERR_UNSUPPORTED;
 }
 
 extern "C" int tpamd_attention(const void *q_dev, const void *k_dev, const void *v_dev, void *out_dev, int64_t B, int64_t Hq,

@@ -703,6 +703,12 @@ __global__ __launch_bounds__(256) void gemm_direct128_kernel(GemmParams p) {
     tile_of_block(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n * p.ranks, tile_m, tile_n);
     const int part_n = tile_n;  // among the column tiles of both ranks
     take_rank(p, tile_n);
+    int k_range = SPLIT ? static_cast<int>(blockIdx.y) : 0;
+    if (SPLIT && p.sum && k_range >= p.splits) {
+        k_range -= p.splits;
+        p.x += p.to.x;
+        p.w += p.to.w;
+    }
     const int m0 = tile_m * BM;
     const int n0 = tile_n * (MODE == MODE_SWIGLU ? BN / 2 : BN);
 
@@ -741,7 +747,7 @@ __global__ __launch_bounds__(256) void gemm_direct128_kernel(GemmParams p) {
 
     // this block's K tiles: [kt0, kt0 + nk)
     const int KT = p.K / BK;
-    const int kt0 = SPLIT ? static_cast<int>(blockIdx.y) * p.kt_per_split : 0;
+    const int kt0 = k_range * p.kt_per_split;
     const int nk = SPLIT ? (KT - kt0 < p.kt_per_split ? KT - kt0 : p.kt_per_split) : KT;
     const int last = nk - 1;
     // loads of local tile j (clamped to the last one: such loads refill a stage nobody reads any more and keep
@@ -926,6 +932,19 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(GemmParams p, int sp
         if (m >= p.M || n >= p.N) return;
         float g[4] = {0.f, 0.f, 0.f, 0.f}, u[4] = {0.f, 0.f, 0.f, 0.f};
         const float *src = tile0 + r * 128 + c4 * 4;
+        uint2 other = make_uint2(0, 0);
+        if (MODE == MODE_LINEAR && p.sum) {  // the second rank's product first
+            for (int sp = splits; sp < 2 * splits; ++sp) {
+                const f32x4 gv = *reinterpret_cast<const f32x4 *>(src + sp * split_stride);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) g[i] += gv[i];
+            }
+            GemmParams q = p;
+            if (q.bias) q.bias += p.to.bias;
+            other = finish4<DT, MODE_LINEAR>(q, g, u, n);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) g[i] = 0.f;
+        }
         for (int sp = 0; sp < splits; ++sp) {
             const f32x4 gv = *reinterpret_cast<const f32x4 *>(src + sp * split_stride);
 #pragma unroll
@@ -937,7 +956,8 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(GemmParams p, int sp
             }
         }
         const char *add_row = MODE == MODE_LINEAR && p.addend != nullptr ? p.addend + static_cast<int64_t>(m) * p.ldadd * 2 : nullptr;
-        const uint2 o = finish4<DT, MODE>(p, g, u, n, add_row);
+        uint2 o = finish4<DT, MODE>(p, g, u, n, add_row);
+        if (MODE == MODE_LINEAR && p.sum) o = make_uint2(add_packed2<DT>(o.x, other.x), add_packed2<DT>(o.y, other.y));
         char *dst = p.y + (static_cast<int64_t>(m) * p.ldy + n) * 2;
         *reinterpret_cast<uint2 *>(dst) = o;
         if (p.copy) *reinterpret_cast<uint2 *>(dst + p.copy) = o;
@@ -2076,6 +2096,55 @@ int launch_direct128(GemmParams p, int cus, hipStream_t s) {
     return TPAMD_OK;
 }
 
+// Two ranks' Linears and their sum in one launch and a finishing pass: 128 x 128 tiles, every rank's K in `splits` ranges. Predicted time (microseconds) of the
+// best split, by the terms of estimate128.
+inline double estimate_sum128(int64_t tiles, int64_t tiles_n, int KT, int cus, double valid_rows, int *splits, bool *deep) {
+    double best = 1e30;
+    const double stream = 2.0 * tiles_n * KT * 16384.0 / 5.0e6;
+    for (int sp = 1; sp <= 4; ++sp) {
+        const int kt = (KT + sp - 1) / sp;
+        const int64_t units = tiles * 2 * sp;
+        if ((sp > 1 && kt < 4) || units > 4ll * cus) break;
+        const double finish = 4.6 + units * 0.065536 * valid_rows * 0.39;
+        const double loop_deep = kt * 0.55, rounds = units <= cus ? 1.0 : static_cast<double>((units + 2 * cus - 1) / (2 * cus));
+        const double t_deep = (loop_deep > stream ? loop_deep : stream) + finish;
+        if (units <= cus && t_deep < best) { best = t_deep; *splits = sp; *deep = true; }
+        const double loop = rounds * kt * (units <= cus ? 0.82 : units <= 2ll * cus ? 0.98 : 0.92);
+        const double t = (loop > stream ? loop : stream) + finish;
+        if (t < best) { best = t; *splits = sp; *deep = false; }
+    }
+    return best;
+}
+
+template <int DT>
+int launch_sum128(GemmParams p, bool deep, hipStream_t s, bool *done) {
+    int dev = 0, cus = 256;
+    TPAMD_HIP(hipGetDevice(&dev));
+    if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
+    const int KT = p.K / 64;
+    p.tiles_m = (p.M + 127) / 128;
+    p.tiles_n = (p.N + 127) / 128;
+    p.kt_per_split = (KT + p.splits - 1) / p.splits;
+    p.splits = (KT + p.kt_per_split - 1) / p.kt_per_split;  // no empty split
+    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
+    const size_t ws_bytes = static_cast<size_t>(2 * p.splits) * tiles * 128 * 128 * sizeof(float);
+    std::lock_guard<std::mutex> hold(splitk_mutex(dev));  // the scratch buffer is ours until both launches are enqueued
+    void *ws = nullptr;
+    if (int rc = splitk_scratch(dev, s, ws_bytes, scratch_reserve(cus), &ws); rc != TPAMD_OK) return rc;
+    if (ws == nullptr) return TPAMD_OK;
+    p.ws = static_cast<float *>(ws);
+    const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(2 * p.splits));
+    const int xq = tuning().gemm_part_x == 0 || tiles > 64 ? 4 : p.M <= 32 ? 1 : p.M <= 64 ? 2 : 4;  // as in launch_direct128
+    int rc = xq == 1 ? (deep ? launch_split128<DT, MODE_LINEAR, 4, 1>(p, grid, dev, s) : launch_split128<DT, MODE_LINEAR, 2, 1>(p, grid, dev, s))
+             : xq == 2 ? (deep ? launch_split128<DT, MODE_LINEAR, 4, 2>(p, grid, dev, s) : launch_split128<DT, MODE_LINEAR, 2, 2>(p, grid, dev, s))
+                       : (deep ? launch_split128<DT, MODE_LINEAR, 4, 4>(p, grid, dev, s) : launch_split128<DT, MODE_LINEAR, 2, 4>(p, grid, dev, s));
+    if (rc != TPAMD_OK) return rc;
+    hipLaunchKernelGGL((splitk_finish_kernel<DT, MODE_LINEAR>), dim3(16, static_cast<unsigned>(tiles)), dim3(256), 0, s, p, p.splits);
+    TPAMD_HIP(hipGetLastError());
+    *done = true;
+    return TPAMD_OK;
+}
+
 // Prefill-sized dispatch; called by linear.hip once M is above the skinny range.
 template <int DT>
 int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
@@ -2192,6 +2261,48 @@ int gemm_dispatch(const void *x, const void *w, const void *w2, const void *bias
         return generic_dispatch(p, dtype, swiglu, s);
     }
     return dtype == TPAMD_BF16 ? gemm_large<TPAMD_BF16>(p, swiglu, s) : gemm_large<TPAMD_F16>(p, swiglu, s);
+}
+
+// Whether launch_sum128 is predicted to take less time than two launches, the second of which adds the first one's result (M above the weight-streaming kernels'
+// range). The models are those of estimate128 and estimate_mid; 512 rows of 4096 x 5504: 33.1 + 5.4 us twice, 59.0 + 5.6 in one; 645 rows, whose
+// unsplit tiles of one rank fill the device, stay in two launches.
+bool sum128_pays(int64_t M, int64_t N, int64_t K, int cus) {
+    if (K % 64 != 0 || tuning().gemm_tile != TUNE_UNSET || tuning().gemm_splitk != TUNE_UNSET) return false;
+    const int KT = static_cast<int>(K / 64);
+    const int64_t tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128, tiles = tiles_m * tiles_n;
+    const double valid = static_cast<double>(M) / (tiles_m * 128.0);
+    bool deep = false;
+    int tmx = 0, tnx = 0, splits = 0;
+    const double once = estimate_sum128(tiles, tiles_n, KT, cus, valid, &splits, &deep);
+    const double t128 = estimate128(tiles, tiles_m, tiles_n, KT, cus, valid, false, &splits, &deep);
+    const double mid = estimate_mid(M, N, KT, cus, false, &tmx, &tnx);
+    return once < 1.9 * (t128 < mid ? t128 : mid);  // where the models are equal one launch was 2-3 % slower (4544 x 7168 at 513 rows, 5120 x 8192 at 468)
+}
+
+// y = the sum of two ranks' 16-bit Linears of one shape, the second one's operands `to` away, stored a second time `copy` bytes on. *done = false, with nothing
+// launched: leading dimensions of 2^22 elements or more, too many tiles, or a stream without scratch memory.
+int gemm_sum_dispatch(const void *x, const void *w, const void *bias, const RankStep &to, void *y, int64_t copy, int64_t M, int64_t N, int64_t K, int64_t ldx,
+                      int64_t ldw, int64_t ldy, int dtype, hipStream_t s, bool *done) {
+    *done = false;
+    if (K % 64 != 0 || ldx >= (1ll << 22) || ldw >= (1ll << 22)) return TPAMD_OK;
+    int dev = 0, cus = 256;
+    TPAMD_HIP(hipGetDevice(&dev));
+    if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
+    GemmParams p{};
+    p.ranks = 1;
+    p.sum = 1;
+    p.to = to;
+    p.copy = copy;
+    p.x = static_cast<const char *>(x);
+    p.w = static_cast<const char *>(w);
+    p.bias = static_cast<const char *>(bias);
+    p.y = static_cast<char *>(y);
+    p.M = static_cast<int>(M); p.N = static_cast<int>(N); p.K = static_cast<int>(K);
+    p.ldx = ldx; p.ldw = ldw; p.ldy = ldy;
+    const int64_t tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
+    bool deep = false;
+    if (estimate_sum128(tiles_m * tiles_n, tiles_n, static_cast<int>(K / 64), cus, static_cast<double>(M) / (tiles_m * 128.0), &p.splits, &deep) >= 1e30) return TPAMD_OK;
+    return dtype == TPAMD_BF16 ? launch_sum128<TPAMD_BF16>(p, deep, s, done) : launch_sum128<TPAMD_F16>(p, deep, s, done);
 }
 
 // gemm_w8_direct_kernel steps K in tiles of 64 and addresses a tile with 32-bit byte offsets from its origin.

@@ -28,6 +28,7 @@ struct GemmParams {
     int ranks;          // 1, or 2: a second rank's columns follow the first one's, `to` leads to its operands
     RankStep to;
     int64_t copy;       // every output is stored a second time that many bytes on (0: once)
+    int sum;            // split-K of the 128 x 128 kernel: `splits` K ranges of each of two ranks, y = the sum of both rounded products
 };
 
 __device__ __forceinline__ bool wide_stores(const GemmParams &p) {  // 16 bytes each

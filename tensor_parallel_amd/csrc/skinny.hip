@@ -46,6 +46,7 @@ struct SkinnyParams {
     int ranks;     // 1, or 2: blockIdx.z is the rank, `to` the way to the second one's operands
     RankStep to;
     int64_t copy;  // every output is stored a second time that many bytes on (0: once)
+    int sum;       // y = round(rank 0's product) + round(rank 1's): one result for both ranks
 };
 
 // This block's rank.
@@ -89,6 +90,19 @@ __device__ __forceinline__ void skinny_store_output(const SkinnyParams &p, float
     }
 }
 
+// One element of the sum of two ranks' Linears from the fp32 sums of each: products rounded to the tensor dtype, then the rounded sum, which is what
+// a Linear whose epilogue adds the other's result gives.
+template <int DT>
+__device__ __forceinline__ void skinny_store_sum(const SkinnyParams &p, float s0, float s1, int m, int n) {
+    if (p.bias) {
+        s0 += half_to_f32<DT>(reinterpret_cast<const uint16_t *>(p.bias)[n]);
+        s1 += half_to_f32<DT>(reinterpret_cast<const uint16_t *>(p.bias + p.to.bias)[n]);
+    }
+    const uint16_t out = f32_to_half<DT>(half_to_f32<DT>(f32_to_half<DT>(s0)) + half_to_f32<DT>(f32_to_half<DT>(s1)));
+    reinterpret_cast<uint16_t *>(p.y)[static_cast<int64_t>(m) * p.ldy + n] = out;
+    if (p.copy) reinterpret_cast<uint16_t *>(p.y + p.copy)[static_cast<int64_t>(m) * p.ldy + n] = out;
+}
+
 // W8 = weight is int8. MT = number of 16-row tiles of x (M <= 16*MT). MODE = SK_LINEAR / SK_SWIGLU.
 //
 // Fetching. The MFMA row operand wants lane l to hold 16 bytes of row l%16 at K slot l/16; loading it that way
@@ -107,10 +121,14 @@ __device__ __forceinline__ void skinny_store_output(const SkinnyParams &p, float
 // same 8 output columns, so a block owns 8 columns instead of 16: one accumulator tile instead of two (95 instead of
 // 160 registers, so several blocks share a CU) and twice the blocks (N = 5504: 688 instead of 344 for 256 CUs).
 // NW = wavefronts per block.
-template <int DT, bool W8, int MT, int MODE, int CG, int NW = SK_WAVES, bool PAIR = false>
+// SUM (single matrix, 16-bit weights, CG = 1): the chunks of the second rank's K follow those of the first one's (p.to leads to its operands), its
+// sums are kept apart, and the block stores the sum of both products. 4 rows of 4096 x 2048 a rank: 12.0 us in two launches, 9.3; of
+// 4096 x 5504 23.0 and 19.7 (4.6 TB/s: what is left is x from L2, 8 wavefronts a CU; 16 of them have half the registers each and gain nothing).
+template <int DT, bool W8, int MT, int MODE, int CG, int NW = SK_WAVES, bool PAIR = false, bool SUM = false>
 __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
     take_rank(p);
     static_assert(!PAIR || (MODE == SK_SWIGLU && CG == 1 && !W8), "PAIR is the gated pair with 16-bit weights");
+    static_assert(!SUM || (MODE == SK_LINEAR && CG == 1 && !W8), "SUM is a single matrix with 16-bit weights");
     constexpr int NMAT = (MODE == SK_SWIGLU && !PAIR) ? 2 : 1;
     constexpr int NA = NMAT * CG;             // weight tiles per chunk: index a = cg * NMAT + matrix
     constexpr bool PRE = CG == 1;             // double-buffered loads
@@ -169,7 +187,19 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[a][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int nchunks = (p.K + CHUNK_K - 1) / CHUNK_K;
+    const int nchunks = (p.K + CHUNK_K - 1) / CHUNK_K, total = SUM ? 2 * nchunks : nchunks;
+    f32x4 acc_first[SUM ? NA : 1][SUM ? MT : 1];  // SUM: the first rank's sums
+    bool past = false;                            // ... once this wavefront is at the second's
+    auto first_done = [&]() {
+#pragma unroll
+        for (int a = 0; a < (SUM ? NA : 0); ++a)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                acc_first[SUM ? a : 0][SUM ? t : 0] = acc[a][t];
+                acc[a][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        past = true;
+    };
 
     // Register double buffers for the weights (and for x when it is small enough). Buffer indices are
     // compile-time constants so that the arrays stay in registers.
@@ -178,6 +208,8 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
     uint4 xv[XPRE ? 2 : 1][MT][XV];
     auto load_w = [&](auto bufc, int c) {
         constexpr int buf = decltype(bufc)::value;
+        const int64_t to_w = SUM && c >= nchunks ? p.to.w : 0;
+        if (SUM && c >= nchunks) c -= nchunks;
         const int64_t off = static_cast<int64_t>(c) * CHUNK_K * wbytes;
 #pragma unroll
         for (int a = 0; a < NA; ++a)
@@ -187,7 +219,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
                 // Past the end of K the row's first bytes are fetched instead (always a load, never a branch, and nothing
                 // is done to the value until it is multiplied): x is zero there, so the product is too.
                 const bool ok = c * CHUNK_K + byte / wbytes < p.K;
-                const char *base = (a % NMAT == 0 ? wp[i & 1] : wp2[i & 1]) + (a / NMAT) * cg_stride;
+                const char *base = (a % NMAT == 0 ? wp[i & 1] : wp2[i & 1]) + (a / NMAT) * cg_stride + to_w;
                 wv[buf][a][i] = nt_load_u4(ok ? base + off + (i >> 1) * 128 : base - cpiece * 16);
             }
     };
@@ -223,7 +255,9 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
     // 256 (16-bit weights) or 512 (int8 weights) bytes of the row
     auto load_x = [&](auto bufc, int c) {
         constexpr int buf = decltype(bufc)::value;
-        const int64_t xoff = static_cast<int64_t>(c) * CHUNK_K * 2;
+        const int64_t to_x = SUM && c >= nchunks ? p.to.x : 0;
+        if (SUM && c >= nchunks) c -= nchunks;
+        const int64_t xoff = static_cast<int64_t>(c) * CHUNK_K * 2 + to_x;
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -238,6 +272,10 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
     auto compute = [&](auto bufc, int c) {
         constexpr int buf = decltype(bufc)::value;
         constexpr int xb = XPRE ? buf : 0;
+        if (SUM && c >= nchunks) {
+            if (!past) first_done();
+            c -= nchunks;
+        }
 #pragma unroll
         for (int a = 0; a < NA; ++a) transpose_w(wv[PRE ? buf : 0][a]);
 #pragma unroll
@@ -286,19 +324,19 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
     // ahead of the prefetch.
     // A prefetch past the wavefront's last chunk is a chunk past the end of K (loads of the rows' first bytes): every
     // pass through the loop issues the same loads, so each wait counts exactly the loads behind the one it needs.
-    auto in_k = [&](int c) { return c < nchunks ? c : nchunks; };
+    auto in_k = [&](int c) { return c < total ? c : total; };
     if constexpr (PRE) {
         int c = wave;
         load_w(B0{}, in_k(c));
         if constexpr (XPRE) load_x(B0{}, in_k(c));
-        while (c < nchunks) {
+        while (c < total) {
             int cn = c + NW;
             if constexpr (!XPRE) load_x(B0{}, c);
             load_w(B1{}, in_k(cn));
             if constexpr (XPRE) load_x(B1{}, in_k(cn));
             compute(B0{}, c);
             c = cn;
-            if (c >= nchunks) break;
+            if (c >= total) break;
             cn = c + NW;
             if constexpr (!XPRE) load_x(B0{}, c);
             load_w(B0{}, in_k(cn));
@@ -307,7 +345,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
             c = cn;
         }
     } else {
-        for (int c = wave; c < nchunks; c += NW) {
+        for (int c = wave; c < total; c += NW) {
             load_w(B0{}, c);
             load_x(B0{}, c);
             compute(B0{}, c);
@@ -374,23 +412,33 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
         }
     }
 
-    // ---- cross-wave reduction, one column group at a time through the same LDS array ------------------
+    if (SUM && !past) first_done();  // no chunk of the second rank for this wavefront
+
+    // ---- cross-wave reduction, one column group (SUM: one rank) at a time through the same LDS array ------------------
+    constexpr int PER_THREAD = (MT * 256 + NW * 64 - 1) / (NW * 64);
+    float first[PER_THREAD];
+    (void)first;
 #pragma unroll
-    for (int g = 0; g < CG; ++g) {
+    for (int g = 0; g < (SUM ? 2 : CG); ++g) {
         if (g > 0) __syncthreads();
 #pragma unroll
         for (int a = 0; a < NMAT; ++a)
 #pragma unroll
             for (int t = 0; t < MT; ++t)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) red[wave][a][t][i][lane] = acc[g * NMAT + a][t][i];
+                for (int i = 0; i < 4; ++i) {
+                    if constexpr (SUM) red[wave][a][t][i][lane] = g == 0 ? acc_first[a][t][i] : acc[a][t][i];
+                    else red[wave][a][t][i][lane] = acc[g * NMAT + a][t][i];
+                }
         __syncthreads();
 
         // thread e -> output (m = e / 16, n_local = e % 16): 16 consecutive threads store one 32-byte row piece
-        for (int e = tid; e < MT * 256; e += NW * 64) {
+#pragma unroll
+        for (int k = 0; k < PER_THREAD; ++k) {
+            const int e = tid + k * NW * 64;
             const int m = e >> 4, nl = e & 15;
-            if (PAIR && nl >= 8) continue;  // tile rows 8-15 are the up sums of columns 0-7
-            const int n = n0 + g * 16 + nl;
+            if (e >= MT * 256 || (PAIR && nl >= 8)) continue;  // tile rows 8-15 are the up sums of columns 0-7
+            const int n = n0 + (SUM ? 0 : g * 16) + nl;
             if (m >= p.M || n >= p.N) continue;
             const int t = m >> 4, src_lane = (nl >> 2) * 16 + (m & 15), i = nl & 3;
             float s0 = 0.f, s1 = 0.f;
@@ -400,7 +448,12 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyParams p) {
                 if constexpr (NMAT == 2) s1 += red[w][1][t][i][src_lane];
                 if constexpr (PAIR) s1 += red[w][0][t][i][src_lane + 32];  // row nl + 8: two lane groups further on
             }
-            skinny_store_output<DT, MODE>(p, s0, s1, m, n);
+            if constexpr (SUM) {
+                if (g == 0) first[k] = s0;
+                else skinny_store_sum<DT>(p, first[k], s0, m, n);
+            } else {
+                skinny_store_output<DT, MODE>(p, s0, s1, m, n);
+            }
         }
     }
 }
@@ -738,6 +791,7 @@ __global__ __launch_bounds__(SK_THREADS) void skinny_w8_split_kernel(SkinnyParam
 
 // y[m][n] = act(sum over splits of part[split][m][n] + bias[n]); VEC: four consecutive n per thread (N a multiple of 4),
 // the planes requested eight at a time and added in plane order
+// p.sum: the planes of both ranks, each rank's added up, then the sum of the two.
 template <int DT, bool VEC>
 __global__ __launch_bounds__(256) void skinny_w8_finish_kernel(SkinnyParams p, const float *part, int splits) {
     take_rank(p);
@@ -747,25 +801,40 @@ __global__ __launch_bounds__(256) void skinny_w8_finish_kernel(SkinnyParams p, c
         const int64_t e = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
         if (e >= plane) return;
         const int m = static_cast<int>(e / p.N), n = static_cast<int>(e % p.N);
-        f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-        int sp = 0;
-        for (; sp + 8 <= splits; sp += 8) {
-            f32x4 t[8];
+        auto added = [&](const float *planes) {
+            f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+            int sp = 0;
+            for (; sp + 8 <= splits; sp += 8) {
+                f32x4 t[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) t[j] = *reinterpret_cast<const f32x4 *>(part + (sp + j) * plane + e);
+                for (int j = 0; j < 8; ++j) t[j] = *reinterpret_cast<const f32x4 *>(planes + (sp + j) * plane + e);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v += t[j];
+                for (int j = 0; j < 8; ++j) v += t[j];
+            }
+            for (; sp < splits; ++sp) v += *reinterpret_cast<const f32x4 *>(planes + sp * plane + e);
+            return v;
+        };
+        const f32x4 v = added(part);
+        if (p.sum) {
+            const f32x4 u = added(part + splits * plane);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) skinny_store_sum<DT>(p, v[i], u[i], m, n + i);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) skinny_store_output<DT, SK_LINEAR>(p, v[i], 0.f, m, n + i);
         }
-        for (; sp < splits; ++sp) v += *reinterpret_cast<const f32x4 *>(part + sp * plane + e);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) skinny_store_output<DT, SK_LINEAR>(p, v[i], 0.f, m, n + i);
     } else {
         const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
         if (e >= plane) return;
         const int m = static_cast<int>(e / p.N), n = static_cast<int>(e % p.N);
-        float v = 0.f;
+        float v = 0.f, u = 0.f;
         for (int sp = 0; sp < splits; ++sp) v += part[sp * plane + e];
-        skinny_store_output<DT, SK_LINEAR>(p, v, 0.f, m, n);
+        if (p.sum) {
+            for (int sp = splits; sp < 2 * splits; ++sp) u += part[sp * plane + e];
+            skinny_store_sum<DT>(p, v, u, m, n);
+        } else {
+            skinny_store_output<DT, SK_LINEAR>(p, v, 0.f, m, n);
+        }
     }
 }
 
@@ -773,8 +842,8 @@ __global__ __launch_bounds__(256) void skinny_w8_finish_kernel(SkinnyParams p, c
 template <int DT>
 int launch_w8_finish(const SkinnyParams &p, const float *part, int splits, hipStream_t s) {
     const int64_t outputs = static_cast<int64_t>(p.M) * p.N;
-    if (p.N % 4 == 0) hipLaunchKernelGGL((skinny_w8_finish_kernel<DT, true>), dim3(static_cast<unsigned>((outputs / 4 + 255) / 256), 1, p.ranks), dim3(256), 0, s, p, part, splits);
-    else hipLaunchKernelGGL((skinny_w8_finish_kernel<DT, false>), dim3(static_cast<unsigned>((outputs + 255) / 256), 1, p.ranks), dim3(256), 0, s, p, part, splits);
+    if (p.N % 4 == 0) hipLaunchKernelGGL((skinny_w8_finish_kernel<DT, true>), dim3(static_cast<unsigned>((outputs / 4 + 255) / 256), 1, p.sum ? 1 : p.ranks), dim3(256), 0, s, p, part, splits);
+    else hipLaunchKernelGGL((skinny_w8_finish_kernel<DT, false>), dim3(static_cast<unsigned>((outputs + 255) / 256), 1, p.sum ? 1 : p.ranks), dim3(256), 0, s, p, part, splits);
     TPAMD_HIP(hipGetLastError());
     return TPAMD_OK;
 }
@@ -1326,6 +1395,80 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(SkinnyParams p) {
     }
 }
 
+// The sum of two ranks' Linears on at most 3 rows: a wavefront owns an output column and streams both ranks' rows of it (at most NP pieces each, all requested
+// back to back), so that a row-parallel Linear of two ranks is one launch with whole rows in flight instead of two, the second of which waits for
+// the first one's results. One row of 4096 x 2048 a rank: 9.4 us in two launches, 7.1 (4.7 TB/s, of
+// which 2 us are the launch); of 4096 x 5504 19.2 and 17.6. Two rows of more than 8 pieces spill at 16 wavefronts.
+template <int DT, int MR, int WAVES, int NP>
+__global__ __launch_bounds__(WAVES * 64) void gemv_sum_kernel(SkinnyParams p) {
+    constexpr int THREADS = WAVES * 64;
+    extern __shared__ __align__(16) char xs[];  // x[rank][MR][K]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = blockIdx.x * WAVES + wave;
+    const int row = n < p.N ? n : p.N - 1;
+    const int row_bytes = p.K * 2;
+    const char *w = p.w + static_cast<int64_t>(row) * p.ldw * 2;
+    constexpr int XL = (NP * 64 + THREADS - 1) / THREADS;  // 16-byte pieces of one row of x per thread
+    uint4 xr[2][MR][XL];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+            for (int i = 0; i < XL; ++i) {
+                const int at = (tid + i * THREADS) * 16;
+                xr[r][m][i] = *reinterpret_cast<const uint4 *>(p.x + (r ? p.to.x : 0) + static_cast<int64_t>(m) * p.ldx * 2 + (at < row_bytes ? at : 0));
+            }
+    uint4 wv[2][NP];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            // pieces past K are fetched from the row's start (always valid) and zeroed
+            const int at = j * 1024 + lane * 16;
+            const bool ok = at < row_bytes;
+            const uint4 a = nt_load_u4(w + (r ? p.to.w : 0) + (ok ? at : 0));
+            wv[r][j] = ok ? a : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+            for (int i = 0; i < XL; ++i) {
+                const int at = (tid + i * THREADS) * 16;
+                if (at < row_bytes) *reinterpret_cast<uint4 *>(xs + (r * MR + m) * row_bytes + at) = xr[r][m][i];
+            }
+    __syncthreads();
+    float acc[2][MR];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int m = 0; m < MR; ++m) acc[r][m] = 0.f;
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            const int at = j * 1024 + lane * 16 < row_bytes ? j * 1024 + lane * 16 : 0;
+#pragma unroll
+            for (int m = 0; m < MR; ++m) acc[r][m] = dot8<DT>(wv[r][j], *reinterpret_cast<const uint4 *>(xs + (r * MR + m) * row_bytes + at), acc[r][m]);
+        }
+#pragma unroll
+    for (int m = 0; m < MR; ++m) {
+        const float s0 = wave_sum_dpp(acc[0][m]), s1 = wave_sum_dpp(acc[1][m]);
+        if (lane == 0 && n < p.N) skinny_store_sum<DT>(p, s0, s1, m, n);
+    }
+}
+
+template <int DT, int WAVES, int NP>
+void launch_gemv_sum(const SkinnyParams &p, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>((p.N + WAVES - 1) / WAVES)), block(WAVES * 64);
+    const size_t lds = static_cast<size_t>(4) * p.M * p.K;
+    if (p.M == 1) hipLaunchKernelGGL((gemv_sum_kernel<DT, 1, WAVES, NP>), grid, block, lds, s, p);
+    else if (p.M == 2) hipLaunchKernelGGL((gemv_sum_kernel<DT, 2, WAVES, NP>), grid, block, lds, s, p);
+    else hipLaunchKernelGGL((gemv_sum_kernel<DT, 3, WAVES, NP>), grid, block, lds, s, p);
+}
+
 template <int DT, bool W8, int MODE, int WAVES, int NP>
 void launch_gemv_rows_m(const SkinnyParams &p, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>((p.N + WAVES - 1) / WAVES), 1, p.ranks), block(WAVES * 64);
@@ -1549,6 +1692,7 @@ int launch_w8_split(const SkinnyParams &p, hipStream_t s, bool *done) {
     cols_per_block = (cols_per_block + 15) / 16 * 16;
     col_blocks = (p.N + cols_per_block - 1) / cols_per_block;
     const dim3 grid(static_cast<unsigned>(col_blocks), static_cast<unsigned>(splits), p.ranks);
+    if (splits == 1 && p.sum) return TPAMD_OK;
     if (splits == 1) {  // nothing to add up: no scratch buffer, no second launch
         if (p.M <= 16) hipLaunchKernelGGL((skinny_w8_split_kernel<DT, 1, 4, true>), grid, dim3(SK_THREADS), 0, s, p, nullptr, cols_per_block);
         else if (p.M <= 32) hipLaunchKernelGGL((skinny_w8_split_kernel<DT, 2, 2, true>), grid, dim3(SK_THREADS), 0, s, p, nullptr, cols_per_block);
@@ -1601,6 +1745,7 @@ int launch_w8_cols_mt(const SkinnyParams &p, int dev, int cus, hipStream_t s, bo
     // the outlier plane is worked on by one block per 8 tiles of a column range (a tile per wavefront)
     const int outlier_blocks = p.n_out > 0 ? (cols_per_block / 16 + WC_NW - 1) / WC_NW : 0;
     const dim3 grid(static_cast<unsigned>(col_blocks), static_cast<unsigned>(k_planes + outlier_blocks), p.ranks);
+    if (planes == 1 && p.sum) return TPAMD_OK;
     if (planes == 1) {
         if (int rc = configure_w8_cols<DT, MT, true>(dev, lds); rc != TPAMD_OK) return rc;
         hipLaunchKernelGGL((skinny_w8_cols_kernel<DT, MT, KU, true>), grid, dim3(WC_NW * 64), lds, s, p, nullptr, cols_per_block, k_planes);
@@ -1960,6 +2105,69 @@ int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bi
     if (w8) return bf ? launch_skinny<TPAMD_BF16, true, SK_LINEAR>(p, s) : launch_skinny<TPAMD_F16, true, SK_LINEAR>(p, s);
     if (swiglu) return bf ? launch_skinny<TPAMD_BF16, false, SK_SWIGLU>(p, s) : launch_skinny<TPAMD_F16, false, SK_SWIGLU>(p, s);
     return bf ? launch_skinny<TPAMD_BF16, false, SK_LINEAR>(p, s) : launch_skinny<TPAMD_F16, false, SK_LINEAR>(p, s);
+}
+
+// y = the sum of two ranks' 16-bit Linears of one shape (M <= 64), the second one's operands `to` away, stored a second time `copy` bytes on. `row_waves`:
+// wavefronts per block of the row kernel, 0 for the MFMA kernel.
+int skinny_sum_dispatch(const void *x, const void *w, const void *bias, const RankStep &to, void *y, int64_t copy, int64_t M, int64_t N, int64_t K, int64_t ldx,
+                        int64_t ldw, int64_t ldy, int dtype, int row_waves, hipStream_t s) {
+    SkinnyParams p{};
+    p.ranks = 1;
+    p.sum = 1;
+    p.to = to;
+    p.copy = copy;
+    p.x = static_cast<const char *>(x);
+    p.w = static_cast<const char *>(w);
+    p.bias = static_cast<const char *>(bias);
+    p.y = static_cast<char *>(y);
+    p.M = static_cast<int>(M); p.N = static_cast<int>(N); p.K = static_cast<int>(K);
+    p.ldx = ldx; p.ldw = ldw; p.ldy = ldy;
+    TPAMD_REQUIRE(row_waves == 0 || (M <= GEMV_MAX_M && K <= 11 * 512 && M * K * 4 <= GEMV_MAX_X_BYTES), "skinny: rows too long for the row kernel");
+    auto run = [&](auto dt) {
+        constexpr int DT = decltype(dt)::value;
+        const dim3 grid(static_cast<unsigned>((N + 15) / 16)), block(SK_THREADS);
+        if (row_waves == 16) {
+            if (K <= 8 * 512) launch_gemv_sum<DT, 16, 8>(p, s);
+            else launch_gemv_sum<DT, 16, 11>(p, s);
+        } else if (row_waves == 8) {
+            if (K <= 4 * 512) launch_gemv_sum<DT, 8, 4>(p, s);
+            else if (K <= 8 * 512) launch_gemv_sum<DT, 8, 8>(p, s);
+            else launch_gemv_sum<DT, 8, 11>(p, s);
+        } else if (M <= 16) hipLaunchKernelGGL((skinny_kernel<DT, false, 1, SK_LINEAR, 1, SK_WAVES, false, true>), grid, block, 0, s, p);
+        else if (M <= 32) hipLaunchKernelGGL((skinny_kernel<DT, false, 2, SK_LINEAR, 1, SK_WAVES, false, true>), grid, block, 0, s, p);
+        else hipLaunchKernelGGL((skinny_kernel<DT, false, 4, SK_LINEAR, 1, SK_WAVES, false, true>), grid, block, 0, s, p);
+    };
+    if (dtype == TPAMD_BF16) run(std::integral_constant<int, TPAMD_BF16>{});
+    else run(std::integral_constant<int, TPAMD_F16>{});
+    TPAMD_HIP(hipGetLastError());
+    return TPAMD_OK;
+}
+
+// The same for int8 weights (2 <= M <= 64) where K is split over blocks: the finishing pass adds both ranks' planes. *done = false: not taken.
+int skinny_w8_sum_dispatch(const void *x, const void *wq, const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out, const void *bias,
+                           const RankStep &to, void *y, int64_t copy, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout, int64_t ldy,
+                           int dtype, hipStream_t s, bool *done) {
+    *done = false;
+    if (M < 2 || M > 64) return TPAMD_OK;
+    SkinnyParams p{};
+    p.ranks = 2;
+    p.sum = 1;
+    p.to = to;
+    p.to.y = 0;
+    p.copy = copy;
+    p.x = static_cast<const char *>(x);
+    p.w = static_cast<const char *>(wq);
+    p.bias = static_cast<const char *>(bias);
+    p.scale = static_cast<const float *>(scale);
+    p.outlier_idx = static_cast<const int *>(outlier_idx);
+    p.w_out = static_cast<const char *>(w_out);
+    p.y = static_cast<char *>(y);
+    p.M = static_cast<int>(M); p.N = static_cast<int>(N); p.K = static_cast<int>(K);
+    p.n_out = static_cast<int>(n_out);
+    p.ldx = ldx; p.ldw = ldw; p.ldy = ldy; p.ld_wout = ld_wout;
+    int rc = dtype == TPAMD_BF16 ? launch_w8_cols<TPAMD_BF16>(p, s, done) : launch_w8_cols<TPAMD_F16>(p, s, done);
+    if (rc != TPAMD_OK || *done) return rc;
+    return dtype == TPAMD_BF16 ? launch_w8_split<TPAMD_BF16>(p, s, done) : launch_w8_split<TPAMD_F16>(p, s, done);
 }
 
 }  // namespace tpamd

@@ -23,7 +23,7 @@ from torch import nn
 
 from . import _native, together
 from . import shard_modules
-from .shard_modules import _guard, is_conv1d, product_in_context
+from .shard_modules import is_conv1d, product_in_context
 
 OutlierChoice = Union[None, Mapping[str, Sequence[int]], Callable[[str, nn.Module], Optional[Sequence[int]]]]
 
@@ -62,11 +62,6 @@ def quantize_rows(w: torch.Tensor, outlier_cols: Optional[torch.Tensor] = None) 
     return q, scale, cols.to(torch.int32), w.detach()[:, cols].contiguous()
 
 
-# Up to this many rows the weights of two ranks stream in one launch, and the sum over ranks is a launch of its own behind them; above, a rank's Linear fills the
-# device and the one that comes last adds the other's result (the Falcon-40B-shaped layer: 16 rows 294 us this way and 301 the other, 1024 rows 1492 and 1462).
-TOGETHER_ROWS = 64
-
-
 class ShardLinearW8(nn.Module):
     """A Linear whose weight is stored as int8 rows with one float32 scale each, plus the outlier input columns in the
     activation dtype; the forward is `tpamd_linear_w8`. Inference only."""
@@ -98,10 +93,8 @@ class ShardLinearW8(nn.Module):
             raise TypeError(f"ShardLinearW8: the input is {input.dtype}, the Linear was quantised for {self.dtype}")
         n_out = self.outlier_idx.numel()
         operands = (input.detach(), self.wq, self.scale, self.outlier_idx if n_out else None, self.w_out if n_out else None, self.bias)
-        if input.numel() <= TOGETHER_ROWS * self.in_features:
-            return _guard(together.linear_w8(*operands), input)
         return product_in_context(self, input, self.out_features, (input,), lambda: together.linear_w8(*operands),
-                                  lambda **more: _native.linear_w8(*operands, **more))
+                                  lambda **more: _native.linear_w8(*operands, **more), lambda rank: together.linear_w8_sum(*operands, rank))
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "

@@ -47,12 +47,14 @@ def _guard(out: torch.Tensor, *inputs: torch.Tensor) -> torch.Tensor:
 def linear_in_context(module: nn.Module, x: torch.Tensor, w: torch.Tensor, bias) -> torch.Tensor:
     """`tpamd_linear` for a shard's Linear; see `product_in_context`."""
     xd, wd, b = x.detach(), w.detach(), None if bias is None else bias.detach()
-    return product_in_context(module, x, w.shape[0], (x, w, bias), lambda: together.linear(xd, wd, b), lambda **more: _native.linear(xd, wd, b, **more))
+    return product_in_context(module, x, w.shape[0], (x, w, bias), lambda: together.linear(xd, wd, b), lambda **more: _native.linear(xd, wd, b, **more),
+                              lambda rank: together.linear_sum(xd, wd, b, rank))
 
 
-def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs: tuple, with_peers, alone) -> torch.Tensor:
+def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs: tuple, with_peers, alone, summed) -> torch.Tensor:
     """A shard's Linear with `columns` outputs, made by with_peers() or, with an addend, alone(addend=, copy=). Inside a wrapped module whose output goes to a
-    "sum" rule (collectives.SumContext) the Linear that was seen to produce that output adds the partial sums already waiting in
+    "sum" rule (collectives.SumContext) the Linear that was seen to produce that output hands over the sum: two ranks that meet in it get it from
+    summed(rank) (`tpamd_linear_sum_ranks`), else the rank that comes last adds the partial sums already waiting in
     the reduction, in its epilogue (`tpamd_linear_add`): the product rounded to the dtype, then one rounded add, which
     is the same arithmetic as the reduction kernel's step."""
     from .collectives import current_sum_context
@@ -62,29 +64,44 @@ def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs:
         return _guard(with_peers(), *inputs)
     key = id(module)
     ctx.calls[key] = ctx.calls.get(key, 0) + 1
-    more = {}
+    out, more = None, {}
     if module.__dict__.get("_tp_feeds_sum") is ctx.owner and ctx.owner is not None:
         if ctx.fused_out is not None:
             raise RuntimeError("tensor_parallel_amd: the Linear that feeds a \"sum\" rule ran twice in one call of its module "
                                "after adding the waiting partial sums; set TPAMD_FUSE_SUM=0")
         waiting = ctx.op.addend_for(ctx.rank)
-        if waiting is not None:
-            t, mask = waiting
-            if t.dtype == x.dtype and t.device == x.device and t.shape == (*x.shape[:-1], columns):
-                more["addend"], ctx.fused_mask = t.detach(), mask
-                if ctx.op.world_size == 2:  # the sum is complete then: a second tensor for the other rank comes out of the same launch
-                    more["copy"] = torch.empty_like(more["addend"], memory_format=torch.contiguous_format)
-        out = alone(**more)
-    # Ranks do not meet in the Linear that feeds the sum (the one that comes last adds the others' partials), nor before a first call has shown which one that is.
-    else:
-        out = with_peers() if "_tp_sum_known" in ctx.owner.__dict__ else alone()
-    out = _guard(out, *inputs)
+        if waiting is None and ctx.op.world_size == 2 and _sum_unwatched(module, ctx.owner):
+            out = summed(ctx.rank)
+        if out is not None:
+            out = _guard(out, *inputs)
+            ctx.fused_out, ctx.fused_mask, ctx.fused_whole = out, 3, out._version
+        else:
+            if waiting is None:  # (a rank that waited for its peer in vain finds what that one has handed in since)
+                waiting = ctx.op.addend_for(ctx.rank)
+            if waiting is not None:
+                t, mask = waiting
+                if t.dtype == x.dtype and t.device == x.device and t.shape == (*x.shape[:-1], columns):
+                    more["addend"], ctx.fused_mask = t.detach(), mask
+                    if ctx.op.world_size == 2:  # the sum is complete then: a second tensor for the other rank comes out of the same launch
+                        more["copy"] = torch.empty_like(more["addend"], memory_format=torch.contiguous_format)
+            out = _guard(alone(**more), *inputs)
+    else:  # ranks meet in other Linears once a first call has shown which one feeds the sum
+        out = _guard(with_peers() if "_tp_sum_known" in ctx.owner.__dict__ else alone(), *inputs)
     if more:
         ctx.fused_out = out
         if "copy" in more and not out.is_inference():  # (whose changes are not counted)
             ctx.fused_copy = more["copy"], out._version
     ctx.last_linear, ctx.last_out = module, out
+    ctx.last_version = None if out.is_inference() else out._version
     return out
+
+
+def _sum_unwatched(module: nn.Module, owner: nn.Module) -> bool:
+    """Whether nobody is told of a Linear's output on its way to the sum, so that it may be the sum already: no hooks on it, on the module around it (the wrapped one)
+    or on all modules; and changes to it would show (they are not counted in inference mode)."""
+    wrapped, hooks = owner.tp_wrapped_module, torch.nn.modules.module
+    return not (torch.is_inference_mode_enabled() or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _has_hooks(module) or _has_hooks(wrapped)) \
+        and (wrapped is module or any(child is module for child in wrapped._modules.values()))
 
 
 def gathered_linear(module: nn.Module, op, rank: int, args, kwargs):

@@ -175,6 +175,53 @@ def _not_together(*_: Any) -> None:
     return None
 
 
+def _linear_sum(calls: List[tuple]) -> Sequence[torch.Tensor]:
+    ranks = [call[:3] for call in sorted(calls, key=lambda call: call[3])]
+    sums = _native.linear_sum_ranks(ranks)
+    if sums is None:  # operands that the kernels do not take, or no scratch memory
+        first = _native.linear(*ranks[0])
+        copy = torch.empty_like(first)
+        sums = [copy, _native.linear(*ranks[1], addend=first, copy=copy)]
+    return sums
+
+
+def linear_sum(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], rank: int) -> Optional[torch.Tensor]:
+    """The sum of two ranks' Linears, a tensor of its own for each; None where this rank is on its own or two launches are faster."""
+    K = x.shape[-1]
+    if K == 0 or w.dim() != 2 or x.dtype is torch.float32 or not _native.linear_sum_pays(x.numel() // K, w.shape[0], K, x.dtype):
+        return None
+    return _call(_not_together, _linear_sum, (x, w, bias), (), (rank,))
+
+
+# Up to this many rows the int8 kernels take two ranks in one launch, and a sum that those cannot add up is a launch of its own behind them; above, a rank's Linear
+# fills the device and adds the other's result (the Falcon-40B-shaped layer: 16 rows 294 us this way and 301 the other, 1024 rows 1492 and 1462).
+W8_TOGETHER_ROWS = 64
+
+
+def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, outlier_idx: Optional[torch.Tensor], w_out: Optional[torch.Tensor],
+              bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    if x.numel() > W8_TOGETHER_ROWS * x.shape[-1]:
+        return _native.linear_w8(x, wq, scale, outlier_idx, w_out, bias)
+    return _call(_native.linear_w8, _native.linear_w8_ranks, (x, wq, scale, outlier_idx, w_out, bias))
+
+
+def _linear_w8_sum(calls: List[tuple]) -> Sequence[torch.Tensor]:
+    ranks = [call[:6] for call in sorted(calls, key=lambda call: call[6])]
+    sums = _native.linear_w8_sum_ranks(ranks)
+    if sums is None:
+        parts = _native.linear_w8_ranks(ranks)
+        copy = torch.empty_like(parts[0])
+        sums = [copy, _native.reduce_partials(parts, copy=copy)]
+    return sums
+
+
+def linear_w8_sum(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, outlier_idx: Optional[torch.Tensor], w_out: Optional[torch.Tensor],
+                  bias: Optional[torch.Tensor], rank: int) -> Optional[torch.Tensor]:
+    if x.numel() > W8_TOGETHER_ROWS * x.shape[-1]:
+        return None
+    return _call(_not_together, _linear_w8_sum, (x, wq, scale, outlier_idx, w_out, bias), (), (rank,))
+
+
 def _gather(calls: List[tuple]) -> Sequence[torch.Tensor]:
     return _native.linear_gather_ranks([call[:3] for call in sorted(calls, key=lambda call: call[3])])  # (every rank's result is the same)
 
@@ -208,11 +255,6 @@ def layer_norm(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], eps:
     if x.numel() >= ALONE_ROWS * w.numel():
         return _native.layer_norm(x, w, b, eps)
     return _call(_native.layer_norm, _native.layer_norm_ranks, (x, w, b), (eps,))
-
-
-def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, outlier_idx: Optional[torch.Tensor], w_out: Optional[torch.Tensor],
-              bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    return _call(_native.linear_w8, _native.linear_w8_ranks, (x, wq, scale, outlier_idx, w_out, bias))
 
 
 def attention_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor,

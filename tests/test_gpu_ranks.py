@@ -204,7 +204,7 @@ def test_a_sum_that_somebody_writes_to_is_copied_as_it_is(rank):
         model(x)
         handle.remove()
     assert len(ranks) == 2 and torch.equal(ranks[0], ranks[1])
-    torch.testing.assert_close(ranks[0], want + 1.0, rtol=2.0 ** -7, atol=0)  # added before or after the sum: two roundings of 2^-9 around 1
+    torch.testing.assert_close(ranks[0], want + 1.0, rtol=0, atol=3 * 2.0 ** -8)  # added before or after the sum: three roundings of values below 2, 2^-8 each
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -223,3 +223,48 @@ def test_int8_linear_adds_a_partial_sum_and_copies_it(rows, cols, K, n_out, gelu
     y = _native.linear_w8(x, q, scale, idx, w_out, act=act, addend=addend, copy=copy)
     assert torch.equal(y, plain + addend) and torch.equal(copy, y)
     assert torch.equal(_native.linear_w8(x, q, scale, idx, w_out, act=act, addend=addend), y)
+
+
+# rows: the row kernel, weight streaming with one, two and four tiles of rows, K ranges of 128 x 128 tiles with part and whole tiles of x; K on both sides of 1024 and of
+# the row kernel's 11 pieces, ragged chunks
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 15, 16, 17, 32, 33, 64, 65, 130, 512, 700, 2100])
+@pytest.mark.parametrize("cols,K,bias", [(4096, 2048, False), (4096, 5504, False), (1028, 1024, True), (516, 1040, False), (2048, 1000, False), (4, 5640, True), (8192, 4096, False), (5120, 1088, True), (1024, 2048, False)])
+def test_the_sum_of_two_ranks_linears(rows, cols, K, bias, dtype):
+    xs, ws = draws(2, rows, K, dtype=dtype), draws(2, cols, K, dtype=dtype, scale=0.05, seed=1)
+    bs = draws(2, cols, dtype=dtype, seed=2) if bias else [None, None]
+    sums = _native.linear_sum_ranks(list(zip(xs, ws, bs)))
+    if sums is None:  # left to two launches
+        assert not _native.linear_sum_pays(rows, cols, K, dtype)
+        return
+    parts = [x.double() @ w.double().t() + (0 if b is None else b.double()) for x, w, b in zip(xs, ws, bs)]
+    assert sums[0].data_ptr() != sums[1].data_ptr() and torch.equal(*sums)
+    # each product rounded to the dtype, then their sum: three roundings, each of half a unit in the last place, and fp32 sums of K products
+    u = 2.0 ** (-8 if dtype is torch.bfloat16 else -11)
+    want = parts[0] + parts[1]
+    bound = u * (parts[0].abs() + parts[1].abs() + want.abs()) * 1.02 + K * 2.0 ** -24 * want.std()
+    assert bool(((sums[0].double() - want).abs() <= bound + 1e-30).all())
+    alone = _native.linear(xs[1], ws[1], bs[1], addend=_native.linear(xs[0], ws[0], bs[0]))
+    assert (sums[0].double() - want).norm() <= 1.05 * (alone.double() - want).norm()
+
+
+@pytest.mark.parametrize("rows", [1, 2, 5, 16, 17, 48, 64, 65])
+@pytest.mark.parametrize("cols,K,n_out", [(2048, 4096, 20), (8192, 16384, 81), (4100, 4112, 3), (16384, 8192, 0)])
+def test_the_sum_of_two_ranks_int8_linears(rows, cols, K, n_out):
+    dtype, calls, parts = torch.float16, [], []
+    for r in range(2):
+        g = torch.Generator(device=DEV).manual_seed(r)
+        x = draws(1, rows, K, dtype=dtype, seed=r)[0]
+        q = torch.randint(-127, 128, (cols, K), device=DEV, generator=g, dtype=torch.int8)
+        scale = torch.rand(cols, device=DEV, generator=g) * 1e-3
+        idx = torch.randperm(K, device=DEV, generator=g)[:n_out].sort().values.to(torch.int32) if n_out else None
+        w_out = draws(1, cols, n_out, dtype=dtype, seed=3 + r)[0] if n_out else None
+        calls.append((x, q, scale, idx, w_out, None))
+        parts.append(_native.linear_w8(*calls[-1]))
+    sums = _native.linear_w8_sum_ranks(calls)
+    if sums is None:
+        return
+    assert sums[0].data_ptr() != sums[1].data_ptr() and torch.equal(*sums)
+    want = parts[0].float() + parts[1].float()  # both rounded products, each of which may be rounded the other way where the planes are cut elsewhere
+    bound = 2.0 ** -11 * (want.abs() + 2 * (parts[0].float().abs() + parts[1].float().abs())) + 1e-6
+    assert bool(((sums[0].float() - want).abs() <= bound).all())
