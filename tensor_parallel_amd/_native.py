@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import os
+from array import array
 from pathlib import Path
 from typing import Optional, Sequence
 
@@ -73,6 +74,10 @@ _DTYPES = {torch.bfloat16: BF16, torch.float16: F16, torch.float32: F32}
 
 class NativeLibraryError(RuntimeError):
     pass
+
+
+class Unsupported(RuntimeError):
+    """The library has no kernel for what it was asked for; nothing was launched."""
 
 
 class CopyJob(ctypes.Structure):
@@ -164,7 +169,7 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_rope_tables.argtypes = [vp, ci, vp, i64, i64, i64, i64, i64, c.c_float, vp, vp, ci, vp]
     lib.tpamd_causal_mask.restype = ci
     lib.tpamd_causal_mask.argtypes = [vp, i64, i64, i64, vp, vp]
-    pp = c.POINTER(vp)
+    pp = vp  # the address of an array of pointers (_Pointers)
     lib.tpamd_linear_ranks.restype = ci
     lib.tpamd_linear_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, i64, i64, ci, ci, vp]
     lib.tpamd_linear_gather_ranks.restype = ci
@@ -238,6 +243,8 @@ def _check(rc: int, what: str) -> None:
         msg = lib().tpamd_last_error().decode("utf-8", "replace")
         if rc == -1:
             raise ValueError(f"{what}: {msg}")
+        if rc == -2:
+            raise Unsupported(f"{what} failed (status {rc}): {msg}")
         raise RuntimeError(f"{what} failed (status {rc}): {msg}")
 
 
@@ -509,30 +516,62 @@ def _check_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]
 
 
 # The *_ranks functions take the operands of several ranks whose tensors agree in shape, strides, dtype and device (together.GreenTurn.meet compares
-# them): what holds for the first rank's holds for all.
-_pointer_arrays = [ctypes.c_void_p * n for n in range(9)]
+# them): what holds for the first rank's holds for all. They are called once per layer and more of an eager forward, whose pace the host sets.
+def _rows(tensors: list) -> tuple:
+    """The tensors as row-major matrices with contiguous rows (their memory, where it is one already) and the elements between rows."""
+    if tensors[0].is_contiguous():
+        return tensors, max(tensors[0].shape[-1], 1)
+    tensors = [_as_2d(t) for t in tensors]
+    return tensors, _ld(tensors[0])
 
 
-def _pointers(tensors: Sequence[torch.Tensor]):
-    n = len(tensors)
-    return (_pointer_arrays[n] if n < len(_pointer_arrays) else ctypes.c_void_p * n)(*[t.data_ptr() for t in tensors])
+def _contiguous(tensors: list) -> list:
+    return tensors if tensors[0].is_contiguous() else [t.contiguous() for t in tensors]
+
+
+def _run(what: str, call, index: int, pointers: list, *args) -> None:
+    """call(addresses of arrays with the data pointers of each list of tensors (None: no array), *args, stream) on HIP device `index`."""
+    n = len(pointers[0])
+    block = array("Q", [t.data_ptr() for tensors in pointers if tensors is not None for t in tensors])
+    at, where = block.buffer_info()[0], []
+    for tensors in pointers:
+        where.append(None if tensors is None else at)
+        if tensors is not None:
+            at += 8 * n
+    prev = torch.cuda.current_device()
+    if prev != index:
+        torch.cuda.set_device(index)
+    try:
+        rc = call(*where, *args, _raw_stream(index) if _raw_stream is not None else torch.cuda.current_stream(index).cuda_stream)
+    finally:
+        if prev != index:
+            torch.cuda.set_device(prev)
+    if rc != 0:
+        _check(rc, what)
+
+
+def _linear_operands(calls: Sequence[tuple]) -> tuple:
+    """x, w, bias of all ranks (None: no bias) and the dimensions M, N, K, ldx, ldw."""
+    x, w, bias = calls[0]
+    _check_linear(x, w, bias)
+    N, K = w.shape
+    xs, ldx = _rows([c[0] for c in calls])
+    ws, ldw = _rows([c[1] for c in calls])
+    return xs, ws, None if bias is None else _contiguous([c[2] for c in calls]), (x.numel() // K if K else xs[0].numel(), N, K, ldx, ldw)
+
+
+def _outputs(x: torch.Tensor, columns: int, n: int) -> list:
+    shape = (*x.shape[:-1], columns)
+    return [torch.empty(shape, dtype=x.dtype, device=x.device) for _ in range(n)]
 
 
 def linear_ranks(calls: Sequence[tuple]) -> list:
     """`linear(x, w, bias)` for the (x, w, bias) of several ranks."""
-    x, w, bias = calls[0]
-    _check_linear(x, w, bias)
-    xs, ws = [_as_2d(c[0]) for c in calls], [_as_2d(c[1]) for c in calls]
-    (M, K), N = xs[0].shape, w.shape[0]
-    ys = [torch.empty((M, N), dtype=x.dtype, device=x.device) for _ in calls]
-    bs = None if bias is None else [c[2].contiguous() for c in calls]
-    with _on_device(x.device):
-        _check(
-            lib().tpamd_linear_ranks(len(calls), _pointers(xs), _pointers(ws), None if bs is None else _pointers(bs), _pointers(ys), M, N, K,
-                                     _ld(xs[0]), _ld(ws[0]), N, dtype_code(x.dtype), ACT_NONE, ctypes.c_void_p(current_stream_ptr(x.device))),
-            "tpamd_linear_ranks",
-        )
-    return [y.view(*x.shape[:-1], N) for y in ys]
+    xs, ws, bs, dims = _linear_operands(calls)
+    x, N = calls[0][0], dims[1]
+    ys = _outputs(x, N, len(calls))
+    _run("tpamd_linear_ranks", functools.partial(lib().tpamd_linear_ranks, len(calls)), x.get_device(), [xs, ws, bs, ys], *dims, N, dtype_code(x.dtype), ACT_NONE)
+    return ys
 
 
 @functools.lru_cache(maxsize=4096)
@@ -543,37 +582,24 @@ def linear_sum_pays(M: int, N: int, K: int, dtype: torch.dtype) -> bool:
 
 def linear_sum_ranks(calls: Sequence[tuple]) -> Optional[list]:
     """The sum of two ranks' `linear(x, w, bias)`, for each a tensor of its own, in one launch; None where there is none for the shape."""
-    x, w, bias = calls[0]
-    _check_linear(x, w, bias)
-    xs, ws = [_as_2d(c[0]) for c in calls], [_as_2d(c[1]) for c in calls]
-    (M, K), N = xs[0].shape, w.shape[0]
-    ys = [torch.empty((M, N), dtype=x.dtype, device=x.device) for _ in calls]
-    bs = None if bias is None else [c[2].contiguous() for c in calls]
-    with _on_device(x.device):
-        rc = lib().tpamd_linear_sum_ranks(_pointers(xs), _pointers(ws), None if bs is None else _pointers(bs), _pointers(ys), M, N, K, _ld(xs[0]), _ld(ws[0]), N,
-                                          dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device)))
-    if rc == -2:
+    xs, ws, bs, dims = _linear_operands(calls)
+    x, N = calls[0][0], dims[1]
+    ys = _outputs(x, N, len(calls))
+    try:
+        _run("tpamd_linear_sum_ranks", lib().tpamd_linear_sum_ranks, x.get_device(), [xs, ws, bs, ys], *dims, N, dtype_code(x.dtype))
+    except Unsupported:
         return None
-    _check(rc, "tpamd_linear_sum_ranks")
-    return [y.view(*x.shape[:-1], N) for y in ys]
+    return ys
 
 
 def linear_gather_ranks(calls: Sequence[tuple]) -> list:
     """The `linear(x, w, bias)` of all ranks side by side along the last axis, for each rank a tensor of its own."""
-    x, w, bias = calls[0]
-    _check_linear(x, w, bias)
-    xs, ws = [_as_2d(c[0]) for c in calls], [_as_2d(c[1]) for c in calls]
-    (M, K), N = xs[0].shape, w.shape[0]
-    whole = N * len(calls)
-    ys = [torch.empty((M, whole), dtype=x.dtype, device=x.device) for _ in calls]
-    bs = None if bias is None else [c[2].contiguous() for c in calls]
-    with _on_device(x.device):
-        _check(
-            lib().tpamd_linear_gather_ranks(len(calls), _pointers(xs), _pointers(ws), None if bs is None else _pointers(bs), _pointers(ys), M, N, K,
-                                            _ld(xs[0]), _ld(ws[0]), whole, dtype_code(x.dtype), ACT_NONE, ctypes.c_void_p(current_stream_ptr(x.device))),
-            "tpamd_linear_gather_ranks",
-        )
-    return [y.view(*x.shape[:-1], whole) for y in ys]
+    xs, ws, bs, dims = _linear_operands(calls)
+    x, whole = calls[0][0], dims[1] * len(calls)
+    ys = _outputs(x, whole, len(calls))
+    _run("tpamd_linear_gather_ranks", functools.partial(lib().tpamd_linear_gather_ranks, len(calls)), x.get_device(), [xs, ws, bs, ys], *dims, whole,
+         dtype_code(x.dtype), ACT_NONE)
+    return ys
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act: int = ACT_NONE,
@@ -652,18 +678,16 @@ def swiglu_up_ranks(calls: Sequence[tuple]) -> list:
     """`swiglu_up(x, wg, wu)` for the operands of several ranks."""
     x, wg, wu = calls[0]
     _check_swiglu_up(x, wg, wu)
-    xs, gs, us = ([_as_2d(c[i]) for c in calls] for i in range(3))
-    if _ld(gs[0]) != _ld(us[0]):
-        gs, us = [g.contiguous() for g in gs], [u.contiguous() for u in us]
-    (M, K), N = xs[0].shape, wg.shape[0]
-    hs = [torch.empty((M, N), dtype=x.dtype, device=x.device) for _ in calls]
-    with _on_device(x.device):
-        _check(
-            lib().tpamd_swiglu_up_ranks(len(calls), _pointers(xs), _pointers(gs), _pointers(us), _pointers(hs), M, N, K, _ld(xs[0]), _ld(gs[0]), N,
-                                        dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device))),
-            "tpamd_swiglu_up_ranks",
-        )
-    return [h.view(*x.shape[:-1], N) for h in hs]
+    xs, ldx = _rows([c[0] for c in calls])
+    gs, ldg = _rows([c[1] for c in calls])
+    us, ldu = _rows([c[2] for c in calls])
+    N, K = wg.shape
+    if ldg != ldu:
+        gs, us, ldg = [g.contiguous() for g in gs], [u.contiguous() for u in us], max(K, 1)
+    hs = _outputs(x, N, len(calls))
+    _run("tpamd_swiglu_up_ranks", functools.partial(lib().tpamd_swiglu_up_ranks, len(calls)), x.get_device(), [xs, gs, us, hs],
+         x.numel() // K if K else xs[0].numel(), N, K, ldx, ldg, N, dtype_code(x.dtype))
+    return hs
 
 
 def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
@@ -677,16 +701,13 @@ def rms_norm_ranks(calls: Sequence[tuple]) -> list:
     require_device(x, "rms_norm")
     if w.dtype != x.dtype or w.get_device() != x.get_device() or w.dim() != 1 or x.dim() == 0 or x.shape[-1] != w.shape[0]:
         raise ValueError(f"rms_norm: x {tuple(x.shape)} {x.dtype} on {x.device} and w {tuple(w.shape)} {w.dtype} on {w.device} do not fit")
-    xs, ws = [_as_2d(c[0]) for c in calls], [c[1].contiguous() for c in calls]
-    rows, D = xs[0].shape
-    ys = [torch.empty((rows, D), dtype=x.dtype, device=x.device) for _ in calls]
-    with _on_device(x.device):
-        _check(
-            lib().tpamd_rms_norm_ranks(len(calls), _pointers(xs), _pointers(ws), _pointers(ys), rows, D, _ld(xs[0]), D, float(eps),
-                                       dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device))),
-            "tpamd_rms_norm",
-        )
-    return [y.view(x.shape) for y in ys]
+    D = w.shape[0]
+    xs, ldx = _rows([c[0] for c in calls])
+    ys = _outputs(x, D, len(calls))
+    if D:
+        _run("tpamd_rms_norm", functools.partial(lib().tpamd_rms_norm_ranks, len(calls)), x.get_device(), [xs, _contiguous([c[1] for c in calls]), ys],
+             x.numel() // D, D, ldx, D, float(eps), dtype_code(x.dtype))
+    return ys
 
 
 def add_rms_norm(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float) -> tuple:
@@ -702,17 +723,14 @@ def add_rms_norm_ranks(calls: Sequence[tuple]) -> list:
             or x.dim() == 0 or x.shape[-1] != w.shape[0]):
         raise ValueError(f"add_rms_norm: r {tuple(r.shape)} {r.dtype} on {r.device}, x {tuple(x.shape)} {x.dtype} on {x.device} and w {tuple(w.shape)} "
                          f"{w.dtype} on {w.device} do not fit")
-    rs, xs, ws = [_as_2d(c[0]) for c in calls], [_as_2d(c[1]) for c in calls], [c[2].contiguous() for c in calls]
-    rows, D = xs[0].shape
-    totals = [torch.empty((rows, D), dtype=x.dtype, device=x.device) for _ in calls]
-    ys = [torch.empty_like(t) for t in totals]
-    with _on_device(x.device):
-        _check(
-            lib().tpamd_add_rms_norm_ranks(len(calls), _pointers(xs), _pointers(rs), _pointers(ws), _pointers(totals), _pointers(ys), rows, D,
-                                           _ld(xs[0]), _ld(rs[0]), D, float(eps), dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device))),
-            "tpamd_add_rms_norm",
-        )
-    return [(total.view(x.shape), y.view(x.shape)) for total, y in zip(totals, ys)]
+    D = w.shape[0]
+    xs, ldx = _rows([c[1] for c in calls])
+    rs, ldr = _rows([c[0] for c in calls])
+    totals, ys = _outputs(x, D, len(calls)), _outputs(x, D, len(calls))
+    if D:
+        _run("tpamd_add_rms_norm", functools.partial(lib().tpamd_add_rms_norm_ranks, len(calls)), x.get_device(),
+             [xs, rs, _contiguous([c[2] for c in calls]), totals, ys], x.numel() // D, D, ldx, ldr, D, float(eps), dtype_code(x.dtype))
+    return list(zip(totals, ys))
 
 
 def layer_norm(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], eps: float) -> torch.Tensor:
@@ -727,17 +745,14 @@ def layer_norm_ranks(calls: Sequence[tuple]) -> list:
     for t in (w, b):
         if t is not None and (t.dtype != x.dtype or t.get_device() != x.get_device() or t.dim() != 1 or x.dim() == 0 or x.shape[-1] != t.shape[0]):
             raise ValueError(f"layer_norm: x {tuple(x.shape)} {x.dtype} on {x.device} and {tuple(t.shape)} {t.dtype} on {t.device} do not fit")
-    xs, ws = [_as_2d(c[0]) for c in calls], [c[1].contiguous() for c in calls]
-    bs = None if b is None else [c[2].contiguous() for c in calls]
-    rows, D = xs[0].shape
-    ys = [torch.empty((rows, D), dtype=x.dtype, device=x.device) for _ in calls]
-    with _on_device(x.device):
-        _check(
-            lib().tpamd_layer_norm_ranks(len(calls), _pointers(xs), _pointers(ws), None if bs is None else _pointers(bs), _pointers(ys), rows, D,
-                                         _ld(xs[0]), D, float(eps), dtype_code(x.dtype), ctypes.c_void_p(current_stream_ptr(x.device))),
-            "tpamd_layer_norm",
-        )
-    return [y.view(x.shape) for y in ys]
+    D = w.shape[0]
+    xs, ldx = _rows([c[0] for c in calls])
+    ys = _outputs(x, D, len(calls))
+    if D:
+        _run("tpamd_layer_norm", functools.partial(lib().tpamd_layer_norm_ranks, len(calls)), x.get_device(),
+             [xs, _contiguous([c[1] for c in calls]), None if b is None else _contiguous([c[2] for c in calls]), ys], x.numel() // D, D, ldx, D, float(eps),
+             dtype_code(x.dtype))
+    return ys
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None, causal: bool = True,

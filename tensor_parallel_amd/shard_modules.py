@@ -178,8 +178,10 @@ def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
 
 # torch's kernel works on a row with one wavefront and does short rows as fast (128 rows of 768 in fp32: 4.0 us there, 3.6 here for two ranks at once), while
 # its call costs the host less: OPT-125m in fp32, 50 norms of 768 a forward, 5.6 ms eager with torch's and 6.1 with these. 16 rows of 8192 in
-# fp16 take 9.3 us there and 4.1 here.
+# fp16 take 9.3 us there and 4.1 here. In between, the host sets the pace of an eager forward with some hundred rows (the Falcon-40B-shaped layer on 150 of them: 890 us
+# with torch's norms, 950 with these), so torch's stay there; 1024 rows take 14.4 us there and 7.3 here.
 LAYER_NORM_ROW = 2048
+LAYER_NORM_FEW_ROWS, LAYER_NORM_MANY_ROWS = 64, 512
 
 _own_layer_norm, _functional_layer_norm = nn.LayerNorm.forward, nn.functional.layer_norm
 
@@ -193,6 +195,7 @@ class ShardLayerNorm(nn.LayerNorm):
         if (nn.LayerNorm.forward is not _own_layer_norm or nn.functional.layer_norm is not _functional_layer_norm or w is None or len(self.normalized_shape) != 1
                 or not _norm_kernel_takes(input, w) or torch.is_autocast_enabled()
                 or b is not None and (type(b) not in (torch.Tensor, nn.Parameter) or b.dtype != w.dtype or b.shape != w.shape or b.get_device() != w.get_device())
+                or LAYER_NORM_FEW_ROWS * w.numel() < input.numel() < LAYER_NORM_MANY_ROWS * w.numel()
                 or torch.is_grad_enabled() and (input.requires_grad or w.requires_grad or b is not None and b.requires_grad)):
             return super().forward(input)
         return together.layer_norm(input, w, b, self.eps)

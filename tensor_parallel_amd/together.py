@@ -228,7 +228,7 @@ def _gather(calls: List[tuple]) -> Sequence[torch.Tensor]:
 
 def linear_gathered(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], rank: int, world: int) -> Optional[torch.Tensor]:
     """The Linears of two ranks with their results side by side, a whole one for each, in one launch; None where this rank is on its own."""
-    if world != 2:
+    if world != 2 or x.numel() == 0:
         return None
     return _call(_not_together, _gather, (x, w, bias), (), (rank,))
 
@@ -251,8 +251,11 @@ def add_rms_norm(r: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float) 
     return _call(_native.add_rms_norm, _native.add_rms_norm_ranks, (r, x, w), (eps,))
 
 
+LAYER_NORM_TOGETHER_ROWS = 64  # more rows of two ranks take as long in one launch as in two
+
+
 def layer_norm(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], eps: float) -> torch.Tensor:
-    if x.numel() >= ALONE_ROWS * w.numel():
+    if x.numel() > LAYER_NORM_TOGETHER_ROWS * w.numel():
         return _native.layer_norm(x, w, b, eps)
     return _call(_native.layer_norm, _native.layer_norm_ranks, (x, w, b), (eps,))
 
