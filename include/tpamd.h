@@ -269,6 +269,13 @@ int tpamd_rope_append(const void *q_dev, const void *k_dev, const void *v_dev, c
                       void *q_out_dev, void *k_cache_dev, void *v_cache_dev, int64_t B, int64_t S, int64_t Hq, int64_t Hkv,
                       int64_t D, int64_t pos0, int64_t cache_len, const int64_t *strides, int dtype, void *stream);
 
+/* The rotary embedding of tpamd_rope_append without a cache (a wrapped attention module's forward on whole sequences, run by
+ * src/tensor_parallel/wrapper.py:69-72): q [B, S, Hq, D] -> q_out [B, Hq, S, D], k [B, S, Hkv, D] -> k_out [B, Hkv, S, D], the same bits.
+ *   strides: 14 element strides, {q batch, q position, q head, k batch, k position, k head, cos/sin batch (0 when shared), cos/sin position,
+ *   q_out batch, q_out head, q_out position, k_out batch, k_out head, k_out position}, multiples of 8; pointers 16-byte aligned; fewer than 2^24 blocks of 256 lanes, 16 bytes of each half of a head row a lane. */
+int tpamd_rope(const void *q_dev, const void *k_dev, const void *cos_dev, const void *sin_dev, void *q_out_dev, void *k_out_dev, int64_t B,
+               int64_t S, int64_t Hq, int64_t Hkv, int64_t D, const int64_t *strides, int dtype, void *stream);
+
 /* Decode step of the same call site with tpamd_rope_append and tpamd_attention in one: one new position per sequence
  * on a rank-local cache that holds pos0 positions (reference: the wrapped attention module's torch ops, as for the two
  * entry points above; src/tensor_parallel/wrapper.py:69-72, aux_actions.py:7-15, slicing_configs.py:430-461).

@@ -61,6 +61,7 @@ EXPORTS = (
     "tpamd_linear_sum_pays",
     "tpamd_linear_w8_sum_ranks",
     "tpamd_reduce_partials_copy",
+    "tpamd_rope",
 )
 
 ABI_VERSION = 6
@@ -161,6 +162,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_attention_decode_rope_devpos.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, vp, i64, c.POINTER(i64), c.c_float, ci, vp]
     lib.tpamd_rope_append.restype = ci
     lib.tpamd_rope_append.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, c.POINTER(i64), ci, vp]
+    lib.tpamd_rope.restype = ci
+    lib.tpamd_rope.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, c.POINTER(i64), ci, vp]
     lib.tpamd_rms_norm.restype = ci
     lib.tpamd_rms_norm.argtypes = [vp, vp, vp, i64, i64, i64, i64, c.c_float, ci, vp]
     lib.tpamd_add_rms_norm.restype = ci
@@ -947,6 +950,33 @@ def attention_decode_rope_ranks(calls: Sequence[tuple]) -> list:
         return [attention_decode_rope(*call) for call in calls]
     _check(rc, "tpamd_attention_decode_rope_ranks")
     return [out for _, _, out in keep]
+
+
+def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> tuple:
+    """Rotary embedding of whole sequences in one launch: q [B, S, Hq, D], k [B, S, Hkv, D] (views of projection outputs), cos / sin [B or 1, S, D];
+    returns them rotated, as [B, Hq, S, D] and [B, Hkv, S, D]. Arithmetic as in `rope_append`."""
+    require_device(q, "rope")
+    if not (q.dtype == k.dtype == cos.dtype == sin.dtype) or q.dtype not in (torch.bfloat16, torch.float16):
+        raise TypeError("rope: every tensor must share bfloat16 or float16")
+    B, S, Hq, D = q.shape
+    if k.dim() != 4 or k.shape[:2] != (B, S) or k.shape[3] != D or cos.shape != sin.shape or cos.dim() != 3 or cos.shape[0] not in (1, B) or cos.shape[1:] != (S, D):
+        raise ValueError(f"rope: shapes q {tuple(q.shape)}, k {tuple(k.shape)}, cos {tuple(cos.shape)}, sin {tuple(sin.shape)} do not fit")
+    for name, t in (("q", q), ("k", k), ("cos", cos), ("sin", sin)):
+        if t.device != q.device or t.stride(-1) != 1:
+            raise ValueError(f"rope: {name} must have contiguous rows on {q.device}")
+    if sin.stride() != cos.stride():
+        sin, cos = sin.contiguous(), cos.contiguous()
+    Hkv = k.shape[2]
+    q_out = torch.empty((B, Hq, S, D), dtype=q.dtype, device=q.device)
+    k_out = torch.empty((B, Hkv, S, D), dtype=q.dtype, device=q.device)
+    strides = (ctypes.c_int64 * 14)(*q.stride()[:3], *k.stride()[:3], cos.stride(0) if cos.shape[0] > 1 else 0, cos.stride(1), *q_out.stride()[:3], *k_out.stride()[:3])
+    with _on_device(q.device):
+        _check(
+            lib().tpamd_rope(q.data_ptr(), k.data_ptr(), cos.data_ptr(), sin.data_ptr(), q_out.data_ptr(), k_out.data_ptr(), B, S, Hq, Hkv, D, strides,
+                             dtype_code(q.dtype), ctypes.c_void_p(current_stream_ptr(q.device))),
+            "tpamd_rope",
+        )
+    return q_out, k_out
 
 
 def attention_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,

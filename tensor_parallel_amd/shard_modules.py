@@ -192,10 +192,11 @@ class ShardLayerNorm(nn.LayerNorm):
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:  # noqa: A002
         w, b = self.weight, self.bias
-        if (nn.LayerNorm.forward is not _own_layer_norm or nn.functional.layer_norm is not _functional_layer_norm or w is None or len(self.normalized_shape) != 1
+        if w is None or LAYER_NORM_FEW_ROWS * w.numel() < input.numel() < LAYER_NORM_MANY_ROWS * w.numel():
+            return super().forward(input)
+        if (nn.LayerNorm.forward is not _own_layer_norm or nn.functional.layer_norm is not _functional_layer_norm or len(self.normalized_shape) != 1
                 or not _norm_kernel_takes(input, w) or torch.is_autocast_enabled()
                 or b is not None and (type(b) not in (torch.Tensor, nn.Parameter) or b.dtype != w.dtype or b.shape != w.shape or b.get_device() != w.get_device())
-                or LAYER_NORM_FEW_ROWS * w.numel() < input.numel() < LAYER_NORM_MANY_ROWS * w.numel()
                 or torch.is_grad_enabled() and (input.requires_grad or w.requires_grad or b is not None and b.requires_grad)):
             return super().forward(input)
         return together.layer_norm(input, w, b, self.eps)
@@ -232,6 +233,51 @@ def _llama_layer_forward(self, hidden_states: torch.Tensor, *args, **kwargs) -> 
     return total + self.mlp(normed)
 
 
+def is_llama_attention(module: nn.Module) -> bool:
+    """transformers' LlamaAttention as the fused forward below knows it."""
+    return type(module).__name__ == "LlamaAttention" and "forward" not in module.__dict__ and _takes_stand_in(type(module), _llama_attention_forward)
+
+
+_ROTARY = {"apply_rotary_pos_emb": (("unsqueeze", "rotate_half"), ("q", "k", "cos", "sin", "unsqueeze_dim", "q_embed", "k_embed")),
+           "rotate_half": (("shape", "torch", "cat"), ("x", "x1", "x2"))}
+
+
+def _llama_attention_forward(self, hidden_states: torch.Tensor, position_embeddings=None, attention_mask=None, past_key_values=None, **kwargs):
+    """The module's own forward on whole sequences without a cache or a mask, on the attention kernel (attention.py), with the rotary embedding as one launch
+    (`tpamd_rope`). Everything else goes to the module's own."""
+    from .attention import IMPLEMENTATION_NAME, attention_forward
+
+    own = self._tp_base.forward
+    if (own is not self._tp_replaced or past_key_values is not None or attention_mask is not None or type(position_embeddings) is not tuple or len(position_embeddings) != 2
+            or self.training or torch.is_grad_enabled() or self.config._attn_implementation != IMPLEMENTATION_NAME or self.head_dim not in (64, 128)
+            or kwargs.get("output_attentions") or "is_causal" in kwargs or hidden_states.dim() != 3 or hidden_states.dtype not in (torch.bfloat16, torch.float16)
+            or not _native.plain_call(hidden_states, *position_embeddings) or not _native.on_hip(hidden_states)):
+        return own(self, hidden_states, position_embeddings=position_embeddings, attention_mask=attention_mask, past_key_values=past_key_values, **kwargs)
+    names = _globals_of(own)
+    cos, sin = position_embeddings
+    # the functions that the module's own forward would look up, as they were when the class was made
+    if (any(names.get(name) is not function for name, function in self._tp_looked_up.items())
+            or names["ALL_ATTENTION_FUNCTIONS"].get_interface(IMPLEMENTATION_NAME, None) is not attention_forward
+            or cos.dtype != hidden_states.dtype or sin.dtype != cos.dtype or cos.dim() != 3 or cos.shape != sin.shape or cos.get_device() != hidden_states.get_device()
+            or cos.shape[0] not in (1, hidden_states.shape[0]) or cos.shape[1:] != (hidden_states.shape[1], self.head_dim) or cos.stride(2) != 1 or sin.stride(2) != 1):
+        return own(self, hidden_states, position_embeddings=position_embeddings, attention_mask=attention_mask, past_key_values=past_key_values, **kwargs)
+    heads = (*hidden_states.shape[:2], -1, self.head_dim)
+    q, k, v = self.q_proj(hidden_states).view(heads), self.k_proj(hidden_states).view(heads), self.v_proj(hidden_states).view(heads)
+    if type(q) is torch.Tensor and type(k) is torch.Tensor and q.dtype == k.dtype == cos.dtype and not (q.data_ptr() % 16 or k.data_ptr() % 16 or cos.data_ptr() % 16 or sin.data_ptr() % 16) \
+            and not any(stride % 8 for t in (q, k, cos, sin) for stride in t.stride()[:-1]) and q.numel() + k.numel() < 1 << 32:
+        q, k = _native.rope(q, k, cos, sin)
+    else:
+        q, k = names["apply_rotary_pos_emb"](q.transpose(1, 2), k.transpose(1, 2), cos, sin)
+    out, weights = attention_forward(self, q, k, v.transpose(1, 2), None, dropout=0.0, scaling=self.scaling, **kwargs)
+    return self.o_proj(out.reshape(*hidden_states.shape[:2], -1)), weights
+
+
+def _globals_of(function) -> dict:
+    while hasattr(function, "__wrapped__"):
+        function = function.__wrapped__
+    return function.__globals__
+
+
 def is_rotary_tables(module: nn.Module) -> bool:
     """The rotary embedding modules of transformers' Llama and Falcon: cos / sin of position * inv_freq, the halves repeated."""
     return type(module).__name__ in ("LlamaRotaryEmbedding", "FalconRotaryEmbedding") and _takes_stand_in(type(module), _rotary_tables_forward) and \
@@ -256,6 +302,11 @@ _STOOD_IN_FOR = {
                         ("self", "hidden_states", "input_dtype", "variance")),
     _llama_layer_forward: (("input_layernorm", "self_attn", "post_attention_layernorm", "mlp"),
                            ("self", "hidden_states", *_LAYER_DEFAULTS, "kwargs", "residual", "_")),
+    _llama_attention_forward: (("shape", "head_dim", "q_proj", "view", "transpose", "k_proj", "v_proj", "apply_rotary_pos_emb", "update", "layer_idx", "ALL_ATTENTION_FUNCTIONS",
+                                "get_interface", "config", "_attn_implementation", "eager_attention_forward", "training", "attention_dropout", "scaling", "reshape",
+                                "contiguous", "o_proj"),
+                               ("self", "hidden_states", "position_embeddings", "attention_mask", "past_key_values", "kwargs", "input_shape", "hidden_shape", "query_states",
+                                "key_states", "value_states", "cos", "sin", "attention_interface", "attn_output", "attn_weights")),
     _rotary_tables_forward: (("inv_freq", "expand", "shape", "to", "torch", "float", "device", "isinstance", "type", "str", "maybe_autocast", "transpose",
                               "cat", "cos", "attention_scaling", "sin", "dtype"),
                              ("self", "x", "position_ids", "inv_freq_expanded", "position_ids_expanded", "device_type", "freqs", "emb", "cos", "sin")),
@@ -272,8 +323,8 @@ _fused_classes: dict = {}
 
 def _fused_class(base: type, forward, doc: str) -> type:
     """Subclass of a module's own class with another forward (isinstance checks keep working, and so does pickling). `_tp_replaced` is the
-    forward it stands in for; once the class has another (None: it had when the subclass was made), that one runs. A decoder layer's
-    class keeps its name, which programs look such layers up by; the others are named as `ShardLinear` is."""
+    forward it stands in for; once the class has another (None: it had when the subclass was made), that one runs. The classes of a decoder layer and its
+    attention keep their names, which programs look such modules up by; the others are named as `ShardLinear` is."""
     cls = _fused_classes.get((base, forward))
     if cls is None:
         def reduce_ex(self, protocol):  # the class is made here and has no name to be found by: pickle what makes it
@@ -284,9 +335,13 @@ def _fused_class(base: type, forward, doc: str) -> type:
             own.__dict__.update(self.__dict__)
             return own
 
-        name = base.__name__ if forward is _llama_layer_forward else "Shard" + base.__name__
+        name = base.__name__ if forward in (_llama_layer_forward, _llama_attention_forward) else "Shard" + base.__name__
         cls = type(name, (base,), {"forward": forward, "__doc__": doc, "__reduce_ex__": reduce_ex, "__prepare_scriptable__": prepare_scriptable, "_tp_base": base,
                                 "_tp_replaced": staticmethod(base.forward if _takes_stand_in(base, forward) else None)})
+        if forward is _llama_attention_forward:  # None in the place of one that is not transformers' own
+            names = _globals_of(base.forward)
+            cls._tp_looked_up = {name: names.get(name) if _native.stock_function(names.get(name), base.__module__, name, *known) else None
+                                 for name, known in _ROTARY.items()}
         cls = _fused_classes.setdefault((base, forward), cls)
     return cls
 
@@ -363,6 +418,8 @@ def install_shard_kernels(shard: nn.Module) -> None:
             module.__class__ = _fused_class(type(module), _rms_norm_forward, "The base class with its forward as one launch (`tpamd_rms_norm`).")
         elif is_llama_layer(module):
             module.__class__ = _fused_class(type(module), _llama_layer_forward, "The base class with an addition and a norm as one launch (`tpamd_add_rms_norm`).")
+        elif is_llama_attention(module):
+            module.__class__ = _fused_class(type(module), _llama_attention_forward, "The base class with the rotary embedding of a forward without a cache as one launch (`tpamd_rope`).")
         elif is_rotary_tables(module):
             module.__class__ = _fused_class(type(module), _rotary_tables_forward, "The base class with its forward as one launch (`tpamd_rope_tables`).")
     for module in shard.modules():

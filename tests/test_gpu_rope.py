@@ -172,3 +172,51 @@ def test_tables_of_more_elements_than_one_launch_takes():
     for b in (0, B // 2, B - 2, B - 1):
         c, s = _native.rope_tables(freq, positions[b:b + 1], 1.0, torch.bfloat16)
         assert torch.equal(cos[b], c[0]) and torch.equal(sin[b], s[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,S,Hq,Hkv,D,shared", [(1, 1, 1, 1, 64, True), (2, 5, 8, 2, 64, False), (3, 129, 16, 16, 128, True), (1, 700, 16, 4, 128, False), (2, 3, 40, 40, 128, True)])
+def test_rope_of_whole_sequences_is_transformers(B, S, Hq, Hkv, D, shared, dtype):
+    from transformers.models.llama.modeling_llama import apply_rotary_pos_emb
+
+    g = torch.Generator(device="cuda").manual_seed(S)
+    qkv = torch.randn(B, S, Hq + 2 * Hkv, D, device="cuda", generator=g).to(dtype)
+    q, k = qkv[:, :, :Hq], qkv[:, :, Hq:Hq + Hkv]
+    cos, sin = (torch.randn(1 if shared else B, S, D, device="cuda", generator=g).to(dtype) for _ in range(2))
+    got = _native.rope(q, k, cos, sin)
+    want = apply_rotary_pos_emb(q.transpose(1, 2), k.transpose(1, 2), cos, sin)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_llama_attention_without_a_cache_is_the_modules_own(monkeypatch):
+    import transformers.models.llama.modeling_llama as llama
+    from transformers import LlamaConfig, LlamaForCausalLM
+
+    import tensor_parallel_amd as tp
+
+    cfg = LlamaConfig(vocab_size=128, hidden_size=256, intermediate_size=512, num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2, head_dim=64,
+                      attn_implementation="eager")
+    torch.manual_seed(0)
+    model = LlamaForCausalLM(cfg).bfloat16().eval().cuda()
+    model.config._attn_implementation = tp.attention.register()
+    split = tp.tensor_parallel(model, ["cuda:0"] * 2)
+    ids = torch.randint(0, 128, (3, 37), device="cuda")
+    calls = []
+    rope = _native.rope
+    monkeypatch.setattr(_native, "rope", lambda *a: calls.append(1) or rope(*a))
+    with torch.no_grad():
+        split(input_ids=ids[:, :5], use_cache=False)
+        calls.clear()
+        got = split(input_ids=ids, use_cache=False).logits
+        assert len(calls) == 4  # two layers, two ranks
+        with monkeypatch.context() as m:  # a program's own rotary embedding runs, and so does a replaced forward
+            seen = []
+            stock = llama.apply_rotary_pos_emb
+            m.setattr(llama, "apply_rotary_pos_emb", lambda *a, **k: seen.append(1) or stock(*a, **k))
+            own = split(input_ids=ids, use_cache=False).logits
+            assert len(seen) == 4 and len(calls) == 4
+        assert torch.equal(got, own)
+        with monkeypatch.context() as m:
+            forward = llama.LlamaAttention.forward
+            m.setattr(llama.LlamaAttention, "forward", lambda self, *a, **k: seen.append(2) or forward(self, *a, **k))
+            assert torch.equal(split(input_ids=ids, use_cache=False).logits, own) and seen[-4:] == [2] * 4 and len(calls) == 4
