@@ -367,6 +367,15 @@ int tpamd_add_rms_norm_ranks(int n, const void *const *x_dev, const void *const 
 int tpamd_layer_norm_ranks(int n, const void *const *x_dev, const void *const *w_dev, const void *const *b_dev, void *const *y_dev, int64_t rows,
                            int64_t D, int64_t ldx, int64_t ldy, float eps, int dtype, void *stream);
 
+int tpamd_rope_tables_ranks(int n, const void *const *inv_freq_dev, int freq_dtype, const void *const *pos_dev, int64_t pos_b, int64_t pos_s,
+                            int64_t B, int64_t S, int64_t half, float scaling, void *const *cos_dev, void *const *sin_dev, int dtype, void *stream);
+int tpamd_causal_mask_ranks(int n, const void *const *q_offset_dev, int64_t kv_offset, int64_t rows, int64_t cols, void *const *mask_dev,
+                            void *stream);
+/* out[r] = a[r] + b[r], rounded, element for element; pointers 16-byte aligned, fewer than 2^33 elements. */
+int tpamd_add_ranks(int n, const void *const *a_dev, const void *const *b_dev, void *const *out_dev, int64_t elements, int dtype, void *stream);
+/* *counts[r] += by, int64 on the device. */
+int tpamd_advance_ranks(int n, void *const *counts_dev, int64_t by, void *stream);
+
 typedef struct {
     const void *q, *k, *v, *cos, *sin;
     void *k_cache, *v_cache, *out;

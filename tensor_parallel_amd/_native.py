@@ -62,6 +62,10 @@ EXPORTS = (
     "tpamd_linear_w8_sum_ranks",
     "tpamd_reduce_partials_copy",
     "tpamd_rope",
+    "tpamd_rope_tables_ranks",
+    "tpamd_causal_mask_ranks",
+    "tpamd_add_ranks",
+    "tpamd_advance_ranks",
 )
 
 ABI_VERSION = 6
@@ -179,6 +183,14 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tpamd_linear_gather_ranks.argtypes = lib.tpamd_linear_ranks.argtypes
     lib.tpamd_linear_add_copy.restype = ci
     lib.tpamd_linear_add_copy.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, ci, ci, vp]
+    lib.tpamd_rope_tables_ranks.restype = ci
+    lib.tpamd_rope_tables_ranks.argtypes = [ci, pp, ci, pp, i64, i64, i64, i64, i64, c.c_float, pp, pp, ci, vp]
+    lib.tpamd_causal_mask_ranks.restype = ci
+    lib.tpamd_causal_mask_ranks.argtypes = [ci, pp, i64, i64, i64, pp, vp]
+    lib.tpamd_add_ranks.restype = ci
+    lib.tpamd_add_ranks.argtypes = [ci, pp, pp, pp, i64, ci, vp]
+    lib.tpamd_advance_ranks.restype = ci
+    lib.tpamd_advance_ranks.argtypes = [ci, pp, i64, vp]
     lib.tpamd_swiglu_up_ranks.restype = ci
     lib.tpamd_swiglu_up_ranks.argtypes = [ci, pp, pp, pp, pp, i64, i64, i64, i64, i64, i64, ci, vp]
     lib.tpamd_rms_norm_ranks.restype = ci
@@ -824,6 +836,60 @@ def causal_mask(q_offset: torch.Tensor, kv_offset: int, q_length: int, kv_length
             "tpamd_causal_mask",
         )
     return out
+
+
+def rope_tables_ranks(calls: Sequence[tuple]) -> list:
+    """`rope_tables(inv_freq, position_ids, scaling, dtype)` for the operands of several ranks (with one scaling and dtype)."""
+    inv_freq, position_ids, scaling, dtype = calls[0]
+    require_device(position_ids, "rope_tables")
+    if inv_freq.dim() != 1 or position_ids.dim() != 2 or position_ids.dtype != torch.int64 or inv_freq.device != position_ids.device:
+        raise ValueError(f"rope_tables: inv_freq {tuple(inv_freq.shape)} and int64 position_ids [B, S] on one device are needed, got "
+                         f"{tuple(position_ids.shape)} {position_ids.dtype}")
+    B, S = position_ids.shape
+    half = inv_freq.shape[0]
+    cos = [torch.empty((B, S, 2 * half), dtype=dtype, device=position_ids.device) for _ in calls]
+    sin = [torch.empty_like(c) for c in cos]
+    n, table = len(calls), lib().tpamd_rope_tables_ranks
+    code, pos_b, pos_s = dtype_code(inv_freq.dtype), position_ids.stride(0), position_ids.stride(1)
+    _run("tpamd_rope_tables", lambda f, p, c, s, stream: table(n, f, code, p, pos_b, pos_s, B, S, half, float(scaling), c, s, dtype_code(dtype), stream),
+         position_ids.get_device(), [_contiguous([c[0] for c in calls]), [c[1] for c in calls], cos, sin])
+    return list(zip(cos, sin))
+
+
+def causal_mask_ranks(calls: Sequence[tuple]) -> list:
+    """`causal_mask(q_offset, kv_offset, q_length, kv_length)` for the offsets of several ranks (with the same numbers)."""
+    q_offset, kv_offset, q_length, kv_length = calls[0]
+    require_device(q_offset, "causal_mask")
+    if q_offset.dtype != torch.int64 or q_offset.numel() != 1:
+        raise ValueError(f"causal_mask: q_offset must be one int64, got {tuple(q_offset.shape)} {q_offset.dtype}")
+    masks = [torch.empty((1, 1, q_length, kv_length), dtype=torch.bool, device=q_offset.device) for _ in calls]
+    n, mask = len(calls), lib().tpamd_causal_mask_ranks
+    _run("tpamd_causal_mask", lambda q, out, stream: mask(n, q, kv_offset, q_length, kv_length, out, stream), q_offset.get_device(), [[c[0] for c in calls], masks])
+    return masks
+
+
+def add_ranks(calls: Sequence[tuple]) -> list:
+    """a + b of several ranks, tensors of one shape and dtype."""
+    a, b = calls[0]
+    if a.shape != b.shape or a.dtype != b.dtype or a.get_device() != b.get_device():
+        raise ValueError(f"add_ranks: {tuple(a.shape)} {a.dtype} and {tuple(b.shape)} {b.dtype} do not fit")
+    xs, rs = _contiguous([c[0] for c in calls]), _contiguous([c[1] for c in calls])
+    if any(t.data_ptr() % 16 for t in xs + rs):
+        return [x + r for x, r in calls]
+    outs = [torch.empty_like(x) for x in xs]
+    _run("tpamd_add_ranks", functools.partial(lib().tpamd_add_ranks, len(calls)), a.get_device(), [xs, rs, outs], a.numel(), dtype_code(a.dtype))
+    return outs
+
+
+def advance_ranks(calls: Sequence[tuple]) -> list:
+    """count.add_(by) for the int64 counts of several ranks."""
+    count, by = calls[0]
+    if count.dtype != torch.int64 or count.numel() != 1:
+        raise ValueError(f"advance_ranks: a count must be one int64, got {tuple(count.shape)} {count.dtype}")
+    if len({c.data_ptr() for c, _ in calls}) < len(calls):  # ranks that share a count: one after the other
+        return [c.add_(by) for c, by in calls]
+    _run("tpamd_advance_ranks", functools.partial(lib().tpamd_advance_ranks, len(calls)), count.get_device(), [[c[0] for c in calls]], by)
+    return [c[0] for c in calls]
 
 
 def rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,

@@ -72,7 +72,7 @@ def attention_mask_of(*args, **kwargs) -> Optional[torch.Tensor]:
             or not _native.stock_function(sdpa_mask, "transformers.masking_utils", "sdpa_mask", *_SDPA_MASK)
             or not _native.stock_function(causal_mask_function, "transformers.masking_utils", "causal_mask_function", *_CAUSAL)):
         return sdpa_mask(*args, **kwargs)
-    return _native.causal_mask(q_offset, kv_offset, q_length, kv_length).expand(kwargs["batch_size"], -1, q_length, kv_length)
+    return together.causal_mask(q_offset, kv_offset, q_length, kv_length).expand(kwargs["batch_size"], -1, q_length, kv_length)
 
 
 def register() -> str:
@@ -229,7 +229,7 @@ def _attend_on_cache(q, k, v, cos, sin, layer, static, scale, layer_idx: int) ->
                 raise ValueError(f"{pos0} cached + {S} new positions do not fit the static cache of {kb.shape[2]}")
             q_rot = _native.rope_append(q, k, v, cos, sin, kb, vb, pos0)
             out = _native.attention(q_rot, kb[:, :, :pos0 + S], vb[:, :, :pos0 + S], scale=scale, causal=True)
-        count.add_(S)
+        together.advance(count, S)
         return out.reshape(B, S, Hq, D)
     pos0 = layer.get_seq_length()
     kb, vb = _buffers_with_room(layer, B, Hkv, D, pos0 + S, k)

@@ -64,10 +64,17 @@ __global__ __launch_bounds__(256) void rope_append_kernel(RopeParams p) {
 
 // cos / sin tables of a forward: out[row][i] = out[row][i + half] = round(f(position[row] * inv_freq[i]) * scaling). One thread per
 // (row, frequency), latency-bound: the module's own forward is ten launches (two casts, a K = 1 matrix product, a
-// concatenation, and three passes for each table), 2 us each in a recorded decode step.
+// concatenation, and three passes for each table), 2 us each in a recorded decode step. blockIdx.y = 1: the tables of a second rank, byte distances in `to`.
+struct TableStep { int64_t freq, pos, cos, sin; };
 template <int DT>
 __global__ __launch_bounds__(256) void rope_tables_kernel(const char *inv_freq, int freq_dtype, const int64_t *pos, int64_t pos_b, int64_t pos_s, int S,
-                                                          int half, float scaling, char *cos_out, char *sin_out, int64_t first, int64_t n) {
+                                                          int half, float scaling, char *cos_out, char *sin_out, int64_t first, int64_t n, TableStep to) {
+    if (blockIdx.y != 0) {
+        inv_freq += to.freq;
+        pos = reinterpret_cast<const int64_t *>(reinterpret_cast<const char *>(pos) + to.pos);
+        cos_out += to.cos;
+        sin_out += to.sin;
+    }
     const int64_t e = first + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (e >= n) return;
     const int64_t row = e / half;
@@ -144,26 +151,44 @@ extern "C" int tpamd_rope_append(const void *q_dev, const void *k_dev, const voi
 
 extern "C" int tpamd_rope_tables(const void *inv_freq_dev, int freq_dtype, const int64_t *pos_dev, int64_t pos_b, int64_t pos_s, int64_t B, int64_t S,
                                  int64_t half, float scaling, void *cos_dev, void *sin_dev, int dtype, void *stream) {
+    const void *pos = pos_dev;
+    return tpamd_rope_tables_ranks(1, &inv_freq_dev, freq_dtype, &pos, pos_b, pos_s, B, S, half, scaling, &cos_dev, &sin_dev, dtype, stream);
+}
+
+extern "C" int tpamd_rope_tables_ranks(int n, const void *const *inv_freq_dev, int freq_dtype, const void *const *pos_dev, int64_t pos_b, int64_t pos_s, int64_t B,
+                                       int64_t S, int64_t half, float scaling, void *const *cos_dev, void *const *sin_dev, int dtype, void *stream) {
     const char *who = "tpamd_rope_tables";
+    TPAMD_REQUIRE(n >= 0 && inv_freq_dev && pos_dev && cos_dev && sin_dev, "%s: null pointer", who);
     TPAMD_REQUIRE((dtype == TPAMD_BF16 || dtype == TPAMD_F16 || dtype == TPAMD_F32) &&
                       (freq_dtype == TPAMD_BF16 || freq_dtype == TPAMD_F16 || freq_dtype == TPAMD_F32), "%s: unknown dtype", who);
     TPAMD_REQUIRE(B >= 0 && S >= 0 && half >= 0 && B < (1ll << 31) && S < (1ll << 31) && half < (1ll << 31), "%s: bad dimension", who);
     if (B == 0 || S == 0 || half == 0) return TPAMD_OK;
-    TPAMD_REQUIRE(inv_freq_dev && pos_dev && cos_dev && sin_dev, "%s: null pointer", who);
+    for (int i = 0; i < n; ++i) TPAMD_REQUIRE(inv_freq_dev[i] && pos_dev[i] && cos_dev[i] && sin_dev[i], "%s: null pointer", who);
     TPAMD_REQUIRE(B * S < (1ll << 31) && B * S * half < (1ll << 38), "%s: too many positions", who);
-    const int64_t n = B * S * half;
+    const int64_t elements = B * S * half;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const char *f = static_cast<const char *>(inv_freq_dev);
-    char *c = static_cast<char *>(cos_dev), *si = static_cast<char *>(sin_dev);
     const int Si = static_cast<int>(S), h = static_cast<int>(half);
     // a launch has at most 2^32 - 1 threads, and one that asks for more runs, without an error, what is left of the count modulo 2^32
-    constexpr int64_t PER_LAUNCH = 1ll << 31;
-    for (int64_t e = 0; e < n; e += PER_LAUNCH) {
-        const int64_t part = n - e < PER_LAUNCH ? n - e : PER_LAUNCH;
-        const dim3 grid(static_cast<unsigned>((part + 255) / 256));
-        if (dtype == TPAMD_BF16) hipLaunchKernelGGL(rope_tables_kernel<TPAMD_BF16>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, e, n);
-        else if (dtype == TPAMD_F16) hipLaunchKernelGGL(rope_tables_kernel<TPAMD_F16>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, e, n);
-        else hipLaunchKernelGGL(rope_tables_kernel<TPAMD_F32>, grid, dim3(256), 0, s, f, freq_dtype, pos_dev, pos_b, pos_s, Si, h, scaling, c, si, e, n);
+    constexpr int64_t PER_LAUNCH = 1ll << 30;  // of each of two ranks
+    for (int i = 0; i < n; i += 2) {
+        const unsigned ranks = i + 1 < n ? 2 : 1;
+        TableStep to{};
+        if (ranks == 2)
+            to = {bytes_from(inv_freq_dev[i], inv_freq_dev[i + 1]), bytes_from(pos_dev[i], pos_dev[i + 1]), bytes_from(cos_dev[i], cos_dev[i + 1]),
+                  bytes_from(sin_dev[i], sin_dev[i + 1])};
+        const char *f = static_cast<const char *>(inv_freq_dev[i]);
+        const int64_t *pos = static_cast<const int64_t *>(pos_dev[i]);
+        char *c = static_cast<char *>(cos_dev[i]), *si = static_cast<char *>(sin_dev[i]);
+        for (int64_t e = 0; e < elements; e += PER_LAUNCH) {
+            const int64_t part = elements - e < PER_LAUNCH ? elements - e : PER_LAUNCH;
+            const dim3 grid(static_cast<unsigned>((part + 255) / 256), ranks);
+            if (dtype == TPAMD_BF16)
+                hipLaunchKernelGGL(rope_tables_kernel<TPAMD_BF16>, grid, dim3(256), 0, s, f, freq_dtype, pos, pos_b, pos_s, Si, h, scaling, c, si, e, elements, to);
+            else if (dtype == TPAMD_F16)
+                hipLaunchKernelGGL(rope_tables_kernel<TPAMD_F16>, grid, dim3(256), 0, s, f, freq_dtype, pos, pos_b, pos_s, Si, h, scaling, c, si, e, elements, to);
+            else
+                hipLaunchKernelGGL(rope_tables_kernel<TPAMD_F32>, grid, dim3(256), 0, s, f, freq_dtype, pos, pos_b, pos_s, Si, h, scaling, c, si, e, elements, to);
+        }
     }
     TPAMD_HIP(hipGetLastError());
     return TPAMD_OK;

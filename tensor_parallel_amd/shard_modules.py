@@ -230,7 +230,8 @@ def _llama_layer_forward(self, hidden_states: torch.Tensor, *args, **kwargs) -> 
     else:
         total = hidden_states + attended
         normed = norm(total)
-    return total + self.mlp(normed)
+    out = self.mlp(normed)
+    return together.add(total, out) if type(out) is torch.Tensor else total + out
 
 
 def is_llama_attention(module: nn.Module) -> bool:
@@ -293,7 +294,7 @@ def _rotary_tables_forward(self, x: torch.Tensor, position_ids: torch.Tensor, **
             or not isinstance(kind, str) or "dynamic" in kind or kind == "longrope"
             or x.dtype not in _KERNEL_DTYPES or f.dtype not in _KERNEL_DTYPES):
         return own(self, x, position_ids, **kwargs)
-    return _native.rope_tables(f, position_ids, self.attention_scaling, x.dtype)
+    return together.rope_tables(f, position_ids, self.attention_scaling, x.dtype)
 
 
 # What each fused forward stands in for: the names its own forward looks up, and that one's arguments and locals.

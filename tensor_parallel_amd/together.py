@@ -265,3 +265,30 @@ def attention_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos
     if isinstance(pos0, torch.Tensor):
         return _call(_native.attention_decode_rope, _native.attention_decode_rope_ranks, (q, k, v, cos, sin, k_cache, v_cache, pos0), (scale,))
     return _call(_native.attention_decode_rope, _native.attention_decode_rope_ranks, (q, k, v, cos, sin, k_cache, v_cache), (pos0, scale))
+
+
+def rope_tables(inv_freq: torch.Tensor, position_ids: torch.Tensor, scaling: float, dtype: torch.dtype) -> tuple:
+    return _call(_native.rope_tables, _native.rope_tables_ranks, (inv_freq, position_ids), (scaling, dtype))
+
+
+def causal_mask(q_offset: torch.Tensor, kv_offset: int, q_length: int, kv_length: int) -> torch.Tensor:
+    return _call(_native.causal_mask, _native.causal_mask_ranks, (q_offset,), (kv_offset, q_length, kv_length))
+
+
+# An addition of more rows takes as long in one launch as in two, and where the host sets the pace torch's own calls are the cheaper ones.
+ADD_TOGETHER_ROWS = 64
+
+
+def add(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """a + b; in one launch for ranks that come with a few rows of the same forms."""
+    if (a.numel() > ADD_TOGETHER_ROWS * a.shape[-1] or a.dtype is not b.dtype or a.shape != b.shape or a.get_device() != b.get_device()
+            or not (a.is_contiguous() and b.is_contiguous()) or not _native.plain_call(a, b)):
+        return a + b
+    return _call(torch.add, _native.add_ranks, (a, b))
+
+
+def advance(count: torch.Tensor, by: int) -> torch.Tensor:
+    """count.add_(by)."""
+    if count.dtype is not torch.int64 or count.numel() != 1:
+        return count.add_(by)
+    return _call(torch.Tensor.add_, _native.advance_ranks, (count,), (by,))

@@ -268,3 +268,20 @@ def test_the_sum_of_two_ranks_int8_linears(rows, cols, K, n_out):
     want = parts[0].float() + parts[1].float()  # both rounded products, each of which may be rounded the other way where the planes are cut elsewhere
     bound = 2.0 ** -11 * (want.abs() + 2 * (parts[0].float().abs() + parts[1].float().abs())) + 1e-6
     assert bool(((sums[0].float() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape,n", [((1, 1), 2), ((3, 7), 3), ((1, 4096), 2), ((5, 257), 2), ((40, 4096), 2)])
+def test_small_calls_of_several_ranks(shape, n, dtype):
+    a, b = draws(n, *shape, dtype=dtype), draws(n, *shape, dtype=dtype, seed=1)
+    assert all(torch.equal(c, x + y) for x, y, c in zip(a, b, _native.add_ranks(list(zip(a, b)))))
+    counts = [torch.tensor(10 + r, device=DEV) for r in range(n)]
+    assert all(x is y for x, y in zip(_native.advance_ranks([(c, 3) for c in counts]), counts)) and [int(c) for c in counts] == [13 + r for r in range(n)]
+    rows, cols = shape
+    offsets = [torch.tensor([cols // 2 + r], device=DEV) for r in range(n)]
+    for offset, mask in zip(offsets, _native.causal_mask_ranks([(o, 1, rows, cols) for o in offsets])):
+        assert torch.equal(mask, _native.causal_mask(offset, 1, rows, cols))
+        assert torch.equal(mask[0, 0], torch.arange(cols, device=DEV)[None] + 1 <= offset + torch.arange(rows, device=DEV)[:, None])
+    freqs, positions = draws(n, 32, dtype=torch.float32, seed=2), [torch.arange(rows * 3, device=DEV).view(rows, 3) + 7 * r for r in range(n)]
+    for f, p, got in zip(freqs, positions, _native.rope_tables_ranks([(f, p, 1.5, dtype) for f, p in zip(freqs, positions)])):
+        assert all(torch.equal(x, y) for x, y in zip(got, _native.rope_tables(f, p, 1.5, dtype)))
