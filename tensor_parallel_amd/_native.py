@@ -1092,7 +1092,7 @@ def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale_: torch.Tensor, outlier_i
     """Weight-only int8 Linear with outlier columns kept in the activation dtype. `addend` and `copy` as in `linear`."""
     x2, wq, scale_, outlier_idx, w_out, b = _w8_operands(x, wq, scale_, outlier_idx, w_out, bias)
     (M, K), N = x2.shape, wq.shape[0]
-    n_out = 0 if outlier_idx is None else int(outlier_idx.numel())
+    n_out = 0 if outlier_idx is None else outlier_idx.numel()
     if addend is not None and (addend.dtype != x.dtype or addend.device != x.device or addend.numel() != M * N or addend.shape[-1] != N):
         raise ValueError("linear_w8: addend must have the shape, dtype and device of the result")
     if copy is not None and (addend is None or copy.dtype != x.dtype or copy.device != x.device or copy.numel() != M * N or not copy.is_contiguous()):
@@ -1131,9 +1131,11 @@ def _w8_operands(x, wq, scale_, outlier_idx, w_out, bias) -> tuple:
     N = wq.shape[0]
     if scale_.shape != (N,):
         raise ValueError(f"linear_w8: scale must have shape [{N}], got {tuple(scale_.shape)}")
-    for name, t in (("wq", wq), ("scale", scale_), ("outlier_idx", outlier_idx), ("w_out", w_out), ("bias", bias)):
-        if t is not None and t.device != x.device:
-            raise ValueError(f"linear_w8: x is on {x.device}, {name} on {t.device}")
+    index = x.get_device()
+    if index < 0 or wq.get_device() != index or scale_.get_device() != index or any(t is not None and t.get_device() != index for t in (outlier_idx, w_out, bias)):
+        for name, t in (("wq", wq), ("scale", scale_), ("outlier_idx", outlier_idx), ("w_out", w_out), ("bias", bias)):
+            if t is not None and t.device != x.device:
+                raise ValueError(f"linear_w8: x is on {x.device}, {name} on {t.device}")
     if bias is not None and (bias.shape != (N,) or bias.dtype != x.dtype):
         raise ValueError("linear_w8: bias must have shape [N] and the dtype of x")
     wq = wq.contiguous()

@@ -16,6 +16,7 @@ weights of the original model from the shards, refuses a model that holds one; i
 """
 from __future__ import annotations
 
+import functools
 from typing import Callable, Mapping, Optional, Sequence, Tuple, Union
 
 import torch
@@ -91,10 +92,13 @@ class ShardLinearW8(nn.Module):
     def forward(self, input: torch.Tensor) -> torch.Tensor:  # noqa: A002
         if input.dtype != self.dtype:
             raise TypeError(f"ShardLinearW8: the input is {input.dtype}, the Linear was quantised for {self.dtype}")
-        n_out = self.outlier_idx.numel()
-        operands = (input.detach(), self.wq, self.scale, self.outlier_idx if n_out else None, self.w_out if n_out else None, self.bias)
-        return product_in_context(self, input, self.out_features, (input,), lambda: together.linear_w8(*operands),
-                                  lambda **more: _native.linear_w8(*operands, **more), lambda rank: together.linear_w8_sum(*operands, rank))
+        idx = self.outlier_idx
+        n_out = idx.numel()
+        operands = (input.detach(), self.wq, self.scale, idx if n_out else None, self.w_out if n_out else None, self.bias)
+        few = input.numel() <= together.W8_TOGETHER_ROWS * input.shape[-1]
+        alone = functools.partial(_native.linear_w8, *operands)
+        return product_in_context(self, input, self.out_features, (input,), functools.partial(together.linear_w8, *operands) if few else alone, alone,
+                                  (lambda rank: together.linear_w8_sum(*operands, rank)) if few else None)
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "

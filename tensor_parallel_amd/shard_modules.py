@@ -54,7 +54,7 @@ def linear_in_context(module: nn.Module, x: torch.Tensor, w: torch.Tensor, bias)
 def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs: tuple, with_peers, alone, summed) -> torch.Tensor:
     """A shard's Linear with `columns` outputs, made by with_peers() or, with an addend, alone(addend=, copy=). Inside a wrapped module whose output goes to a
     "sum" rule (collectives.SumContext) the Linear that was seen to produce that output hands over the sum: two ranks that meet in it get it from
-    summed(rank) (`tpamd_linear_sum_ranks`), else the rank that comes last adds the partial sums already waiting in
+    summed(rank) (`tpamd_linear_sum_ranks`; None: not to be had), else the rank that comes last adds the partial sums already waiting in
     the reduction, in its epilogue (`tpamd_linear_add`): the product rounded to the dtype, then one rounded add, which
     is the same arithmetic as the reduction kernel's step."""
     from .collectives import current_sum_context
@@ -70,7 +70,7 @@ def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs:
             raise RuntimeError("tensor_parallel_amd: the Linear that feeds a \"sum\" rule ran twice in one call of its module "
                                "after adding the waiting partial sums; set TPAMD_FUSE_SUM=0")
         waiting = ctx.op.addend_for(ctx.rank)
-        if waiting is None and ctx.op.world_size == 2 and _sum_unwatched(module, ctx.owner):
+        if waiting is None and summed is not None and ctx.op.world_size == 2 and _sum_unwatched(module, ctx.owner):
             out = summed(ctx.rank)
         if out is not None:
             out = _guard(out, *inputs)

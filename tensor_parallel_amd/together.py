@@ -200,8 +200,6 @@ W8_TOGETHER_ROWS = 64
 
 def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, outlier_idx: Optional[torch.Tensor], w_out: Optional[torch.Tensor],
               bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    if x.numel() > W8_TOGETHER_ROWS * x.shape[-1]:
-        return _native.linear_w8(x, wq, scale, outlier_idx, w_out, bias)
     return _call(_native.linear_w8, _native.linear_w8_ranks, (x, wq, scale, outlier_idx, w_out, bias))
 
 
@@ -217,8 +215,6 @@ def _linear_w8_sum(calls: List[tuple]) -> Sequence[torch.Tensor]:
 
 def linear_w8_sum(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, outlier_idx: Optional[torch.Tensor], w_out: Optional[torch.Tensor],
                   bias: Optional[torch.Tensor], rank: int) -> Optional[torch.Tensor]:
-    if x.numel() > W8_TOGETHER_ROWS * x.shape[-1]:
-        return None
     return _call(_not_together, _linear_w8_sum, (x, wq, scale, outlier_idx, w_out, bias), (), (rank,))
 
 
