@@ -1153,7 +1153,7 @@ def _w8_operands(x, wq, scale_, outlier_idx, w_out, bias) -> tuple:
 def _w8_ranks(calls: Sequence[tuple]) -> tuple:
     ranks, keep = (W8Rank * len(calls))(), []
     for rank, call in zip(ranks, calls):
-        ops = _w8_operands(*call)
+        ops = _w8_operands(*call[:6])
         x2, wq = ops[:2]
         (M, K), N = x2.shape, wq.shape[0]
         y = torch.empty((M, N), dtype=x2.dtype, device=x2.device)
@@ -1165,11 +1165,11 @@ def _w8_ranks(calls: Sequence[tuple]) -> tuple:
 
 
 def linear_w8_ranks(calls: Sequence[tuple]) -> list:
-    """`linear_w8(x, wq, scale, outlier_idx, w_out, bias)` for the operands of several ranks."""
-    x = calls[0][0]
+    """`linear_w8(x, wq, scale, outlier_idx, w_out, bias, act)` for the operands of several ranks."""
+    x, act = calls[0][0], calls[0][6] if len(calls[0]) > 6 else ACT_NONE
     with _on_device(x.device):
         ranks, keep, dims = _w8_ranks(calls)
-        _check(lib().tpamd_linear_w8_ranks(len(calls), ranks, *dims, ACT_NONE, ctypes.c_void_p(current_stream_ptr(x.device))), "tpamd_linear_w8_ranks")
+        _check(lib().tpamd_linear_w8_ranks(len(calls), ranks, *dims, act, ctypes.c_void_p(current_stream_ptr(x.device))), "tpamd_linear_w8_ranks")
     return [y.view(*x.shape[:-1], y.shape[1]) for _, y in keep]
 
 

@@ -90,15 +90,18 @@ class ShardLinearW8(nn.Module):
         return cls(wq, scale, idx, w_out, bias, weight.dtype)
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:  # noqa: A002
+        return self._product(input, _native.ACT_NONE)
+
+    def _product(self, input: torch.Tensor, act: int) -> torch.Tensor:  # noqa: A002
         if input.dtype != self.dtype:
             raise TypeError(f"ShardLinearW8: the input is {input.dtype}, the Linear was quantised for {self.dtype}")
         idx = self.outlier_idx
         n_out = idx.numel()
         operands = (input.detach(), self.wq, self.scale, idx if n_out else None, self.w_out if n_out else None, self.bias)
         few = input.numel() <= together.W8_TOGETHER_ROWS * input.shape[-1]
-        alone = functools.partial(_native.linear_w8, *operands)
-        return product_in_context(self, input, self.out_features, (input,), functools.partial(together.linear_w8, *operands) if few else alone, alone,
-                                  (lambda rank: together.linear_w8_sum(*operands, rank)) if few else None)
+        alone = functools.partial(_native.linear_w8, *operands, act=act)
+        return product_in_context(self, input, self.out_features, (input,), functools.partial(together.linear_w8, *operands, act) if few else alone, alone,
+                                  (lambda rank: together.linear_w8_sum(*operands, rank)) if few and act == _native.ACT_NONE else None)
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "

@@ -279,6 +279,36 @@ def _globals_of(function) -> dict:
     return function.__globals__
 
 
+def is_falcon_mlp(module: nn.Module) -> bool:
+    return type(module).__name__ == "FalconMLP" and "forward" not in module.__dict__ and _takes_stand_in(type(module), _falcon_mlp_forward)
+
+
+_own_gelu, _functional_gelu = nn.GELU.forward, nn.functional.gelu
+
+
+def _is_erf_gelu(act) -> bool:
+    """Whether this module is the GELU of the error function, torch's or transformers', and nothing else."""
+    if act is None or "forward" in act.__dict__ or nn.functional.gelu is not _functional_gelu:
+        return False
+    if type(act) is nn.GELU:
+        return act.approximate == "none" and nn.GELU.forward is _own_gelu
+    return type(act).__name__ == "GELUActivation" and act.__dict__.get("act") is _functional_gelu and \
+        _native.stock_function(type(act).forward, "transformers.activations", "GELUActivation.forward", ("act",), ("self", "input"))
+
+
+def _falcon_mlp_forward(self, x: torch.Tensor) -> torch.Tensor:
+    """The module's own forward on a few rows with the activation in the epilogue of an int8 Linear before it, on the sum in 32 bits: a recorded step of 16 rows through a
+    Falcon-40B-shaped layer 287 -> 281 us. Over many rows the error functions at the end of each tile take longer than torch's pass over memory (1024 rows 1490 -> 1515 us)."""
+    from .int8 import ShardLinearW8
+
+    own, up, act, hooks = self._tp_base.forward, self._modules.get("dense_h_to_4h"), self._modules.get("act"), torch.nn.modules.module
+    if (x.dim() == 0 or x.numel() > together.W8_TOGETHER_ROWS * x.shape[-1] or own is not self._tp_replaced or type(up) is not ShardLinearW8 or "forward" in up.__dict__ or not _is_erf_gelu(act)
+            or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _has_hooks(up) or _has_hooks(act) or not _native.plain_call(x)
+            or torch.is_grad_enabled() and x.requires_grad):
+        return own(self, x)
+    return self.dense_4h_to_h(up._product(x, _native.ACT_GELU))
+
+
 def is_rotary_tables(module: nn.Module) -> bool:
     """The rotary embedding modules of transformers' Llama and Falcon: cos / sin of position * inv_freq, the halves repeated."""
     return type(module).__name__ in ("LlamaRotaryEmbedding", "FalconRotaryEmbedding") and _takes_stand_in(type(module), _rotary_tables_forward) and \
@@ -308,6 +338,7 @@ _STOOD_IN_FOR = {
                                 "contiguous", "o_proj"),
                                ("self", "hidden_states", "position_embeddings", "attention_mask", "past_key_values", "kwargs", "input_shape", "hidden_shape", "query_states",
                                 "key_states", "value_states", "cos", "sin", "attention_interface", "attn_output", "attn_weights")),
+    _falcon_mlp_forward: (("act", "dense_h_to_4h", "dense_4h_to_h"), ("self", "x")),
     _rotary_tables_forward: (("inv_freq", "expand", "shape", "to", "torch", "float", "device", "isinstance", "type", "str", "maybe_autocast", "transpose",
                               "cat", "cos", "attention_scaling", "sin", "dtype"),
                              ("self", "x", "position_ids", "inv_freq_expanded", "position_ids_expanded", "device_type", "freqs", "emb", "cos", "sin")),
@@ -421,6 +452,8 @@ def install_shard_kernels(shard: nn.Module) -> None:
             module.__class__ = _fused_class(type(module), _llama_layer_forward, "The base class with an addition and a norm as one launch (`tpamd_add_rms_norm`).")
         elif is_llama_attention(module):
             module.__class__ = _fused_class(type(module), _llama_attention_forward, "The base class with the rotary embedding of a forward without a cache as one launch (`tpamd_rope`).")
+        elif is_falcon_mlp(module):
+            module.__class__ = _fused_class(type(module), _falcon_mlp_forward, "The base class with the activation in an int8 Linear's epilogue (`tpamd_linear_w8`).")
         elif is_rotary_tables(module):
             module.__class__ = _fused_class(type(module), _rotary_tables_forward, "The base class with its forward as one launch (`tpamd_rope_tables`).")
     for module in shard.modules():

@@ -199,8 +199,8 @@ W8_TOGETHER_ROWS = 64
 
 
 def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, outlier_idx: Optional[torch.Tensor], w_out: Optional[torch.Tensor],
-              bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    return _call(_native.linear_w8, _native.linear_w8_ranks, (x, wq, scale, outlier_idx, w_out, bias))
+              bias: Optional[torch.Tensor] = None, act: int = _native.ACT_NONE) -> torch.Tensor:
+    return _call(_native.linear_w8, _native.linear_w8_ranks, (x, wq, scale, outlier_idx, w_out, bias), (act,))
 
 
 def _linear_w8_sum(calls: List[tuple]) -> Sequence[torch.Tensor]:

@@ -127,3 +127,45 @@ def test_outlier_columns_by_name_and_conv1d():
     assert n == 2 and block.fc.outlier_idx.tolist() == [3, 17] and block.proj.outlier_idx.tolist() == [0]
     assert block.proj.in_features == 96 and block.proj.out_features == 48
     torch.testing.assert_close(got, want, rtol=5e-2, atol=5e-2 * want.std().item())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 300])
+def test_activation_of_a_falcon_mlp_in_the_first_linear(M, dtype, monkeypatch):
+    """Alone and in a launch of two ranks; a block whose activation or first Linear somebody watches keeps its own forward."""
+    from transformers import FalconConfig
+    from transformers.models.falcon.modeling_falcon import FalconMLP
+
+    from tensor_parallel_amd import _native, shard_modules
+
+    g, K, N = torch.Generator().manual_seed(M), 256, 1024
+    mlp = FalconMLP(FalconConfig(hidden_size=K, bias=False)).to(DEV, dtype)
+    with torch.no_grad():
+        mlp.dense_h_to_4h.weight.copy_(torch.randn(N, K, generator=g) * 0.1)
+    weight = mlp.dense_h_to_4h.weight.detach()
+    cols = torch.randperm(K, generator=g)[:3].sort().values
+    shard_modules.install_shard_kernels(mlp)
+    assert quantize_linears_(mlp, outlier_cols=lambda name, m: cols.tolist() if name == "dense_h_to_4h" else None) == 2
+    x = torch.randn(M, K, generator=g).to(DEV, dtype)
+    product, acts = ShardLinearW8._product, []
+    monkeypatch.setattr(ShardLinearW8, "_product", lambda self, input, act: acts.append(act) or product(self, input, act))
+    second, mlp.dense_4h_to_h = mlp.dense_4h_to_h, torch.nn.Identity()
+    wq, scale, w_out = oq.quantize_rows(weight.float().cpu().numpy(), cols.numpy())
+    want = torch.nn.functional.gelu(torch.from_numpy(oq.linear_w8_f64(x.float().cpu().numpy(), wq, scale, cols.numpy(), w_out)))
+    with torch.no_grad():
+        got = mlp(x)
+        # GELU's slope is below 1.13: the Linear's own bound, times that; and the step in between rounded to the dtype where the Linear does not make it
+        torch.testing.assert_close(got.double().cpu(), want, rtol=RTOL, atol=1.13 * RTOL * 0.1 * math.sqrt(K))
+        up = mlp.dense_h_to_4h
+        call = (x, up.wq, up.scale, up.outlier_idx, up.w_out, None, _native.ACT_GELU)
+        for y in _native.linear_w8_ranks([call, call]):
+            torch.testing.assert_close(y.double().cpu(), want, rtol=RTOL, atol=1.13 * RTOL * 0.1 * math.sqrt(K))
+        mlp.dense_4h_to_h, handle = second, mlp.act.register_forward_hook(lambda *_: None)
+        first = _native.ACT_GELU if M <= 64 else _native.ACT_NONE
+        assert acts == [first]
+        mlp(x)
+        handle.remove()
+        mlp(x)
+        mlp.act = torch.nn.GELU(approximate="tanh")
+        mlp(x)
+    assert acts == [first, *[_native.ACT_NONE] * 2, first, *[_native.ACT_NONE] * 3]
