@@ -371,7 +371,7 @@ int tpamd_rope_tables_ranks(int n, const void *const *inv_freq_dev, int freq_dty
                             int64_t B, int64_t S, int64_t half, float scaling, void *const *cos_dev, void *const *sin_dev, int dtype, void *stream);
 int tpamd_causal_mask_ranks(int n, const void *const *q_offset_dev, int64_t kv_offset, int64_t rows, int64_t cols, void *const *mask_dev,
                             void *stream);
-/* out[r] = a[r] + b[r], rounded, element for element; pointers 16-byte aligned, fewer than 2^33 elements. */
+/* out[r] = a[r] + b[r], rounded, element for element; pointers 16-byte aligned, fewer than 2^32 elements. */
 int tpamd_add_ranks(int n, const void *const *a_dev, const void *const *b_dev, void *const *out_dev, int64_t elements, int dtype, void *stream);
 /* *counts[r] += by, int64 on the device. */
 int tpamd_advance_ranks(int n, void *const *counts_dev, int64_t by, void *stream);

@@ -21,7 +21,9 @@ __global__ __launch_bounds__(256) void causal_mask_kernel(const int64_t *q_offse
     for (int64_t i = blockIdx.y; i < rows; i += gridDim.y) out[i * cols + j] = kv_offset + j <= first + i ? 1 : 0;
 }
 
-// The counts of cached positions of several ranks, advanced by one launch (torch: one per rank, 2-4 us each in a recorded step and layer).
+// The counts of cached positions of several ranks, advanced by one launch of one wavefront: latency, 4.5 us in a recorded step and layer where torch's
+// additions took 1.9-4.6 us for each of two ranks (with the additions behind the MLPs, the tables and the mask of both ranks in one launch each:
+// 260 -> 249 us of a two-layer step of one row, 408 -> 400 of 40).
 struct Counts {
     int64_t *at[8];
 };
@@ -50,8 +52,9 @@ extern "C" int tpamd_causal_mask_ranks(int n, const void *const *q_offset_dev, i
     // grids of fewer than 2^32 threads: rows beyond those of a grid are taken by its blocks in turn
     const int64_t blocks = (cols + 255) / 256, most = ((1ll << 23) - 1) / blocks > 0 ? ((1ll << 23) - 1) / blocks : 1;
     const int64_t height = rows < most ? rows : most;
-    for (int i = 0; i < n; i += 2) {
-        const bool two = i + 1 < n;
+    const int together = blocks < (1 << 22) ? 2 : 1;
+    for (int i = 0; i < n; i += together) {
+        const bool two = together == 2 && i + 1 < n;
         const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(height < 65535 ? height : 65535), two ? 2 : 1);
         hipLaunchKernelGGL(causal_mask_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const int64_t *>(q_offset_dev[i]), kv_offset, rows, cols,
                            static_cast<uint8_t *>(mask_dev[i]), two ? bytes_from(q_offset_dev[i], q_offset_dev[i + 1]) : 0,

@@ -312,7 +312,7 @@ void launch(NormParams p, int64_t rows, int ranks, bool vec, hipStream_t s) {
 }
 
 // out = a + b, rounded, for both ranks of a launch (blockIdx.y): the addition behind a decoder layer's MLP, which torch makes rank by rank (3.2-4.6 us each in a recorded
-// step). x, r: the operands; n 16-byte chunks, then the elements behind them.
+// step; one launch of 4.6-4.8 for both). Latency at the sizes that come here, so plain 16-byte chunks, one a lane. x, r: the operands; n 16-byte chunks, then the elements behind them.
 template <int DT>
 __global__ __launch_bounds__(256) void add_ranks_kernel(NormParams p, int64_t n, int tail) {
     take_rank(p);
@@ -434,7 +434,7 @@ extern "C" int tpamd_add_ranks(int n, const void *const *a_dev, const void *cons
     const char *who = "tpamd_add_ranks";
     TPAMD_REQUIRE(n >= 0 && a_dev && b_dev && out_dev, "%s: null pointer", who);
     TPAMD_REQUIRE(dtype == TPAMD_BF16 || dtype == TPAMD_F16 || dtype == TPAMD_F32, "%s: unknown dtype %d", who, dtype);
-    TPAMD_REQUIRE(elements >= 0 && elements < (1ll << 33), "%s: bad dimension", who);  // fewer than 2^31 threads a rank
+    TPAMD_REQUIRE(elements >= 0 && elements < (1ll << 32), "%s: bad dimension", who);  // at most 2^31 threads in a launch of two ranks
     if (elements == 0) return TPAMD_OK;
     for (int i = 0; i < n; ++i)
         TPAMD_REQUIRE(a_dev[i] && b_dev[i] && out_dev[i] && aligned(a_dev[i], 16) && aligned(b_dev[i], 16) && aligned(out_dev[i], 16),
