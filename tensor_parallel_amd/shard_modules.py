@@ -302,8 +302,8 @@ def _falcon_mlp_forward(self, x: torch.Tensor) -> torch.Tensor:
     from .int8 import ShardLinearW8
 
     own, up, act, hooks = self._tp_base.forward, self._modules.get("dense_h_to_4h"), self._modules.get("act"), torch.nn.modules.module
-    if (x.dim() == 0 or x.numel() > together.W8_TOGETHER_ROWS * x.shape[-1] or own is not self._tp_replaced or type(up) is not ShardLinearW8 or "forward" in up.__dict__ or not _is_erf_gelu(act)
-            or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _has_hooks(up) or _has_hooks(act) or not _native.plain_call(x)
+    if (own is not self._tp_replaced or type(up) is not ShardLinearW8 or not _native.plain_call(x) or x.dim() == 0 or x.numel() > together.W8_TOGETHER_ROWS * x.shape[-1]
+            or "forward" in up.__dict__ or not _is_erf_gelu(act) or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _has_hooks(up) or _has_hooks(act)
             or torch.is_grad_enabled() and x.requires_grad):
         return own(self, x)
     return self.dense_4h_to_h(up._product(x, _native.ACT_GELU))
@@ -355,8 +355,8 @@ _fused_classes: dict = {}
 
 def _fused_class(base: type, forward, doc: str) -> type:
     """Subclass of a module's own class with another forward (isinstance checks keep working, and so does pickling). `_tp_replaced` is the
-    forward it stands in for; once the class has another (None: it had when the subclass was made), that one runs. The classes of a decoder layer and its
-    attention keep their names, which programs look such modules up by; the others are named as `ShardLinear` is."""
+    forward it stands in for; once the class has another (None: it had when the subclass was made), that one runs. The classes of a decoder layer, its
+    attention and its MLP keep their names, which programs look such modules up by; the others are named as `ShardLinear` is."""
     cls = _fused_classes.get((base, forward))
     if cls is None:
         def reduce_ex(self, protocol):  # the class is made here and has no name to be found by: pickle what makes it
@@ -367,7 +367,7 @@ def _fused_class(base: type, forward, doc: str) -> type:
             own.__dict__.update(self.__dict__)
             return own
 
-        name = base.__name__ if forward in (_llama_layer_forward, _llama_attention_forward) else "Shard" + base.__name__
+        name = base.__name__ if forward in (_llama_layer_forward, _llama_attention_forward, _falcon_mlp_forward) else "Shard" + base.__name__
         cls = type(name, (base,), {"forward": forward, "__doc__": doc, "__reduce_ex__": reduce_ex, "__prepare_scriptable__": prepare_scriptable, "_tp_base": base,
                                 "_tp_replaced": staticmethod(base.forward if _takes_stand_in(base, forward) else None)})
         if forward is _llama_attention_forward:  # None in the place of one that is not transformers' own
