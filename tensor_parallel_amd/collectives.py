@@ -19,7 +19,7 @@ from typing import Any, Callable, List, Optional
 import torch
 
 from . import _native
-from .shard_modules import _guard
+from .shard_modules import _guard, hands_through
 from .slicing import concat_dim
 from .together import GreenTurn, current_turn, set_turn_lock  # noqa: F401 - the names under which forwards look them up
 
@@ -71,11 +71,14 @@ _contexts: contextvars.ContextVar = contextvars.ContextVar("tpamd_sum_contexts",
 class SumContext:
     """One call of a wrapped module whose output 0 goes to `op`, on one rank."""
 
-    __slots__ = ("op", "rank", "owner", "last_linear", "last_out", "calls", "fused_out", "fused_mask", "fused_copy", "fused_whole", "last_version")
+    __slots__ = ("op", "rank", "owner", "last_linear", "last_out", "last_version", "calls", "fused_linear", "fused_out", "fused_version", "fused_mask", "fused_copy",
+                 "fused_whole")
 
     def __init__(self, op: "DeviceAllReduce", rank: int, owner: Any):
         self.op, self.rank, self.owner = op, rank, owner
-        self.last_linear = self.last_out = self.last_version = self.fused_out = self.fused_copy = self.fused_whole = None
+        self.last_linear = self.last_out = self.last_version = None
+        self.fused_linear = self.fused_out = self.fused_version = self.fused_copy = None
+        self.fused_whole = False  # fused_out was made as a sum over all ranks
         self.calls: dict = {}
         self.fused_mask = 0
 
@@ -85,13 +88,19 @@ class SumContext:
         teaches the Linear that produced exactly this value (and ran once) that it feeds the sum: next time it may fold."""
         if self.fused_out is not None:
             if value is not self.fused_out:
-                raise RuntimeError(
-                    "tensor_parallel_amd: a row-parallel Linear added the other ranks' partial sums in its epilogue, but its "
-                    "module then returned a different tensor; set TPAMD_FUSE_SUM=0 to keep the sum in its own kernel")
+                raise self.lost("its module then returned a different tensor")
         elif self.last_linear is not None:
-            feeds = value is self.last_out and self.calls.get(id(self.last_linear)) == 1 and (self.last_version is None or value._version == self.last_version)
+            feeds = value is self.last_out and self.calls.get(id(self.last_linear)) == 1
+            if feeds:  # unchanged, which has to be known by the module's forward where changes are not counted
+                feeds = value._version == self.last_version if self.last_version is not None else hands_through(self.owner.tp_wrapped_module, self.last_linear)
             self.last_linear.__dict__["_tp_feeds_sum"] = self.owner if feeds else None
             self.owner.__dict__["_tp_sum_known"] = True
+
+    def lost(self, why: str) -> RuntimeError:
+        """The value holds other ranks' parts of the sum and is not what is to be summed: nothing can make it that. The Linear does not fold in its next call."""
+        self.fused_linear.__dict__["_tp_feeds_sum"] = None
+        return RuntimeError("tensor_parallel_amd: a row-parallel Linear added the other ranks' partial sums in its epilogue, but "
+                            f"{why}; set TPAMD_FUSE_SUM=0 to keep the sum in its own kernel")
 
 
 def push_sum_context(ctx: Optional[SumContext]) -> None:
@@ -241,15 +250,11 @@ class DeviceAllReduce(CollectiveOperation):
         mask = 1 << rank
         ctx = current_sum_context()
         if ctx is not None and ctx.op is self and ctx.fused_out is not None and x is ctx.fused_out:
+            if ctx.fused_version is not None and ctx.fused_version != x._version:
+                raise ctx.lost("it was then changed in place on its way to the \"sum\" rule")
             mask |= ctx.fused_mask  # this value already holds what the rank's Linear was given by addend_for()
-            if ctx.fused_whole is not None:
-                if ctx.fused_whole != x._version:
-                    raise RuntimeError(
-                        "tensor_parallel_amd: the output of a row-parallel Linear was changed in place on its way to a \"sum\" rule; it held the sum over the "
-                        "ranks already. Set TPAMD_FUSE_SUM=0 to keep the sum in its own kernel")
-                self._whole[rank] = True
-            if ctx.fused_copy is not None and ctx.fused_copy[1] == x._version:  # nobody has written to the value since
-                self._copy = ctx.fused_copy[0]
+            self._whole[rank] = ctx.fused_whole
+            self._copy = ctx.fused_copy
         self._masks[rank] = mask
         try:
             return super().__call__(x, rank)

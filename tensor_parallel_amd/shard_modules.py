@@ -51,12 +51,12 @@ def linear_in_context(module: nn.Module, x: torch.Tensor, w: torch.Tensor, bias)
                               lambda rank: together.linear_sum(xd, wd, b, rank))
 
 
-def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs: tuple, with_peers, alone, summed) -> torch.Tensor:
+def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs: tuple, with_peers, alone, summed, learned: bool = True) -> torch.Tensor:
     """A shard's Linear with `columns` outputs, made by with_peers() or, with an addend, alone(addend=, copy=). Inside a wrapped module whose output goes to a
     "sum" rule (collectives.SumContext) the Linear that was seen to produce that output hands over the sum: two ranks that meet in it get it from
     summed(rank) (`tpamd_linear_sum_ranks`; None: not to be had), else the rank that comes last adds the partial sums already waiting in
     the reduction, in its epilogue (`tpamd_linear_add`): the product rounded to the dtype, then one rounded add, which
-    is the same arithmetic as the reduction kernel's step."""
+    is the same arithmetic as the reduction kernel's step. `learned`: having been seen to produce it is enough (see _may_hold_sum)."""
     from .collectives import current_sum_context
 
     ctx = current_sum_context()
@@ -65,16 +65,16 @@ def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs:
     key = id(module)
     ctx.calls[key] = ctx.calls.get(key, 0) + 1
     out, more = None, {}
-    if module.__dict__.get("_tp_feeds_sum") is ctx.owner and ctx.owner is not None:
+    if module.__dict__.get("_tp_feeds_sum") is ctx.owner and ctx.owner is not None and _may_hold_sum(module, ctx.owner, learned):
         if ctx.fused_out is not None:
             raise RuntimeError("tensor_parallel_amd: the Linear that feeds a \"sum\" rule ran twice in one call of its module "
                                "after adding the waiting partial sums; set TPAMD_FUSE_SUM=0")
         waiting = ctx.op.addend_for(ctx.rank)
-        if waiting is None and summed is not None and ctx.op.world_size == 2 and _sum_unwatched(module, ctx.owner):
+        if waiting is None and summed is not None and ctx.op.world_size == 2 and _is_last_child(module, ctx.owner.tp_wrapped_module):
             out = summed(ctx.rank)
         if out is not None:
             out = _guard(out, *inputs)
-            ctx.fused_out, ctx.fused_mask, ctx.fused_whole = out, 3, out._version
+            ctx.fused_mask, ctx.fused_whole = 3, True
         else:
             if waiting is None:  # (a rank that waited for its peer in vain finds what that one has handed in since)
                 waiting = ctx.op.addend_for(ctx.rank)
@@ -87,21 +87,38 @@ def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs:
             out = _guard(alone(**more), *inputs)
     else:  # ranks meet in other Linears once a first call has shown which one feeds the sum
         out = _guard(with_peers() if "_tp_sum_known" in ctx.owner.__dict__ else alone(), *inputs)
-    if more:
-        ctx.fused_out = out
-        if "copy" in more and not out.is_inference():  # (whose changes are not counted)
-            ctx.fused_copy = more["copy"], out._version
     ctx.last_linear, ctx.last_out = module, out
-    ctx.last_version = None if out.is_inference() else out._version
+    ctx.last_version = None if out.is_inference() else out._version  # (changes of an inference tensor are not counted)
+    if more or ctx.fused_whole:
+        ctx.fused_linear, ctx.fused_out, ctx.fused_version, ctx.fused_copy = module, out, ctx.last_version, more.get("copy")
     return out
 
 
-def _sum_unwatched(module: nn.Module, owner: nn.Module) -> bool:
-    """Whether nobody is told of a Linear's output on its way to the sum, so that it may be the sum already: no hooks on it, on the module around it (the wrapped one)
-    or on all modules; and changes to it would show (they are not counted in inference mode)."""
+def _may_hold_sum(module: nn.Module, owner: nn.Module, learned: bool) -> bool:
+    """Whether a Linear's output may hold other ranks' parts already on its way to the sum: nobody who is told of it there would see or change more than this rank's
+    part. Not with hooks on the Linear, on the module around it (the wrapped one) or on all modules, nor with a forward that a program has put around the
+    Linear's. Then either the wrapped module is known to return it untouched, or (`learned`) it did so when it was last seen without, and a
+    change shows in the tensor's version, which raises; in inference mode versions stand still."""
     wrapped, hooks = owner.tp_wrapped_module, torch.nn.modules.module
-    return not (torch.is_inference_mode_enabled() or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _has_hooks(module) or _has_hooks(wrapped)) \
-        and (wrapped is module or any(child is module for child in wrapped._modules.values()))
+    if hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _has_hooks(module) or _has_hooks(wrapped) or "forward" in module.__dict__:
+        return False
+    return learned and not torch.is_inference_mode_enabled() or hands_through(wrapped, module)
+
+
+def _is_last_child(module: nn.Module, wrapped: nn.Module) -> bool:
+    """No module lies between the wrapped one and the Linear that feeds its sum, whose hooks would be told of the output."""
+    return wrapped is module or any(child is module for child in wrapped._modules.values())
+
+
+def hands_through(wrapped: nn.Module, module: nn.Module) -> bool:
+    """Whether the wrapped module is this Linear, or has one of the forwards below (or the transformers one it stands in for), which return what this Linear gave."""
+    if wrapped is module:
+        return True
+    own, cls = wrapped.__dict__.get("forward"), type(wrapped)
+    if own is not None:
+        return getattr(own, "__func__", None) is _gated_mlp_forward and wrapped._modules.get("down_proj") is module
+    last = "o_proj" if cls.forward is _llama_attention_forward else "dense_4h_to_h" if cls.forward is _falcon_mlp_forward else None
+    return last is not None and cls._tp_base.forward is cls._tp_replaced and wrapped._modules.get(last) is module
 
 
 def gathered_linear(module: nn.Module, op, rank: int, args, kwargs):
