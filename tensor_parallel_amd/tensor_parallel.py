@@ -22,6 +22,7 @@ from torch import nn
 
 from .autoconfig import get_default_config
 from .collectives import GreenTurn, Turn, set_turn_lock
+from .together import keeps_turn
 from .config import Config, add_lora_rules
 from .int8 import ShardLinearW8
 from .kv_cache import is_kv_cache, rank_caches
@@ -274,7 +275,7 @@ def _apply_in_greenlets(modules: Sequence[nn.Module], inputs, kwargs_tup, device
     ranks = [_greenlet.greenlet(functools.partial(body, i, m, a, k), parent=hub)
              for i, (m, a, k) in enumerate(zip(modules, inputs, kwargs_tup))]
     with torch.cuda.device(device) if device.type == "cuda" else contextlib.nullcontext():
-        turn = GreenTurn(len(ranks), device.index if device.type == "cuda" else None)
+        turn = GreenTurn(len(ranks), device.index if device.type == "cuda" else None, not any(keeps_turn(m) for m in modules))
         turn.ring = list(ranks)
         while turn.ring:
             turn.ring[turn.at].switch()  # comes back when a rank has returned

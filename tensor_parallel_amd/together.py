@@ -8,18 +8,31 @@ last makes the call for all of them (`tpamd_*_ranks`). Two Llama-2-7B-shaped ran
 positions 321 -> 278 us, 8 on 2048 479 -> 423, 40 on 1000 (grouped queries) 534 -> 454; the Falcon-40B-shaped int8 layer, 16 on 2048, 372 -> 339.
 On the host a meeting costs 4 to 5 us for both ranks, about what the call that it saves costs (eager decode steps and scoring stay where they were, within 2 %).
 
-A rank meets its peers only in the state it was started in (`_thread_state`): inside a stream, a grad or autocast mode or a function
-mode of its own, giving the turn away would take its peers there.
+A rank meets its peers only in the state it was started in (`_thread_state`): in a stream, a grad or autocast mode, a function mode or with switches (default
+dtype, attention backends, deterministic algorithms) of its own it keeps the turn, because giving it away would take its peers there. Waiting in a collective it has to
+give it away: its peers then go on in the state that they were started in, and it finds its own again (`_as_started`).
+
+What cannot be seen so is what a program holds across a library call: with a lock held there, the peer that asks for the lock would wait for a rank that cannot go on.
+Models whose own forwards (not those of torch and transformers) enter a `with` block or acquire something therefore do not meet (`keeps_turn`, which looks at a model in
+its first forward). What it does not find, a lock taken in one hook and given back in another, say, has to be kept to one call, or meeting switched off: TPAMD_MEET=0.
+Collectives give the turn away in any case.
 """
 from __future__ import annotations
 
+import contextlib
 import contextvars
+import dis
+import os
 import threading
+import types
 from typing import Any, Callable, List, Optional, Sequence
 
 import torch
+from torch.utils._python_dispatch import _pop_mode, _push_mode
 
 from . import _native
+
+MEET = os.environ.get("TPAMD_MEET", "1") != "0"
 
 # The turn of the running forward, per rank: context variables are per thread and per greenlet.
 _turn: contextvars.ContextVar = contextvars.ContextVar("tpamd_turn", default=None)
@@ -37,22 +50,122 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _current_device = getattr(torch._C, "_cuda_getDevice", None)
 _grad, _inference, _autocast = torch.is_grad_enabled, torch.is_inference_mode_enabled, torch.is_autocast_enabled
 _function_modes, _dispatch_modes = torch._C._len_torch_function_stack, torch._C._len_torch_dispatch_stack
+_autocast_deeper, _autocast_back = torch.autocast_increment_nesting, torch.autocast_decrement_nesting
+_default_dtype, _deterministic, _tf32 = torch.get_default_dtype, torch._C._get_deterministic_algorithms, torch._C._get_cublas_allow_tf32
+_flash, _efficient, _math, _cudnn = (getattr(torch._C, f"_get_{name}_sdp_enabled") for name in ("flash", "mem_efficient", "math", "cudnn"))
 
 
 def _thread_state(index: Optional[int]) -> tuple:
-    """What of the calling thread's state a rank would find changed if a peer gave it the turn from somewhere else. `index`: of the HIP device, or None."""
-    return (_grad(), _inference(), _autocast(), _function_modes(), _dispatch_modes(),
+    """What of the calling thread's state a rank would find changed if a peer gave it the turn from somewhere else. `index`: of the HIP device, or None. Read
+    in every library call (about a microsecond): an autocast scope shows by the depth of scopes, whatever device and dtype it is for."""
+    return (_grad(), _inference(), _autocast(), _autocast_deeper() + _autocast_back(), _function_modes(), _dispatch_modes(), _default_dtype(),
+            _flash(), _efficient(), _math(), _cudnn(), _deterministic(), _tf32(),
             None if index is None else (_current_device(), _raw_stream(index)))
 
 
+def _of_device(get, put, device: str) -> tuple:
+    return lambda: get(device), lambda value: put(device, value)
+
+
+# What of that state can be set, and all that belongs to it: reading and setting.
+_SETTINGS = [
+    (_grad, torch._C._set_grad_enabled),
+    *(_of_device(get, put, device) for device in ("cuda", "cpu") for get, put in ((_autocast, torch.set_autocast_enabled), (torch.get_autocast_dtype, torch.set_autocast_dtype))),
+    (torch.is_autocast_cache_enabled, torch.set_autocast_cache_enabled),
+    (_default_dtype, torch.set_default_dtype),
+    (_flash, torch._C._set_sdp_use_flash), (_efficient, torch._C._set_sdp_use_mem_efficient), (_math, torch._C._set_sdp_use_math),
+    (_cudnn, torch._C._set_sdp_use_cudnn),
+    (lambda: (_deterministic(), torch._C._get_deterministic_algorithms_warn_only()), lambda value: torch._C._set_deterministic_algorithms(value[0], warn_only=value[1])),
+    (_tf32, torch._C._set_cublas_allow_tf32),
+]
+
+
+def _settings() -> list:
+    return [get() for get, _ in _SETTINGS]
+
+
+def _set(values: list) -> None:
+    for (get, put), value in zip(_SETTINGS, values):
+        if get() != value:
+            put(value)
+
+
+@contextlib.contextmanager
+def _as_started(turn: "GreenTurn"):
+    """For a rank that gives the turn away in a state of its own: the state that the ranks were started in, inside, and its own again behind."""
+    own, index = _settings(), turn.index
+    where = None if index is None else (torch._C._cuda_getCurrentStream(index), _current_device())
+    modes, dispatch = [], []
+    while _function_modes() > turn.state[4]:
+        modes.append(torch._C._pop_torch_function_stack())
+    while _dispatch_modes() > turn.state[5]:
+        dispatch.append(_pop_mode())
+    inference = torch._C._InferenceMode(turn.state[1])
+    inference.__enter__()
+    _set(turn.settings)
+    if index is not None:
+        stream, device_index, device_type = turn.stream
+        torch._C._cuda_setStream(stream_id=stream, device_index=device_index, device_type=device_type)
+        torch.cuda.set_device(turn.state[-1][0])
+    try:
+        yield
+    finally:
+        inference.__exit__(None, None, None)
+        for mode in reversed(dispatch):
+            _push_mode(mode)
+        for mode in reversed(modes):
+            torch._C._push_on_torch_function_stack(mode)
+        _set(own)
+        if where is not None:
+            (stream, device_index, device_type), device = where
+            torch._C._cuda_setStream(stream_id=stream, device_index=device_index, device_type=device_type)
+            torch.cuda.set_device(device)
+
+
+_LIBRARIES = ("torch", "transformers", "tensor_parallel_amd")
+
+
+def _holds(f, cls: type, seen: set) -> bool:
+    """Whether a program's function, what it decorates, or a method or function that it calls by name enters a `with` block or acquires something."""
+    f = getattr(f, "func", getattr(f, "__func__", f))  # functools.partial, a bound method
+    code = getattr(f, "__code__", None)
+    if code is None:
+        return type(f).__module__.split(".")[0] not in ("builtins", *_LIBRARIES)
+    if code in seen:
+        return False
+    seen.add(code)
+    inner = [cell.cell_contents for cell in f.__closure__ or () if isinstance(cell.cell_contents, types.FunctionType)]
+    if f.__globals__.get("__name__", "").split(".")[0] not in _LIBRARIES:
+        codes = [code]
+        for c in codes:
+            codes += [k for k in c.co_consts if isinstance(k, types.CodeType)]
+            if "acquire" in c.co_names or "enter_context" in c.co_names or any(op.opname in ("SETUP_WITH", "BEFORE_WITH") for op in dis.get_instructions(c)):
+                return True
+        called = [getattr(cls, name, None) or f.__globals__.get(name) for c in codes for name in c.co_names]
+        inner += [g for g in called if isinstance(g, types.FunctionType)]
+    return any(_holds(g, cls, seen) for g in inner)
+
+
+def keeps_turn(module: Any) -> bool:
+    """Whether a forward of this module may hold something across a library call (see above). Looked for once: kept with the module."""
+    if not isinstance(module, torch.nn.Module):
+        return False
+    keeps = module.__dict__.get("_tp_keeps_turn")
+    if keeps is None:
+        forwards = {(type(m), m.__dict__.get("forward")) for m in module.modules() if m._modules}
+        keeps = module.__dict__["_tp_keeps_turn"] = any(_holds(own or cls.forward, cls, set()) for cls, own in forwards)
+    return keeps
+
+
 class _Meeting:
-    __slots__ = ("one", "many", "more", "calls", "results", "error")
+    __slots__ = ("one", "many", "more", "calls", "results", "error", "parted")
 
     def __init__(self, one, many, more):
         self.one, self.many, self.more = one, many, more
         self.calls: List[tuple] = []
         self.results: Optional[Sequence[Any]] = None
         self.error: Optional[BaseException] = None
+        self.parted = False
 
 
 def _alike(a: tuple, b: tuple) -> bool:
@@ -69,29 +182,39 @@ class GreenTurn:
     them (tensor_parallel._apply_in_greenlets). `idle` counts the waits since a collective or a meeting was last complete or a rank returned: when every
     rank has waited twice, all wait for something that will not come."""
 
-    __slots__ = ("ring", "at", "idle", "failed", "world", "index", "state", "open")
+    __slots__ = ("ring", "at", "idle", "failed", "world", "index", "state", "settings", "stream", "meets", "open")
 
-    def __init__(self, world: int = 1, index: Optional[int] = None):
+    def __init__(self, world: int = 1, index: Optional[int] = None, meets: bool = True):
         self.ring: List[Any] = []
         self.at = self.idle = 0
         self.failed = False
         self.world = world
         self.index = index
-        self.state = _thread_state(index)
+        self.state, self.settings = _thread_state(index), _settings()
+        self.stream = None if index is None else torch._C._cuda_getCurrentStream(index)
+        self.meets = meets and MEET and world > 1
         self.open: List[_Meeting] = []  # meetings that not every rank has come to, oldest first
 
     def wait(self, timeout: float = 0.0) -> bool:
+        if _thread_state(self.index) == self.state:
+            self._pass_on()
+        else:
+            with _as_started(self):
+                self._pass_on()
+        return True
+
+    def _pass_on(self) -> None:
+        """Gives the turn to the next rank, in the state that the ranks were started in; comes back in that state."""
         ring = self.ring
         self.idle += 1
         if self.idle > 2 * len(ring):
             self.idle = 0
-            if not self.part():
+            if not self._part():
                 self.failed = True
         at = self.at + 1
         self.at = at = at if at < len(ring) else 0
         if len(ring) > 1:
             ring[at].switch()
-        return True
 
     def wake(self) -> None:
         self.idle = 0
@@ -109,7 +232,7 @@ class GreenTurn:
 
     def meet(self, one: Callable[..., Any], many: Callable[[List[tuple]], Sequence[Any]], tensors: tuple, more: tuple, own: tuple = ()) -> Any:
         """one(*tensors, *more, *own), made as many([...]) for all ranks that come with tensors of the same forms and the same `more`, in the order in
-        which they came. A rank whose peers do not come (they wait elsewhere or have returned) makes the call alone (`part`)."""
+        which they came. A rank whose peers do not come (they wait elsewhere or have returned) makes the call alone (`_part`)."""
         for meeting in self.open:
             if meeting.one is one and meeting.more == more and _alike(meeting.calls[0][0], tensors):
                 break
@@ -129,27 +252,26 @@ class GreenTurn:
             while meeting.results is None and meeting.error is None:
                 if self.failed:
                     raise threading.BrokenBarrierError
-                self.wait()
+                if meeting.parted:
+                    return one(*tensors, *more, *own)
+                self._pass_on()
         if meeting.error is not None:
             raise meeting.error
         return meeting.results[place]
 
-    def part(self) -> bool:
-        """Nobody gets any further: the calls handed in so far are made one by one. False: there were none."""
+    def _part(self) -> bool:
+        """Nobody gets any further: the ranks make the calls handed in so far alone. False: there were none."""
         if not self.open:
             return False
         meetings, self.open = self.open, []
         for m in meetings:
-            try:
-                m.results = [m.one(*tensors, *m.more, *own) for tensors, own in m.calls]
-            except BaseException as e:
-                m.error = e
+            m.parted = True
         return True
 
 
 def _call(one: Callable[..., Any], many: Callable[[List[tuple]], Sequence[Any]], tensors: tuple, more: tuple = (), own: tuple = ()) -> Any:
     turn = _turn.get()
-    if type(turn) is not GreenTurn or turn.world < 2 or turn.failed or _thread_state(turn.index) != turn.state:
+    if type(turn) is not GreenTurn or not turn.meets or turn.failed or _thread_state(turn.index) != turn.state:
         return one(*tensors, *more, *own)
     return turn.meet(one, many, tensors, more, own)
 

@@ -139,6 +139,44 @@ def test_ranks_that_do_not_fit_each_other_make_their_calls_alone():
             close(a, b, torch.bfloat16)
 
 
+@pytest.mark.parametrize("first", ["library call", "collective"])
+def test_a_rank_that_waits_in_a_stream_of_its_own_leaves_its_peers_theirs(first):
+    """Rank 1 waits in a collective inside a stream and an inference mode of its own, rank 0 for a library call that nobody else makes or for that collective."""
+    from tensor_parallel_amd import together
+    from tensor_parallel_amd.collectives import CollectiveOperation
+    from tensor_parallel_amd.tensor_parallel import _apply_in_greenlets
+
+    side, op = torch.cuda.Stream(), CollectiveOperation(2, lambda *xs: [sum(xs)] * 2, timeout=5.0)
+    x, w = draws(1, 5, 256, dtype=torch.bfloat16)[0], draws(1, 128, 256, dtype=torch.bfloat16, seed=1)[0]
+    streams = {0: [], 1: []}
+
+    def body(r):
+        here = lambda: streams[r].append((torch.cuda.current_stream(), torch.is_inference_mode_enabled(), torch.is_grad_enabled()))  # noqa: E731
+        here()
+        if r == 0:
+            y = together.linear(x, w) if first == "library call" else None
+            for _ in range(3):
+                op(1, 0)
+                here()
+            return y
+        op(2, 1) if first == "collective" else None
+        with torch.inference_mode(), torch.cuda.stream(side):
+            for _ in range(3 - (first == "collective")):
+                op(2, 1)
+                here()
+        here()
+
+    with torch.no_grad():
+        main = torch.cuda.current_stream()
+        y, _ = _apply_in_greenlets([body, body], [(0,), (1,)], [{}] * 2, DEV)
+        assert torch.cuda.current_stream() == main and not torch.is_grad_enabled()
+    torch.cuda.synchronize()
+    assert all(seen == (main, False, False) for seen in streams[0]) and len(streams[0]) == 4
+    assert streams[1][0] == streams[1][-1] == (main, False, False) and all(seen == (side, True, False) for seen in streams[1][1:-1])
+    if y is not None:
+        close(y, x.float() @ w.float().t(), torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("rows", [1, 3, 4, 16, 33, 64, 129, 700])
 @pytest.mark.parametrize("cols,K,n", [(4, 8, 2), (384, 768, 2), (3072, 768, 2), (1000, 1088, 2), (516, 264, 3), (7, 30, 2)])

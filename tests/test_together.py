@@ -1,6 +1,7 @@
 """Ranks that hand equal calls in together (together.py), on the CPU with the library calls stubbed: which ranks meet, what each gets back, and
 that nobody waits for a peer that does not come."""
 import contextlib
+import threading
 
 import pytest
 import torch
@@ -158,3 +159,153 @@ def test_gathered_columns_are_in_rank_order_whoever_came_first(monkeypatch):
     for got in run(body, body):  # whoever came last goes on first
         assert all(torch.equal(y, want) for y in got)
     assert run(lambda r: together.linear_gathered(*operands(r), None, r, 2), lambda r: r) == [None, 1]  # the peer does not come: nothing is gathered
+
+
+@contextlib.contextmanager
+def _default_dtype(dtype):
+    before = torch.get_default_dtype()
+    torch.set_default_dtype(dtype)
+    try:
+        yield
+    finally:
+        torch.set_default_dtype(before)
+
+
+@contextlib.contextmanager
+def _deterministic():
+    torch.use_deterministic_algorithms(True)
+    try:
+        yield
+    finally:
+        torch.use_deterministic_algorithms(False)
+
+
+def _scopes():
+    from torch.nn.attention import SDPBackend, sdpa_kernel
+
+    return {"default dtype": lambda: _default_dtype(torch.bfloat16), "attention backend": lambda: sdpa_kernel(SDPBackend.MATH), "deterministic": _deterministic,
+            "autocast on the host": lambda: torch.autocast("cpu", dtype=torch.bfloat16), "autocast dtype": lambda: torch.autocast("cpu", dtype=torch.float16, enabled=False),
+            "no grad": torch.no_grad, "inference": torch.inference_mode, "default device": lambda: torch.device("cpu")}
+
+
+def _state():
+    backends = torch.backends.cuda
+    return (torch.is_grad_enabled(), torch.is_inference_mode_enabled(), torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda"),
+            torch.is_autocast_enabled("cpu"), torch.get_autocast_dtype("cpu"), torch.get_default_dtype(), torch.are_deterministic_algorithms_enabled(),
+            backends.flash_sdp_enabled(), backends.mem_efficient_sdp_enabled(), backends.math_sdp_enabled(), torch._C._len_torch_function_stack())
+
+
+@pytest.mark.parametrize("ranks", [(0,), (0, 1)])
+@pytest.mark.parametrize("scope", list(_scopes()))
+def test_a_scope_of_one_rank_is_not_seen_by_another(calls, scope, ranks):
+    """Two library calls and a collective inside the scope, one of each behind it."""
+    from tensor_parallel_amd.collectives import CollectiveOperation
+
+    op, before = CollectiveOperation(2, lambda *xs: [sum(xs)] * 2, timeout=5.0), _state()
+    with _scopes()[scope]():
+        within = _state()
+    assert within != before and _state() == before
+
+    def body(r):
+        outside = []
+        for _ in range(2):
+            with _scopes()[scope]() if r in ranks else contextlib.nullcontext():
+                expected = within if r in ranks else before
+                states = [_state()]
+                for _ in range(2):
+                    together.linear(*operands(r))
+                    states.append(_state())
+                assert op(r + 1, r) == 3
+                states.append(_state())
+                together.linear(*operands(r))
+                states.append(_state())
+                assert states == [expected] * len(states)
+            outside.append(_state())
+            together.linear(*operands(r))
+            op(r, r)
+            outside.append(_state())
+        assert outside == [before] * len(outside)
+
+    run(body, body)
+    assert _state() == before
+
+
+def test_calls_that_nobody_comes_to_are_made_in_the_state_of_their_rank(monkeypatch):
+    """The peer waits in a collective, inside a scope of its own, when it turns out that it does not come."""
+    from tensor_parallel_amd.collectives import CollectiveOperation
+
+    op, states = CollectiveOperation(2, lambda *xs: [sum(xs)] * 2, timeout=5.0), []
+    monkeypatch.setattr(_native, "linear", lambda x, w, b=None: states.append(_state()) or torch.nn.functional.linear(x, w, b))
+    before = _state()
+
+    def body(r):
+        if r == 0:
+            together.linear(*operands(0))
+            op(1, 0)
+        else:
+            with torch.inference_mode(), _default_dtype(torch.float64):
+                op(2, 1)
+
+    run(body, body)
+    assert states == [before]
+
+
+LOCK = threading.Lock()
+
+
+class _Locked(torch.nn.Module):
+    def __init__(self, how):
+        super().__init__()
+        self.how, self.inner = how, torch.nn.Module()
+        self.inner.forward = lambda x, w: together.linear(x, w)
+
+    def forward(self, x, w):
+        if self.how == "with":
+            with LOCK:
+                return self.inner(x, w)
+        return self._acquired(x, w) if self.how == "in a method" else self._plain(x, w)
+
+    def _acquired(self, x, w):
+        LOCK.acquire()
+        try:
+            return self.inner(x, w)
+        finally:
+            LOCK.release()
+
+    def _plain(self, x, w):
+        return self.inner(x, w)
+
+
+class _Unlocked(torch.nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.inner = torch.nn.Linear(1, 1)
+
+    def forward(self, x, w):
+        return together.linear(x, w)
+
+
+@pytest.mark.parametrize("how", ["with", "in a method", "not at all"])
+def test_a_rank_whose_model_may_hold_a_lock_keeps_the_turn(calls, how):
+    models = [_Locked(how) for _ in range(2)] if how != "not at all" else [_Unlocked() for _ in range(2)]
+    for r, y in enumerate(_apply_in_greenlets(models, [operands(r) for r in range(2)], [{}] * 2, CPU)):
+        assert torch.equal(y, torch.nn.functional.linear(*operands(r)))
+    assert calls == ([2] if how == "not at all" else [1, 1])
+
+
+def test_meeting_can_be_switched_off(calls, monkeypatch):
+    monkeypatch.setattr(together, "MEET", False)
+    run(lambda r: together.linear(*operands(r)), lambda r: together.linear(*operands(r)))
+    assert calls == [1, 1]
+
+
+def test_models_of_the_libraries_meet():
+    transformers = pytest.importorskip("transformers")
+    from tensor_parallel_amd.shard_modules import install_shard_kernels
+
+    llama = transformers.LlamaForCausalLM(transformers.LlamaConfig(vocab_size=32, hidden_size=32, intermediate_size=48, num_hidden_layers=1, num_attention_heads=2))
+    falcon = transformers.FalconModel(transformers.FalconConfig(vocab_size=32, hidden_size=32, num_hidden_layers=1, num_attention_heads=2))
+    opt = transformers.OPTForCausalLM(transformers.OPTConfig(vocab_size=32, hidden_size=32, num_hidden_layers=1, num_attention_heads=2, ffn_dim=64, word_embed_proj_dim=32))
+    for model in (llama, falcon, opt):
+        install_shard_kernels(model)
+        assert not together.keeps_turn(model)
