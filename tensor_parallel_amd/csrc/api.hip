@@ -598,9 +598,9 @@ extern "C" int tpamd_linear_w8_ranks(int n, const tpamd_w8_rank *ranks, int64_t 
                                  bytes_from(a.scale, b.scale), o ? bytes_from(a.outlier_idx, b.outlier_idx) : 0, o ? bytes_from(a.w_out, b.w_out) : 0};
             const int rc = skinny_dispatch(a.x, a.wq, nullptr, a.bias, nullptr, 0, a.scale, a.outlier_idx, a.w_out, n_out, a.y, M, N, K, ldx, ldw, ldy,
                                            ld_wout, dtype, act, false, true, static_cast<hipStream_t>(stream), &to);
-            if (rc != TPAMD_OK) return rc;
-            ++i;
-            continue;
+            if (rc == TPAMD_OK) ++i;
+            if (rc == TPAMD_OK) continue;
+            if (rc != TPAMD_ERR_UNSUPPORTED) return rc;  // else nothing was launched: too little scratch memory for two
         }
         const int rc = tpamd_linear_w8(a.x, a.wq, a.scale, a.outlier_idx, a.w_out, n_out, a.bias, a.y, M, N, K, ldx, ldw, ld_wout, ldy, dtype, act, stream);
         if (rc != TPAMD_OK) return rc;

@@ -68,8 +68,9 @@ int device_cus(int dev, int *cus_out);
 // fp32 scratch memory of the K-split kernels (split-K partial tiles, split-key attention partials): defined in
 // runtime.hip. Callers hold splitk_mutex(dev), the lock of their device, from the lookup until their launches that use
 // the buffer are enqueued (two host threads that share a stream must not interleave a K-split launch and its finishing
-// pass), and pass reserve = scratch_reserve(CUs), so that a stream's buffer is allocated with the size every shape can live
-// with: four 128 x 128 partial tiles per CU, and 4 MiB for the packed outlier columns of an int8 Linear beside them.
+// pass), and pass reserve = scratch_reserve(CUs), so that a stream's buffer is allocated with the size every shape of one rank can
+// live with: four 128 x 128 partial tiles per CU, and 4 MiB for the packed outlier columns of an int8 Linear beside them. It never grows: what two ranks
+// of a launch would need beyond it is done rank by rank.
 static inline size_t scratch_reserve(int cus) { return static_cast<size_t>(4) * cus * 128 * 128 * sizeof(float) + (static_cast<size_t>(4) << 20); }
 std::mutex &splitk_mutex(int dev);
 int splitk_scratch(int dev, hipStream_t stream, size_t need, size_t reserve, void **out);

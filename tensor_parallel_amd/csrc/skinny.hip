@@ -1668,6 +1668,18 @@ inline W8Path pick_w8_path(const SkinnyParams &p, int cus) {
     return wide ? W8_COLS : W8_PLAIN;
 }
 
+// Scratch memory for the partial sums of an int8 Linear, `need` bytes for all its ranks. *ws = NULL: none, and the caller takes the unsplit kernel.
+// TPAMD_ERR_UNSUPPORTED: a stream's buffer holds one rank's planes and not two's, so the ranks go one after the other, each on the kernel that its own size asks
+// for (16384 x 8192 with outlier columns from 61 rows on, 9 planes: 75.5 MB at 64 rows, a buffer has 71.3; both ranks unsplit took 138 us, one after the other 104).
+int w8_scratch(const SkinnyParams &p, int dev, int cus, hipStream_t s, size_t need, void **ws) {
+    if (int rc = splitk_scratch(dev, s, need, scratch_reserve(cus), ws); rc != TPAMD_OK || *ws != nullptr || p.ranks == 1 || p.sum) return rc;
+    void *one = nullptr;
+    if (int rc = splitk_scratch(dev, s, need / p.ranks, scratch_reserve(cus), &one); rc != TPAMD_OK) return rc;
+    if (one == nullptr) return TPAMD_OK;
+    set_error("linear_w8: scratch memory for one rank's partial sums at a time");
+    return TPAMD_ERR_UNSUPPORTED;
+}
+
 // int8 weights, K split over blocks: K at least 4096, at most 64 rows and 256 outlier columns.
 // Needs the per-device scratch buffer for the partial sums; without it (first use under stream capture) the
 // caller takes the unsplit kernel.
@@ -1704,7 +1716,7 @@ int launch_w8_split(const SkinnyParams &p, hipStream_t s, bool *done) {
     const size_t need = static_cast<size_t>(splits) * p.ranks * p.M * p.N * sizeof(float);
     std::lock_guard<std::mutex> hold(splitk_mutex(dev));
     void *ws = nullptr;
-    const int rc = splitk_scratch(dev, s, need, scratch_reserve(cus), &ws);
+    const int rc = w8_scratch(p, dev, cus, s, need, &ws);
     if (rc != TPAMD_OK) return rc;
     if (ws == nullptr) return TPAMD_OK;
     float *part = static_cast<float *>(ws);
@@ -1757,7 +1769,7 @@ int launch_w8_cols_mt(const SkinnyParams &p, int dev, int cus, hipStream_t s, bo
     const size_t need = static_cast<size_t>(planes) * p.ranks * p.M * p.N * sizeof(float);
     std::lock_guard<std::mutex> hold(splitk_mutex(dev));
     void *ws = nullptr;
-    const int rc = splitk_scratch(dev, s, need, scratch_reserve(cus), &ws);
+    const int rc = w8_scratch(p, dev, cus, s, need, &ws);
     if (rc != TPAMD_OK) return rc;
     if (ws == nullptr) return TPAMD_OK;
     float *part = static_cast<float *>(ws);

@@ -323,3 +323,24 @@ def test_small_calls_of_several_ranks(shape, n, dtype):
     freqs, positions = draws(n, 32, dtype=torch.float32, seed=2), [torch.arange(rows * 3, device=DEV).view(rows, 3) + 7 * r for r in range(n)]
     for f, p, got in zip(freqs, positions, _native.rope_tables_ranks([(f, p, 1.5, dtype) for f, p in zip(freqs, positions)])):
         assert all(torch.equal(x, y) for x, y in zip(got, _native.rope_tables(f, p, 1.5, dtype)))
+
+
+@pytest.mark.parametrize("rows", [60, 61, 64])
+def test_two_ranks_whose_partial_sums_outgrow_a_streams_buffer_take_their_own_kernels(rows):
+    """Nine planes of 16384 columns for each of two ranks: 71.3 MB of scratch memory hold them up to 60 rows."""
+    cols, K, n_out, calls = 16384, 8192, 41, []
+    for r in range(2):
+        g = torch.Generator(device=DEV).manual_seed(r)
+        q = torch.randint(-127, 128, (cols, K), device=DEV, generator=g, dtype=torch.int8)
+        idx = torch.randperm(K, device=DEV, generator=g)[:n_out].sort().values.to(torch.int32)
+        calls.append((draws(1, rows, K, dtype=torch.float16, seed=r)[0], q, torch.rand(cols, device=DEV, generator=g) * 1e-3, idx,
+                      draws(1, cols, n_out, dtype=torch.float16, seed=3 + r)[0], None))
+    _native.linear_w8(calls[0][0][:8], *calls[0][1:])  # this stream's buffer has the usual size
+    assert 9 * 60 * cols * 4 * 2 <= _native.scratch_of_stream(DEV)[1] < 9 * 61 * cols * 4 * 2
+    for y, call in zip(_native.linear_w8_ranks(calls), calls):
+        alone = _native.linear_w8(*call)
+        x, q, scale, idx, w_out, _ = call
+        want = x.double() @ (q.double() * scale.double()[:, None]).t() + x[:, idx.long()].double() @ w_out.double().t()
+        close(y, want.float(), torch.float16)
+        if rows > 60:  # the same kernel, which adds up in the same order
+            assert torch.equal(y, alone)
