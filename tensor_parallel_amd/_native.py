@@ -871,6 +871,7 @@ def causal_mask_ranks(calls: Sequence[tuple]) -> list:
 def add_ranks(calls: Sequence[tuple]) -> list:
     """a + b of several ranks, tensors of one shape and dtype."""
     a, b = calls[0]
+    require_device(a, "add_ranks")
     if a.shape != b.shape or a.dtype != b.dtype or a.get_device() != b.get_device():
         raise ValueError(f"add_ranks: {tuple(a.shape)} {a.dtype} and {tuple(b.shape)} {b.dtype} do not fit")
     xs, rs = _contiguous([c[0] for c in calls]), _contiguous([c[1] for c in calls])
@@ -884,6 +885,7 @@ def add_ranks(calls: Sequence[tuple]) -> list:
 def advance_ranks(calls: Sequence[tuple]) -> list:
     """count.add_(by) for the int64 counts of several ranks."""
     count, by = calls[0]
+    require_device(count, "advance_ranks")
     if count.dtype != torch.int64 or count.numel() != 1:
         raise ValueError(f"advance_ranks: a count must be one int64, got {tuple(count.shape)} {count.dtype}")
     if len({c.data_ptr() for c, _ in calls}) < len(calls):  # ranks that share a count: one after the other

@@ -407,6 +407,6 @@ def add(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
 
 def advance(count: torch.Tensor, by: int) -> torch.Tensor:
     """count.add_(by)."""
-    if count.dtype is not torch.int64 or count.numel() != 1:
+    if count.dtype is not torch.int64 or count.numel() != 1 or not count.is_cuda or not _native.plain_call(count):
         return count.add_(by)
     return _call(torch.Tensor.add_, _native.advance_ranks, (count,), (by,))

@@ -309,3 +309,17 @@ def test_models_of_the_libraries_meet():
     for model in (llama, falcon, opt):
         install_shard_kernels(model)
         assert not together.keeps_turn(model)
+
+
+def test_counts_in_host_memory_are_advanced_there(monkeypatch):
+    """A static cache's count that a program keeps on the host (a prompt of several positions reads it there) has no address for a kernel."""
+    monkeypatch.setattr(_native, "advance_ranks", lambda calls: pytest.fail("a kernel was given an address in host memory"))
+    counts = [torch.tensor(10 + r) for r in range(2)]
+    assert run(*[lambda r: together.advance(counts[r], 3)] * 2) == counts and [int(c) for c in counts] == [13, 14]
+
+
+@pytest.mark.parametrize("call", ["advance_ranks", "add_ranks"])
+def test_small_calls_of_several_ranks_want_device_memory(call):
+    items = [(torch.tensor(1), 1)] * 2 if call == "advance_ranks" else [(torch.ones(8), torch.ones(8))] * 2
+    with pytest.raises(_native.NativeLibraryError, match="HIP device"):
+        getattr(_native, call)(items)
