@@ -101,7 +101,7 @@ class ShardLinearW8(nn.Module):
         few = input.numel() <= together.W8_TOGETHER_ROWS * input.shape[-1]
         alone = functools.partial(_native.linear_w8, *operands, act=act)
         return product_in_context(self, input, self.out_features, (input,), functools.partial(together.linear_w8, *operands, act) if few else alone, alone,
-                                  (lambda rank: together.linear_w8_sum(*operands, rank)) if few and act == _native.ACT_NONE else None, learned=False)
+                                  (lambda rank, op: together.linear_w8_sum(*operands, rank, op)) if few and act == _native.ACT_NONE else None, learned=False)
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "

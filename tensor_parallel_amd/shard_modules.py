@@ -48,13 +48,13 @@ def linear_in_context(module: nn.Module, x: torch.Tensor, w: torch.Tensor, bias)
     """`tpamd_linear` for a shard's Linear; see `product_in_context`."""
     xd, wd, b = x.detach(), w.detach(), None if bias is None else bias.detach()
     return product_in_context(module, x, w.shape[0], (x, w, bias), lambda: together.linear(xd, wd, b), lambda **more: _native.linear(xd, wd, b, **more),
-                              lambda rank: together.linear_sum(xd, wd, b, rank))
+                              lambda rank, op: together.linear_sum(xd, wd, b, rank, op))
 
 
 def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs: tuple, with_peers, alone, summed, learned: bool = True) -> torch.Tensor:
     """A shard's Linear with `columns` outputs, made by with_peers() or, with an addend, alone(addend=, copy=). Inside a wrapped module whose output goes to a
     "sum" rule (collectives.SumContext) the Linear that was seen to produce that output hands over the sum: two ranks that meet in it get it from
-    summed(rank) (`tpamd_linear_sum_ranks`; None: not to be had), else the rank that comes last adds the partial sums already waiting in
+    summed(rank, op) (`tpamd_linear_sum_ranks`; None: not to be had), else the rank that comes last adds the partial sums already waiting in
     the reduction, in its epilogue (`tpamd_linear_add`): the product rounded to the dtype, then one rounded add, which
     is the same arithmetic as the reduction kernel's step. `learned`: having been seen to produce it is enough (see _may_hold_sum)."""
     from .collectives import current_sum_context
@@ -71,7 +71,7 @@ def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs:
                                "after adding the waiting partial sums; set TPAMD_FUSE_SUM=0")
         waiting = ctx.op.addend_for(ctx.rank)
         if waiting is None and summed is not None and ctx.op.world_size == 2 and _is_last_child(module, ctx.owner.tp_wrapped_module):
-            out = summed(ctx.rank)
+            out = summed(ctx.rank, ctx.op)
         if out is not None:
             out = _guard(out, *inputs)
             ctx.fused_mask, ctx.fused_whole = 3, True
@@ -132,7 +132,7 @@ def gathered_linear(module: nn.Module, op, rank: int, args, kwargs):
     x, w, bias = args[0], module.weight, module.bias
     if not _native.plain_call(x, w) or not x.is_cuda or op.dim not in (-1, x.dim() - 1) or x.dtype != w.dtype:
         return None
-    whole = together.linear_gathered(x.detach(), w.detach(), None if bias is None else bias.detach(), rank, op.world_size)
+    whole = together.linear_gathered(x.detach(), w.detach(), None if bias is None else bias.detach(), rank, op.world_size, op)
     return None if whole is None else _guard(whole, x, w, bias)
 
 

@@ -234,7 +234,7 @@ class GreenTurn:
         """one(*tensors, *more, *own), made as many([...]) for all ranks that come with tensors of the same forms and the same `more`, in the order in
         which they came. A rank whose peers do not come (they wait elsewhere or have returned) makes the call alone (`_part`)."""
         for meeting in self.open:
-            if meeting.one is one and meeting.more == more and _alike(meeting.calls[0][0], tensors):
+            if meeting.one is one and meeting.many is many and meeting.more == more and _alike(meeting.calls[0][0], tensors):
                 break
         else:
             meeting = _Meeting(one, many, more)
@@ -298,7 +298,7 @@ def _not_together(*_: Any) -> None:
 
 
 def _linear_sum(calls: List[tuple]) -> Sequence[torch.Tensor]:
-    ranks = [call[:3] for call in sorted(calls, key=lambda call: call[3])]
+    ranks = [call[:3] for call in sorted(calls, key=lambda call: call[-1])]
     sums = _native.linear_sum_ranks(ranks)
     if sums is None:  # operands that the kernels do not take, or no scratch memory
         first = _native.linear(*ranks[0])
@@ -307,12 +307,13 @@ def _linear_sum(calls: List[tuple]) -> Sequence[torch.Tensor]:
     return sums
 
 
-def linear_sum(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], rank: int) -> Optional[torch.Tensor]:
-    """The sum of two ranks' Linears, a tensor of its own for each; None where this rank is on its own or two launches are faster."""
+def linear_sum(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], rank: int, op: Any = None) -> Optional[torch.Tensor]:
+    """The sum of two ranks' Linears, a tensor of its own for each; None where this rank is on its own or two launches are faster. `op`: the collective that
+    it is for, which both ranks have to name."""
     K = x.shape[-1]
     if K == 0 or w.dim() != 2 or x.dtype is torch.float32 or not _native.linear_sum_pays(x.numel() // K, w.shape[0], K, x.dtype):
         return None
-    return _call(_not_together, _linear_sum, (x, w, bias), (), (rank,))
+    return _call(_not_together, _linear_sum, (x, w, bias), (op,), (rank,))
 
 
 # Up to this many rows the int8 kernels take two ranks in one launch, and a sum that those cannot add up is a launch of its own behind them; above, a rank's Linear
@@ -326,7 +327,7 @@ def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, outlier_id
 
 
 def _linear_w8_sum(calls: List[tuple]) -> Sequence[torch.Tensor]:
-    ranks = [call[:6] for call in sorted(calls, key=lambda call: call[6])]
+    ranks = [call[:6] for call in sorted(calls, key=lambda call: call[-1])]
     sums = _native.linear_w8_sum_ranks(ranks)
     if sums is None:
         parts = _native.linear_w8_ranks(ranks)
@@ -336,19 +337,19 @@ def _linear_w8_sum(calls: List[tuple]) -> Sequence[torch.Tensor]:
 
 
 def linear_w8_sum(x: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, outlier_idx: Optional[torch.Tensor], w_out: Optional[torch.Tensor],
-                  bias: Optional[torch.Tensor], rank: int) -> Optional[torch.Tensor]:
-    return _call(_not_together, _linear_w8_sum, (x, wq, scale, outlier_idx, w_out, bias), (), (rank,))
+                  bias: Optional[torch.Tensor], rank: int, op: Any = None) -> Optional[torch.Tensor]:
+    return _call(_not_together, _linear_w8_sum, (x, wq, scale, outlier_idx, w_out, bias), (op,), (rank,))
 
 
 def _gather(calls: List[tuple]) -> Sequence[torch.Tensor]:
-    return _native.linear_gather_ranks([call[:3] for call in sorted(calls, key=lambda call: call[3])])  # (every rank's result is the same)
+    return _native.linear_gather_ranks([call[:3] for call in sorted(calls, key=lambda call: call[-1])])  # (every rank's result is the same)
 
 
-def linear_gathered(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], rank: int, world: int) -> Optional[torch.Tensor]:
-    """The Linears of two ranks with their results side by side, a whole one for each, in one launch; None where this rank is on its own."""
+def linear_gathered(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], rank: int, world: int, op: Any = None) -> Optional[torch.Tensor]:
+    """The Linears of two ranks with their results side by side, a whole one for each, in one launch; None where this rank is on its own. `op` as above."""
     if world != 2 or x.numel() == 0:
         return None
-    return _call(_not_together, _gather, (x, w, bias), (), (rank,))
+    return _call(_not_together, _gather, (x, w, bias), (op,), (rank,))
 
 
 def swiglu_up(x: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor) -> torch.Tensor:

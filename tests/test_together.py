@@ -323,3 +323,22 @@ def test_small_calls_of_several_ranks_want_device_memory(call):
     items = [(torch.tensor(1), 1)] * 2 if call == "advance_ranks" else [(torch.ones(8), torch.ones(8))] * 2
     with pytest.raises(_native.NativeLibraryError, match="HIP device"):
         getattr(_native, call)(items)
+
+
+@pytest.mark.parametrize("kinds", [("sum", "sum"), ("gather", "gather"), ("sum", "gather"), ("gather", "sum")])
+def test_ranks_at_different_collectives_are_not_taken_for_one_call(monkeypatch, kinds):
+    """Linears of equal forms, one rank's for one collective and the other's for another."""
+    for name in ("linear_sum_ranks", "linear_gather_ranks"):
+        monkeypatch.setattr(_native, name, lambda items: pytest.fail("two collectives were taken for one"))
+    monkeypatch.setattr(_native, "linear_sum_pays", lambda *_: True)
+    ops = [object(), object()]
+
+    def body(r):
+        if kinds[r] == "sum":
+            return together.linear_sum(*operands(r), None, r, ops[r])
+        return together.linear_gathered(*operands(r), None, r, 2, ops[r])
+
+    assert run(body, body) == [None, None]
+    if kinds[0] != kinds[1]:  # two kinds for one op, which no rule makes
+        ops[1] = ops[0]
+        assert run(body, body) == [None, None]
