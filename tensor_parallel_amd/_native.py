@@ -1020,6 +1020,11 @@ def attention_decode_rope_ranks(calls: Sequence[tuple]) -> list:
     return [out for _, _, out in keep]
 
 
+def rope_takes(B: int, S: int, heads: int, D: int) -> bool:
+    """Whether `rope` rotates `heads` query and key heads of this many sequences and positions in a launch (which has fewer than 2^32 threads)."""
+    return B < 1 << 24 and S < 1 << 24 and heads < 1 << 16 and B * S * ((heads * (D // 16) + 255) // 256) < 1 << 24
+
+
 def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> tuple:
     """Rotary embedding of whole sequences in one launch: q [B, S, Hq, D], k [B, S, Hkv, D] (views of projection outputs), cos / sin [B or 1, S, D];
     returns them rotated, as [B, Hq, S, D] and [B, Hkv, S, D]. Arithmetic as in `rope_append`."""

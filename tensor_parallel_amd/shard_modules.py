@@ -282,7 +282,7 @@ def _llama_attention_forward(self, hidden_states: torch.Tensor, position_embeddi
     heads = (*hidden_states.shape[:2], -1, self.head_dim)
     q, k, v = self.q_proj(hidden_states).view(heads), self.k_proj(hidden_states).view(heads), self.v_proj(hidden_states).view(heads)
     if type(q) is torch.Tensor and type(k) is torch.Tensor and q.dtype == k.dtype == cos.dtype and not (q.data_ptr() % 16 or k.data_ptr() % 16 or cos.data_ptr() % 16 or sin.data_ptr() % 16) \
-            and not any(stride % 8 for t in (q, k, cos, sin) for stride in t.stride()[:-1]) and q.numel() + k.numel() < 1 << 32:
+            and not any(stride % 8 for t in (q, k, cos, sin) for stride in t.stride()[:-1]) and _native.rope_takes(*q.shape[:2], q.shape[2] + k.shape[2], self.head_dim):
         q, k = _native.rope(q, k, cos, sin)
     else:
         q, k = names["apply_rotary_pos_emb"](q.transpose(1, 2), k.transpose(1, 2), cos, sin)

@@ -311,3 +311,50 @@ def test_rotary_tables_take_the_arguments_of_the_modules_own_forward(kernels):
         for got, want in zip(model.rotary_emb(x=x, position_ids=position_ids, **kwargs), own.rotary_emb(x=x, position_ids=position_ids, **kwargs)):
             assert torch.equal(got, want)
     assert kernels == ["rope_tables"]
+
+
+@pytest.mark.parametrize("B,S,heads,D,takes", [(1, 5, 2, 64, True), (1, 2 ** 24 - 1, 2, 64, True), (1, 2 ** 24, 2, 64, False), (2 ** 24, 1, 4, 128, False), (2 ** 12, 2 ** 12, 2, 64, False),
+                                               (2 ** 12, 2 ** 12 - 1, 64, 64, True), (2 ** 12, 2 ** 12 - 1, 65, 64, False), (2 ** 11, 2 ** 12 - 1, 64, 128, True),
+                                               (2 ** 11, 2 ** 12 + 1, 64, 128, False), (1, 1, 2 ** 16 - 1, 128, True), (1, 1, 2 ** 16, 128, False)])
+def test_rope_takes_what_its_launch_holds(B, S, heads, D, takes):
+    """The library's own answer for these sizes, asked with addresses that it refuses in the next step (8 is no multiple of 16)."""
+    import ctypes
+
+    assert _native.rope_takes(B, S, heads, D) == takes
+    rc = _native.lib().tpamd_rope(8, 8, 8, 8, 8, 8, B, S, heads // 2, heads - heads // 2, D, (ctypes.c_int64 * 14)(*[8] * 14), _native.BF16, None)
+    assert rc == (-2 if takes else -1), _native.lib().tpamd_last_error()
+
+
+@pytest.mark.parametrize("takes", [False, True])
+def test_an_attention_that_is_too_long_for_the_rope_kernel_keeps_torchs_rotation(kernels, monkeypatch, takes):
+    from tensor_parallel_amd import attention
+
+    torch.manual_seed(0)
+    config = tf.LlamaConfig(vocab_size=32, hidden_size=128, intermediate_size=48, num_hidden_layers=1, num_attention_heads=2)
+    model = tf.LlamaModel(config).eval().requires_grad_(False).bfloat16()
+    shard_modules.install_shard_kernels(model)
+    model.config._attn_implementation = attention.register()
+    rotated = []
+
+    def attend(module, q, k, v, mask, **kwargs):
+        rotated.append((q, k))
+        return q.transpose(1, 2), None
+
+    def rope(q, k, cos, sin):
+        kernels.append("rope")
+        names = shard_modules._globals_of(type(model.layers[0].self_attn)._tp_base.forward)
+        return names["apply_rotary_pos_emb"](q.transpose(1, 2), k.transpose(1, 2), cos, sin)
+
+    monkeypatch.setattr(attention, "attention_forward", attend)
+    tf.modeling_utils.ALL_ATTENTION_FUNCTIONS.register(attention.IMPLEMENTATION_NAME, attend)
+    monkeypatch.setattr(_native, "rope", rope)
+    monkeypatch.setattr(_native, "rope_takes", lambda B, S, heads, D: (B, S, heads, D) == (2, 5, 4, 64) and takes)
+    monkeypatch.setattr(_native, "linear", lambda x, w, b=None, **_: torch.nn.functional.linear(x, w, b))
+    try:
+        x, position_ids = torch.randn(2, 5, 128).bfloat16(), torch.arange(5)[None]
+        with torch.no_grad():
+            model.layers[0].self_attn(x, position_embeddings=model.rotary_emb(x, position_ids), attention_mask=None)
+    finally:
+        monkeypatch.undo()
+        attention.register()
+    assert kernels.count("rope") == takes and len(rotated) == 1
