@@ -102,6 +102,8 @@ class TensorParallelWrapper(nn.Module):
     """Holds one module as `tp_wrapped_module`; calls go through the rank's rules, every other attribute is the
     wrapped module's."""
 
+    _gather_op = None  # of a wrapper that was saved before there was one
+
     def __init__(self, module: nn.Module, input_actions: MappedActions, output_actions: MappedActions, *, rank: int, world_size: int):
         super().__init__()
         self.tp_wrapped_module = module

@@ -816,3 +816,17 @@ def test_shards_with_fused_modules_can_be_pickled_and_copied():
         x = torch.randn(2, 32)
         with torch.no_grad():
             assert torch.equal(other.norm(x), model.norm(x))
+
+
+def test_a_wrapper_that_was_saved_without_a_gather_runs():
+    """A pickled wrapper whose rules hold no collective, from before wrappers knew which gather their module's output goes to."""
+    import pickle
+
+    import torch
+
+    from tensor_parallel_amd.wrapper import TensorParallelWrapper
+
+    wrapper = TensorParallelWrapper(torch.nn.ReLU(), {}, {}, rank=0, world_size=2)
+    del wrapper.__dict__["_gather_op"]
+    x = torch.randn(3, 4)
+    assert torch.equal(pickle.loads(pickle.dumps(wrapper))(x), x.relu())
