@@ -1097,9 +1097,7 @@ def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale_: torch.Tensor, outlier_i
               w_out: Optional[torch.Tensor], bias: Optional[torch.Tensor] = None, act: int = ACT_NONE,
               addend: Optional[torch.Tensor] = None, copy: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Weight-only int8 Linear with outlier columns kept in the activation dtype. `addend` and `copy` as in `linear`."""
-    x2, wq, scale_, outlier_idx, w_out, b = _w8_operands(x, wq, scale_, outlier_idx, w_out, bias)
-    (M, K), N = x2.shape, wq.shape[0]
-    n_out = 0 if outlier_idx is None else outlier_idx.numel()
+    (x2, wq, scale_, outlier_idx, w_out, b), (M, N, K, n_out) = _w8_operands(x, wq, scale_, outlier_idx, w_out, bias)
     if addend is not None and (addend.dtype != x.dtype or addend.device != x.device or addend.numel() != M * N or addend.shape[-1] != N):
         raise ValueError("linear_w8: addend must have the shape, dtype and device of the result")
     if copy is not None and (addend is None or copy.dtype != x.dtype or copy.device != x.device or copy.numel() != M * N or not copy.is_contiguous()):
@@ -1125,11 +1123,12 @@ def linear_w8(x: torch.Tensor, wq: torch.Tensor, scale_: torch.Tensor, outlier_i
 
 
 def _w8_operands(x, wq, scale_, outlier_idx, w_out, bias) -> tuple:
-    """The checked operands of an int8 Linear as the library takes them (no outlier columns: None)."""
+    """The checked operands of an int8 Linear as the library takes them (no outlier columns: None), and M, N, K and the number of outlier columns."""
     require_device(x, "linear_w8")
-    if wq.dtype != torch.int8 or scale_.dtype != torch.float32:
+    dtype = x.dtype
+    if wq.dtype is not torch.int8 or scale_.dtype is not torch.float32:
         raise TypeError("linear_w8: wq must be int8 and scale float32")
-    if x.dtype not in (torch.bfloat16, torch.float16):
+    if dtype is not torch.bfloat16 and dtype is not torch.float16:
         raise TypeError(f"linear_w8: x must be bfloat16 or float16, got {x.dtype}")
     x2 = _as_2d(x)
     M, K = x2.shape
@@ -1139,35 +1138,34 @@ def _w8_operands(x, wq, scale_, outlier_idx, w_out, bias) -> tuple:
     if scale_.shape != (N,):
         raise ValueError(f"linear_w8: scale must have shape [{N}], got {tuple(scale_.shape)}")
     index = x.get_device()
-    if index < 0 or wq.get_device() != index or scale_.get_device() != index or any(t is not None and t.get_device() != index for t in (outlier_idx, w_out, bias)):
+    if (index < 0 or wq.get_device() != index or scale_.get_device() != index or outlier_idx is not None and outlier_idx.get_device() != index
+            or w_out is not None and w_out.get_device() != index or bias is not None and bias.get_device() != index):
         for name, t in (("wq", wq), ("scale", scale_), ("outlier_idx", outlier_idx), ("w_out", w_out), ("bias", bias)):
             if t is not None and t.device != x.device:
                 raise ValueError(f"linear_w8: x is on {x.device}, {name} on {t.device}")
-    if bias is not None and (bias.shape != (N,) or bias.dtype != x.dtype):
-        raise ValueError("linear_w8: bias must have shape [N] and the dtype of x")
-    wq = wq.contiguous()
-    n_out = 0 if outlier_idx is None else int(outlier_idx.numel())
-    if n_out:
-        if outlier_idx.dtype != torch.int32 or w_out is None or w_out.shape != (N, n_out) or w_out.dtype != x.dtype:
-            raise ValueError("linear_w8: outlier_idx must be int32 [n_out] and w_out [N, n_out] in the dtype of x")
-        if n_out > K:
-            raise ValueError(f"linear_w8: {n_out} outlier columns for K = {K}")
-        w_out = w_out.contiguous()
-        outlier_idx = outlier_idx.contiguous()
-    return x2, wq, scale_.contiguous(), outlier_idx if n_out else None, w_out if n_out else None, None if bias is None else bias.contiguous()
+    if bias is not None:
+        if bias.shape != (N,) or bias.dtype is not dtype:
+            raise ValueError("linear_w8: bias must have shape [N] and the dtype of x")
+        bias = bias.contiguous()
+    n_out = 0 if outlier_idx is None else outlier_idx.numel()
+    if n_out == 0:
+        return (x2, wq.contiguous(), scale_.contiguous(), None, None, bias), (M, N, K, 0)
+    if outlier_idx.dtype is not torch.int32 or w_out is None or w_out.shape != (N, n_out) or w_out.dtype is not dtype:
+        raise ValueError("linear_w8: outlier_idx must be int32 [n_out] and w_out [N, n_out] in the dtype of x")
+    if n_out > K:
+        raise ValueError(f"linear_w8: {n_out} outlier columns for K = {K}")
+    return (x2, wq.contiguous(), scale_.contiguous(), outlier_idx.contiguous(), w_out.contiguous(), bias), (M, N, K, n_out)
 
 
 def _w8_ranks(calls: Sequence[tuple]) -> tuple:
     ranks, keep = (W8Rank * len(calls))(), []
     for rank, call in zip(ranks, calls):
-        ops = _w8_operands(*call[:6])
-        x2, wq = ops[:2]
-        (M, K), N = x2.shape, wq.shape[0]
+        ops, (M, N, K, n_out) = _w8_operands(*call[:6])
+        x2 = ops[0]
         y = torch.empty((M, N), dtype=x2.dtype, device=x2.device)
         keep.append((ops, y))
         rank.x, rank.wq, rank.scale, rank.outlier_idx, rank.w_out, rank.bias = (None if t is None else t.data_ptr() for t in ops)
         rank.y = y.data_ptr()
-    n_out = 0 if ops[3] is None else int(ops[3].numel())
     return ranks, keep, (n_out, M, N, K, _ld(x2), K, max(n_out, 1), N, dtype_code(x2.dtype))
 
 

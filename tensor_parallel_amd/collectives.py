@@ -11,7 +11,6 @@ before the reduction by the stream itself; the host-side barrier only makes sure
 """
 from __future__ import annotations
 
-import contextvars
 import os
 import threading
 from typing import Any, Callable, List, Optional
@@ -21,7 +20,7 @@ import torch
 from . import _native
 from .shard_modules import _guard, hands_through
 from .slicing import concat_dim
-from .together import GreenTurn, current_turn, set_turn_lock  # noqa: F401 - the names under which forwards look them up
+from .together import GreenTurn, current_sum_context, current_turn, pop_sum_context, push_sum_context, set_turn_lock  # noqa: F401 - the names under which forwards look them up
 
 RENDEZVOUS_TIMEOUT_S = 600.0
 
@@ -62,10 +61,9 @@ class Turn:
 # A module whose output rule is "sum" usually ends in its row-parallel Linear (attention output projection, MLP down
 # projection). The rank that reaches that Linear while the partials of the other ranks are already waiting in the op
 # can add them in the GEMM's epilogue (`tpamd_linear_add`) instead of leaving a separate M x N pass to the reduction
-# kernel. A wrapper with such a rule publishes a SumContext for its rank while its module runs; shard Linears
+# kernel. A wrapper with such a rule publishes a SumContext for its rank while its module runs (together.push_sum_context); shard Linears
 # consult it (shard_modules.linear_in_context); the op learns from it what the value it is handed already contains.
 FUSE_SUM = os.environ.get("TPAMD_FUSE_SUM", "1") != "0"
-_contexts: contextvars.ContextVar = contextvars.ContextVar("tpamd_sum_contexts", default=None)
 
 
 class SumContext:
@@ -101,23 +99,6 @@ class SumContext:
         self.fused_linear.__dict__["_tp_feeds_sum"] = None
         return RuntimeError("tensor_parallel_amd: a row-parallel Linear added the other ranks' partial sums in its epilogue, but "
                             f"{why}; set TPAMD_FUSE_SUM=0 to keep the sum in its own kernel")
-
-
-def push_sum_context(ctx: Optional[SumContext]) -> None:
-    stack = _contexts.get()
-    if stack is None:
-        stack = []
-        _contexts.set(stack)
-    stack.append(ctx)
-
-
-def pop_sum_context() -> None:
-    _contexts.get().pop()
-
-
-def current_sum_context() -> Optional[SumContext]:
-    stack = _contexts.get()
-    return stack[-1] if stack else None
 
 
 def _rendezvous(barrier: threading.Barrier, timeout: float) -> None:

@@ -24,7 +24,7 @@ from torch import nn
 
 from . import _native, together
 from . import shard_modules
-from .shard_modules import is_conv1d, product_in_context
+from .shard_modules import _guard, is_conv1d, product_in_context
 
 OutlierChoice = Union[None, Mapping[str, Sequence[int]], Callable[[str, nn.Module], Optional[Sequence[int]]]]
 
@@ -95,11 +95,14 @@ class ShardLinearW8(nn.Module):
     def _product(self, input: torch.Tensor, act: int) -> torch.Tensor:  # noqa: A002
         if input.dtype != self.dtype:
             raise TypeError(f"ShardLinearW8: the input is {input.dtype}, the Linear was quantised for {self.dtype}")
-        idx = self.outlier_idx
+        tensors = self._buffers
+        idx = tensors["outlier_idx"]
         n_out = idx.numel()
-        operands = (input.detach(), self.wq, self.scale, idx if n_out else None, self.w_out if n_out else None, self.bias)
+        operands = (input.detach(), tensors["wq"], tensors["scale"], idx if n_out else None, tensors["w_out"] if n_out else None, tensors["bias"])
         few = input.numel() <= together.W8_TOGETHER_ROWS * input.shape[-1]
-        alone = functools.partial(_native.linear_w8, *operands, act=act)
+        if together.current_sum_context() is None:  # (what product_in_context does then: a prompt's host calls set its pace)
+            return _guard(together.linear_w8(*operands, act) if few else _native.linear_w8(*operands, act), input)
+        alone = functools.partial(_native.linear_w8, *operands, act)
         return product_in_context(self, input, self.out_features, (input,), functools.partial(together.linear_w8, *operands, act) if few else alone, alone,
                                   (lambda rank, op: together.linear_w8_sum(*operands, rank, op)) if few and act == _native.ACT_NONE else None, learned=False)
 

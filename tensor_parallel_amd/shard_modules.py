@@ -57,9 +57,7 @@ def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs:
     summed(rank, op) (`tpamd_linear_sum_ranks`; None: not to be had), else the rank that comes last adds the partial sums already waiting in
     the reduction, in its epilogue (`tpamd_linear_add`): the product rounded to the dtype, then one rounded add, which
     is the same arithmetic as the reduction kernel's step. `learned`: having been seen to produce it is enough (see _may_hold_sum)."""
-    from .collectives import current_sum_context
-
-    ctx = current_sum_context()
+    ctx = together.current_sum_context()
     if ctx is None:
         return _guard(with_peers(), *inputs)
     key = id(module)

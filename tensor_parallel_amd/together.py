@@ -46,6 +46,27 @@ def current_turn():
     return _turn.get()
 
 
+# The calls of wrapped modules that a rank is in (collectives.SumContext; None: one whose output goes to no foldable sum), innermost last.
+_contexts: contextvars.ContextVar = contextvars.ContextVar("tpamd_sum_contexts", default=None)
+
+
+def push_sum_context(ctx) -> None:
+    stack = _contexts.get()
+    if stack is None:
+        stack = []
+        _contexts.set(stack)
+    stack.append(ctx)
+
+
+def pop_sum_context() -> None:
+    _contexts.get().pop()
+
+
+def current_sum_context():
+    stack = _contexts.get()
+    return stack[-1] if stack else None
+
+
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _current_device = getattr(torch._C, "_cuda_getDevice", None)
 _grad, _inference, _autocast = torch.is_grad_enabled, torch.is_inference_mode_enabled, torch.is_autocast_enabled
