@@ -25,6 +25,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _native, together
+from .shard_modules import returned
 
 IMPLEMENTATION_NAME = "tpamd"
 
@@ -266,7 +267,7 @@ def _fused_rotary_forward(self, hidden_states: torch.Tensor, position_embeddings
     q, k, v = _project_qkv(self, hidden_states, D)
     cos, sin = position_embeddings
     out = _attend_on_cache(q, k, v, cos, sin, layer, static, getattr(self, "scaling", None), self.layer_idx)
-    return self.o_proj(out.reshape(B, S, -1)), None
+    return returned(self, _fused_rotary_forward, self.o_proj, out.reshape(B, S, -1)), None
 
 
 def _fused_falcon_forward(self, hidden_states: torch.Tensor, alibi=None, attention_mask=None, position_ids=None, layer_past=None,
@@ -294,7 +295,7 @@ def _fused_falcon_forward(self, hidden_states: torch.Tensor, alibi=None, attenti
     q, k, v = qkv[:, :, :, :per], qkv[:, :, :, per], qkv[:, :, :, per + 1]
     cos, sin = position_embeddings
     out = _attend_on_cache(q, k, v, cos, sin, layer, static, self.inv_norm_factor, self.layer_idx)
-    return self.dense(out.reshape(B, S, self.num_heads * D)), None
+    return returned(self, _fused_falcon_forward, self.dense, out.reshape(B, S, self.num_heads * D)), None
 
 
 FUSABLE_ATTENTION_CLASSES = ("LlamaAttention",)

@@ -70,13 +70,14 @@ class SumContext:
     """One call of a wrapped module whose output 0 goes to `op`, on one rank."""
 
     __slots__ = ("op", "rank", "owner", "last_linear", "last_out", "last_version", "calls", "fused_linear", "fused_out", "fused_version", "fused_mask", "fused_copy",
-                 "fused_whole")
+                 "fused_whole", "returned")
 
     def __init__(self, op: "DeviceAllReduce", rank: int, owner: Any):
         self.op, self.rank, self.owner = op, rank, owner
         self.last_linear = self.last_out = self.last_version = None
         self.fused_linear = self.fused_out = self.fused_version = self.fused_copy = None
         self.fused_whole = False  # fused_out was made as a sum over all ranks
+        self.returned = None  # the Linear whose output the module's forward said it would return as it is (shard_modules.returned)
         self.calls: dict = {}
         self.fused_mask = 0
 
@@ -90,7 +91,7 @@ class SumContext:
         elif self.last_linear is not None:
             feeds = value is self.last_out and self.calls.get(id(self.last_linear)) == 1
             if feeds:  # unchanged, which has to be known by the module's forward where changes are not counted
-                feeds = value._version == self.last_version if self.last_version is not None else hands_through(self.owner.tp_wrapped_module, self.last_linear)
+                feeds = value._version == self.last_version if self.last_version is not None else hands_through(self, self.last_linear)
             self.last_linear.__dict__["_tp_feeds_sum"] = self.owner if feeds else None
             self.owner.__dict__["_tp_sum_known"] = True
 

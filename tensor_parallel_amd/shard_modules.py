@@ -63,7 +63,7 @@ def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs:
     key = id(module)
     ctx.calls[key] = ctx.calls.get(key, 0) + 1
     out, more = None, {}
-    if module.__dict__.get("_tp_feeds_sum") is ctx.owner and ctx.owner is not None and _may_hold_sum(module, ctx.owner, learned):
+    if module.__dict__.get("_tp_feeds_sum") is ctx.owner and ctx.owner is not None and _may_hold_sum(module, ctx, learned):
         if ctx.fused_out is not None:
             raise RuntimeError("tensor_parallel_amd: the Linear that feeds a \"sum\" rule ran twice in one call of its module "
                                "after adding the waiting partial sums; set TPAMD_FUSE_SUM=0")
@@ -92,15 +92,15 @@ def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs:
     return out
 
 
-def _may_hold_sum(module: nn.Module, owner: nn.Module, learned: bool) -> bool:
+def _may_hold_sum(module: nn.Module, ctx, learned: bool) -> bool:
     """Whether a Linear's output may hold other ranks' parts already on its way to the sum: nobody who is told of it there would see or change more than this rank's
     part. Not with hooks on the Linear, on the module around it (the wrapped one) or on all modules, nor with a forward that a program has put around the
     Linear's. Then either the wrapped module is known to return it untouched, or (`learned`) it did so when it was last seen without, and a
     change shows in the tensor's version, which raises; in inference mode versions stand still."""
-    wrapped, hooks = owner.tp_wrapped_module, torch.nn.modules.module
+    wrapped, hooks = ctx.owner.tp_wrapped_module, torch.nn.modules.module
     if hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _has_hooks(module) or _has_hooks(wrapped) or "forward" in module.__dict__:
         return False
-    return learned and not torch.is_inference_mode_enabled() or hands_through(wrapped, module)
+    return learned and not torch.is_inference_mode_enabled() or hands_through(ctx, module)
 
 
 def _is_last_child(module: nn.Module, wrapped: nn.Module) -> bool:
@@ -108,9 +108,19 @@ def _is_last_child(module: nn.Module, wrapped: nn.Module) -> bool:
     return wrapped is module or any(child is module for child in wrapped._modules.values())
 
 
-def hands_through(wrapped: nn.Module, module: nn.Module) -> bool:
-    """Whether the wrapped module is this Linear, or has one of the forwards below (or the transformers one it stands in for), which return what this Linear gave."""
-    if wrapped is module:
+def returned(self: nn.Module, forward, linear: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """linear(x), which this forward of the module `self` (an attribute of it) returns as it is: a wrapper around the module is told."""
+    ctx = together.current_sum_context()
+    if ctx is not None and ctx.owner.tp_wrapped_module is self and getattr(self.__dict__.get("forward"), "__func__", None) is forward:
+        ctx.returned = linear
+    return linear(x)
+
+
+def hands_through(ctx, module: nn.Module) -> bool:
+    """Whether the wrapped module is this Linear, said that it returns what the Linear gives, or has one of the forwards below (or the transformers one it stands in
+    for), which do."""
+    wrapped = ctx.owner.tp_wrapped_module
+    if wrapped is module or ctx.returned is module:
         return True
     own, cls = wrapped.__dict__.get("forward"), type(wrapped)
     if own is not None:

@@ -169,3 +169,38 @@ def test_activation_of_a_falcon_mlp_in_the_first_linear(M, dtype, monkeypatch):
         mlp.act = torch.nn.GELU(approximate="tanh")
         mlp(x)
     assert acts == [first, *[_native.ACT_NONE] * 2, first, *[_native.ACT_NONE] * 3]
+
+
+@pytest.mark.parametrize("inference", [False, True])
+@pytest.mark.parametrize("family", ["falcon int8", "llama"])
+def test_sums_behind_fused_attentions_need_no_reduction(family, inference, monkeypatch):
+    """A prompt of 2 x 70 positions: the output projection of a fused attention hands the sum over the ranks to its wrapper, as an MLP's down projection does."""
+    from transformers import DynamicCache, FalconConfig, FalconForCausalLM, LlamaConfig, LlamaForCausalLM
+
+    from tensor_parallel_amd import _native, collectives
+
+    torch.manual_seed(0)
+    if family == "llama":
+        config = LlamaConfig(vocab_size=300, hidden_size=512, intermediate_size=768, num_hidden_layers=1, num_attention_heads=8, attn_implementation="eager")
+        model = LlamaForCausalLM(config).to(torch.bfloat16).eval()
+        model.config._attn_implementation = tp.attention.register()
+    else:
+        config = FalconConfig(vocab_size=300, hidden_size=512, num_hidden_layers=1, num_attention_heads=8, num_kv_heads=4, new_decoder_architecture=True, alibi=False, bias=False)
+        model = FalconForCausalLM(config).to(torch.bfloat16).eval()
+    split = tp.tensor_parallel(model, [DEV, DEV])
+    assert tp.attention.fuse_rotary_(split, assume_no_padding=True) == 2
+    if family != "llama":
+        quantize_linears_(split, skip=lambda name, m: "lm_head" in name)
+    ids = torch.randint(2, 300, (2, 70), device=DEV)
+    reduced, reduce = [], _native.reduce_partials
+    monkeypatch.setattr(_native, "reduce_partials", lambda parts, **more: reduced.append(len(parts)) or reduce(parts, **more))
+    with torch.inference_mode() if inference else torch.no_grad():
+        monkeypatch.setattr(collectives, "FUSE_SUM", False)
+        want = split(input_ids=ids, past_key_values=DynamicCache(), use_cache=True).logits
+        assert len(reduced) == (2 if family == "llama" else 3)  # attention, MLP and the head that shares the embedding
+        monkeypatch.setattr(collectives, "FUSE_SUM", True)
+        for _ in range(3):  # the first shows which Linears feed the sums
+            reduced.clear()
+            got = split(input_ids=ids, past_key_values=DynamicCache(), use_cache=True).logits
+            torch.testing.assert_close(got.float(), want.float(), rtol=RTOL, atol=RTOL * want.float().std().item())
+    assert reduced == []

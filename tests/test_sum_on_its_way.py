@@ -1,5 +1,7 @@
 """Row-parallel Linears that feed a "sum" rule, two ranks of one device on the CPU with the library calls stubbed: whatever a program does to such a Linear's output
 on its way to the rule, what the rule delivers is the sum of what every rank's module returned, or an error."""
+import types
+
 import pytest
 import torch
 from torch import nn
@@ -7,7 +9,7 @@ from torch import nn
 from tensor_parallel_amd import _native, together
 from tensor_parallel_amd.collectives import DeviceAllReduce
 from tensor_parallel_amd.int8 import ShardLinearW8
-from tensor_parallel_amd.shard_modules import ShardLinear
+from tensor_parallel_amd.shard_modules import ShardLinear, returned
 from tensor_parallel_amd.tensor_parallel import RANK_GREENLETS, _apply_in_greenlets
 from tensor_parallel_amd.wrapper import TensorParallelWrapper
 
@@ -186,3 +188,33 @@ def test_a_module_that_always_changes_the_output_in_place(kind, change):
     for inference in (True, True, True, False, False, True, False):
         got, want = forward(models, 4, inference)
         check(got, 2 * want if change == "scales" else want + 2)
+
+
+def own_forward(self, x):
+    """As the fused attention forwards, which return what their last Linear gives."""
+    return returned(self, own_forward, self.linear, x)
+
+
+@pytest.mark.parametrize("inference", [False, True])
+@pytest.mark.parametrize("rows", [4, 200])
+@pytest.mark.parametrize("kind", ["16 bits", "int8"])
+def test_the_linear_of_a_forward_that_returns_its_output_makes_the_sum(folds, kind, rows, inference):
+    models = shards(kind, True)
+    for m in models:
+        m.tp_wrapped_module.forward = types.MethodType(own_forward, m.tp_wrapped_module)
+    for _ in range(3):
+        check(*forward(models, rows, inference))
+    assert folds[-1] == ("whole" if kind == "16 bits" or rows <= together.W8_TOGETHER_ROWS else "addend")
+    # a program puts a forward of its own around that one
+    for m in models:
+        inner = m.tp_wrapped_module.forward
+        m.tp_wrapped_module.forward = lambda x, inner=inner: inner(x).mul_(2)
+    failures = 0
+    for _ in range(4):
+        try:
+            got, want = forward(models, rows, inference)
+            check(got, 2 * want)
+        except RuntimeError as e:
+            assert "in place" in str(e)
+            failures += 1
+    assert failures <= 2 if kind == "16 bits" and not inference else failures == 0
