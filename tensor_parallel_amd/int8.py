@@ -95,10 +95,9 @@ class ShardLinearW8(nn.Module):
     def _product(self, input: torch.Tensor, act: int) -> torch.Tensor:  # noqa: A002
         if input.dtype != self.dtype:
             raise TypeError(f"ShardLinearW8: the input is {input.dtype}, the Linear was quantised for {self.dtype}")
-        tensors = self._buffers
-        idx = tensors["outlier_idx"]
+        idx = self.outlier_idx
         n_out = idx.numel()
-        operands = (input.detach(), tensors["wq"], tensors["scale"], idx if n_out else None, tensors["w_out"] if n_out else None, tensors["bias"])
+        operands = (input.detach(), self.wq, self.scale, idx if n_out else None, self.w_out if n_out else None, self.bias)
         few = input.numel() <= together.W8_TOGETHER_ROWS * input.shape[-1]
         if together.current_sum_context() is None:  # (what product_in_context does then: a prompt's host calls set its pace)
             return _guard(together.linear_w8(*operands, act) if few else _native.linear_w8(*operands, act), input)

@@ -216,9 +216,10 @@ class ShardLayerNorm(nn.LayerNorm):
     for it (_norm_kernel_takes; derivatives, autocast, a program's own function in the place of torch's)."""
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:  # noqa: A002
-        w, b = self.weight, self.bias
+        w = self.weight
         if w is None or LAYER_NORM_FEW_ROWS * w.numel() < input.numel() < LAYER_NORM_MANY_ROWS * w.numel():
             return super().forward(input)
+        b = self.bias
         if (nn.LayerNorm.forward is not _own_layer_norm or nn.functional.layer_norm is not _functional_layer_norm or len(self.normalized_shape) != 1
                 or not _norm_kernel_takes(input, w) or torch.is_autocast_enabled()
                 or b is not None and (type(b) not in (torch.Tensor, nn.Parameter) or b.dtype != w.dtype or b.shape != w.shape or b.get_device() != w.get_device())
@@ -326,10 +327,12 @@ def _falcon_mlp_forward(self, x: torch.Tensor) -> torch.Tensor:
     Falcon-40B-shaped layer 287 -> 281 us. Over many rows the error functions at the end of each tile take longer than torch's pass over memory (1024 rows 1490 -> 1515 us)."""
     from .int8 import ShardLinearW8
 
-    own, up, act, hooks = self._tp_base.forward, self._modules.get("dense_h_to_4h"), self._modules.get("act"), torch.nn.modules.module
-    if (own is not self._tp_replaced or type(up) is not ShardLinearW8 or not _native.plain_call(x) or x.dim() == 0 or x.numel() > together.W8_TOGETHER_ROWS * x.shape[-1]
-            or "forward" in up.__dict__ or not _is_erf_gelu(act) or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _has_hooks(up) or _has_hooks(act)
-            or torch.is_grad_enabled() and x.requires_grad):
+    own = self._tp_base.forward
+    if x.dim() == 0 or x.numel() > together.W8_TOGETHER_ROWS * x.shape[-1]:
+        return own(self, x)
+    up, act, hooks = self._modules.get("dense_h_to_4h"), self._modules.get("act"), torch.nn.modules.module
+    if (own is not self._tp_replaced or type(up) is not ShardLinearW8 or not _native.plain_call(x) or "forward" in up.__dict__ or not _is_erf_gelu(act)
+            or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _has_hooks(up) or _has_hooks(act) or torch.is_grad_enabled() and x.requires_grad):
         return own(self, x)
     return self.dense_4h_to_h(up._product(x, _native.ACT_GELU))
 
