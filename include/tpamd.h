@@ -353,7 +353,8 @@ int tpamd_swiglu_up_ranks(int n, const void *const *x_dev, const void *const *wg
  * way (many rows, short rows, fp32) or a stream has no scratch memory. */
 int tpamd_linear_sum_ranks(const void *const *x_dev, const void *const *w_dev, const void *const *bias_dev /* NULL: none */, void *const *y_dev,
                            int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int dtype, void *stream);
-/* 1 where tpamd_linear_sum_ranks takes aligned operands of these sizes, else 0 (host arithmetic on the sizes and the tuning knobs). */
+/* 1 where tpamd_linear_sum_ranks takes aligned operands of these sizes, else 0 (host arithmetic on the sizes, the tuning knobs and the current
+ * device's number of CUs; a stream without scratch memory is not looked at). */
 int tpamd_linear_sum_pays(int64_t M, int64_t N, int64_t K, int dtype);
 int tpamd_rms_norm_ranks(int n, const void *const *x_dev, const void *const *w_dev, void *const *y_dev, int64_t rows, int64_t D,
                          int64_t ldx, int64_t ldy, float eps, int dtype, void *stream);

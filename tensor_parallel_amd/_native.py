@@ -496,7 +496,7 @@ def _ld(t: torch.Tensor) -> int:
 def reload_tuning() -> None:
     """Make the library read its TPAMD_* environment variables again (it reads them once, at load time)."""
     lib().tpamd_tuning_reload()
-    linear_sum_pays.cache_clear()
+    _linear_sum_pays.cache_clear()
 
 
 def scratch_of_stream(device: torch.device, stream_ptr: Optional[int] = None) -> tuple:
@@ -589,10 +589,18 @@ def linear_ranks(calls: Sequence[tuple]) -> list:
     return ys
 
 
+def linear_sum_pays(M: int, N: int, K: int, dtype: torch.dtype, index: Optional[int] = None) -> bool:
+    """Whether `linear_sum_ranks` has a launch for these sizes that is faster than two (a rule on sizes, tuning knobs and the CUs of HIP device `index`, of the
+    current one if None)."""
+    if index is None:
+        index = torch.cuda.current_device()
+    return index >= 0 and _linear_sum_pays(M, N, K, dtype, index)
+
+
 @functools.lru_cache(maxsize=4096)
-def linear_sum_pays(M: int, N: int, K: int, dtype: torch.dtype) -> bool:
-    """Whether `linear_sum_ranks` has a launch for these sizes that is faster than two (a rule on sizes and tuning knobs)."""
-    return lib().tpamd_linear_sum_pays(M, N, K, dtype_code(dtype)) == 1
+def _linear_sum_pays(M: int, N: int, K: int, dtype: torch.dtype, index: int) -> bool:
+    with _on_device(torch.device("cuda", index)):
+        return lib().tpamd_linear_sum_pays(M, N, K, dtype_code(dtype)) == 1
 
 
 def linear_sum_ranks(calls: Sequence[tuple]) -> Optional[list]:

@@ -1,5 +1,6 @@
 // C ABI entry points for the shard Linears, plus the library's error plumbing.
 #include "common.h"
+#include "gemm_model.h"
 
 #include <string.h>
 
@@ -306,22 +307,17 @@ extern "C" int tpamd_linear_gather_ranks(int n, const void *const *x_dev, const 
 //   16 rows  4096 x 2048  13.4 /          10.1        4096 x 5504 25.2 /      21.5     8192 x 4096 30.6 /      27.1     5120 x 6912 34.5 / 39.3, 31.1 in tiles
 //   40 rows  4096 x 2048  19.9 /               14.0   4096 x 5504 35.3 /      26.8     8192 x 4096 38.3 /      35.4     5120 x 6912 40.8 /      32.2
 // So the row kernel takes one row, and two where they are short or few; weight streaming the others up to the row count it has for one matrix of both ranks' K,
-// unless its tiles are a ragged number of rounds; K ranges of tiles the rest while they are predicted to be faster than two launches. Two launches keep
-// matrices that the kernels for one of them stream as fast: one of long rows at 1 row (4096 x 8192: 24.9, 26.2 in one; ragged 5120 x 5504: 24.1, 26.8), ragged ones
-// between K = 2048 and 3072 at 2 (4544 x 2752: 15.1, 15.8) and of 1.5 rounds or more from K = 3072 on up to 16 (7168 x 4096 at 8 rows: 25.1, 29.1). On 372 random
-// shapes (1024-8192 columns, K 1024-8192, 1-600 rows) one launch took 0.77 of the time of two in the geometric mean, and was slower on the 18 that these exceptions
-// and the margin of sum128_pays take out and on 5120 x 2048 at 3 rows (13.2, 13.7).
+// unless its tiles are a ragged number of rounds; K ranges of tiles the rest, above 64 rows while they are predicted to be faster than two launches. What stays in two
+// launches and why: sum_in_two_launches (gemm_model.h).
 enum SumPath { SUM_NONE, SUM_ROWS8, SUM_ROWS16, SUM_STREAM, SUM_TILES };
 static int sum_path(int64_t M, int64_t N, int64_t K, SumPath *path) {
     *path = SUM_NONE;
-    if (K < 1024 || M < 1) return TPAMD_OK;  // no shorter row was measured
     int dev = 0, cus = 256;
     TPAMD_HIP(hipGetDevice(&dev));
     if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
+    if (sum_in_two_launches(M, N, K, cus)) return TPAMD_OK;
     const int64_t tiles = (N + 15) / 16;
     const bool ragged = tiles > cus && tiles % cus != 0;
-    if (M == 1 && K > (ragged ? 4096 : 11 * 512)) return TPAMD_OK;
-    if (ragged && ((M <= 2 && K > 2048 && K < 3072) || (M > 1 && M <= SKINNY_MAX_M && K >= 3072 && tiles * 2 >= 3ll * cus))) return TPAMD_OK;
     if (K <= 11 * 512 && (M == 1 || (M == 2 && (K <= 2048 || N <= 2048)) || (M == 3 && K <= 2048 && N <= 1024))) {
         *path = M == 1 && K > 2048 && N >= 4096 ? SUM_ROWS16 : SUM_ROWS8;
         return TPAMD_OK;
@@ -331,7 +327,7 @@ static int sum_path(int64_t M, int64_t N, int64_t K, SumPath *path) {
         if (int rc = skinny_row_limit(N, 2 * K, &rows); rc != TPAMD_OK) return rc;
     }
     if (M <= rows && !ragged) *path = SUM_STREAM;
-    else if (M <= 64 ? K % 64 == 0 && (M > 1 || !ragged) : sum128_pays(M, N, K, cus)) *path = SUM_TILES;
+    else if (M <= 64 ? K % 64 == 0 && (N + 127) / 128 * 2 <= 4ll * cus : sum128_pays(M, N, K, cus)) *path = SUM_TILES;  // (the tiles that scratch memory holds)
     return TPAMD_OK;
 }
 

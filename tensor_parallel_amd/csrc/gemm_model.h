@@ -50,6 +50,34 @@ inline bool w8_slabs_without_scratch(int64_t M, int64_t N, int64_t K, bool outli
     return M / 64.0 * (5.0 + k * (5.5 + N / 512.0)) <= 6.0 + k * (outliers ? 53.0 : 36.0);
 }
 
+// Rows, columns and K of a row-parallel Linear whose sum over two ranks stays in two launches (tpamd_linear, then tpamd_linear_add_copy) whatever the kernels for
+// both ranks could take of it: where one launch measured slower, and what was not measured. In a HIP graph on rotated weights, one launch / two: 227 random
+// shapes of 1024-8192 columns, K 1024-8192 and 1-600 rows 0.76 (geometric mean), of which five above 1.02. Those, and what 550 more timings of longer and wider
+// matrices found, are the exceptions here, by rounds of one 16-column tile per CU (a ragged count does not end on a whole round):
+//  - 1 row: long rows, which the kernel for one matrix streams as fast (4096 x 8192: 24.9 us in two, 26.2 in one; ragged 5120 x 5504: 24.1, 26.8).
+//  - 2 rows of at most 2048 columns beyond the row kernel's K (1024 x 8192: 13.2, 16.0; 2048 x 6144 to x 16384 0.99-1.12); of a ragged count at K up to 4096
+//    (5568 x 4096: 20.4, 27.3; 4544 x 2752: 15.1, 15.8). 3 rows of those at K near 2048 (5120 x 2048 1.12, 10240 x 2048 1.33).
+//  - up to 16 rows of ragged counts from 4/3 rounds and K = 4096 on (5568 and 6000 columns: x 4096 1.04-1.13, x 6144 1.00-1.07, x 8192 1.07-1.19), from 3/2 rounds and
+//    K = 3072 on (7168 x 4096 at 8 rows: 25.1, 29.1).
+//  - more than two rounds (8192 columns): 3 to 16 rows of ragged counts (8704-18432 columns 0.77-1.48), 9 to 16 of whole ones on K above 2048 (20480 x 6144 at 16
+//    rows: 85.2, 98.7; the columns that one matrix's kernels take several tiles a block); from 17 rows on K above 2048 or more than four rounds (18432 x 4096 at 24
+//    rows: 81.3, 100.5; 10240 x 8192: 76.7, 94.4), where nothing predicts which side is faster.
+// With them, wider than 8192 columns 0.84 (244 timings, before 0.91 of 436 with 85 above 1.02; now 4, at most 1.04); another 229 random shapes in the first range 0.75, two above 1.02
+// (1888 x 8192 at 315 rows 1.07). Left as they are: K = 6144 on 4864-5120 columns (1.00-1.13 in two runs, x 5632 and x 7168 0.87-0.97), 8192 x 28672 at 16 and 256 rows (1.10).
+inline bool sum_in_two_launches(int64_t M, int64_t N, int64_t K, int cus) {
+    if (K < 1024 || M < 1) return true;  // no shorter row was measured
+    const int64_t tiles = (N + 15) / 16;
+    const bool ragged = tiles > cus && tiles % cus != 0;
+    if (M == 1) return ragged ? K > 4096 || (K > 2048 && K < 3072) : K > 11 * 512;
+    if (M == 2 && (N <= 2048 ? K > 11 * 512 : ragged && K > 2048 && K <= 4096)) return true;
+    if (M == 3 && ragged && K > 1536 && K <= 2048) return true;
+    if (tiles > 2ll * cus) {
+        if (M <= 16) return ragged ? M > 2 || K > 2048 : M > 8 && K > 2048;
+        return K > 2048 || tiles > 4ll * cus;
+    }
+    return M <= 16 && ragged && (tiles * 2 >= 3ll * cus ? K >= 3072 : tiles * 3 >= 4ll * cus && K >= 4096);
+}
+
 // A K split count that the environment asks for, as a launch takes it: 1 to `most`, none without a K tile.
 inline int forced_splits(int wanted, int KT, int most) {
     const int top = KT < most ? KT : most;

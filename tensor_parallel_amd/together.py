@@ -332,7 +332,7 @@ def linear_sum(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], r
     """The sum of two ranks' Linears, a tensor of its own for each; None where this rank is on its own or two launches are faster. `op`: the collective that
     it is for, which both ranks have to name."""
     K = x.shape[-1]
-    if K == 0 or w.dim() != 2 or x.dtype is torch.float32 or not _native.linear_sum_pays(x.numel() // K, w.shape[0], K, x.dtype):
+    if K == 0 or w.dim() != 2 or x.dtype is torch.float32 or not _native.linear_sum_pays(x.numel() // K, w.shape[0], K, x.dtype, x.get_device()):
         return None
     return _call(_not_together, _linear_sum, (x, w, bias), (op,), (rank,))
 

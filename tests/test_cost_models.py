@@ -44,3 +44,13 @@ def test_slabs_are_taken_without_scratch_memory_where_they_measured_faster(tmp_p
              (200, 8192, 4096, 1, 0), (65, 28672, 4096, 0, 0), (65, 28672, 4096, 1, 0), (256, 1024, 16384, 1, 1), (400, 1024, 16384, 0, 0), (100, 16384, 8192, 0, 0)]
     rows = ask(tmp_path, "".join(f'printf("%d\\n", w8_slabs_without_scratch({m}, {n}, {k}, {o}) ? 1 : 0);\n' for m, n, k, o, _ in cases))
     assert [r[0] for r in rows] == [c[4] for c in cases]
+
+
+def test_sums_of_two_ranks_stay_in_two_launches_where_those_measured_faster(tmp_path):
+    """Rows, columns and K, and whether one launch of both ranks took longer than two on 256 CUs (by 4 % or more; the others took at most 0.98 of two)."""
+    cases = [(2, 1024, 8192, 1), (2, 2048, 16384, 1), (2, 2048, 5632, 0), (2, 2304, 8192, 0), (2, 5568, 4096, 1), (2, 4864, 4096, 1), (2, 5120, 4608, 0), (3, 5120, 2048, 1), (3, 10240, 2048, 1),
+             (3, 4096, 2048, 0), (8, 5568, 4096, 1), (16, 6000, 8192, 1), (8, 5120, 8192, 0), (8, 7168, 4096, 1), (8, 6000, 3584, 0), (1, 4096, 8192, 1), (1, 4096, 4096, 0),
+             (4, 14336, 2048, 1), (12, 9216, 1024, 1), (2, 9216, 2048, 0), (8, 12288, 4096, 0), (16, 20480, 6144, 1), (16, 32768, 4096, 1), (16, 16384, 2048, 0), (24, 18432, 4096, 1),
+             (24, 10240, 8192, 1), (64, 9216, 4096, 1), (128, 9216, 8192, 1), (24, 20480, 1024, 1), (40, 12288, 2048, 0), (64, 16384, 1024, 0), (40, 8192, 14336, 0), (512, 4096, 5504, 0)]
+    rows = ask(tmp_path, "".join(f'printf("%d\\n", sum_in_two_launches({m}, {n}, {k}, 256) ? 1 : 0);\n' for m, n, k, _ in cases))
+    assert [r[0] for r in rows] == [c[3] for c in cases]
