@@ -205,19 +205,27 @@ def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
 # its call costs the host less: OPT-125m in fp32, 50 norms of 768 a forward, 5.6 ms eager with torch's and 6.1 with these. 16 rows of 8192 in
 # fp16 take 9.3 us there and 4.1 here. In between, the host sets the pace of an eager forward with some hundred rows (the Falcon-40B-shaped layer on 150 of them: 890 us
 # with torch's norms, 950 with these), so torch's stay there; 1024 rows take 14.4 us there and 7.3 here.
-LAYER_NORM_ROW = 2048
+# The rows have to be whole 16-byte chunks, at most as many as a block holds in registers: the kernel for any others reads a row three times, element by element (two ranks' 1024
+# rows of 16384 in fp32: 62 us with torch's, 124 with it; of 18432 in bf16 52 and 150, of 8196 28 and 54).
+LAYER_NORM_ROW, LAYER_NORM_ROW_BYTES = 2048, 32768
 LAYER_NORM_FEW_ROWS, LAYER_NORM_MANY_ROWS = 64, 512
+
+
+def _layer_norm_pays(w: torch.Tensor) -> bool:
+    row = w.numel() * w.element_size()
+    return w.numel() >= LAYER_NORM_ROW and row <= LAYER_NORM_ROW_BYTES and row % 16 == 0
+
 
 _own_layer_norm, _functional_layer_norm = nn.LayerNorm.forward, nn.functional.layer_norm
 
 
 class ShardLayerNorm(nn.LayerNorm):
-    """`nn.LayerNorm` over a last axis of at least LAYER_NORM_ROW elements whose forward is `tpamd_layer_norm_ranks`; the base class's own forward runs where that one does not stand in
+    """`nn.LayerNorm` over a last axis that the kernel is made for (_layer_norm_pays) whose forward is `tpamd_layer_norm_ranks`; the base class's own forward runs where that one does not stand in
     for it (_norm_kernel_takes; derivatives, autocast, a program's own function in the place of torch's)."""
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:  # noqa: A002
         w = self.weight
-        if w is None or LAYER_NORM_FEW_ROWS * w.numel() < input.numel() < LAYER_NORM_MANY_ROWS * w.numel():
+        if w is None or LAYER_NORM_FEW_ROWS * w.numel() < input.numel() < LAYER_NORM_MANY_ROWS * w.numel() or not _layer_norm_pays(w):
             return super().forward(input)
         b = self.bias
         if (nn.LayerNorm.forward is not _own_layer_norm or nn.functional.layer_norm is not _functional_layer_norm or len(self.normalized_shape) != 1
@@ -472,7 +480,7 @@ def install_shard_kernels(shard: nn.Module) -> None:
             module.__class__ = ShardLinear
         elif is_conv1d(module) and type(module).__name__ == "Conv1D" and module.weight.dim() == 2 and module.weight.dtype in _KERNEL_DTYPES:
             module.__class__ = _shard_conv1d_class(type(module))
-        elif type(module) is nn.LayerNorm and module.weight is not None and module.weight.dtype in _KERNEL_DTYPES and module.weight.numel() >= LAYER_NORM_ROW:
+        elif type(module) is nn.LayerNorm and module.weight is not None and module.weight.dtype in _KERNEL_DTYPES and _layer_norm_pays(module.weight):
             module.__class__ = ShardLayerNorm
         elif is_rms_norm(module) and module.weight.dtype in _KERNEL_DTYPES:
             module.__class__ = _fused_class(type(module), _rms_norm_forward, "The base class with its forward as one launch (`tpamd_rms_norm`).")

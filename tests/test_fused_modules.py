@@ -358,3 +358,20 @@ def test_an_attention_that_is_too_long_for_the_rope_kernel_keeps_torchs_rotation
         monkeypatch.undo()
         attention.register()
     assert kernels.count("rope") == takes and len(rotated) == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("D,fp32,half", [(2040, False, False), (2048, True, True), (2052, True, False), (2049, False, False), (8192, True, True), (8196, False, False), (8200, False, True),
+                                         (16384, False, True), (16392, False, False)])
+def test_layer_norms_of_rows_that_the_kernel_does_not_hold_are_torchs(kernels, monkeypatch, D, fp32, half, dtype):
+    """Whole 16-byte chunks and up to 32 KiB of them; also of a norm that was moved to another dtype after its class was changed."""
+    monkeypatch.setattr(_native, "layer_norm", lambda x, w, b, eps: kernels.append("layer_norm") or torch.nn.functional.layer_norm(x, (D,), w, b, eps))
+    takes = {torch.float32: fp32, torch.float16: half}
+    for before in takes:
+        kernels.clear()
+        norm, x = torch.nn.LayerNorm(D).to(before), torch.randn(3, D).to(dtype)
+        shard_modules.install_shard_kernels(torch.nn.Sequential(norm))
+        assert (type(norm) is shard_modules.ShardLayerNorm) == takes[before]
+        with torch.no_grad():
+            norm.to(dtype)(x)
+        assert kernels == ["layer_norm"] * (takes[before] and takes[dtype])
