@@ -69,11 +69,12 @@ FUSE_SUM = os.environ.get("TPAMD_FUSE_SUM", "1") != "0"
 class SumContext:
     """One call of a wrapped module whose output 0 goes to `op`, on one rank."""
 
-    __slots__ = ("op", "rank", "owner", "last_linear", "last_out", "last_version", "calls", "fused_linear", "fused_out", "fused_version", "fused_mask", "fused_copy",
+    __slots__ = ("op", "rank", "owner", "wrapped", "last_linear", "last_out", "last_version", "calls", "fused_linear", "fused_out", "fused_version", "fused_mask", "fused_copy",
                  "fused_whole", "returned")
 
-    def __init__(self, op: "DeviceAllReduce", rank: int, owner: Any):
+    def __init__(self, op: "DeviceAllReduce", rank: int, owner: Any, wrapped: Any = None):
         self.op, self.rank, self.owner = op, rank, owner
+        self.wrapped = owner.tp_wrapped_module if wrapped is None else wrapped  # (a wrapper looks its attributes up in the module as well: a microsecond each)
         self.last_linear = self.last_out = self.last_version = None
         self.fused_linear = self.fused_out = self.fused_version = self.fused_copy = None
         self.fused_whole = False  # fused_out was made as a sum over all ranks

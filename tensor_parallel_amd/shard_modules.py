@@ -68,7 +68,7 @@ def product_in_context(module: nn.Module, x: torch.Tensor, columns: int, inputs:
             raise RuntimeError("tensor_parallel_amd: the Linear that feeds a \"sum\" rule ran twice in one call of its module "
                                "after adding the waiting partial sums; set TPAMD_FUSE_SUM=0")
         waiting = ctx.op.addend_for(ctx.rank)
-        if waiting is None and summed is not None and ctx.op.world_size == 2 and _is_last_child(module, ctx.owner.tp_wrapped_module):
+        if waiting is None and summed is not None and ctx.op.world_size == 2 and _is_last_child(module, ctx.wrapped):
             out = summed(ctx.rank, ctx.op)
         if out is not None:
             out = _guard(out, *inputs)
@@ -97,7 +97,7 @@ def _may_hold_sum(module: nn.Module, ctx, learned: bool) -> bool:
     part. Not with hooks on the Linear, on the module around it (the wrapped one) or on all modules, nor with a forward that a program has put around the
     Linear's. Then either the wrapped module is known to return it untouched, or (`learned`) it did so when it was last seen without, and a
     change shows in the tensor's version, which raises; in inference mode versions stand still."""
-    wrapped, hooks = ctx.owner.tp_wrapped_module, torch.nn.modules.module
+    wrapped, hooks = ctx.wrapped, torch.nn.modules.module
     if hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _has_hooks(module) or _has_hooks(wrapped) or "forward" in module.__dict__:
         return False
     return learned and not torch.is_inference_mode_enabled() or hands_through(ctx, module)
@@ -111,7 +111,7 @@ def _is_last_child(module: nn.Module, wrapped: nn.Module) -> bool:
 def returned(self: nn.Module, forward, linear: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """linear(x), which this forward of the module `self` (an attribute of it) returns as it is: a wrapper around the module is told."""
     ctx = together.current_sum_context()
-    if ctx is not None and ctx.owner.tp_wrapped_module is self and getattr(self.__dict__.get("forward"), "__func__", None) is forward:
+    if ctx is not None and ctx.wrapped is self and getattr(self.__dict__.get("forward"), "__func__", None) is forward:
         ctx.returned = linear
     return linear(x)
 
@@ -119,7 +119,7 @@ def returned(self: nn.Module, forward, linear: nn.Module, x: torch.Tensor) -> to
 def hands_through(ctx, module: nn.Module) -> bool:
     """Whether the wrapped module is this Linear, said that it returns what the Linear gives, or has one of the forwards below (or the transformers one it stands in
     for), which do."""
-    wrapped = ctx.owner.tp_wrapped_module
+    wrapped = ctx.wrapped
     if wrapped is module or ctx.returned is module:
         return True
     own, cls = wrapped.__dict__.get("forward"), type(wrapped)

@@ -121,17 +121,18 @@ class TensorParallelWrapper(nn.Module):
         call_args, call_kwargs = args, kwargs
         if self.input_actions:
             call_args, call_kwargs = process_input(self.input_actions, self.rank, self.world_size, *args, **kwargs)
+        wrapped = self._modules["tp_wrapped_module"]
         if self._gather_op is not None:
-            whole = gathered_linear(self.tp_wrapped_module, self._gather_op, self.rank, call_args, call_kwargs)
+            whole = gathered_linear(wrapped, self._gather_op, self.rank, call_args, call_kwargs)
             if whole is not None:
                 return whole
         # Every wrapper publishes its own context, or none: Linears and rules inside a wrapper without a foldable sum must
         # not be taken for those of an enclosing module whose output is summed.
         foldable = self._sum_op is not None and self._sum_op.fusable
-        ctx = SumContext(self._sum_op, self.rank, self) if foldable else None
+        ctx = SumContext(self._sum_op, self.rank, self, wrapped) if foldable else None
         push_sum_context(ctx)
         try:
-            result = self.tp_wrapped_module(*call_args, **call_kwargs)
+            result = wrapped(*call_args, **call_kwargs)
             if ctx is not None:
                 ctx.settle(_output_zero(result))
             return process_output(result, self.output_actions, rank=self.rank, world_size=self.world_size)
