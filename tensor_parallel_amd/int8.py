@@ -63,6 +63,12 @@ def quantize_rows(w: torch.Tensor, outlier_cols: Optional[torch.Tensor] = None) 
     return q, scale, cols.to(torch.int32), w.detach()[:, cols].contiguous()
 
 
+# From 65 to this many rows a Linear neither meets its peer nor hands a sum over: the host sets the pace of an eager prompt there, and the reduction kernel's launch costs it
+# less than keeping book of what a module returns (the Falcon-40B-shaped layer on 200 / 400 / 512 rows: 965 / 975 / 1012 us, 1000 / 1005 / 1047 with
+# the sum in the Linears; on 600 / 850 / 1024 rows, where the device does, 1268 / 1457 / 1573 and 1261 / 1449 / 1562).
+W8_ALONE_ROWS = 512
+
+
 class ShardLinearW8(nn.Module):
     """A Linear whose weight is stored as int8 rows with one float32 scale each, plus the outlier input columns in the
     activation dtype; the forward is `tpamd_linear_w8`. Inference only."""
@@ -99,8 +105,8 @@ class ShardLinearW8(nn.Module):
         n_out = idx.numel()
         operands = (input.detach(), self.wq, self.scale, idx if n_out else None, self.w_out if n_out else None, self.bias)
         few = input.numel() <= together.W8_TOGETHER_ROWS * input.shape[-1]
-        if together.current_sum_context() is None:  # (what product_in_context does then: a prompt's host calls set its pace)
-            return _guard(together.linear_w8(*operands, act) if few else _native.linear_w8(*operands, act), input)
+        if not few and input.numel() <= W8_ALONE_ROWS * input.shape[-1]:
+            return _guard(_native.linear_w8(*operands, act), input)
         alone = functools.partial(_native.linear_w8, *operands, act)
         return product_in_context(self, input, self.out_features, (input,), functools.partial(together.linear_w8, *operands, act) if few else alone, alone,
                                   (lambda rank, op: together.linear_w8_sum(*operands, rank, op)) if few and act == _native.ACT_NONE else None, learned=False)

@@ -338,7 +338,7 @@ def linear_sum(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], r
 
 
 # Up to this many rows the int8 kernels take two ranks in one launch, and a sum that those cannot add up is a launch of its own behind them; above, a rank's Linear
-# fills the device and adds the other's result (the Falcon-40B-shaped layer: 16 rows 294 us this way and 301 the other, 1024 rows 1492 and 1462).
+# fills the device and, from int8.W8_ALONE_ROWS on, adds the other's result (the Falcon-40B-shaped layer: 16 rows 294 us this way and 301 the other, 1024 rows 1492 and 1462).
 W8_TOGETHER_ROWS = 64
 
 

@@ -174,7 +174,7 @@ def test_activation_of_a_falcon_mlp_in_the_first_linear(M, dtype, monkeypatch):
 @pytest.mark.parametrize("inference", [False, True])
 @pytest.mark.parametrize("family", ["falcon int8", "llama"])
 def test_sums_behind_fused_attentions_need_no_reduction(family, inference, monkeypatch):
-    """A prompt of 2 x 70 positions: the output projection of a fused attention hands the sum over the ranks to its wrapper, as an MLP's down projection does."""
+    """A prompt of 2 x 300 positions: the output projection of a fused attention hands the sum over the ranks to its wrapper, as an MLP's down projection does."""
     from transformers import DynamicCache, FalconConfig, FalconForCausalLM, LlamaConfig, LlamaForCausalLM
 
     from tensor_parallel_amd import _native, collectives
@@ -191,7 +191,7 @@ def test_sums_behind_fused_attentions_need_no_reduction(family, inference, monke
     assert tp.attention.fuse_rotary_(split, assume_no_padding=True) == 2
     if family != "llama":
         quantize_linears_(split, skip=lambda name, m: "lm_head" in name)
-    ids = torch.randint(2, 300, (2, 70), device=DEV)
+    ids = torch.randint(2, 300, (2, 300), device=DEV)
     reduced, reduce = [], _native.reduce_partials
     monkeypatch.setattr(_native, "reduce_partials", lambda parts, **more: reduced.append(len(parts)) or reduce(parts, **more))
     with torch.inference_mode() if inference else torch.no_grad():

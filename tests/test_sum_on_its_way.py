@@ -8,7 +8,7 @@ from torch import nn
 
 from tensor_parallel_amd import _native, together
 from tensor_parallel_amd.collectives import DeviceAllReduce
-from tensor_parallel_amd.int8 import ShardLinearW8
+from tensor_parallel_amd.int8 import W8_ALONE_ROWS, ShardLinearW8
 from tensor_parallel_amd.shard_modules import ShardLinear, returned
 from tensor_parallel_amd.tensor_parallel import RANK_GREENLETS, _apply_in_greenlets
 from tensor_parallel_amd.wrapper import TensorParallelWrapper
@@ -96,6 +96,11 @@ def forward(models, rows, inference=False):
         return _apply_in_greenlets(models, [(x,) for x in xs], [{}] * 2, torch.device("cpu")), want
 
 
+def made(kind, rows):
+    """How the sum is made where the Linear may make it."""
+    return "whole" if kind == "16 bits" or rows <= together.W8_TOGETHER_ROWS else "reduction" if rows <= W8_ALONE_ROWS else "addend"
+
+
 def check(got, want):
     for y in got:
         assert torch.equal(y.float(), want)
@@ -103,19 +108,19 @@ def check(got, want):
 
 @pytest.mark.parametrize("inference", [False, True])
 @pytest.mark.parametrize("around", [False, True])
-@pytest.mark.parametrize("rows", [4, 200])
+@pytest.mark.parametrize("rows", [4, 200, 600])
 @pytest.mark.parametrize("kind", ["16 bits", "int8"])
 def test_the_linear_makes_the_sum_where_nobody_sees_its_output(folds, kind, rows, around, inference):
     models = shards(kind, around)
     for _ in range(3):
         check(*forward(models, rows, inference))
     # a module that is not known here may have done something to the output that does not show: not in inference mode, and not for int8 weights at all
-    assert folds[-1] == ("reduction" if around and (inference or kind == "int8") else "whole" if kind == "16 bits" or rows <= together.W8_TOGETHER_ROWS else "addend")
+    assert folds[-1] == ("reduction" if around and (inference or kind == "int8") else made(kind, rows))
 
 
 @pytest.mark.parametrize("which", [(0,), (1,), (0, 1)])
 @pytest.mark.parametrize("hook", ["scales", "new tensor", "on the module around", "in front of all", "a forward put around"])
-@pytest.mark.parametrize("rows", [4, 200])
+@pytest.mark.parametrize("rows", [4, 200, 600])
 @pytest.mark.parametrize("kind", ["16 bits", "int8"])
 def test_a_hook_sees_and_changes_its_own_ranks_part(kind, rows, hook, which):
     models = shards(kind, True)
@@ -159,7 +164,7 @@ def test_a_hook_sees_and_changes_its_own_ranks_part(kind, rows, hook, which):
 
 @pytest.mark.parametrize("inference", [False, True])
 @pytest.mark.parametrize("change", ["scales", "adds"])
-@pytest.mark.parametrize("rows", [4, 200])
+@pytest.mark.parametrize("rows", [4, 200, 600])
 @pytest.mark.parametrize("kind", ["16 bits", "int8"])
 def test_a_module_that_starts_to_change_the_output_in_place(kind, rows, change, inference):
     models = shards(kind, True)
@@ -196,7 +201,7 @@ def own_forward(self, x):
 
 
 @pytest.mark.parametrize("inference", [False, True])
-@pytest.mark.parametrize("rows", [4, 200])
+@pytest.mark.parametrize("rows", [4, 200, 600])
 @pytest.mark.parametrize("kind", ["16 bits", "int8"])
 def test_the_linear_of_a_forward_that_returns_its_output_makes_the_sum(folds, kind, rows, inference):
     models = shards(kind, True)
@@ -204,7 +209,7 @@ def test_the_linear_of_a_forward_that_returns_its_output_makes_the_sum(folds, ki
         m.tp_wrapped_module.forward = types.MethodType(own_forward, m.tp_wrapped_module)
     for _ in range(3):
         check(*forward(models, rows, inference))
-    assert folds[-1] == ("whole" if kind == "16 bits" or rows <= together.W8_TOGETHER_ROWS else "addend")
+    assert folds[-1] == made(kind, rows)
     # a program puts a forward of its own around that one
     for m in models:
         inner = m.tp_wrapped_module.forward
