@@ -187,3 +187,44 @@ def test_two_summed_outputs_of_one_module_share_the_op(monkeypatch):
     ref = model.float()(x.float().cpu())
     for got, r in zip(outs[-1], ref):
         torch.testing.assert_close(got.float().cpu(), r, rtol=2e-2, atol=2e-2 * r.std().item())
+
+
+@pytest.mark.parametrize("inference", [False, True])
+@pytest.mark.parametrize("tokens", [1, 5, 40, 300])
+def test_two_ranks_meet_in_the_linear_that_makes_the_sum(monkeypatch, tokens, inference):
+    """K = 1024 a rank, from which on both products and their sum are one launch; then with a hook on a rank's Linear, which sees and doubles that rank's part alone."""
+    block, model_tp = build(2, d=512, f=2048)
+    x = torch.randn(1, tokens, 512).to(torch.bfloat16).to(DEV)
+    hidden = block.float().mlp
+    h = (hidden.act_fn(hidden.gate_proj(x.float().cpu())) * hidden.up_proj(x.float().cpu())).detach()
+    parts = [(h[..., r * 1024:(r + 1) * 1024] @ hidden.down_proj.weight.detach()[:, r * 1024:(r + 1) * 1024].t()).to(DEV) for r in range(2)]
+    sums, make = [], _native.linear_sum_ranks
+    monkeypatch.setattr(_native, "linear_sum_ranks", lambda calls: sums.append(make(calls)) or sums[-1])
+
+    def check(out, want, scales):
+        # both products and the sum may be rounded the other way where K is added up in another order: a unit in the last place (2^-7) of each at most
+        size = sum(s * p.abs() for s, p in zip(scales, parts)) + want.float().abs()
+        assert bool(((out.float() - want.float()).abs() <= 1.1 * 2.0 ** -7 * size + 1e-6).all())
+
+    with torch.inference_mode() if inference else torch.no_grad():
+        monkeypatch.setattr(collectives, "FUSE_SUM", False)
+        want = [model_tp(x) for _ in range(2)][-1]
+        assert sums == []
+        monkeypatch.setattr(collectives, "FUSE_SUM", True)
+        for _ in range(4):
+            check(model_tp(x), want, (1, 1))
+        assert len(sums) == (3 if _native.linear_sum_pays(tokens, 512, 1024, torch.bfloat16) else 0) and all(s is not None for s in sums)
+        assert sums or tokens == 300
+        for rank in range(2):
+            seen = []
+            handle = model_tp.module_shards[rank].mlp.tp_wrapped_module.down_proj.register_forward_hook(lambda m, i, out: seen.append(out.clone()) or out.mul_(2))
+            sums.clear()
+            scales = (2, 1) if rank == 0 else (1, 2)
+            monkeypatch.setattr(collectives, "FUSE_SUM", False)
+            want2 = model_tp(x)
+            monkeypatch.setattr(collectives, "FUSE_SUM", True)
+            for _ in range(3):
+                check(model_tp(x), want2, scales)
+            handle.remove()
+            assert sums == [] and len(seen) == 4 and all(torch.allclose(s.float(), seen[0].float(), rtol=2.0 ** -7, atol=2.0 ** -7 * seen[0].float().std().item()) for s in seen)
+        check(model_tp(x), want, (1, 1))

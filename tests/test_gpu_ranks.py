@@ -300,8 +300,10 @@ def test_the_sum_of_two_ranks_int8_linears(rows, cols, K, n_out):
         calls.append((x, q, scale, idx, w_out, None))
         parts.append(_native.linear_w8(*calls[-1]))
     sums = _native.linear_w8_sum_ranks(calls)
-    if sums is None:
+    if sums is None:  # no planes to add up, or too many rows: these two matrices split K over blocks
+        assert (cols, K) not in ((8192, 16384), (16384, 8192)) or rows not in (16, 17, 48)
         return
+    assert rows not in (1, 65)
     assert sums[0].data_ptr() != sums[1].data_ptr() and torch.equal(*sums)
     want = parts[0].float() + parts[1].float()  # both rounded products, each of which may be rounded the other way where the planes are cut elsewhere
     bound = 2.0 ** -11 * (want.abs() + 2 * (parts[0].float().abs() + parts[1].float().abs())) + 1e-6
