@@ -203,7 +203,8 @@ def _rms_norm_forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
 
 # torch's kernel works on a row with one wavefront and does short rows as fast (128 rows of 768 in fp32: 4.0 us there, 3.6 here for two ranks at once), while
 # its call costs the host less: OPT-125m in fp32, 50 norms of 768 a forward, 5.6 ms eager with torch's and 6.1 with these. 16 rows of 8192 in
-# fp16 take 9.3 us there and 4.1 here. In between, the host sets the pace of an eager forward with some hundred rows (the Falcon-40B-shaped layer on 150 of them: 890 us
+# fp16 take 9.3 us there and 4.1 here; 1 to 64 rows of 2048 / 4096 / 8192 in fp32 3.1-3.4 / 3.8-4.2 / 5.4-5.9 for each rank there and 2.3-2.6 / 2.7-3.1 / 3.2-4.0 for both here.
+# In between, the host sets the pace of an eager forward with some hundred rows (the Falcon-40B-shaped layer on 150 of them: 890 us
 # with torch's norms, 950 with these), so torch's stay there; 1024 rows take 14.4 us there and 7.3 here.
 # The rows have to be whole 16-byte chunks, at most as many as a block holds in registers: the kernel for any others reads a row three times, element by element (two ranks' 1024
 # rows of 16384 in fp32: 62 us with torch's, 124 with it; of 18432 in bf16 52 and 150, of 8196 28 and 54).
@@ -332,7 +333,8 @@ def _is_erf_gelu(act) -> bool:
 
 def _falcon_mlp_forward(self, x: torch.Tensor) -> torch.Tensor:
     """The module's own forward on a few rows with the activation in the epilogue of an int8 Linear before it, on the sum in 32 bits: a recorded step of 16 rows through a
-    Falcon-40B-shaped layer 287 -> 281 us. Over many rows the error functions at the end of each tile take longer than torch's pass over memory (1024 rows 1490 -> 1515 us)."""
+    Falcon-40B-shaped layer 287 -> 281 us. Both ranks' first Linears with the activation take 0.67-0.94 of what they and torch's two
+    passes do at 1 to 64 rows (16384 x 8192 at 64: 97.0 -> 90.6 us). Over many rows the error functions at the end of each tile take longer than torch's pass over memory (1024 rows 1490 -> 1515)."""
     from .int8 import ShardLinearW8
 
     own = self._tp_base.forward

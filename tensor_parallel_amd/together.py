@@ -6,7 +6,8 @@ would follow one another on the device, each with 1/W of the work: a decode step
 too small to fill the device. So a rank that reaches a call which its peers will make too gives the turn away (`GreenTurn.meet`), and whoever comes
 last makes the call for all of them (`tpamd_*_ranks`). Two Llama-2-7B-shaped rank shards of two layers, recorded decode step: one row on 500
 positions 321 -> 278 us, 8 on 2048 479 -> 423, 40 on 1000 (grouped queries) 534 -> 454; the Falcon-40B-shaped int8 layer, 16 on 2048, 372 -> 339.
-On the host a meeting costs 4 to 5 us for both ranks, about what the call that it saves costs (eager decode steps and scoring stay where they were, within 2 %).
+On the host a meeting costs about 3 us for both ranks (0.5 of them for looking at the thread's state), less than the call that it saves: eager steps on a growing cache
+1290 -> 1200 us on two rank shards, 2600 -> 2520 on four.
 
 A rank meets its peers only in the state it was started in (`_thread_state`): in a stream, a grad or autocast mode, a function mode or with switches (default
 dtype, attention backends, deterministic algorithms) of its own it keeps the turn, because giving it away would take its peers there. Waiting in a collective it has to
@@ -298,7 +299,9 @@ def _call(one: Callable[..., Any], many: Callable[[List[tuple]], Sequence[Any]],
 
 
 # From this many rows on a product fills the device by itself, in 256 x 256 tiles that take two ranks in two launches anyway, and each rank's
-# follow-up work finds its operands still cached: prefill of 4096 rows 3312 us rank by rank, 3325 together; of 2103 rows 1758 and 1730.
+# follow-up work finds its operands still cached: prefill of 4096 rows 3312 us rank by rank, 3325 together; of 2103 rows 1758 and 1730. 1605 random shapes (512-16384 columns, K
+# 1024-8192) in a HIP graph, time of one launch for both in that of two, Linears / gated pairs: 17-256 rows 0.67 / 0.71, 257-512 0.69 / 0.80, 513-1024 0.77 / 0.92, 1025-2048
+# 0.86 / 0.93, 2049-3000 0.93 / 1.00, 3001-4000 0.97 / 0.99.
 ALONE_ROWS = 4096
 
 
