@@ -11,7 +11,8 @@ On the host a meeting costs about 3 us for both ranks (0.5 of them for looking a
 
 A rank meets its peers only in the state it was started in (`_thread_state`): in a stream, a grad or autocast mode, a function mode or with switches (default
 dtype, attention backends, deterministic algorithms) of its own it keeps the turn, because giving it away would take its peers there. Waiting in a collective it has to
-give it away: its peers then go on in the state that they were started in, and it finds its own again (`_as_started`).
+give it away: its peers then go on in the streams and modes that they were started in, and it finds its own again (`_as_started`). The switches are the whole process's
+and stay as they are there, for its peers as for any thread.
 
 What cannot be seen so is what a program holds across a library call: with a lock held there, the peer that asks for the lock would wait for a rank that cannot go on.
 Models whose own forwards (not those of torch and transformers) enter a `with` block or acquire something therefore do not meet (`keeps_turn`, which looks at a model in
@@ -89,16 +90,12 @@ def _of_device(get, put, device: str) -> tuple:
     return lambda: get(device), lambda value: put(device, value)
 
 
-# What of that state can be set, and all that belongs to it: reading and setting.
+# What of that state is the calling thread's, and all that belongs to it: reading and setting. The others (default dtype, attention backends, deterministic algorithms, fp32
+# products) are the process's: a difference may be another thread's doing, which may be loading a model under its default dtype, and is not to be touched.
 _SETTINGS = [
     (_grad, torch._C._set_grad_enabled),
     *(_of_device(get, put, device) for device in ("cuda", "cpu") for get, put in ((_autocast, torch.set_autocast_enabled), (torch.get_autocast_dtype, torch.set_autocast_dtype))),
     (torch.is_autocast_cache_enabled, torch.set_autocast_cache_enabled),
-    (_default_dtype, torch.set_default_dtype),
-    (_flash, torch._C._set_sdp_use_flash), (_efficient, torch._C._set_sdp_use_mem_efficient), (_math, torch._C._set_sdp_use_math),
-    (_cudnn, torch._C._set_sdp_use_cudnn),
-    (lambda: (_deterministic(), torch._C._get_deterministic_algorithms_warn_only()), lambda value: torch._C._set_deterministic_algorithms(value[0], warn_only=value[1])),
-    (_tf32, torch._C._set_cublas_allow_tf32),
 ]
 
 
@@ -114,7 +111,7 @@ def _set(values: list) -> None:
 
 @contextlib.contextmanager
 def _as_started(turn: "GreenTurn"):
-    """For a rank that gives the turn away in a state of its own: the state that the ranks were started in, inside, and its own again behind."""
+    """For a rank that gives the turn away in a state of its own: the streams and modes that the ranks were started in, inside, and its own again behind."""
     own, index = _settings(), turn.index
     where = None if index is None else (torch._C._cuda_getCurrentStream(index), _current_device())
     modes, dispatch = [], []
@@ -226,7 +223,7 @@ class GreenTurn:
         return True
 
     def _pass_on(self) -> None:
-        """Gives the turn to the next rank, in the state that the ranks were started in; comes back in that state."""
+        """Gives the turn to the next rank, in the streams and modes that the ranks were started in; comes back in those."""
         ring = self.ring
         self.idle += 1
         if self.idle > 2 * len(ring):

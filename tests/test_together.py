@@ -188,6 +188,9 @@ def _scopes():
             "no grad": torch.no_grad, "inference": torch.inference_mode, "default device": lambda: torch.device("cpu")}
 
 
+PROCESS_WIDE = ("default dtype", "attention backend", "deterministic")
+
+
 def _state():
     backends = torch.backends.cuda
     return (torch.is_grad_enabled(), torch.is_inference_mode_enabled(), torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda"),
@@ -198,7 +201,7 @@ def _state():
 @pytest.mark.parametrize("ranks", [(0,), (0, 1)])
 @pytest.mark.parametrize("scope", list(_scopes()))
 def test_a_scope_of_one_rank_is_not_seen_by_another(calls, scope, ranks):
-    """Two library calls and a collective inside the scope, one of each behind it."""
+    """Two library calls and a collective inside the scope, one of each behind it; no collective where the scope is the process's."""
     from tensor_parallel_amd.collectives import CollectiveOperation
 
     op, before = CollectiveOperation(2, lambda *xs: [sum(xs)] * 2, timeout=5.0), _state()
@@ -215,7 +218,7 @@ def test_a_scope_of_one_rank_is_not_seen_by_another(calls, scope, ranks):
                 for _ in range(2):
                     together.linear(*operands(r))
                     states.append(_state())
-                assert op(r + 1, r) == 3
+                assert scope in PROCESS_WIDE or op(r + 1, r) == 3
                 states.append(_state())
                 together.linear(*operands(r))
                 states.append(_state())
@@ -243,7 +246,7 @@ def test_calls_that_nobody_comes_to_are_made_in_the_state_of_their_rank(monkeypa
             together.linear(*operands(0))
             op(1, 0)
         else:
-            with torch.inference_mode(), _default_dtype(torch.float64):
+            with torch.inference_mode(), torch.autocast("cpu", dtype=torch.bfloat16):
                 op(2, 1)
 
     run(body, body)
@@ -342,3 +345,36 @@ def test_ranks_at_different_collectives_are_not_taken_for_one_call(monkeypatch, 
     if kinds[0] != kinds[1]:  # two kinds for one op, which no rule makes
         ops[1] = ops[0]
         assert run(body, body) == [None, None]
+
+
+def test_a_process_wide_switch_of_another_thread_is_left_alone():
+    """A program may load a model under a default dtype in one thread while another runs a forward, whose ranks wait in collectives."""
+    from tensor_parallel_amd.collectives import CollectiveOperation
+
+    op, seen = CollectiveOperation(2, lambda *xs: [sum(xs)] * 2, timeout=5.0), []
+    switched, done = threading.Event(), threading.Event()
+
+    def loads():
+        with _default_dtype(torch.float64):
+            switched.set()
+            done.wait(10)
+            seen.append(torch.get_default_dtype())
+
+    other = threading.Thread(target=loads)
+
+    def body(r):
+        if r == 0:
+            other.start()
+            switched.wait(10)
+        for _ in range(3):
+            with torch.inference_mode() if r == 0 else contextlib.nullcontext():  # a state of this rank's own as well
+                op(r, r)
+                seen.append(torch.get_default_dtype())
+                assert torch.is_inference_mode_enabled() == (r == 0)
+
+    try:
+        run(body, body)
+    finally:
+        done.set()
+        other.join()
+    assert seen == [torch.float64] * 7 and torch.get_default_dtype() is torch.float32
