@@ -23,6 +23,8 @@ int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bi
                     int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int64_t ld_wout, int dtype, int act, bool swiglu, bool w8,
                     hipStream_t s, const RankStep *second = nullptr, int64_t copy = 0);
 
+bool stream_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int ranks, bool swiglu, bool sum, int cus);
+
 bool w8_direct_ok(int64_t K, int64_t ldx, int64_t ldw);
 int gemm_w8_dispatch(const void *x, const void *wq, const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out,
                      const void *bias, const void *addend, int64_t ldadd, int64_t copy, void *y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
@@ -92,6 +94,19 @@ int pair_row_limit(int64_t N, int64_t K, int64_t *rows) {
     if (K >= 2048 && K <= 6144 && (N + 7) / 8 <= cus) *rows = 32;
     return TPAMD_OK;
 }
+// Rows that skinny_dispatch takes of `ranks` matrices (pair: gated pairs) of N columns each in one launch: those of the kernels above, and what stream_kernel takes.
+int decode_rows(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int ranks, bool pair, int64_t *rows) {
+    *rows = SKINNY_MAX_M;
+    if (M <= SKINNY_MAX_M || M > 64) return TPAMD_OK;
+    int dev = 0, cus = 256;
+    TPAMD_HIP(hipGetDevice(&dev));
+    if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
+    if (stream_pays(M, N, K, ldx, ldw, ranks, pair, false, cus)) {
+        *rows = 64;
+        return TPAMD_OK;
+    }
+    return pair ? (M <= 32 ? pair_row_limit(ranks * N, K, rows) : TPAMD_OK) : skinny_row_limit(ranks * N, K, rows);
+}
 constexpr int64_t SKINNY_W8_SLAB = 64;
 
 // What the MFMA kernels need from 16-bit operands: 16-byte aligned rows of x and w, 8-byte aligned groups of 4
@@ -137,8 +152,8 @@ int tpamd::linear_entry(const char *who, const void *x_dev, const void *w_dev, c
                       (addend_dev == nullptr || (aligned(addend_dev, 8) && ldadd % 4 == 0)) && aligned(copy_dev, 8);
     const int64_t copy = bytes_from(y_dev, copy_dev);
     int64_t skinny_rows = SKINNY_MAX_M;
-    if (fast && M > SKINNY_MAX_M && M <= 64) {
-        rc = skinny_row_limit(N, K, &skinny_rows);
+    if (fast) {
+        rc = decode_rows(M, N, K, ldx, ldw, 1, false, &skinny_rows);
         if (rc != TPAMD_OK) return rc;
     }
     if (fast && M <= skinny_rows)
@@ -181,8 +196,8 @@ extern "C" int tpamd_swiglu_up(const void *x_dev, const void *wg_dev, const void
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool fast = dtype != TPAMD_F32 && mfma_ok(x_dev, wg_dev, wu_dev, nullptr, h_dev, N, K, ldx, ldw, ldh);
     int64_t pair_rows = SKINNY_MAX_M;
-    if (fast && M > SKINNY_MAX_M && M <= 32) {
-        rc = pair_row_limit(N, K, &pair_rows);
+    if (fast) {
+        rc = decode_rows(M, N, K, ldx, ldw, 1, true, &pair_rows);
         if (rc != TPAMD_OK) return rc;
     }
     if (fast && M <= pair_rows)
@@ -224,9 +239,7 @@ static int matmul_ranks(const char *who, int n, const void *const *x, const void
         to.bias = bytes_from(b0, b1);
         to.y = bytes_from(y[i], y[i + 1]);
         int64_t rows = SKINNY_MAX_M;
-        if (M > SKINNY_MAX_M && M <= 64) {
-            if (int rc = pair ? (M <= 32 ? pair_row_limit(2 * N, K, &rows) : TPAMD_OK) : skinny_row_limit(2 * N, K, &rows); rc != TPAMD_OK) return rc;
-        }
+        if (int rc = decode_rows(M, N, K, ldx, ldw, 2, pair, &rows); rc != TPAMD_OK) return rc;
         const int rc = M <= rows ? skinny_dispatch(x[i], w[i], pair ? w2[i] : nullptr, b0, nullptr, 0, nullptr, nullptr, nullptr, 0, y[i], M, N, K, ldx, ldw,
                                                    ldy, 0, dtype, act, pair, false, static_cast<hipStream_t>(stream), &to)
                                  : gemm_dispatch(x[i], w[i], pair ? w2[i] : nullptr, b0, nullptr, 0, y[i], M, N, K, ldx, ldw, ldy, dtype, act, pair, false,
@@ -290,8 +303,8 @@ extern "C" int tpamd_linear_gather_ranks(int n, const void *const *x_dev, const 
     const int64_t copy = bytes_from(y_dev[0], y_dev[1]);
     hipStream_t s = static_cast<hipStream_t>(stream);
     int64_t rows = dtype == TPAMD_F32 ? 0 : SKINNY_MAX_M;
-    if (dtype != TPAMD_F32 && M > SKINNY_MAX_M && M <= 64) {
-        if (int rc = skinny_row_limit(2 * N, K, &rows); rc != TPAMD_OK) return rc;
+    if (dtype != TPAMD_F32) {
+        if (int rc = decode_rows(M, N, K, ldx, ldw, 2, false, &rows); rc != TPAMD_OK) return rc;
     }
     if (M <= rows)
         return skinny_dispatch(x_dev[0], w_dev[0], nullptr, b0, nullptr, 0, nullptr, nullptr, nullptr, 0, y_dev[0], M, N, K, ldx, ldw, ldy, 0, dtype, act, false,
@@ -310,11 +323,15 @@ extern "C" int tpamd_linear_gather_ranks(int n, const void *const *x_dev, const 
 // unless its tiles are a ragged number of rounds; K ranges of tiles the rest, above 64 rows while they are predicted to be faster than two launches. What stays in two
 // launches and why: sum_in_two_launches (gemm_model.h).
 enum SumPath { SUM_NONE, SUM_ROWS8, SUM_ROWS16, SUM_STREAM, SUM_TILES };
-static int sum_path(int64_t M, int64_t N, int64_t K, SumPath *path) {
+static int sum_path(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, SumPath *path) {
     *path = SUM_NONE;
     int dev = 0, cus = 256;
     TPAMD_HIP(hipGetDevice(&dev));
     if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
+    if (stream_pays(M, N, K, ldx, ldw, 2, false, true, cus)) {
+        *path = SUM_STREAM;
+        return TPAMD_OK;
+    }
     if (sum_in_two_launches(M, N, K, cus)) return TPAMD_OK;
     const int64_t tiles = (N + 15) / 16;
     const bool ragged = tiles > cus && tiles % cus != 0;
@@ -333,7 +350,7 @@ static int sum_path(int64_t M, int64_t N, int64_t K, SumPath *path) {
 
 extern "C" int tpamd_linear_sum_pays(int64_t M, int64_t N, int64_t K, int dtype) {
     SumPath path = SUM_NONE;
-    return dtype != TPAMD_F32 && sum_path(M, N, K, &path) == TPAMD_OK && path != SUM_NONE ? 1 : 0;
+    return dtype != TPAMD_F32 && sum_path(M, N, K, K, K, &path) == TPAMD_OK && path != SUM_NONE ? 1 : 0;
 }
 
 // Row-parallel Linears of two ranks and their sum, delivered to both. TPAMD_ERR_UNSUPPORTED, with nothing launched, where two launches
@@ -350,7 +367,7 @@ extern "C" int tpamd_linear_sum_ranks(const void *const *x_dev, const void *cons
     if (M == 0 || N == 0) return TPAMD_OK;
     SumPath path = SUM_NONE;
     if (fast) {
-        if (int rc = sum_path(M, N, K, &path); rc != TPAMD_OK) return rc;
+        if (int rc = sum_path(M, N, K, ldx, ldw, &path); rc != TPAMD_OK) return rc;
     }
     if (path != SUM_NONE) {
         const void *b0 = bias_dev ? bias_dev[0] : nullptr, *b1 = bias_dev ? bias_dev[1] : nullptr;

@@ -36,6 +36,7 @@ Tuning read_tuning() {
     t.skinny_xlds = env_int("TPAMD_SKINNY_XLDS");
     t.skinny_max_m = env_int("TPAMD_SKINNY_MAX_M");
     t.gemv_rows = env_int("TPAMD_GEMV_ROWS");
+    t.stream = env_int("TPAMD_STREAM");
     t.attn_splits = env_int("TPAMD_ATTN_SPLITS");
     t.attn_ring = env_int("TPAMD_ATTN_RING");
     t.copy_tile_units = env_int("TPAMD_COPY_TILE_UNITS");

@@ -12,7 +12,7 @@
 //
 // The weight is either the activation dtype (bf16/f16) or int8 (weight-only quantisation: converted to
 // the activation dtype in registers, exact for |q| <= 128).
-#include "common.h"
+#include "skinny.h"
 
 #include <stdlib.h>
 #include <mutex>
@@ -25,38 +25,8 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-enum { SK_LINEAR = 0, SK_SWIGLU = 1 };
 constexpr int SK_WAVES = 8;
 constexpr int SK_THREADS = SK_WAVES * 64;
-
-struct SkinnyParams {
-    const char *x;
-    const char *w;
-    const char *w2;
-    const char *bias;
-    const float *scale;        // int8 path: per output row
-    const int *outlier_idx;    // int8 path
-    const char *w_out;         // int8 path: [N, n_out] in activation dtype
-    const char *addend;        // linear: added to the rounded result, or NULL
-    char *y;
-    int M, N, K;
-    int n_out;
-    int64_t ldx, ldw, ldy, ld_wout, ldadd;
-    int act;
-    int ranks;     // 1, or 2: blockIdx.z is the rank, `to` the way to the second one's operands
-    RankStep to;
-    int64_t copy;  // every output is stored a second time that many bytes on (0: once)
-    int sum;       // y = round(rank 0's product) + round(rank 1's): one result for both ranks
-};
-
-// This block's rank.
-__device__ __forceinline__ void take_rank(SkinnyParams &p) {
-    if (blockIdx.z == 0) return;
-    p.x += p.to.x; p.w += p.to.w; p.w2 += p.to.w2; p.bias += p.to.bias; p.y += p.to.y;
-    p.scale = reinterpret_cast<const float *>(reinterpret_cast<const char *>(p.scale) + p.to.scale);
-    p.outlier_idx = reinterpret_cast<const int *>(reinterpret_cast<const char *>(p.outlier_idx) + p.to.outlier_idx);
-    p.w_out += p.to.w_out;
-}
 
 template <int DT>
 __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
@@ -64,43 +34,6 @@ __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     else
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
-// One output element from its fp32 sums (s1 = the up sum of a gated pair): the reference's op chain with its
-// roundings to the tensor dtype (gate and up products, SiLU, product), or bias and activation.
-template <int DT, int MODE>
-__device__ __forceinline__ void skinny_store_output(const SkinnyParams &p, float s0, float s1, int m, int n) {
-    uint16_t out;
-    if constexpr (MODE == SK_SWIGLU) {
-        const float gv = half_to_f32<DT>(f32_to_half<DT>(s0));
-        const float u = half_to_f32<DT>(f32_to_half<DT>(s1));
-        const float sl = half_to_f32<DT>(f32_to_half<DT>(silu_f32(gv)));
-        out = f32_to_half<DT>(sl * u);
-    } else {
-        float v = s0;
-        if (p.bias) v += half_to_f32<DT>(reinterpret_cast<const uint16_t *>(p.bias)[n]);
-        if (p.act == TPAMD_ACT_GELU) v = gelu_erf(v);
-        out = f32_to_half<DT>(v);
-        if (p.addend != nullptr)  // one step of the sum over rank partials: both operands in the tensor dtype
-            out = f32_to_half<DT>(half_to_f32<DT>(out) + half_to_f32<DT>(reinterpret_cast<const uint16_t *>(p.addend)[static_cast<int64_t>(m) * p.ldadd + n]));
-    }
-    reinterpret_cast<uint16_t *>(p.y)[static_cast<int64_t>(m) * p.ldy + n] = out;
-    if constexpr (MODE == SK_LINEAR) {
-        if (p.copy) reinterpret_cast<uint16_t *>(p.y + p.copy)[static_cast<int64_t>(m) * p.ldy + n] = out;
-    }
-}
-
-// One element of the sum of two ranks' Linears from the fp32 sums of each: products rounded to the tensor dtype, then the rounded sum, which is what
-// a Linear whose epilogue adds the other's result gives.
-template <int DT>
-__device__ __forceinline__ void skinny_store_sum(const SkinnyParams &p, float s0, float s1, int m, int n) {
-    if (p.bias) {
-        s0 += half_to_f32<DT>(reinterpret_cast<const uint16_t *>(p.bias)[n]);
-        s1 += half_to_f32<DT>(reinterpret_cast<const uint16_t *>(p.bias + p.to.bias)[n]);
-    }
-    const uint16_t out = f32_to_half<DT>(half_to_f32<DT>(f32_to_half<DT>(s0)) + half_to_f32<DT>(f32_to_half<DT>(s1)));
-    reinterpret_cast<uint16_t *>(p.y)[static_cast<int64_t>(m) * p.ldy + n] = out;
-    if (p.copy) reinterpret_cast<uint16_t *>(p.y + p.copy)[static_cast<int64_t>(m) * p.ldy + n] = out;
 }
 
 // W8 = weight is int8. MT = number of 16-row tiles of x (M <= 16*MT). MODE = SK_LINEAR / SK_SWIGLU.
@@ -2088,6 +2021,10 @@ int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bi
     p.ldx = ldx; p.ldw = ldw; p.ldy = ldy; p.ld_wout = ld_wout;
     p.act = act;
     const bool bf = dtype == TPAMD_BF16;
+    int dev = 0, cus = 256;
+    TPAMD_HIP(hipGetDevice(&dev));
+    if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
+    if (!w8 && stream_pays(M, N, K, ldx, ldw, p.ranks, swiglu, false, cus)) return stream_dispatch(p, dtype, swiglu, s);
     // 2 and 3 rows of int8 weights are faster through the K-split kernel where it applies
     if (w8 && M >= 2 && M <= GEMV_MAX_M) {
         bool done = false;
@@ -2097,9 +2034,6 @@ int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bi
     if (M <= GEMV_MAX_M && M * K * 2 <= GEMV_MAX_X_BYTES) {
         RowsPath path = ROWS_W8;
         if (!w8) {
-            int dev = 0, cus = 256;
-            TPAMD_HIP(hipGetDevice(&dev));
-            if (int rc_cus = device_cus(dev, &cus); rc_cus != TPAMD_OK) return rc_cus;
             const int knob = tuning().gemv_rows;  // -1: the MFMA kernels; other values: launch_gemv_rows
             path = knob == -1 ? ROWS_MFMA : knob != TUNE_UNSET ? ROWS_W8 : pick_rows_path(swiglu, M, N * p.ranks, K, cus);
         }
@@ -2134,6 +2068,10 @@ int skinny_sum_dispatch(const void *x, const void *w, const void *bias, const Ra
     p.y = static_cast<char *>(y);
     p.M = static_cast<int>(M); p.N = static_cast<int>(N); p.K = static_cast<int>(K);
     p.ldx = ldx; p.ldw = ldw; p.ldy = ldy;
+    int dev = 0, cus = 256;
+    TPAMD_HIP(hipGetDevice(&dev));
+    if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
+    if (stream_pays(M, N, K, ldx, ldw, 2, false, true, cus)) return stream_dispatch(p, dtype, false, s);
     TPAMD_REQUIRE(row_waves == 0 || (M <= GEMV_MAX_M && K <= 11 * 512 && M * K * 4 <= GEMV_MAX_X_BYTES), "skinny: rows too long for the row kernel");
     auto run = [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
