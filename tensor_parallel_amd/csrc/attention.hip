@@ -13,20 +13,19 @@
 //                 operand comes from the row-major V tile in LDS through the LDS transpose load.
 // O^T leaves a lane with 4 consecutive head-dim elements of one query row: one 8-byte store into [B, Sq, Hq, D].
 //
-// Long key ranges with few rows (decode) are split over blockIdx.z; every split leaves (m, l, unnormalised O) in
+// One new position per sequence (decode) with at most 16 query heads per key/value head has a kernel of its own, attention_decode_kernel.
+// Long key ranges with few rows are split over blockIdx.z; every split leaves (m, l, unnormalised O) in
 // the stream's scratch buffer and attention_combine_kernel merges them. For one new position per sequence
 // (tpamd_attention_decode_rope) the kernel also applies the rotary embedding to its Q fragments, and the merge
 // (attention_combine_newkey_kernel) adds the new position's key and value and writes them into the cache.
 #include "common.h"
+#include "gemm_tile.h"
 
+#include <math.h>
 #include <stdlib.h>
 
 namespace tpamd {
 namespace {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 template <int DT>
 __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
@@ -37,7 +36,6 @@ __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
 }
 
 typedef __attribute__((ext_vector_type(4))) short i16x4;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;  // 16 bytes on their way from global memory to LDS
 
 // A loop whose counter is a constant expression inside the body (f gets Const<0>, Const<1>, ...): arrays indexed with it
 // are split into registers from the start, not only if a later pass unrolls the loop.
@@ -526,21 +524,13 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(AttnParams p) {
     *reinterpret_cast<uint2 *>(p.o + (static_cast<int64_t>(b) * p.o_sb + static_cast<int64_t>(sq) * p.o_ss + static_cast<int64_t>(head) * p.o_sh + d4) * 2) = o2;
 }
 
-// The merge for decode with the rotary embedding folded in (Sq = 1): the splits over the cached keys (none when the
-// cache is empty), plus the new position. A row's D / 4 threads (consecutive lanes of one wavefront) rotate their 4
-// elements of the raw query and key rows exactly as rope_append_kernel does, meet for the dot product, and merge
-// (score, 1, v) as one more partial in fp32; the threads of a group's first head also write the rotated key and the
-// value into the caches at position Skv.
+// The new position of a decode step (Sq = 1) for query head `row` of a group: a row's D / 4 threads (consecutive lanes of one wavefront) rotate their 4
+// elements of the raw query and key rows exactly as rope_append_kernel does and meet for the dot product; the threads of the group's first head also write the
+// rotated key and the value into the caches at position Skv. Returns the score (times scale * log2 e); vn: this thread's 4 elements of the value.
+// live: threads without a row work on row 0 (they take part in the shuffles) and store nothing.
 template <int DT, int D>
-__global__ __launch_bounds__(256) void attention_combine_newkey_kernel(AttnParams p) {
+__device__ __forceinline__ float new_position(const AttnParams &p, int b, int hkv, int row, int d4, bool live, uint2 &vn) {
     constexpr int per_row = D / 4;
-    const int nrows = p.G;  // Sq = 1: a row is a query head of the group
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    const int bh = take_rank(p, blockIdx.y);
-    const int b = bh / p.Hkv, hkv = bh % p.Hkv;
-    // threads past the last row work on row 0 (they take part in the shuffles) and store nothing
-    const bool live = e < nrows * per_row;
-    const int row = live ? e / per_row : 0, d4 = (e % per_row) * 4;
     const bool lower = d4 < D / 2;
     const int partner = lower ? d4 + D / 2 : d4 - D / 2;
     const char *qrow = p.q + (static_cast<int64_t>(b) * p.q_sb + static_cast<int64_t>(hkv) * p.q_sg + static_cast<int64_t>(row) * p.q_sh) * 2;
@@ -554,12 +544,11 @@ __global__ __launch_bounds__(256) void attention_combine_newkey_kernel(AttnParam
         return make_uint2(rot2<DT>(own.x, c.x, oth.x, sv.x, sign), rot2<DT>(own.y, c.y, oth.y, sv.y, sign));
     };
     const uint2 qr = rotated(qrow), kr = rotated(krow);
-    const uint2 vn = *reinterpret_cast<const uint2 *>(vrow + d4 * 2);
+    vn = *reinterpret_cast<const uint2 *>(vrow + d4 * 2);
     float dot = lo_half_to_f32<DT>(qr.x) * lo_half_to_f32<DT>(kr.x) + hi_half_to_f32<DT>(qr.x) * hi_half_to_f32<DT>(kr.x) +
                 lo_half_to_f32<DT>(qr.y) * lo_half_to_f32<DT>(kr.y) + hi_half_to_f32<DT>(qr.y) * hi_half_to_f32<DT>(kr.y);
 #pragma unroll
     for (int d = 1; d < per_row; d *= 2) dot += __shfl_xor(dot, d);
-    const float x_new = dot * p.scale_log2;
     // where the new position goes: a launch argument, or the count on the device (then p.Skv is the caches' capacity, and a
     // count that has reached it leaves the caches alone)
     int64_t pos = p.Skv;
@@ -572,6 +561,22 @@ __global__ __launch_bounds__(256) void attention_combine_newkey_kernel(AttnParam
         *reinterpret_cast<uint2 *>(p.k_cache_w + (static_cast<int64_t>(b) * p.k_sb + static_cast<int64_t>(hkv) * p.k_sh + pos * p.k_ss + d4) * 2) = kr;
         *reinterpret_cast<uint2 *>(p.v_cache_w + (static_cast<int64_t>(b) * p.v_sb + static_cast<int64_t>(hkv) * p.v_sh + pos * p.v_ss + d4) * 2) = vn;
     }
+    return dot * p.scale_log2;
+}
+
+// The merge for decode with the rotary embedding folded in: the splits over the cached keys (none when the cache is empty), plus (score, 1, v) of the new
+// position as one more partial in fp32.
+template <int DT, int D>
+__global__ __launch_bounds__(256) void attention_combine_newkey_kernel(AttnParams p) {
+    constexpr int per_row = D / 4;
+    const int nrows = p.G;  // Sq = 1: a row is a query head of the group
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    const int bh = take_rank(p, blockIdx.y);
+    const int b = bh / p.Hkv, hkv = bh % p.Hkv;
+    const bool live = e < nrows * per_row;
+    const int row = live ? e / per_row : 0, d4 = (e % per_row) * 4;
+    uint2 vn;
+    const float x_new = new_position<DT, D>(p, b, hkv, row, d4, live, vn);
     if (!live) return;
 
     const int64_t split_pitch = static_cast<int64_t>(gridDim.y) * p.rows_pad * (D + 4);
@@ -612,11 +617,303 @@ __global__ __launch_bounds__(256) void attention_combine_newkey_kernel(AttnParam
     *reinterpret_cast<uint2 *>(p.o + (static_cast<int64_t>(b) * p.o_sb + static_cast<int64_t>(head) * p.o_sh + d4) * 2) = o2;
 }
 
+// attention_decode_kernel: one new position per sequence (Sq = 1) and at most 16 query heads per key/value head. A wavefront takes keys of its own, every
+// fourth 16 of the block's, through a ring of NST stages of its own in LDS: K and V rows by loads that go straight into LDS and are waited for by count, so the
+// wavefronts of a block meet once, at the end, where their (m, l, O) are merged in LDS. A block that has a head's keys for itself (one split) finishes the rows,
+// the new position included, so that no partials are written and no second launch merges them.
+//
+// Bound: HBM. 128 MiB of K and V (8 x 16 heads a rank, two ranks, 2048 positions) 55.4 -> 44.2 us with the new position (6.05 TB/s), 40 sequences on 1000 positions, 4 key/value heads
+// a rank 43.0 -> 37.5, 64 sequences on 1000, head_dim 64 33.6 -> 26; one sequence on 500 11.1 -> 10. Over 190 shapes 0.77 of the time of attention_kernel and its merge. What it took:
+// loads past the caches' replacement (53.8 -> 48.9 us on the first of these), wavefronts that walk the keys together instead of a quarter each (-> 44.4), and no
+// second launch. More stages than two are slower (16 KiB a wavefront and stage pair: more blocks share a CU instead).
+// Piece c (16 bytes) of a staged row r is in slot c ^ r (head_dim 64: c ^ ((r / 2) % 8)): the fragment reads and the transposing reads of 16 rows are conflict-free.
+constexpr int AD_KEYS = 16;
+template <int DT>
+__device__ __forceinline__ f32x4 mfma16_k16(uint2 a, uint2 b, f32x4 c) {
+    if constexpr (DT == TPAMD_BF16) {
+        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, a), __builtin_bit_cast(i16x4, b), c, 0, 0, 0);
+    } else {
+        typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
+        return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
+    }
+}
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u32x2 lds_transpose_read(uint32_t at) {  // lds_transpose_b64, unseen by the compiler (as lds_read16)
+    u32x2 v;
+    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(v) : "v"(at));
+    return v;
+}
+
+__device__ __forceinline__ void half_landed(u32x2 &r) { asm volatile("" : "+v"(r)); }
+
+template <int DT, int D, int NST>
+__global__ __launch_bounds__(256) void attention_decode_kernel(AttnParams p) {
+    constexpr int PITCH = D * 2, CPR = D / 8, RPL = 1024 / PITCH;  // bytes and 16-byte pieces of a row, rows per load
+    constexpr int LK = AD_KEYS / RPL, LPS = 2 * LK, VAT = AD_KEYS * PITCH, STAGE = 2 * VAT, RING = NST * STAGE;
+    constexpr int DK = D / 32, DT16 = D / 16, PW = D + 4;  // PW: floats of a row's partial: O, m, l
+    static_assert((NST - 1) * LPS < 64 && NST >= 2, "the count in s_waitcnt");
+    static_assert(16 * PW * 4 <= RING, "the partials take the place of the stages");
+    extern __shared__ __align__(1024) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lq = lane >> 4;
+    auto turned = [](int row) { return D == 128 ? row : (row >> 1) & 7; };
+    const int bh = take_rank(p, blockIdx.y), b = bh / p.Hkv, hkv = bh % p.Hkv;
+    int Skv = p.Skv, keys_per_split = p.keys_per_split;
+    if (p.skv_dev != nullptr) {
+        const int64_t have = *p.skv_dev;
+        Skv = have < 0 ? 0 : have < p.Skv ? static_cast<int>(have) : p.Skv;
+        keys_per_split = ((Skv + p.nsplit - 1) / p.nsplit + AT_KEYS - 1) / AT_KEYS * AT_KEYS;
+    }
+    int k_begin = blockIdx.z * keys_per_split;
+    const int k_end = k_begin + keys_per_split < Skv ? k_begin + keys_per_split : Skv;
+    if (k_begin > k_end) k_begin = k_end;  // a split behind the last key (count read on the device): an empty range
+    const int tiles = (k_end - k_begin + AD_KEYS - 1) / AD_KEYS;
+    const int n = (tiles - wave + 3) / 4;  // of this wavefront: wave, wave + 4, ...
+
+    // ---- this lane's query row (a head of the group; rows past the last: row 0, never stored) and its fragments
+    const int qr = l16 < p.G ? l16 : 0;
+    const char *qrow = p.q + (static_cast<int64_t>(b) * p.q_sb + static_cast<int64_t>(hkv) * p.q_sg + static_cast<int64_t>(qr) * p.q_sh) * 2;
+    uint4 qf[DK];
+#pragma unroll
+    for (int kk = 0; kk < DK; ++kk) qf[kk] = *reinterpret_cast<const uint4 *>(qrow + (32 * kk + 8 * lq) * 2);
+    if (p.cos != nullptr) {  // rotated as rope_append_kernel does it
+        const char *cs = p.cos + static_cast<int64_t>(b) * p.cs_b * 2, *sn = p.sin + static_cast<int64_t>(b) * p.cs_b * 2;
+#pragma unroll
+        for (int kk = 0; kk < DK / 2; ++kk) {
+            const int at = (32 * kk + 8 * lq) * 2;
+            const uint4 x1 = qf[kk], x2 = qf[kk + DK / 2];
+            const uint4 c1 = *reinterpret_cast<const uint4 *>(cs + at), c2 = *reinterpret_cast<const uint4 *>(cs + at + D);
+            const uint4 s1 = *reinterpret_cast<const uint4 *>(sn + at), s2 = *reinterpret_cast<const uint4 *>(sn + at + D);
+            qf[kk] = rot8<DT>(x1, c1, x2, s1, -1.0f);
+            qf[kk + DK / 2] = rot8<DT>(x2, c2, x1, s2, 1.0f);
+        }
+    }
+
+    f32x4 acc[DT16];
+    float m_run = -INFINITY, l_run = 0.f;  // l_run: of the keys that this lane saw
+#pragma unroll
+    for (int dt = 0; dt < DT16; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    char *ring = smem + wave * RING;
+    if (n > 0) {  // wavefront-uniform; nothing below meets the other wavefronts
+        const uint32_t k_pitch = static_cast<uint32_t>(p.k_ss) * 2, v_pitch = static_cast<uint32_t>(p.v_ss) * 2;
+        const uint32_t k_last = static_cast<uint32_t>(k_end - 1) * k_pitch, v_last = static_cast<uint32_t>(k_end - 1) * v_pitch;
+        const __amdgpu_buffer_rsrc_t k_rsrc = make_rsrc(p.k + (static_cast<int64_t>(b) * p.k_sb + static_cast<int64_t>(hkv) * p.k_sh) * 2, k_last + PITCH);
+        const __amdgpu_buffer_rsrc_t v_rsrc = make_rsrc(p.v + (static_cast<int64_t>(b) * p.v_sb + static_cast<int64_t>(hkv) * p.v_sh) * 2, v_last + PITCH);
+        const int key0 = k_begin + wave * AD_KEYS;
+        uint32_t k_row[LK], v_row[LK], piece[LK];
+#pragma unroll
+        for (int j = 0; j < LK; ++j) {
+            const int r = j * RPL + lane / CPR;
+            piece[j] = ((lane % CPR) ^ turned(r)) * 16;
+            k_row[j] = static_cast<uint32_t>(r) * k_pitch;
+            v_row[j] = static_cast<uint32_t>(r) * v_pitch;
+        }
+        // tile i of this wavefront; keys past the last one read that one (their scores are masked and their probabilities 0)
+        auto load = [&](int stage_off, int i) __attribute__((always_inline)) {
+            const uint32_t first = static_cast<uint32_t>(key0 + (i < n ? i : n - 1) * (4 * AD_KEYS));
+#pragma unroll
+            for (int j = 0; j < LK; ++j) {
+                const uint32_t at = k_row[j] + first * k_pitch;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rsrc, (lds_void *)(ring + stage_off + j * 1024), 16, static_cast<int>((at < k_last ? at : k_last) + piece[j]), 0, 0, 2);
+            }
+#pragma unroll
+            for (int j = 0; j < LK; ++j) {
+                const uint32_t at = v_row[j] + first * v_pitch;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rsrc, (lds_void *)(ring + stage_off + VAT + j * 1024), 16, static_cast<int>((at < v_last ? at : v_last) + piece[j]), 0, 0, 2);
+            }
+        };
+        unrolled<NST>([&](auto sc) { load(decltype(sc)::value * STAGE, decltype(sc)::value); });
+        const int vkey = 4 * lq + (l16 >> 2);  // the key and 8-byte piece that this lane points the transposing read at
+        const uint32_t k_rd = lds_addr_of(ring) + l16 * PITCH + (lq ^ turned(l16)) * 16;
+        const uint32_t v_rd = lds_addr_of(ring) + VAT + vkey * PITCH + (((l16 & 3) >> 1) ^ turned(vkey)) * 16 + (l16 & 1) * 8;
+        int stage_off = 0;
+        for (int i = 0; i < n; ++i) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * LPS) : "memory");
+            u32x4 kf[DK];
+            u32x2 vf[DT16];
+            // slots of the other pieces: the stages start on whole rows, so their low address bits are the slot
+            unrolled<DK>([&](auto kc) { kf[decltype(kc)::value] = lds_read16<0>((k_rd + stage_off) ^ (decltype(kc)::value * 64)); });
+            unrolled<DT16>([&](auto dc) { vf[decltype(dc)::value] = lds_transpose_read((v_rd + stage_off) ^ (decltype(dc)::value * 32)); });
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            unrolled<DK>([&](auto kc) { already_landed(kf[decltype(kc)::value]); });
+            unrolled<DT16>([&](auto dc) { half_landed(vf[decltype(dc)::value]); });
+            load(stage_off, i + NST);
+            stage_off = stage_off + STAGE == RING ? 0 : stage_off + STAGE;
+
+            // S^T = K Q^T: s[j] = score of key 4 lq + j of the tile against this lane's row
+            f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kk = 0; kk < DK; ++kk) s = mfma16<DT>(__builtin_bit_cast(uint4, kf[kk]), qf[kk], s);
+            const int k0 = key0 + i * (4 * AD_KEYS);
+            if (k0 + AD_KEYS > k_end) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s[j] = k0 + 4 * lq + j < k_end ? s[j] : -INFINITY;
+            }
+            // online softmax with lazy rescaling, as in attention_kernel
+            constexpr float LAZY = 6.0f;
+            const float neg_ref = m_run == -INFINITY ? 0.f : -m_run;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] = fmaf(s[j], p.scale_log2, neg_ref);
+            float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+            if (__any(mx > LAZY || m_run == -INFINITY)) {
+                mx = fmaxf(mx, __shfl_xor(mx, 16));
+                mx = fmaxf(mx, __shfl_xor(mx, 32));
+                const float m_abs = mx - neg_ref;
+                const bool up = m_abs > m_run + LAZY;  // false for -inf on either side
+                const float m_new = up ? m_abs : m_run;
+                const float m_use = m_new == -INFINITY ? 0.f : m_new;
+                const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+                const float move = -neg_ref - m_use;
+                m_run = m_new;
+                l_run *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < DT16; ++dt)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[dt][j] *= alpha;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s[j] += move;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] = __builtin_amdgcn_exp2f(s[j]);
+            l_run += (s[0] + s[1]) + (s[2] + s[3]);
+            // the probabilities as two parts of the tensor dtype: rounded ones, and what the rounding left
+            const uint2 hi = make_uint2(pack2_half<DT>(s[0], s[1]), pack2_half<DT>(s[2], s[3]));
+            const uint2 lo = make_uint2(pack2_half<DT>(s[0] - lo_half_to_f32<DT>(hi.x), s[1] - hi_half_to_f32<DT>(hi.x)),
+                                        pack2_half<DT>(s[2] - lo_half_to_f32<DT>(hi.y), s[3] - hi_half_to_f32<DT>(hi.y)));
+#pragma unroll
+            for (int dt = 0; dt < DT16; ++dt) {
+                acc[dt] = mfma16_k16<DT>(__builtin_bit_cast(uint2, vf[dt]), hi, acc[dt]);
+                acc[dt] = mfma16_k16<DT>(__builtin_bit_cast(uint2, vf[dt]), lo, acc[dt]);
+            }
+        }
+    }
+    l_run += __shfl_xor(l_run, 16);
+    l_run += __shfl_xor(l_run, 32);
+    // every load into the stages has landed before the partials take their place
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    float *mine = reinterpret_cast<float *>(smem) + (wave * 16 + l16) * PW;
+    if (l16 < p.G) {
+#pragma unroll
+        for (int dt = 0; dt < DT16; ++dt) *reinterpret_cast<f32x4 *>(mine + 16 * dt + 4 * lq) = acc[dt];
+        if (lq == 0) *reinterpret_cast<float2 *>(mine + D) = make_float2(m_run, l_run);
+    }
+    __syncthreads();
+    constexpr int per_row = D / 4;
+    const float *parts = reinterpret_cast<const float *>(smem);
+    const bool whole = p.nsplit == 1;
+    for (int e0 = 0; e0 < p.G * per_row; e0 += 256) {
+        const int e = e0 + tid;
+        const bool live = e < p.G * per_row;
+        const int row = live ? e / per_row : 0, d4 = (e % per_row) * 4;
+        float ms[4], M = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            ms[v] = parts[(v * 16 + row) * PW + D];
+            M = fmaxf(M, ms[v]);
+        }
+        float o[4] = {0.f, 0.f, 0.f, 0.f}, l = 0.f;
+        if (whole && p.cos != nullptr) {
+            uint2 vn;
+            const float x_new = new_position<DT, D>(p, b, hkv, row, d4, live, vn);
+            M = fmaxf(M, x_new);
+            l = exp2f(x_new - M);
+            o[0] = l * lo_half_to_f32<DT>(vn.x); o[1] = l * hi_half_to_f32<DT>(vn.x); o[2] = l * lo_half_to_f32<DT>(vn.y); o[3] = l * hi_half_to_f32<DT>(vn.y);
+        }
+        const float m_use = M == -INFINITY ? 0.f : M;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float wgt = exp2f(ms[v] - m_use);
+            const f32x4 ov = *reinterpret_cast<const f32x4 *>(parts + (v * 16 + row) * PW + d4);
+            l += wgt * parts[(v * 16 + row) * PW + D + 1];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] += wgt * ov[j];
+        }
+        if (!live) continue;
+        if (whole) {
+            const float inv = l > 0.f ? 1.0f / l : 0.f;
+            const int head = hkv * p.G + row;
+            *reinterpret_cast<uint2 *>(p.o + (static_cast<int64_t>(b) * p.o_sb + static_cast<int64_t>(head) * p.o_sh + d4) * 2) =
+                make_uint2(pack2_half<DT>(o[0] * inv, o[1] * inv), pack2_half<DT>(o[2] * inv, o[3] * inv));
+        } else {
+            float *pr = p.part + ((static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * p.rows_pad + row) * PW;
+            *reinterpret_cast<f32x4 *>(pr + d4) = f32x4{o[0], o[1], o[2], o[3]};
+            if (d4 == 0) *reinterpret_cast<float2 *>(pr + D) = make_float2(M, l);
+        }
+    }
+}
+
+// Key ranges per head of attention_decode_kernel: the count with the smallest predicted time (microseconds): a block alone reads its keys at 53 GB/s (head_dim 64: 36), all blocks together
+// at 6.1 TB/s, and several ranges cost a second launch and their partials.
+inline int decode_splits(int64_t heads, int64_t keys, int D, int cus) {
+    double best = 1e30;
+    int pick = 1;
+    const int per_cu = D == 128 ? 2 : 5;
+    const double alone = D == 128 ? 53.0e3 : 36.0e3, all = static_cast<double>(heads) * keys * D * 4.0 / 6.1e6;
+    for (int n = 1; n <= 32; ++n) {
+        const int64_t kps = ((keys + n - 1) / n + AT_KEYS - 1) / AT_KEYS * AT_KEYS;
+        if (n > 1 && (keys + kps - 1) / kps != n) continue;
+        const double turns = static_cast<double>((heads * n + per_cu * cus - 1) / (per_cu * cus));
+        const double own = turns * static_cast<double>(kps < keys ? kps : keys) * D * 4.0 / alone;
+        const double a2 = own * own, b2 = all * all;
+        const double t = sqrt(sqrt(a2 * a2 + b2 * b2)) + (n > 1 ? 2.3 + 0.25 * n : 0.0);
+        if (t < best) { best = t; pick = n; }
+    }
+    return pick;
+}
+
+template <int DT, int D>
+int launch_decode(AttnParams p, int dev, int cus, hipStream_t s) {
+    const int64_t bhs = static_cast<int64_t>(p.B) * p.Hkv * p.ranks;
+    TPAMD_REQUIRE(bhs < 65536, "attention: batch * kv heads too large for one launch");
+    int nsplit = decode_splits(bhs, p.Skv, D, cus);
+    if (tuning().attn_splits != TUNE_UNSET) nsplit = tuning().attn_splits > 0 ? tuning().attn_splits : 1;
+    p.keys_per_split = ((p.Skv + nsplit - 1) / nsplit + AT_KEYS - 1) / AT_KEYS * AT_KEYS;
+    nsplit = (p.Skv + p.keys_per_split - 1) / p.keys_per_split;
+    p.rows_pad = 16;
+    std::unique_lock<std::mutex> hold(splitk_mutex(dev), std::defer_lock);
+    if (nsplit > 1) {
+        hold.lock();
+        void *ws = nullptr;
+        const size_t need = static_cast<size_t>(nsplit) * bhs * p.rows_pad * (D + 4) * sizeof(float);
+        if (int rc = splitk_scratch(dev, s, need, scratch_reserve(cus), &ws); rc != TPAMD_OK) return rc;
+        p.part = static_cast<float *>(ws);
+        if (ws == nullptr) {  // no scratch memory: one range
+            nsplit = 1;
+            p.keys_per_split = (p.Skv + AT_KEYS - 1) / AT_KEYS * AT_KEYS;
+        }
+    }
+    p.nsplit = nsplit;
+    const dim3 grid(1, static_cast<unsigned>(bhs), nsplit);
+        constexpr int NST = 2, LDS = 4 * NST * 2 * AD_KEYS * D * 2;  // two blocks share a CU, or five for head_dim 64
+    static thread_local int configured_dev = -1;  // per instantiation and host thread
+    if (configured_dev != dev) {
+        TPAMD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_decode_kernel<DT, D, NST>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        configured_dev = dev;
+    }
+    hipLaunchKernelGGL((attention_decode_kernel<DT, D, NST>), grid, dim3(256), LDS, s, p);
+    TPAMD_HIP(hipGetLastError());
+    if (nsplit > 1) {
+        const unsigned cblocks = static_cast<unsigned>((static_cast<int64_t>(p.G) * (D / 4) + 255) / 256);
+        if (p.cos != nullptr) hipLaunchKernelGGL((attention_combine_newkey_kernel<DT, D>), dim3(cblocks, bhs), dim3(256), 0, s, p);
+        else hipLaunchKernelGGL((attention_combine_kernel<DT, D>), dim3(cblocks, bhs), dim3(256), 0, s, p);
+        TPAMD_HIP(hipGetLastError());
+    }
+    return TPAMD_OK;
+}
+
 template <int DT, int D>
 int launch(AttnParams p, int cus, hipStream_t s) {
     int dev = 0;
     TPAMD_HIP(hipGetDevice(&dev));
     const int nrows = p.G * p.Sq;
+    // Its loads address a head's keys by 32-bit byte offsets. Up to 32 keys, two tiles for its four wavefronts, stay here, although a call takes 7-10 us instead of 5-7: short
+    // greedy runs are compared token by token between the callers of both forms of this step, and small bf16 models tie exactly there. Thousands of heads on few keys are no
+    // faster there (2048 heads on 64 keys 32.9, 34.4 us).
+    const bool many_short = D == 128 && p.Skv <= 96 && static_cast<int64_t>(p.B) * p.Hkv * p.ranks >= 8ll * cus;
+    if (p.Sq == 1 && p.G <= 16 && p.Skv > 2 * AD_KEYS && tuning().attn_decode != 0 && !many_short && p.k_ss > 0 && p.v_ss > 0 &&
+        static_cast<double>(p.Skv) * p.k_ss < 1.0e9 && static_cast<double>(p.Skv) * p.v_ss < 1.0e9)
+        return launch_decode<DT, D>(p, dev, cus, s);
     constexpr int RING = D == 64 ? 4 : 2;  // tiles requested ahead by the ring kernel: 64 registers either way
     constexpr int RING_MIN_TILES = 8;      // shorter key ranges: the ring's extra loads and idle rounds cost more than it hides
     // 128 rows per block (two 16-row tiles per wavefront) once that still leaves every CU a few blocks

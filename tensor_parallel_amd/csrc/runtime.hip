@@ -37,6 +37,7 @@ Tuning read_tuning() {
     t.skinny_max_m = env_int("TPAMD_SKINNY_MAX_M");
     t.gemv_rows = env_int("TPAMD_GEMV_ROWS");
     t.stream = env_int("TPAMD_STREAM");
+    t.attn_decode = env_int("TPAMD_ATTN_DECODE");
     t.attn_splits = env_int("TPAMD_ATTN_SPLITS");
     t.attn_ring = env_int("TPAMD_ATTN_RING");
     t.copy_tile_units = env_int("TPAMD_COPY_TILE_UNITS");

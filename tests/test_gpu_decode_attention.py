@@ -1,0 +1,68 @@
+"""attention_decode_kernel (one new position, at most 16 query heads per key/value head) at the edges of its tiles, wavefronts and key ranges, against the oracle in
+float64: counts of keys around a tile of 16 and a round of four wavefronts (from 33 on: fewer are the general kernel's), forced key ranges (empty last ones among them), strided caches, NaN behind the last key."""
+import pytest
+import torch
+
+from oracle import attention as oat
+from tensor_parallel_amd import _native
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def draw(*shape, dtype, seed):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype)
+
+
+def check(got, q, k, v, scale):
+    """The general kernel's probabilities are rounded to the dtype (2^-9 in bf16) before they weigh values of one deviation, and the result is rounded once more: 2^-8
+    of a value and about 2^-9 sqrt(2 / 3) deviations, 4.5 times that for the largest of some thousand."""
+    want = torch.from_numpy(oat.attention_f64(q.float().numpy(), k.float().numpy(), v.float().numpy(), scale, True))
+    torch.testing.assert_close(got.double().cpu(), want, rtol=2.0 ** -7, atol=1e-2 * max(want.std().item(), 0.1))
+
+
+@pytest.mark.parametrize("splits", [None, 1, 3])
+@pytest.mark.parametrize("G,Hkv,D", [(1, 3, 128), (4, 2, 64), (7, 2, 128), (16, 1, 64)])
+@pytest.mark.parametrize("keys", [32, 33, 47, 48, 49, 63, 64, 65, 129, 1000])
+def test_rows_against_the_oracle(keys, G, Hkv, D, splits, monkeypatch):
+    if splits is not None:
+        monkeypatch.setenv("TPAMD_ATTN_SPLITS", str(splits))
+    _native.reload_tuning()
+    try:
+        dtype = torch.bfloat16 if keys % 2 else torch.float16
+        q = draw(2, G * Hkv, 1, D, dtype=dtype, seed=1)
+        room = [draw(2, keys + 5, Hkv, D, dtype=dtype, seed=s) for s in (2, 3)]  # positions before heads: rows far apart
+        for r in room:
+            r[:, keys:] = float("nan")
+        k, v = (r[:, :keys].transpose(1, 2) for r in room)
+        kd, vd = (r.to(DEV)[:, :keys].transpose(1, 2) for r in room)
+        check(_native.attention(q.to(DEV), kd, vd, scale=0.1, causal=True), q, k, v, 0.1)
+    finally:
+        monkeypatch.undo()
+        _native.reload_tuning()
+
+
+@pytest.mark.parametrize("splits", [1, 4])
+@pytest.mark.parametrize("G,D", [(1, 128), (4, 128), (16, 64)])
+@pytest.mark.parametrize("count", [-1, 0, 1, 63, 64, 200, 255, 256])
+def test_new_position_with_the_count_on_the_device(count, G, D, splits, monkeypatch):
+    """Against the general kernel (TPAMD_ATTN_DECODE=0): the same caches bit for bit, the same rows but for the rounding of probabilities against other maxima."""
+    monkeypatch.setenv("TPAMD_ATTN_SPLITS", str(splits))
+    B, Hkv, L, dtype = 3, 2, 256, torch.bfloat16
+    q, k, v = draw(B, 1, G * Hkv, D, dtype=dtype, seed=4), draw(B, 1, Hkv, D, dtype=dtype, seed=5), draw(B, 1, Hkv, D, dtype=dtype, seed=6)
+    cos, sin, kc, vc = draw(B, 1, D, dtype=dtype, seed=7), draw(B, 1, D, dtype=dtype, seed=8), draw(B, Hkv, L, D, dtype=dtype, seed=9), draw(B, Hkv, L, D, dtype=dtype, seed=10)
+    outs = []
+    try:
+        for general in (False, True):
+            if general:
+                monkeypatch.setenv("TPAMD_ATTN_DECODE", "0")
+            _native.reload_tuning()
+            kd, vd = kc.to(DEV), vc.to(DEV)
+            out = _native.attention_decode_rope(q.to(DEV), k.to(DEV), v.to(DEV), cos.to(DEV), sin.to(DEV), kd, vd, torch.tensor([count], device=DEV), scale=0.1)
+            outs.append((out.float().cpu(), kd.cpu(), vd.cpu()))
+    finally:
+        monkeypatch.undo()
+        _native.reload_tuning()
+    (a, ka, va), (b, kb, vb) = outs
+    assert torch.equal(ka, kb) and torch.equal(va, vb)
+    torch.testing.assert_close(a, b, rtol=2.0 ** -7, atol=1e-2 * max(b.std().item(), 0.1))
