@@ -2154,20 +2154,20 @@ int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
     // the direct kernels address a tile with 32-bit byte offsets from the tile origin and step K in tiles of 64
     const bool direct_ok = p.K % 64 == 0 && p.K >= 64 && p.ldx < (1ll << 22) && p.ldw < (1ll << 22);
     // 256 x 256 tiles or 128 x 128 tiles (with K split): whichever the cost models predict to be faster. The 256 tiles
-    // run in rounds of one per CU; fitted on the same timings, a K tile takes 1.47 us in a full round (the part is
-    // power-limited then), 1.2 us in a round that fills at most three quarters of the CUs and 1.3 us in between.
+    // run in rounds of one per CU; over 104 launches of more than half a round (the shapes of MID_TILES) a launch takes 4.8 us, a round 5.9, a K tile 1.37 in a full round
+    // (the part is power-limited then), 1.25 in a round that fills at most three quarters of the CUs and 1.42 in between.
     const int64_t big_tiles = static_cast<int64_t>((p.M + 255) / 256) * ((p.N + (swiglu ? 127 : 255)) / (swiglu ? 128 : 256));
     const int64_t small_tiles = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + (swiglu ? 63 : 127)) / (swiglu ? 64 : 128)) * p.ranks;
     const int KT = static_cast<int>(p.K / 64);
     auto rounds256 = [&](int64_t units, int kt) {
         const int64_t full = units / cus, last = units % cus;
-        return kt * (full * 1.47 + (last == 0 ? 0.0 : last * 4 <= 3ll * cus ? 1.2 : 1.3));
+        return 4.8 + 5.9 * (full + (last > 0)) + kt * (full * 1.37 + (last == 0 ? 0.0 : last * 4 <= 3ll * cus ? 1.25 : 1.42));
     };
     const double stream = stream_floor(p.N, p.K, swiglu);  // the pair 8192 x 8192 at 17 rows took 79.8 us on this tiling in four splits, predicted
                                                            // 57 without this term, and 63.8 us on the other
     auto floor256 = [&](double loop) { return loop > stream ? loop : stream; };
     double t256 = floor256(rounds256(big_tiles, KT));
-    // ... or split over K while all units still fit one round; the partial tiles cost 9 us + 0.33 us per MB (more than
+    // ... or split over K while all units still fit one round; the partial tiles cost 3 us + 0.33 us per MB (more than
     // with the small tiles: all blocks finish together, so nothing overlaps the writes and the finishing pass)
     int splits256 = 1;
     const double valid256 = static_cast<double>(p.M) / (((p.M + 255) / 256) * 256.0);
@@ -2175,7 +2175,7 @@ int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
         const int kt = (KT + sp - 1) / sp;
         if (kt < 4) break;
         const int64_t units = big_tiles * sp;
-        const double t = floor256(rounds256(units, kt)) + 9.0 + units * 0.262144 * valid256 * 0.33;
+        const double t = floor256(rounds256(units, kt)) + 3.0 + units * 0.262144 * valid256 * 0.33;
         if (t < t256) { t256 = t; splits256 = sp; }
     }
     if (tuning().gemm_splitk256 != TUNE_UNSET) splits256 = tuning().gemm_splitk256;
@@ -2183,8 +2183,8 @@ int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
     int unused_splits = 1;
     bool unused_deep = false;
     const int64_t small_tiles_m = (p.M + 127) / 128;
-    const double t128 = estimate128(small_tiles, small_tiles_m, small_tiles / small_tiles_m, KT, cus,
-                                    static_cast<double>(p.M) / (small_tiles_m * 128.0), swiglu, &unused_splits, &unused_deep);
+    const double t128 = beside_mid(estimate128(small_tiles, small_tiles_m, small_tiles / small_tiles_m, KT, cus,
+                                               static_cast<double>(p.M) / (small_tiles_m * 128.0), swiglu, &unused_splits, &unused_deep), p.M);
     if (direct_ok) {
         int tmx = 0, tnx = 0;
         if (tuning().gemm_tile != TUNE_UNSET) {
@@ -2273,8 +2273,8 @@ bool sum128_pays(int64_t M, int64_t N, int64_t K, int cus) {
     const double valid = static_cast<double>(M) / (tiles_m * 128.0);
     bool deep = false;
     int tmx = 0, tnx = 0, splits = 0;
-    const double once = estimate_sum128(tiles, tiles_n, KT, cus, valid, &splits, &deep);
-    const double t128 = estimate128(tiles, tiles_m, tiles_n, KT, cus, valid, false, &splits, &deep);
+    const double once = beside_mid(estimate_sum128(tiles, tiles_n, KT, cus, valid, &splits, &deep), M);
+    const double t128 = beside_mid(estimate128(tiles, tiles_m, tiles_n, KT, cus, valid, false, &splits, &deep), M);
     const double mid = estimate_mid(M, N, KT, cus, false, &tmx, &tnx);
     return once < 1.9 * (t128 < mid ? t128 : mid);  // where the models are equal one launch was 2-3 % slower (4544 x 7168 at 513 rows, 5120 x 8192 at 468)
 }

@@ -198,12 +198,20 @@ int launch_mid(GemmParams p, hipStream_t s) {
 
 template <int DT, int MODE>
 int launch_mid_tile(const GemmParams &p, int tmx, int tnx, hipStream_t s) {
-    switch (tmx * 16 + tnx) {
-        case 4 * 16 + 6: return launch_mid<DT, MODE, 4, 6, 3>(p, s);
-        case 4 * 16 + 8: return launch_mid<DT, MODE, 4, 8, 3>(p, s);
-        case 6 * 16 + 6: return launch_mid<DT, MODE, 6, 6, 3>(p, s);
-        case 6 * 16 + 8: return launch_mid<DT, MODE, 6, 8, 2>(p, s);
+#define MID_TILE(tmx, tnx, stages) case tmx * 16 + tnx: return launch_mid<DT, MODE, tmx, tnx, stages>(p, s)
+    switch (tmx * 16 + tnx) {  // three stages where they fit
+        MID_TILE(4, 6, 3);
+        MID_TILE(4, 8, 3);
+        MID_TILE(5, 6, 3);
+        MID_TILE(5, 8, 3);
+        MID_TILE(6, 6, 3);
+        MID_TILE(6, 8, 2);
+        MID_TILE(7, 6, 3);
+        MID_TILE(7, 8, 2);
+        MID_TILE(8, 6, 2);
+        MID_TILE(8, 8, 2);
     }
+#undef MID_TILE
     set_error("gemm: no tile of %d x %d rows", 32 * tmx, 32 * tnx);
     return TPAMD_ERR_UNSUPPORTED;
 }

@@ -9,17 +9,24 @@ inline double stream_floor(int64_t N, int64_t K, bool swiglu) { return static_ca
 
 // Predicted time (microseconds) of gemm_mid_kernel on the best of its tiles, and that tile: a launch, rounds of one block per CU, each with
 // a fixed cost (first tiles, epilogue) and a time per K tile, shorter where the last round leaves CUs idle (the part clocks higher).
-// Non-negative least squares on relative errors over 237 shapes (9 matrices at 128-8192 rows, 90 random ones), each tile forced and timed
-// inside a HIP graph. Over those, all at 128 rows or more, the choice among these tiles, the 256 x 256 and the 128 x 128 tiling is 1.7 % off the
-// best one (geometric mean; 6.4 % without these tiles) and nowhere slower than without them. Examples: the pair 5504 x 4096 at 512 rows 64 -> 51 us (128 x 192; two
-// K splits of 256 x 256 before) and at 645 rows 84 -> 60 us, 4096 x 5504 at 2103 rows 105 -> 78 us (192 x 192; 144 tiles of 256 x 256 before).
+// Non-negative least squares on relative errors over 220 shapes (128-8192 rows, 1000-16000 columns, K 1024-8192, one and two ranks), each tile forced and timed
+// inside a HIP graph. Over those the choice among these tiles, the 256 x 256 and the 128 x 128 tiling is 0.9 % off the best one (geometric mean); with four
+// of these tiles and models of the other two tilings without a cost per launch and round it was 6.8 % off. Examples (us, before -> now): the pair 5504 x 4096 of two ranks at 512
+// rows 103 -> 87 (256 x 192), at 1024 rows 177 -> 169, 16000 x 4096 of two ranks at 645 rows 188 -> 147 (224 x 192), 3072 x 4096 at 2103 rows 115 -> 91 (224 x 256: 240 tiles
+// on 256 CUs), 6144 x 4096 at 4096 rows 183 -> 166 (512 tiles of 256 x 192 instead of 384 of 256 x 256), 2048 x 5120 x 1024 64 -> 54.
 struct MidTile { int tmx, tnx; double launch, round, full, idle[3]; };  // idle: last round at most 1/2, at most 3/4, more of the CUs
-constexpr MidTile MID_TILES[2][4] = {
-    {{4, 6, 0.5, 5.0, 0.643, {0.537, 0.588, 0.693}}, {4, 8, 0.4, 5.8, 0.827, {0.663, 0.740, 0.820}},
-     {6, 6, 2.6, 6.7, 0.858, {0.635, 0.714, 0.789}}, {6, 8, 0.1, 5.4, 1.226, {0.922, 0.977, 1.211}}},
-    {{4, 6, 0.7, 3.2, 0.642, {0.661, 0.715, 0.688}}, {4, 8, 1.4, 3.6, 0.837, {0.756, 0.808, 0.832}},
-     {6, 6, 0.0, 7.2, 0.827, {0.727, 0.755, 0.820}}, {6, 8, 1.3, 2.0, 1.223, {1.099, 1.088, 1.233}}},
+constexpr MidTile MID_TILES[2][10] = {
+    {{4, 6, 2.8, 4.7, 0.659, {0.603, 0.631, 0.662}}, {4, 8, 2.8, 5.1, 0.822, {0.737, 0.785, 0.839}}, {5, 6, 2.2, 5.5, 0.758, {0.643, 0.680, 0.774}},
+     {5, 8, 3.0, 5.0, 0.989, {0.788, 0.893, 0.954}}, {6, 6, 3.4, 5.9, 0.871, {0.682, 0.745, 0.836}}, {6, 8, 2.3, 5.0, 1.154, {1.126, 1.208, 1.209}},
+     {7, 6, 4.0, 6.4, 0.991, {0.755, 0.825, 0.957}}, {7, 8, 1.6, 6.7, 1.266, {1.171, 1.236, 1.287}}, {8, 6, 3.1, 6.2, 1.159, {1.058, 1.086, 1.135}},
+     {8, 8, 2.2, 7.0, 1.381, {1.223, 1.256, 1.356}}},
+    {{4, 6, 2.9, 3.7, 0.682, {0.616, 0.631, 0.738}}, {4, 8, 3.0, 4.9, 0.846, {0.734, 0.764, 0.817}}, {5, 6, 3.1, 4.5, 0.778, {0.644, 0.697, 0.751}},
+     {5, 8, 2.5, 5.9, 0.971, {0.790, 0.871, 0.918}}, {6, 6, 2.3, 6.1, 0.866, {0.714, 0.754, 0.857}}, {6, 8, 2.9, 5.3, 1.186, {1.137, 1.199, 1.219}},
+     {7, 6, 3.3, 6.3, 0.995, {0.766, 0.818, 0.907}}, {7, 8, 3.2, 5.9, 1.304, {1.160, 1.262, 1.305}}, {8, 6, 2.5, 6.9, 1.155, {1.067, 1.091, 1.191}},
+     {8, 8, 3.8, 7.0, 1.411, {1.200, 1.282, 1.444}}},
 };
+// The prediction for the 128 x 128 tiling beside these, above 128 rows: what a fit over the same 220 shapes makes of estimate128 (gemm.hip), whose own fit has no cost per launch.
+inline double beside_mid(double estimate128_us, int64_t M) { return M > 128 ? 2.5 + 1.1 * estimate128_us : estimate128_us; }
 
 // Up to 128 rows, where nothing was fitted, at least what streaming the weights takes. Without that floor few rows of a wide matrix were
 // predicted faster than HBM and taken off the 128 x 128 tiling, where a tie leaves them (us there / on these tiles): 28672 x 4096 at
