@@ -689,6 +689,8 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnParams p) {
         }
     }
 
+    // Probabilities are kept 2^SHIFT times as large (at most 2^15): the smaller of their two parts is then normal in fp16 down to 2^-13 and not zero down to 2^-23.
+    constexpr float SHIFT = DT == TPAMD_F16 ? 9.0f : 0.0f, LESS = DT == TPAMD_F16 ? 1.0f - 0x1p-10f : 1.0f - 0x1p-7f;  // less than 1 by two roundings of the dtype
     f32x4 acc[DT16];
     float m_run = -INFINITY, l_run = 0.f;  // l_run: of the keys that this lane saw
 #pragma unroll
@@ -748,6 +750,11 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnParams p) {
             if (k0 + AD_KEYS > k_end) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) s[j] = k0 + 4 * lq + j < k_end ? s[j] : -INFINITY;
+                // and their values are zero: the last key's, which were loaded in their place, may be infinite
+                const int have = k_end - k0 - 4 * lq;
+                const uint32_t m0 = have >= 2 ? 0xffffffffu : have == 1 ? 0xffffu : 0u, m1 = have >= 4 ? 0xffffffffu : have == 3 ? 0xffffu : 0u;
+#pragma unroll
+                for (int dt = 0; dt < DT16; ++dt) vf[dt] &= u32x2{m0, m1};
             }
             // online softmax with lazy rescaling, as in attention_kernel
             constexpr float LAZY = 6.0f;
@@ -774,10 +781,11 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnParams p) {
                 for (int j = 0; j < 4; ++j) s[j] += move;
             }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) s[j] = __builtin_amdgcn_exp2f(s[j]);
+            for (int j = 0; j < 4; ++j) s[j] = __builtin_amdgcn_exp2f(s[j] + SHIFT);
             l_run += (s[0] + s[1]) + (s[2] + s[3]);
-            // the probabilities as two parts of the tensor dtype: rounded ones, and what the rounding left
-            const uint2 hi = make_uint2(pack2_half<DT>(s[0], s[1]), pack2_half<DT>(s[2], s[3]));
+            // the probabilities as two parts of the tensor dtype: one rounded that is always the smaller, and what is left. Both are above zero (an infinite value times a rest of
+            // zero, or of the other sign, would be NaN)
+            const uint2 hi = make_uint2(pack2_half<DT>(s[0] * LESS, s[1] * LESS), pack2_half<DT>(s[2] * LESS, s[3] * LESS));
             const uint2 lo = make_uint2(pack2_half<DT>(s[0] - lo_half_to_f32<DT>(hi.x), s[1] - hi_half_to_f32<DT>(hi.x)),
                                         pack2_half<DT>(s[2] - lo_half_to_f32<DT>(hi.y), s[3] - hi_half_to_f32<DT>(hi.y)));
 #pragma unroll
@@ -796,7 +804,7 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnParams p) {
     if (l16 < p.G) {
 #pragma unroll
         for (int dt = 0; dt < DT16; ++dt) *reinterpret_cast<f32x4 *>(mine + 16 * dt + 4 * lq) = acc[dt];
-        if (lq == 0) *reinterpret_cast<float2 *>(mine + D) = make_float2(m_run, l_run);
+        if (lq == 0) *reinterpret_cast<float2 *>(mine + D) = make_float2(m_run - SHIFT, l_run);
     }
     __syncthreads();
     constexpr int per_row = D / 4;
@@ -885,7 +893,7 @@ int launch_decode(AttnParams p, int dev, int cus, hipStream_t s) {
     }
     p.nsplit = nsplit;
     const dim3 grid(1, static_cast<unsigned>(bhs), nsplit);
-        constexpr int NST = 2, LDS = 4 * NST * 2 * AD_KEYS * D * 2;  // two blocks share a CU, or five for head_dim 64
+    constexpr int NST = 2, LDS = 4 * NST * 2 * AD_KEYS * D * 2;  // two blocks share a CU, or five for head_dim 64
     static thread_local int configured_dev = -1;  // per instantiation and host thread
     if (configured_dev != dev) {
         TPAMD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_decode_kernel<DT, D, NST>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));

@@ -42,6 +42,23 @@ def test_rows_against_the_oracle(keys, G, Hkv, D, splits, monkeypatch):
         _native.reload_tuning()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("keys,at", [(64, 0), (64, 63), (65, 64), (75, 74), (79, 33), (1000, 999)])
+def test_an_infinite_value_stays_infinite(keys, at, D, dtype):
+    """One infinite element among the values: its column is infinite, as in the general kernel, and no other is touched. Equal scores make all probabilities one."""
+    q, k, v = (draw(2, 2, n, D, dtype=dtype, seed=s).to(DEV) for n, s in ((1, 1), (keys, 2), (keys, 3)))
+    q.zero_()
+    v[1, 1, at, 5] = float("inf")
+    v[0, 1, at, D - 1] = float("-inf")
+    got = _native.attention(q, k, v, scale=0.1, causal=True).float()
+    want = v.float().mean(2, keepdim=True).transpose(1, 2)
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and not torch.isnan(got).any()
+    finite = torch.isfinite(want)
+    # sums of up to 1000 values in fp32, rounded once to the dtype
+    torch.testing.assert_close(got[finite], want[finite], rtol=2.0 ** (-8 if dtype is torch.bfloat16 else -11), atol=1e-5)
+
+
 @pytest.mark.parametrize("splits", [1, 4])
 @pytest.mark.parametrize("G,D", [(1, 128), (4, 128), (16, 64)])
 @pytest.mark.parametrize("count", [-1, 0, 1, 63, 64, 200, 255, 256])
