@@ -14,7 +14,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 OUT_DIR = PKG / "_lib"
 LIB = OUT_DIR / "libtpamd.so"
-SOURCES = ["api.hip", "runtime.hip", "noalloc.hip", "slice.hip", "reduce.hip", "gemm.hip", "gemm_mid.hip", "skinny.hip", "stream.hip", "attention.hip", "rope.hip", "norm.hip", "mask.hip"]
+SOURCES = ["api.hip", "runtime.hip", "noalloc.hip", "slice.hip", "reduce.hip", "gemm.hip", "gemm_mid.hip", "skinny.hip", "stream.hip", "stream_w8.hip", "attention.hip", "rope.hip", "norm.hip", "mask.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

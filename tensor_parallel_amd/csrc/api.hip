@@ -388,7 +388,7 @@ extern "C" int tpamd_linear_sum_ranks(const void *const *x_dev, const void *cons
     return TPAMD_ERR_UNSUPPORTED;
 }
 
-// The same for int8 weights on 2 to 64 rows whose kernels split K over blocks.
+// The same for int8 weights on 2 to 64 rows: stream_w8_kernel, or kernels that split K over blocks.
 extern "C" int tpamd_linear_w8_sum_ranks(const tpamd_w8_rank *ranks, int64_t n_out, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout,
                                          int64_t ldy, int dtype, void *stream) {
     const char *who = "tpamd_linear_w8_sum_ranks";

@@ -76,5 +76,8 @@ __device__ __forceinline__ void skinny_store_sum(const SkinnyParams &p, float s0
 // the launch (operands of mfma_ok).
 bool stream_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int ranks, bool swiglu, bool sum, int cus);
 int stream_dispatch(const SkinnyParams &p, int dtype, bool swiglu, hipStream_t s);
+// stream_w8.hip, the same for int8 weights.
+bool stream_w8_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t n_out, int ranks, bool sum, int cus);
+int stream_w8_dispatch(const SkinnyParams &p, int dtype, hipStream_t s);
 
 }  // namespace tpamd

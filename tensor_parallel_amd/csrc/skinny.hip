@@ -1572,7 +1572,7 @@ int launch_resident(const SkinnyParams &p, int cus, hipStream_t s) {
     return TPAMD_OK;
 }
 
-// Which of the three int8 kernels takes 2 to 64 rows: the K-split kernel whose wavefronts own columns ("cols": x of the
+// Which of these three int8 kernels takes 2 to 64 rows that stream_w8_kernel does not (stream_w8_pays): the K-split kernel whose wavefronts own columns ("cols": x of the
 // split in LDS, fp32 partial planes, a finishing pass), the older K-split kernel ("split": x in registers) or the unsplit
 // one. Fitted on a sweep of 600 shapes (N 2048-28672, K 2048-16384, 2-64 rows, each kernel forced, inside a HIP graph on
 // weights that rotate through more memory than the caches hold) and checked on 290 random ones: 0.8 % and 0.7 % off the
@@ -2025,6 +2025,7 @@ int skinny_dispatch(const void *x, const void *w, const void *w2, const void *bi
     TPAMD_HIP(hipGetDevice(&dev));
     if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
     if (!w8 && stream_pays(M, N, K, ldx, ldw, p.ranks, swiglu, false, cus)) return stream_dispatch(p, dtype, swiglu, s);
+    if (w8 && stream_w8_pays(M, N, K, ldx, ldw, n_out, p.ranks, false, cus)) return stream_w8_dispatch(p, dtype, s);
     // 2 and 3 rows of int8 weights are faster through the K-split kernel where it applies
     if (w8 && M >= 2 && M <= GEMV_MAX_M) {
         bool done = false;
@@ -2093,7 +2094,7 @@ int skinny_sum_dispatch(const void *x, const void *w, const void *bias, const Ra
     return TPAMD_OK;
 }
 
-// The same for int8 weights (2 <= M <= 64) where K is split over blocks: the finishing pass adds both ranks' planes. *done = false: not taken.
+// The same for int8 weights (2 <= M <= 64): stream_w8_kernel, or where K is split over blocks, whose finishing pass adds both ranks' planes. *done = false: not taken.
 int skinny_w8_sum_dispatch(const void *x, const void *wq, const void *scale, const void *outlier_idx, const void *w_out, int64_t n_out, const void *bias,
                            const RankStep &to, void *y, int64_t copy, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ld_wout, int64_t ldy,
                            int dtype, hipStream_t s, bool *done) {
@@ -2115,6 +2116,13 @@ int skinny_w8_sum_dispatch(const void *x, const void *wq, const void *scale, con
     p.M = static_cast<int>(M); p.N = static_cast<int>(N); p.K = static_cast<int>(K);
     p.n_out = static_cast<int>(n_out);
     p.ldx = ldx; p.ldw = ldw; p.ldy = ldy; p.ld_wout = ld_wout;
+    int dev = 0, cus = 256;
+    TPAMD_HIP(hipGetDevice(&dev));
+    if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
+    if (stream_w8_pays(M, N, K, ldx, ldw, n_out, 2, true, cus)) {
+        *done = true;
+        return stream_w8_dispatch(p, dtype, s);
+    }
     int rc = dtype == TPAMD_BF16 ? launch_w8_cols<TPAMD_BF16>(p, s, done) : launch_w8_cols<TPAMD_F16>(p, s, done);
     if (rc != TPAMD_OK || *done) return rc;
     return dtype == TPAMD_BF16 ? launch_w8_split<TPAMD_BF16>(p, s, done) : launch_w8_split<TPAMD_F16>(p, s, done);
