@@ -226,7 +226,7 @@ static bool stream_cut(int64_t N, int ranks, bool swiglu, bool sum, int cus, int
 //  - Linears of 3 to 16 rows: up to 12288 columns of both ranks (0.76-1.0), and where the other kernels are at their worst: K over 8192 (0.69-0.95), more than 8 rows
 //    on wide matrices of short rows (9216 x 2048 a rank 0.75). Others 1.03-1.1. Pairs: K over 8192 (0.84-0.98), more than 8 rows on short rows that are not whole KiB (0.86-0.95).
 //  - of 17 to 64 rows: one block per CU holds all columns (Linears 0.58-0.95 within the limit on x, pairs 0.63-1.0), or two take turns up to 32 rows (0.79-0.98); pairs in two
-//    turns 0.70-0.94. Short rows of wide matrices are left out (11008 x 1408 at 47 rows 16.6 -> 20.0 us), and pairs whose staged rows would be a tenth padding (6912 x 5120 1.06-1.27).
+//    turns 0.70-0.94; Linears in two turns at 34 to 64 rows 1.03-1.30 (16000 x 4096 of two ranks at 40 rows, fp16, 52.6 -> 57.7 us). Short rows of wide matrices are left out (11008 x 1408 at 47 rows 16.6 -> 20.0 us), and pairs whose staged rows would be a tenth padding (6912 x 5120 1.06-1.27).
 bool stream_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int ranks, bool swiglu, bool sum, int cus) {
     int blocks = 0, rows = 0, groups = 0;
     if (tuning().stream == 0 || M < 2 || M > 64 || K % 64 != 0 || K < 64 || ldx >= (1ll << 22) || ldw >= (1ll << 22) || cus < ranks) return false;

@@ -75,7 +75,7 @@ def test_falcon_mlp_shard_full_shape():
 @pytest.mark.parametrize("M", [1, 2, 4, 16, 32, 64])
 def test_falcon_mlp_shard_full_shape_every_decode_batch(M):
     """BASELINE config 5 at its real shape through the DEFAULT dispatch at batch 1, 16, 32 and 64 (the row-streaming
-    kernel at 1, the K-split kernel whose wavefronts own columns from 2 rows on at this size): both matrices against the closed-form definition in
+    kernel at 1, the one-block-per-CU kernel from 2 rows on, at 64 the K-split kernel whose wavefronts own columns): both matrices against the closed-form definition in
     float64. The down projection is fed the device's own hidden activations."""
     d, f = 8192, 16384
     x, wq1, s1, c1, o1 = make_case(M, f, d, 41, torch.float16, 0)
