@@ -219,6 +219,16 @@ static bool stream_cut(int64_t N, int ranks, bool swiglu, bool sum, int cus, int
     return false;
 }
 
+// Whether the environment names another kernel for such a launch: a choice among those that took it before, by the switches that these read at its rows. (Not those that
+// choose a form of one of them: TPAMD_GEMM_W4, _STAGES, _PART_X.)
+static bool other_kernel_named(int64_t M, bool swiglu) {
+    const Tuning &t = tuning();
+    auto set = [](int knob) { return knob != TUNE_UNSET; };
+    if (set(t.skinny_cg) || set(t.skinny_resident) || (swiglu && (set(t.skinny_pair) || set(t.skinny_xlds)))) return true;
+    if (M > 16) return set(t.skinny_max_m) || set(t.gemm_tile) || set(t.gemm_splitk) || set(t.gemm_splitk256);
+    return M <= 3 && set(t.gemv_rows);
+}
+
 // Where stream_kernel is the faster one. Fitted on 500 shapes of both ranks, timed in a HIP graph on rotated weights against the kernels that took them before
 // (TPAMD_STREAM=0 and =1); by rows:
 //  - a sum of two ranks: 2 to 16 rows always (0.72-1.0 of the time; two rows of a narrow matrix stay with the row kernel), above while a CU reads x in less time than
@@ -232,6 +242,7 @@ bool stream_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int 
     if (tuning().stream == 0 || M < 2 || M > 64 || K % 64 != 0 || K < 64 || ldx >= (1ll << 22) || ldw >= (1ll << 22) || cus < ranks) return false;
     if (!stream_cut(N, ranks, swiglu, sum, cus, &blocks, &rows, &groups)) return false;
     if (tuning().stream == 1) return true;
+    if (other_kernel_named(M, swiglu)) return false;
     const int64_t all = N * (sum ? 1 : ranks);
     const int cols = static_cast<int>((N + blocks - 1) / blocks) * (swiglu ? 2 : 1);
     const bool full = cols * 10 >= rows * 9;

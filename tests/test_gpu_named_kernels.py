@@ -1,0 +1,65 @@
+"""A switch that names a kernel (TPAMD_SKINNY_*, TPAMD_GEMV_ROWS, TPAMD_GEMM_TILE and its K splits) is followed also where the rule would have taken
+stream_kernel. Which kernel ran is seen in the bits: both sides sum in fixed orders of their own, and of some ten thousand rounded sums some
+differ between two orders."""
+import pytest
+import torch
+
+from tensor_parallel_amd import _native
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def draw(*shape, seed, scale=1.0):
+    return (torch.randn(*shape, device=DEV, generator=torch.Generator(device=DEV).manual_seed(seed)) * scale).half()
+
+
+def linear(rows, cols, K):
+    x, w = draw(rows, K, seed=1), draw(cols, K, seed=2, scale=0.05)
+    return lambda: _native.linear(x, w)
+
+
+def pair(rows, cols, K):
+    x, g, u = draw(rows, K, seed=1), draw(cols, K, seed=2, scale=0.05), draw(cols, K, seed=3, scale=0.05)
+    return lambda: _native.swiglu_up(x, g, u)
+
+
+def sums(rows, cols, K):
+    calls = [(draw(rows, K, seed=r), draw(cols, K, seed=5 + r, scale=0.05), None) for r in range(2)]
+
+    def run():
+        both = _native.linear_sum_ranks(calls)  # None: two launches
+        return both[0] if both is not None else _native.linear(*calls[1], addend=_native.linear(*calls[0]))
+
+    return run
+
+
+@pytest.mark.parametrize("make,rows,cols,K,knobs", [
+    (linear, 12, 5504, 4096, {"TPAMD_SKINNY_RESIDENT": 1}),
+    (linear, 12, 5504, 4096, {"TPAMD_SKINNY_CG": 2}),
+    (linear, 3, 4096, 4096, {"TPAMD_GEMV_ROWS": 8}),
+    (linear, 40, 4608, 2048, {"TPAMD_SKINNY_MAX_M": 64}),
+    (linear, 40, 4608, 2048, {"TPAMD_SKINNY_MAX_M": 16}),
+    (linear, 40, 4608, 2048, {"TPAMD_GEMM_TILE": 128, "TPAMD_GEMM_SPLITK": 8}),
+    (linear, 48, 4608, 2048, {"TPAMD_GEMM_TILE": 256, "TPAMD_GEMM_SPLITK256": 3}),
+    (linear, 24, 4608, 4096, {"TPAMD_GEMM_TILE": 128192}),
+    (pair, 12, 5504, 11008, {"TPAMD_SKINNY_XLDS": 0}),
+    (pair, 12, 5504, 11008, {"TPAMD_SKINNY_PAIR": 0, "TPAMD_SKINNY_XLDS": 0}),
+    (pair, 40, 5504, 4096, {"TPAMD_GEMM_TILE": 128}),
+    (sums, 24, 4096, 4096, {"TPAMD_GEMM_TILE": 128, "TPAMD_GEMM_SPLITK": 4}),
+    (sums, 24, 4096, 4096, {"TPAMD_SKINNY_MAX_M": 16}),
+])
+def test_a_named_kernel_runs(make, rows, cols, K, knobs, tune):
+    run = make(rows, cols, K)
+    chosen = run()
+    tune("TPAMD_STREAM", 1)
+    stream = run()
+    assert torch.equal(chosen, stream)  # a shape that the rule takes
+    for knob, value in knobs.items():
+        tune(knob, value)
+    assert torch.equal(run(), stream)  # named as well: TPAMD_STREAM=1 comes first
+    tune("TPAMD_STREAM", 0)
+    named = run()
+    assert not torch.equal(named, stream)
+    tune("TPAMD_STREAM", "")  # as if it were not set
+    assert torch.equal(run(), named)
