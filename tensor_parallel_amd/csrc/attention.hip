@@ -918,8 +918,9 @@ int launch(AttnParams p, int cus, hipStream_t s) {
     // Its loads address a head's keys by 32-bit byte offsets. Up to 32 keys, two tiles for its four wavefronts, stay here, although a call takes 7-10 us instead of 5-7: short
     // greedy runs are compared token by token between the callers of both forms of this step, and small bf16 models tie exactly there. Thousands of heads on few keys are no
     // faster there (2048 heads on 64 keys 32.9, 34.4 us).
+    // TPAMD_ATTN_RING names a form of the general kernel.
     const bool many_short = D == 128 && p.Skv <= 96 && static_cast<int64_t>(p.B) * p.Hkv * p.ranks >= 8ll * cus;
-    if (p.Sq == 1 && p.G <= 16 && p.Skv > 2 * AD_KEYS && tuning().attn_decode != 0 && !many_short && p.k_ss > 0 && p.v_ss > 0 &&
+    if (p.Sq == 1 && p.G <= 16 && p.Skv > 2 * AD_KEYS && tuning().attn_decode != 0 && tuning().attn_ring == TUNE_UNSET && !many_short && p.k_ss > 0 && p.v_ss > 0 &&
         static_cast<double>(p.Skv) * p.k_ss < 1.0e9 && static_cast<double>(p.Skv) * p.v_ss < 1.0e9)
         return launch_decode<DT, D>(p, dev, cus, s);
     constexpr int RING = D == 64 ? 4 : 2;  // tiles requested ahead by the ring kernel: 64 registers either way

@@ -1,5 +1,5 @@
-"""A switch that names a kernel (TPAMD_SKINNY_*, TPAMD_GEMV_ROWS, TPAMD_GEMM_TILE and its K splits) is followed also where the rule would have taken
-stream_kernel. Which kernel ran is seen in the bits: both sides sum in fixed orders of their own, and of some ten thousand rounded sums some
+"""A switch that names a kernel (TPAMD_SKINNY_*, TPAMD_GEMV_ROWS, TPAMD_GEMM_TILE and its K splits, TPAMD_ATTN_RING) is followed also where the rules would have taken
+stream_kernel or attention_decode_kernel. Which kernel ran is seen in the bits: both sides sum in fixed orders of their own, and of some ten thousand rounded sums some
 differ between two orders."""
 import pytest
 import torch
@@ -62,4 +62,17 @@ def test_a_named_kernel_runs(make, rows, cols, K, knobs, tune):
     named = run()
     assert not torch.equal(named, stream)
     tune("TPAMD_STREAM", "")  # as if it were not set
+    assert torch.equal(run(), named)
+
+
+@pytest.mark.parametrize("ring", [0, 1])
+@pytest.mark.parametrize("D", [64, 128])
+def test_a_named_form_of_the_general_attention_kernel_runs(D, ring, tune):
+    q, k, v = draw(8, 16, 1, D, seed=1), draw(8, 16, 700, D, seed=2), draw(8, 16, 700, D, seed=3)
+    run = lambda: _native.attention(q, k, v, causal=True)
+    decode = run()
+    tune("TPAMD_ATTN_RING", ring)
+    named = run()
+    assert not torch.equal(named, decode)
+    tune("TPAMD_ATTN_DECODE", 0)
     assert torch.equal(run(), named)
