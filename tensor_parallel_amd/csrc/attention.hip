@@ -915,13 +915,14 @@ int launch(AttnParams p, int cus, hipStream_t s) {
     int dev = 0;
     TPAMD_HIP(hipGetDevice(&dev));
     const int nrows = p.G * p.Sq;
-    // Its loads address a head's keys by 32-bit byte offsets. Up to 32 keys, two tiles for its four wavefronts, stay here, although a call takes 7-10 us instead of 5-7: short
-    // greedy runs are compared token by token between the callers of both forms of this step, and small bf16 models tie exactly there. Thousands of heads on few keys are no
-    // faster there (2048 heads on 64 keys 32.9, 34.4 us).
-    // TPAMD_ATTN_RING names a form of the general kernel.
+    // attention_decode_kernel from the first key on (1 to 1024 heads on 16 and 32 keys: 0.64 of the general kernel's time with a new position, at most 0.77; 0.92 without, at
+    // most 1.05), so that a step takes one kernel whether the count of keys is known here or only the capacity of the caches. Its loads address a head's keys, the tile
+    // behind the last one included, by 32-bit byte offsets. Thousands of heads on few keys are no faster
+    // there (2048 heads on 64 keys 32.9, 34.4 us). TPAMD_ATTN_RING names a form of the general kernel.
     const bool many_short = D == 128 && p.Skv <= 96 && static_cast<int64_t>(p.B) * p.Hkv * p.ranks >= 8ll * cus;
-    if (p.Sq == 1 && p.G <= 16 && p.Skv > 2 * AD_KEYS && tuning().attn_decode != 0 && tuning().attn_ring == TUNE_UNSET && !many_short && p.k_ss > 0 && p.v_ss > 0 &&
-        static_cast<double>(p.Skv) * p.k_ss < 1.0e9 && static_cast<double>(p.Skv) * p.v_ss < 1.0e9)
+    const double reach = static_cast<double>(p.Skv) + AD_KEYS;
+    if (p.Sq == 1 && p.G <= 16 && p.Skv > 0 && tuning().attn_decode != 0 && tuning().attn_ring == TUNE_UNSET && !many_short && p.k_ss > 0 && p.v_ss > 0 &&
+        reach * p.k_ss < 1.0e9 && reach * p.v_ss < 1.0e9)
         return launch_decode<DT, D>(p, dev, cus, s);
     constexpr int RING = D == 64 ? 4 : 2;  // tiles requested ahead by the ring kernel: 64 registers either way
     constexpr int RING_MIN_TILES = 8;      // shorter key ranges: the ring's extra loads and idle rounds cost more than it hides

@@ -1,5 +1,5 @@
 """attention_decode_kernel (one new position, at most 16 query heads per key/value head) at the edges of its tiles, wavefronts and key ranges, against the oracle in
-float64: counts of keys around a tile of 16 and a round of four wavefronts (from 33 on: fewer are the general kernel's), forced key ranges (empty last ones among them), strided caches, NaN behind the last key."""
+float64: counts of keys around a tile of 16 and a round of four wavefronts, forced key ranges (empty last ones among them), strided caches, NaN behind the last key."""
 import pytest
 import torch
 
@@ -23,7 +23,7 @@ def check(got, q, k, v, scale):
 
 @pytest.mark.parametrize("splits", [None, 1, 3])
 @pytest.mark.parametrize("G,Hkv,D", [(1, 3, 128), (4, 2, 64), (7, 2, 128), (16, 1, 64)])
-@pytest.mark.parametrize("keys", [32, 33, 47, 48, 49, 63, 64, 65, 129, 1000])
+@pytest.mark.parametrize("keys", [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 129, 1000])
 def test_rows_against_the_oracle(keys, G, Hkv, D, splits, monkeypatch):
     if splits is not None:
         monkeypatch.setenv("TPAMD_ATTN_SPLITS", str(splits))
@@ -57,6 +57,20 @@ def test_an_infinite_value_stays_infinite(keys, at, D, dtype):
     finite = torch.isfinite(want)
     # sums of up to 1000 values in fp32, rounded once to the dtype
     torch.testing.assert_close(got[finite], want[finite], rtol=2.0 ** (-8 if dtype is torch.bfloat16 else -11), atol=1e-5)
+
+
+@pytest.mark.parametrize("G,D", [(1, 128), (16, 64)])
+@pytest.mark.parametrize("count", [1, 15, 16, 17, 31, 32, 33, 64])
+def test_few_keys_take_one_kernel_wherever_the_count_is(count, G, D):
+    """A step on a cache of fixed length, whose count is on the device, and on a cache that holds just these keys: one range on the same kernel, so the same bits."""
+    B, Hkv, dtype = 3, 2, torch.bfloat16
+    q, k, v, cos, sin = (draw(B, 1, n, D, dtype=dtype, seed=s).to(DEV) for n, s in ((G * Hkv, 4), (Hkv, 5), (Hkv, 6), (1, 7), (1, 8)))
+    cos, sin = cos[:, 0], sin[:, 0]
+    kc, vc = (draw(B, Hkv, 65, D, dtype=dtype, seed=s).to(DEV) for s in (9, 10))
+    k1, v1, k2, v2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
+    grown = _native.attention_decode_rope(q, k, v, cos, sin, k1, v1, count, scale=0.1)
+    fixed = _native.attention_decode_rope(q, k, v, cos, sin, k2, v2, torch.tensor([count], device=DEV), scale=0.1)
+    assert torch.equal(grown, fixed) and torch.equal(k1, k2) and torch.equal(v1, v2)
 
 
 @pytest.mark.parametrize("splits", [1, 4])
