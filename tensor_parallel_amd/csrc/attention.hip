@@ -917,12 +917,16 @@ int launch(AttnParams p, int cus, hipStream_t s) {
     const int nrows = p.G * p.Sq;
     // attention_decode_kernel from the first key on (1 to 1024 heads on 16 and 32 keys: 0.64 of the general kernel's time with a new position, at most 0.77; 0.92 without, at
     // most 1.05), so that a step takes one kernel whether the count of keys is known here or only the capacity of the caches. Its loads address a head's keys, the tile
-    // behind the last one included, by 32-bit byte offsets. Thousands of heads on few keys are no faster
-    // there (2048 heads on 64 keys 32.9, 34.4 us). TPAMD_ATTN_RING names a form of the general kernel.
-    const bool many_short = D == 128 && p.Skv <= 96 && static_cast<int64_t>(p.B) * p.Hkv * p.ranks >= 8ll * cus;
+    // behind the last one included, by 32-bit byte offsets.
+    // Left to the general kernel (which a TPAMD_ATTN_RING names too): 33 to 64 keys without a new position, one tile of it, for a handful of heads or for hundreds (us
+    // there / here: 8 heads 4.1 / 4.5, 512 7.2 / 8.9; 16 to 256 heads 0.93-1.05; of 64 elements 8 heads 3.2 / 3.7, 1024 6.7 / 8.0), and thousands of heads on few keys
+    // (2048 on 64 32.9 / 34.4).
+    const int64_t heads = static_cast<int64_t>(p.B) * p.Hkv * p.ranks;
+    const bool one_tile = p.cos == nullptr && p.Skv > 2 * AD_KEYS && p.Skv <= AT_KEYS && (heads <= 8 || heads * D >= 160ll * cus);
+    const bool many_short = D == 128 && p.Skv <= 96 && heads >= 8ll * cus;
+    const bool here = tuning().attn_decode != TUNE_UNSET ? tuning().attn_decode != 0 : tuning().attn_ring == TUNE_UNSET && !one_tile && !many_short;
     const double reach = static_cast<double>(p.Skv) + AD_KEYS;
-    if (p.Sq == 1 && p.G <= 16 && p.Skv > 0 && tuning().attn_decode != 0 && tuning().attn_ring == TUNE_UNSET && !many_short && p.k_ss > 0 && p.v_ss > 0 &&
-        reach * p.k_ss < 1.0e9 && reach * p.v_ss < 1.0e9)
+    if (here && p.Sq == 1 && p.G <= 16 && p.Skv > 0 && p.k_ss > 0 && p.v_ss > 0 && reach * p.k_ss < 1.0e9 && reach * p.v_ss < 1.0e9)
         return launch_decode<DT, D>(p, dev, cus, s);
     constexpr int RING = D == 64 ? 4 : 2;  // tiles requested ahead by the ring kernel: 64 registers either way
     constexpr int RING_MIN_TILES = 8;      // shorter key ranges: the ring's extra loads and idle rounds cost more than it hides

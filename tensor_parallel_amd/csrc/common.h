@@ -54,7 +54,7 @@ struct Tuning {
     int skinny_xlds;         // TPAMD_SKINNY_XLDS: 0 = gated pair at 4-16 rows through the older kernels
     int gemv_rows;           // TPAMD_GEMV_ROWS: wavefronts per block of the unrolled M <= 3 kernel (4, 8, 16); 0 = the general kernel, -1 = the MFMA kernels
     int stream;              // TPAMD_STREAM: 0 = no launch on stream_kernel and stream_w8_kernel, 1 = every launch that they take
-    int attn_decode;         // TPAMD_ATTN_DECODE: 0 = one new position per sequence through the general attention kernel
+    int attn_decode;         // TPAMD_ATTN_DECODE: 0 = one new position per sequence through the general attention kernel, 1 = every such call that attention_decode_kernel takes
     int attn_splits;         // TPAMD_ATTN_SPLITS: key-range splits of the attention kernel
     int attn_ring;           // TPAMD_ATTN_RING: 1 / 0 = the few-row attention kernel with / without several K / V tiles in flight
     int copy_tile_units;     // TPAMD_COPY_TILE_UNITS: 16-byte units per copy tile

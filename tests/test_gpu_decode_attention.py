@@ -1,5 +1,5 @@
 """attention_decode_kernel (one new position, at most 16 query heads per key/value head) at the edges of its tiles, wavefronts and key ranges, against the oracle in
-float64: counts of keys around a tile of 16 and a round of four wavefronts, forced key ranges (empty last ones among them), strided caches, NaN behind the last key."""
+float64 (TPAMD_ATTN_DECODE=1 sends it what its rule would leave to the general kernel): counts of keys around a tile of 16 and a round of four wavefronts, forced key ranges (empty last ones among them), strided caches, NaN behind the last key."""
 import pytest
 import torch
 
@@ -27,6 +27,7 @@ def check(got, q, k, v, scale):
 def test_rows_against_the_oracle(keys, G, Hkv, D, splits, monkeypatch):
     if splits is not None:
         monkeypatch.setenv("TPAMD_ATTN_SPLITS", str(splits))
+    monkeypatch.setenv("TPAMD_ATTN_DECODE", "1")
     _native.reload_tuning()
     try:
         dtype = torch.bfloat16 if keys % 2 else torch.float16

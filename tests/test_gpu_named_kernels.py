@@ -76,3 +76,17 @@ def test_a_named_form_of_the_general_attention_kernel_runs(D, ring, tune):
     assert not torch.equal(named, decode)
     tune("TPAMD_ATTN_DECODE", 0)
     assert torch.equal(run(), named)
+
+
+@pytest.mark.parametrize("heads,keys,D,general", [(8, 64, 128, True), (4, 33, 64, True), (8, 32, 128, False), (8, 65, 128, False), (32, 64, 128, False), (320, 60, 128, True),
+                                                  (512, 64, 64, False), (640, 64, 64, True)])
+def test_one_tile_of_keys_takes_the_faster_attention_kernel(heads, keys, D, general, tune):
+    """33 to 64 keys without a new position, where attention_decode_kernel measured slower (256 CUs)."""
+    q, k, v = draw(heads // 4, 4, 1, D, seed=1), draw(heads // 4, 4, keys, D, seed=2), draw(heads // 4, 4, keys, D, seed=3)
+    run = lambda: _native.attention(q, k, v, causal=True)
+    chosen = run()
+    both = []
+    for decode in (0, 1):
+        tune("TPAMD_ATTN_DECODE", decode)
+        both.append(run())
+    assert not torch.equal(*both) and torch.equal(chosen, both[0 if general else 1])
