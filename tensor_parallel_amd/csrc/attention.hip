@@ -19,6 +19,7 @@
 // (tpamd_attention_decode_rope) the kernel also applies the rotary embedding to its Q fragments, and the merge
 // (attention_combine_newkey_kernel) adds the new position's key and value and writes them into the cache.
 #include "common.h"
+#include "attention_model.h"
 #include "gemm_tile.h"
 
 #include <math.h>
@@ -849,25 +850,6 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnParams p) {
             if (d4 == 0) *reinterpret_cast<float2 *>(pr + D) = make_float2(M, l);
         }
     }
-}
-
-// Key ranges per head of attention_decode_kernel: the count with the smallest predicted time (microseconds): a block alone reads its keys at 53 GB/s (head_dim 64: 36), all blocks together
-// at 6.1 TB/s, and several ranges cost a second launch and their partials.
-inline int decode_splits(int64_t heads, int64_t keys, int D, int cus) {
-    double best = 1e30;
-    int pick = 1;
-    const int per_cu = D == 128 ? 2 : 5;
-    const double alone = D == 128 ? 53.0e3 : 36.0e3, all = static_cast<double>(heads) * keys * D * 4.0 / 6.1e6;
-    for (int n = 1; n <= 32; ++n) {
-        const int64_t kps = ((keys + n - 1) / n + AT_KEYS - 1) / AT_KEYS * AT_KEYS;
-        if (n > 1 && (keys + kps - 1) / kps != n) continue;
-        const double turns = static_cast<double>((heads * n + per_cu * cus - 1) / (per_cu * cus));
-        const double own = turns * static_cast<double>(kps < keys ? kps : keys) * D * 4.0 / alone;
-        const double a2 = own * own, b2 = all * all;
-        const double t = sqrt(sqrt(a2 * a2 + b2 * b2)) + (n > 1 ? 2.3 + 0.25 * n : 0.0);
-        if (t < best) { best = t; pick = n; }
-    }
-    return pick;
 }
 
 template <int DT, int D>

@@ -43,6 +43,16 @@ def test_rows_against_the_oracle(keys, G, Hkv, D, splits, monkeypatch):
         _native.reload_tuning()
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_a_head_alone_on_many_keys(D):
+    """More than 32 ranges, which the merge takes as it takes fewer."""
+    q, k, v = (draw(1, 1, n, D, dtype=torch.float16, seed=s) for n, s in ((1, 1), (40003, 2), (40003, 3)))
+    got = _native.attention(q.to(DEV), k.to(DEV), v.to(DEV), scale=0.3, causal=True)
+    want = torch.from_numpy(oat.attention_f64(q.float().numpy(), k.float().numpy(), v.float().numpy(), 0.3, True))
+    # the result is rounded once (2^-11 of a value); probabilities carry 2^-21 and fp32 sums 2^-24 a step, below 2^-12 deviations of the 40003 weighed values
+    torch.testing.assert_close(got.double().cpu(), want, rtol=2.0 ** -10, atol=2.0 ** -9 * want.std().item())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("keys,at", [(64, 0), (64, 63), (65, 64), (75, 74), (79, 33), (1000, 999)])
