@@ -33,6 +33,8 @@ __global__ __launch_bounds__(ST_NW * 64) void stream_kernel(SkinnyParams p) {
     static_assert(NR % RP == 0 && XR % RP == 0 && UP % RP == 0, "whole loads");
     static_assert(ST_NW * RING <= ST_LDS_KB * 1024 && D >= 2 && (D - 1) * L < 64, "LDS, and the count in s_waitcnt");
     static_assert(NT * MT * 1024 <= RING, "the partial sums take the place of the stages");
+    constexpr int XLAST = XR - (MT - 1) * 16;  // staged rows of the last 16 of x: the lanes of the others read these again
+    static_assert(NT * 16 * PITCH <= STAGE && NB * 1024 + ((MT - 1) * 16 + XLAST) * PITCH <= STAGE && (XLAST & (XLAST - 1)) == 0, "fragments are read inside their stage");
     extern __shared__ __align__(16) char smem[];
     if constexpr (!SUM) take_rank(p);
 
@@ -85,6 +87,7 @@ __global__ __launch_bounds__(ST_NW * 64) void stream_kernel(SkinnyParams p) {
 
     unrolled<D>([&](auto sc) { load(decltype(sc)::value * STAGE, decltype(sc)::value); });
     const uint32_t rd = lds_addr_of(ring) + l16 * PITCH;
+    const uint32_t rd_last = lds_addr_of(ring) + (l16 & (XLAST - 1)) * PITCH;
     uint32_t kk_off[KK];
 #pragma unroll
     for (int k = 0; k < KK; ++k) kk_off[k] = static_cast<uint32_t>(((k * 4 + lq) ^ (l16 >> 1)) * 16);
@@ -94,9 +97,9 @@ __global__ __launch_bounds__(ST_NW * 64) void stream_kernel(SkinnyParams p) {
         u32x4 wq[KK][NT], xq[KK][MT];
         unrolled<KK>([&](auto hc) {
             constexpr int h = decltype(hc)::value;
-            const uint32_t at = rd + stage_off + kk_off[h];
+            const uint32_t at = rd + stage_off + kk_off[h], at_last = rd_last + stage_off + kk_off[h];
             unrolled<NT>([&](auto bc) { wq[h][decltype(bc)::value] = lds_read16<decltype(bc)::value * 16 * PITCH>(at); });
-            unrolled<MT>([&](auto ac) { xq[h][decltype(ac)::value] = lds_read16<NB * 1024 + decltype(ac)::value * 16 * PITCH>(at); });
+            unrolled<MT>([&](auto ac) { xq[h][decltype(ac)::value] = lds_read16<NB * 1024 + decltype(ac)::value * 16 * PITCH>(decltype(ac)::value == MT - 1 ? at_last : at); });
         });
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         unrolled<KK>([&](auto hc) {

@@ -28,6 +28,8 @@ __global__ __launch_bounds__(SW_NW * 64) void stream_w8_kernel(SkinnyParams p) {
     static_assert(NR % 8 == 0 && XR % 4 == 0, "whole loads");
     static_assert(SW_NW * RING <= SW_LDS_KB * 1024 && D >= 2 && (D - 1) * L < 64, "LDS, and the count in s_waitcnt");
     static_assert(NT * MT * 1024 <= RING, "the partial sums take the place of the stages");
+    constexpr int XLAST = XR - (MT - 1) * 16;  // as in stream_kernel
+    static_assert(NT * 16 * WP <= STAGE && NB * 1024 + ((MT - 1) * 16 + XLAST) * XP <= STAGE && (XLAST & (XLAST - 1)) == 0, "fragments are read inside their stage");
     extern __shared__ __align__(16) char smem[];
     if constexpr (!SUM) take_rank(p);
 
@@ -123,6 +125,7 @@ __global__ __launch_bounds__(SW_NW * 64) void stream_w8_kernel(SkinnyParams p) {
     if (og < groups) outlier_x();
     // 16 weights of a lane, elements 64 v + 16 lq ... + 16 of a unit, meet two pieces of a row of x
     const uint32_t rd_w = lds_addr_of(ring) + l16 * WP, rd_x = lds_addr_of(ring) + NB * 1024 + l16 * XP;
+    const uint32_t rd_last = lds_addr_of(ring) + NB * 1024 + (l16 & (XLAST - 1)) * XP;
     uint32_t w_at[2], x_at[4];
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
@@ -140,7 +143,7 @@ __global__ __launch_bounds__(SW_NW * 64) void stream_w8_kernel(SkinnyParams p) {
         });
         unrolled<4>([&](auto oc) {
             constexpr int o = decltype(oc)::value;
-            unrolled<MT>([&](auto ac) { xq[o][decltype(ac)::value] = lds_read16<decltype(ac)::value * 16 * XP>(rd_x + stage_off + x_at[o]); });
+            unrolled<MT>([&](auto ac) { xq[o][decltype(ac)::value] = lds_read16<decltype(ac)::value * 16 * XP>((decltype(ac)::value == MT - 1 ? rd_last : rd_x) + stage_off + x_at[o]); });
         });
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         unrolled<2>([&](auto vc) { unrolled<NT>([&](auto bc) { already_landed(wq[decltype(vc)::value][decltype(bc)::value]); }); });
