@@ -123,13 +123,9 @@ def add_lora_rules(model: nn.Module, config: Config) -> Config:
     return config
 
 
-def get_parameter_name_mapping(names: Iterable[str], tensor_parallel_config: Config) -> Mapping[str, str]:
-    """Original parameter name -> name inside the sharded model (config.py:157-191).
-
-    Every module that has an input or output rule gets wrapped, and the wrapper holds the module as
-    `tp_wrapped_module`; so "tp_wrapped_module." is inserted after each place where a module pattern
-    (trailing "$" dropped, "\\." appended unless it already ends with ".") matches the name."""
-    names = list(names)
+def wrapped_module_patterns(tensor_parallel_config: Config) -> list:
+    """Patterns that find, in a parameter's name, the ends of the modules that get wrapped: those of the modules with an input or output rule
+    (trailing "$" dropped, "\\." appended unless it already ends with ".")."""
     seen = set()
     for regex in chain(tensor_parallel_config.input_rules, tensor_parallel_config.output_rules):
         pattern = regex.pattern
@@ -138,13 +134,24 @@ def get_parameter_name_mapping(names: Iterable[str], tensor_parallel_config: Con
         if not pattern.endswith("."):
             pattern += r"\."
         seen.add(pattern)
-    compiled = [re.compile(p) for p in seen]
+    return [re.compile(p) for p in seen]
 
+
+def wrapped_names(names: Iterable[str], patterns: Sequence[re.Pattern]) -> Mapping[str, str]:
+    """`get_parameter_name_mapping` with the patterns at hand."""
     mapping = {}
     for name in names:
-        cuts = sorted(m.end() for m in (p.search(name) for p in compiled) if m is not None)
+        cuts = sorted(m.end() for m in (p.search(name) for p in patterns) if m is not None)
         new_name = name
         for pos in reversed(cuts):
             new_name = new_name[:pos] + "tp_wrapped_module." + new_name[pos:]
         mapping[name] = new_name
     return mapping
+
+
+def get_parameter_name_mapping(names: Iterable[str], tensor_parallel_config: Config) -> Mapping[str, str]:
+    """Original parameter name -> name inside the sharded model (config.py:157-191).
+
+    Every module that has an input or output rule gets wrapped, and the wrapper holds the module as
+    `tp_wrapped_module`; so "tp_wrapped_module." is inserted after each place where a module's pattern matches the name."""
+    return wrapped_names(names, wrapped_module_patterns(tensor_parallel_config))

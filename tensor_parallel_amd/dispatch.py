@@ -6,7 +6,7 @@ from typing import Dict, Optional
 
 import torch
 
-from .config import Config, get_parameter_name_mapping
+from .config import Config, wrapped_module_patterns, wrapped_names
 from .slicing import BatchSlicer
 from .state_actions import SegmentedAction, StateAction
 from .utils import find_tied_weight_aliases
@@ -58,33 +58,36 @@ def convert_state_dict(
     HIP device (`device`, or the device of the inputs, or the current one).
     Tied weights are not handled, as in the reference.
     """
+    patterns = wrapped_module_patterns(tensor_parallel_config)  # a name rule that does not serve is refused before anything is allocated
     batch = BatchSlicer(device, early=True)
     names = list(input_state_dict.keys())
     actions: Dict[str, Optional[StateAction]] = {}  # found in the first rank's turn: a name's rule is the same for every rank
     shards = []
-    for rank in range(world_size):
-        for name in names:
-            if rank == 0:
-                actions[name] = next((action for pattern, action in tensor_parallel_config.state_rules.items() if pattern.search(name) is not None), None)
-            action, state = actions[name], input_state_dict[name]
-            if action is None:
-                shards.append(state)
-            elif isinstance(action, SegmentedAction) and state is not None:
-                shards.append(batch.add(state, action.spec(tuple(state.shape), rank)))
-            else:
-                shards.append(action(state, rank=rank))
-    batch.run()
-    # the names of the output while the last copies run
-    renamed = get_parameter_name_mapping(names, tensor_parallel_config)
-    output: Dict[str, torch.Tensor] = {}
-    made = iter(shards)
-    for rank in range(world_size):
-        for name in names:
-            output[f"module_shards.{rank}.{renamed[name]}"] = next(made)
-        output[f"_sanity_check_params.{rank}"] = torch.empty(0, device="cpu")
-    if batch.device is not None and (batch.plan is not None or batch.launched):
-        torch.cuda.synchronize(batch.device)  # uploaded sources are dropped with the batch
-    batch.close()
+    try:
+        for rank in range(world_size):
+            for name in names:
+                if rank == 0:
+                    actions[name] = next((action for pattern, action in tensor_parallel_config.state_rules.items() if pattern.search(name) is not None), None)
+                action, state = actions[name], input_state_dict[name]
+                if action is None:
+                    shards.append(state)
+                elif isinstance(action, SegmentedAction) and state is not None:
+                    shards.append(batch.add(state, action.spec(tuple(state.shape), rank)))
+                else:
+                    shards.append(action(state, rank=rank))
+        batch.run()
+        # the names of the output while the last copies run
+        renamed = wrapped_names(names, patterns)
+        output: Dict[str, torch.Tensor] = {}
+        made = iter(shards)
+        for rank in range(world_size):
+            for name in names:
+                output[f"module_shards.{rank}.{renamed[name]}"] = next(made)
+            output[f"_sanity_check_params.{rank}"] = torch.empty(0, device="cpu")
+        if batch.device is not None and (batch.plan is not None or batch.launched):
+            torch.cuda.synchronize(batch.device)  # uploaded sources are dropped with the batch
+    finally:
+        batch.close()
     if for_pretrained:
         output = {"wrapped_model." + name: tensor for name, tensor in output.items()}
     return output

@@ -167,6 +167,34 @@ def test_convert_state_dict_names_and_shapes_golden(case):
     assert out[pre + "module_shards.0.model.norm.weight"] is state["model.norm.weight"]
 
 
+def test_convert_state_dict_refuses_a_bad_name_rule_before_it_allocates(monkeypatch):
+    """Module patterns become name patterns before the first tensor is sliced; and whatever fails later, the batch gives its sources back."""
+    from tensor_parallel_amd import dispatch
+
+    log = []
+
+    class Recorder(dispatch.BatchSlicer):
+        def add(self, *args, **kwargs):
+            log.append("add")
+            return super().add(*args, **kwargs)
+
+        def close(self):
+            log.append("close")
+            super().close()
+
+    monkeypatch.setattr(dispatch, "BatchSlicer", Recorder)
+    state = {"m.w": torch.empty(4, 6, device="meta"), "m.b": torch.empty(4, device="meta")}
+    cfg = tp.Config({r"w$": tp.Split(2, 0)}, {}, {}, {})
+    cfg.output_rules = {re.compile(rb"^m$"): {0: "sum"}}  # a pattern of bytes finds no name
+    with pytest.raises(TypeError):
+        tp.convert_state_dict(state, cfg, 2)
+    assert "add" not in log
+    cfg = tp.Config({r"w$": tp.Split(2, 0), r"b$": lambda tensor, rank: tensor[7]}, {}, {}, {})
+    with pytest.raises(IndexError):
+        tp.convert_state_dict(state, cfg, 2)
+    assert log == ["add", "close"]
+
+
 def test_llama_7b_and_falcon_40b_tables_give_the_baseline_shapes():
     llama = SimpleNamespace(model_type="llama", hidden_size=4096, num_attention_heads=32, num_key_value_heads=32)
     state = {
