@@ -1,5 +1,6 @@
 #include "skinny.h"
 #include "gemm_tile.h"
+#include "stream_model.h"
 
 namespace tpamd {
 namespace {
@@ -204,24 +205,6 @@ int launch_stream(const SkinnyParams &p, bool swiglu, int nr, int blocks, hipStr
 
 }  // namespace
 
-// How a launch of `ranks` matrices (sum: two ranks' K) would be cut: blocks of a rank and staged weight rows; false: not at all.
-static bool stream_cut(int64_t N, int ranks, bool swiglu, bool sum, int cus, int *blocks, int *rows, int *groups) {
-    const int64_t share = sum ? cus : cus / ranks, most = sum ? 48 : 96;
-    for (*groups = 1; *groups <= 4; ++*groups) {
-        int64_t b = *groups * share;
-        if (b > (N + 15) / 16) b = (N + 15) / 16;
-        const int64_t cols = (N + b - 1) / b;
-        int64_t nr = swiglu ? (cols + 7) / 8 * 16 : (cols + 7) / 8 * 8;
-        if (nr < (swiglu ? 32 : 16)) nr = swiglu ? 32 : 16;
-        if (nr > 24) nr = (nr + 15) / 16 * 16;
-        if (nr > most) continue;
-        *blocks = static_cast<int>(b);
-        *rows = static_cast<int>(nr);
-        return true;
-    }
-    return false;
-}
-
 // Whether the environment names another kernel for such a launch: a choice among those that took it before, by the switches that these read at its rows. (Not those that
 // choose a form of one of them: TPAMD_GEMM_W4, _STAGES, _PART_X.)
 static bool other_kernel_named(int64_t M, bool swiglu) {
@@ -232,43 +215,20 @@ static bool other_kernel_named(int64_t M, bool swiglu) {
     return M <= 3 && set(t.gemv_rows);
 }
 
-// Where stream_kernel is the faster one. Fitted on 500 shapes of both ranks, timed in a HIP graph on rotated weights against the kernels that took them before
-// (TPAMD_STREAM=0 and =1); by rows:
-//  - a sum of two ranks: 2 to 16 rows always (0.72-1.0 of the time; two rows of a narrow matrix stay with the row kernel), above while a CU reads x in less time than
-//    K ranges of tiles need for their planes and second launch (4096 x 2048 up to 42 rows, 4096 x 5504 up to 24, 8192 x 14336 up to 30; at 64 rows 1.07, 1.22, 1.28).
-//  - Linears of 3 to 16 rows: up to 12288 columns of both ranks (0.76-1.0), and where the other kernels are at their worst: K over 8192 (0.69-0.95), more than 8 rows
-//    on wide matrices of short rows (9216 x 2048 a rank 0.75). Others 1.03-1.1. Pairs: K over 8192 (0.84-0.98), more than 8 rows on short rows that are not whole KiB (0.86-0.95).
-//  - of 17 to 64 rows: one block per CU holds all columns (Linears 0.58-0.95 within the limit on x, pairs 0.63-1.0), or two take turns up to 32 rows (0.79-0.98); pairs in two
-//    turns 0.70-0.94; Linears in two turns at 34 to 64 rows 1.03-1.30 (16000 x 4096 of two ranks at 40 rows, fp16, 52.6 -> 57.7 us). Short rows of wide matrices are left out (11008 x 1408 at 47 rows 16.6 -> 20.0 us), and pairs whose staged rows would be a tenth padding (6912 x 5120 1.06-1.27).
+// Where stream_kernel takes a launch: whatever it can with TPAMD_STREAM=1, else where it is the faster one (stream_model.h).
 bool stream_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int ranks, bool swiglu, bool sum, int cus) {
-    int blocks = 0, rows = 0, groups = 0;
     if (tuning().stream == 0 || M < 2 || M > 64 || K % 64 != 0 || K < 64 || ldx >= (1ll << 22) || ldw >= (1ll << 22) || cus < ranks) return false;
-    if (!stream_cut(N, ranks, swiglu, sum, cus, &blocks, &rows, &groups)) return false;
-    if (tuning().stream == 1) return true;
-    if (other_kernel_named(M, swiglu)) return false;
-    const int64_t all = N * (sum ? 1 : ranks);
-    const int cols = static_cast<int>((N + blocks - 1) / blocks) * (swiglu ? 2 : 1);
-    const bool full = cols * 10 >= rows * 9;
-    const double mb = static_cast<double>(all) * K * (sum ? 2 : 1) * (swiglu ? 4.0e-6 : 2.0e-6);
-    const double x_us = static_cast<double>(M) * K * (sum ? 4.0 : 2.0) / 70.0e3;  // one CU reading x
-    if (K < 1024 || mb < 4.0) return false;
-    if (sum) return M == 2 ? N >= 4096 : M <= 16 || x_us < (full ? 3.5 : 3.0) + 0.045 * mb;
-    if (M < 3 || (swiglu && M < 4)) return false;
-    if (M <= 16) {
-        if (K > 8192 && all >= 4096) return true;
-        if (swiglu) return M > 8 && K < 3072 && K % 1024 != 0 && all >= 4096 && all <= 24576;
-        return all <= 12288 ? M <= 8 || K >= 2048 : M > 8 && K >= 1408 && K < 4096 && all >= 18432 && all <= 24576;
-    }
-    if (swiglu) return all >= 2048 && (groups == 1 || (full && (groups == 2 ? K >= 2048 : groups == 3 && M <= 32 && K >= 4096)));
-    return groups == 1 ? x_us < 3.0 + 0.04 * mb && (K >= 2048 || all <= 12288) : groups == 2 && M <= 32 && K >= 2048;
+    if (tuning().stream == 1) return stream_cut(N, ranks, swiglu, sum, cus).groups > 0;
+    return !other_kernel_named(M, swiglu) && stream_measured_faster(M, N, K, ranks, swiglu, sum, cus);
 }
 
 int stream_dispatch(const SkinnyParams &p, int dtype, bool swiglu, hipStream_t s) {
-    int dev = 0, cus = 256, blocks = 0, rows = 0, groups = 0;
+    int dev = 0, cus = 256;
     TPAMD_HIP(hipGetDevice(&dev));
     if (int rc = device_cus(dev, &cus); rc != TPAMD_OK) return rc;
-    TPAMD_REQUIRE(stream_cut(p.N, p.sum ? 1 : p.ranks, swiglu, p.sum, cus, &blocks, &rows, &groups), "stream: no cut of %d columns", p.N);
-    return dtype == TPAMD_BF16 ? launch_stream<TPAMD_BF16>(p, swiglu, rows, blocks, s) : launch_stream<TPAMD_F16>(p, swiglu, rows, blocks, s);
+    const StreamCut cut = stream_cut(p.N, p.sum ? 1 : p.ranks, swiglu, p.sum, cus);
+    TPAMD_REQUIRE(cut.groups > 0, "stream: no cut of %d columns", p.N);
+    return dtype == TPAMD_BF16 ? launch_stream<TPAMD_BF16>(p, swiglu, cut.rows, cut.blocks, s) : launch_stream<TPAMD_F16>(p, swiglu, cut.rows, cut.blocks, s);
 }
 
 }  // namespace tpamd

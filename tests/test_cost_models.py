@@ -1,4 +1,5 @@
-"""The cost models that choose between the GEMM kernels (csrc/gemm_model.h) and cut decode attention into key ranges (csrc/attention_model.h) are host code: compiled into a small program and asked here."""
+"""The cost models that choose between the GEMM kernels (csrc/gemm_model.h) cut decode attention into key ranges (csrc/attention_model.h) and choose stream_kernel
+(csrc/stream_model.h) are host code: compiled into a small program and asked here."""
 import shutil
 import subprocess
 from pathlib import Path
@@ -63,3 +64,16 @@ def test_key_ranges_of_a_decode_step_are_counts_that_measured_fast(tmp_path):
     rows = ask(tmp_path, "".join(f'printf("%d\\n", decode_splits({heads}, {keys}, {D}, 256));\n' for heads, keys, D, _, _ in cases), "attention_model.h")
     for case, (count,) in zip(cases, rows):
         assert case[3] <= count <= case[4], (case, count)
+
+
+def test_stream_kernel_is_left_to_the_launches_that_it_measured_faster_on(tmp_path):
+    """Ranks in the launch (sum: 0), gated pair, rows, columns, K, and whether stream_kernel takes it: differences of 7 % or more on 256 CUs, either way."""
+    cases = [(2, 1, 64, 6144, 1408, 0), (1, 1, 40, 2048, 14336, 0), (1, 1, 28, 2048, 2944, 0), (1, 1, 24, 2048, 1408, 1), (2, 1, 40, 8192, 5120, 0), (2, 1, 36, 8192, 8192, 1),
+             (1, 1, 36, 11008, 1024, 0), (2, 1, 24, 5504, 4096, 1), (1, 1, 40, 5504, 4096, 1), (2, 1, 28, 1024, 4416, 0), (1, 1, 36, 2048, 2048, 1),
+             (1, 0, 3, 452, 8192, 0), (1, 0, 3, 1024, 4096, 0), (1, 0, 3, 11008, 2048, 0), (1, 0, 3, 5200, 1024, 1), (2, 0, 8, 4096, 1024, 0), (1, 0, 12, 2048, 8128, 0),
+             (1, 0, 12, 4608, 14336, 1), (1, 0, 16, 4096, 2048, 1), (1, 0, 28, 3072, 5120, 0), (1, 0, 28, 5120, 2752, 1), (2, 0, 32, 16000, 2688, 0), (2, 0, 28, 16000, 4096, 1),
+             (2, 0, 24, 6144, 4096, 1), (2, 0, 36, 2048, 1984, 1), (2, 0, 56, 1024, 2048, 0),
+             (0, 0, 64, 16000, 1408, 0), (0, 0, 36, 16000, 4096, 1), (0, 0, 8, 4096, 5504, 1), (0, 0, 24, 4096, 2048, 1), (0, 0, 64, 4096, 5504, 0)]
+    rows = ask(tmp_path, "".join(f'printf("%d\\n", stream_measured_faster({m}, {n}, {k}, {ranks or 2}, {"true" if pair else "false"}, {"false" if ranks else "true"}, 256) ? 1 : 0);\n'
+                                 for ranks, pair, m, n, k, _ in cases), "stream_model.h")
+    assert [(c[:5], r[0]) for c, r in zip(cases, rows)] == [(c[:5], c[5]) for c in cases]
