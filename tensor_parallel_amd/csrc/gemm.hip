@@ -1985,47 +1985,6 @@ int configure128(int dev) {
     return TPAMD_OK;
 }
 
-// Predicted time (microseconds) of the 128 x 128 tiling, with the K split and the number of LDS stages that give it,
-// from a small cost model fitted on this part (least squares over 290 timings of 48 mid-sized shapes, then two sweeps of
-// 100 shapes at 64-2048 rows with every split count and both stage counts, 1500 timings).
-//  - two stages (two blocks fit a CU): a block that has its CU to itself takes 0.82 per K tile, two blocks sharing a CU
-//    0.98 each (the pace of the CU's global->LDS path), 0.92 when blocks queue for several rounds of two per CU;
-//  - four stages (one block per CU, three K tiles of look-ahead), in rounds of one block per CU: split launches 0.55 per
-//    K tile; unsplit ones 0.60 when there is one row tile (every block streams weights nobody shares, about 27 GB/s
-//    per CU), 0.42 with at most half the CUs busy and 0.55 otherwise for a single matrix, 0.62 (two row tiles) / 0.44 and
-//    0.64 for the gated pair;
-//  - no launch streams its weights (tiles_n column tiles of 16 KiB per K tile) faster than 5 TB/s;
-//  - the partial tiles cost 4.6 + 0.39 per MB (written, read back and finished by a second launch; valid_rows = the
-//    fraction of the tiles' rows that lie inside M: the others are not stored).
-// Over the second sweep the choices are within 1.8 % of the best (split, stages) per shape; with two stages only they
-// were 4.7 % off the best split (a single matrix 4096 x 4096 at 1024 rows: 51.5 us unsplit on two stages, 33.7 us on four).
-inline double estimate128(int64_t tiles, int64_t tiles_m, int64_t tiles_n, int KT, int cus, double valid_rows, bool swiglu, int *splits,
-                          bool *deep) {
-    double best = 1e30;
-    *splits = 1;
-    *deep = false;
-    const double stream = static_cast<double>(tiles_n) * KT * 16384.0 / 5.0e6;
-    for (int sp = 1; sp <= 8; ++sp) {
-        const int kt = (KT + sp - 1) / sp;
-        if (sp > 1 && (kt < 4 || tiles * sp > 4ll * cus)) break;  // too little K per split / more than the scratch buffer holds
-        const int64_t units = tiles * sp;
-        const double finish = sp > 1 ? 4.6 + units * 0.065536 * valid_rows * 0.39 : 0.0;
-        const double per_deep = sp > 1 ? 0.55
-                                : tiles_m == 1 ? 0.60
-                                : units * 2 <= cus ? (swiglu ? (tiles_m == 2 ? 0.62 : 0.44) : 0.42)
-                                : (swiglu ? 0.64 : 0.55);
-        const double loop_deep = static_cast<double>((units + cus - 1) / cus) * kt * per_deep;
-        const double t_deep = (loop_deep > stream ? loop_deep : stream) + finish;
-        if ((sp == 1 || units <= cus) && t_deep < best) { best = t_deep; *splits = sp; *deep = true; }  // split launches: one round only (measured)
-        const double rounds = units <= cus ? 1.0 : static_cast<double>((units + 2 * cus - 1) / (2 * cus));
-        const double per_kt = units <= cus ? 0.82 : units <= 2ll * cus ? 0.98 : 0.92;
-        const double loop = rounds * kt * per_kt;
-        const double t = (loop > stream ? loop : stream) + finish;
-        if (t < best) { best = t; *splits = sp; *deep = false; }
-    }
-    return best;
-}
-
 template <int DT, int MODE, int NS, int XQ>
 int launch_split128(const GemmParams &p, dim3 grid, int dev, hipStream_t s) {
     if (int rc = configure128<DT, MODE, NS, true, XQ>(dev); rc != TPAMD_OK) return rc;
@@ -2096,26 +2055,7 @@ int launch_direct128(GemmParams p, int cus, hipStream_t s) {
     return TPAMD_OK;
 }
 
-// Two ranks' Linears and their sum in one launch and a finishing pass: 128 x 128 tiles, every rank's K in `splits` ranges. Predicted time (microseconds) of the
-// best split, by the terms of estimate128.
-inline double estimate_sum128(int64_t tiles, int64_t tiles_n, int KT, int cus, double valid_rows, int *splits, bool *deep) {
-    double best = 1e30;
-    const double stream = 2.0 * tiles_n * KT * 16384.0 / 5.0e6;
-    for (int sp = 1; sp <= 4; ++sp) {
-        const int kt = (KT + sp - 1) / sp;
-        const int64_t units = tiles * 2 * sp;
-        if ((sp > 1 && kt < 4) || units > 4ll * cus) break;
-        const double finish = 4.6 + units * 0.065536 * valid_rows * 0.39;
-        const double loop_deep = kt * 0.55, rounds = units <= cus ? 1.0 : static_cast<double>((units + 2 * cus - 1) / (2 * cus));
-        const double t_deep = (loop_deep > stream ? loop_deep : stream) + finish;
-        if (units <= cus && t_deep < best) { best = t_deep; *splits = sp; *deep = true; }
-        const double loop = rounds * kt * (units <= cus ? 0.82 : units <= 2ll * cus ? 0.98 : 0.92);
-        const double t = (loop > stream ? loop : stream) + finish;
-        if (t < best) { best = t; *splits = sp; *deep = false; }
-    }
-    return best;
-}
-
+// Two ranks' Linears and their sum in one launch and a finishing pass: 128 x 128 tiles, every rank's K in `splits` ranges (estimate_sum128, gemm_model.h).
 template <int DT>
 int launch_sum128(GemmParams p, bool deep, hipStream_t s, bool *done) {
     int dev = 0, cus = 256;
@@ -2153,48 +2093,14 @@ int gemm_large(GemmParams p, bool swiglu, hipStream_t s) {
     if (int rc_cus = device_cus(dev, &cus); rc_cus != TPAMD_OK) return rc_cus;
     // the direct kernels address a tile with 32-bit byte offsets from the tile origin and step K in tiles of 64
     const bool direct_ok = p.K % 64 == 0 && p.K >= 64 && p.ldx < (1ll << 22) && p.ldw < (1ll << 22);
-    // 256 x 256 tiles or 128 x 128 tiles (with K split): whichever the cost models predict to be faster. The 256 tiles
-    // run in rounds of one per CU; over 104 launches of more than half a round (the shapes of MID_TILES) a launch takes 4.8 us, a round 5.9, a K tile 1.37 in a full round
-    // (the part is power-limited then), 1.25 in a round that fills at most three quarters of the CUs and 1.42 in between.
-    const int64_t big_tiles = static_cast<int64_t>((p.M + 255) / 256) * ((p.N + (swiglu ? 127 : 255)) / (swiglu ? 128 : 256));
-    const int64_t small_tiles = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + (swiglu ? 63 : 127)) / (swiglu ? 64 : 128)) * p.ranks;
-    const int KT = static_cast<int>(p.K / 64);
-    auto rounds256 = [&](int64_t units, int kt) {
-        const int64_t full = units / cus, last = units % cus;
-        return 4.8 + 5.9 * (full + (last > 0)) + kt * (full * 1.37 + (last == 0 ? 0.0 : last * 4 <= 3ll * cus ? 1.25 : 1.42));
-    };
-    const double stream = stream_floor(p.N, p.K, swiglu);  // the pair 8192 x 8192 at 17 rows took 79.8 us on this tiling in four splits, predicted
-                                                           // 57 without this term, and 63.8 us on the other
-    auto floor256 = [&](double loop) { return loop > stream ? loop : stream; };
-    double t256 = floor256(rounds256(big_tiles, KT));
-    // ... or split over K while all units still fit one round; the partial tiles cost 3 us + 0.33 us per MB (more than
-    // with the small tiles: all blocks finish together, so nothing overlaps the writes and the finishing pass)
-    int splits256 = 1;
-    const double valid256 = static_cast<double>(p.M) / (((p.M + 255) / 256) * 256.0);
-    for (int sp = 2; sp <= 8 && big_tiles * sp <= cus; ++sp) {
-        const int kt = (KT + sp - 1) / sp;
-        if (kt < 4) break;
-        const int64_t units = big_tiles * sp;
-        const double t = floor256(rounds256(units, kt)) + 3.0 + units * 0.262144 * valid256 * 0.33;
-        if (t < t256) { t256 = t; splits256 = sp; }
-    }
-    if (tuning().gemm_splitk256 != TUNE_UNSET) splits256 = tuning().gemm_splitk256;
-    t256 *= p.ranks;  // this tiling takes two ranks in two launches: whole rounds of large tiles gain nothing from one
-    int unused_splits = 1;
-    bool unused_deep = false;
-    const int64_t small_tiles_m = (p.M + 127) / 128;
-    const double t128 = beside_mid(estimate128(small_tiles, small_tiles_m, small_tiles / small_tiles_m, KT, cus,
-                                               static_cast<double>(p.M) / (small_tiles_m * 128.0), swiglu, &unused_splits, &unused_deep), p.M);
+    const TileChoice choice = choose_tile(p.M, p.N, static_cast<int>(p.K / 64), cus, swiglu, p.ranks);
+    const int forced = tuning().gemm_tile;
     if (direct_ok) {
-        int tmx = 0, tnx = 0;
-        if (tuning().gemm_tile != TUNE_UNSET) {
-            if (tuning().gemm_tile > 1000) { tmx = tuning().gemm_tile / 32000; tnx = tuning().gemm_tile % 1000 / 32; }
-        } else if (estimate_mid(p.M, p.N, KT, cus, swiglu, &tmx, &tnx, p.ranks) >= (t256 < t128 ? t256 : t128)) {
-            tmx = 0;
-        }
+        const int tmx = forced != TUNE_UNSET ? (forced > 1000 ? forced / 32000 : 0) : choice.tmx, tnx = forced != TUNE_UNSET ? forced % 1000 / 32 : choice.tnx;
         if (tmx > 0) return gemm_mid(p, DT, swiglu, tmx, tnx, s);
     }
-    const bool big = tuning().gemm_tile != TUNE_UNSET ? tuning().gemm_tile == 256 : t256 < t128;
+    const bool big = forced != TUNE_UNSET ? forced == 256 : choice.big;
+    const int splits256 = tuning().gemm_splitk256 != TUNE_UNSET ? tuning().gemm_splitk256 : choice.splits256;
     if (p.ranks == 2 && (big || !direct_ok)) {
         p.ranks = 1;
         if (int rc = gemm_large<DT>(p, swiglu, s); rc != TPAMD_OK) return rc;
@@ -2263,20 +2169,10 @@ int gemm_dispatch(const void *x, const void *w, const void *w2, const void *bias
     return dtype == TPAMD_BF16 ? gemm_large<TPAMD_BF16>(p, swiglu, s) : gemm_large<TPAMD_F16>(p, swiglu, s);
 }
 
-// Whether launch_sum128 is predicted to take less time than two launches, the second of which adds the first one's result (M above the weight-streaming kernels'
-// range). The models are those of estimate128 and estimate_mid; 512 rows of 4096 x 5504: 33.1 + 5.4 us twice, 59.0 + 5.6 in one; 645 rows, whose
-// unsplit tiles of one rank fill the device, stay in two launches.
+// Whether launch_sum128 is predicted to take less time than two launches (M above the weight-streaming kernels' range).
 bool sum128_pays(int64_t M, int64_t N, int64_t K, int cus) {
     if (K % 64 != 0 || tuning().gemm_tile != TUNE_UNSET || tuning().gemm_splitk != TUNE_UNSET) return false;
-    const int KT = static_cast<int>(K / 64);
-    const int64_t tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128, tiles = tiles_m * tiles_n;
-    const double valid = static_cast<double>(M) / (tiles_m * 128.0);
-    bool deep = false;
-    int tmx = 0, tnx = 0, splits = 0;
-    const double once = beside_mid(estimate_sum128(tiles, tiles_n, KT, cus, valid, &splits, &deep), M);
-    const double t128 = beside_mid(estimate128(tiles, tiles_m, tiles_n, KT, cus, valid, false, &splits, &deep), M);
-    const double mid = estimate_mid(M, N, KT, cus, false, &tmx, &tnx);
-    return once < 1.9 * (t128 < mid ? t128 : mid);  // where the models are equal one launch was 2-3 % slower (4544 x 7168 at 513 rows, 5120 x 8192 at 468)
+    return sum_predicted_faster(M, N, static_cast<int>(K / 64), cus);
 }
 
 // y = the sum of two ranks' 16-bit Linears of one shape, the second one's operands `to` away, stored a second time `copy` bytes on. *done = false, with nothing

@@ -8,25 +8,24 @@ namespace tpamd {
 inline double stream_floor(int64_t N, int64_t K, bool swiglu) { return static_cast<double>(N) * K * (swiglu ? 4.0 : 2.0) / 5.0e6; }
 
 // Predicted time (microseconds) of gemm_mid_kernel on the best of its tiles, and that tile: a launch, rounds of one block per CU, each with
-// a fixed cost (first tiles, epilogue) and a time per K tile, shorter where the last round leaves CUs idle (the part clocks higher).
-// Non-negative least squares on relative errors over 220 shapes (128-8192 rows, 1000-16000 columns, K 1024-8192, one and two ranks), each tile forced and timed
-// inside a HIP graph. Over those the choice among these tiles, the 256 x 256 and the 128 x 128 tiling is 0.9 % off the best one (geometric mean); with four
-// of these tiles and models of the other two tilings without a cost per launch and round it was 6.8 % off. Examples (us, before -> now): the pair 5504 x 4096 of two ranks at 512
-// rows 103 -> 87 (256 x 192), at 1024 rows 177 -> 169, 16000 x 4096 of two ranks at 645 rows 188 -> 147 (224 x 192), 3072 x 4096 at 2103 rows 115 -> 91 (224 x 256: 240 tiles
+// a fixed cost (first tiles, epilogue) and a time per K tile, shorter where the last round leaves CUs idle (the part clocks higher); 3 % more for two ranks, whose
+// tiles share less in the caches.
+// Non-negative least squares on relative errors over 985 shapes (65-8192 rows, 600-28000 columns, K 1024-14336, single matrices and pairs, one and two ranks), each tile forced and timed
+// inside a HIP graph, those of up to 128 rows left out of the fit. Over all of them the choice among these tiles, the 256 x 256 and the 128 x 128 tiling (choose_tile) is 0.8 % off the best
+// one (geometric mean; 45 by more than 5 %, at worst 27 %); with four of these tiles and models without a cost per launch and round it was 4.6 % off. Examples (us, then -> now): the pair 5504 x 4096 of two
+// ranks at 512 rows 103 -> 87 (256 x 192), 16000 x 4096 of two ranks at 645 rows 188 -> 147 (224 x 192), 3072 x 4096 at 2103 rows 115 -> 91 (224 x 256: 240 tiles
 // on 256 CUs), 6144 x 4096 at 4096 rows 183 -> 166 (512 tiles of 256 x 192 instead of 384 of 256 x 256), 2048 x 5120 x 1024 64 -> 54.
 struct MidTile { int tmx, tnx; double launch, round, full, idle[3]; };  // idle: last round at most 1/2, at most 3/4, more of the CUs
 constexpr MidTile MID_TILES[2][10] = {
-    {{4, 6, 2.8, 4.7, 0.659, {0.603, 0.631, 0.662}}, {4, 8, 2.8, 5.1, 0.822, {0.737, 0.785, 0.839}}, {5, 6, 2.2, 5.5, 0.758, {0.643, 0.680, 0.774}},
-     {5, 8, 3.0, 5.0, 0.989, {0.788, 0.893, 0.954}}, {6, 6, 3.4, 5.9, 0.871, {0.682, 0.745, 0.836}}, {6, 8, 2.3, 5.0, 1.154, {1.126, 1.208, 1.209}},
-     {7, 6, 4.0, 6.4, 0.991, {0.755, 0.825, 0.957}}, {7, 8, 1.6, 6.7, 1.266, {1.171, 1.236, 1.287}}, {8, 6, 3.1, 6.2, 1.159, {1.058, 1.086, 1.135}},
-     {8, 8, 2.2, 7.0, 1.381, {1.223, 1.256, 1.356}}},
-    {{4, 6, 2.9, 3.7, 0.682, {0.616, 0.631, 0.738}}, {4, 8, 3.0, 4.9, 0.846, {0.734, 0.764, 0.817}}, {5, 6, 3.1, 4.5, 0.778, {0.644, 0.697, 0.751}},
-     {5, 8, 2.5, 5.9, 0.971, {0.790, 0.871, 0.918}}, {6, 6, 2.3, 6.1, 0.866, {0.714, 0.754, 0.857}}, {6, 8, 2.9, 5.3, 1.186, {1.137, 1.199, 1.219}},
-     {7, 6, 3.3, 6.3, 0.995, {0.766, 0.818, 0.907}}, {7, 8, 3.2, 5.9, 1.304, {1.160, 1.262, 1.305}}, {8, 6, 2.5, 6.9, 1.155, {1.067, 1.091, 1.191}},
-     {8, 8, 3.8, 7.0, 1.411, {1.200, 1.282, 1.444}}},
+    {{4, 6, 0.9, 5.1, 0.670, {0.558, 0.648, 0.666}}, {4, 8, 0.9, 5.5, 0.854, {0.700, 0.779, 0.869}}, {5, 6, 1.2, 6.1, 0.765, {0.628, 0.687, 0.754}},
+     {5, 8, 1.6, 5.9, 0.999, {0.781, 0.873, 0.958}}, {6, 6, 1.6, 7.0, 0.872, {0.682, 0.750, 0.839}}, {6, 8, 0.0, 5.2, 1.225, {1.041, 1.178, 1.267}},
+     {7, 6, 1.8, 7.6, 0.986, {0.760, 0.858, 0.961}}, {7, 8, 0.0, 6.6, 1.322, {1.106, 1.253, 1.311}}, {8, 6, 0.0, 7.2, 1.157, {0.987, 1.093, 1.184}},
+     {8, 8, 0.5, 7.4, 1.442, {1.161, 1.303, 1.379}}},
+    {{4, 6, 2.1, 3.8, 0.703, {0.568, 0.639, 0.687}}, {4, 8, 1.1, 4.9, 0.872, {0.720, 0.815, 0.877}}, {5, 6, 2.0, 5.2, 0.776, {0.631, 0.710, 0.759}},
+     {5, 8, 2.2, 5.3, 1.013, {0.798, 0.884, 1.005}}, {6, 6, 2.6, 5.8, 0.890, {0.692, 0.758, 0.845}}, {6, 8, 0.3, 5.0, 1.247, {1.084, 1.253, 1.300}},
+     {7, 6, 2.6, 6.4, 1.000, {0.767, 0.854, 0.958}}, {7, 8, 0.0, 6.6, 1.316, {1.136, 1.320, 1.400}}, {8, 6, 1.5, 6.1, 1.185, {1.000, 1.110, 1.171}},
+     {8, 8, 0.8, 7.5, 1.436, {1.189, 1.359, 1.402}}},
 };
-// The prediction for the 128 x 128 tiling beside these, above 128 rows: what a fit over the same 220 shapes makes of estimate128 (gemm.hip), whose own fit has no cost per launch.
-inline double beside_mid(double estimate128_us, int64_t M) { return M > 128 ? 2.5 + 1.1 * estimate128_us : estimate128_us; }
 
 // Up to 128 rows, where nothing was fitted, at least what streaming the weights takes. Without that floor few rows of a wide matrix were
 // predicted faster than HBM and taken off the 128 x 128 tiling, where a tie leaves them (us there / on these tiles): 28672 x 4096 at
@@ -40,10 +39,137 @@ inline double estimate_mid(int64_t M, int64_t N, int KT, int cus, bool swiglu, i
         const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * ranks, full = tiles / cus, last = tiles % cus;
         double us = t.launch + full * (t.round + KT * t.full);
         if (last > 0) us += t.round + KT * t.idle[last * 2 <= cus ? 0 : last * 4 <= 3ll * cus ? 1 : 2];
+        if (ranks == 2) us *= 1.03;
         if (us < best) { best = us; *tmx = t.tmx; *tnx = t.tnx; }
     }
     const double stream = stream_floor(N * ranks, 64ll * KT, swiglu);
     return M <= 128 && best < stream ? stream : best;
+}
+
+// Predicted time (microseconds) of the 128 x 128 tiling, with the K split and the number of LDS stages that give it,
+// from a small cost model fitted on this part (least squares over 290 timings of 48 mid-sized shapes, then two sweeps of
+// 100 shapes at 64-2048 rows with every split count and both stage counts, 1500 timings).
+//  - two stages (two blocks fit a CU): a block that has its CU to itself takes 0.82 per K tile, two blocks sharing a CU
+//    0.98 each (the pace of the CU's global->LDS path), 0.92 when blocks queue for several rounds of two per CU;
+//  - four stages (one block per CU, three K tiles of look-ahead), in rounds of one block per CU: split launches 0.55 per
+//    K tile; unsplit ones 0.60 when there is one row tile (every block streams weights nobody shares, about 27 GB/s
+//    per CU), 0.42 with at most half the CUs busy and 0.55 otherwise for a single matrix, 0.62 (two row tiles) / 0.44 and
+//    0.64 for the gated pair;
+//  - no launch streams its weights (tiles_n column tiles of 16 KiB per K tile) faster than 5 TB/s;
+//  - the partial tiles cost 4.6 + 0.39 per MB (written, read back and finished by a second launch; valid_rows = the
+//    fraction of the tiles' rows that lie inside M: the others are not stored).
+// Over the second sweep the choices are within 1.8 % of the best (split, stages) per shape; with two stages only they
+// were 4.7 % off the best split (a single matrix 4096 x 4096 at 1024 rows: 51.5 us unsplit on two stages, 33.7 us on four).
+inline double estimate128(int64_t tiles, int64_t tiles_m, int64_t tiles_n, int KT, int cus, double valid_rows, bool swiglu, int *splits,
+                          bool *deep) {
+    double best = 1e30;
+    *splits = 1;
+    *deep = false;
+    const double stream = static_cast<double>(tiles_n) * KT * 16384.0 / 5.0e6;
+    for (int sp = 1; sp <= 8; ++sp) {
+        const int kt = (KT + sp - 1) / sp;
+        if (sp > 1 && (kt < 4 || tiles * sp > 4ll * cus)) break;  // too little K per split / more than the scratch buffer holds
+        const int64_t units = tiles * sp;
+        const double finish = sp > 1 ? 4.6 + units * 0.065536 * valid_rows * 0.39 : 0.0;
+        const double per_deep = sp > 1 ? 0.55
+                                : tiles_m == 1 ? 0.60
+                                : units * 2 <= cus ? (swiglu ? (tiles_m == 2 ? 0.62 : 0.44) : 0.42)
+                                : (swiglu ? 0.64 : 0.55);
+        const double loop_deep = static_cast<double>((units + cus - 1) / cus) * kt * per_deep;
+        const double t_deep = (loop_deep > stream ? loop_deep : stream) + finish;
+        if ((sp == 1 || units <= cus) && t_deep < best) { best = t_deep; *splits = sp; *deep = true; }  // split launches: one round only (measured)
+        const double rounds = units <= cus ? 1.0 : static_cast<double>((units + 2 * cus - 1) / (2 * cus));
+        const double per_kt = units <= cus ? 0.82 : units <= 2ll * cus ? 0.98 : 0.92;
+        const double loop = rounds * kt * per_kt;
+        const double t = (loop > stream ? loop : stream) + finish;
+        if (t < best) { best = t; *splits = sp; *deep = false; }
+    }
+    return best;
+}
+
+// Two ranks' Linears and their sum in one launch and a finishing pass: 128 x 128 tiles, every rank's K in `splits` ranges. Predicted time (microseconds) of the
+// best split, by the terms of estimate128.
+inline double estimate_sum128(int64_t tiles, int64_t tiles_n, int KT, int cus, double valid_rows, int *splits, bool *deep) {
+    double best = 1e30;
+    const double stream = 2.0 * tiles_n * KT * 16384.0 / 5.0e6;
+    for (int sp = 1; sp <= 4; ++sp) {
+        const int kt = (KT + sp - 1) / sp;
+        const int64_t units = tiles * 2 * sp;
+        if ((sp > 1 && kt < 4) || units > 4ll * cus) break;
+        const double finish = 4.6 + units * 0.065536 * valid_rows * 0.39;
+        const double loop_deep = kt * 0.55, rounds = units <= cus ? 1.0 : static_cast<double>((units + 2 * cus - 1) / (2 * cus));
+        const double t_deep = (loop_deep > stream ? loop_deep : stream) + finish;
+        if (units <= cus && t_deep < best) { best = t_deep; *splits = sp; *deep = true; }
+        const double loop = rounds * kt * (units <= cus ? 0.82 : units <= 2ll * cus ? 0.98 : 0.92);
+        const double t = (loop > stream ? loop : stream) + finish;
+        if (t < best) { best = t; *splits = sp; *deep = false; }
+    }
+    return best;
+}
+
+// Predicted time (microseconds) of a rank on the 256 x 256 tiling, and its K splits. The tiles run in rounds of one per CU; fitted on the same shapes (launches of more than half a round), a launch takes
+// 4.7, a round 6.3, a K tile 1.42 in a full round (the part is power-limited then), 1.26 in a round that fills at most three quarters of the CUs and 1.43 in between. Split over K while all
+// units fit one round: the partial tiles cost 4.5 us + 0.33 us per MB. (8192 x 8192 gated at 17 rows took 79.8 us here in four splits, predicted 57 without the floor, and 63.8 on 128 x 128.)
+inline double estimate256(int64_t M, int64_t N, int KT, int cus, bool swiglu, int *splits) {
+    const int64_t tiles = ((M + 255) / 256) * ((N + (swiglu ? 127 : 255)) / (swiglu ? 128 : 256));
+    const double floor = stream_floor(N, 64ll * KT, swiglu), valid = static_cast<double>(M) / (((M + 255) / 256) * 256.0);
+    double best = 1e30;
+    *splits = 1;
+    for (int sp = 1; sp <= 8; ++sp) {
+        const int kt = (KT + sp - 1) / sp;
+        const int64_t units = tiles * sp, full = units / cus, last = units % cus;
+        if (sp > 1 && (units > cus || kt < 4)) break;
+        const double loop = 4.7 + 6.3 * (full + (last > 0)) + kt * (full * 1.42 + (last == 0 ? 0.0 : last * 4 <= 3ll * cus ? 1.26 : 1.43));
+        const double us = (loop > floor ? loop : floor) + (sp > 1 ? 4.5 + units * 0.262144 * valid * 0.33 : 0.0);
+        if (us < best) { best = us; *splits = sp; }
+    }
+    return best;
+}
+
+// The prediction for the 128 x 128 tiling beside the others, above 128 rows: what the same shapes make of estimate128, whose own fit has no cost per launch. Launches of one round of blocks
+// with four stages are faster than the others by it, unsplit pairs that fill more than half of the CUs most of all (2200 x 5120 at 641 rows 39.8 us; 51 on 128 x 192, predicted 57).
+inline double beside_mid(double estimate128_us, int64_t M, int64_t units, int64_t tiles_m, bool deep, bool unsplit_pair, int cus) {
+    if (M <= 128) return estimate128_us;
+    const double per = !deep || units > cus ? 1.1 : tiles_m < 3 ? 1.05 : unsplit_pair && units * 2 > cus ? 0.8 : 0.95;
+    return 2.5 + per * estimate128_us;
+}
+inline double beside_mid128(int64_t M, int64_t N, int KT, int cus, bool swiglu, int ranks) {
+    const int64_t tiles_m = (M + 127) / 128, tiles_n = (N + (swiglu ? 63 : 127)) / (swiglu ? 64 : 128) * ranks;
+    int splits = 1;
+    bool deep = false;
+    const double us = estimate128(tiles_m * tiles_n, tiles_m, tiles_n, KT, cus, static_cast<double>(M) / (tiles_m * 128.0), swiglu, &splits, &deep);
+    return beside_mid(us, M, tiles_m * tiles_n * splits, tiles_m, deep, swiglu && splits == 1, cus);
+}
+
+// What takes a Linear or gated pair of `ranks` matrices above the weight-streaming kernels' rows: a tile of gemm_mid_kernel (tmx > 0), 256 x 256 tiles, which take two ranks in two launches
+// (whole rounds of large tiles gain nothing from one), or 128 x 128 tiles.
+struct TileChoice {
+    int tmx, tnx;
+    bool big;
+    int splits256;
+};
+inline TileChoice choose_tile(int64_t M, int64_t N, int KT, int cus, bool swiglu, int ranks) {
+    TileChoice c{0, 0, false, 1};
+    const double t256 = estimate256(M, N, KT, cus, swiglu, &c.splits256) * ranks, t128 = beside_mid128(M, N, KT, cus, swiglu, ranks);
+    c.big = t256 < t128;
+    if (estimate_mid(M, N, KT, cus, swiglu, &c.tmx, &c.tnx, ranks) >= (c.big ? t256 : t128)) c.tmx = 0;
+    return c;
+}
+
+// Whether two ranks' Linears and their sum on 128 x 128 tiles take less time than two launches, the second of which adds the first one's result. 512 rows of 4096 x 5504: 33.1 + 5.4 us twice, 59.0 +
+// 5.6 in one; 645 rows, whose unsplit tiles of one rank fill the device, stay in two launches. Where the models are equal one launch was 2-3 % slower (4544 x 7168 at 513 rows, 5120 x 8192 at 468).
+// Over 161 shapes of 65-1500 rows one launch takes 82, at 0.72 of the time of two (at worst 1.04); without the 256 x 256 tiling among the alternatives 8 more, at 1.004 (938 x 4096 x 14336 228 -> 272 us).
+inline bool sum_predicted_faster(int64_t M, int64_t N, int KT, int cus) {
+    const int64_t tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128, tiles = tiles_m * tiles_n;
+    int tmx = 0, tnx = 0, splits = 0;
+    bool deep = false;
+    const double us = estimate_sum128(tiles, tiles_n, KT, cus, static_cast<double>(M) / (tiles_m * 128.0), &splits, &deep);
+    const double once = beside_mid(us, M, tiles * 2 * splits, tiles_m, deep, false, cus);
+    double other = beside_mid128(M, N, KT, cus, false, 1);
+    const double mid = estimate_mid(M, N, KT, cus, false, &tmx, &tnx), big = estimate256(M, N, KT, cus, false, &splits);
+    if (mid < other) other = mid;
+    if (big < other) other = big;
+    return once < 1.9 * other;
 }
 
 // Rows, columns and K of an int8 Linear whose stream has no scratch memory (captured before its first use, or beyond the 32 buffers of a

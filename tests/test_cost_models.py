@@ -77,3 +77,21 @@ def test_stream_kernel_is_left_to_the_launches_that_it_measured_faster_on(tmp_pa
     rows = ask(tmp_path, "".join(f'printf("%d\\n", stream_measured_faster({m}, {n}, {k}, {ranks or 2}, {"true" if pair else "false"}, {"false" if ranks else "true"}, 256) ? 1 : 0);\n'
                                  for ranks, pair, m, n, k, _ in cases), "stream_model.h")
     assert [(c[:5], r[0]) for c, r in zip(cases, rows)] == [(c[:5], c[5]) for c in cases]
+
+
+def test_tiles_are_chosen_that_measured_fast(tmp_path):
+    """Ranks, gated pair, rows, columns, K, and what measured within 5 % of the best on 256 CUs (a gemm_mid_kernel tile as 1000 * rows + columns, 256 or 128): shapes on which the models were 10 to 28 % off,
+    and others of every kind."""
+    cases = [(1, 1, 641, 2200, 5120, {128}), (1, 1, 1507, 1120, 5376, {128}), (2, 1, 727, 1024, 5184, {128}), (1, 1, 222, 7800, 5504, {128}), (2, 1, 776, 1596, 5120, {128192}),
+             (2, 1, 5049, 3072, 11008, {256}), (2, 1, 3684, 4096, 8192, {256}), (1, 1, 384, 5120, 5120, {128}), (2, 0, 5429, 5504, 8192, {256}),
+             (2, 1, 512, 5504, 4096, {256192}), (2, 0, 645, 16000, 4096, {224192}), (1, 0, 2103, 4096, 5504, {192192})]
+    rows = ask(tmp_path, "TileChoice c;\n" + "".join(
+        f'c = choose_tile({m}, {n}, {k // 64}, 256, {"true" if pair else "false"}, {ranks}); printf("%d\\n", c.tmx ? 32000 * c.tmx + 32 * c.tnx : c.big ? 256 : 128);\n' for ranks, pair, m, n, k, _ in cases))
+    assert [(c[:5], int(r[0])) for c, r in zip(cases, rows) if int(r[0]) not in c[5]] == []
+
+
+def test_sums_on_128_tiles_are_left_where_256_tiles_of_each_rank_measured_faster(tmp_path):
+    """Rows, columns, K, and whether one launch of both ranks was the faster one."""
+    cases = [(938, 4096, 14336, 0), (1464, 2416, 13440, 0), (1048, 1800, 4096, 0), (512, 4096, 5504, 1), (645, 4096, 5504, 0), (128, 4096, 4096, 1)]
+    rows = ask(tmp_path, "".join(f'printf("%d\\n", sum_predicted_faster({m}, {n}, {k // 64}, 256) ? 1 : 0);\n' for m, n, k, _ in cases))
+    assert [r[0] for r in rows] == [c[3] for c in cases]
