@@ -295,7 +295,8 @@ static bool stream_w8_cut(int64_t M, int64_t N, int ranks, bool sum, int cus, in
 // rotated weights against the three kernels of pick_w8_path and their finishing pass (TPAMD_STREAM=0 and =1). Sums 0.80 of the time where it is taken or not together (the better one each time: 0.79),
 // Linears 0.83 (0.82). The lines: x, which every CU reads whole, in microseconds at 70 GB/s a CU against the weights in MB (sums of 4096 x 8192 at 32 rows 27.5 -> 31.2 us, Linears of
 // 1024 x 8192 13.4 -> 14.9); fewer than 2048 columns leave CUs idle (sums of 1024 x 14336 at 4 rows 1.37); 16384 columns or more of rows of one or two KiB, which no skew spreads over the
-// memory channels (14336 x 1024 of two ranks at 32 rows 1.31, one 16384 x 2048 at 4 rows 1.20; rows of 1408 bytes 0.79).
+// memory channels (14336 x 1024 of two ranks at 32 rows 1.31, one 16384 x 2048 at 4 rows 1.20; rows of 1408 bytes 0.79); sums of 2048 columns, half of the CUs, on long rows (x 14336 at 4
+// rows 17.2 -> 22.7 us, now 16.5). Over 2434 other shapes 0.83 of the time, 2.1 % off the better choice, 56 of them more than 3 % slower, at worst 13 %.
 bool stream_w8_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t n_out, int ranks, bool sum, int cus) {
     int blocks = 0, rows = 0, groups = 0;
     if (tuning().stream == 0 || M < 2 || M > 32 || K % 128 != 0 || n_out > 256 || ldx >= (1ll << 22) || ldw >= (1ll << 22) || cus < ranks) return false;
@@ -305,7 +306,7 @@ bool stream_w8_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, i
     const int64_t all = N * (sum ? 1 : ranks);
     const double mb = static_cast<double>(all) * K * (sum ? 2.0e-6 : 1.0e-6), x_us = static_cast<double>(M) * K * (sum ? 4.0 : 2.0) / 70.0e3;
     if (K < 1024 || all < 2048) return false;
-    if (sum) return x_us < 2.0 + 0.08 * mb;
+    if (sum) return x_us < 2.0 + 0.08 * mb && !(N <= 2048 && K > 6144 && M >= 4);
     return x_us < 0.14 * mb && !(all >= 16384 && K <= 2048 && K % 1024 == 0);
 }
 

@@ -90,3 +90,19 @@ def test_one_tile_of_keys_takes_the_faster_attention_kernel(heads, keys, D, gene
         tune("TPAMD_ATTN_DECODE", decode)
         both.append(run())
     assert not torch.equal(*both) and torch.equal(chosen, both[0 if general else 1])
+
+
+@pytest.mark.parametrize("rows,cols,K,stream", [(4, 2048, 14336, False), (8, 2048, 11264, False), (3, 2048, 14336, True), (4, 2048, 6144, True), (4, 3072, 14336, True)])
+def test_int8_sums_on_half_of_the_cus_leave_stream_kernel(rows, cols, K, stream, tune):
+    """Two ranks' sums of 2048 columns, half a block per CU: on long rows other launches measured faster from 4 rows on."""
+    g = torch.Generator(device=DEV).manual_seed(1)
+    calls = [(draw(rows, K, seed=r), torch.randint(-127, 128, (cols, K), dtype=torch.int8, device=DEV, generator=g), torch.rand(cols, device=DEV, generator=g) * 1e-3, None, None, None)
+             for r in range(2)]
+
+    def run():
+        both = _native.linear_w8_sum_ranks(calls)
+        return both[0] if both is not None else _native.linear_w8(*calls[1], addend=_native.linear_w8(*calls[0]))
+
+    chosen = run()
+    tune("TPAMD_STREAM", 1)
+    assert torch.equal(chosen, run()) == stream
