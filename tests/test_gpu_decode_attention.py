@@ -70,6 +70,31 @@ def test_an_infinite_value_stays_infinite(keys, at, D, dtype):
     torch.testing.assert_close(got[finite], want[finite], rtol=2.0 ** (-8 if dtype is torch.bfloat16 else -11), atol=1e-5)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("splits", [1, 4])
+@pytest.mark.parametrize("D", [64, 128])
+def test_infinities_and_nans_beside_a_new_position(D, splits, dtype, monkeypatch):
+    """Infinite and undefined values in the cache, in several ranges, and in the new position: each makes its own column of its own sequence so, and no other. Equal scores: all
+    probabilities are one."""
+    monkeypatch.setenv("TPAMD_ATTN_SPLITS", str(splits))
+    _native.reload_tuning()
+    try:
+        B, Hkv, keys = 3, 2, 250
+        q, k, v, cos, sin = (draw(B, 1, n, D, dtype=dtype, seed=s).to(DEV) for n, s in ((2 * Hkv, 4), (Hkv, 5), (Hkv, 6), (1, 7), (1, 8)))
+        kc, vc = (draw(B, Hkv, keys + 1, D, dtype=dtype, seed=s).to(DEV) for s in (9, 10))
+        q.zero_()
+        vc[0, 1, 70, 5], vc[0, 1, 200, 6], vc[1, 0, 249, D - 1], v[1, 0, 1, 3], v[2, 0, 0, 0] = float("inf"), float("-inf"), float("nan"), float("inf"), float("nan")
+        got = _native.attention_decode_rope(q, k, v, cos[:, 0], sin[:, 0], kc, vc, keys, scale=0.1).float()[:, 0]
+    finally:
+        monkeypatch.undo()
+        _native.reload_tuning()
+    want = vc.float().mean(2).repeat_interleave(2, 1)  # the new position's values are in the cache now
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(torch.sign(got[torch.isinf(got)]), torch.sign(want[torch.isinf(want)]))
+    finite = torch.isfinite(want)
+    # sums of 251 values in fp32, rounded once to the dtype
+    torch.testing.assert_close(got[finite], want[finite], rtol=2.0 ** (-8 if dtype is torch.bfloat16 else -11), atol=1e-5)
+
+
 @pytest.mark.parametrize("G,D", [(1, 128), (16, 64)])
 @pytest.mark.parametrize("count", [1, 15, 16, 17, 31, 32, 33, 64])
 def test_few_keys_take_one_kernel_wherever_the_count_is(count, G, D):

@@ -398,10 +398,11 @@ def test_x_resident_weight_streaming_kernel(dtype, M, N, K, tune):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [17, 31, 32, 33, 48, 64])
 @pytest.mark.parametrize("N,K", [(2048, 4096), (4096, 5504), (1000, 2056), (132, 8192), (3072, 3072)])
-def test_single_matrix_with_few_tiles_at_17_to_64_rows(dtype, M, N, K):
+def test_single_matrix_with_few_tiles_at_17_to_64_rows(tune, dtype, M, N, K):
     """A single 16-bit matrix with at most one 16-column tile per CU stays on the weight-streaming kernel up to 32 rows
     (up to 64 with rows of at most 3072 elements; not at all with long rows on few tiles, which the tiled kernels split
-    over K): two and four row tiles of x, a partly filled last one, a ragged last K chunk, bias and GELU."""
+    over K) where stream_kernel does not take it (TPAMD_STREAM=0): two and four row tiles of x, a partly filled last one, a ragged last K chunk, bias and GELU."""
+    tune("TPAMD_STREAM", 0)
     x, w, b = rnd((M, K), 1, 1.0, dtype), rnd((N, K), 0, 0.02, dtype), rnd((N,), 2, 0.1, dtype)
     got = _native.linear(x.to(DEV), w.to(DEV), b.to(DEV), act=_native.ACT_GELU)
     check_half(got, F.gelu(F.linear(x.float(), w.float(), b.float())), K)
@@ -411,10 +412,11 @@ def test_single_matrix_with_few_tiles_at_17_to_64_rows(dtype, M, N, K):
 @pytest.mark.parametrize("M", [17, 20, 32, 33, 50, 64])
 @pytest.mark.parametrize("N,K", [(4608, 4096), (5504, 4096), (4100, 2048)])
 def test_k_split_tiles_with_part_of_the_x_tile(tune, dtype, M, N, K):
-    """17 to 64 rows of a single matrix with more than one 16-column tile per CU go to the K-split 128 x 128 kernel, which
-    then loads only the quarter or half of the x tile that exists and lets the two wavefronts of the missing rows only
+    """17 to 64 rows of a single matrix with more than one 16-column tile per CU go to the K-split 128 x 128 kernel where
+    stream_kernel does not take them (TPAMD_STREAM=0), which then loads only the quarter or half of the x tile that exists and lets the two wavefronts of the missing rows only
     load: against the fp32 host product, and bit for bit what the kernel with whole tiles gives (bias, GELU and the
     fused addend included; a ragged last column tile)."""
+    tune("TPAMD_STREAM", 0)
     x, w, b = rnd((M, K), 1, 1.0, dtype).to(DEV), rnd((N, K), 0, 0.02, dtype).to(DEV), rnd((N,), 2, 0.1, dtype).to(DEV)
     other = rnd((M, N), 7, 1.0, dtype).to(DEV)
     part = _native.linear(x, w, b, act=_native.ACT_GELU)
@@ -485,9 +487,10 @@ def test_gated_pair_with_x_staged_in_lds(dtype, M, N, K, tune):
 @pytest.mark.parametrize("M", [17, 24, 31, 32])
 @pytest.mark.parametrize("N,K", [(1376, 4096), (2048, 2048), (1000, 2056), (132, 5504)])
 def test_gated_pair_with_few_tiles_at_17_to_32_rows(dtype, M, N, K, tune):
-    """A gated pair with at most one 8-column tile per CU stays on the weight-streaming kernel up to 32 rows (two row
-    tiles of x, the second partly filled; a ragged last K chunk; a column count that is not a multiple of 8): against
+    """A gated pair with at most one 8-column tile per CU stays on the weight-streaming kernel up to 32 rows where
+    stream_kernel does not take it (TPAMD_STREAM=0; two row tiles of x, the second partly filled; a ragged last K chunk; a column count that is not a multiple of 8): against
     the oracle's gated hidden state, and against the tiled kernels that take these rows on wider matrices."""
+    tune("TPAMD_STREAM", 0)
     x, w, w2 = rnd((M, K), 1, 1.0, dtype).to(DEV), rnd((N, K), 0, 0.02, dtype).to(DEV), rnd((N, K), 5, 0.02, dtype).to(DEV)
     h = _native.swiglu_up(x, w, w2)
     sigma = (0.02 * math.sqrt(K)) ** 2
@@ -552,10 +555,11 @@ def test_other_dispatch_paths_inside_a_hip_graph(case, tune):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [1, 2, 3])
 @pytest.mark.parametrize("N,K", [(2048, 512), (2053, 520), (4100, 5504), (6000, 1032), (3000, 8192), (4096, 4096), (8192, 6656), (8200, 4096), (4608, 8192), (1376, 6144)])
-def test_row_streaming_kernel_on_wide_matrices(dtype, M, N, K):
+def test_row_streaming_kernel_on_wide_matrices(tune, dtype, M, N, K):
     """M <= 3 and thousands of output columns (ragged column count, ragged last K step): against the fp32 host
     product, the gated pair against the oracle, the fused sum bit for bit. The shapes reach every choice of the rule
-    for these row counts: blocks of 4, 8 and 16 wavefronts, the general row kernel, the MFMA kernels at 2 rows."""
+    for these row counts without stream_kernel (TPAMD_STREAM=0): blocks of 4, 8 and 16 wavefronts, the general row kernel, the MFMA kernels at 2 rows."""
+    tune("TPAMD_STREAM", 0)
     x, w, w2, b = rnd((M, K), 1, 1.0, dtype).to(DEV), rnd((N, K), 0, 0.02, dtype).to(DEV), rnd((N, K), 5, 0.02, dtype).to(DEV), rnd((N,), 2, 0.1, dtype).to(DEV)
     lin = _native.linear(x, w, b)
     check_half(lin, F.linear(x.float().cpu(), w.float().cpu(), b.float().cpu()), K)

@@ -43,7 +43,8 @@ def test_edges_of_a_tile(tile, over, K):
     total = _native.linear(xs[1], ws[1], addend=first, copy=copy)
     close(total, wants[0] + wants[1], dtype, 3)
     assert torch.equal(total, copy)
-    half = cols // 2
-    pairs = [(x, w[:half], w[half:2 * half]) for x, w in zip(xs, ws)]
+    # a pair's tile has half as many columns: two tiles of gate and up rows, 4 rows fewer or more
+    half = tile % 1000 + 4 * over
+    pairs = [(x, draw(half, K, dtype=dtype, seed=5 + r, scale=0.1), draw(half, K, dtype=dtype, seed=7 + r, scale=0.1)) for r, x in enumerate(xs)]
     for h, (x, g, u) in zip(_native.swiglu_up_ranks(pairs), pairs):
         close(h, torch.nn.functional.silu(x.float() @ g.float().t()) * (x.float() @ u.float().t()), dtype, 4)

@@ -1,5 +1,7 @@
 """stream_kernel (decode-sized Linears, gated pairs and sums of two ranks on one block per CU) where it can go wrong: around its row and column counts, K that
 does not fill every wavefront, and every form of the epilogue; TPAMD_STREAM=1 sends it what its rule would leave to the other kernels."""
+import ctypes
+
 import pytest
 import torch
 
@@ -62,7 +64,8 @@ def test_gated_pair(rows, cols, K):
     hs = _native.swiglu_up_ranks(list(zip(xs, gs, us)))
     for x, g, u, h in zip(xs, gs, us, hs):
         close(h, torch.nn.functional.silu(x.float() @ g.float().t()) * (x.float() @ u.float().t()), dtype, 4)
-    assert torch.isfinite(hs[0]).all() and _native.swiglu_up(xs[0], gs[0], us[0]).shape == hs[0].shape
+    # one rank alone is cut differently
+    close(_native.swiglu_up(xs[0], gs[0], us[0]), torch.nn.functional.silu(xs[0].float() @ gs[0].float().t()) * (xs[0].float() @ us[0].float().t()), dtype, 4)
 
 
 @pytest.mark.parametrize("rows", [2, 8, 9, 17, 32, 33, 40, 64])
@@ -83,3 +86,24 @@ def test_strided_rows_of_x_and_rows_past_the_end_stay_out():
     wide[37:], w[1036:] = float("nan"), float("nan")
     y = _native.linear(wide[:37, :512], w[:1036])
     close(y, wide[:37, :512].float() @ w[:1036].float().t(), torch.bfloat16)
+
+
+@pytest.mark.parametrize("rows,cols,K", [(8, 516, 192), (17, 3076, 320), (40, 1032, 1088)])
+def test_pitches_of_weights_and_outputs(rows, cols, K):
+    """Through the C entry points: weights and outputs with room between their rows, which holds NaN and is left alone."""
+    dtype, code, stream = torch.bfloat16, _native.dtype_code(torch.bfloat16), ctypes.c_void_p(torch.cuda.current_stream(DEV).cuda_stream)
+    x, g, u = draw(rows, K, dtype=dtype, seed=1), draw(cols, K + 24, dtype=dtype, seed=2, scale=0.05), draw(cols, K + 24, dtype=dtype, seed=3, scale=0.05)
+    g[:, K:], u[:, K:] = float("nan"), float("nan")
+    y = torch.full((rows + 1, cols + 20), 7.0, dtype=dtype, device=DEV)
+    gate, up = x.float() @ g[:, :K].float().t(), x.float() @ u[:, :K].float().t()
+    assert _native.lib().tpamd_linear(x.data_ptr(), g.data_ptr(), None, y.data_ptr(), rows, cols, K, K, K + 24, cols + 20, code, _native.ACT_NONE, stream) == 0
+    close(y[:rows, :cols], gate, dtype)
+    assert bool((y[:, cols:] == 7.0).all()) and bool((y[rows] == 7.0).all())
+    assert _native.lib().tpamd_swiglu_up(x.data_ptr(), g.data_ptr(), u.data_ptr(), y.data_ptr(), rows, cols, K, K, K + 24, cols + 20, code, stream) == 0
+    close(y[:rows, :cols], torch.nn.functional.silu(gate) * up, dtype, 4)
+    assert bool((y[:, cols:] == 7.0).all()) and bool((y[rows] == 7.0).all())
+    both = torch.full((2, rows + 1, cols + 20), 7.0, dtype=dtype, device=DEV)
+    two = lambda *t: (ctypes.c_void_p * 2)(*[v.data_ptr() for v in t])
+    assert _native.lib().tpamd_linear_sum_ranks(two(x, x), two(g, u), None, two(both[0], both[1]), rows, cols, K, K, K + 24, cols + 20, code, stream) == 0
+    close(both[0, :rows, :cols], gate + up, dtype, 3)
+    assert torch.equal(both[0], both[1]) and bool((both[:, :, cols:] == 7.0).all()) and bool((both[:, rows] == 7.0).all())

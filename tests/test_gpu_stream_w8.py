@@ -1,5 +1,7 @@
 """stream_w8_kernel (int8 Linears of 2 to 32 rows and sums of two ranks on one block per CU) where it can go wrong: around its row and column counts, K that does not fill
 every wavefront, outlier columns in none, one or several groups per wavefront, every form of the epilogue; TPAMD_STREAM=1 sends it what its rule would leave to others."""
+import ctypes
+
 import pytest
 import torch
 
@@ -68,3 +70,22 @@ def test_sum_of_two_ranks(rows, cols, K, n_out):
     sums = _native.linear_w8_sum_ranks(calls)
     close(sums[0], wants[0] + wants[1], dtype, 3)
     assert torch.equal(sums[0], sums[1]) and sums[0].data_ptr() != sums[1].data_ptr()
+
+
+@pytest.mark.parametrize("rows,cols,K,n_out", [(8, 516, 384, 33), (17, 4608, 640, 0), (32, 1032, 1152, 40)])
+def test_pitches_of_weights_and_outputs(rows, cols, K, n_out):
+    """Through the C entry point: weights, outlier weights and outputs with room between their rows, which holds the largest codes or NaN and is left alone."""
+    dtype = torch.float16
+    (x, wq, scale, idx, w_out, bias), want = rank(rows, cols, K, n_out, dtype, 5)
+    wide = torch.full((cols, K + 48), 127, dtype=torch.int8, device=DEV)
+    wide[:, :K] = wq
+    wide_out = torch.full((cols, n_out + 3), float("nan"), dtype=dtype, device=DEV)
+    if n_out:
+        wide_out[:, :n_out] = w_out
+    y = torch.full((rows + 1, cols + 20), 7.0, dtype=dtype, device=DEV)
+    rc = _native.lib().tpamd_linear_w8(x.data_ptr(), wide.data_ptr(), scale.data_ptr(), idx.data_ptr() if n_out else None, wide_out.data_ptr() if n_out else None, n_out,
+                                       None if bias is None else bias.data_ptr(), y.data_ptr(), rows, cols, K, x.stride(0), K + 48, n_out + 3, cols + 20,
+                                       _native.dtype_code(dtype), _native.ACT_NONE, ctypes.c_void_p(torch.cuda.current_stream(DEV).cuda_stream))
+    assert rc == 0
+    close(y[:rows, :cols], want, dtype)
+    assert bool((y[:, cols:] == 7.0).all()) and bool((y[rows] == 7.0).all())
