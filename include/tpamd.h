@@ -286,14 +286,16 @@ int tpamd_rope(const void *q_dev, const void *k_dev, const void *cos_dev, const 
  *   out [B, Hq, D] = softmax(scale * rot(q) . [cache keys, rot(k)]^T) [cache values, v].
  * One launch, or two where the keys of a head are cut into ranges, instead of three: the attention kernel rotates its query fragments itself; it or
  * the merge of the ranges' partial results adds the new position (its score in fp32 from the rotated rows) and writes the
- * cache rows. Rounding differs from the two-call sequence only in that the new position's probability is not rounded to
- * `dtype` before it weighs its value.
+ * cache rows. It differs from the two-call sequence in rounding: the new position's probability is not rounded to `dtype` before it
+ * weighs its value, the two forms may cut the keys into different ranges, and the kernel for up to 16 query heads per key/value head carries
+ * probabilities as two parts of `dtype` where the general one rounds them.
  *   strides: 16 element strides, {q batch, q head, q group, k batch, k head, v batch, v head, cos/sin batch (0 when
  *   shared), k_cache batch, k_cache head, k_cache position, v_cache batch, v_cache head, v_cache position, out batch,
  *   out head}; the first 14 multiples of 8, the last two of 4; pointers 16-byte aligned (out: 8).
- * Beyond 16 query heads per key/value head, and on caches of up to 32 positions, needs the stream's scratch buffer for the partial
- * results: TPAMD_ERR_UNSUPPORTED when there is none (the stream's first use of it under capture, or a batch too large for it);
- * callers then use the two entry points above. */
+ * A call may need the stream's scratch buffer for partial results: TPAMD_ERR_UNSUPPORTED when there is none (the stream's first use of it
+ * under capture, or a batch too large for it); callers then use the two entry points above. (It does beyond 16 query heads per
+ * key/value head, for thousands of heads on at most 96 positions, for caches that span more than 10^9 elements between the first and the
+ * last position of a head, and where the environment chooses the general kernel; others do without it, in one range.) */
 int tpamd_attention_decode_rope(const void *q_dev, const void *k_dev, const void *v_dev, const void *cos_dev,
                                 const void *sin_dev, void *k_cache_dev, void *v_cache_dev, void *out_dev, int64_t B,
                                 int64_t Hq, int64_t Hkv, int64_t D, int64_t pos0, int64_t cache_len, const int64_t *strides,

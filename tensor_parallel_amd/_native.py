@@ -1063,7 +1063,7 @@ def rope(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor)
 def attention_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                           k_cache: torch.Tensor, v_cache: torch.Tensor, pos0, scale: Optional[float] = None,
                           out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """`rope_append` and `attention` for one new position per sequence, in two launches instead of three.
+    """`rope_append` and `attention` for one new position per sequence, in one or two launches instead of two or three.
     q [B, 1, Hq, D] or [B, 1, Hkv, Hq / Hkv, D], k / v [B, 1, Hkv, D] (views of the projection output), cos / sin [B or 1, 1, D]
     (or [1, D] / [D]); the caches [B, Hkv, L, D] hold pos0 positions and receive the new one at pos0. Returns [B, 1, Hq, D].
     Where the library has no scratch buffer for the stream (first use under graph capture) the two calls are made instead.

@@ -60,7 +60,7 @@ constexpr int64_t SKINNY_MAX_M = 16;
 //                                                              (longer rows: streaming up to 32 rows)
 //   2048 x 8192  14.4 16.4 21.0 22.9 / 13.2 13.9 15.1 16.0     1536 x 6144  11.8 13.6 17.1 18.5 / 11.7 12.2 12.6 13.1
 //                                                              (K >= 6144 on at most half a tile per CU: tiled from 17 rows)
-// With more tiles the tiled kernels win from 17 rows on (11008 x 4096: 26.5 29.0 36.2 39.0 / 24.6 25.4 25.3 26.5), and the
+// Beside stream_kernel, which is asked first (decode_rows). With more tiles the tiled kernels win from 17 rows on (11008 x 4096: 26.5 29.0 36.2 39.0 / 24.6 25.4 25.3 26.5), and the
 // gated pair is faster through them at all of these sizes.
 int skinny_row_limit(int64_t N, int64_t K, int64_t *rows) {
     *rows = SKINNY_MAX_M;
@@ -312,17 +312,18 @@ extern "C" int tpamd_linear_gather_ranks(int n, const void *const *x_dev, const 
     return gemm_dispatch(x_dev[0], w_dev[0], nullptr, b0, nullptr, 0, y_dev[0], M, N, K, ldx, ldw, ldy, dtype, act, false, false, s, &to, copy);
 }
 
-// What takes the sum of two ranks' row-parallel Linears. Measured inside a HIP graph on rotated weights against tpamd_linear + tpamd_linear_add_copy (us, two
+// What takes the sum of two ranks' row-parallel Linears: stream_kernel at 2 to 64 rows where it is the faster one (stream_model.h: 3 to 16 rows of whole 64-element units always, 4096 x 5504 at 16 rows
+// 20.3 us, 22.1 by what follows), else what follows. Measured inside a HIP graph on rotated weights against tpamd_linear + tpamd_linear_add_copy (us, two
 // launches / row kernel with 8 wavefronts / with 16 / MFMA weight streaming / K ranges of 128 x 128 tiles):
 //   1 row    4096 x 2048   9.4 /  7.1  7.2            4096 x 5504 19.2 / 18.6 17.6     8192 x 4096 24.1 / 23.5 22.7     1024 x 1408 5.8 / 3.4  4.4
 //   2 rows   4096 x 2048  10.2 /  8.3  8.7            4096 x 5504 20.3 / 22.2 43.1     8192 x 4096 26.5 / 30.4 41.9     2048 x 2816 10.0 / 7.6 11.5
 //   4 rows   4096 x 2048  12.0 /           9.3        4096 x 5504 23.0 /      19.7     8192 x 4096 28.4 /      23.8     2048 x 2816 11.7 /      8.3
 //   16 rows  4096 x 2048  13.4 /          10.1        4096 x 5504 25.2 /      21.5     8192 x 4096 30.6 /      27.1     5120 x 6912 34.5 / 39.3, 31.1 in tiles
 //   40 rows  4096 x 2048  19.9 /               14.0   4096 x 5504 35.3 /      26.8     8192 x 4096 38.3 /      35.4     5120 x 6912 40.8 /      32.2
-// So the row kernel takes one row, and two where they are short or few; weight streaming the others up to the row count it has for one matrix of both ranks' K,
+// So beside stream_kernel the row kernel takes one row, and two where they are short or few; weight streaming the others up to the row count it has for one matrix of both ranks' K,
 // unless its tiles are a ragged number of rounds; K ranges of tiles the rest, above 64 rows while they are predicted to be faster than two launches. What stays in two
 // launches and why: sum_in_two_launches (gemm_model.h).
-enum SumPath { SUM_NONE, SUM_ROWS8, SUM_ROWS16, SUM_STREAM, SUM_TILES };
+enum SumPath { SUM_NONE, SUM_STREAM, SUM_ROWS8, SUM_ROWS16, SUM_SKINNY, SUM_TILES };
 static int sum_path(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, SumPath *path) {
     *path = SUM_NONE;
     int dev = 0, cus = 256;
@@ -343,7 +344,7 @@ static int sum_path(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, S
     if (M > SKINNY_MAX_M && M <= 64) {
         if (int rc = skinny_row_limit(N, 2 * K, &rows); rc != TPAMD_OK) return rc;
     }
-    if (M <= rows && !ragged) *path = SUM_STREAM;
+    if (M <= rows && !ragged) *path = SUM_SKINNY;
     else if (M <= 64 ? K % 64 == 0 && (N + 127) / 128 * 2 <= 4ll * cus : sum128_pays(M, N, K, cus)) *path = SUM_TILES;  // (the tiles that scratch memory holds)
     return TPAMD_OK;
 }

@@ -623,10 +623,12 @@ __global__ __launch_bounds__(256) void attention_combine_newkey_kernel(AttnParam
 // wavefronts of a block meet once, at the end, where their (m, l, O) are merged in LDS. A block that has a head's keys for itself (one split) finishes the rows,
 // the new position included, so that no partials are written and no second launch merges them.
 //
-// Bound: HBM. 128 MiB of K and V (8 x 16 heads a rank, two ranks, 2048 positions) 55.4 -> 44.2 us with the new position (6.05 TB/s), 40 sequences on 1000 positions, 4 key/value heads
-// a rank 43.0 -> 37.5, 64 sequences on 1000, head_dim 64 33.6 -> 26; one sequence on 500 11.1 -> 10. Over 190 shapes 0.77 of the time of attention_kernel and its merge. What it took:
+// Bound: HBM. 256 MiB of K and V (8 x 16 heads a rank, two ranks, 2048 positions) 52.5 -> 43.6 us with the new position (6.15 TB/s), 40 sequences on 1000 positions, 4 key/value heads
+// a rank 42.6 -> 36.9, 64 sequences of 8 heads of 64 elements a rank on 1000 56.4 -> 46.1 (5.7 TB/s), 16 of 4 key/value heads of 64 on 2048 21.9 -> 18.7; one sequence on 500 10.2 -> 10.1.
+// Over 361 shapes 0.78 of the time of attention_kernel and its merge with a new position, 0.87 without. What it took:
 // loads past the caches' replacement (53.8 -> 48.9 us on the first of these), wavefronts that walk the keys together instead of a quarter each (-> 44.4), and no
-// second launch. More stages than two are slower (16 KiB a wavefront and stage pair: more blocks share a CU instead).
+// second launch. More stages than two are slower (16 KiB a wavefront and stage pair: more blocks share a CU instead). Slower than attention_kernel by up to 1.2 us: one
+// key/value head in all on 350 to 500 keys (7.2 -> 8.4), and few heads on caches of fixed length that are nearly empty (1 head on 141 of 564 positions 7.6 -> 8.8).
 // Piece c (16 bytes) of a staged row r is in slot c ^ r (head_dim 64: c ^ ((r / 2) % 8)): the fragment reads and the transposing reads of 16 rows are conflict-free.
 constexpr int AD_KEYS = 16;
 template <int DT>
@@ -785,7 +787,7 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnParams p) {
             for (int j = 0; j < 4; ++j) s[j] = __builtin_amdgcn_exp2f(s[j] + SHIFT);
             l_run += (s[0] + s[1]) + (s[2] + s[3]);
             // the probabilities as two parts of the tensor dtype: one rounded that is always the smaller, and what is left. Both are above zero (an infinite value times a rest of
-            // zero, or of the other sign, would be NaN)
+            // zero, or of the other sign, would be NaN); in fp16 so down to 2^-23 of the largest, below which a value that is infinite may become NaN, as in attention_kernel below 2^-25
             const uint2 hi = make_uint2(pack2_half<DT>(s[0] * LESS, s[1] * LESS), pack2_half<DT>(s[2] * LESS, s[3] * LESS));
             const uint2 lo = make_uint2(pack2_half<DT>(s[0] - lo_half_to_f32<DT>(hi.x), s[1] - hi_half_to_f32<DT>(hi.x)),
                                         pack2_half<DT>(s[2] - lo_half_to_f32<DT>(hi.y), s[3] - hi_half_to_f32<DT>(hi.y)));

@@ -16,8 +16,8 @@ namespace {
 //           tile g is read out; then the fragments of tile g + 1, and tile g + NS into the stage of tile g, spread over the MFMAs
 // Bound: the matrix pipe at the clock its power leaves (1.8-2.0 GHz), the start and the epilogue of a launch, and CUs without a tile. By the SQ counters
 // of 2103 rows in fp16 the pipes are busy 54 % of a launch of 242 tiles of 192 x 192 and 58 % of one of 473 gated tiles of 192 x 256 (two rounds); the
-// fragment reads keep LDS busy 15-20 % of it and wavefronts wait for LDS 4-5 % of their time. A K tile of 192 x 192 takes 0.64 us on an idle
-// chip and 0.83 in a full round, where its MFMAs need 0.48 at 2.4 GHz; 192 x 256, on two stages, 0.92-1.23 (0.64).
+// fragment reads keep LDS busy 15-20 % of it and wavefronts wait for LDS 4-5 % of their time. A K tile of 192 x 192 takes 0.69 us
+// with half of the CUs idle and 0.88 in a full round, where its MFMAs need 0.48 at 2.4 GHz; 192 x 256, on two stages, 1.04-1.25 (0.64): the fits of MID_TILES.
 template <int DT, int MODE, int TMX, int TNX, int NS>
 __global__ __launch_bounds__(256) void gemm_mid_kernel(GemmParams p) {
     constexpr int BM = 32 * TMX, BN = 32 * TNX, BN_OUT = MODE == MODE_SWIGLU ? BN / 2 : BN;

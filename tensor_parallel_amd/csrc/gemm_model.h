@@ -183,8 +183,9 @@ inline bool w8_slabs_without_scratch(int64_t M, int64_t N, int64_t K, bool outli
     return M / 64.0 * (5.0 + k * (5.5 + N / 512.0)) <= 6.0 + k * (outliers ? 53.0 : 36.0);
 }
 
-// Rows, columns and K of a row-parallel Linear whose sum over two ranks stays in two launches (tpamd_linear, then tpamd_linear_add_copy) whatever the kernels for
-// both ranks could take of it: where one launch measured slower, and what was not measured. In a HIP graph on rotated weights, one launch / two: 227 random
+// Rows, columns and K of a row-parallel Linear whose sum over two ranks stays in two launches (tpamd_linear, then tpamd_linear_add_copy) whatever the older kernels for
+// both ranks could take of it: where one launch of those measured slower, and what was not measured. Asked only where stream_kernel does not take the sum (stream_model.h), so that what stands
+// here for 2 to 16 rows is for K that is no multiple of 64, little weight, and TPAMD_STREAM=0; the timings are those of the older kernels. In a HIP graph on rotated weights, one launch / two: 227 random
 // shapes of 1024-8192 columns, K 1024-8192 and 1-600 rows 0.76 (geometric mean), of which five above 1.02. Those, and what 550 more timings of longer and wider
 // matrices found, are the exceptions here, by rounds of one 16-column tile per CU (a ragged count does not end on a whole round):
 //  - 1 row: long rows, which the kernel for one matrix streams as fast (4096 x 8192: 24.9 us in two, 26.2 in one; ragged 5120 x 5504: 24.1, 26.8).
