@@ -11,6 +11,7 @@ Action values for inputs/outputs are a StateAction, a callable `(x, rank=...)`, 
 from __future__ import annotations
 
 import dataclasses
+import functools
 import logging
 import re
 from itertools import chain
@@ -123,18 +124,19 @@ def add_lora_rules(model: nn.Module, config: Config) -> Config:
     return config
 
 
+@functools.lru_cache(maxsize=256)
+def _module_end(pattern: str) -> re.Pattern:
+    """Finds the end of a module that `pattern` matches in a parameter's name: trailing "$" dropped, "\\." appended unless it already ends with "."."""
+    if pattern.endswith("$"):
+        pattern = pattern[:-1]
+    if not pattern.endswith("."):
+        pattern += r"\."
+    return re.compile(pattern)
+
+
 def wrapped_module_patterns(tensor_parallel_config: Config) -> list:
-    """Patterns that find, in a parameter's name, the ends of the modules that get wrapped: those of the modules with an input or output rule
-    (trailing "$" dropped, "\\." appended unless it already ends with ".")."""
-    seen = set()
-    for regex in chain(tensor_parallel_config.input_rules, tensor_parallel_config.output_rules):
-        pattern = regex.pattern
-        if pattern.endswith("$"):
-            pattern = pattern[:-1]
-        if not pattern.endswith("."):
-            pattern += r"\."
-        seen.add(pattern)
-    return [re.compile(p) for p in seen]
+    """Patterns that find, in a parameter's name, the ends of the modules that get wrapped: those of the modules with an input or output rule."""
+    return list({_module_end(regex.pattern) for regex in chain(tensor_parallel_config.input_rules, tensor_parallel_config.output_rules)})
 
 
 def wrapped_names(names: Iterable[str], patterns: Sequence[re.Pattern]) -> Mapping[str, str]:
